@@ -101,40 +101,63 @@ struct SpmmArgs {
 constexpr int kNoCarry = -1;
 constexpr int kMerged = -2;
 
+// Global memory is read and written in packs that need the alignment of one element only (the
+// hardware takes a 16-byte access at any multiple of four bytes): rows of a width that is no
+// whole number of packs begin anywhere.
+template <typename T, int VEC>
+struct Unaligned {
+    typedef T type __attribute__((ext_vector_type(VEC), aligned(sizeof(T))));
+};
+template <typename T>
+struct Unaligned<T, 1> {
+    typedef T type;
+};
+
+template <typename T, int VEC>
+__device__ __forceinline__ Pack<T, VEC> to_pack(const typename Unaligned<T, VEC>::type &v) {
+    Pack<T, VEC> x;
+    if constexpr (VEC == 1) x.v[0] = v;
+    else
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) x.v[i] = v[i];
+    return x;
+}
+template <typename T, int VEC>
+__device__ __forceinline__ typename Unaligned<T, VEC>::type of_pack(const Pack<T, VEC> &x) {
+    typename Unaligned<T, VEC>::type v;
+    if constexpr (VEC == 1) v = x.v[0];
+    else
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) v[i] = x.v[i];
+    return v;
+}
+
 template <typename T, int VEC>
 __device__ __forceinline__ Pack<T, VEC> load_pack(const T *p) {
-    return *reinterpret_cast<const Pack<T, VEC> *>(p);
+    return to_pack<T, VEC>(*reinterpret_cast<const typename Unaligned<T, VEC>::type *>(p));
 }
 // Streaming load for rows that this launch reads once.
 template <typename T, int VEC>
 __device__ __forceinline__ Pack<T, VEC> load_pack_stream(const T *p) {
-    Pack<T, VEC> x;
-    if constexpr (VEC == 1) {
-        x.v[0] = __builtin_nontemporal_load(p);
-    } else {
-        typedef T vec_t __attribute__((ext_vector_type(VEC)));
-        const vec_t v = __builtin_nontemporal_load(reinterpret_cast<const vec_t *>(p));
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) x.v[i] = v[i];
-    }
-    return x;
+    return to_pack<T, VEC>(__builtin_nontemporal_load(reinterpret_cast<const typename Unaligned<T, VEC>::type *>(p)));
 }
 template <typename T, int VEC>
 __device__ __forceinline__ void store_pack(T *p, const Pack<T, VEC> &x) {
-    *reinterpret_cast<Pack<T, VEC> *>(p) = x;
+    *reinterpret_cast<typename Unaligned<T, VEC>::type *>(p) = of_pack<T, VEC>(x);
 }
 // Streaming store for rows that are written once and not read again by this launch.
 template <typename T, int VEC>
 __device__ __forceinline__ void store_pack_stream(T *p, const Pack<T, VEC> &x) {
-    if constexpr (VEC == 1) {
-        __builtin_nontemporal_store(x.v[0], p);
-    } else {
-        typedef T vec_t __attribute__((ext_vector_type(VEC)));
-        vec_t v;
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) v[i] = x.v[i];
-        __builtin_nontemporal_store(v, reinterpret_cast<vec_t *>(p));
-    }
+    __builtin_nontemporal_store(of_pack<T, VEC>(x), reinterpret_cast<typename Unaligned<T, VEC>::type *>(p));
+}
+
+// First feature of the pack that starts at multiple `f` of VEC: where F is no whole number of packs
+// the last pack of a row is moved back to end with the row and overlaps the one before it.  Both
+// lanes then compute the same values for the shared elements and store them with one
+// instruction of one wave (pick_shape allows the overlap for rows of one tile only).
+template <int VEC>
+__device__ __forceinline__ int64_t pack_start(int64_t F, int64_t f) {
+    return VEC > 1 && f > F - VEC ? F - VEC : f;
 }
 
 // Per-lane feature offsets of the TILES tiles; foff[t] < 0 marks a tile beyond F.
@@ -143,7 +166,7 @@ __device__ __forceinline__ void feature_offsets(int64_t F, int lane, int64_t fof
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
         int64_t f = ((int64_t)(blockIdx.y * TILES + t) * LPR + lane) * VEC;
-        foff[t] = f < F ? f : -1;
+        foff[t] = f < F ? pack_start<VEC>(F, f) : -1;
     }
 }
 
@@ -255,8 +278,11 @@ __device__ __forceinline__ Pack<T, VEC> gather(const SpmmArgs<T> &a, int c, int 
     else
         x = load_pack<T, VEC>(base + off);
     if constexpr (MODE == MODE_SIGN_MASK) {
-        // VEC divides 32, so the bits of one pack lie in one word
-        const uint32_t bits = a.signs[(int64_t)c * a.sign_words + (foff >> 5)] >> (foff & 31);
+        const uint32_t *words = a.signs + (int64_t)c * a.sign_words;
+        uint32_t bits = words[foff >> 5] >> (foff & 31);
+        // VEC divides 32, so the bits of one pack lie in one word, unless the pack was moved back
+        if (VEC > 1 && (a.F & (VEC - 1)) != 0 && (foff & 31) > 32 - VEC)
+            bits |= words[(foff >> 5) + 1] << (32 - (foff & 31));
 #pragma unroll
         for (int i = 0; i < VEC; ++i) x.v[i] = ((bits >> i) & 1u) ? x.v[i] : T(0);
     }
@@ -680,7 +706,8 @@ __global__ __launch_bounds__(kBlock) void spmm_carry_reduce_kernel(SpmmArgs<T> a
     int head_row = -1, tail_row = -1;
     T *slot0 = a.carry_out + (int64_t)(2 * chunk) * a.F;
     T *slot1 = slot0 + a.F;
-    for (int64_t f = (int64_t)sub * VEC; f < a.F; f += (int64_t)LPR * VEC) {
+    for (int64_t nominal = (int64_t)sub * VEC; nominal < a.F; nominal += (int64_t)LPR * VEC) {
+        const int64_t f = pack_start<VEC>(a.F, nominal);
         Pack<T, VEC> acc, zero;
 #pragma unroll
         for (int i = 0; i < VEC; ++i) acc.v[i] = zero.v[i] = T(0);
@@ -694,7 +721,8 @@ __global__ __launch_bounds__(kBlock) void spmm_carry_reduce_kernel(SpmmArgs<T> a
                 // timing; sent as an atomic only so that the lane need not wait for Y.
                 T *y = a.Y + (int64_t)out_row(a, cur) * a.F + f;
 #pragma unroll
-                for (int i = 0; i < VEC; ++i) unsafeAtomicAdd(y + i, acc.v[i]);
+                for (int i = 0; i < VEC; ++i)
+                    if (f + i >= nominal) unsafeAtomicAdd(y + i, acc.v[i]);  // the elements before are the lane's before
                 return;
             }
             if (from_before) {
@@ -792,7 +820,8 @@ __global__ __launch_bounds__(kBlock) void spmm_fixup_kernel(SpmmArgs<T> a) {
     if (row >= 0) {
         const int64_t group0 = (int64_t)(s0 / stride) * stride;
 #pragma unroll 1
-        for (int64_t f = (int64_t)sub * VEC; f < a.F; f += (int64_t)LPR * VEC) {
+        for (int64_t nominal = (int64_t)sub * VEC; nominal < a.F; nominal += (int64_t)LPR * VEC) {
+            const int64_t f = pack_start<VEC>(a.F, nominal);
             Pack<T, VEC> acc, zero;
 #pragma unroll
             for (int i = 0; i < VEC; ++i) acc.v[i] = zero.v[i] = T(0);
@@ -854,7 +883,7 @@ __global__ __launch_bounds__(kBlock) void spmm_fixup_kernel(SpmmArgs<T> a) {
 #pragma unroll
         for (int i = 0; i < VEC; ++i) zero.v[i] = T(0);
         for (int64_t f = (int64_t)sub * VEC; f < a.F; f += (int64_t)LPR * VEC)
-            store_pack_stream<T, VEC>(a.Y + (int64_t)erow * a.F + f, zero);
+            store_pack_stream<T, VEC>(a.Y + (int64_t)erow * a.F + pack_start<VEC>(a.F, f), zero);
     }
 }
 
@@ -877,7 +906,8 @@ __global__ __launch_bounds__(kBlock) void spmm_fixup_rows_kernel(SpmmArgs<T> a) 
         const int64_t s0 = a.rowptr[row] / a.seg_nnz;           // the run the row starts in
         const int64_t group0 = s0 / a.merge_stride * a.merge_stride;  // first run of that run's workgroup
 #pragma unroll 1
-        for (int64_t f = (int64_t)sub * VEC; f < a.F; f += (int64_t)LPR * VEC) {
+        for (int64_t nominal = (int64_t)sub * VEC; nominal < a.F; nominal += (int64_t)LPR * VEC) {
+            const int64_t f = pack_start<VEC>(a.F, nominal);
             Pack<T, VEC> acc, zero;
 #pragma unroll
             for (int i = 0; i < VEC; ++i) acc.v[i] = zero.v[i] = T(0);
@@ -913,7 +943,7 @@ __global__ __launch_bounds__(kBlock) void spmm_fixup_rows_kernel(SpmmArgs<T> a) 
 #pragma unroll
     for (int i = 0; i < VEC; ++i) zero.v[i] = T(0);
     for (int64_t f = (int64_t)sub * VEC; f < a.F; f += (int64_t)LPR * VEC)
-        store_pack_stream<T, VEC>(a.Y + (int64_t)erow * a.F + f, zero);
+        store_pack_stream<T, VEC>(a.Y + (int64_t)erow * a.F + pack_start<VEC>(a.F, f), zero);
 }
 
 // ------------------------------------------------------------------- dispatch --
@@ -921,26 +951,25 @@ struct Shape {
     int vec, lpr, tiles, grid_y;
 };
 
-// Lane layout for a feature width: the widest vector the width and the pointers'
-// alignment allow, then as many lanes as a row needs (power of two, 4..64).
-// min_lpr: narrow the vectors (down to single words) while a row would take fewer lanes than
-// this.  The nnz schedule asks for 16: with 4 lanes per run a wave walks 16 runs at once, each
-// with its own row changes (F = 16: 0.106 -> 0.089 ms for the forward vertex stage of the web
-// graph); the row schedule is faster with the widest vectors (0.036 against 0.053 ms).
+// Lane layout for a feature width.  Packs need no alignment and the last one of a row may overlap the
+// one before it (pack_start), so rows of up to 64 packs of four take packs whatever their
+// width: 47 features are 12 lanes of four (the nnz kernel of a 50,001-vertex graph took 27.8 us
+// with one feature a lane, 22.8 us so).  Longer rows are walked in several tiles, where an overlap
+// would add a carry twice, and take the widest packs that divide the width.
+// runs: the layout of the nnz schedule, which wants 16 lanes or more per run -- with 4 lanes a
+// wave walks 16 runs at once, each with its own row changes (F = 16: 0.106 -> 0.089 ms for the forward
+// vertex stage of the web graph) -- and so takes the narrowest packs that 16 lanes hold.
+// The row schedule is faster with the widest packs (0.036 against 0.053 ms).
 template <typename T>
-Shape pick_shape(int64_t F, const void *p0, const void *p1, const void *p2, const void *p3, int min_lpr = 4) {
-    auto aligned = [&](size_t bytes) {
-        auto ok = [&](const void *p) { return p == nullptr || (reinterpret_cast<uintptr_t>(p) % bytes) == 0; };
-        return ok(p0) && ok(p1) && ok(p2) && ok(p3);
-    };
+Shape pick_shape(int64_t F, bool runs) {
     Shape s;
     s.vec = 1;
     if (sizeof(T) == 4) {
-        if (F % 4 == 0 && aligned(16)) s.vec = 4;
-        else if (F % 2 == 0 && aligned(8)) s.vec = 2;
-        while (s.vec > 1 && F / s.vec < min_lpr) s.vec /= 2;
+        if (runs) s.vec = F <= 16 ? 1 : (F <= 32 ? 2 : 4);
+        else s.vec = F < 2 ? 1 : (F < 4 ? 2 : 4);
+        if (F > 4 * kWave) s.vec = F % 4 == 0 ? 4 : (F % 2 == 0 ? 2 : 1);
     }
-    const int64_t slots = F / s.vec;
+    const int64_t slots = ceil_div(F, (int64_t)s.vec);
     int lpr = pow2_ceil(slots);
     if (lpr < 4) lpr = 4;
     if (lpr > 64) lpr = 64;
@@ -1152,15 +1181,14 @@ int spmm_typed(const cgnn_csr *A, const void *X, const void *X1, int64_t split, 
     if (mode == MODE_DUAL && A->nnz > 0 && A->val == nullptr)
         return fail(CGNN_EINVAL, "spmm: the two-source product needs stored values");
     if (kernel == CGNN_SPMM_ROW) {
-        Shape s = pick_shape<T>(F, X, Y, X1, nullptr);
+        const Shape s = pick_shape<T>(F, false);
         return launch<T>(KIND_ROW, mode, s, a, A->rows, stream);
     }
     if (A->nnz > 0 && A->rowidx == nullptr) return fail(CGNN_EINVAL, "spmm: nnz schedule needs rowidx");
     const int seg = seg_len(A);
     const int64_t nseg = ceil_div(A->nnz, seg);
-    // the lane layout decides how many runs a workgroup merges (the carries sit at multiples
-    // of 256 bytes in the workspace, so the workspace stands for them in the alignment check)
-    const Shape s = pick_shape<T>(F, X, Y, ws, mode == MODE_DUAL ? X1 : M, 16);
+    // the lane layout decides how many runs a workgroup merges
+    const Shape s = pick_shape<T>(F, true);
     const int runs_per_workgroup = kBlock / s.lpr;
     const CarryLevels levels = carry_levels(nseg, F, sizeof(T), wants_levels(A, seg, runs_per_workgroup));
     if (nseg > 0 && (ws == nullptr || ws_bytes < levels.total)) {

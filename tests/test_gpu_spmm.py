@@ -426,3 +426,23 @@ def test_blocks_without_stored_values(kernel, F):
     assert np.array_equal(fresh[whole], want[whole]) and np.array_equal(acc[whole], want_acc[whole])
     empty = np.diff(vlist) == 0
     assert np.array_equal(acc[empty], out0[empty]) and not fresh[empty].any()
+
+
+@pytest.mark.parametrize("F", [2, 3, 5, 17, 33, 47, 63, 65, 127, 255, 257, 259])
+@pytest.mark.parametrize("kernel", [abi.SPMM_ROW, abi.SPMM_NNZ])
+def test_rows_that_are_no_whole_packs(F, kernel):
+    """The last pack of such a row overlaps the one before it: every element must receive its
+    sum, its carries and (accumulating) its old value exactly once, in rows that one run holds and
+    in rows whose carries pass through the reduction levels."""
+    rng = np.random.default_rng(F)
+    lens = [3, 20_000, 0, 1, 70, 0, 700, 2, 0, 64, 65, 9]
+    cols = 400
+    vlist = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    elist = rng.integers(0, cols, size=int(vlist[-1])).astype(np.int64)
+    value = (rng.standard_normal(len(elist)) * 0.3 / np.sqrt(np.repeat(lens, lens))).astype(np.float32)
+    x = rng.standard_normal((cols, F)).astype(np.float32)
+    out0 = rng.standard_normal((len(lens), F)).astype(np.float32)
+    want = np.zeros((len(lens), F))
+    np.add.at(want, np.repeat(np.arange(len(lens)), lens), value[:, None].astype(np.float64) * x[elist])
+    np.testing.assert_allclose(_run(vlist, elist, value, x, kernel, seg=8), want, rtol=1e-4, atol=2e-5)
+    np.testing.assert_allclose(_run(vlist, elist, value, x, kernel, out0, seg=8), want + out0, rtol=1e-4, atol=2e-5)
