@@ -17,7 +17,7 @@ SPMM_AUTO, SPMM_ROW, SPMM_NNZ = 0, 1, 2
 
 EXPORTS = [
     "cgnn_last_error", "cgnn_version",
-    "cgnn_spmm_schedule", "cgnn_spmm_run_length", "cgnn_spmm_run_starts", "cgnn_spmm_workspace_bytes", "cgnn_spmm", "cgnn_spmm_dual",
+    "cgnn_spmm_schedule", "cgnn_spmm_run_length", "cgnn_spmm_run_starts", "cgnn_spmm_wg_shape", "cgnn_spmm_wg_runs", "cgnn_spmm_workspace_bytes", "cgnn_spmm", "cgnn_spmm_dual",
     "cgnn_spmm_static_scratch_bytes", "cgnn_spmm_static_init", "cgnn_spmm_static",
     "cgnn_csr_prepare_i64", "cgnn_csr_expand_rows", "cgnn_narrow_ids", "cgnn_csr_compose_columns",
     "cgnn_csr_transpose_workspace_bytes", "cgnn_csr_transpose_device",
@@ -42,6 +42,8 @@ class CsrStruct(ctypes.Structure):
         ("cut_rows", ctypes.c_void_p), ("empty_rows", ctypes.c_void_p),
         ("n_cut_rows", ctypes.c_int32), ("n_empty_rows", ctypes.c_int32),
         ("run_start", ctypes.c_void_p),
+        ("wg_runs", ctypes.c_void_p), ("arrivals", ctypes.c_void_p),
+        ("wg_groups", ctypes.c_int32), ("wg_len", ctypes.c_int32),
     ]
 
 

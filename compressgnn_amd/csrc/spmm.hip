@@ -31,6 +31,13 @@
 //     is used it is the only addition to that element), so results are reproducible run
 //     to run.
 //
+//   * workgroup runs -- the nnz schedule without a pass behind it, for blocks that bring a table of their
+//     runs (cgnn_csr.wg_runs).  The entries are dealt to workgroups (wg_len positions each, a row of at
+//     most that many entries never divided) and a workgroup's share to its lane groups, so the pieces of a
+//     row meet in LDS and the row is written there, once.  A row longer than wg_len leaves one piece
+//     per workgroup in memory; the workgroup that finds itself the last to arrive at the row adds the pieces
+//     up, in ascending order, so the sum does not depend on which one that is.
+//
 // Modes: VAL (stored values), UNIT (all values 1), RELU_MASK (unit values, gathered
 // rows zeroed where a second matrix is <= 0), DUAL (columns below `split` gather from
 // X, the others from X1; the two partial sums are kept apart and combined as
@@ -94,7 +101,14 @@ struct SpmmArgs {
     const int32_t *empty_rows;  // and the stored rows without entries
     int32_t n_cut_rows, n_empty_rows;
     const int32_t *run_start;   // nnz schedule: first non-zero of every run, [nseg + 1], or NULL (run_boundary)
+    int32_t *arrivals;          // workgroup runs: per workgroup and feature tile, the pieces stored so far of the row
+                                // that goes on behind it; zero before and after every launch
+    int32_t wg_len;             // workgroup runs: non-zeros per workgroup (run_start is the table of cgnn_csr.wg_runs)
 };
+
+// An entry of the table of workgroup runs is the first non-zero of a run, with this bit set when the row
+// found there began before it.
+constexpr int32_t kRowGoesOn = INT32_MIN;
 
 // carry_row values below zero: the run carries nothing, or its carry was added to that
 // of an earlier run of the same workgroup (the row of Y is the one of that earlier run).
@@ -452,17 +466,191 @@ __device__ __forceinline__ int run_boundary(const SpmmArgs<T> &a, int e) {
     return (a.rowptr[r + 1] - s0 <= a.seg_nnz) ? s0 : e;
 }
 
+// What a workgroup's runs left of the rows that are divided among them, put together: the end of the
+// kernel below for workgroup runs.  Every lane group holds the sum of the row that goes on behind its run
+// (`continues`, in acc) and in `heads` the part of a row that came into its run and ended there; still
+// `open`: one row covers the whole run.  The lane group a row begins in adds the parts of those behind it, in
+// ascending order.  Slots of 2 * workgroups rows of a.carry hold the pieces of the rows that pass from one
+// workgroup to the next: 2 * w for the row that comes into workgroup w, 2 * w + 1 for one that begins in it.
 template <typename T, int VEC, int LPR, int TILES, int MODE>
+__device__ __forceinline__ void join_rows(const SpmmArgs<T> &a, int block, int lane, int grp, const int64_t foff[TILES],
+                                          const Acc<T, VEC, TILES, MODE> &acc, bool continues, bool open, int y_row, int *flags, Pack<T, VEC> (*tails)[kBlock],
+                                          Pack<T, VEC> (*heads)[kBlock]) {
+    constexpr int GPB = kBlock / LPR;
+    constexpr int kContinues = 1, kWholeRun = 2;
+    Pack<T, VEC> part[TILES];
+#pragma unroll
+    for (int t = 0; t < TILES; ++t)
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) part[t].v[i] = acc.total(T(0), t, i);
+    const bool whole_run = continues && open;
+    if (lane == 0) flags[grp] = (continues ? kContinues : 0) | (whole_run ? kWholeRun : 0);
+    if (continues) {
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) tails[t][threadIdx.x] = part[t];
+    }
+    __syncthreads();
+    const int64_t groups = (int64_t)a.blocks * GPB;
+    if (!a.accumulate) {  // rows without entries
+#pragma unroll 1
+        for (int64_t item = (int64_t)block * GPB + grp; item < a.n_empty_rows; item += groups) {
+            T *y = a.Y + (int64_t)out_row(a, a.empty_rows[item]) * a.F;
+            Pack<T, VEC> zero;
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) zero.v[i] = T(0);
+#pragma unroll
+            for (int t = 0; t < TILES; ++t)
+                if (foff[t] >= 0) store_pack_stream<T, VEC>(y + foff[t], zero);
+        }
+    }
+    if (block >= a.blocks) return;  // the grid is rounded up
+    auto add_to = [&](Pack<T, VEC>(&sum)[TILES], const Pack<T, VEC>(*from)[kBlock], int g) {
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            const Pack<T, VEC> o = from[t][g * LPR + lane];
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) sum[t].v[i] = sum[t].v[i] + o.v[i];
+        }
+    };
+    // adds the parts of a row in the lane groups from g on; true if the row ends among them
+    auto follow = [&](Pack<T, VEC>(&sum)[TILES], int g) {
+#pragma unroll 1
+        for (; g < GPB; ++g) {
+            const bool on = (flags[g] & kWholeRun) != 0;
+            add_to(sum, on ? tails : heads, g);
+            if (!on) return true;
+        }
+        return false;
+    };
+    // A piece goes past this XCD's L2, element by element as relaxed atomics of the device's scope,
+    // and so do the reads of the workgroup that adds the pieces up: a release fence instead would write back
+    // and drop the whole L2, for every piece (the web graph's forward vertex stage took 785 us that way).
+    auto store_piece = [&](int64_t slot, const Pack<T, VEC>(&sum)[TILES]) {
+        T *p = a.carry + slot * a.F;
+#pragma unroll
+        for (int t = 0; t < TILES; ++t)
+            if (foff[t] >= 0)
+#pragma unroll
+                for (int i = 0; i < VEC; ++i)
+                    __hip_atomic_store(p + foff[t] + i, sum[t].v[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    auto store_row = [&](int row, const Pack<T, VEC>(&sum)[TILES]) {
+        T *y = a.Y + (int64_t)row * a.F;
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            if (foff[t] < 0) continue;
+            Pack<T, VEC> o = sum[t];
+            if constexpr (MODE == MODE_VAL)
+                if (a.accumulate) {
+                    const Pack<T, VEC> base = load_pack<T, VEC>(y + foff[t]);
+#pragma unroll
+                    for (int i = 0; i < VEC; ++i) o.v[i] = base.v[i] + o.v[i];
+                }
+            store_pack<T, VEC>(y + foff[t], o);
+        }
+    };
+    const bool comes_in = a.run_start[block * GPB] < 0, goes_out = a.run_start[(block + 1) * GPB] < 0;
+    if (grp == 0 && comes_in) {
+        Pack<T, VEC> sum[TILES];
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            const Pack<T, VEC> ended = heads[t][threadIdx.x];
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) sum[t].v[i] = whole_run ? part[t].v[i] : ended.v[i];
+        }
+        if (whole_run) follow(sum, 1);
+        store_piece(2 * (int64_t)block, sum);
+    }
+    if (continues && !whole_run) {
+        if (follow(part, grp + 1)) store_row(y_row, part);
+        else store_piece(2 * (int64_t)block + 1, part);
+    }
+    if (!comes_in && !goes_out) return;
+    // Rows that this workgroup shares with others.
+    __shared__ int arrived_last;
+    const int first_row = a.rowidx[a.run_start[block * GPB] & ~kRowGoesOn];
+    const int last_row = a.rowidx[(a.run_start[(block + 1) * GPB] & ~kRowGoesOn) - 1];
+#pragma unroll 1
+    for (int side = 0; side < 2; ++side) {
+        if (side == 0 ? !comes_in : (!goes_out || (comes_in && first_row == last_row))) continue;
+        const int row = side == 0 ? first_row : last_row;
+        const int w0 = a.rowptr[row] / a.wg_len, w1 = (a.rowptr[row + 1] - 1) / a.wg_len;
+        // every store of the piece has reached memory before the arrival is counted
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            int32_t *count = a.arrivals + (int64_t)blockIdx.y * a.blocks + w0;
+            const bool last = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == w1 - w0;
+            if (last) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // ready for the next launch
+            arrived_last = last;
+        }
+        __syncthreads();
+        if (arrived_last) {
+            // the lane groups take consecutive pieces each, and the first adds their sums up
+            const int n = w1 - w0 + 1;
+            const int j0 = (int)((int64_t)n * grp / GPB), j1 = (int)((int64_t)n * (grp + 1) / GPB);
+            Pack<T, VEC> sum[TILES];
+#pragma unroll
+            for (int t = 0; t < TILES; ++t)
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) sum[t].v[i] = T(0);
+            constexpr int kBatch = 4;
+#pragma unroll 1
+            for (int j = j0; j < j1; j += kBatch) {
+                Pack<T, VEC> piece[kBatch][TILES];
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) {
+                    const int64_t slot = j + u == 0 ? 2 * (int64_t)w0 + 1 : 2 * (int64_t)(w0 + j + u);
+#pragma unroll
+                    for (int t = 0; t < TILES; ++t)
+                        if (j + u < j1 && foff[t] >= 0)
+#pragma unroll
+                            for (int i = 0; i < VEC; ++i)
+                                piece[u][t].v[i] = __hip_atomic_load(a.carry + slot * a.F + foff[t] + i, __ATOMIC_RELAXED,
+                                                                     __HIP_MEMORY_SCOPE_AGENT);
+                }
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u)
+                    if (j + u < j1)
+#pragma unroll
+                        for (int t = 0; t < TILES; ++t)
+                            if (foff[t] >= 0)
+#pragma unroll
+                                for (int i = 0; i < VEC; ++i) sum[t].v[i] = sum[t].v[i] + piece[u][t].v[i];
+            }
+#pragma unroll
+            for (int t = 0; t < TILES; ++t) tails[t][threadIdx.x] = sum[t];
+            __syncthreads();
+            if (grp == 0) {
+#pragma unroll 1
+                for (int g = 1; g < GPB; ++g) add_to(sum, tails, g);
+                store_row(out_row(a, row), sum);
+            }
+        }
+        __syncthreads();
+    }
+}
+
+template <typename T, int VEC, int LPR, int TILES, int MODE, bool WGRUNS>
 __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spmm_nnz_kernel(SpmmArgs<T> a) {
     constexpr int GPB = kBlock / LPR;
     __shared__ int wg_row[GPB];
     __shared__ Pack<T, VEC> wg_carry[TILES][kBlock];
+    __shared__ Pack<T, VEC> wg_head[WGRUNS ? TILES : 1][WGRUNS ? kBlock : 1];
     const int lane = threadIdx.x % LPR, grp = threadIdx.x / LPR;
-    int seg = logical_block(a) * GPB + grp;
+    const int block = logical_block(a);
+    int seg = block * GPB + grp;
     if constexpr (LPR == kWave) seg = __builtin_amdgcn_readfirstlane(seg);
     int e0 = 0, e1 = 0;
+    bool continues = false;    // the last row of the run goes on in the next one
+    bool open = false;         // WGRUNS: the row at hand began before the run
     if (seg < a.nseg) {
-        if (a.run_start != nullptr) {  // one load instead of two dependent ones
+        if constexpr (WGRUNS) {
+            const int r0 = a.run_start[seg], r1 = a.run_start[seg + 1];
+            e0 = r0 & ~kRowGoesOn, e1 = r1 & ~kRowGoesOn;
+            open = r0 < 0, continues = r1 < 0;
+        } else if (a.run_start != nullptr) {  // one load instead of two dependent ones
             e0 = a.run_start[seg];
             e1 = a.run_start[seg + 1];
         } else {
@@ -477,7 +665,26 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
     Acc<T, VEC, TILES, MODE> acc;
     acc.clear();
     int cur = -1;
-    bool continues = false;
+    int cur_out = -1;
+    // A row ends inside the run: it is written, or (the part of it that lies in this run) put aside
+    // for the lane group where the row began.
+    auto finish_row = [&](int y_row) {
+        if constexpr (WGRUNS) {
+            if (open) {
+                open = false;
+#pragma unroll
+                for (int t = 0; t < TILES; ++t)
+#pragma unroll
+                    for (int i = 0; i < VEC; ++i) wg_head[t][threadIdx.x].v[i] = acc.total(T(0), t, i);
+                return;
+            }
+        }
+        write_row<T, VEC, TILES, MODE>(a.Y, a.F, y_row, foff, acc, a.accumulate);
+    };
+    // the names of rows: see below
+    constexpr bool kNamesRowsOfY = !(MODE == MODE_DUAL && VEC * LPR * sizeof(T) >= 512);
+    auto named = [&](int stored_row) { return kNamesRowsOfY ? out_row(a, stored_row) : stored_row; };
+    auto row_of_y = [&](int name) { return kNamesRowsOfY ? name : out_row(a, name); };
     if (active) {
         // A run names its rows by the row of Y they are written to (rowmap[stored row], which the
         // lanes look up beside their entries), so that closing a row inside the run needs no load
@@ -489,16 +696,12 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
         // waves per SIMD): the F = 128 kernel, bound by its traffic either way, took 221 us with it
         // and takes 213 us without (F = 16: 76 -> 62 us with it; the 18.5 M-vertex graph at F = 64:
         // 13.6 -> 13.4 ms; the mask modes, which have no rowmap, lose the wait and nothing else).
-        constexpr bool kNamesRowsOfY = !(MODE == MODE_DUAL && VEC * LPR * sizeof(T) >= 512);
-        auto named = [&](int stored_row) { return kNamesRowsOfY ? out_row(a, stored_row) : stored_row; };
-        auto row_of_y = [&](int name) { return kNamesRowsOfY ? name : out_row(a, name); };
-        int cur_out;
         // looked at when the run is done: the stored row of the last entry (the row a carry belongs
         // to) and the row of the entry behind the run; asked for beside the entries
         int last_row, row_behind;
         if constexpr (!kNamesRowsOfY) {  // the names are the stored rows: the first is read here, the last is at hand at the end
             cur_out = a.rowidx[e0];
-            row_behind = e1 < a.nnz ? a.rowidx[e1] : -1;
+            if constexpr (!WGRUNS) row_behind = e1 < a.nnz ? a.rowidx[e1] : -1;
         }
         if constexpr (LPR >= kUnroll && sizeof(T) == 4) {
             // As in the row schedule: the lanes of the group load one entry each, and the
@@ -519,8 +722,10 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                 if constexpr (kNamesRowsOfY) {
                     // with every batch of entries, so that no load of the run waits for another but
                     // the row numbers for their rows (the same two words each time)
-                    last_row = a.rowidx[e1 - 1];
-                    row_behind = e1 < a.nnz ? a.rowidx[e1] : -1;
+                    if constexpr (!WGRUNS) {
+                        last_row = a.rowidx[e1 - 1];
+                        row_behind = e1 < a.nnz ? a.rowidx[e1] : -1;
+                    }
                     // the run begins with the row of its first entry
                     const int batch_first = __builtin_amdgcn_ds_bpermute(group_lane0, my_o);
                     if (e == e0) cur_out = batch_first;
@@ -567,7 +772,7 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                             if (u0 + u < cnt) {
                                 if (o[u] != cur_out) {
                                     // the row ends inside this run: finish it here
-                                    write_row<T, VEC, TILES, MODE>(a.Y, a.F, row_of_y(cur_out), foff, acc, a.accumulate);
+                                    finish_row(row_of_y(cur_out));
                                     acc.clear();
                                     cur_out = o[u];
                                 }
@@ -582,8 +787,10 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
         } else {
             if constexpr (kNamesRowsOfY) {
                 cur_out = named(a.rowidx[e0]);
-                last_row = a.rowidx[e1 - 1];
-                row_behind = e1 < a.nnz ? a.rowidx[e1] : -1;
+                if constexpr (!WGRUNS) {
+                    last_row = a.rowidx[e1 - 1];
+                    row_behind = e1 < a.nnz ? a.rowidx[e1] : -1;
+                }
             }
             for (int e = e0; e < e1; e += kUnroll) {
                 int o[kUnroll], c[kUnroll];
@@ -610,7 +817,7 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                     if (e + u < e1) {
                         if (o[u] != cur_out) {
                             // the row ends inside this run: finish it here
-                            write_row<T, VEC, TILES, MODE>(a.Y, a.F, row_of_y(cur_out), foff, acc, a.accumulate);
+                            finish_row(row_of_y(cur_out));
                             acc.clear();
                             cur_out = o[u];
                         }
@@ -619,9 +826,17 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                 }
             }
         }
-        cur = kNamesRowsOfY ? last_row : cur_out;
-        continues = row_behind == cur;
-        if (!continues) write_row<T, VEC, TILES, MODE>(a.Y, a.F, row_of_y(cur_out), foff, acc, a.accumulate);
+        if constexpr (!WGRUNS) {
+            cur = kNamesRowsOfY ? last_row : cur_out;
+            continues = row_behind == cur;
+        }
+        if (!continues) finish_row(row_of_y(cur_out));
+    }
+    if constexpr (WGRUNS) {
+        join_rows<T, VEC, LPR, TILES, MODE>(a, block, lane, grp, foff, acc, continues, open,
+                                            continues && active ? row_of_y(cur_out) : -1, wg_row, wg_carry,
+                                            wg_head);
+        return;
     }
     // The carries of one row are added per workgroup: the first of its lane groups that
     // carries the row takes those of the groups behind it, in ascending order.
@@ -983,6 +1198,9 @@ Shape pick_shape(int64_t F, bool runs) {
     return s;
 }
 
+// The layout of the nnz schedule for a feature width.
+Shape shape_of(int64_t F, int dtype) { return dtype == CGNN_F64 ? pick_shape<double>(F, true) : pick_shape<float>(F, true); }
+
 enum { KIND_ROW = 0, KIND_NNZ = 1, KIND_FIXUP = 2, KIND_REDUCE = 3, KIND_FIXUP_ROWS = 4 };
 
 template <typename T, int VEC, int LPR, int TILES>
@@ -1005,16 +1223,20 @@ int launch_shape(int kind, int mode, const SpmmArgs<T> &args, int64_t items, int
                 hipLaunchKernelGGL((spmm_row_kernel<T, VEC, LPR, TILES, MODE_VAL>), grid, block, 0, stream, a);
             break;
         case KIND_NNZ:
-            if (mode == MODE_VAL)
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_VAL>), grid, block, 0, stream, a);
+            if (a.arrivals != nullptr && mode == MODE_DUAL)
+                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_DUAL, true>), grid, block, 0, stream, a);
+            else if (a.arrivals != nullptr)
+                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_VAL, true>), grid, block, 0, stream, a);
+            else if (mode == MODE_VAL)
+                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_VAL, false>), grid, block, 0, stream, a);
             else if (mode == MODE_UNIT)
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_UNIT>), grid, block, 0, stream, a);
+                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_UNIT, false>), grid, block, 0, stream, a);
             else if (mode == MODE_DUAL)
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_DUAL>), grid, block, 0, stream, a);
+                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_DUAL, false>), grid, block, 0, stream, a);
             else if (mode == MODE_SIGN_MASK)
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_SIGN_MASK>), grid, block, 0, stream, a);
+                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_SIGN_MASK, false>), grid, block, 0, stream, a);
             else
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_RELU_MASK>), grid, block, 0, stream, a);
+                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_RELU_MASK, false>), grid, block, 0, stream, a);
             break;
         case KIND_FIXUP: {  // a lane group per carry, and (when not accumulating) a thread per row
             const int64_t for_rows = a.accumulate ? 0 : ceil_div((int64_t)a.rows, kBlock);
@@ -1160,6 +1382,21 @@ CarryLevels carry_levels(int64_t nseg, int64_t F, size_t elt, bool reduce) {
     return L;
 }
 
+// Pieces of the rows that workgroup runs divide among workgroups: two slots per workgroup.
+size_t wg_piece_bytes(int64_t workgroups, int64_t F, size_t elt) { return 2 * (size_t)workgroups * (size_t)F * elt; }
+
+// Non-zeros per lane group of the workgroup runs: as short as fills the card (lane groups resident at
+// once: 7 workgroups per compute unit), since a run is a chain of dependent rounds of gathers and a small
+// product is nothing but the time of its longest chain; not under 8 (two rounds: below that the ends of a
+// run cost more than its entries), not over the block's run length.
+constexpr int64_t kResidentWorkgroups = 256 * 7;
+
+int wg_run_len(const cgnn_csr *A, int groups) {
+    const int64_t fill = ceil_div(ceil_div(A->nnz, kResidentWorkgroups * groups), kUnroll) * kUnroll;
+    const int longest = seg_len(A);
+    return (int)(fill < 8 ? (longest < 8 ? longest : 8) : (fill > longest ? longest : fill));
+}
+
 template <typename T>
 int spmm_typed(const cgnn_csr *A, const void *X, const void *X1, int64_t split, const void *M, void *Y, int64_t F,
                int accumulate, int kernel, int mode, void *ws, size_t ws_bytes, hipStream_t stream) {
@@ -1174,6 +1411,7 @@ int spmm_typed(const cgnn_csr *A, const void *X, const void *X1, int64_t split, 
         a.M = nullptr;
         M = nullptr;
     }
+    const bool may_choose = kernel == CGNN_SPMM_AUTO;
     kernel = resolve_kernel(A, kernel);
     if (masked) kernel = CGNN_SPMM_NNZ;  // masks exist for the nnz schedule only
     // unit values without the multiplications; a product that adds to Y stays with the plain mode, the only one that reads Y
@@ -1185,11 +1423,27 @@ int spmm_typed(const cgnn_csr *A, const void *X, const void *X1, int64_t split, 
         return launch<T>(KIND_ROW, mode, s, a, A->rows, stream);
     }
     if (A->nnz > 0 && A->rowidx == nullptr) return fail(CGNN_EINVAL, "spmm: nnz schedule needs rowidx");
-    const int seg = seg_len(A);
-    const int64_t nseg = ceil_div(A->nnz, seg);
     // the lane layout decides how many runs a workgroup merges
     const Shape s = pick_shape<T>(F, true);
     const int runs_per_workgroup = kBlock / s.lpr;
+    if (may_choose && A->wg_runs != nullptr && A->arrivals != nullptr && A->wg_groups == runs_per_workgroup && A->nnz > 0) {
+        const int64_t workgroups = ceil_div(A->nnz, A->wg_len);
+        const size_t need = wg_piece_bytes(workgroups, F, sizeof(T));
+        if (ws == nullptr || ws_bytes < need) {
+            set_error("spmm: workspace of %zu bytes needed, %zu given", need, ws_bytes);
+            return CGNN_EWORKSPACE;
+        }
+        a.run_start = A->wg_runs;
+        a.arrivals = A->arrivals;
+        a.wg_len = A->wg_len;
+        a.nseg = (int32_t)(workgroups * runs_per_workgroup);
+        a.carry = static_cast<T *>(ws);
+        a.empty_rows = A->empty_rows;
+        a.n_empty_rows = A->n_empty_rows;
+        return launch<T>(KIND_NNZ, mode == MODE_UNIT ? MODE_VAL : mode, s, a, a.nseg, stream);
+    }
+    const int seg = seg_len(A);
+    const int64_t nseg = ceil_div(A->nnz, seg);
     const CarryLevels levels = carry_levels(nseg, F, sizeof(T), wants_levels(A, seg, runs_per_workgroup));
     if (nseg > 0 && (ws == nullptr || ws_bytes < levels.total)) {
         set_error("spmm: workspace of %zu bytes needed, %zu given", levels.total, ws_bytes);
@@ -1259,6 +1513,28 @@ __global__ void run_starts_kernel(const int32_t *__restrict__ rowptr, const int3
     const int r = rowidx[e];
     const int s0 = rowptr[r];
     run_start[s] = (rowptr[r + 1] - s0 <= seg) ? s0 : (int32_t)e;
+}
+
+// The table of workgroup runs (cgnn_csr.wg_runs): entry w * groups + g is where lane group g of workgroup w
+// begins, with kRowGoesOn set when the row there began earlier.
+__global__ void wg_runs_kernel(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ rowidx, int32_t nnz,
+                               int32_t wg_len, int32_t groups, int64_t n, int32_t *__restrict__ runs) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int run_len = wg_len / groups;
+    // e moved back to the start of its row when the row has at most `whole` entries
+    auto begin_of = [&](int64_t e, int whole) -> int32_t {
+        if (e >= nnz) return nnz;
+        const int r = rowidx[e], s0 = rowptr[r];
+        return rowptr[r + 1] - s0 <= whole ? s0 : (int32_t)e;
+    };
+    const int64_t w = i / groups, g = i % groups;
+    const int32_t b0 = begin_of(w * wg_len, wg_len), b1 = begin_of((w + 1) * wg_len, wg_len);
+    const int64_t share = ((int64_t)b1 - b0 + groups - 1) / groups;
+    const int64_t e = b0 + g * share;
+    const int32_t s = g == 0 ? b0 : (e >= b1 ? b1 : begin_of(e, run_len));
+    const bool goes_on = s < nnz && rowptr[rowidx[s]] < s;
+    runs[i] = goes_on ? s | kRowGoesOn : s;
 }
 
 // rowidx[e] = largest r with rowptr[r] <= e (rows without entries are skipped).
@@ -1383,6 +1659,29 @@ extern "C" int cgnn_spmm_schedule(int64_t rows, int64_t nnz, int32_t max_row_nnz
 
 extern "C" int cgnn_spmm_run_length(const cgnn_csr *A) { return A == nullptr ? 0 : seg_len(A); }
 
+extern "C" int cgnn_spmm_wg_shape(const cgnn_csr *A, int64_t F, int dtype, int32_t *groups, int32_t *wg_len,
+                                  int64_t *arrivals) {
+    int rc = check_csr(A, "cgnn_spmm_wg_shape");
+    if (rc != CGNN_OK) return rc;
+    CGNN_REQUIRE(groups && wg_len && arrivals && F >= 1, "cgnn_spmm_wg_shape: bad argument");
+    const Shape s = shape_of(F, dtype);
+    *groups = kBlock / s.lpr;
+    *wg_len = wg_run_len(A, *groups) * *groups;
+    *arrivals = ceil_div(A->nnz, *wg_len) * s.grid_y;
+    return CGNN_OK;
+}
+
+extern "C" int cgnn_spmm_wg_runs(const cgnn_csr *A, int32_t groups, int32_t wg_len, int32_t *runs, cgnn_stream_t stream) {
+    int rc = check_csr(A, "cgnn_spmm_wg_runs");
+    if (rc != CGNN_OK) return rc;
+    CGNN_REQUIRE(runs != nullptr && groups >= 1 && wg_len >= groups && wg_len % groups == 0, "cgnn_spmm_wg_runs: bad argument");
+    CGNN_REQUIRE(A->nnz == 0 || A->rowidx != nullptr, "cgnn_spmm_wg_runs: the block needs rowidx");
+    const int64_t n = ceil_div(A->nnz, wg_len) * groups + 1;
+    hipLaunchKernelGGL(wg_runs_kernel, dim3((unsigned)ceil_div(n, kBlock)), dim3(kBlock), 0, stream, A->rowptr, A->rowidx,
+                       (int32_t)A->nnz, wg_len, groups, n, runs);
+    return check_launch("spmm_wg_runs");
+}
+
 extern "C" size_t cgnn_spmm_static_scratch_bytes(void) { return kStaticScratchBytes; }
 
 extern "C" int cgnn_spmm_static_init(void) {
@@ -1417,9 +1716,11 @@ extern "C" int cgnn_spmm_static(const cgnn_csr *A, int dtype, const void *X, voi
 extern "C" size_t cgnn_spmm_workspace_bytes(const cgnn_csr *A, int64_t F, int dtype, int kernel) {
     if (A == nullptr || A->nnz <= 0 || F <= 0) return 0;
     if (resolve_kernel(A, kernel) == CGNN_SPMM_ROW) return 0;
+    if (kernel == CGNN_SPMM_AUTO && A->wg_runs != nullptr && A->arrivals != nullptr &&
+        A->wg_groups == kBlock / shape_of(F, dtype).lpr)
+        return wg_piece_bytes(ceil_div(A->nnz, A->wg_len), F, dtype == CGNN_F64 ? 8 : 4);
     const int seg = seg_len(A);
-    // an upper bound: the lane layout (which depends on the pointers' alignment) can only
-    // remove reduction levels
+    // an upper bound: the lane layout can only remove reduction levels
     return carry_levels(ceil_div(A->nnz, seg), F, dtype == CGNN_F64 ? 8 : 4, wants_levels(A, seg, 1)).total;
 }
 

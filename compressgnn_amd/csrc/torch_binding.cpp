@@ -10,6 +10,7 @@
 #include <hip/hip_runtime_api.h>
 #include <torch/extension.h>
 
+#include <algorithm>
 #include <deque>
 #include <memory>
 #include <mutex>
@@ -52,10 +53,16 @@ void require_gpu(const Tensor &t, const char *name) {
 // gives each stream a plan (or a block) of its own.
 struct Scratch {
     Tensor buf;
-    Tensor get(size_t bytes, const Tensor &like) {
+    Tensor arrivals;  // counters that every product leaves at zero
+    const Tensor &get(size_t bytes, const Tensor &like) {
         if (!buf.defined() || (size_t)buf.numel() < bytes || buf.device() != like.device())
             buf = torch::empty({(int64_t)std::max<size_t>(bytes, 1)}, like.options().dtype(torch::kUInt8));
         return buf;
+    }
+    int32_t *counters(int64_t n, const Tensor &like) {
+        if (!arrivals.defined() || arrivals.numel() < n || arrivals.device() != like.device())
+            arrivals = torch::zeros({std::max<int64_t>(n, 1)}, like.options().dtype(torch::kInt32));
+        return arrivals.data_ptr<int32_t>();
     }
 };
 
@@ -71,6 +78,15 @@ struct DeviceCsr {
     Tensor cut_rows, empty_rows;  // the rows the runs of the nnz schedule cut / the rows without entries
     Tensor run_start;  // nnz schedule: where every run begins (made with rowidx)
     std::shared_ptr<Scratch> scratch = std::make_shared<Scratch>();
+    // Whether AUTO may take workgroup runs, which divide long rows at other places than the nnz schedule
+    // of the C ABI does (a plan's blocks do; a block on its own keeps the sums of the C ABI unless asked).
+    bool workgroup_runs = false;
+    // their tables made so far: one per lane layout, so a handful at most
+    struct WgRuns {
+        int32_t groups, len;
+        Tensor table;
+    };
+    std::vector<WgRuns> wg_runs;
 
     cgnn_csr view() const {
         cgnn_csr a{};
@@ -133,11 +149,29 @@ struct DeviceCsr {
         run_start = starts;
     }
 
-    Tensor workspace(int64_t F, int dtype, int kernel, size_t *bytes) {
+    // The block as a product of width F reads it, and the scratch for that product.
+    cgnn_csr prepare(int64_t F, int dtype, int kernel, void **ws, size_t *bytes) {
         ensure_rowidx(kernel);
         cgnn_csr a = view();
+        if (workgroup_runs && kernel == CGNN_SPMM_AUTO && nnz > 0 && empty_rows.defined() &&
+            cgnn_spmm_schedule(rows, nnz, max_row_nnz, kernel) == CGNN_SPMM_NNZ) {
+            int64_t arrivals = 0;
+            ok(cgnn_spmm_wg_shape(&a, F, dtype, &a.wg_groups, &a.wg_len, &arrivals), "spmm_wg_shape");
+            auto found = std::find_if(wg_runs.begin(), wg_runs.end(), [&](const WgRuns &r) {
+                return r.groups == a.wg_groups && r.len == a.wg_len;
+            });
+            if (found == wg_runs.end()) {
+                Tensor table = torch::empty({(nnz + a.wg_len - 1) / a.wg_len * a.wg_groups + 1}, rowptr.options());
+                ok(cgnn_spmm_wg_runs(&a, a.wg_groups, a.wg_len, table.data_ptr<int32_t>(), current_stream(rowptr)),
+                   "spmm_wg_runs");
+                found = wg_runs.insert(wg_runs.end(), WgRuns{a.wg_groups, a.wg_len, table});
+            }
+            a.wg_runs = found->table.data_ptr<int32_t>();
+            a.arrivals = scratch->counters(arrivals, rowptr);
+        }
         *bytes = cgnn_spmm_workspace_bytes(&a, F, dtype, kernel);
-        return scratch->get(*bytes, rowptr);
+        *ws = *bytes ? scratch->get(*bytes, rowptr).data_ptr() : nullptr;
+        return a;
     }
 };
 
@@ -237,9 +271,9 @@ Tensor block_spmm(DeviceCsr &A, const Tensor &mat, c10::optional<Tensor> optiona
     }
     if (A.rows == 0 || F == 0) return out;
     size_t bytes = 0;
-    Tensor ws = A.workspace(F, dtype, kernel, &bytes);
-    cgnn_csr a = A.view();
-    ok(cgnn_spmm(&a, dtype, mat.data_ptr(), out.data_ptr(), F, accumulate, kernel, ws.data_ptr(), bytes,
+    void *ws = nullptr;
+    cgnn_csr a = A.prepare(F, dtype, kernel, &ws, &bytes);
+    ok(cgnn_spmm(&a, dtype, mat.data_ptr(), out.data_ptr(), F, accumulate, kernel, ws, bytes,
                  current_stream(mat)),
        "spmm");
     return out;
@@ -345,7 +379,9 @@ struct PropagationPlan {
     std::deque<Composed> composed;
 
     void adopt(const std::shared_ptr<DeviceCsr> &block) {
-        if (block) block->scratch = scratch;
+        if (!block) return;
+        block->scratch = scratch;
+        block->workgroup_runs = true;
     }
     bool fused() const { return fuse_final && vertex_stage && vertex_stage_t; }
     void require_split_blocks() const {
@@ -373,12 +409,12 @@ Tensor final_stage(PropagationPlan &p, const std::string &prefix, DeviceCsr *mer
         if (out.numel() == 0) return out;
         const int dtype = dtype_code(x);
         size_t bytes = 0;
-        Tensor ws = merged->workspace(F, dtype, p.kernel, &bytes);
+        void *ws = nullptr;
+        cgnn_csr a = merged->prepare(F, dtype, p.kernel, &ws, &bytes);
         hipStream_t stream = reinterpret_cast<hipStream_t>(current_stream(x));
         const int id = p.timer.open(prefix + "final", stream);
-        cgnn_csr a = merged->view();
-        ok(cgnn_spmm_dual(&a, p.V, dtype, x.data_ptr(), rule_x.data_ptr(), out.data_ptr(), F, p.kernel,
-                          ws.data_ptr(), bytes, current_stream(x)),
+        ok(cgnn_spmm_dual(&a, p.V, dtype, x.data_ptr(), rule_x.data_ptr(), out.data_ptr(), F, p.kernel, ws, bytes,
+                          current_stream(x)),
            "spmm_dual");
         p.timer.close(id, stream);
         return out;
@@ -468,11 +504,11 @@ Tensor propagate_forward_gathered(PropagationPlan &p, Tensor reps, Tensor index)
     if (out.numel() == 0) return out;
     const int dtype = dtype_code(reps);
     size_t bytes = 0;
-    Tensor ws = stage->workspace(F, dtype, p.kernel, &bytes);
+    void *ws = nullptr;
+    cgnn_csr a = stage->prepare(F, dtype, p.kernel, &ws, &bytes);
     hipStream_t stream = reinterpret_cast<hipStream_t>(current_stream(reps));
     const int id = p.timer.open("fwd.final", stream);
-    cgnn_csr a = stage->view();
-    ok(cgnn_spmm_dual(&a, p.V, dtype, reps.data_ptr(), rule_out.data_ptr(), out.data_ptr(), F, p.kernel, ws.data_ptr(), bytes,
+    ok(cgnn_spmm_dual(&a, p.V, dtype, reps.data_ptr(), rule_out.data_ptr(), out.data_ptr(), F, p.kernel, ws, bytes,
                       current_stream(reps)),
        "spmm_dual");
     p.timer.close(id, stream);
@@ -1158,9 +1194,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         .def_property("seg_nnz", [](DeviceCsr &self) { return self.seg_nnz; },
                       [](DeviceCsr &self, int32_t seg) {
                           self.seg_nnz = seg;
-                          self.run_start = Tensor();  // made again by the next product
+                          self.run_start = Tensor();  // made again by the next product, like the workgroup runs
+                          self.wg_runs.clear();
                           if (self.cut_rows.defined()) self.list_rows();  // the lists belong to a run length
                       })
+        .def_readwrite("workgroup_runs", &DeviceCsr::workgroup_runs)
         .def_readonly("cut_rows", &DeviceCsr::cut_rows)
         .def_readonly("run_start", &DeviceCsr::run_start)
         .def_readonly("empty_rows", &DeviceCsr::empty_rows)

@@ -83,6 +83,20 @@ typedef struct cgnn_csr {
      * row is never cut: the run begins with it), else e.  Must be exact when given (not checked).
      * Results are unchanged. */
     const int32_t *run_start;
+    /* NNZ schedule under AUTO, optional (NULL = the runs above and a pass that completes the rows they cut):
+     * the runs dealt by workgroup, so that a row is completed where its pieces meet.  Positions are
+     * dealt to ceil(nnz / wg_len) workgroups: workgroup w begins at w * wg_len, or at the start of the row
+     * found there when that row has at most wg_len entries.  Its wg_groups lane groups begin at equal
+     * shares of what the workgroup holds, each moved back to the start of its row when that row has at most
+     * wg_len / wg_groups entries.  wg_runs[w * wg_groups + g] holds these beginnings
+     * ([ceil(nnz / wg_len) * wg_groups + 1]), with the top bit set when the row found there begins
+     * earlier; filled by cgnn_spmm_wg_runs for the shape that cgnn_spmm_wg_shape names (a table of another
+     * shape is not used).  empty_rows must be given with it.  arrivals: counters, as many as
+     * cgnn_spmm_wg_shape says, that are zero before the first call and zero again after every call; calls
+     * that share them must not overlap in time. */
+    const int32_t *wg_runs;
+    int32_t *arrivals;
+    int32_t wg_groups, wg_len;
 } cgnn_csr;
 
 const char *cgnn_last_error(void);
@@ -102,6 +116,12 @@ int cgnn_spmm_run_length(const cgnn_csr *A);
 /* Fills run_start[ceil(nnz / K) + 1] (K = cgnn_spmm_run_length(A)) for a block that has rowidx: the
  * optional table of cgnn_csr.run_start, as defined there.  No counterpart in the reference. */
 int cgnn_spmm_run_starts(const cgnn_csr *A, int32_t *run_start, cgnn_stream_t stream);
+
+/* The workgroup runs that AUTO takes for products of width F with this block, if it resolves to the NNZ
+ * schedule: lane groups per workgroup, non-zeros per workgroup and the number of arrival counters.
+ * cgnn_spmm_wg_runs fills the table (cgnn_csr.wg_runs) of such a shape; the block needs rowidx. */
+int cgnn_spmm_wg_shape(const cgnn_csr *A, int64_t F, int dtype, int32_t *groups, int32_t *wg_len, int64_t *arrivals);
+int cgnn_spmm_wg_runs(const cgnn_csr *A, int32_t groups, int32_t wg_len, int32_t *runs, cgnn_stream_t stream);
 
 /* Bytes of scratch cgnn_spmm needs for this block, feature width and schedule
  * (the carry-out rows of the NNZ schedule).  0 for the ROW schedule. */

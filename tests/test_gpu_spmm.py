@@ -446,3 +446,47 @@ def test_rows_that_are_no_whole_packs(F, kernel):
     np.add.at(want, np.repeat(np.arange(len(lens)), lens), value[:, None].astype(np.float64) * x[elist])
     np.testing.assert_allclose(_run(vlist, elist, value, x, kernel, seg=8), want, rtol=1e-4, atol=2e-5)
     np.testing.assert_allclose(_run(vlist, elist, value, x, kernel, out0, seg=8), want + out0, rtol=1e-4, atol=2e-5)
+
+
+@pytest.mark.parametrize("F", [1, 16, 47, 64, 128, 256, 600, 1100])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_workgroup_runs(F, accumulate):
+    """Products of a block with workgroup runs (what the blocks of a plan take): rows that end where a run or a workgroup's
+    share ends (or one entry beside it), rows over many workgroups, empty rows at both ends; against float64
+    and, for rows that no run divides, the bits of the sequential sum.  The first product runs over NaN, so
+    that a piece read without having been written shows; a second one checks that the arrival counters are
+    back at zero."""
+    import ctypes
+    import compressgnn_runtime as rt
+    rng = np.random.default_rng(F)
+    t = lambda a: torch.from_numpy(a).to(DEV)
+    dev = torch.device(DEV)
+    cols, seg = 300, 32
+    # the shape for a block of about this size
+    probe = abi.DeviceCsr.from_host(1, 1, np.array([0, 6000]), np.zeros(6000, np.int64), None, DEV, seg_nnz=seg)
+    groups, wg_len, arrivals = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int64()
+    abi.check(abi.lib().cgnn_spmm_wg_shape(ctypes.byref(probe.struct()), abi.i64(F), abi.F32, ctypes.byref(groups),
+                                           ctypes.byref(wg_len), ctypes.byref(arrivals)))
+    W, K = wg_len.value, wg_len.value // groups.value
+    lens = [0, 3, W - 3, W, W + 1, 2 * W, 0, K, K + 1, K - 1, 5 * W + 1, 1, 2, W - 1, 17, 0, 9 * W, 4 * K, 0]
+    lens += list(rng.integers(0, 2 * K, 40)) + [3 * W + 5, 0]
+    vlist = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    elist = rng.integers(0, cols, size=int(vlist[-1])).astype(np.int64)
+    value = (rng.standard_normal(len(elist)) * 0.3 / np.sqrt(np.repeat(np.maximum(lens, 1), lens))).astype(np.float32)
+    x = rng.standard_normal((cols, F)).astype(np.float32)
+    out0 = rng.standard_normal((len(lens), F)).astype(np.float32) if accumulate else np.zeros((len(lens), F), np.float32)
+    want = out0.astype(np.float64)
+    np.add.at(want, np.repeat(np.arange(len(lens)), lens), value[:, None].astype(np.float64) * x[elist])
+    sequential = oracle.spmm(vlist, elist, value, x, out0.copy())
+    whole = np.array(lens) <= K
+    for dtype, tol in ((np.float32, 2e-5), (np.float64, 1e-13)):
+        A = rt.DeviceCsr(t(vlist), t(elist), t(value.astype(dtype)), len(lens), cols, dev, seg)
+        A.workgroup_runs = True
+        X = t(x.astype(dtype))
+        product = lambda X: A.spmm(X, t(out0.astype(dtype)) if accumulate else None)
+        product(torch.full_like(X, float("nan")))
+        got = product(X).cpu().numpy()
+        np.testing.assert_allclose(got, want, rtol=tol, atol=tol)
+        assert np.array_equal(got, product(X).cpu().numpy())
+        if dtype == np.float32:
+            assert np.array_equal(got[whole], sequential[whole])
