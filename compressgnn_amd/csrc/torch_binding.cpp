@@ -8,6 +8,8 @@
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <hip/hip_runtime_api.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
 #include <torch/extension.h>
 
 #include <algorithm>
@@ -526,6 +528,35 @@ Tensor propagate_backward(PropagationPlan &p, Tensor grad) {
     for (size_t i = p.r2r_t.size(); i-- > 0;)
         rule_g = timed_spmm(p, "bwd.level" + std::to_string(i), *p.r2r_t[i], rule_g, rule_g);
     return final_stage(p, "bwd.", p.vertex_stage_t.get(), p.r2v_t, rule_g, p.v2v_t, grad);
+}
+
+// One propagation as a step of autograd.  The node is native, so a training step takes neither the
+// interpreter nor its lock on the way back (the engine's thread and the caller's would pass the lock to each
+// other): forward and gradient over 2,708 vertices, @HOST@.
+struct PropagateBackward : torch::autograd::Node {
+    std::shared_ptr<PropagationPlan> plan;
+    torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
+        if (!grads[0].defined()) return {Tensor()};
+        at::NoGradGuard no_grad;
+        return {propagate_backward(*plan, grads[0])};
+    }
+    std::string name() const override { return "PropagateBackward"; }
+};
+
+Tensor propagate(const std::shared_ptr<PropagationPlan> &plan, const Tensor &x) {
+    const bool differentiable = at::GradMode::is_enabled() && x.requires_grad();
+    Tensor out;
+    {
+        at::NoGradGuard no_grad;
+        out = propagate_forward(*plan, x);
+    }
+    if (differentiable) {
+        std::shared_ptr<PropagateBackward> node(new PropagateBackward(), torch::autograd::deleteNode);
+        node->plan = plan;
+        node->set_next_edges(torch::autograd::collect_next_edges(x));
+        torch::autograd::set_history(out, node);
+    }
+    return out;
 }
 
 // ---------------------------------------------------- transformation compression ----
@@ -1177,6 +1208,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("signs"), py::arg("groups"), py::arg("members") = py::none());
     m.def("csr_transpose", &csr_transpose, "CSR -> CSC of an int64 block on the GPU, SparseTensor.csc() order",
           py::arg("rowptr"), py::arg("col"), py::arg("value"), py::arg("cols"));
+    m.def("propagate", &propagate, "plan.forward(x) with plan.backward as its gradient", py::arg("plan"), py::arg("x"));
     m.def("version", []() { return std::string(cgnn_version()); });
     py::class_<DeviceCsr, std::shared_ptr<DeviceCsr>>(m, "DeviceCsr")
         .def(py::init([](Tensor rowptr, Tensor col, c10::optional<Tensor> value, int64_t rows, int64_t cols,
