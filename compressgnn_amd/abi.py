@@ -23,7 +23,8 @@ EXPORTS = [
     "cgnn_csr_transpose_workspace_bytes", "cgnn_csr_transpose_device",
     "cgnn_compress_batch_workspace_bytes", "cgnn_compress_csr_batch_device",
     "cgnn_lsh_scan_workspace_bytes", "cgnn_lsh_hash", "cgnn_lsh_scan", "cgnn_lsh_finish",
-    "cgnn_lsh_group_workspace_bytes", "cgnn_lsh_group",
+    "cgnn_lsh_group_workspace_bytes", "cgnn_lsh_group", "cgnn_lsh_group_small_rows", "cgnn_cluster_sums_workspace_bytes",
+    "cgnn_cluster_sums", "cgnn_cluster_divide", "cgnn_column_sums_workspace_bytes", "cgnn_column_sums",
     "cgnn_cluster_members_workspace_bytes", "cgnn_cluster_members",
     "cgnn_cluster_mean_workspace_bytes", "cgnn_cluster_mean", "cgnn_cluster_mean_backward",
     "cgnn_reconstruct", "cgnn_reconstruct_backward", "cgnn_sign_words", "cgnn_reconstruct_signs",
@@ -62,8 +63,10 @@ def lib():
         for name in ("cgnn_spmm_workspace_bytes", "cgnn_spmm_static_scratch_bytes", "cgnn_lsh_scan_workspace_bytes", "cgnn_lsh_group_workspace_bytes",
                      "cgnn_cluster_members_workspace_bytes", "cgnn_cluster_mean_workspace_bytes",
                      "cgnn_csr_transpose_workspace_bytes", "cgnn_compress_batch_workspace_bytes",
+                     "cgnn_cluster_sums_workspace_bytes", "cgnn_column_sums_workspace_bytes",
                      "cgnn_exclusive_sum_workspace_bytes", "cgnn_sample_relabel_workspace_bytes"):
             getattr(L, name).restype = ctypes.c_size_t
+        L.cgnn_lsh_group_small_rows.restype = ctypes.c_int64
         _lib = L
     return _lib
 

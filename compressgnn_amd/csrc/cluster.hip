@@ -2,6 +2,7 @@
 // histogram, occupancy scan, id remap, row gathers (mean backward, reconstruct with
 // fused bias + ReLU).  The per-cluster sums (mean forward, reconstruct backward) run
 // on the member lists through the nnz-schedule SpMM in spmm.hip.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -10,6 +11,10 @@ namespace cgnn {
 
 int spmm_members(const cgnn_csr *A, int dtype, const void *X, const void *M, void *Y, int64_t F,
                  int mask, void *ws, size_t ws_bytes, hipStream_t stream);
+
+int spmm_member_runs(const cgnn_csr *A, int dtype, const void *X, const void *M, void *Y, int64_t F, int mask, bool mean,
+                     bool first_row_empty, int32_t *arrivals, void *ws, size_t ws_bytes, hipStream_t stream);
+size_t spmm_member_runs_bytes(const cgnn_csr *A, int64_t F, int dtype, int64_t *arrivals);
 
 namespace {
 
@@ -987,6 +992,85 @@ __global__ __launch_bounds__(kBlock) void divide_counts_kernel(T *reps, const in
     }
 }
 
+// out[f] = sum over the rows of X[., f].  A workgroup sums a stretch of rows of one slab of features
+// (kSumLanes lanes across it, the lane groups walking the rows), the last workgroup of a slab to arrive
+// adds the stretches up in ascending order; one launch.  torch's sum over the rows took 20 us for 249 x 16 and
+// 33 us for 45,000 x 256 (46 MB); this takes 3.4 us and 14.6 us.
+constexpr int kSumLanes = 16;
+constexpr int kSumStretches = 64;   // at most this many workgroups per slab: the last one adds up four stretches per lane group
+constexpr int kSumRows = 64;        // at least this many rows per workgroup
+constexpr int kSumUnroll = 8;
+
+template <typename T, int VEC>
+__global__ __launch_bounds__(kBlock) void column_sums_kernel(const T *__restrict__ X, int64_t rows, int64_t F,
+                                                             int64_t stretch, T *pieces, int32_t *arrivals,
+                                                             T *__restrict__ out) {
+    constexpr int GPB = kBlock / kSumLanes;
+    __shared__ LPack<T, VEC> part[kBlock];
+    __shared__ bool arrived_last;
+    const int lane = threadIdx.x % kSumLanes, grp = threadIdx.x / kSumLanes;
+    const int64_t f = ((int64_t)blockIdx.y * kSumLanes + lane) * VEC;
+    const bool on = f < F;
+    const int64_t r1 = min(rows, (int64_t)(blockIdx.x + 1) * stretch);
+    LPack<T, VEC> sum;
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) sum.v[i] = T(0);
+    for (int64_t r = (int64_t)blockIdx.x * stretch + grp; r < r1; r += (int64_t)kSumUnroll * GPB) {
+        LPack<T, VEC> x[kSumUnroll];
+#pragma unroll
+        for (int u = 0; u < kSumUnroll; ++u) {
+            const bool live = on && r + (int64_t)u * GPB < r1;
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) x[u].v[i] = T(0);
+            if (live) x[u] = *reinterpret_cast<const LPack<T, VEC> *>(X + (r + (int64_t)u * GPB) * F + f);
+        }
+#pragma unroll
+        for (int u = 0; u < kSumUnroll; ++u)
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) sum.v[i] = sum.v[i] + x[u].v[i];
+    }
+    auto add_groups = [&]() {  // the first lane group's sum becomes the workgroup's
+        part[threadIdx.x] = sum;
+        __syncthreads();
+        if (grp == 0)
+#pragma unroll
+            for (int g = 1; g < GPB; ++g)
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) sum.v[i] = sum.v[i] + part[g * kSumLanes + lane].v[i];
+    };
+    add_groups();
+    if (gridDim.x > 1) {
+        // device-scope relaxed accesses and a count, as the rows of workgroup runs are completed (spmm.hip)
+        if (grp == 0 && on)
+#pragma unroll
+            for (int i = 0; i < VEC; ++i)
+                __hip_atomic_store(pieces + (int64_t)blockIdx.x * F + f + i, sum.v[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const bool last = __hip_atomic_fetch_add(arrivals + blockIdx.y, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                              (int)gridDim.x - 1;
+            if (last) __hip_atomic_store(arrivals + blockIdx.y, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            arrived_last = last;
+        }
+        __syncthreads();
+        if (!arrived_last) return;
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) sum.v[i] = T(0);
+        const int share = ((int)gridDim.x + GPB - 1) / GPB;
+        if (on)
+            for (int k = grp * share; k < min((grp + 1) * share, (int)gridDim.x); ++k)
+#pragma unroll
+                for (int i = 0; i < VEC; ++i)
+                    sum.v[i] = sum.v[i] + __hip_atomic_load(pieces + (int64_t)k * F + f + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        add_groups();
+    }
+    if (grp == 0 && on)
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) out[f + i] = sum.v[i];
+}
+
 __global__ void copy16_kernel(const uint4 *__restrict__ src, uint4 *__restrict__ dst, size_t n) {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
          i += (size_t)gridDim.x * blockDim.x)
@@ -1162,6 +1246,75 @@ extern "C" int cgnn_cluster_mean(int64_t N, int64_t F, int64_t groups, int64_t m
     if (rc != CGNN_OK) return rc;
     if (dtype == CGNN_F32) return divide_counts<float>(reps, counts, groups, F, stream);
     return divide_counts<double>(reps, counts, groups, F, stream);
+}
+
+extern "C" size_t cgnn_cluster_sums_workspace_bytes(int64_t N, int64_t F, int64_t groups, int dtype, int64_t *arrivals) {
+    if (arrivals) *arrivals = 0;
+    if (N <= 0 || F <= 0 || groups <= 0) return 0;
+    cgnn_csr A = members_csr(N, groups, nullptr, nullptr, nullptr);
+    int64_t n = 0;
+    const size_t bytes = spmm_member_runs_bytes(&A, F, dtype, &n);
+    if (arrivals) *arrivals = n;
+    return bytes;
+}
+
+extern "C" int cgnn_cluster_sums(int64_t N, int64_t F, int64_t groups, int dtype, const void *X, int mask, const void *M,
+                                 const int32_t *offsets, const int32_t *perm, const int32_t *sorted_id, int mean,
+                                 int first_group_empty, void *sums, void *workspace, size_t workspace_bytes,
+                                 int32_t *arrivals, cgnn_stream_t stream) {
+    CGNN_REQUIRE(N > 0 && F > 0 && groups > 0 && N < INT32_MAX - 65536, "cgnn_cluster_sums: bad size");
+    CGNN_REQUIRE(dtype == CGNN_F32 || dtype == CGNN_F64, "cgnn_cluster_sums: dtype must be f32 or f64");
+    CGNN_REQUIRE(mask >= 0 && mask <= 2 && !(mask && mean), "cgnn_cluster_sums: a mask (0, 1 or 2) or means, not both");
+    CGNN_REQUIRE(X && offsets && perm && sorted_id && sums && arrivals && (mask == 0 || M), "cgnn_cluster_sums: null array");
+    cgnn_csr A = members_csr(N, groups, offsets, perm, sorted_id);
+    return spmm_member_runs(&A, dtype, X, M, sums, F, mask, mean != 0, first_group_empty != 0, arrivals, workspace,
+                            workspace_bytes, stream);
+}
+
+extern "C" int cgnn_cluster_divide(int64_t F, int64_t groups, int dtype, const int32_t *counts, void *sums,
+                                   cgnn_stream_t stream) {
+    CGNN_REQUIRE(F >= 0 && groups >= 0, "cgnn_cluster_divide: bad size");
+    CGNN_REQUIRE(dtype == CGNN_F32 || dtype == CGNN_F64, "cgnn_cluster_divide: dtype must be f32 or f64");
+    if (F == 0 || groups == 0) return CGNN_OK;
+    CGNN_REQUIRE(counts && sums, "cgnn_cluster_divide: null array");
+    if (dtype == CGNN_F32) return divide_counts<float>(sums, counts, groups, F, stream);
+    return divide_counts<double>(sums, counts, groups, F, stream);
+}
+
+// Rows per workgroup of column_sums_kernel.
+static int64_t sum_stretch(int64_t rows) {
+    const int64_t even = ceil_div(rows, kSumStretches);
+    return even < kSumRows ? kSumRows : even;
+}
+
+extern "C" size_t cgnn_column_sums_workspace_bytes(int64_t rows, int64_t F, int dtype, int64_t *arrivals) {
+    if (arrivals) *arrivals = 0;
+    if (rows <= 0 || F <= 0) return 0;
+    if (arrivals) *arrivals = ceil_div(F, kSumLanes);
+    return (size_t)ceil_div(rows, sum_stretch(rows)) * (size_t)F * (dtype == CGNN_F64 ? 8 : 4);
+}
+
+extern "C" int cgnn_column_sums(int64_t rows, int64_t F, int dtype, const void *X, void *out, void *workspace,
+                                size_t workspace_bytes, int32_t *arrivals, cgnn_stream_t stream) {
+    CGNN_REQUIRE(rows > 0 && F > 0, "cgnn_column_sums: bad size");
+    CGNN_REQUIRE(dtype == CGNN_F32 || dtype == CGNN_F64, "cgnn_column_sums: dtype must be f32 or f64");
+    CGNN_REQUIRE(X && out && arrivals, "cgnn_column_sums: null array");
+    if (workspace == nullptr || workspace_bytes < cgnn_column_sums_workspace_bytes(rows, F, dtype, nullptr))
+        return fail(CGNN_EWORKSPACE, "cgnn_column_sums: workspace too small");
+    const int64_t stretch = sum_stretch(rows);
+    // packs of four where the slab they make is filled and the rows are whole packs
+    const bool wide = dtype == CGNN_F32 && F % 4 == 0 && F > kSumLanes && reinterpret_cast<uintptr_t>(X) % 16 == 0;
+    const dim3 grid((unsigned)ceil_div(rows, stretch), (unsigned)ceil_div(F, kSumLanes * (wide ? 4 : 1)));
+    if (wide)
+        hipLaunchKernelGGL((column_sums_kernel<float, 4>), grid, dim3(kBlock), 0, stream, static_cast<const float *>(X), rows,
+                           F, stretch, static_cast<float *>(workspace), arrivals, static_cast<float *>(out));
+    else if (dtype == CGNN_F32)
+        hipLaunchKernelGGL((column_sums_kernel<float, 1>), grid, dim3(kBlock), 0, stream, static_cast<const float *>(X), rows,
+                           F, stretch, static_cast<float *>(workspace), arrivals, static_cast<float *>(out));
+    else
+        hipLaunchKernelGGL((column_sums_kernel<double, 1>), grid, dim3(kBlock), 0, stream, static_cast<const double *>(X),
+                           rows, F, stretch, static_cast<double *>(workspace), arrivals, static_cast<double *>(out));
+    return check_launch("column_sums");
 }
 
 template <typename T, int OP>

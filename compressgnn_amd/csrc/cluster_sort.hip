@@ -506,6 +506,148 @@ __global__ void group_counts_kernel(const int32_t *__restrict__ offsets, int32_t
     }
 }
 
+// The whole grouping of a small assignment in one workgroup: the sort, the ids, the member lists, the sizes
+// and the summary (which may lie in pinned host memory: plain stores).  The passes above are eight
+// launches of 2 to 9 us each whatever they hold; this one takes 11 us for 2,708 rows and 8 bits.  Up to
+// kSmallRows rows: keys and row numbers of two passes then fit the LDS of a compute unit, and a key is ranked
+// eight steps into its wave's share.
+constexpr int kSmallRows = 8192;
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallWaves = kSmallThreads / kWave;
+constexpr int kSmallItems = kSmallRows / kSmallThreads;
+
+__global__ __launch_bounds__(kSmallThreads) void group_small_kernel(const int32_t *__restrict__ codes, int N, int passes, int code_mask,
+                                                                    int64_t *__restrict__ ids, int32_t *__restrict__ offsets,
+                                                                    int32_t *__restrict__ perm, int32_t *__restrict__ sorted_id,
+                                                                    int32_t *__restrict__ counts, int32_t *__restrict__ summary) {
+    __shared__ int32_t keys[2][kSmallRows];
+    __shared__ uint16_t rows[2][kSmallRows];
+    __shared__ int wave_count[kSmallWaves][kDigits];
+    __shared__ int digit_start[kDigits];
+    __shared__ int tmp[kSmallWaves];
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const int per_wave = ((N + kSmallWaves - 1) / kSmallWaves + kWave - 1) / kWave * kWave;  // a multiple of 64, at most 512
+    for (int i = threadIdx.x; i < N; i += kSmallThreads) {
+        keys[0][i] = codes[i] & code_mask;
+        rows[0][i] = (uint16_t)i;
+    }
+    int from = 0;
+    for (int p = 0; p < passes; ++p) {
+        const int shift = p * kDigitBits;
+        for (int i = threadIdx.x; i < kSmallWaves * kDigits; i += kSmallThreads) wave_count[i / kDigits][i % kDigits] = 0;
+        __syncthreads();
+        int key[kSmallItems], rank[kSmallItems];
+        const int base = wave * per_wave;
+#pragma unroll
+        for (int it = 0; it < kSmallItems; ++it) {
+            const int i = base + it * kWave + lane;
+            const bool live = it * kWave < per_wave && i < N;
+            key[it] = live ? keys[from][i] : 0;
+            const int d = digit_of(key[it], shift);
+            const unsigned long long peers = same_digit(d, __ballot(live));
+            rank[it] = 0;
+            if (live) {
+                const int seen_before = wave_count[wave][d];
+                rank[it] = seen_before + __popcll(peers & below);
+                if ((peers & below) == 0) wave_count[wave][d] = seen_before + __popcll(peers);
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+        __syncthreads();
+        int running = 0, inc = 0;
+        if (threadIdx.x < kDigits) {
+            for (int w = 0; w < kSmallWaves; ++w) {
+                const int c = wave_count[w][threadIdx.x];
+                wave_count[w][threadIdx.x] = running;
+                running += c;
+            }
+            inc = running;
+#pragma unroll
+            for (int s = 1; s < kWave; s <<= 1) {
+                const int n = __shfl_up(inc, s, kWave);
+                if (lane >= s) inc += n;
+            }
+            if (lane == kWave - 1) tmp[wave] = inc;
+        }
+        __syncthreads();
+        if (threadIdx.x < kDigits) {
+            int before = 0;
+            for (int w = 0; w < wave; ++w) before += tmp[w];
+            digit_start[threadIdx.x] = before + inc - running;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int it = 0; it < kSmallItems; ++it) {
+            const int i = base + it * kWave + lane;
+            if (it * kWave < per_wave && i < N) {
+                const int d = digit_of(key[it], shift);
+                const int at = digit_start[d] + wave_count[wave][d] + rank[it];
+                keys[from ^ 1][at] = key[it];
+                rows[from ^ 1][at] = rows[from][i];
+            }
+        }
+        from ^= 1;
+        __syncthreads();
+    }
+    // the id of a position: how many runs of equal codes have begun
+    const int p0 = threadIdx.x * kSmallItems;
+    bool head[kSmallItems];
+    int mine = 0;
+#pragma unroll
+    for (int u = 0; u < kSmallItems; ++u) {
+        const int p = p0 + u;
+        head[u] = p < N && (p == 0 || keys[from][p] != keys[from][p - 1]);
+        mine += head[u];
+    }
+    int inc = mine;
+#pragma unroll
+    for (int s = 1; s < kWave; s <<= 1) {
+        const int n = __shfl_up(inc, s, kWave);
+        if (lane >= s) inc += n;
+    }
+    if (lane == kWave - 1) tmp[wave] = inc;
+    __syncthreads();
+    int id = inc - mine, groups = 0;
+#pragma unroll
+    for (int w = 0; w < kSmallWaves; ++w) {
+        if (w < wave) id += tmp[w];
+        groups += tmp[w];
+    }
+    int32_t *start = keys[from ^ 1];  // of every group; the buffer of the pass before is free (groups <= N)
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kSmallItems; ++u) {
+        const int p = p0 + u;
+        if (p >= N) break;
+        if (head[u]) start[id++] = p;
+        sorted_id[p] = id;
+        const int row = rows[from][p];
+        perm[p] = row;
+        ids[row] = id;
+    }
+    __syncthreads();
+    int largest = 0;
+    for (int g = threadIdx.x; g < groups; g += kSmallThreads) {
+        const int s = start[g], c = (g + 1 < groups ? start[g + 1] : N) - s;
+        offsets[g + 1] = s;
+        counts[g + 1] = c;
+        largest = max(largest, c);
+    }
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1) largest = max(largest, __shfl_xor(largest, d, kWave));
+    if (lane == 0) tmp[wave] = largest;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kSmallWaves; ++w) largest = max(largest, tmp[w]);
+        offsets[0] = 0;
+        counts[0] = 0;
+        offsets[groups + 1] = N;
+        summary[0] = groups;
+        summary[1] = largest;
+    }
+}
+
 __global__ void group_empty_kernel(int32_t *offsets, int32_t *counts, int32_t *summary) {
     offsets[0] = offsets[1] = 0;
     counts[0] = 0;
@@ -554,8 +696,11 @@ GroupLayout group_layout(int64_t N, int bits) {
 
 using namespace cgnn;
 
+extern "C" int64_t cgnn_lsh_group_small_rows(void) { return kSmallRows; }
+
 extern "C" size_t cgnn_lsh_group_workspace_bytes(int64_t N, int bits) {
     if (N <= 0 || N >= INT32_MAX || bits < 0 || bits > 30) return 0;
+    if (N <= kSmallRows) return 0;
     // two columns (sorted codes; the keys or the payload between passes), the sort's counters,
     // and the code table (up to 16 bits) or the run heads and their scan (beyond)
     return group_layout(N, bits).total();
@@ -572,6 +717,11 @@ extern "C" int cgnn_lsh_group(int64_t N, int bits, const int32_t *raw_code, int6
         return check_launch("lsh_group");
     }
     CGNN_REQUIRE(raw_code && ids && perm && sorted_id, "cgnn_lsh_group: null array");
+    if (N <= kSmallRows) {
+        hipLaunchKernelGGL(group_small_kernel, dim3(1), dim3(kSmallThreads), 0, stream, raw_code, (int)N, radix_passes(bits),
+                           (int)(((int64_t)1 << bits) - 1), ids, offsets, perm, sorted_id, counts, summary);
+        return check_launch("lsh_group");
+    }
     if (workspace == nullptr || workspace_bytes < cgnn_lsh_group_workspace_bytes(N, bits))
         return fail(CGNN_EWORKSPACE, "cgnn_lsh_group: workspace too small");
     const GroupLayout L = group_layout(N, bits);

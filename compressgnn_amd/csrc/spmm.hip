@@ -38,7 +38,7 @@
 //     per workgroup in memory; the workgroup that finds itself the last to arrive at the row adds the pieces
 //     up, in ascending order, so the sum does not depend on which one that is.
 //
-// Modes: VAL (stored values), UNIT (all values 1), RELU_MASK (unit values, gathered
+// Modes: VAL (stored values), UNIT (all values 1: member lists, whose rows are gathered once), RELU_MASK (unit values, gathered
 // rows zeroed where a second matrix is <= 0), DUAL (columns below `split` gather from
 // X, the others from X1; the two partial sums are kept apart and combined as
 // (0 + sum1) + sum0, which is what two successive accumulating products give).
@@ -60,6 +60,10 @@ constexpr int kRowUnroll = 4;     // same for the row schedule (8: 9 % slower on
 constexpr int kXcds = 8;          // accelerator dies of an MI355X, each with its own L2
 constexpr int kDefaultSeg = 64;   // non-zeros per lane group in the nnz schedule
 
+// Where the runs of the nnz kernel come from: positions that are multiples of the run length, the table of
+// workgroup runs, or the same rule worked out by every lane group (member lists, which are new with every
+// assignment: a launch for their table would cost more than the few dependent loads).
+enum { WGRUNS_NONE = 0, WGRUNS_TABLE = 1, WGRUNS_COMPUTED = 2 };
 enum { MODE_VAL = 0, MODE_UNIT = 1, MODE_RELU_MASK = 2, MODE_DUAL = 3, MODE_SIGN_MASK = 4 };
 
 template <typename T, int VEC>
@@ -96,19 +100,39 @@ struct SpmmArgs {
     int32_t merge_stride;
     int32_t stretch_log2;  // log2 of the workgroups per XCD stretch (see logical_block); set at launch
     int32_t blocks;        // workgroups with work (the grid rounds this up to a multiple of kXcds)
-    int32_t read_once;     // MODE_UNIT: every row of X is gathered once (member lists), so with streaming loads
     const int32_t *cut_rows;    // spmm_fixup_rows_kernel: the stored rows that the runs cut, ascending
     const int32_t *empty_rows;  // and the stored rows without entries
     int32_t n_cut_rows, n_empty_rows;
     const int32_t *run_start;   // nnz schedule: first non-zero of every run, [nseg + 1], or NULL (run_boundary)
     int32_t *arrivals;          // workgroup runs: per workgroup and feature tile, the pieces stored so far of the row
                                 // that goes on behind it; zero before and after every launch
-    int32_t wg_len;             // workgroup runs: non-zeros per workgroup (run_start is the table of cgnn_csr.wg_runs)
+    int32_t wg_len;             // workgroup runs: non-zeros per workgroup (run_start is the table of cgnn_csr.wg_runs, or NULL)
+    int32_t keep;               // ... a row of at most this many entries is never divided, whatever the lengths
+    int32_t find_empty;         // ... the rows without entries are found from rowptr, not from a list
+    int32_t mean;               // ... every row is divided by its number of entries
 };
 
 // An entry of the table of workgroup runs is the first non-zero of a run, with this bit set when the row
 // found there began before it.
 constexpr int32_t kRowGoesOn = INT32_MIN;
+
+// Where lane group g of workgroup w begins, as such an entry (the rule stands at cgnn_csr.wg_runs).
+__device__ __forceinline__ int32_t wg_run_begin(const int32_t *rowptr, const int32_t *rowidx, int32_t nnz, int32_t wg_len,
+                                                int32_t groups, int32_t keep, int64_t w, int g) {
+    // e moved back to the start of its row when the row has at most `whole` entries
+    auto begin_of = [&](int64_t e, int whole) -> int32_t {
+        if (e >= nnz) return nnz;
+        const int r = rowidx[e], s0 = rowptr[r];
+        return rowptr[r + 1] - s0 <= whole ? s0 : (s0 < e ? (int32_t)e | kRowGoesOn : (int32_t)e);
+    };
+    const int run_len = wg_len / groups;
+    const int32_t b0 = begin_of(w * wg_len, wg_len > keep ? wg_len : keep);
+    if (g == 0) return b0;
+    const int32_t b1 = begin_of((w + 1) * wg_len, wg_len > keep ? wg_len : keep);
+    const int32_t first = b0 & ~kRowGoesOn, end = b1 & ~kRowGoesOn;
+    const int32_t e = first + g * ((end - first + groups - 1) / groups);
+    return e >= end ? b1 : begin_of(e, run_len > keep ? run_len : keep);
+}
 
 // carry_row values below zero: the run carries nothing, or its carry was added to that
 // of an earlier run of the same workgroup (the row of Y is the one of that earlier run).
@@ -244,7 +268,7 @@ struct Acc {
 // Y[row] = (accumulate ? Y[row] : 0) + acc
 template <typename T, int VEC, int TILES, int MODE>
 __device__ __forceinline__ void write_row(T *Y, int64_t F, int row, const int64_t foff[TILES],
-                                          const Acc<T, VEC, TILES, MODE> &acc, int accumulate) {
+                                          const Acc<T, VEC, TILES, MODE> &acc, int accumulate, T divisor = T(1)) {
     T *yrow = Y + (int64_t)row * F;
     // Only the plain product (MODE_VAL) can add to an existing Y.  The other modes write every row once, and
     // knowing that at compile time keeps a load of Y out of the block that closes a row inside a run of the
@@ -262,14 +286,17 @@ __device__ __forceinline__ void write_row(T *Y, int64_t F, int row, const int64_
         }
 #pragma unroll
         for (int i = 0; i < VEC; ++i) o.v[i] = acc.total(o.v[i], t, i);
+        if constexpr (MODE == MODE_UNIT)
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) o.v[i] = o.v[i] / divisor;
         if (accumulate) store_pack<T, VEC>(yrow + foff[t], o);
         else store_pack_stream<T, VEC>(yrow + foff[t], o);
     }
 }
 
-// Gather one feature tile of column c (source chosen by `src` in MODE_DUAL, masked by
+// kRowBytes: what the lanes of a row span.  Gather one feature tile of column c (source chosen by `src` in MODE_DUAL, masked by
 // M in MODE_RELU_MASK and by the bits of `signs` in MODE_SIGN_MASK).
-template <typename T, int VEC, int MODE>
+template <typename T, int VEC, int MODE, int kRowBytes>
 __device__ __forceinline__ Pack<T, VEC> gather(const SpmmArgs<T> &a, int c, int src, int64_t foff) {
     Pack<T, VEC> x;
     if (foff < 0) {
@@ -286,8 +313,12 @@ __device__ __forceinline__ Pack<T, VEC> gather(const SpmmArgs<T> &a, int c, int 
         c -= src ? a.split : 0;
     }
     const int64_t off = (int64_t)c * (int32_t)a.F + foff;  // F < 2^31: one 32 x 32 -> 64 bit multiply
-    // rows that are gathered once (member lists; masks exist for those only) are not kept in the caches
-    if (MODE == MODE_RELU_MASK || MODE == MODE_SIGN_MASK || (MODE == MODE_UNIT && a.read_once))
+    // Rows that are gathered once (member lists, which the modes without values exist for) are not kept in the
+    // caches -- unless they are shorter than a cache line, whose other half is a row that is still to come (16
+    // features, 10^6 rows: 44 us so, 32 us kept).  A choice at compile time: the compiler merges the two loads of a
+    // branch into one that is kept.  Kept rows cost the kernel that writes next most: behind the means of 2.4 M rows
+    // the spread of 256 features took 725 us for 485 and the gradient of the means 283 us for 175.
+    if constexpr ((MODE == MODE_RELU_MASK || MODE == MODE_SIGN_MASK || MODE == MODE_UNIT) && kRowBytes > 128)
         x = load_pack_stream<T, VEC>(base + off);
     else
         x = load_pack<T, VEC>(base + off);
@@ -418,7 +449,7 @@ __global__ __launch_bounds__(kBlock) void spmm_row_kernel(SpmmArgs<T> a) {
                         if (u0 + u < cnt) {  // no gathers behind the row's end: repeated ones still cost issue slots
 #pragma unroll
                             for (int t = 0; t < TILES; ++t)
-                                x[u][t] = gather<T, VEC, MODE>(a, c[u], kPlain ? 0 : c[u] >= a.split, fld[t]);
+                                x[u][t] = gather<T, VEC, MODE, (int)(VEC * LPR * sizeof(T))>(a, c[u], kPlain ? 0 : c[u] >= a.split, fld[t]);
                         }
 #pragma unroll
                     for (int u = 0; u < RU; ++u)
@@ -443,7 +474,7 @@ __global__ __launch_bounds__(kBlock) void spmm_row_kernel(SpmmArgs<T> a) {
             for (int u = 0; u < kRowUnroll; ++u)
                 if (e + u < e1) {
 #pragma unroll
-                    for (int t = 0; t < TILES; ++t) x[u][t] = gather<T, VEC, MODE>(a, c[u], c[u] >= a.split, foff[t]);
+                    for (int t = 0; t < TILES; ++t) x[u][t] = gather<T, VEC, MODE, (int)(VEC * LPR * sizeof(T))>(a, c[u], c[u] >= a.split, foff[t]);
                 }
 #pragma unroll
             for (int u = 0; u < kRowUnroll; ++u)
@@ -469,12 +500,14 @@ __device__ __forceinline__ int run_boundary(const SpmmArgs<T> &a, int e) {
 // What a workgroup's runs left of the rows that are divided among them, put together: the end of the
 // kernel below for workgroup runs.  Every lane group holds the sum of the row that goes on behind its run
 // (`continues`, in acc) and in `heads` the part of a row that came into its run and ended there; still
-// `open`: one row covers the whole run.  The lane group a row begins in adds the parts of those behind it, in
+// `open`: one row covers the whole run; begin, behind: the table's entries for the first run of this workgroup
+// and of the next.  The lane group a row begins in adds the parts of those behind it, in
 // ascending order.  Slots of 2 * workgroups rows of a.carry hold the pieces of the rows that pass from one
 // workgroup to the next: 2 * w for the row that comes into workgroup w, 2 * w + 1 for one that begins in it.
 template <typename T, int VEC, int LPR, int TILES, int MODE>
 __device__ __forceinline__ void join_rows(const SpmmArgs<T> &a, int block, int lane, int grp, const int64_t foff[TILES],
-                                          const Acc<T, VEC, TILES, MODE> &acc, bool continues, bool open, int y_row, int *flags, Pack<T, VEC> (*tails)[kBlock],
+                                          const Acc<T, VEC, TILES, MODE> &acc, bool continues, bool open, int y_row,
+                                          int32_t begin, int32_t behind, int *flags, Pack<T, VEC> (*tails)[kBlock],
                                           Pack<T, VEC> (*heads)[kBlock]) {
     constexpr int GPB = kBlock / LPR;
     constexpr int kContinues = 1, kWholeRun = 2;
@@ -492,9 +525,11 @@ __device__ __forceinline__ void join_rows(const SpmmArgs<T> &a, int block, int l
     __syncthreads();
     const int64_t groups = (int64_t)a.blocks * GPB;
     if (!a.accumulate) {  // rows without entries
+        const int candidates = a.find_empty ? a.rows : a.n_empty_rows;
 #pragma unroll 1
-        for (int64_t item = (int64_t)block * GPB + grp; item < a.n_empty_rows; item += groups) {
-            T *y = a.Y + (int64_t)out_row(a, a.empty_rows[item]) * a.F;
+        for (int64_t item = (int64_t)block * GPB + grp; item < candidates; item += groups) {
+            if (a.find_empty && a.rowptr[item] != a.rowptr[item + 1]) continue;
+            T *y = a.Y + (int64_t)out_row(a, a.find_empty ? (int)item : a.empty_rows[item]) * a.F;
             Pack<T, VEC> zero;
 #pragma unroll
             for (int i = 0; i < VEC; ++i) zero.v[i] = T(0);
@@ -536,6 +571,9 @@ __device__ __forceinline__ void join_rows(const SpmmArgs<T> &a, int block, int l
     };
     auto store_row = [&](int row, const Pack<T, VEC>(&sum)[TILES]) {
         T *y = a.Y + (int64_t)row * a.F;
+        T divisor = T(1);
+        if constexpr (MODE == MODE_UNIT)
+            if (a.mean) divisor = (T)(a.rowptr[row + 1] - a.rowptr[row]);  // blocks without a row map
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
             if (foff[t] < 0) continue;
@@ -546,10 +584,13 @@ __device__ __forceinline__ void join_rows(const SpmmArgs<T> &a, int block, int l
 #pragma unroll
                     for (int i = 0; i < VEC; ++i) o.v[i] = base.v[i] + o.v[i];
                 }
+            if constexpr (MODE == MODE_UNIT)
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) o.v[i] = o.v[i] / divisor;
             store_pack<T, VEC>(y + foff[t], o);
         }
     };
-    const bool comes_in = a.run_start[block * GPB] < 0, goes_out = a.run_start[(block + 1) * GPB] < 0;
+    const bool comes_in = begin < 0, goes_out = behind < 0;
     if (grp == 0 && comes_in) {
         Pack<T, VEC> sum[TILES];
 #pragma unroll
@@ -568,8 +609,7 @@ __device__ __forceinline__ void join_rows(const SpmmArgs<T> &a, int block, int l
     if (!comes_in && !goes_out) return;
     // Rows that this workgroup shares with others.
     __shared__ int arrived_last;
-    const int first_row = a.rowidx[a.run_start[block * GPB] & ~kRowGoesOn];
-    const int last_row = a.rowidx[(a.run_start[(block + 1) * GPB] & ~kRowGoesOn) - 1];
+    const int first_row = a.rowidx[begin & ~kRowGoesOn], last_row = a.rowidx[(behind & ~kRowGoesOn) - 1];
 #pragma unroll 1
     for (int side = 0; side < 2; ++side) {
         if (side == 0 ? !comes_in : (!goes_out || (comes_in && first_row == last_row))) continue;
@@ -632,12 +672,12 @@ __device__ __forceinline__ void join_rows(const SpmmArgs<T> &a, int block, int l
     }
 }
 
-template <typename T, int VEC, int LPR, int TILES, int MODE, bool WGRUNS>
+template <typename T, int VEC, int LPR, int TILES, int MODE, int WGRUNS>
 __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spmm_nnz_kernel(SpmmArgs<T> a) {
     constexpr int GPB = kBlock / LPR;
     __shared__ int wg_row[GPB];
     __shared__ Pack<T, VEC> wg_carry[TILES][kBlock];
-    __shared__ Pack<T, VEC> wg_head[WGRUNS ? TILES : 1][WGRUNS ? kBlock : 1];
+    __shared__ Pack<T, VEC> wg_head[WGRUNS != WGRUNS_NONE ? TILES : 1][WGRUNS != WGRUNS_NONE ? kBlock : 1];
     const int lane = threadIdx.x % LPR, grp = threadIdx.x / LPR;
     const int block = logical_block(a);
     int seg = block * GPB + grp;
@@ -645,9 +685,19 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
     int e0 = 0, e1 = 0;
     bool continues = false;    // the last row of the run goes on in the next one
     bool open = false;         // WGRUNS: the row at hand began before the run
+    int32_t wg_begin = 0, wg_behind = 0;
     if (seg < a.nseg) {
-        if constexpr (WGRUNS) {
-            const int r0 = a.run_start[seg], r1 = a.run_start[seg + 1];
+        if constexpr (WGRUNS != WGRUNS_NONE) {
+            int32_t r0, r1;
+            if constexpr (WGRUNS == WGRUNS_TABLE) {
+                r0 = a.run_start[seg], r1 = a.run_start[seg + 1];
+            } else {
+                auto begin_of = [&](int w, int g) {
+                    return wg_run_begin(a.rowptr, a.rowidx, a.nnz, a.wg_len, GPB, a.keep, w, g);
+                };
+                wg_begin = begin_of(block, 0), wg_behind = begin_of(block + 1, 0);
+                r0 = begin_of(block, grp), r1 = grp + 1 < GPB ? begin_of(block, grp + 1) : wg_behind;
+            }
             e0 = r0 & ~kRowGoesOn, e1 = r1 & ~kRowGoesOn;
             open = r0 < 0, continues = r1 < 0;
         } else if (a.run_start != nullptr) {  // one load instead of two dependent ones
@@ -668,8 +718,9 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
     int cur_out = -1;
     // A row ends inside the run: it is written, or (the part of it that lies in this run) put aside
     // for the lane group where the row began.
-    auto finish_row = [&](int y_row) {
-        if constexpr (WGRUNS) {
+    int row_e0 = e0;  // where the row at hand begins in the run
+    auto finish_row = [&](int y_row, int end) {
+        if constexpr (WGRUNS != WGRUNS_NONE) {
             if (open) {
                 open = false;
 #pragma unroll
@@ -679,7 +730,8 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                 return;
             }
         }
-        write_row<T, VEC, TILES, MODE>(a.Y, a.F, y_row, foff, acc, a.accumulate);
+        write_row<T, VEC, TILES, MODE>(a.Y, a.F, y_row, foff, acc, a.accumulate,
+                                       WGRUNS == WGRUNS_COMPUTED && MODE == MODE_UNIT && a.mean ? (T)(end - row_e0) : T(1));
     };
     // the names of rows: see below
     constexpr bool kNamesRowsOfY = !(MODE == MODE_DUAL && VEC * LPR * sizeof(T) >= 512);
@@ -701,7 +753,7 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
         int last_row, row_behind;
         if constexpr (!kNamesRowsOfY) {  // the names are the stored rows: the first is read here, the last is at hand at the end
             cur_out = a.rowidx[e0];
-            if constexpr (!WGRUNS) row_behind = e1 < a.nnz ? a.rowidx[e1] : -1;
+            if constexpr (WGRUNS == WGRUNS_NONE) row_behind = e1 < a.nnz ? a.rowidx[e1] : -1;
         }
         if constexpr (LPR >= kUnroll && sizeof(T) == 4) {
             // As in the row schedule: the lanes of the group load one entry each, and the
@@ -722,7 +774,7 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                 if constexpr (kNamesRowsOfY) {
                     // with every batch of entries, so that no load of the run waits for another but
                     // the row numbers for their rows (the same two words each time)
-                    if constexpr (!WGRUNS) {
+                    if constexpr (WGRUNS == WGRUNS_NONE) {
                         last_row = a.rowidx[e1 - 1];
                         row_behind = e1 < a.nnz ? a.rowidx[e1] : -1;
                     }
@@ -765,14 +817,15 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                             if (kGatherAll || u0 + u < cnt) {
 #pragma unroll
                                 for (int t = 0; t < TILES; ++t)
-                                    x[u][t] = gather<T, VEC, MODE>(a, c[u], kPlain ? 0 : c[u] >= a.split, fld[t]);
+                                    x[u][t] = gather<T, VEC, MODE, (int)(VEC * LPR * sizeof(T))>(a, c[u], kPlain ? 0 : c[u] >= a.split, fld[t]);
                             }
 #pragma unroll
                         for (int u = 0; u < kUnroll; ++u) {
                             if (u0 + u < cnt) {
                                 if (o[u] != cur_out) {
                                     // the row ends inside this run: finish it here
-                                    finish_row(row_of_y(cur_out));
+                                    finish_row(row_of_y(cur_out), e + u0 + u);
+                                    row_e0 = e + u0 + u;
                                     acc.clear();
                                     cur_out = o[u];
                                 }
@@ -787,7 +840,7 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
         } else {
             if constexpr (kNamesRowsOfY) {
                 cur_out = named(a.rowidx[e0]);
-                if constexpr (!WGRUNS) {
+                if constexpr (WGRUNS == WGRUNS_NONE) {
                     last_row = a.rowidx[e1 - 1];
                     row_behind = e1 < a.nnz ? a.rowidx[e1] : -1;
                 }
@@ -810,14 +863,15 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                     if (e + u < e1) {
 #pragma unroll
                         for (int t = 0; t < TILES; ++t)
-                            x[u][t] = gather<T, VEC, MODE>(a, c[u], c[u] >= a.split, foff[t]);
+                            x[u][t] = gather<T, VEC, MODE, (int)(VEC * LPR * sizeof(T))>(a, c[u], c[u] >= a.split, foff[t]);
                     }
 #pragma unroll
                 for (int u = 0; u < kUnroll; ++u) {
                     if (e + u < e1) {
                         if (o[u] != cur_out) {
                             // the row ends inside this run: finish it here
-                            finish_row(row_of_y(cur_out));
+                            finish_row(row_of_y(cur_out), e + u);
+                            row_e0 = e + u;
                             acc.clear();
                             cur_out = o[u];
                         }
@@ -826,16 +880,18 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                 }
             }
         }
-        if constexpr (!WGRUNS) {
+        if constexpr (WGRUNS == WGRUNS_NONE) {
             cur = kNamesRowsOfY ? last_row : cur_out;
             continues = row_behind == cur;
         }
-        if (!continues) finish_row(row_of_y(cur_out));
+        if (!continues) finish_row(row_of_y(cur_out), e1);
     }
-    if constexpr (WGRUNS) {
+    if constexpr (WGRUNS != WGRUNS_NONE) {
+        if constexpr (WGRUNS == WGRUNS_TABLE)
+            if (seg < a.nseg) wg_begin = a.run_start[block * GPB], wg_behind = a.run_start[(block + 1) * GPB];
         join_rows<T, VEC, LPR, TILES, MODE>(a, block, lane, grp, foff, acc, continues, open,
-                                            continues && active ? row_of_y(cur_out) : -1, wg_row, wg_carry,
-                                            wg_head);
+                                            continues && active ? row_of_y(cur_out) : -1, wg_begin, wg_behind, wg_row,
+                                            wg_carry, wg_head);
         return;
     }
     // The carries of one row are added per workgroup: the first of its lane groups that
@@ -1223,20 +1279,27 @@ int launch_shape(int kind, int mode, const SpmmArgs<T> &args, int64_t items, int
                 hipLaunchKernelGGL((spmm_row_kernel<T, VEC, LPR, TILES, MODE_VAL>), grid, block, 0, stream, a);
             break;
         case KIND_NNZ:
-            if (a.arrivals != nullptr && mode == MODE_DUAL)
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_DUAL, true>), grid, block, 0, stream, a);
+            if (a.arrivals != nullptr && a.run_start == nullptr) {
+                if (mode == MODE_UNIT)
+                    hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_UNIT, WGRUNS_COMPUTED>), grid, block, 0, stream, a);
+                else if (mode == MODE_SIGN_MASK)
+                    hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_SIGN_MASK, WGRUNS_COMPUTED>), grid, block, 0, stream, a);
+                else
+                    hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_RELU_MASK, WGRUNS_COMPUTED>), grid, block, 0, stream, a);
+            } else if (a.arrivals != nullptr && mode == MODE_DUAL)
+                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_DUAL, WGRUNS_TABLE>), grid, block, 0, stream, a);
             else if (a.arrivals != nullptr)
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_VAL, true>), grid, block, 0, stream, a);
+                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_VAL, WGRUNS_TABLE>), grid, block, 0, stream, a);
             else if (mode == MODE_VAL)
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_VAL, false>), grid, block, 0, stream, a);
+                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_VAL, WGRUNS_NONE>), grid, block, 0, stream, a);
             else if (mode == MODE_UNIT)
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_UNIT, false>), grid, block, 0, stream, a);
+                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_UNIT, WGRUNS_NONE>), grid, block, 0, stream, a);
             else if (mode == MODE_DUAL)
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_DUAL, false>), grid, block, 0, stream, a);
+                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_DUAL, WGRUNS_NONE>), grid, block, 0, stream, a);
             else if (mode == MODE_SIGN_MASK)
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_SIGN_MASK, false>), grid, block, 0, stream, a);
+                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_SIGN_MASK, WGRUNS_NONE>), grid, block, 0, stream, a);
             else
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_RELU_MASK, false>), grid, block, 0, stream, a);
+                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_RELU_MASK, WGRUNS_NONE>), grid, block, 0, stream, a);
             break;
         case KIND_FIXUP: {  // a lane group per carry, and (when not accumulating) a thread per row
             const int64_t for_rows = a.accumulate ? 0 : ceil_div((int64_t)a.rows, kBlock);
@@ -1404,7 +1467,6 @@ int spmm_typed(const cgnn_csr *A, const void *X, const void *X1, int64_t split, 
     if (mode != MODE_DUAL) split = INT32_MAX;  // every column comes from X
     SpmmArgs<T> a = make_args<T>(A, X, X1, split, M, Y, F, accumulate);
     const bool masked = mode == MODE_RELU_MASK || mode == MODE_SIGN_MASK;
-    a.read_once = mode == MODE_UNIT || masked;  // asked for by name: the cluster reductions
     if (mode == MODE_SIGN_MASK) {  // M holds bits, not rows
         a.signs = static_cast<const uint32_t *>(M);
         a.sign_words = (int32_t)ceil_div(F, 32);
@@ -1414,8 +1476,6 @@ int spmm_typed(const cgnn_csr *A, const void *X, const void *X1, int64_t split, 
     const bool may_choose = kernel == CGNN_SPMM_AUTO;
     kernel = resolve_kernel(A, kernel);
     if (masked) kernel = CGNN_SPMM_NNZ;  // masks exist for the nnz schedule only
-    // unit values without the multiplications; a product that adds to Y stays with the plain mode, the only one that reads Y
-    if (mode == MODE_VAL && A->val == nullptr && kernel == CGNN_SPMM_NNZ && !accumulate) mode = MODE_UNIT;
     if (mode == MODE_DUAL && A->nnz > 0 && A->val == nullptr)
         return fail(CGNN_EINVAL, "spmm: the two-source product needs stored values");
     if (kernel == CGNN_SPMM_ROW) {
@@ -1440,7 +1500,7 @@ int spmm_typed(const cgnn_csr *A, const void *X, const void *X1, int64_t split, 
         a.carry = static_cast<T *>(ws);
         a.empty_rows = A->empty_rows;
         a.n_empty_rows = A->n_empty_rows;
-        return launch<T>(KIND_NNZ, mode == MODE_UNIT ? MODE_VAL : mode, s, a, a.nseg, stream);
+        return launch<T>(KIND_NNZ, mode, s, a, a.nseg, stream);
     }
     const int seg = seg_len(A);
     const int64_t nseg = ceil_div(A->nnz, seg);
@@ -1520,21 +1580,7 @@ __global__ void run_starts_kernel(const int32_t *__restrict__ rowptr, const int3
 __global__ void wg_runs_kernel(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ rowidx, int32_t nnz,
                                int32_t wg_len, int32_t groups, int64_t n, int32_t *__restrict__ runs) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int run_len = wg_len / groups;
-    // e moved back to the start of its row when the row has at most `whole` entries
-    auto begin_of = [&](int64_t e, int whole) -> int32_t {
-        if (e >= nnz) return nnz;
-        const int r = rowidx[e], s0 = rowptr[r];
-        return rowptr[r + 1] - s0 <= whole ? s0 : (int32_t)e;
-    };
-    const int64_t w = i / groups, g = i % groups;
-    const int32_t b0 = begin_of(w * wg_len, wg_len), b1 = begin_of((w + 1) * wg_len, wg_len);
-    const int64_t share = ((int64_t)b1 - b0 + groups - 1) / groups;
-    const int64_t e = b0 + g * share;
-    const int32_t s = g == 0 ? b0 : (e >= b1 ? b1 : begin_of(e, run_len));
-    const bool goes_on = s < nnz && rowptr[rowidx[s]] < s;
-    runs[i] = goes_on ? s | kRowGoesOn : s;
+    if (i < n) runs[i] = wg_run_begin(rowptr, rowidx, nnz, wg_len, groups, 0, i / groups, (int)(i % groups));
 }
 
 // rowidx[e] = largest r with rowptr[r] <= e (rows without entries are skipped).
@@ -1605,6 +1651,46 @@ int spmm_members(const cgnn_csr *A, int dtype, const void *X, const void *M, voi
     if (dtype == CGNN_F64)
         return spmm_typed<double>(A, X, nullptr, 0, M, Y, F, 0, CGNN_SPMM_NNZ, mode, ws, ws_bytes, stream);
     return fail(CGNN_EUNSUPPORTED, "spmm: dtype must be f32 or f64");
+}
+
+// The same sums in one launch (workgroup runs): mask as above; mean: divided by the number of members;
+// first_row_empty: row 0 is the only one without members (offsets[0] = 0 is then the list of the empty rows, and
+// A->rows may be a bound on the number of rows).  A member list of at most kDefaultSeg rows is summed in
+// ascending order, undivided, like there.
+int spmm_member_runs(const cgnn_csr *A, int dtype, const void *X, const void *M, void *Y, int64_t F, int mask, bool mean,
+                     bool first_row_empty, int32_t *arrivals, void *ws, size_t ws_bytes, hipStream_t stream) {
+    auto run = [&](auto zero) {
+        typedef decltype(zero) T;
+        const Shape s = pick_shape<T>(F, true);
+        const int groups = kBlock / s.lpr, wg_len = wg_run_len(A, groups) * groups;
+        const int64_t workgroups = ceil_div(A->nnz, wg_len);
+        if (ws == nullptr || ws_bytes < wg_piece_bytes(workgroups, F, sizeof(T)))
+            return fail(CGNN_EWORKSPACE, "member sums: workspace too small");
+        SpmmArgs<T> a = make_args<T>(A, X, nullptr, INT32_MAX, M, Y, F, 0);
+        if (mask == 2) {
+            a.signs = static_cast<const uint32_t *>(M);
+            a.sign_words = (int32_t)ceil_div(F, 32);
+        }
+        a.arrivals = arrivals;
+        a.wg_len = wg_len;
+        a.keep = kDefaultSeg;
+        a.nseg = (int32_t)(workgroups * groups);
+        a.carry = static_cast<T *>(ws);
+        a.find_empty = !first_row_empty;
+        a.empty_rows = A->rowptr;
+        a.n_empty_rows = first_row_empty ? 1 : 0;
+        a.mean = mean;
+        return launch<T>(KIND_NNZ, mask == 2 ? MODE_SIGN_MASK : (mask == 1 ? MODE_RELU_MASK : MODE_UNIT), s, a, a.nseg, stream);
+    };
+    return dtype == CGNN_F32 ? run(0.0f) : run(0.0);
+}
+
+size_t spmm_member_runs_bytes(const cgnn_csr *A, int64_t F, int dtype, int64_t *arrivals) {
+    const Shape s = shape_of(F, dtype);
+    const int groups = kBlock / s.lpr;
+    const int64_t workgroups = ceil_div(A->nnz, wg_run_len(A, groups) * groups);
+    *arrivals = workgroups * s.grid_y;
+    return wg_piece_bytes(workgroups, F, dtype == CGNN_F64 ? 8 : 4);
 }
 
 // ------------------------------------------- scratch that nobody allocates -------

@@ -9,7 +9,9 @@
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <hip/hip_runtime_api.h>
 #include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
 #include <torch/extension.h>
 
 #include <algorithm>
@@ -44,6 +46,48 @@ int dtype_code(const Tensor &t) {
 
 void require_gpu(const Tensor &t, const char *name) {
     TORCH_CHECK(t.is_cuda(), name, " must be a GPU tensor: this build of compressgnn_runtime has no CPU operators");
+}
+
+// Counters of the kernels whose last workgroup to arrive finishes a row (cgnn_csr.arrivals): every launch
+// leaves them at zero, so the launches of one stream share one set, and streams, which may overlap, each have
+// their own.  At most kStreams sets are held; the one used longest ago goes back to the allocator when another
+// stream comes.  Under a stream capture the set belongs to the graph (its zeroing is recorded with it).
+struct ArrivalPool {
+    static constexpr size_t kStreams = 32;
+    struct Set {
+        int device;
+        void *stream;
+        Tensor counters;
+    };
+    std::deque<Set> sets;  // most recently used first
+    std::mutex lock;
+
+    Tensor get(int64_t n, const Tensor &like) {
+        auto options = like.options().dtype(torch::kInt32).requires_grad(false);
+        hipStream_t stream = reinterpret_cast<hipStream_t>(current_stream(like));
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (stream != nullptr && hipStreamIsCapturing(stream, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone)
+            return torch::zeros({n}, options);
+        std::lock_guard<std::mutex> hold(lock);
+        const int device = like.device().index();
+        auto it = std::find_if(sets.begin(), sets.end(), [&](const Set &s) { return s.device == device && s.stream == stream; });
+        Set set{device, stream, Tensor()};
+        if (it != sets.end()) {
+            set = *it;
+            if (it != sets.begin()) sets.erase(it);
+            else if (set.counters.numel() >= n) return set.counters;
+            else sets.pop_front();
+        }
+        if (!set.counters.defined() || set.counters.numel() < n) set.counters = torch::zeros({std::max<int64_t>(2 * n, 4096)}, options);
+        sets.push_front(set);
+        while (sets.size() > kStreams) sets.pop_back();
+        return set.counters;
+    }
+};
+
+ArrivalPool &arrival_pool() {
+    static ArrivalPool *pool = new ArrivalPool();  // never destroyed: tensors must not outlive the allocator at exit
+    return *pool;
 }
 
 // ----------------------------------------------------------------- CSR blocks ----
@@ -532,7 +576,8 @@ Tensor propagate_backward(PropagationPlan &p, Tensor grad) {
 
 // One propagation as a step of autograd.  The node is native, so a training step takes neither the
 // interpreter nor its lock on the way back (the engine's thread and the caller's would pass the lock to each
-// other): forward and gradient over 2,708 vertices, @HOST@.
+// other): forward and gradient over 2,708 vertices took 69 us through a Python function and take 54 us so, 29
+// of them the engine's own.
 struct PropagateBackward : torch::autograd::Node {
     std::shared_ptr<PropagationPlan> plan;
     torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
@@ -641,37 +686,74 @@ std::vector<Tensor> cluster_workspace(Tensor input, int64_t bits) {
 // is at most min(N, 2^bits): every kernel runs on buffers of that bound, so the device
 // never waits for the host; the one scalar read of a refresh (cluster_kernel.cu:146-147)
 // comes last and only trims the views.
-std::tuple<Tensor, Tensor, int64_t, std::vector<Tensor>> cluster_assign_members(Tensor input, Tensor planes,
-                                                                                int64_t bits) {
+struct Assigned {
+    Tensor ids, counts, reps;
+    int64_t active = 0;
+    std::vector<Tensor> members;
+};
+
+// with_reps: the means of the rows over the clusters as well, launched before the host read where the buffer
+// for all clusters there could be is small (kSmallReps elements; the rows behind the last cluster stay unused).
+constexpr int64_t kSmallReps = int64_t(1) << 22;
+
+Tensor member_sums(const char *op, const Tensor &rows, int mask, const void *M, const std::vector<Tensor> &m, int64_t groups,
+                   bool mean, bool first_group_empty);
+
+Assigned assign(Tensor input, Tensor planes, int64_t bits, bool with_reps) {
     const char *op = "cluster_assign";
     const int64_t buckets = buckets_for(op, bits);
     expect_planes(op, input, planes, bits);
     c10::hip::HIPGuardMasqueradingAsCUDA guard(input.device());
-    const int64_t N = input.size(0);
+    const int64_t N = input.size(0), F = input.size(1);
     auto ints = input.options().dtype(torch::kInt32);
-    Tensor ids = torch::empty({N}, input.options().dtype(torch::kInt64));
-    Tensor perm = torch::empty({N}, ints), sorted_id = torch::empty({N}, ints);
+    Assigned a;
+    a.ids = torch::empty({N}, input.options().dtype(torch::kInt64));
     auto host_scalar = [](int64_t v) { return torch::full({1}, v, torch::TensorOptions().dtype(torch::kInt64)); };
-    if (N == 0)
-        return {ids, torch::zeros({1}, ints), 0, {torch::zeros({2}, ints), perm, sorted_id, host_scalar(0)}};
+    if (N == 0) {
+        a.counts = torch::zeros({1}, ints);
+        a.members = {torch::zeros({2}, ints), torch::empty({0}, ints), torch::empty({0}, ints), host_scalar(0)};
+        if (with_reps) a.reps = torch::zeros({1, F}, input.options());
+        return a;
+    }
     const int64_t cap = std::min<int64_t>(N, buckets);
-    Tensor raw = torch::empty({N}, ints);
-    Tensor offsets = torch::empty({cap + 2}, ints), counts = torch::empty({cap + 1}, ints);
-    Tensor summary_dev = torch::empty({2}, ints);  // number of groups, largest group
+    // each on its own: with the three in one buffer the spread over perm took 512 us for 484 at 2.4 M x 256
+    Tensor perm = torch::empty({N}, ints), sorted_id = torch::empty({N}, ints), codes = torch::empty({N}, ints);
+    int32_t *raw = codes.data_ptr<int32_t>();
+    Tensor sizes = torch::empty({2 * cap + 3}, ints);
+    Tensor offsets = sizes.narrow(0, 0, cap + 2), counts = sizes.narrow(0, cap + 2, cap + 1);
+    // number of groups, largest group: on the host at once where the grouping writes it with plain stores
+    const bool direct = N <= cgnn_lsh_group_small_rows();
+    Tensor summary = direct ? torch::empty({2}, torch::TensorOptions().dtype(torch::kInt32).pinned_memory(true))
+                            : torch::empty({2}, ints);
     auto stream = current_stream(input);
-    ok(cgnn_lsh_hash(N, input.size(1), (int)bits, dtype_code(input), input.data_ptr(), planes.data_ptr(),
-                     raw.data_ptr<int32_t>(), nullptr, stream),
-       "lsh_hash");
+    ok(cgnn_lsh_hash(N, F, (int)bits, dtype_code(input), input.data_ptr(), planes.data_ptr(), raw, nullptr, stream), "lsh_hash");
     const size_t bytes = cgnn_lsh_group_workspace_bytes(N, (int)bits);
     Tensor ws = torch::empty({(int64_t)std::max<size_t>(bytes, 1)}, input.options().dtype(torch::kUInt8));
-    ok(cgnn_lsh_group(N, (int)bits, raw.data_ptr<int32_t>(), ids.data_ptr<int64_t>(), offsets.data_ptr<int32_t>(),
-                      perm.data_ptr<int32_t>(), sorted_id.data_ptr<int32_t>(), counts.data_ptr<int32_t>(),
-                      summary_dev.data_ptr<int32_t>(), ws.data_ptr(), bytes, stream),
+    ok(cgnn_lsh_group(N, (int)bits, raw, a.ids.data_ptr<int64_t>(), offsets.data_ptr<int32_t>(), perm.data_ptr<int32_t>(),
+                      sorted_id.data_ptr<int32_t>(), counts.data_ptr<int32_t>(), summary.data_ptr<int32_t>(), ws.data_ptr(), bytes,
+                      stream),
        "lsh_group");
-    Tensor summary = summary_dev.cpu();  // the one host read of a refresh
-    const int active = summary.data_ptr<int32_t>()[0];
-    return {ids, counts.narrow(0, 0, active + 1), (int64_t)active,
-            {offsets.narrow(0, 0, active + 2), perm, sorted_id, host_scalar(summary.data_ptr<int32_t>()[1])}};
+    const std::vector<Tensor> wide_lists = {offsets, perm, sorted_id};
+    const bool early = with_reps && F > 0 && (cap + 1) * F <= kSmallReps;
+    if (early) a.reps = member_sums("cluster_mean", input, 0, nullptr, wide_lists, cap + 1, true, true);
+    // the one host read of a refresh
+    if (direct) {
+        TORCH_CHECK(hipStreamSynchronize(reinterpret_cast<hipStream_t>(stream)) == hipSuccess, op, ": the stream reported an error");
+    } else {
+        summary = summary.cpu();
+    }
+    a.active = summary.data_ptr<int32_t>()[0];
+    a.counts = counts.narrow(0, 0, a.active + 1);
+    a.members = {offsets.narrow(0, 0, a.active + 2), perm, sorted_id, host_scalar(summary.data_ptr<int32_t>()[1])};
+    if (early) a.reps = a.reps.narrow(0, 0, a.active + 1);
+    else if (with_reps && F > 0) a.reps = member_sums("cluster_mean", input, 0, nullptr, a.members, a.active + 1, true, true);
+    else if (with_reps) a.reps = torch::zeros({a.active + 1, F}, input.options());
+    return a;
+}
+
+std::tuple<Tensor, Tensor, int64_t, std::vector<Tensor>> cluster_assign_members(Tensor input, Tensor planes, int64_t bits) {
+    Assigned a = assign(input, planes, bits, false);
+    return {a.ids, a.counts, a.active, a.members};
 }
 
 // Member lists by the index tensor they belong to.  The operators with the reference's
@@ -821,7 +903,22 @@ std::vector<Tensor> members_or_build(const char *op, const c10::optional<std::ve
     return known;
 }
 
-int64_t largest_group(const std::vector<Tensor> &m) { return m.size() == 4 ? m[3].item<int64_t>() : 0; }
+// Sums (or means) over the members of every group, [groups, F]; rows has at least one element.
+Tensor member_sums(const char *op, const Tensor &rows, int mask, const void *M, const std::vector<Tensor> &m, int64_t groups,
+                   bool mean, bool first_group_empty) {
+    const int64_t N = rows.size(0), F = rows.size(1);
+    const int dtype = dtype_code(rows);
+    Tensor out = torch::empty({groups, F}, rows.options());
+    int64_t arrivals = 0;
+    const size_t bytes = cgnn_cluster_sums_workspace_bytes(N, F, groups, dtype, &arrivals);
+    Tensor ws = torch::empty({(int64_t)std::max<size_t>(bytes, 1)}, rows.options().dtype(torch::kUInt8));
+    Tensor counters = arrival_pool().get(arrivals, rows);
+    ok(cgnn_cluster_sums(N, F, groups, dtype, rows.data_ptr(), mask, M, m[0].data_ptr<int32_t>(), m[1].data_ptr<int32_t>(),
+                         m[2].data_ptr<int32_t>(), mean, first_group_empty, out.data_ptr(), ws.data_ptr(), bytes,
+                         counters.data_ptr<int32_t>(), current_stream(rows)),
+       op);
+    return out;
+}
 
 // cluster_mean_cuda (cluster_kernel.cu:158-170).  `members` (from cluster_members, for
 // the same index) avoids rebuilding the member lists on every call.
@@ -833,13 +930,9 @@ Tensor cluster_mean(Tensor input, Tensor index, Tensor count, c10::optional<std:
     const int64_t N = input.size(0), F = input.size(1), groups = count.numel();
     if (input.numel() == 0) return torch::zeros({groups, F}, input.options());
     auto m = members_or_build(op, members, index, groups);
-    Tensor out = torch::empty({groups, F}, input.options());
-    const size_t bytes = cgnn_cluster_mean_workspace_bytes(N, F, groups, dtype_code(input));
-    Tensor ws = torch::empty({(int64_t)std::max<size_t>(bytes, 1)}, input.options().dtype(torch::kUInt8));
-    ok(cgnn_cluster_mean(N, F, groups, largest_group(m), dtype_code(input), input.data_ptr(), m[0].data_ptr<int32_t>(),
-                         m[1].data_ptr<int32_t>(), m[2].data_ptr<int32_t>(), count.data_ptr<int32_t>(), out.data_ptr(),
-                         ws.data_ptr(), bytes, current_stream(input)),
-       op);
+    Tensor out = member_sums(op, input, 0, nullptr, m, groups, false, false);
+    // the caller's counts need not be the lengths of the lists
+    ok(cgnn_cluster_divide(F, groups, dtype_code(input), count.data_ptr<int32_t>(), out.data_ptr(), current_stream(input)), op);
     return out;
 }
 
@@ -922,14 +1015,7 @@ Tensor cluster_reconstruct_backward(Tensor grad, Tensor index, Tensor output, in
     const int64_t N = grad.size(0), F = grad.size(1);
     if (grad.numel() == 0 || groups == 0) return torch::zeros({groups, F}, grad.options());
     auto m = members_or_build(op, members, index, groups);
-    Tensor out = torch::empty({groups, F}, grad.options());
-    const size_t bytes = cgnn_cluster_mean_workspace_bytes(N, F, groups, dtype_code(grad));
-    Tensor ws = torch::empty({(int64_t)std::max<size_t>(bytes, 1)}, grad.options().dtype(torch::kUInt8));
-    ok(cgnn_reconstruct_backward(N, F, groups, largest_group(m), dtype_code(grad), grad.data_ptr(), output.data_ptr(),
-                                 m[0].data_ptr<int32_t>(), m[1].data_ptr<int32_t>(), m[2].data_ptr<int32_t>(),
-                                 relu ? 1 : 0, out.data_ptr(), ws.data_ptr(), bytes, current_stream(grad)),
-       op);
-    return out;
+    return member_sums(op, grad, relu ? 1 : 0, relu ? output.data_ptr() : nullptr, m, groups, false, false);
 }
 
 // The ReLU form of cluster_reconstruct that also returns the sign of every output element as one
@@ -976,15 +1062,163 @@ Tensor cluster_reconstruct_backward_signs(Tensor grad, Tensor index, Tensor sign
     c10::hip::HIPGuardMasqueradingAsCUDA guard(grad.device());
     if (grad.numel() == 0 || groups == 0) return torch::zeros({groups, F}, grad.options());
     auto m = members_or_build(op, members, index, groups);
-    Tensor out = torch::empty({groups, F}, grad.options());
-    const size_t bytes = cgnn_cluster_mean_workspace_bytes(N, F, groups, dtype_code(grad));
-    Tensor ws = torch::empty({(int64_t)std::max<size_t>(bytes, 1)}, grad.options().dtype(torch::kUInt8));
-    ok(cgnn_reconstruct_backward_signs(N, F, groups, largest_group(m), dtype_code(grad), grad.data_ptr(),
-                                       reinterpret_cast<const uint32_t *>(signs.data_ptr<int32_t>()),
-                                       m[0].data_ptr<int32_t>(), m[1].data_ptr<int32_t>(), m[2].data_ptr<int32_t>(),
-                                       out.data_ptr(), ws.data_ptr(), bytes, current_stream(grad)),
+    return member_sums(op, grad, 2, signs.data_ptr<int32_t>(), m, groups, false, false);
+}
+
+// ------------------------------------------------------ the layers' autograd steps ----
+//
+// Native nodes, for the reason given at PropagateBackward.  They give first-order gradients (as the reference's
+// functions do): a gradient asked for with create_graph cannot be differentiated again and says so.
+
+torch::autograd::variable_list first_order(torch::autograd::variable_list grads, bool recorded) {
+    if (!recorded) return grads;
+    auto refuse = std::make_shared<torch::autograd::DelayedError>(
+        "trying to differentiate twice a function that has first-order gradients only (once_differentiable)", 1);
+    for (Tensor &g : grads)
+        if (g.defined()) g = (*refuse)({g.requires_grad() ? g : g.detach().requires_grad_()})[0];
+    return grads;
+}
+
+template <typename Node>
+std::shared_ptr<Node> node_over(const Tensor &a, const Tensor &b = Tensor()) {
+    std::shared_ptr<Node> node(new Node(), torch::autograd::deleteNode);
+    node->set_next_edges(b.defined() ? torch::autograd::collect_next_edges(a, b) : torch::autograd::collect_next_edges(a));
+    return node;
+}
+
+using Members = c10::optional<std::vector<Tensor>>;
+
+struct MeanBackward : torch::autograd::Node {
+    torch::autograd::SavedVariable index, counts;
+    Members members;
+    torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
+        if (!grads[0].defined()) return {Tensor()};
+        const bool recorded = at::GradMode::is_enabled();
+        Tensor out;
+        {
+            at::NoGradGuard no_grad;
+            out = cluster_mean_backward(grads[0].contiguous(), index.unpack(), counts.unpack(), members);
+        }
+        return first_order({out}, recorded);
+    }
+    void release_variables() override {
+        index.reset_data();
+        counts.reset_data();
+        members.reset();
+    }
+    std::string name() const override { return "ClusterMeanBackward"; }
+};
+
+void attach_mean(Tensor &reps, const Tensor &x, const Tensor &index, const Tensor &counts, const Members &members) {
+    if (!at::GradMode::is_enabled() || !x.requires_grad()) return;
+    auto node = node_over<MeanBackward>(x);
+    node->index = torch::autograd::SavedVariable(index, false);
+    node->counts = torch::autograd::SavedVariable(counts, false);
+    node->members = members;
+    torch::autograd::set_history(reps, node);
+}
+
+// Representatives of an assignment that is held: the means of x over its clusters (the counts are the
+// lengths of its lists).
+Tensor cluster_representatives(Tensor x, Tensor index, Tensor counts, std::vector<Tensor> members) {
+    const char *op = "cluster_mean";
+    Tensor reps;
+    {
+        at::AutoDispatchBelowADInplaceOrView plain;
+        Tensor rows = x.contiguous();
+        expect(op, rows, {{Role::Features, "input", &rows}, {Role::Ids, "index", &index}, {Role::Counts, "count", &counts}});
+        TORCH_CHECK(index.numel() == rows.size(0), op, ": ", rows.size(0), " rows but ", index.numel(), " cluster ids");
+        expect_members(op, members, index, counts.numel());
+        c10::hip::HIPGuardMasqueradingAsCUDA guard(rows.device());
+        reps = rows.numel() == 0 ? torch::zeros({counts.numel(), rows.size(1)}, rows.options())
+                                 : member_sums(op, rows, 0, nullptr, members, counts.numel(), true, false);
+    }
+    attach_mean(reps, x, index, counts, members);
+    return reps;
+}
+
+// A refresh: (representatives, ids, counts, active, member lists).
+std::tuple<Tensor, Tensor, Tensor, int64_t, std::vector<Tensor>> cluster_refresh(Tensor x, Tensor planes, int64_t bits) {
+    Assigned a;
+    {
+        at::AutoDispatchBelowADInplaceOrView plain;
+        a = assign(x.contiguous(), planes.contiguous(), bits, true);
+    }
+    attach_mean(a.reps, x, a.ids, a.counts, a.members);
+    return {a.reps, a.ids, a.counts, a.active, a.members};
+}
+
+// Column sums of a [rows, F] matrix: the gradient of a bias.
+Tensor column_sums(const Tensor &x) {
+    const char *op = "column_sums";
+    expect(op, x, {{Role::Features, "x", &x}});
+    const int64_t rows = x.size(0), F = x.size(1);
+    if (x.numel() == 0) return torch::zeros({F}, x.options());
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    Tensor out = torch::empty({F}, x.options());
+    int64_t arrivals = 0;
+    const size_t bytes = cgnn_column_sums_workspace_bytes(rows, F, dtype_code(x), &arrivals);
+    Tensor ws = torch::empty({(int64_t)std::max<size_t>(bytes, 1)}, x.options().dtype(torch::kUInt8));
+    Tensor counters = arrival_pool().get(arrivals, x);
+    ok(cgnn_column_sums(rows, F, dtype_code(x), x.data_ptr(), out.data_ptr(), ws.data_ptr(), bytes, counters.data_ptr<int32_t>(),
+                        current_stream(x)),
        op);
     return out;
+}
+
+struct ReconstructBackward : torch::autograd::Node {
+    torch::autograd::SavedVariable index, signs;  // signs: one bit per element, where the rows went through a ReLU
+    Members members;
+    int64_t groups = 0;
+    bool relu = false, with_bias = false;
+    torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
+        const size_t inputs = with_bias ? 2 : 1;
+        if (!grads[0].defined()) return torch::autograd::variable_list(inputs);
+        const bool recorded = at::GradMode::is_enabled();
+        torch::autograd::variable_list out;
+        {
+            at::NoGradGuard no_grad;
+            const Tensor d_rows = grads[0].contiguous(), ids = index.unpack();
+            // without a ReLU the operator does not read the rows it is given as output
+            out.push_back(relu ? cluster_reconstruct_backward_signs(d_rows, ids, signs.unpack(), groups, members)
+                               : cluster_reconstruct_backward(d_rows, ids, d_rows, groups, false, members));
+            if (with_bias) out.push_back(task_should_compute_output(1) ? column_sums(out[0]) : Tensor());
+        }
+        return first_order(std::move(out), recorded);
+    }
+    void release_variables() override {
+        index.reset_data();
+        signs.reset_data();
+        members.reset();
+    }
+    std::string name() const override { return "ReconstructBackward"; }
+};
+
+// rows[i] = act(reps[index[i]] + bias) with its gradients.  The ReLU mask of the gradient is kept as one bit
+// per element, written by the kernel that produces the rows (the reference keeps the rows themselves:
+// layer/CompressgnnReconstruct.py:16-22); without a ReLU nothing of the [N, F] output is needed again.
+Tensor reconstruct(Tensor reps, Tensor index, c10::optional<Tensor> bias, bool relu, Members members) {
+    Tensor rows, signs, ids;
+    {
+        at::AutoDispatchBelowADInplaceOrView plain;
+        ids = index.contiguous();
+        c10::optional<Tensor> b;
+        if (bias.has_value() && bias->defined()) b = bias->contiguous();
+        if (relu) std::tie(rows, signs) = cluster_reconstruct_signs(reps.contiguous(), ids, b, members);
+        else rows = cluster_reconstruct(reps.contiguous(), ids, b, false, members);
+    }
+    const bool with_bias = bias.has_value() && bias->defined();
+    if (at::GradMode::is_enabled() && (reps.requires_grad() || (with_bias && bias->requires_grad()))) {
+        auto node = with_bias ? node_over<ReconstructBackward>(reps, *bias) : node_over<ReconstructBackward>(reps);
+        node->index = torch::autograd::SavedVariable(ids, false);
+        if (relu) node->signs = torch::autograd::SavedVariable(signs, false);
+        node->members = std::move(members);
+        node->groups = reps.size(0);
+        node->relu = relu;
+        node->with_bias = with_bias;
+        torch::autograd::set_history(rows, node);
+    }
+    return rows;
 }
 
 // (colptr, row, value) of a block held as int64 tensors on a GPU: the CSR of its transpose,
@@ -1208,6 +1442,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("signs"), py::arg("groups"), py::arg("members") = py::none());
     m.def("csr_transpose", &csr_transpose, "CSR -> CSC of an int64 block on the GPU, SparseTensor.csc() order",
           py::arg("rowptr"), py::arg("col"), py::arg("value"), py::arg("cols"));
+    m.def("cluster_refresh", &cluster_refresh,
+          "(representatives, ids, counts, active, [offsets, perm, sorted_id]) of an assignment refresh, with the gradient of "
+          "the representatives", py::arg("x"), py::arg("planes"), py::arg("bits"));
+    m.def("cluster_representatives", &cluster_representatives, "means over the clusters of an assignment, with their gradient",
+          py::arg("x"), py::arg("index"), py::arg("counts"), py::arg("members"));
+    m.def("reconstruct", &reconstruct, "act(reps[index] + bias) with its gradients", py::arg("reps"), py::arg("index"),
+          py::arg("bias"), py::arg("relu"), py::arg("members") = py::none());
+    m.def("column_sums", &column_sums, "sum over the rows of a matrix");
     m.def("propagate", &propagate, "plan.forward(x) with plan.backward as its gradient", py::arg("plan"), py::arg("x"));
     m.def("version", []() { return std::string(cgnn_version()); });
     py::class_<DeviceCsr, std::shared_ptr<DeviceCsr>>(m, "DeviceCsr")

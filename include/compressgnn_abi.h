@@ -283,10 +283,36 @@ int cgnn_cluster_members(int64_t N, int64_t groups, const int64_t *ids, int32_t 
  * the number of groups, summary[1] = the size of the largest group.  counts needs room for min(N, 2^bits)+1 entries and offsets for one more; entries
  * beyond active+1 (active+2) are left untouched.  Replaces cluster_kernel.cu:143-150 and
  * the atomics of hash_ids (cluster_kernel.cu:41-59). */
+/* Up to cgnn_lsh_group_small_rows() rows the whole of it is one launch that needs no workspace and writes the
+ * summary with plain stores, so that it may lie in pinned host memory. */
+int64_t cgnn_lsh_group_small_rows(void);
 size_t cgnn_lsh_group_workspace_bytes(int64_t N, int bits);
 int cgnn_lsh_group(int64_t N, int bits, const int32_t *raw_code, int64_t *ids, int32_t *offsets,
                    int32_t *perm, int32_t *sorted_id, int32_t *counts, int32_t *summary,
                    void *workspace, size_t workspace_bytes, cgnn_stream_t stream);
+
+/* The sums over the members of every group in one launch, the form the layers use: sums[g,:] = the sum over
+ * members i of group g of X[i,:] -- divided by their number if mean is set; mask 1: elements dropped where
+ * M[N x F] <= 0, mask 2: where a bit of M[N x ceil(F / 32)] is clear (as in cgnn_reconstruct_backward and its
+ * _signs form).  A group of at most 64 members is summed in ascending order; a larger one in an order that
+ * depends on the sizes alone.  first_group_empty: group 0 and no other has no members; groups may then be
+ * an upper bound (rows behind the last group are left untouched), which spares the caller the host read before it.
+ * arrivals: counters (as many as the size query reports), zero before and after the call, as in cgnn_csr.
+ * N > 0 and F > 0. */
+size_t cgnn_cluster_sums_workspace_bytes(int64_t N, int64_t F, int64_t groups, int dtype, int64_t *arrivals);
+int cgnn_cluster_sums(int64_t N, int64_t F, int64_t groups, int dtype, const void *X, int mask, const void *M,
+                      const int32_t *offsets, const int32_t *perm, const int32_t *sorted_id, int mean,
+                      int first_group_empty, void *sums, void *workspace, size_t workspace_bytes, int32_t *arrivals,
+                      cgnn_stream_t stream);
+
+/* sums[g,:] /= max(counts[g], 1). */
+int cgnn_cluster_divide(int64_t F, int64_t groups, int dtype, const int32_t *counts, void *sums, cgnn_stream_t stream);
+
+/* out[f] = sum over the rows r of X[r,f] (the gradient of a bias), in a fixed order; rows > 0 and F > 0;
+ * arrivals as above. */
+size_t cgnn_column_sums_workspace_bytes(int64_t rows, int64_t F, int dtype, int64_t *arrivals);
+int cgnn_column_sums(int64_t rows, int64_t F, int dtype, const void *X, void *out, void *workspace, size_t workspace_bytes,
+                     int32_t *arrivals, cgnn_stream_t stream);
 
 /* reps[g,:] = (sum over members i of group g, ascending i, of X[i,:]) / max(counts[g],1).
  * max_members: size of the largest group if the caller knows it (it decides whether the

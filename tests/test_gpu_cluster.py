@@ -373,3 +373,40 @@ def test_reference_signature_operators_read_the_host_once_per_index():
             rt.cluster_reconstruct(hidden, foreign, bias, True)
         with pytest.raises(RuntimeError, match="outside"):
             rt.cluster_mean(x, foreign, counts)
+
+
+@pytest.mark.parametrize("bits", [0, 1, 8, 9, 16, 20, 30])
+@pytest.mark.parametrize("n", [1, 63, 64, 1025, 8191, 8192, 8193])
+def test_refresh_through_the_layers_entry(n, bits):
+    """cluster_refresh on both sides of the row count up to which one workgroup groups the rows: ids, sizes and
+    member lists against the oracle, the representatives against float64 means, and the same means from
+    the lists it returned."""
+    import compressgnn_runtime as rt
+    rng = np.random.default_rng(n + bits)
+    x = (rng.standard_normal((n, 12)) + 3.0 * rng.integers(0, 3, (n, 1))).astype(np.float32)
+    planes = rng.standard_normal((12, bits)).astype(np.float32)
+    want_ids, want_counts, want_active = oracle.assign(x, planes, bits)
+    X = torch.from_numpy(x).to(DEV)
+    reps, ids, counts, active, lists = rt.cluster_refresh(X, torch.from_numpy(planes).to(DEV), bits)
+    assert active == want_active and np.array_equal(ids.cpu().numpy(), want_ids)
+    assert np.array_equal(counts.cpu().numpy(), want_counts) and int(lists[3]) == want_counts.max()
+    order = np.argsort(want_ids, kind="stable")
+    assert np.array_equal(lists[1].cpu().numpy(), order) and np.array_equal(lists[2].cpu().numpy(), want_ids[order])
+    assert np.array_equal(lists[0].cpu().numpy(), np.concatenate([[0], np.cumsum(want_counts)]))
+    sums = np.zeros((active + 1, 12))
+    np.add.at(sums, want_ids, x.astype(np.float64))
+    np.testing.assert_allclose(reps.cpu().numpy(), sums / np.maximum(want_counts, 1)[:, None], rtol=1e-5, atol=2e-5)
+    assert torch.equal(rt.cluster_representatives(X, ids, counts, lists), reps)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("rows,width", [(1, 1), (63, 16), (64, 17), (65, 20), (4097, 64), (5000, 68), (20011, 130)])
+def test_column_sums(rows, width, dtype):
+    """One stretch and many, widths of packs and of single features, twice (the counters return to zero)."""
+    import compressgnn_runtime as rt
+    x = torch.randn(rows, width, dtype=dtype, device=DEV)
+    want = x.double().sum(0)
+    tol = 1e-12 if dtype == torch.float64 else 1e-6
+    for _ in range(2):
+        got = rt.column_sums(x).double()
+        assert float((got - want).abs().max()) <= tol * max(1.0, float(x.double().abs().sum(0).max()))
