@@ -24,7 +24,7 @@ EXPORTS = [
     "cgnn_compress_batch_workspace_bytes", "cgnn_compress_csr_batch_device",
     "cgnn_lsh_scan_workspace_bytes", "cgnn_lsh_hash", "cgnn_lsh_scan", "cgnn_lsh_finish",
     "cgnn_lsh_group_workspace_bytes", "cgnn_lsh_group", "cgnn_lsh_group_small_rows", "cgnn_cluster_sums_workspace_bytes",
-    "cgnn_cluster_sums", "cgnn_cluster_divide", "cgnn_column_sums_workspace_bytes", "cgnn_column_sums",
+    "cgnn_cluster_sums", "cgnn_column_sums_workspace_bytes", "cgnn_column_sums",
     "cgnn_cluster_members_workspace_bytes", "cgnn_cluster_members",
     "cgnn_cluster_mean_workspace_bytes", "cgnn_cluster_mean", "cgnn_cluster_mean_backward",
     "cgnn_reconstruct", "cgnn_reconstruct_backward", "cgnn_sign_words", "cgnn_reconstruct_signs",

@@ -10,10 +10,10 @@
 namespace cgnn {
 
 int spmm_members(const cgnn_csr *A, int dtype, const void *X, const void *M, void *Y, int64_t F,
-                 int mask, void *ws, size_t ws_bytes, hipStream_t stream);
+                 int mask, void *ws, size_t ws_bytes, hipStream_t stream, bool *mean = nullptr);
 
-int spmm_member_runs(const cgnn_csr *A, int dtype, const void *X, const void *M, void *Y, int64_t F, int mask, bool mean,
-                     bool first_row_empty, int32_t *arrivals, void *ws, size_t ws_bytes, hipStream_t stream);
+int spmm_member_runs(const cgnn_csr *A, int dtype, const void *X, const void *M, void *Y, int64_t F, int mask, int32_t *arrivals,
+                     void *ws, size_t ws_bytes, hipStream_t stream);
 size_t spmm_member_runs_bytes(const cgnn_csr *A, int64_t F, int dtype, int64_t *arrivals);
 
 namespace {
@@ -977,14 +977,15 @@ int launch_gather(const GatherArgs<T> &a, hipStream_t stream) {
     return launch_gather_lpr<T, 1, OP>(a, stream);
 }
 
-// reps[g, :] /= max(counts[g], 1), VEC features per thread (a row holds `slots` such pieces).
+// reps[g, :] /= max(counts[g], 1) (counts == NULL: the length of the group's list), VEC features per thread (a row holds `slots` such pieces).
 template <typename T, int VEC>
-__global__ __launch_bounds__(kBlock) void divide_counts_kernel(T *reps, const int32_t *counts, int64_t total_slots,
+__global__ __launch_bounds__(kBlock) void divide_counts_kernel(T *reps, const int32_t *counts,
+                                                              const int32_t *offsets, int64_t total_slots,
                                                               uint32_t slots) {
     const bool narrow = total_slots < ((int64_t)1 << 32);  // the row of a piece by a 32-bit division
     for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < total_slots; i += (int64_t)gridDim.x * kBlock) {
         const int64_t g = narrow ? (int64_t)((uint32_t)i / slots) : i / (int64_t)slots;
-        const T c = (T)max(counts[g], 1);
+        const T c = (T)max(counts ? counts[g] : offsets[g + 1] - offsets[g], 1);
         LPack<T, VEC> v = *reinterpret_cast<const LPack<T, VEC> *>(reps + i * VEC);
 #pragma unroll
         for (int k = 0; k < VEC; ++k) v.v[k] = v.v[k] / c;
@@ -1214,7 +1215,7 @@ extern "C" size_t cgnn_cluster_mean_workspace_bytes(int64_t N, int64_t F, int64_
 }
 
 template <typename T>
-static int divide_counts(void *reps, const int32_t *counts, int64_t groups, int64_t F,
+static int divide_counts(void *reps, const int32_t *counts, const int32_t *offsets, int64_t groups, int64_t F,
                          hipStream_t stream) {
     if (groups * F == 0) return CGNN_OK;
     constexpr int WIDE = 16 / sizeof(T);
@@ -1225,10 +1226,10 @@ static int divide_counts(void *reps, const int32_t *counts, int64_t groups, int6
     if (blocks > 65536) blocks = 65536;
     if (wide)
         hipLaunchKernelGGL((divide_counts_kernel<T, WIDE>), dim3((unsigned)blocks), dim3(kBlock), 0, stream,
-                           static_cast<T *>(reps), counts, total, (uint32_t)slots);
+                           static_cast<T *>(reps), counts, offsets, total, (uint32_t)slots);
     else
         hipLaunchKernelGGL((divide_counts_kernel<T, 1>), dim3((unsigned)blocks), dim3(kBlock), 0, stream,
-                           static_cast<T *>(reps), counts, total, (uint32_t)slots);
+                           static_cast<T *>(reps), counts, offsets, total, (uint32_t)slots);
     return check_launch("divide_counts");
 }
 
@@ -1239,13 +1240,15 @@ extern "C" int cgnn_cluster_mean(int64_t N, int64_t F, int64_t groups, int64_t m
     CGNN_REQUIRE(N >= 0 && F >= 0 && groups >= 1, "cgnn_cluster_mean: bad size");
     CGNN_REQUIRE(dtype == CGNN_F32 || dtype == CGNN_F64, "cgnn_cluster_mean: dtype must be f32 or f64");
     if (F == 0) return CGNN_OK;
-    CGNN_REQUIRE(offsets && counts && reps, "cgnn_cluster_mean: null array");
+    CGNN_REQUIRE(offsets && reps, "cgnn_cluster_mean: null array");
     CGNN_REQUIRE(N == 0 || (X && perm && sorted_id), "cgnn_cluster_mean: null array");
     cgnn_csr A = members_csr(N, groups, offsets, perm, sorted_id, max_members);
-    int rc = spmm_members(&A, dtype, X, nullptr, reps, F, 0, workspace, workspace_bytes, stream);
-    if (rc != CGNN_OK) return rc;
-    if (dtype == CGNN_F32) return divide_counts<float>(reps, counts, groups, F, stream);
-    return divide_counts<double>(reps, counts, groups, F, stream);
+    // counts == NULL: the lengths of the lists, which the sums are divided by where a row is finished
+    bool mean = counts == nullptr;
+    int rc = spmm_members(&A, dtype, X, nullptr, reps, F, 0, workspace, workspace_bytes, stream, &mean);
+    if (rc != CGNN_OK || mean) return rc;
+    if (dtype == CGNN_F32) return divide_counts<float>(reps, counts, offsets, groups, F, stream);
+    return divide_counts<double>(reps, counts, offsets, groups, F, stream);
 }
 
 extern "C" size_t cgnn_cluster_sums_workspace_bytes(int64_t N, int64_t F, int64_t groups, int dtype, int64_t *arrivals) {
@@ -1259,26 +1262,17 @@ extern "C" size_t cgnn_cluster_sums_workspace_bytes(int64_t N, int64_t F, int64_
 }
 
 extern "C" int cgnn_cluster_sums(int64_t N, int64_t F, int64_t groups, int dtype, const void *X, int mask, const void *M,
-                                 const int32_t *offsets, const int32_t *perm, const int32_t *sorted_id, int mean,
-                                 int first_group_empty, void *sums, void *workspace, size_t workspace_bytes,
-                                 int32_t *arrivals, cgnn_stream_t stream) {
+                                 const int32_t *offsets, const int32_t *perm, const int32_t *sorted_id, void *sums,
+                                 void *workspace, size_t workspace_bytes, int32_t *arrivals, cgnn_stream_t stream) {
     CGNN_REQUIRE(N > 0 && F > 0 && groups > 0 && N < INT32_MAX - 65536, "cgnn_cluster_sums: bad size");
     CGNN_REQUIRE(dtype == CGNN_F32 || dtype == CGNN_F64, "cgnn_cluster_sums: dtype must be f32 or f64");
-    CGNN_REQUIRE(mask >= 0 && mask <= 2 && !(mask && mean), "cgnn_cluster_sums: a mask (0, 1 or 2) or means, not both");
+    CGNN_REQUIRE(mask >= 0 && mask <= 2, "cgnn_cluster_sums: mask must be 0, 1 or 2");
     CGNN_REQUIRE(X && offsets && perm && sorted_id && sums && arrivals && (mask == 0 || M), "cgnn_cluster_sums: null array");
     cgnn_csr A = members_csr(N, groups, offsets, perm, sorted_id);
-    return spmm_member_runs(&A, dtype, X, M, sums, F, mask, mean != 0, first_group_empty != 0, arrivals, workspace,
-                            workspace_bytes, stream);
-}
-
-extern "C" int cgnn_cluster_divide(int64_t F, int64_t groups, int dtype, const int32_t *counts, void *sums,
-                                   cgnn_stream_t stream) {
-    CGNN_REQUIRE(F >= 0 && groups >= 0, "cgnn_cluster_divide: bad size");
-    CGNN_REQUIRE(dtype == CGNN_F32 || dtype == CGNN_F64, "cgnn_cluster_divide: dtype must be f32 or f64");
-    if (F == 0 || groups == 0) return CGNN_OK;
-    CGNN_REQUIRE(counts && sums, "cgnn_cluster_divide: null array");
-    if (dtype == CGNN_F32) return divide_counts<float>(sums, counts, groups, F, stream);
-    return divide_counts<double>(sums, counts, groups, F, stream);
+    int64_t n = 0;
+    spmm_member_runs_bytes(&A, F, dtype, &n);
+    if (n == 0) return fail(CGNN_EUNSUPPORTED, "cgnn_cluster_sums: too many rows for this form (the size query reports no counters)");
+    return spmm_member_runs(&A, dtype, X, M, sums, F, mask, arrivals, workspace, workspace_bytes, stream);
 }
 
 // Rows per workgroup of column_sums_kernel.

@@ -95,8 +95,8 @@ struct SpmmArgs {
     int32_t seg_nnz;
     int32_t split;
     int32_t accumulate;
-    // Runs per workgroup of the nnz kernel that wrote carry_row/carry (its carries are
-    // merged per workgroup: see kMerged), or 1 for the plain list a reduction level writes.
+    // Runs whose carries the nnz kernel that wrote carry_row/carry has merged (see kMerged and
+    // merged_runs), or 1 for the plain list a reduction level writes.
     int32_t merge_stride;
     int32_t stretch_log2;  // log2 of the workgroups per XCD stretch (see logical_block); set at launch
     int32_t blocks;        // workgroups with work (the grid rounds this up to a multiple of kXcds)
@@ -109,7 +109,7 @@ struct SpmmArgs {
     int32_t wg_len;             // workgroup runs: non-zeros per workgroup (run_start is the table of cgnn_csr.wg_runs, or NULL)
     int32_t keep;               // ... a row of at most this many entries is never divided, whatever the lengths
     int32_t find_empty;         // ... the rows without entries are found from rowptr, not from a list
-    int32_t mean;               // ... every row is divided by its number of entries
+    int32_t mean;               // MODE_UNIT, plain runs: every row is divided by its number of entries
 };
 
 // An entry of the table of workgroup runs is the first non-zero of a run, with this bit set when the row
@@ -571,9 +571,6 @@ __device__ __forceinline__ void join_rows(const SpmmArgs<T> &a, int block, int l
     };
     auto store_row = [&](int row, const Pack<T, VEC>(&sum)[TILES]) {
         T *y = a.Y + (int64_t)row * a.F;
-        T divisor = T(1);
-        if constexpr (MODE == MODE_UNIT)
-            if (a.mean) divisor = (T)(a.rowptr[row + 1] - a.rowptr[row]);  // blocks without a row map
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
             if (foff[t] < 0) continue;
@@ -584,9 +581,6 @@ __device__ __forceinline__ void join_rows(const SpmmArgs<T> &a, int block, int l
 #pragma unroll
                     for (int i = 0; i < VEC; ++i) o.v[i] = base.v[i] + o.v[i];
                 }
-            if constexpr (MODE == MODE_UNIT)
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) o.v[i] = o.v[i] / divisor;
             store_pack<T, VEC>(y + foff[t], o);
         }
     };
@@ -710,6 +704,8 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
     }
     // e0 >= e1 inside the list cannot happen for a well-formed CSR
     const bool active = e0 < e1;
+    // means: a row that began before the run is divided by the pass that adds its carries up
+    const bool began_before = WGRUNS == WGRUNS_NONE && MODE == MODE_UNIT && a.mean && active && e0 > 0 && a.rowidx[e0 - 1] == a.rowidx[e0];
     int64_t foff[TILES];
     feature_offsets<VEC, LPR, TILES>(a.F, lane, foff);
     Acc<T, VEC, TILES, MODE> acc;
@@ -731,7 +727,7 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
             }
         }
         write_row<T, VEC, TILES, MODE>(a.Y, a.F, y_row, foff, acc, a.accumulate,
-                                       WGRUNS == WGRUNS_COMPUTED && MODE == MODE_UNIT && a.mean ? (T)(end - row_e0) : T(1));
+                                       MODE == MODE_UNIT && a.mean && !(began_before && row_e0 == e0) ? (T)(end - row_e0) : T(1));
     };
     // the names of rows: see below
     constexpr bool kNamesRowsOfY = !(MODE == MODE_DUAL && VEC * LPR * sizeof(T) >= 512);
@@ -894,8 +890,8 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                                             wg_carry, wg_head);
         return;
     }
-    // The carries of one row are added per workgroup: the first of its lane groups that
-    // carries the row takes those of the groups behind it, in ascending order.
+    // The carries of one row are added per workgroup (or per merge_stride lane groups of it): the first lane
+    // group that carries the row takes those of the groups behind it, in ascending order.
     Pack<T, VEC> part[TILES];
 #pragma unroll
     for (int t = 0; t < TILES; ++t)
@@ -910,10 +906,11 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
     if (seg >= a.nseg) return;
     int mark = kNoCarry;
     if (continues) {
-        const bool first = grp == 0 || wg_row[grp - 1] != cur;
+        const int merged = a.merge_stride;  // at most GPB, a power of two
+        const bool first = (grp & (merged - 1)) == 0 || wg_row[grp - 1] != cur;
         mark = first ? cur : kMerged;
         if (first) {
-            for (int g = grp + 1; g < GPB && wg_row[g] == cur; ++g)
+            for (int g = grp + 1; (g & (merged - 1)) != 0 && wg_row[g] == cur; ++g)
 #pragma unroll
                 for (int t = 0; t < TILES; ++t) {
                     const Pack<T, VEC> o = wg_carry[t][g * LPR + lane];
@@ -1133,6 +1130,11 @@ __global__ __launch_bounds__(kBlock) void spmm_fixup_kernel(SpmmArgs<T> a) {
             Pack<T, VEC> o = load_pack<T, VEC>(y);
 #pragma unroll
             for (int i = 0; i < VEC; ++i) o.v[i] = o.v[i] + acc.v[i];
+            if (MERGED && a.mean) {
+                const T n = (T)(row_end - a.rowptr[row]);
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) o.v[i] = o.v[i] / n;
+            }
             store_pack<T, VEC>(y, o);
         }
     }
@@ -1252,6 +1254,22 @@ Shape pick_shape(int64_t F, bool runs) {
     s.tiles = (lpr == 64 && slots > 64 && sizeof(T) == 4) ? 2 : 1;
     s.grid_y = (int)ceil_div(slots, (int64_t)s.lpr * s.tiles);
     return s;
+}
+
+// How many consecutive runs of the nnz schedule merge their carries before these reach memory: part of the
+// order in which a long row is summed, and so a function of the width alone, not of the lane layout (a workgroup
+// of the layout in use holds as many runs or a multiple of them).  What divides the rows of an assignment into
+// clusters differently at the last bit flips ReLUs behind their means.
+template <typename T>
+int merged_runs(int64_t F) {
+    int64_t vec = 1;
+    if (sizeof(T) == 4) {
+        vec = F % 4 == 0 ? 4 : (F % 2 == 0 ? 2 : 1);
+        while (vec > 1 && F / vec < 16) vec /= 2;
+    }
+    int lpr = pow2_ceil(F / vec);
+    if (vec != 4) lpr = lpr <= 4 ? 4 : (lpr <= 16 ? 16 : 64);
+    return kBlock / (lpr < 4 ? 4 : (lpr > 64 ? 64 : lpr));
 }
 
 // The layout of the nnz schedule for a feature width.
@@ -1460,9 +1478,11 @@ int wg_run_len(const cgnn_csr *A, int groups) {
     return (int)(fill < 8 ? (longest < 8 ? longest : 8) : (fill > longest ? longest : fill));
 }
 
+// mean (may be NULL; MODE_UNIT): whether the rows are wanted divided by their numbers of entries; false on return
+// if that is left to the caller (rows so long that their carries go through the reduction levels).
 template <typename T>
 int spmm_typed(const cgnn_csr *A, const void *X, const void *X1, int64_t split, const void *M, void *Y, int64_t F,
-               int accumulate, int kernel, int mode, void *ws, size_t ws_bytes, hipStream_t stream) {
+               int accumulate, int kernel, int mode, void *ws, size_t ws_bytes, hipStream_t stream, bool *mean = nullptr) {
     if (A->rows == 0 || F == 0) return CGNN_OK;
     if (mode != MODE_DUAL) split = INT32_MAX;  // every column comes from X
     SpmmArgs<T> a = make_args<T>(A, X, X1, split, M, Y, F, accumulate);
@@ -1485,8 +1505,8 @@ int spmm_typed(const cgnn_csr *A, const void *X, const void *X1, int64_t split, 
     if (A->nnz > 0 && A->rowidx == nullptr) return fail(CGNN_EINVAL, "spmm: nnz schedule needs rowidx");
     // the lane layout decides how many runs a workgroup merges
     const Shape s = pick_shape<T>(F, true);
-    const int runs_per_workgroup = kBlock / s.lpr;
-    if (may_choose && A->wg_runs != nullptr && A->arrivals != nullptr && A->wg_groups == runs_per_workgroup && A->nnz > 0) {
+    const int lane_groups = kBlock / s.lpr, runs_per_workgroup = merged_runs<T>(F);
+    if (may_choose && A->wg_runs != nullptr && A->arrivals != nullptr && A->wg_groups == lane_groups && A->nnz > 0) {
         const int64_t workgroups = ceil_div(A->nnz, A->wg_len);
         const size_t need = wg_piece_bytes(workgroups, F, sizeof(T));
         if (ws == nullptr || ws_bytes < need) {
@@ -1496,7 +1516,7 @@ int spmm_typed(const cgnn_csr *A, const void *X, const void *X1, int64_t split, 
         a.run_start = A->wg_runs;
         a.arrivals = A->arrivals;
         a.wg_len = A->wg_len;
-        a.nseg = (int32_t)(workgroups * runs_per_workgroup);
+        a.nseg = (int32_t)(workgroups * lane_groups);
         a.carry = static_cast<T *>(ws);
         a.empty_rows = A->empty_rows;
         a.n_empty_rows = A->n_empty_rows;
@@ -1505,6 +1525,8 @@ int spmm_typed(const cgnn_csr *A, const void *X, const void *X1, int64_t split, 
     const int seg = seg_len(A);
     const int64_t nseg = ceil_div(A->nnz, seg);
     const CarryLevels levels = carry_levels(nseg, F, sizeof(T), wants_levels(A, seg, runs_per_workgroup));
+    if (mean != nullptr) *mean = *mean && levels.count == 1;
+    a.mean = mean != nullptr && *mean;
     if (nseg > 0 && (ws == nullptr || ws_bytes < levels.total)) {
         set_error("spmm: workspace of %zu bytes needed, %zu given", levels.total, ws_bytes);
         return CGNN_EWORKSPACE;
@@ -1641,24 +1663,22 @@ __global__ void compose_columns_kernel(const int32_t *__restrict__ col, int64_t 
 
 }  // namespace
 
-// Entry used by the cluster reductions (unit values; mask: 0 none, 1 the rows of M, where M <= 0 drops
+// Entry used by the cluster reductions (mean: as for spmm_typed; unit values; mask: 0 none, 1 the rows of M, where M <= 0 drops
 // the element, 2 M holds ceil(F / 32) words of bits per row, where a clear bit drops it).
 int spmm_members(const cgnn_csr *A, int dtype, const void *X, const void *M, void *Y, int64_t F,
-                 int mask, void *ws, size_t ws_bytes, hipStream_t stream) {
+                 int mask, void *ws, size_t ws_bytes, hipStream_t stream, bool *mean) {
     const int mode = mask == 2 ? MODE_SIGN_MASK : (mask == 1 ? MODE_RELU_MASK : MODE_UNIT);
     if (dtype == CGNN_F32)
-        return spmm_typed<float>(A, X, nullptr, 0, M, Y, F, 0, CGNN_SPMM_NNZ, mode, ws, ws_bytes, stream);
+        return spmm_typed<float>(A, X, nullptr, 0, M, Y, F, 0, CGNN_SPMM_NNZ, mode, ws, ws_bytes, stream, mean);
     if (dtype == CGNN_F64)
-        return spmm_typed<double>(A, X, nullptr, 0, M, Y, F, 0, CGNN_SPMM_NNZ, mode, ws, ws_bytes, stream);
+        return spmm_typed<double>(A, X, nullptr, 0, M, Y, F, 0, CGNN_SPMM_NNZ, mode, ws, ws_bytes, stream, mean);
     return fail(CGNN_EUNSUPPORTED, "spmm: dtype must be f32 or f64");
 }
 
-// The same sums in one launch (workgroup runs): mask as above; mean: divided by the number of members;
-// first_row_empty: row 0 is the only one without members (offsets[0] = 0 is then the list of the empty rows, and
-// A->rows may be a bound on the number of rows).  A member list of at most kDefaultSeg rows is summed in
-// ascending order, undivided, like there.
-int spmm_member_runs(const cgnn_csr *A, int dtype, const void *X, const void *M, void *Y, int64_t F, int mask, bool mean,
-                     bool first_row_empty, int32_t *arrivals, void *ws, size_t ws_bytes, hipStream_t stream) {
+// The same sums in one launch (workgroup runs): mask as above.  A member list of at most kDefaultSeg rows is
+// summed in ascending order, undivided, like there; a longer one in another order.
+int spmm_member_runs(const cgnn_csr *A, int dtype, const void *X, const void *M, void *Y, int64_t F, int mask, int32_t *arrivals,
+                     void *ws, size_t ws_bytes, hipStream_t stream) {
     auto run = [&](auto zero) {
         typedef decltype(zero) T;
         const Shape s = pick_shape<T>(F, true);
@@ -1676,18 +1696,22 @@ int spmm_member_runs(const cgnn_csr *A, int dtype, const void *X, const void *M,
         a.keep = kDefaultSeg;
         a.nseg = (int32_t)(workgroups * groups);
         a.carry = static_cast<T *>(ws);
-        a.find_empty = !first_row_empty;
-        a.empty_rows = A->rowptr;
-        a.n_empty_rows = first_row_empty ? 1 : 0;
-        a.mean = mean;
+        a.find_empty = 1;
         return launch<T>(KIND_NNZ, mask == 2 ? MODE_SIGN_MASK : (mask == 1 ? MODE_RELU_MASK : MODE_UNIT), s, a, a.nseg, stream);
     };
     return dtype == CGNN_F32 ? run(0.0f) : run(0.0);
 }
 
+// 0 arrivals: the plain runs and their pass are the better form.  That is where the launch fills the card
+// several times over: a workgroup finds its runs by four dependent loads from memory and its lane groups wait for each
+// other at the end, which cost 2.4 M rows of 256 features 35 us of 553, more than the pass (14 us); where the
+// card is filled once or less the pass and its launch cost more (10^6 rows of 16 features: 37 us either way,
+// 2,708 rows: 12 us for 18).
 size_t spmm_member_runs_bytes(const cgnn_csr *A, int64_t F, int dtype, int64_t *arrivals) {
     const Shape s = shape_of(F, dtype);
     const int groups = kBlock / s.lpr;
+    *arrivals = 0;
+    if (A->nnz > kResidentWorkgroups * groups * kDefaultSeg) return 0;
     const int64_t workgroups = ceil_div(A->nnz, wg_run_len(A, groups) * groups);
     *arrivals = workgroups * s.grid_y;
     return wg_piece_bytes(workgroups, F, dtype == CGNN_F64 ? 8 : 4);

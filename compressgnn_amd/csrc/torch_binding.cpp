@@ -686,6 +686,8 @@ std::vector<Tensor> cluster_workspace(Tensor input, int64_t bits) {
 // is at most min(N, 2^bits): every kernel runs on buffers of that bound, so the device
 // never waits for the host; the one scalar read of a refresh (cluster_kernel.cu:146-147)
 // comes last and only trims the views.
+int64_t largest_group(const std::vector<Tensor> &m) { return m.size() == 4 ? m[3].item<int64_t>() : 0; }
+
 struct Assigned {
     Tensor ids, counts, reps;
     int64_t active = 0;
@@ -693,11 +695,13 @@ struct Assigned {
 };
 
 // with_reps: the means of the rows over the clusters as well, launched before the host read where the buffer
-// for all clusters there could be is small (kSmallReps elements; the rows behind the last cluster stay unused).
+// for all clusters there could be is small (kSmallReps elements; the rows behind the last cluster stay unused) and
+// no cluster can be so large that its size, which is not known yet, would change how it is summed.
 constexpr int64_t kSmallReps = int64_t(1) << 22;
+constexpr int64_t kSmallClusters = int64_t(1) << 16;
 
-Tensor member_sums(const char *op, const Tensor &rows, int mask, const void *M, const std::vector<Tensor> &m, int64_t groups,
-                   bool mean, bool first_group_empty);
+Tensor member_means(const char *op, const Tensor &rows, const Tensor *counts, const std::vector<Tensor> &m, int64_t groups,
+                    int64_t largest);
 
 Assigned assign(Tensor input, Tensor planes, int64_t bits, bool with_reps) {
     const char *op = "cluster_assign";
@@ -734,8 +738,8 @@ Assigned assign(Tensor input, Tensor planes, int64_t bits, bool with_reps) {
                       stream),
        "lsh_group");
     const std::vector<Tensor> wide_lists = {offsets, perm, sorted_id};
-    const bool early = with_reps && F > 0 && (cap + 1) * F <= kSmallReps;
-    if (early) a.reps = member_sums("cluster_mean", input, 0, nullptr, wide_lists, cap + 1, true, true);
+    const bool early = with_reps && F > 0 && (cap + 1) * F <= kSmallReps && N <= kSmallClusters;
+    if (early) a.reps = member_means("cluster_mean", input, nullptr, wide_lists, cap + 1, N);
     // the one host read of a refresh
     if (direct) {
         TORCH_CHECK(hipStreamSynchronize(reinterpret_cast<hipStream_t>(stream)) == hipSuccess, op, ": the stream reported an error");
@@ -746,7 +750,7 @@ Assigned assign(Tensor input, Tensor planes, int64_t bits, bool with_reps) {
     a.counts = counts.narrow(0, 0, a.active + 1);
     a.members = {offsets.narrow(0, 0, a.active + 2), perm, sorted_id, host_scalar(summary.data_ptr<int32_t>()[1])};
     if (early) a.reps = a.reps.narrow(0, 0, a.active + 1);
-    else if (with_reps && F > 0) a.reps = member_sums("cluster_mean", input, 0, nullptr, a.members, a.active + 1, true, true);
+    else if (with_reps && F > 0) a.reps = member_means("cluster_mean", input, nullptr, a.members, a.active + 1, largest_group(a.members));
     else if (with_reps) a.reps = torch::zeros({a.active + 1, F}, input.options());
     return a;
 }
@@ -903,19 +907,46 @@ std::vector<Tensor> members_or_build(const char *op, const c10::optional<std::ve
     return known;
 }
 
-// Sums (or means) over the members of every group, [groups, F]; rows has at least one element.
-Tensor member_sums(const char *op, const Tensor &rows, int mask, const void *M, const std::vector<Tensor> &m, int64_t groups,
-                   bool mean, bool first_group_empty) {
+// Sums over the members of every group, [groups, F]; rows has at least one element.  mask as in cgnn_cluster_sums.
+Tensor member_sums(const char *op, const Tensor &rows, int mask, const void *M, const std::vector<Tensor> &m, int64_t groups) {
+    const int64_t N = rows.size(0), F = rows.size(1);
+    const int dtype = dtype_code(rows);
+    const int32_t *offsets = m[0].data_ptr<int32_t>(), *perm = m[1].data_ptr<int32_t>(), *sorted_id = m[2].data_ptr<int32_t>();
+    const auto stream = current_stream(rows);
+    Tensor out = torch::empty({groups, F}, rows.options());
+    int64_t arrivals = 0;
+    size_t bytes = cgnn_cluster_sums_workspace_bytes(N, F, groups, dtype, &arrivals);
+    if (arrivals == 0) bytes = cgnn_cluster_mean_workspace_bytes(N, F, groups, dtype);
+    Tensor ws = torch::empty({(int64_t)std::max<size_t>(bytes, 1)}, rows.options().dtype(torch::kUInt8));
+    if (arrivals > 0) {
+        Tensor counters = arrival_pool().get(arrivals, rows);
+        ok(cgnn_cluster_sums(N, F, groups, dtype, rows.data_ptr(), mask, M, offsets, perm, sorted_id, out.data_ptr(), ws.data_ptr(),
+                             bytes, counters.data_ptr<int32_t>(), stream),
+           op);
+    } else if (mask == 2) {
+        ok(cgnn_reconstruct_backward_signs(N, F, groups, largest_group(m), dtype, rows.data_ptr(), static_cast<const uint32_t *>(M),
+                                           offsets, perm, sorted_id, out.data_ptr(), ws.data_ptr(), bytes, stream),
+           op);
+    } else {
+        ok(cgnn_reconstruct_backward(N, F, groups, largest_group(m), dtype, rows.data_ptr(), M, offsets, perm, sorted_id, mask,
+                                     out.data_ptr(), ws.data_ptr(), bytes, stream),
+           op);
+    }
+    return out;
+}
+
+// Means over the members of every group: by the caller's counts, or (NULL) by the lengths of the lists.
+// largest: the size of the largest group or a bound on it, 0 if unknown.
+Tensor member_means(const char *op, const Tensor &rows, const Tensor *counts, const std::vector<Tensor> &m, int64_t groups,
+                    int64_t largest) {
     const int64_t N = rows.size(0), F = rows.size(1);
     const int dtype = dtype_code(rows);
     Tensor out = torch::empty({groups, F}, rows.options());
-    int64_t arrivals = 0;
-    const size_t bytes = cgnn_cluster_sums_workspace_bytes(N, F, groups, dtype, &arrivals);
+    const size_t bytes = cgnn_cluster_mean_workspace_bytes(N, F, groups, dtype);
     Tensor ws = torch::empty({(int64_t)std::max<size_t>(bytes, 1)}, rows.options().dtype(torch::kUInt8));
-    Tensor counters = arrival_pool().get(arrivals, rows);
-    ok(cgnn_cluster_sums(N, F, groups, dtype, rows.data_ptr(), mask, M, m[0].data_ptr<int32_t>(), m[1].data_ptr<int32_t>(),
-                         m[2].data_ptr<int32_t>(), mean, first_group_empty, out.data_ptr(), ws.data_ptr(), bytes,
-                         counters.data_ptr<int32_t>(), current_stream(rows)),
+    ok(cgnn_cluster_mean(N, F, groups, largest, dtype, rows.data_ptr(), m[0].data_ptr<int32_t>(), m[1].data_ptr<int32_t>(),
+                         m[2].data_ptr<int32_t>(), counts ? counts->data_ptr<int32_t>() : nullptr, out.data_ptr(),
+                         ws.data_ptr(), bytes, current_stream(rows)),
        op);
     return out;
 }
@@ -927,13 +958,10 @@ Tensor cluster_mean(Tensor input, Tensor index, Tensor count, c10::optional<std:
     expect(op, input, {{Role::Features, "input", &input}, {Role::Ids, "index", &index}, {Role::Counts, "count", &count}});
     TORCH_CHECK(index.numel() == input.size(0), op, ": ", input.size(0), " rows but ", index.numel(), " cluster ids");
     c10::hip::HIPGuardMasqueradingAsCUDA guard(input.device());
-    const int64_t N = input.size(0), F = input.size(1), groups = count.numel();
-    if (input.numel() == 0) return torch::zeros({groups, F}, input.options());
+    const int64_t groups = count.numel();
+    if (input.numel() == 0) return torch::zeros({groups, input.size(1)}, input.options());
     auto m = members_or_build(op, members, index, groups);
-    Tensor out = member_sums(op, input, 0, nullptr, m, groups, false, false);
-    // the caller's counts need not be the lengths of the lists
-    ok(cgnn_cluster_divide(F, groups, dtype_code(input), count.data_ptr<int32_t>(), out.data_ptr(), current_stream(input)), op);
-    return out;
+    return member_means(op, input, &count, m, groups, largest_group(m));  // the counts need not be the lists' lengths
 }
 
 // The order in which a gather produces its rows: the member list `perm` when the caller has one
@@ -1015,7 +1043,7 @@ Tensor cluster_reconstruct_backward(Tensor grad, Tensor index, Tensor output, in
     const int64_t N = grad.size(0), F = grad.size(1);
     if (grad.numel() == 0 || groups == 0) return torch::zeros({groups, F}, grad.options());
     auto m = members_or_build(op, members, index, groups);
-    return member_sums(op, grad, relu ? 1 : 0, relu ? output.data_ptr() : nullptr, m, groups, false, false);
+    return member_sums(op, grad, relu ? 1 : 0, relu ? output.data_ptr() : nullptr, m, groups);
 }
 
 // The ReLU form of cluster_reconstruct that also returns the sign of every output element as one
@@ -1062,7 +1090,7 @@ Tensor cluster_reconstruct_backward_signs(Tensor grad, Tensor index, Tensor sign
     c10::hip::HIPGuardMasqueradingAsCUDA guard(grad.device());
     if (grad.numel() == 0 || groups == 0) return torch::zeros({groups, F}, grad.options());
     auto m = members_or_build(op, members, index, groups);
-    return member_sums(op, grad, 2, signs.data_ptr<int32_t>(), m, groups, false, false);
+    return member_sums(op, grad, 2, signs.data_ptr<int32_t>(), m, groups);
 }
 
 // ------------------------------------------------------ the layers' autograd steps ----
@@ -1131,7 +1159,7 @@ Tensor cluster_representatives(Tensor x, Tensor index, Tensor counts, std::vecto
         expect_members(op, members, index, counts.numel());
         c10::hip::HIPGuardMasqueradingAsCUDA guard(rows.device());
         reps = rows.numel() == 0 ? torch::zeros({counts.numel(), rows.size(1)}, rows.options())
-                                 : member_sums(op, rows, 0, nullptr, members, counts.numel(), true, false);
+                                 : member_means(op, rows, nullptr, members, counts.numel(), largest_group(members));
     }
     attach_mean(reps, x, index, counts, members);
     return reps;

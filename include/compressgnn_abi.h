@@ -291,22 +291,17 @@ int cgnn_lsh_group(int64_t N, int bits, const int32_t *raw_code, int64_t *ids, i
                    int32_t *perm, int32_t *sorted_id, int32_t *counts, int32_t *summary,
                    void *workspace, size_t workspace_bytes, cgnn_stream_t stream);
 
-/* The sums over the members of every group in one launch, the form the layers use: sums[g,:] = the sum over
- * members i of group g of X[i,:] -- divided by their number if mean is set; mask 1: elements dropped where
- * M[N x F] <= 0, mask 2: where a bit of M[N x ceil(F / 32)] is clear (as in cgnn_reconstruct_backward and its
- * _signs form).  A group of at most 64 members is summed in ascending order; a larger one in an order that
- * depends on the sizes alone.  first_group_empty: group 0 and no other has no members; groups may then be
- * an upper bound (rows behind the last group are left untouched), which spares the caller the host read before it.
+/* The sums over the members of every group in one launch, the form the gradients use: sums[g,:] = the sum over
+ * members i of group g of X[i,:]; mask 1: elements dropped where M[N x F] <= 0, mask 2: where a bit of
+ * M[N x ceil(F / 32)] is clear (as in cgnn_reconstruct_backward and its _signs form).  A group of at most 64
+ * members is summed in ascending order; a larger one in an order that depends on the sizes alone.
  * arrivals: counters (as many as the size query reports), zero before and after the call, as in cgnn_csr.
- * N > 0 and F > 0. */
+ * N > 0 and F > 0.  No counters reported: there are so many rows that cgnn_reconstruct_backward and its _signs form
+ * are faster, and this form is refused. */
 size_t cgnn_cluster_sums_workspace_bytes(int64_t N, int64_t F, int64_t groups, int dtype, int64_t *arrivals);
 int cgnn_cluster_sums(int64_t N, int64_t F, int64_t groups, int dtype, const void *X, int mask, const void *M,
-                      const int32_t *offsets, const int32_t *perm, const int32_t *sorted_id, int mean,
-                      int first_group_empty, void *sums, void *workspace, size_t workspace_bytes, int32_t *arrivals,
-                      cgnn_stream_t stream);
-
-/* sums[g,:] /= max(counts[g], 1). */
-int cgnn_cluster_divide(int64_t F, int64_t groups, int dtype, const int32_t *counts, void *sums, cgnn_stream_t stream);
+                      const int32_t *offsets, const int32_t *perm, const int32_t *sorted_id, void *sums, void *workspace,
+                      size_t workspace_bytes, int32_t *arrivals, cgnn_stream_t stream);
 
 /* out[f] = sum over the rows r of X[r,f] (the gradient of a bias), in a fixed order; rows > 0 and F > 0;
  * arrivals as above. */
@@ -317,7 +312,9 @@ int cgnn_column_sums(int64_t rows, int64_t F, int dtype, const void *X, void *ou
 /* reps[g,:] = (sum over members i of group g, ascending i, of X[i,:]) / max(counts[g],1).
  * max_members: size of the largest group if the caller knows it (it decides whether the
  * sums of very large groups need the multi-level carry reduction), 0 if not.  The
- * workspace size covers either case.
+ * workspace size covers either case.  counts may be NULL: the lengths of the lists (groups may then be an upper
+ * bound on their number: offsets, and reps, beyond the last group are read and written within that bound, without
+ * a meaning, which spares a caller the host read of the number before this call).
  * Replaces cluster_mean_cuda (cluster_kernel.cu:158-170). */
 size_t cgnn_cluster_mean_workspace_bytes(int64_t N, int64_t F, int64_t groups, int dtype);
 int cgnn_cluster_mean(int64_t N, int64_t F, int64_t groups, int64_t max_members, int dtype, const void *X,
