@@ -13,7 +13,7 @@ import torch
 from torch import Tensor
 
 from CompressgnnSPMM import Compressgnn_SPMM
-from CooPhases import CooPlanCache, CooPropagateFunction
+from CooPhases import CooPlanCache, coo_propagate
 from compress_graph import CompressGraph
 from type import Size
 
@@ -51,7 +51,7 @@ class Propagate(torch.nn.Module):
         if vertex_cnt is None or rule_cnt is None:
             raise ValueError("multi-phase propagation needs vertex_cnt and rule_cnt")
         plan = self._coo_plans.get(edge_index, edge_weight, vertex_cnt, rule_cnt)
-        return self.update(CooPropagateFunction.apply(plan, x))
+        return self.update(coo_propagate(plan, x))
 
     def propagate(self, edge_index, x: Tensor, edge_weight: Optional[Tensor] = None, size: Size = None):
         """One hop over an uncompressed graph given as a [2, E] edge tensor: out[dst] += weight * x[src]
@@ -65,7 +65,7 @@ class Propagate(torch.nn.Module):
             raise ValueError("propagate() supports aggr='add' only")
         weights = None if edge_weight is None else [edge_weight]
         plan = self._coo_plans.get([edge_index], weights, x.size(0), 0)
-        return self.update(CooPropagateFunction.apply(plan, x))
+        return self.update(coo_propagate(plan, x))
 
     def message(self, x_j: Tensor) -> Tensor:
         return x_j

@@ -735,3 +735,50 @@ def test_uncompressed_hop_over_an_edge_tensor():
     assert_within(ones.detach().cpu().numpy(), prep_oracle.coo_propagate(x_np, [edges], [np.ones(E, np.float32)], V, 0))
     with pytest.raises(TypeError):
         prop.propagate([e_t], x, w_t)
+
+
+@pytest.mark.parametrize("weights", [True, False])
+@pytest.mark.parametrize("kind", ["chain", "deep_chain", "no_rules", "used_before_complete", "vertex_source_late"])
+def test_phase_lists_of_every_shape(kind, weights):
+    """Phase lists that are a compressed chain (with and without levels, too deep to fold, without rules) and lists
+    that are not (a rule reached after it was a source; a vertex as a source of a later phase), forward and
+    gradient against the gather + scatter-add loop in float64."""
+    from CooPhases import CooPhasePlan, coo_propagate
+    rng = np.random.default_rng(3)
+    V, R, F = 90, 0 if kind == "no_rules" else 40, 20
+    vert = lambda n: rng.integers(0, V, n)
+    lo = lambda a, b, n: V + rng.integers(a, b, n)
+    phases = [(vert(400), np.concatenate([vert(300), lo(0, 10, 100) if R else vert(100)]))]
+    if kind == "chain":
+        phases += [(lo(0, 10, 60), vert(60))]
+    if kind in ("deep_chain", "used_before_complete", "vertex_source_late"):
+        steps = 20 if kind == "deep_chain" else 3
+        for k in range(steps):  # rules of stage k feed stage k + 1 (two rules a stage) and vertices
+            a = 0 if k == 0 else 10 + (k - 1)
+            b = 10 if k == 0 else a + 1
+            phases += [(np.concatenate([lo(a, b, 8), lo(a, b, 12)]), np.concatenate([lo(10 + k, 11 + k, 8), vert(12)]))]
+    if kind == "used_before_complete":
+        phases += [(lo(11, 12, 9), lo(0, 10, 9))]
+    if kind == "vertex_source_late":
+        phases += [(vert(9), vert(9))]
+    w = [rng.standard_normal(len(s)).astype(np.float32) if weights else None for s, _ in phases]
+    t = lambda a: torch.from_numpy(a).to(DEV)
+    edges = [torch.stack([t(s), t(d)]) for s, d in phases]
+    plan = CooPhasePlan(edges, [t(a) for a in w] if weights else None, V, R)
+    assert (plan.chain is not None) == (kind in ("chain", "deep_chain", "no_rules"))
+    x, g = rng.standard_normal((V, F)).astype(np.float32), rng.standard_normal((V, F)).astype(np.float32)
+    full = np.zeros((V + R, F))
+    for k, (s, d) in enumerate(phases):
+        source = x.astype(np.float64) if k == 0 else full.copy()
+        np.add.at(full, d, (1.0 if w[k] is None else w[k][:, None].astype(np.float64)) * source[s])
+    back = np.concatenate([g.astype(np.float64), np.zeros((R, F))])
+    gx = np.zeros((V, F))
+    for k in range(len(phases) - 1, -1, -1):
+        s, d = phases[k]
+        move = (1.0 if w[k] is None else w[k][:, None].astype(np.float64)) * back[d]
+        np.add.at(gx if k == 0 else back, s, move)
+    X = t(x).requires_grad_()
+    out = coo_propagate(plan, X)
+    (got,) = torch.autograd.grad(out, X, t(g))
+    np.testing.assert_allclose(out.detach().cpu().numpy(), full[:V], rtol=1e-4, atol=1e-4 * np.abs(full[:V]).max())
+    np.testing.assert_allclose(got.cpu().numpy(), gx, rtol=1e-4, atol=1e-4 * np.abs(gx).max())
