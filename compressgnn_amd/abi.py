@@ -17,7 +17,7 @@ SPMM_AUTO, SPMM_ROW, SPMM_NNZ = 0, 1, 2
 
 EXPORTS = [
     "cgnn_last_error", "cgnn_version",
-    "cgnn_spmm_schedule", "cgnn_spmm_run_length", "cgnn_spmm_run_starts", "cgnn_spmm_wg_shape", "cgnn_spmm_wg_runs", "cgnn_spmm_workspace_bytes", "cgnn_spmm", "cgnn_spmm_dual",
+    "cgnn_spmm_schedule", "cgnn_spmm_run_length", "cgnn_spmm_run_starts", "cgnn_spmm_wg_shape", "cgnn_spmm_wg_runs", "cgnn_spmm_once", "cgnn_spmm_once_workspace_bytes", "cgnn_spmm_workspace_bytes", "cgnn_spmm", "cgnn_spmm_dual",
     "cgnn_spmm_static_scratch_bytes", "cgnn_spmm_static_init", "cgnn_spmm_static",
     "cgnn_csr_prepare_i64", "cgnn_csr_expand_rows", "cgnn_narrow_ids", "cgnn_csr_compose_columns",
     "cgnn_csr_transpose_workspace_bytes", "cgnn_csr_transpose_device",
@@ -63,7 +63,7 @@ def lib():
         for name in ("cgnn_spmm_workspace_bytes", "cgnn_spmm_static_scratch_bytes", "cgnn_lsh_scan_workspace_bytes", "cgnn_lsh_group_workspace_bytes",
                      "cgnn_cluster_members_workspace_bytes", "cgnn_cluster_mean_workspace_bytes",
                      "cgnn_csr_transpose_workspace_bytes", "cgnn_compress_batch_workspace_bytes",
-                     "cgnn_cluster_sums_workspace_bytes", "cgnn_column_sums_workspace_bytes",
+                     "cgnn_spmm_once_workspace_bytes", "cgnn_cluster_sums_workspace_bytes", "cgnn_column_sums_workspace_bytes",
                      "cgnn_exclusive_sum_workspace_bytes", "cgnn_sample_relabel_workspace_bytes"):
             getattr(L, name).restype = ctypes.c_size_t
         L.cgnn_lsh_group_small_rows.restype = ctypes.c_int64

@@ -61,8 +61,8 @@ constexpr int kXcds = 8;          // accelerator dies of an MI355X, each with it
 constexpr int kDefaultSeg = 64;   // non-zeros per lane group in the nnz schedule
 
 // Where the runs of the nnz kernel come from: positions that are multiples of the run length, the table of
-// workgroup runs, or the same rule worked out by every lane group (member lists, which are new with every
-// assignment: a launch for their table would cost more than the few dependent loads).
+// workgroup runs, or the same rule worked out by every lane group (blocks that are new with every call -- member
+// lists, cgnn_spmm_once: a launch for their table would cost more than the few dependent loads).
 enum { WGRUNS_NONE = 0, WGRUNS_TABLE = 1, WGRUNS_COMPUTED = 2 };
 enum { MODE_VAL = 0, MODE_UNIT = 1, MODE_RELU_MASK = 2, MODE_DUAL = 3, MODE_SIGN_MASK = 4 };
 
@@ -1300,6 +1300,8 @@ int launch_shape(int kind, int mode, const SpmmArgs<T> &args, int64_t items, int
             if (a.arrivals != nullptr && a.run_start == nullptr) {
                 if (mode == MODE_UNIT)
                     hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_UNIT, WGRUNS_COMPUTED>), grid, block, 0, stream, a);
+                else if (mode == MODE_VAL)
+                    hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_VAL, WGRUNS_COMPUTED>), grid, block, 0, stream, a);
                 else if (mode == MODE_SIGN_MASK)
                     hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_SIGN_MASK, WGRUNS_COMPUTED>), grid, block, 0, stream, a);
                 else
@@ -1475,7 +1477,8 @@ constexpr int64_t kResidentWorkgroups = 256 * 7;
 int wg_run_len(const cgnn_csr *A, int groups) {
     const int64_t fill = ceil_div(ceil_div(A->nnz, kResidentWorkgroups * groups), kUnroll) * kUnroll;
     const int longest = seg_len(A);
-    return (int)(fill < 8 ? (longest < 8 ? longest : 8) : (fill > longest ? longest : fill));
+    if (fill < 8) return longest < 8 ? longest : 8;
+    return (int)(fill <= 2 * longest ? fill : longest);
 }
 
 // mean (may be NULL; MODE_UNIT): whether the rows are wanted divided by their numbers of entries; false on return
@@ -1618,6 +1621,122 @@ __global__ void expand_rows_kernel(const P *__restrict__ rowptr, int64_t rows, i
             else hi = mid;
         }
         rowidx[e] = (int32_t)lo;
+    }
+}
+
+// The int32 form of a block that is given as int64 arrays for one product: row pointers, columns and the row of
+// every entry, in one launch.  Rows and entries are walked as one list -- every row in front of its entries, row r at
+// position rowptr[r] + r -- and a workgroup takes kOnceItems * kBlock consecutive places of it, so neither hubs (a
+// workgroup per 16 rows took 41 us for 100,003 rows of 1.0 M entries of a web graph, whose hubs are neighbours) nor the
+// thousands of empty rows of the youngest vertices (2,048 entries per workgroup: 22 us) keep one longer than the others.
+// It looks for the two ends of its stretch with all its threads at once (256 row pointers a step), marks the entries
+// that rows begin at and spreads the marks by a running maximum: 8.6 us.  Row pointers and columns narrowed apart and a
+// binary search per entry were three launches of 25 us, behind 26 us for the length of the longest row and its
+// way to the host.
+constexpr int kOnceItems = 8;
+constexpr int kOncePlaces = kOnceItems * kBlock;
+
+__global__ __launch_bounds__(kBlock) void csr_once_kernel(const int64_t *__restrict__ rowptr64, const int64_t *__restrict__ col64,
+                                                          int64_t rows, int64_t nnz, int32_t *__restrict__ rowptr,
+                                                          int32_t *__restrict__ col, int32_t *__restrict__ rowidx) {
+    __shared__ int32_t begins[kOncePlaces];  // the row that begins at an entry of the stretch, or -1
+    __shared__ int waves[2][kBlock / kWave];
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int64_t places[2] = {(int64_t)blockIdx.x * kOncePlaces, min(rows + nnz, (int64_t)(blockIdx.x + 1) * kOncePlaces)};
+#pragma unroll
+    for (int u = 0; u < kOnceItems; ++u) begins[u * kBlock + threadIdx.x] = -1;
+    // the largest row at or before each of the two places lies in [lo, hi); row lo does throughout
+    int64_t lo[2] = {0, 0}, hi[2] = {rows, rows};
+    while (hi[0] - lo[0] > 1 || hi[1] - lo[1] > 1) {
+        int64_t step[2], at[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            step[k] = (hi[k] - lo[k] + kBlock - 1) / kBlock;
+            const int64_t r = lo[k] + step[k] * threadIdx.x;
+            at[k] = r < hi[k] ? rowptr64[r] + r : INT64_MAX;
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int n = __popcll(__ballot(threadIdx.x == 0 || at[k] <= places[k]));
+            if (lane == 0) waves[k][wave] = n;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            int below = 0;
+#pragma unroll
+            for (int w = 0; w < kBlock / kWave; ++w) below += waves[k][w];
+            lo[k] += step[k] * (below - 1);
+            hi[k] = min(hi[k], lo[k] + step[k]);
+        }
+        __syncthreads();
+    }
+    // first entry and first row of the stretch, and those behind it
+    int64_t entry[2], row[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int64_t start = rowptr64[lo[k]];
+        const bool on_row = start + lo[k] >= places[k];  // the place is that of the row itself
+        entry[k] = on_row ? start : places[k] - lo[k] - 1;
+        row[k] = on_row ? lo[k] : lo[k] + 1;
+        // row pointers that are none must not lead out of the arrays
+        entry[k] = max((int64_t)0, min(nnz, entry[k]));
+    }
+    if (places[1] == rows + nnz) entry[1] = nnz, row[1] = rows;
+    const int64_t e0 = entry[0];
+    const int held = (int)max((int64_t)0, min((int64_t)kOncePlaces, entry[1] - e0));
+    int64_t c[kOnceItems], at[kOnceItems], end[kOnceItems];
+#pragma unroll
+    for (int u = 0; u < kOnceItems; ++u) {
+        const int k = u * kBlock + threadIdx.x;
+        const int64_t r = row[0] + k;
+        c[u] = k < held ? col64[e0 + k] : 0;
+        at[u] = r < row[1] ? rowptr64[r] : 0;
+        end[u] = r < row[1] ? rowptr64[r + 1] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < kOnceItems; ++u) {
+        const int64_t r = row[0] + u * kBlock + threadIdx.x;
+        if (r >= row[1]) break;
+        rowptr[r] = (int32_t)at[u];
+        if (r == rows - 1) rowptr[rows] = (int32_t)end[u];
+        // rows without entries begin where another does: not marked, so one row a mark
+        const int64_t k = at[u] - e0;
+        if (end[u] > at[u] && k >= 0 && k < held) begins[k] = (int32_t)r;
+    }
+    __syncthreads();
+    // thread t spreads the marks over entries t * kOnceItems ...; what comes before the first mark belongs to the
+    // row in front of the stretch
+    int32_t mark[kOnceItems];
+#pragma unroll
+    for (int u = 0; u < kOnceItems; ++u) {
+        mark[u] = begins[threadIdx.x * kOnceItems + u];
+        if (u > 0) mark[u] = max(mark[u], mark[u - 1]);
+    }
+    int upto = mark[kOnceItems - 1];
+#pragma unroll
+    for (int s = 1; s < kWave; s <<= 1) {
+        const int n = __shfl_up(upto, s, kWave);
+        if (lane >= s) upto = max(upto, n);
+    }
+    if (lane == kWave - 1) waves[0][wave] = upto;
+    int before = __shfl_up(upto, 1, kWave);
+    if (lane == 0) before = -1;
+    __syncthreads();
+    before = max(before, (int)row[0] - 1);
+#pragma unroll
+    for (int w = 0; w < kBlock / kWave; ++w)
+        if (w < wave) before = max(before, waves[0][w]);
+#pragma unroll
+    for (int u = 0; u < kOnceItems; ++u) begins[threadIdx.x * kOnceItems + u] = max(mark[u], before);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kOnceItems; ++u) {
+        const int k = u * kBlock + threadIdx.x;
+        if (k < held) {
+            col[e0 + k] = (int32_t)c[u];
+            rowidx[e0 + k] = begins[k];
+        }
     }
 }
 
@@ -1768,6 +1887,81 @@ extern "C" int cgnn_spmm_schedule(int64_t rows, int64_t nnz, int32_t max_row_nnz
 }
 
 extern "C" int cgnn_spmm_run_length(const cgnn_csr *A) { return A == nullptr ? 0 : seg_len(A); }
+
+namespace {
+
+struct OnceLayout {
+    size_t rowptr, col, rowidx, pieces, total;
+    int groups, wg_len;
+    int64_t workgroups;
+};
+
+OnceLayout once_layout(int64_t rows, int64_t nnz, int64_t F, int dtype) {
+    cgnn_csr A{};
+    A.rows = rows;
+    A.nnz = nnz;
+    A.seg_nnz = 32;  // as for the blocks of a plan
+    OnceLayout L;
+    L.groups = kBlock / shape_of(F, dtype).lpr;
+    L.wg_len = wg_run_len(&A, L.groups) * L.groups;
+    L.workgroups = ceil_div(nnz, L.wg_len);
+    L.rowptr = 0;
+    L.col = align_up((size_t)(rows + 1) * sizeof(int32_t), 256);
+    L.rowidx = L.col + align_up((size_t)nnz * sizeof(int32_t), 256);
+    L.pieces = L.rowidx + align_up((size_t)nnz * sizeof(int32_t), 256);
+    L.total = L.pieces + wg_piece_bytes(L.workgroups, F, dtype == CGNN_F64 ? 8 : 4);
+    return L;
+}
+
+template <typename T>
+int spmm_once(const OnceLayout &L, int64_t rows, int64_t nnz, const void *val, int dtype, const void *X, void *Y, int64_t F,
+              int accumulate, char *ws, int32_t *arrivals, hipStream_t stream) {
+    cgnn_csr A{};
+    A.rows = rows;
+    A.nnz = nnz;
+    A.rowptr = reinterpret_cast<const int32_t *>(ws + L.rowptr);
+    A.colidx = reinterpret_cast<const int32_t *>(ws + L.col);
+    A.rowidx = reinterpret_cast<const int32_t *>(ws + L.rowidx);
+    A.val = val;
+    SpmmArgs<T> a = make_args<T>(&A, X, nullptr, INT32_MAX, nullptr, Y, F, accumulate);
+    a.arrivals = arrivals;
+    a.wg_len = L.wg_len;
+    a.keep = kDefaultSeg;
+    a.nseg = (int32_t)(L.workgroups * L.groups);
+    a.carry = reinterpret_cast<T *>(ws + L.pieces);
+    a.find_empty = 1;
+    return launch<T>(KIND_NNZ, MODE_VAL, pick_shape<T>(F, true), a, a.nseg, stream);
+}
+
+}  // namespace
+
+extern "C" size_t cgnn_spmm_once_workspace_bytes(int64_t rows, int64_t nnz, int64_t F, int dtype, int64_t *arrivals) {
+    if (arrivals) *arrivals = 0;
+    if (rows <= 0 || nnz <= 0 || F <= 0) return 0;
+    const OnceLayout L = once_layout(rows, nnz, F, dtype);
+    if (arrivals) *arrivals = L.workgroups * shape_of(F, dtype).grid_y;
+    return L.total;
+}
+
+extern "C" int cgnn_spmm_once(int64_t rows, int64_t nnz, const int64_t *rowptr, const int64_t *col, const void *val, int dtype,
+                              const void *X, void *Y, int64_t F, int accumulate, void *workspace, size_t workspace_bytes,
+                              int32_t *arrivals, cgnn_stream_t stream) {
+    const int64_t lim = (int64_t)INT32_MAX - 65536;
+    CGNN_REQUIRE(rows > 0 && nnz > 0 && F > 0 && rows < lim && nnz < lim, "cgnn_spmm_once: sizes must be in [1, 2^31 - 65536)");
+    CGNN_REQUIRE(dtype == CGNN_F32 || dtype == CGNN_F64, "cgnn_spmm_once: dtype must be f32 or f64");
+    CGNN_REQUIRE(rowptr && col && X && Y && arrivals, "cgnn_spmm_once: null array");
+    const OnceLayout L = once_layout(rows, nnz, F, dtype);
+    if (workspace == nullptr || workspace_bytes < L.total) return fail(CGNN_EWORKSPACE, "cgnn_spmm_once: workspace too small");
+    char *ws = static_cast<char *>(workspace);
+    hipLaunchKernelGGL(csr_once_kernel, dim3((unsigned)ceil_div(rows + nnz, kOncePlaces)), dim3(kBlock), 0, stream,
+                       rowptr, col, rows, nnz, reinterpret_cast<int32_t *>(ws + L.rowptr), reinterpret_cast<int32_t *>(ws + L.col),
+                       reinterpret_cast<int32_t *>(ws + L.rowidx));
+    int rc = check_launch("csr_once");
+    if (rc != CGNN_OK) return rc;
+    if (dtype == CGNN_F32)
+        return spmm_once<float>(L, rows, nnz, val, dtype, X, Y, F, accumulate, ws, arrivals, stream);
+    return spmm_once<double>(L, rows, nnz, val, dtype, X, Y, F, accumulate, ws, arrivals, stream);
+}
 
 extern "C" int cgnn_spmm_wg_shape(const cgnn_csr *A, int64_t F, int dtype, int32_t *groups, int32_t *wg_len,
                                   int64_t *arrivals) {

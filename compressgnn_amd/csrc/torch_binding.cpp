@@ -326,7 +326,7 @@ Tensor block_spmm(DeviceCsr &A, const Tensor &mat, c10::optional<Tensor> optiona
 }
 
 // spmm_func of the reference (src/runtime/csrc/sparse/spmm.cpp:11-22): CSR given as
-// int64 tensors, prepared on every call.  Graph blocks that are used repeatedly should
+// int64 tensors, narrowed on every call.  Graph blocks that are used repeatedly should
 // be wrapped in a DeviceCsr once instead.
 Tensor spmm_func(Tensor vlist, Tensor elist, Tensor value, Tensor mat, std::string method,
                  c10::optional<Tensor> optional_out) {
@@ -337,8 +337,39 @@ Tensor spmm_func(Tensor vlist, Tensor elist, Tensor value, Tensor mat, std::stri
     const int kernel = kernel_of_method(method);
     TORCH_CHECK(vlist.scalar_type() == torch::kInt64 && elist.scalar_type() == torch::kInt64,
                 "vlist and elist must be int64");
-    auto blk = make_csr(vlist, elist, value, vlist.size(-1) - 1, mat.size(0), mat.device(), 0, c10::nullopt, false);
-    return block_spmm(*blk, mat, optional_out, kernel);
+    const int64_t rows = vlist.size(-1) - 1, nnz = elist.numel();
+    const bool plain = mat.dim() == 2 && mat.is_contiguous() && vlist.dim() == 1 && elist.dim() == 1 && rows > 0 && nnz > 0 &&
+                       mat.size(1) > 0 && vlist.device() == mat.device() && elist.device() == mat.device() &&
+                       value.device() == mat.device();
+    if (kernel != CGNN_SPMM_AUTO || !plain) {
+        auto blk = make_csr(vlist, elist, value, rows, mat.size(0), mat.device(), 0, c10::nullopt, false);
+        return block_spmm(*blk, mat, optional_out, kernel);
+    }
+    const int64_t F = mat.size(1), lim = (int64_t)INT32_MAX - 65536;
+    TORCH_CHECK(rows < lim && mat.size(0) < lim && nnz < lim, "block exceeds the int32 index range of the kernels");
+    TORCH_CHECK(value.numel() == nnz, "value must have one entry per non-zero");
+    TORCH_CHECK(value.scalar_type() == mat.scalar_type(), "value and mat must have the same dtype");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(mat.device());
+    const int dtype = dtype_code(mat);
+    const Tensor rowptr = vlist.contiguous(), col = elist.contiguous(), val = value.contiguous();
+    Tensor out;
+    const bool accumulate = optional_out.has_value() && optional_out->defined();
+    if (accumulate) {
+        out = optional_out->contiguous();  // as in block_spmm
+        require_gpu(out, "out");
+        TORCH_CHECK(out.dim() == 2 && out.size(0) == rows && out.size(1) == F && out.scalar_type() == mat.scalar_type(),
+                    "out must be [rows, F] of mat's dtype");
+    } else {
+        out = torch::empty({rows, F}, mat.options());
+    }
+    int64_t arrivals = 0;
+    const size_t bytes = cgnn_spmm_once_workspace_bytes(rows, nnz, F, dtype, &arrivals);
+    Tensor ws = torch::empty({(int64_t)bytes}, mat.options().dtype(torch::kUInt8));
+    Tensor counters = arrival_pool().get(arrivals, mat);
+    ok(cgnn_spmm_once(rows, nnz, rowptr.data_ptr<int64_t>(), col.data_ptr<int64_t>(), val.data_ptr(), dtype, mat.data_ptr(),
+                      out.data_ptr(), F, accumulate, ws.data_ptr(), bytes, counters.data_ptr<int32_t>(), current_stream(mat)),
+       "spmm");
+    return out;
 }
 
 // ------------------------------------------------------- compressed propagation ----

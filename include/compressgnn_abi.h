@@ -127,6 +127,17 @@ int cgnn_spmm_wg_runs(const cgnn_csr *A, int32_t groups, int32_t wg_len, int32_t
  * (the carry-out rows of the NNZ schedule).  0 for the ROW schedule. */
 size_t cgnn_spmm_workspace_bytes(const cgnn_csr *A, int64_t F, int dtype, int kernel);
 
+/* One product of a block given as int64 arrays, as cgnn_spmm under AUTO but without what a block that is kept
+ * has made once: the arrays are narrowed by the call (one launch), the schedule is the NNZ one with workgroup runs
+ * whatever the rows look like, and nothing is read by the host.  A row of at most 64 entries is summed in
+ * ascending order.  arrivals: counters as in cgnn_csr, as many as the size query reports.  rows, nnz and F must
+ * be positive; the columns must lie in X (not checked).
+ * Replaces spmm_func: src/runtime/csrc/sparse/spmm.cpp:11-22. */
+size_t cgnn_spmm_once_workspace_bytes(int64_t rows, int64_t nnz, int64_t F, int dtype, int64_t *arrivals);
+int cgnn_spmm_once(int64_t rows, int64_t nnz, const int64_t *rowptr, const int64_t *col, const void *val, int dtype,
+                   const void *X, void *Y, int64_t F, int accumulate, void *workspace, size_t workspace_bytes,
+                   int32_t *arrivals, cgnn_stream_t stream);
+
 /* Y[rows x F] (+)= A * X[cols x F].
  * accumulate == 0: every row of Y is written (empty rows become 0);
  * accumulate != 0: Y += A*X, rows without entries are left untouched, and Y may be

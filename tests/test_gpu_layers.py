@@ -782,3 +782,32 @@ def test_phase_lists_of_every_shape(kind, weights):
     (got,) = torch.autograd.grad(out, X, t(g))
     np.testing.assert_allclose(out.detach().cpu().numpy(), full[:V], rtol=1e-4, atol=1e-4 * np.abs(full[:V]).max())
     np.testing.assert_allclose(got.cpu().numpy(), gx, rtol=1e-4, atol=1e-4 * np.abs(gx).max())
+
+
+@pytest.mark.parametrize("shape", ["one_row", "no_long_rows", "hubs_first", "empty_tail", "empty_head", "places_full", "mixed"])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_spmm_func_on_blocks_of_every_shape(shape, accumulate):
+    """The operator on int64 tensors narrows its block in stretches of 2,048 rows and entries: rows that end or begin
+    with a stretch, rows over several stretches, thousands of empty rows in front, behind and between; against
+    float64, and bit for bit where a row has at most 64 entries."""
+    import compressgnn_runtime as rt
+    rng = np.random.default_rng(17)
+    lens = {"one_row": [5000], "no_long_rows": rng.integers(0, 9, 3000), "hubs_first": [9000, 2048, 2047, 2049] + [1] * 500,
+            "empty_tail": [3, 70, 2] + [0] * 9000, "empty_head": [0] * 9000 + [1, 3000, 64, 65],
+            "places_full": [2047, 2047, 2046, 0, 2047, 1023, 1023, 0, 0],
+            "mixed": np.where(rng.random(4000) < 0.6, 0, rng.integers(0, 200, 4000))}[shape]
+    lens = np.asarray(lens, np.int64)
+    vlist = np.concatenate([[0], np.cumsum(lens)])
+    cols, F = 700, 20
+    elist = rng.integers(0, cols, int(vlist[-1]))
+    value = (rng.standard_normal(len(elist)) * 0.3 / np.sqrt(np.maximum(np.repeat(lens, lens), 1))).astype(np.float32)
+    x = rng.standard_normal((cols, F)).astype(np.float32)
+    out0 = rng.standard_normal((len(lens), F)).astype(np.float32) if accumulate else np.zeros((len(lens), F), np.float32)
+    want = out0.astype(np.float64)
+    np.add.at(want, np.repeat(np.arange(len(lens)), lens), value[:, None].astype(np.float64) * x[elist])
+    t = lambda a: torch.from_numpy(a).to(DEV)
+    for _ in range(2):
+        got = rt.spmm_func(t(vlist), t(elist), t(value), t(x), "auto", t(out0.copy()) if accumulate else None).cpu().numpy()
+        assert_within(got, want, rtol=1e-5, atol=2e-5)
+    short = lens <= 64
+    assert np.array_equal(got[short], oracle.spmm(vlist, elist, value, x, out0.copy())[short])
