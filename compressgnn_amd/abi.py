@@ -30,7 +30,7 @@ EXPORTS = [
     "cgnn_reconstruct", "cgnn_reconstruct_backward", "cgnn_sign_words", "cgnn_reconstruct_signs",
     "cgnn_reconstruct_backward_signs", "cgnn_copy_bytes", "cgnn_read_bytes", "cgnn_fill_bytes",
     "cgnn_exclusive_sum_workspace_bytes", "cgnn_exclusive_sum_i32", "cgnn_sample_count", "cgnn_sample_fill",
-    "cgnn_sample_relabel_begin", "cgnn_sample_relabel_workspace_bytes", "cgnn_sample_relabel",
+    "cgnn_sample_relabel_begin", "cgnn_sample_relabel_workspace_bytes", "cgnn_sample_relabel", "cgnn_sample_layers_workspace_bytes", "cgnn_sample_layers", "cgnn_sample_layers_write",
 ]
 
 
@@ -63,7 +63,7 @@ def lib():
         for name in ("cgnn_spmm_workspace_bytes", "cgnn_spmm_static_scratch_bytes", "cgnn_lsh_scan_workspace_bytes", "cgnn_lsh_group_workspace_bytes",
                      "cgnn_cluster_members_workspace_bytes", "cgnn_cluster_mean_workspace_bytes",
                      "cgnn_csr_transpose_workspace_bytes", "cgnn_compress_batch_workspace_bytes",
-                     "cgnn_spmm_once_workspace_bytes", "cgnn_cluster_sums_workspace_bytes", "cgnn_column_sums_workspace_bytes",
+                     "cgnn_sample_layers_workspace_bytes", "cgnn_spmm_once_workspace_bytes", "cgnn_cluster_sums_workspace_bytes", "cgnn_column_sums_workspace_bytes",
                      "cgnn_exclusive_sum_workspace_bytes", "cgnn_sample_relabel_workspace_bytes"):
             getattr(L, name).restype = ctypes.c_size_t
         L.cgnn_lsh_group_small_rows.restype = ctypes.c_int64

@@ -25,6 +25,13 @@
 // the position of the frontier vertex among the samples and the step of the selection loop),
 // so a sample does not depend on scheduling.  The reference draws from torch's sequential CPU
 // generator; the streams differ by construction, everything downstream of a stream is the same.
+//
+// A call whose fan-outs bound every layer (cgnn_sample_layers) goes without the sizes in between: the neighbours of
+// frontier vertex i stand in slots i * fan-out ..., whose order is the order of the list, so that nothing is summed up
+// before they are drawn; the sizes stay on the device, every launch covers the most there can be, and the
+// host reads once, when the outputs have to be allocated.  One mini-batch of 1,024 seeds with fan-outs 25 and 10
+// took 47 launches and four host reads (256 us) layer by layer; it takes eight and one (60 us);
+// 16,384 seeds with 25 and 15 went from 384 to 105 us, most of it the chains of loads through the rules.
 #include "common.h"
 
 namespace cgnn {
@@ -35,6 +42,7 @@ int occupancy_scan(const int32_t *in, int64_t n, int32_t *out, void *scratch, hi
 namespace {
 
 constexpr int kUnseen = INT32_MAX;
+__device__ __forceinline__ int64_t ceil_div_dev(int64_t a, int64_t b) { return (a + b - 1) / b; }
 constexpr int kLdsPicks = 1024;  // random positions a wave keeps in LDS
 
 struct Graph {
@@ -72,6 +80,30 @@ __device__ __forceinline__ int64_t draw(uint64_t seed, int64_t layer, int64_t i,
     return (int64_t)__umul64hi(u, (uint64_t)high);
 }
 
+// Entry k of a rule: its own list, then the children that the descent takes.
+__device__ int64_t below_rule(const Graph &g, int64_t rule, int64_t k) {
+    for (int level = 0; level < g.levels; ++level) {
+        const int64_t own = g.r2v_ptr[rule], own_count = g.r2v_ptr[rule + 1] - own;
+        if (k < own_count) return g.r2v_idx[own + k];
+        k -= own_count;
+        for (int64_t c = g.r2r_ptr[level][rule]; c < g.r2r_ptr[level][rule + 1]; ++c) {
+            const int64_t child = g.r2r_idx[level][c];
+            const int64_t child_degree = g.r_degree[child];
+            if (k < child_degree) {
+                rule = child;
+                break;
+            }
+            k -= child_degree;
+        }
+    }
+    const int64_t own = g.r2v_ptr[rule], own_count = g.r2v_ptr[rule + 1] - own;
+    if (k < own_count) return g.r2v_idx[own + k];
+    // The descent found less than r_degree promised (degrees that do not fit the hierarchy).
+    // The reference goes on to the next rule with k - degree, which is negative by now, and
+    // indexes before that rule's list; here the position counts as out of range.
+    return -1;
+}
+
 // -------------------------------------------------------- the expanded in-list ------
 // The k-th neighbour in the order of storage_api.h:6-70: v2v entries; then, rule by rule of
 // the vertex's v2r entries, the rule's expanded list (its r2v entries, then its children's
@@ -83,30 +115,8 @@ __device__ int64_t neighbor_at(const Graph &g, int64_t node, int64_t k) {
     if (g.v2r_ptr == nullptr) return -1;  // a plain graph: no rules
     k -= v2v_count;
     for (int64_t e = g.v2r_ptr[node]; e < g.v2r_ptr[node + 1]; ++e) {
-        int64_t rule = g.v2r_idx[e];
-        const int64_t degree = g.r_degree[rule];
-        if (k < degree) {
-            for (int level = 0; level < g.levels; ++level) {
-                const int64_t own = g.r2v_ptr[rule], own_count = g.r2v_ptr[rule + 1] - own;
-                if (k < own_count) return g.r2v_idx[own + k];
-                k -= own_count;
-                for (int64_t c = g.r2r_ptr[level][rule]; c < g.r2r_ptr[level][rule + 1]; ++c) {
-                    const int64_t child = g.r2r_idx[level][c];
-                    const int64_t child_degree = g.r_degree[child];
-                    if (k < child_degree) {
-                        rule = child;
-                        break;
-                    }
-                    k -= child_degree;
-                }
-            }
-            const int64_t own = g.r2v_ptr[rule], own_count = g.r2v_ptr[rule + 1] - own;
-            if (k < own_count) return g.r2v_idx[own + k];
-            // The descent found less than r_degree promised (degrees that do not fit the hierarchy).
-            // The reference goes on to the next rule with k - degree, which is negative by now, and
-            // indexes before that rule's list; here the position counts as out of range.
-            return -1;
-        }
+        const int64_t rule = g.v2r_idx[e], degree = g.r_degree[rule];
+        if (k < degree) return below_rule(g, rule, k);
         k -= degree;
     }
     return -1;
@@ -268,6 +278,356 @@ __global__ __launch_bounds__(kBlock) void sample_fill_kernel(LayerArgs a) {
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
     for (int64_t t = lane; t < count; t += kWave) put(t, neighbor_at(g, node, pick_at(t)));
+}
+
+// ------------------------------------------------------- layers of a bounded size ----
+// A vertex has one entry in number_of: kUnseen, or kClaim + the first slot of the layer that holds it, or the number it
+// was given.  Smaller is final, so that claims are atomic minima that never touch a number.
+constexpr int32_t kClaim = 1 << 30;
+constexpr int kChunkItems = 4;
+constexpr int kChunk = kChunkItems * kBlock;  // slots per workgroup when they are ranked
+constexpr int kTail = 8;                      // chunks a thread sums up when all are counted
+constexpr int kRegPicks = kWave;              // fan-outs up to this keep the chosen positions in registers, one a lane
+
+struct BoundedLayer {
+    int64_t fanout, n_cap;   // most vertices of the frontier
+    int32_t *slots;          // [n_cap * fanout] neighbours, -1 behind the last
+    uint64_t *before;        // [chunks] neighbours, and << 32 vertices they introduce, in the chunks in front
+};
+
+// state of a layer: position of its frontier among the samples, vertices in it, edges of the layers before, chunks
+// ranked so far
+struct BoundedArgs {
+    Graph g;
+    int64_t n_input;
+    const int64_t *input;
+    int32_t *number_of, *samples;  // samples: without the input, which stands in front of them
+    int32_t *state;          // [layers + 1][4]
+    int32_t *status;         // [2] CGNN_SAMPLE_* of the first error; whether a full list went beyond its bounds
+    int32_t *summary;        // last layer: number of samples, edges, status, 1 (pinned host memory)
+    uint64_t seed;
+    int32_t layer, layers;
+    BoundedLayer at[CGNN_SAMPLE_MAX_BOUNDED];
+    int64_t first_chunk[CGNN_SAMPLE_MAX_BOUNDED + 1];  // of a layer, when all are written at once
+    int64_t *out_samples, *out_source, *out_neighbor;
+};
+
+__global__ __launch_bounds__(kBlock) void bounded_begin_kernel(BoundedArgs a) {
+    const int64_t stride = (int64_t)gridDim.x * kBlock, t0 = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    for (int64_t v = t0; v < a.g.vertex_cnt; v += stride) a.number_of[v] = kUnseen;
+    if (t0 < 4 * (a.layers + 1)) a.state[t0] = t0 == 1 ? (int32_t)a.n_input : 0;
+    if (t0 < 2) a.status[t0] = CGNN_SAMPLE_OK;
+}
+
+template <int LANES>
+__device__ __forceinline__ bool any_lane(bool yes) {
+    return (__ballot(yes) >> (threadIdx.x % kWave / LANES * LANES) & (~uint64_t(0) >> (kWave - LANES))) != 0;
+}
+
+template <int LANES, typename V>
+__device__ __forceinline__ V inclusive_sum(V v, int lane) {
+#pragma unroll
+    for (int s = 1; s < LANES; s <<= 1) {
+        const V up = __shfl_up(v, s, LANES);
+        if (lane >= s) v += up;
+    }
+    return v;
+}
+
+// The first lane whose value, none smaller than that of the lane before, is greater than k.
+template <int LANES, typename V>
+__device__ __forceinline__ int first_above(V values, V k) {
+    int p = 0;
+#pragma unroll
+    for (int s = LANES / 2; s > 0; s >>= 1)
+        if (__shfl(values, p + s - 1, LANES) <= k) p += s;
+    return p;
+}
+
+// Entries k of a vertex's list (neighbor_at), one a lane: its rules are searched LANES at a time, because one by one
+// each costs two loads that wait for each other, and a hub has hundreds.
+template <int LANES>
+__device__ __forceinline__ int64_t neighbors_at(const Graph &g, int64_t node, int64_t k, bool wanted, int lane) {
+    const int64_t v2v_start = g.v2v_ptr[node], v2v_count = g.v2v_ptr[node + 1] - v2v_start;
+    int64_t neighbor = -1;
+    if (wanted && k < v2v_count) {
+        neighbor = g.v2v_idx[v2v_start + k];
+        wanted = false;  // all lanes stay for the exchange below
+    }
+    if (g.v2r_ptr == nullptr) return neighbor;
+    k -= v2v_count;
+    const int64_t end = g.v2r_ptr[node + 1];
+    int64_t rule = -1;
+    for (int64_t e0 = g.v2r_ptr[node]; e0 < end && any_lane<LANES>(wanted && rule < 0); e0 += LANES) {
+        const int64_t mine = e0 + lane < end ? g.v2r_idx[e0 + lane] : -1;
+        const int64_t degree = mine >= 0 ? g.r_degree[mine] : 0;
+        const int64_t sum = inclusive_sum<LANES>(degree, lane);
+        int64_t most = sum;
+        if (any_lane<LANES>(degree < 0))  // then not every sum is above those in front of it
+#pragma unroll
+            for (int s = 1; s < LANES; s <<= 1) {
+                const int64_t up = __shfl_up(most, s, LANES);
+                if (lane >= s && up > most) most = up;
+            }
+        const int p = first_above<LANES>(most, k);
+        const int64_t found = __shfl(mine, p, LANES), before = __shfl(sum - degree, p, LANES);
+        const int64_t above = __shfl(most, LANES - 1, LANES), all = __shfl(sum, LANES - 1, LANES);
+        if (rule >= 0) continue;
+        if (k < above) {
+            rule = found;
+            k -= before;
+        } else {
+            k -= all;
+        }
+    }
+    return wanted && rule >= 0 ? below_rule(g, rule, k) : neighbor;
+}
+
+// LANES lanes per frontier vertex (as many as the fan-out asks for: a step waits for one load after another, and
+// with a wave per vertex most lanes of it wait for nothing), into the vertex's slots.  The first layer also
+// numbers the input, a vertex given twice by its first position.
+template <int LANES>
+__global__ __launch_bounds__(kBlock) void bounded_fill_kernel(BoundedArgs a) {
+    const BoundedLayer &l = a.at[a.layer];
+    const int lane = threadIdx.x % LANES;
+    const int64_t i = (int64_t)blockIdx.x * (kBlock / LANES) + threadIdx.x / LANES;
+    const int32_t first = a.state[4 * a.layer], n = a.state[4 * a.layer + 1];
+    if (i >= n) return;
+    const Graph &g = a.g;
+    const int fanout = (int)l.fanout;
+    const int64_t node = a.layer == 0 ? a.input[i] : a.samples[first + i], slot0 = i * fanout;
+    auto put = [&](int t, int64_t neighbor) {
+        if (neighbor < 0 || neighbor >= g.vertex_cnt) {
+            atomicCAS(a.status, CGNN_SAMPLE_OK, neighbor == -1 ? CGNN_SAMPLE_OUT_OF_RANGE : CGNN_SAMPLE_BAD_VERTEX);
+            neighbor = 0;
+        }
+        l.slots[slot0 + t] = (int32_t)neighbor;
+        const int32_t claim = kClaim + (int32_t)(slot0 + t);
+        if (a.number_of[neighbor] > claim) atomicMin(&a.number_of[neighbor], claim);
+    };
+    auto full_list = [&]() -> int {  // its length, or -1: longer than the fan-out (or by rules that lead nowhere)
+        const int64_t v2v_start = g.v2v_ptr[node], v2v_count = g.v2v_ptr[node + 1] - v2v_start;
+        if (v2v_count > fanout) return -1;
+        if (lane < v2v_count) put(lane, g.v2v_idx[v2v_start + lane]);
+        int count = (int)v2v_count;
+        if (g.v2r_ptr == nullptr) return count;
+        // Depth by depth, a rule a lane, in the order in which a walk in pre-order meets the rules of a depth.  Sizes
+        // are cut off where they are too large in any case, so that two sums fit into one.
+        const int64_t v2r_start = g.v2r_ptr[node], v2r_count = g.v2r_ptr[node + 1] - v2r_start;
+        if (v2r_count > LANES) return -1;
+        auto cut = [](int64_t size) { return (int)(size < 0 ? 0 : size > LANES ? LANES + 1 : size); };
+        int rules = (int)v2r_count;
+        int64_t rule = lane < rules ? g.v2r_idx[v2r_start + lane] : 0;
+        for (int depth = 0; rules > 0; ++depth) {
+            int64_t own_start = 0, child_start = 0;
+            int own = 0, children = 0;
+            if (lane < rules) {
+                own_start = g.r2v_ptr[rule];
+                own = cut(g.r2v_ptr[rule + 1] - own_start);
+                if (depth < g.levels) {
+                    child_start = g.r2r_ptr[depth][rule];
+                    children = cut(g.r2r_ptr[depth][rule + 1] - child_start);
+                }
+            }
+            const int sums = inclusive_sum<LANES>(own | children << 16, lane), all = __shfl(sums, LANES - 1, LANES);
+            const int owns = sums & 0xffff, all_own = all & 0xffff, descend = sums >> 16, all_descend = all >> 16;
+            if (count + all_own > fanout || all_descend > LANES) return -1;
+            const int p = first_above<LANES>(owns, lane);
+            const int64_t from = __shfl(own_start - (owns - own), p, LANES);
+            if (lane < all_own) put(count + lane, g.r2v_idx[from + lane]);
+            count += all_own;
+            rules = all_descend;
+            const int q = first_above<LANES>(descend, lane);
+            const int64_t child = __shfl(child_start - (descend - children), q, LANES);
+            if (lane < rules) rule = g.r2r_idx[depth][child + lane];
+        }
+        return count;
+    };
+    int count = 0;
+    if (node < 0 || node >= g.vertex_cnt) {
+        atomicCAS(a.status, CGNN_SAMPLE_OK, CGNN_SAMPLE_BAD_VERTEX);
+    } else {
+        if (a.layer == 0 && lane == 0) atomicMin(&a.number_of[node], (int32_t)i);
+        const int64_t degree = degree_of(g, node);
+        if (degree > fanout) {
+            // The selection loop of sample_fill_kernel with a step per lane: the draws do not depend on each other, only
+            // whether a drawn position was taken before does.
+            count = fanout;
+            const int64_t j = degree - count + lane;
+            int64_t pick = lane < count ? draw(a.seed, a.layer, first + i, j, j) : -1;
+            for (int s = 1; s < count; ++s) {
+                const int64_t rnd = __shfl(pick, s, LANES);
+                const bool taken = any_lane<LANES>(lane < s && pick == rnd);
+                if (lane == s && taken) pick = j;
+            }
+            const int64_t neighbor = neighbors_at<LANES>(g, node, pick, lane < count, lane);
+            if (lane < count) put(lane, neighbor);
+        } else if (degree > 0) {
+            count = full_list();
+            if (count < 0) {  // the call is done again layer by layer
+                a.status[1] = 1;
+                count = 0;
+            }
+        }
+    }
+    for (int t = count + lane; t < fanout; t += LANES) l.slots[slot0 + t] = -1;
+}
+
+// The slots of a thread in a chunk of a layer with `slots` of them: neighbours (or -1), and which introduce a vertex.
+struct ChunkSlots {
+    int32_t v[kChunkItems];
+    unsigned introduces;
+    int live, fresh;
+};
+
+__device__ __forceinline__ ChunkSlots chunk_slots(const BoundedArgs &a, const BoundedLayer &l, int64_t slots, int64_t chunk,
+                                                  bool ranks) {
+    ChunkSlots c;
+    const int64_t s0 = chunk * kChunk + threadIdx.x * kChunkItems;
+    if (s0 + kChunkItems <= slots) {
+        const int4 four = *reinterpret_cast<const int4 *>(l.slots + s0);
+        c.v[0] = four.x, c.v[1] = four.y, c.v[2] = four.z, c.v[3] = four.w;
+    } else {
+#pragma unroll
+        for (int u = 0; u < kChunkItems; ++u) c.v[u] = s0 + u < slots ? l.slots[s0 + u] : -1;
+    }
+    c.introduces = 0;
+    c.live = c.fresh = 0;
+    int32_t number[kChunkItems];
+#pragma unroll
+    for (int u = 0; u < kChunkItems; ++u)  // all loads before the first use
+        number[u] = ranks ? a.number_of[c.v[u] < 0 ? 0 : c.v[u]] : 0;
+#pragma unroll
+    for (int u = 0; u < kChunkItems; ++u) {
+        if (c.v[u] < 0) continue;
+        ++c.live;
+        if (number[u] == kClaim + (int32_t)(s0 + u)) {
+            c.introduces |= 1u << u;
+            ++c.fresh;
+        }
+    }
+    return c;
+}
+
+// Exclusive sums of two values over the workgroup, and the totals.
+__device__ __forceinline__ int2 chunk_sums(int live, int fresh, int2 *total) {
+    __shared__ int2 wave_sum[kBlock / kWave];
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    int a = live, b = fresh;
+#pragma unroll
+    for (int s = 1; s < kWave; s <<= 1) {
+        const int x = __shfl_up(a, s, kWave), y = __shfl_up(b, s, kWave);
+        if (lane >= s) a += x, b += y;
+    }
+    __syncthreads();
+    if (lane == kWave - 1) wave_sum[wave] = make_int2(a, b);
+    __syncthreads();
+    int2 before = make_int2(a - live, b - fresh), all = make_int2(0, 0);
+#pragma unroll
+    for (int w = 0; w < kBlock / kWave; ++w) {
+        if (w < wave) before.x += wave_sum[w].x, before.y += wave_sum[w].y;
+        all.x += wave_sum[w].x, all.y += wave_sum[w].y;
+    }
+    *total = all;
+    return before;
+}
+
+// How many neighbours a chunk holds and how many vertices they introduce; the last chunk to be counted sums the
+// chunks up and sets the state of the next layer.
+__global__ __launch_bounds__(kBlock) void bounded_count_kernel(BoundedArgs a) {
+    const BoundedLayer &l = a.at[a.layer];
+    int32_t *state = a.state + 4 * a.layer;
+    const int64_t n = state[1], held = ceil_div_dev(n * l.fanout, kChunk), chunks = held < 1 ? 1 : held;
+    if (blockIdx.x >= chunks) return;
+    const ChunkSlots c = chunk_slots(a, l, n * l.fanout, blockIdx.x, true);
+    int2 total;
+    chunk_sums(c.live, c.fresh, &total);
+    __shared__ bool arrived_last;
+    if (threadIdx.x == 0) {  // read by another XCD in this launch: as the pieces of workgroup runs (spmm.hip)
+        __hip_atomic_store(l.before + blockIdx.x, (uint64_t)total.y << 32 | (uint32_t)total.x, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_waitcnt(0);
+        arrived_last = __hip_atomic_fetch_add(state + 3, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == chunks - 1;
+    }
+    __syncthreads();
+    if (!arrived_last) return;
+    int2 running = make_int2(0, 0);
+    for (int64_t k0 = (int64_t)threadIdx.x * kTail; k0 - threadIdx.x * kTail < chunks; k0 += kBlock * kTail) {
+        uint64_t pair[kTail];
+        int2 sum = make_int2(0, 0), all;
+#pragma unroll
+        for (int u = 0; u < kTail; ++u)  // all loads in flight
+            pair[u] = k0 + u < chunks ? __hip_atomic_load(l.before + k0 + u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+#pragma unroll
+        for (int u = 0; u < kTail; ++u) sum.x += (int)(uint32_t)pair[u], sum.y += (int)(pair[u] >> 32);
+        int2 before = chunk_sums(sum.x, sum.y, &all);
+        before.x += running.x, before.y += running.y;
+#pragma unroll
+        for (int u = 0; u < kTail; ++u) {
+            if (k0 + u < chunks) l.before[k0 + u] = (uint64_t)before.y << 32 | (uint32_t)before.x;
+            before.x += (int)(uint32_t)pair[u], before.y += (int)(pair[u] >> 32);
+        }
+        running.x += all.x, running.y += all.y;
+    }
+    if (threadIdx.x == 0) {
+        const int32_t end = state[0] + (int32_t)n;
+        state[4] = end;
+        state[5] = running.y;
+        state[6] = state[2] + running.x;
+        if (a.layer == a.layers - 1) {
+            a.summary[0] = end + running.y;
+            a.summary[1] = state[2] + running.x;
+            a.summary[2] = a.status[1] ? -1 : a.status[0];
+            __hip_atomic_store(a.summary + 3, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+}
+
+// The vertices that a layer introduces take the numbers behind its frontier, in the order of their slots.
+__global__ __launch_bounds__(kBlock) void bounded_assign_kernel(BoundedArgs a) {
+    const BoundedLayer &l = a.at[a.layer];
+    const int32_t *state = a.state + 4 * a.layer;
+    const int64_t n = state[1];
+    if ((int64_t)blockIdx.x * kChunk >= n * l.fanout) return;
+    const ChunkSlots c = chunk_slots(a, l, n * l.fanout, blockIdx.x, true);
+    int2 total;
+    int32_t number = state[4] + (int32_t)(l.before[blockIdx.x] >> 32) + chunk_sums(c.live, c.fresh, &total).y;
+#pragma unroll
+    for (int u = 0; u < kChunkItems; ++u)
+        if (c.introduces >> u & 1u) {
+            // no other slot has this claim
+            a.number_of[c.v[u]] = number;
+            a.samples[number++] = c.v[u];
+        }
+}
+
+// The edges of all layers and the samples, in arrays of their exact sizes.
+__global__ __launch_bounds__(kBlock) void bounded_write_kernel(BoundedArgs a) {
+    const int64_t chunks = a.first_chunk[a.layers];
+    if ((int64_t)blockIdx.x >= chunks) {
+        const int64_t i = (blockIdx.x - chunks) * (int64_t)kBlock + threadIdx.x;
+        if (i < a.state[4 * a.layers] + a.state[4 * a.layers + 1]) a.out_samples[i] = i < a.n_input ? a.input[i] : a.samples[i];
+        return;
+    }
+    int layer = 0;
+    while (layer + 1 < a.layers && (int64_t)blockIdx.x >= a.first_chunk[layer + 1]) ++layer;
+    const BoundedLayer &l = a.at[layer];
+    const int32_t *state = a.state + 4 * layer;
+    const int64_t chunk = blockIdx.x - a.first_chunk[layer], n = state[1];
+    if (chunk * kChunk >= n * l.fanout) return;
+    const ChunkSlots c = chunk_slots(a, l, n * l.fanout, chunk, false);
+    int2 total;
+    int64_t e = (int64_t)state[2] + (int32_t)l.before[chunk] + chunk_sums(c.live, 0, &total).x;
+    int64_t i = (chunk * kChunk + threadIdx.x * kChunkItems) / l.fanout, t = chunk * kChunk + threadIdx.x * kChunkItems - i * l.fanout;
+#pragma unroll
+    for (int u = 0; u < kChunkItems; ++u) {
+        if (c.v[u] >= 0) {
+            a.out_source[e] = state[0] + i;
+            a.out_neighbor[e++] = a.number_of[c.v[u]];
+        }
+        if (++t == l.fanout) t = 0, ++i;
+    }
 }
 
 // ------------------------------------------------------------------- relabelling ----
@@ -571,4 +931,121 @@ extern "C" int cgnn_sample_relabel(int64_t total, const int64_t *neighbors, int6
     hipLaunchKernelGGL(relabel_lookup_kernel, dim3(blocks), dim3(kBlock), 0, stream, neighbors, total, local_of, seen_at,
                        numbers);
     return check_launch("sample_relabel");
+}
+
+// ------------------------------------------------------- layers of a bounded size ----
+namespace {
+
+struct BoundedLayout {
+    size_t number_of, samples, state, status, total;
+    size_t slots[CGNN_SAMPLE_MAX_BOUNDED], before[CGNN_SAMPLE_MAX_BOUNDED];
+    int64_t n_cap[CGNN_SAMPLE_MAX_BOUNDED], chunks[CGNN_SAMPLE_MAX_BOUNDED];
+    int64_t samples_cap;
+};
+
+// The most slots a call may have in all its layers: 512 MB of them.
+constexpr int64_t kMostSlots = int64_t(1) << 27;
+
+// false: the fan-outs do not bound the call well enough, or it has too many layers
+bool bounded_layout(int64_t vertex_cnt, int64_t n_input, int layers, const int64_t *fanouts, BoundedLayout *L) {
+    if (layers < 1 || layers > CGNN_SAMPLE_MAX_BOUNDED || n_input < 1 || vertex_cnt < 1) return false;
+    size_t at = 0;
+    auto take = [&](int64_t ints) {
+        const size_t here = at;
+        at += align_up((size_t)ints * sizeof(int32_t), 256);
+        return here;
+    };
+    L->number_of = take(vertex_cnt);
+    L->state = take(4 * (layers + 1));
+    L->status = take(2);
+    int64_t n = n_input, all = 0;
+    L->samples_cap = n_input;
+    for (int k = 0; k < layers; ++k) {
+        if (fanouts[k] < 1 || fanouts[k] > kRegPicks || n > kMostSlots / fanouts[k]) return false;
+        const int64_t slots = n * fanouts[k];
+        all += slots;
+        if (all > kMostSlots) return false;
+        L->n_cap[k] = n;
+        L->chunks[k] = ceil_div(slots, kChunk);
+        L->slots[k] = take(slots);
+        L->before[k] = take(2 * L->chunks[k]);
+        n = slots < vertex_cnt ? slots : vertex_cnt;  // a layer adds every vertex once
+        L->samples_cap += n;
+    }
+    if (L->samples_cap > n_input + vertex_cnt) L->samples_cap = n_input + vertex_cnt;
+    L->samples = take(L->samples_cap);
+    L->total = at;
+    return true;
+}
+
+BoundedArgs bounded_args(const cgnn_sample_graph *graph, int64_t n_input, const int64_t *input, int layers, const int64_t *fanouts,
+                         uint64_t seed, const BoundedLayout &L, void *workspace) {
+    BoundedArgs a{};
+    char *base = static_cast<char *>(workspace);
+    auto ints = [&](size_t at) { return reinterpret_cast<int32_t *>(base + at); };
+    a.g = graph_of(graph);
+    a.n_input = n_input;
+    a.input = input;
+    a.number_of = ints(L.number_of), a.samples = ints(L.samples);
+    a.state = ints(L.state), a.status = ints(L.status);
+    a.seed = seed;
+    a.layers = layers;
+    for (int k = 0; k < layers; ++k) {
+        a.at[k] = BoundedLayer{fanouts[k], L.n_cap[k], ints(L.slots[k]), reinterpret_cast<uint64_t *>(base + L.before[k])};
+        a.first_chunk[k + 1] = a.first_chunk[k] + L.chunks[k];
+    }
+    return a;
+}
+
+}  // namespace
+
+extern "C" size_t cgnn_sample_layers_workspace_bytes(int64_t vertex_cnt, int64_t n_input, int layers, const int64_t *fanouts) {
+    BoundedLayout L;
+    return fanouts != nullptr && vertex_cnt < INT32_MAX && bounded_layout(vertex_cnt, n_input, layers, fanouts, &L) ? L.total : 0;
+}
+
+extern "C" int cgnn_sample_layers(const cgnn_sample_graph *graph, int64_t n_input, const int64_t *input, int layers,
+                                  const int64_t *fanouts, uint64_t seed, int32_t *summary, void *workspace,
+                                  size_t workspace_bytes, cgnn_stream_t stream) {
+    int rc = check_graph(graph, "cgnn_sample_layers");
+    if (rc != CGNN_OK) return rc;
+    BoundedLayout L;
+    CGNN_REQUIRE(input && fanouts && summary, "cgnn_sample_layers: null array");
+    if (!bounded_layout(graph->vertex_cnt, n_input, layers, fanouts, &L))
+        return fail(CGNN_EUNSUPPORTED, "cgnn_sample_layers: these fan-outs do not bound the call (see the size query)");
+    if (workspace == nullptr || workspace_bytes < L.total) return fail(CGNN_EWORKSPACE, "cgnn_sample_layers: workspace too small");
+    BoundedArgs a = bounded_args(graph, n_input, input, layers, fanouts, seed, L, workspace);
+    a.summary = summary;
+    summary[3] = 0;
+    hipLaunchKernelGGL(bounded_begin_kernel, dim3(blocks_for(graph->vertex_cnt)), dim3(kBlock), 0, stream, a);
+    for (int k = 0; k < layers; ++k) {
+        a.layer = k;
+        const int lanes = fanouts[k] <= 16 ? 16 : fanouts[k] <= 32 ? 32 : kWave;
+        const dim3 grid((unsigned)ceil_div(L.n_cap[k], kBlock / lanes));
+        if (lanes == 16) hipLaunchKernelGGL((bounded_fill_kernel<16>), grid, dim3(kBlock), 0, stream, a);
+        else if (lanes == 32) hipLaunchKernelGGL((bounded_fill_kernel<32>), grid, dim3(kBlock), 0, stream, a);
+        else hipLaunchKernelGGL((bounded_fill_kernel<kWave>), grid, dim3(kBlock), 0, stream, a);
+        hipLaunchKernelGGL(bounded_count_kernel, dim3((unsigned)L.chunks[k]), dim3(kBlock), 0, stream, a);
+        hipLaunchKernelGGL(bounded_assign_kernel, dim3((unsigned)L.chunks[k]), dim3(kBlock), 0, stream, a);
+    }
+    return check_launch("sample_layers");
+}
+
+extern "C" int cgnn_sample_layers_write(const cgnn_sample_graph *graph, int64_t n_input, const int64_t *input, int layers,
+                                        const int64_t *fanouts, int64_t samples, int64_t edges, int64_t *out_samples,
+                                        int64_t *out_source, int64_t *out_neighbor, void *workspace, size_t workspace_bytes,
+                                        cgnn_stream_t stream) {
+    int rc = check_graph(graph, "cgnn_sample_layers_write");
+    if (rc != CGNN_OK) return rc;
+    BoundedLayout L;
+    CGNN_REQUIRE(input && fanouts && bounded_layout(graph->vertex_cnt, n_input, layers, fanouts, &L),
+                 "cgnn_sample_layers_write: not the arguments of cgnn_sample_layers");
+    CGNN_REQUIRE(samples >= n_input && samples <= L.samples_cap && edges >= 0, "cgnn_sample_layers_write: sizes are those of the summary");
+    CGNN_REQUIRE(out_samples && (edges == 0 || (out_source && out_neighbor)), "cgnn_sample_layers_write: null array");
+    if (workspace == nullptr || workspace_bytes < L.total) return fail(CGNN_EWORKSPACE, "cgnn_sample_layers_write: workspace too small");
+    BoundedArgs a = bounded_args(graph, n_input, input, layers, fanouts, 0, L, workspace);
+    a.out_samples = out_samples, a.out_source = out_source, a.out_neighbor = out_neighbor;
+    hipLaunchKernelGGL(bounded_write_kernel, dim3((unsigned)(a.first_chunk[layers] + ceil_div(samples, kBlock))), dim3(kBlock), 0,
+                       stream, a);
+    return check_launch("sample_layers_write");
 }

@@ -15,6 +15,7 @@
 #include <torch/extension.h>
 
 #include <algorithm>
+#include <chrono>
 #include <deque>
 #include <memory>
 #include <mutex>
@@ -1354,17 +1355,46 @@ std::tuple<Tensor, Tensor, Tensor> run_sampler(SampleGraph &G, const Tensor &inp
     auto u8 = input_node.options().dtype(torch::kUInt8);
     const Tensor input = input_node.contiguous();
     const int64_t n_input = input.numel();
+    auto raise_on = [&](int32_t code) {
+        TORCH_CHECK_INDEX(code != CGNN_SAMPLE_OUT_OF_RANGE, "Neighbor index out of range");
+        TORCH_CHECK(code != CGNN_SAMPLE_BAD_VERTEX, op, ": a vertex id outside [0, ", g.vertex_cnt, ")");
+        TORCH_CHECK(code != CGNN_SAMPLE_TOO_MANY, op, ": a layer of more than 2^31 - 2 neighbours");
+    };
+    const int layers = (int)std::min<size_t>(num_neighbors.size(), INT_MAX);
+    if (const size_t bytes = cgnn_sample_layers_workspace_bytes(g.vertex_cnt, n_input, layers, num_neighbors.data())) {
+        Tensor ws = torch::empty({(int64_t)bytes}, u8);
+        Tensor summary = torch::empty({4}, torch::TensorOptions().dtype(torch::kInt32).pinned_memory(true));
+        ok(cgnn_sample_layers(&g, n_input, input.data_ptr<int64_t>(), layers, num_neighbors.data(), (uint64_t)seed,
+                              summary.data_ptr<int32_t>(), ws.data_ptr(), bytes, stream),
+           op);
+        // The sizes are there while the last launch still runs: look for them for a while (a stream with little work ahead
+        // has them within 200 us), and otherwise wait for the stream, which also reports its errors.
+        const int32_t *sizes = summary.data_ptr<int32_t>();
+        const auto patience = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+        while (__atomic_load_n(sizes + 3, __ATOMIC_ACQUIRE) == 0)
+            if (std::chrono::steady_clock::now() > patience) {
+                TORCH_CHECK(hipStreamSynchronize(reinterpret_cast<hipStream_t>(stream)) == hipSuccess, op,
+                            ": the stream reported an error");
+                TORCH_CHECK(__atomic_load_n(sizes + 3, __ATOMIC_ACQUIRE) == 1, op, ": the sizes were not written");
+                break;
+            }
+        if (sizes[2] != -1) {  // -1: degrees that do not bound the lists; the layers then go one by one
+            raise_on(sizes[2]);
+            Tensor samples = torch::empty({sizes[0]}, i64), source = torch::empty({sizes[1]}, i64), neighbor = torch::empty({sizes[1]}, i64);
+            ok(cgnn_sample_layers_write(&g, n_input, input.data_ptr<int64_t>(), layers, num_neighbors.data(), sizes[0], sizes[1],
+                                        samples.data_ptr<int64_t>(), source.data_ptr<int64_t>(), neighbor.data_ptr<int64_t>(),
+                                        ws.data_ptr(), bytes, stream),
+               op);
+            if (swap_roles) return {samples, neighbor, source};
+            return {samples, source, neighbor};
+        }
+    }
     Tensor local_of = torch::empty({std::max<int64_t>(g.vertex_cnt, 1)}, i32), seen_at = torch::empty_like(local_of);
     Tensor status = torch::empty({1}, i32);
     ok(cgnn_sample_relabel_begin(g.vertex_cnt, n_input, n_input ? input.data_ptr<int64_t>() : nullptr,
                                  local_of.data_ptr<int32_t>(), seen_at.data_ptr<int32_t>(), status.data_ptr<int32_t>(),
                                  stream),
        op);
-    auto raise_on = [&](int32_t code) {
-        TORCH_CHECK_INDEX(code != CGNN_SAMPLE_OUT_OF_RANGE, "Neighbor index out of range");
-        TORCH_CHECK(code != CGNN_SAMPLE_BAD_VERTEX, op, ": a vertex id outside [0, ", g.vertex_cnt, ")");
-        TORCH_CHECK(code != CGNN_SAMPLE_TOO_MANY, op, ": a layer of more than 2^31 - 2 neighbours");
-    };
     Tensor samples = input.clone();
     std::vector<Tensor> sources, numbers;
     int64_t begin = 0, end = n_input;

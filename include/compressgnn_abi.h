@@ -448,6 +448,23 @@ int cgnn_sample_relabel(int64_t total, const int64_t *neighbors, int64_t base, i
                         int32_t *seen_at, int64_t *samples, int64_t *numbers, int64_t *new_count,
                         void *workspace, size_t workspace_bytes, cgnn_stream_t stream);
 
+/* All layers of a call whose fan-outs (each between 1 and 64, at most CGNN_SAMPLE_MAX_BOUNDED of them) bound its
+ * size: the same samples as the entries above, with one host read.  cgnn_sample_layers draws, numbers and counts;
+ * summary (pinned host memory) then holds the number of samples, the number of edges, a status of CGNN_SAMPLE_*, or -1
+ * if the full list of a vertex is not bounded by its degree, in which case the entries above have to be used, and, written
+ * last, before the stream has come to its end, 1.  cgnn_sample_layers_write, with the same arguments and workspace,
+ * writes samples[samples], and per edge the position of its vertex and of the neighbour among them.  Size
+ * query: 0 if the fan-outs do not bound the call. */
+#define CGNN_SAMPLE_MAX_BOUNDED 8
+size_t cgnn_sample_layers_workspace_bytes(int64_t vertex_cnt, int64_t n_input, int layers, const int64_t *fanouts);
+int cgnn_sample_layers(const cgnn_sample_graph *graph, int64_t n_input, const int64_t *input, int layers,
+                       const int64_t *fanouts, uint64_t seed, int32_t *summary, void *workspace, size_t workspace_bytes,
+                       cgnn_stream_t stream);
+int cgnn_sample_layers_write(const cgnn_sample_graph *graph, int64_t n_input, const int64_t *input, int layers,
+                             const int64_t *fanouts, int64_t samples, int64_t edges, int64_t *out_samples,
+                             int64_t *out_source, int64_t *out_neighbor, void *workspace, size_t workspace_bytes,
+                             cgnn_stream_t stream);
+
 /* --------------------------------------------------------------- utilities ---- */
 
 /* A plain device-to-device copy kernel of n bytes (n % 16 == 0); the calibration

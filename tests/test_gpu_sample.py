@@ -231,3 +231,42 @@ def test_sampler_errors():
         sampler.neighbor_sample_cg_sim(*on_device(lying), torch.from_numpy(with_rules).to(DEV), [worst - 1], seed=2)
     # the device is fine afterwards
     check(b, dev_blocks, np.array([1, 2, 3], np.int64), [2, 2], seed=3)
+
+
+@pytest.mark.parametrize("fan", [[15, 3], [16, 17], [31, 32], [33, 2], [64, 1], [65, 2], [1] * 8, [1] * 9])
+def test_layers_of_a_bounded_size(fan):
+    """Fan-outs around the lanes that a vertex gets and the bounds of the call with one host read; a hub whose 300 rules
+    are searched a chunk at a time (one with a negative degree); vertices whose full list is longer than their
+    degree says, or stands behind more rules than lanes."""
+    rng = np.random.default_rng(31)
+    V, R = 500, 400
+    csr = lambda lists: (np.concatenate([[0], np.cumsum([len(x) for x in lists])]).astype(np.int64),
+                         np.array([y for x in lists for y in x], np.int64))
+    own = [list(rng.integers(0, V, int(rng.integers(0, 4)))) for _ in range(R)]
+    children = [list(rng.integers(300, 340, int(rng.integers(0, 3)))) if r < 100 else [] for r in range(R)]
+    own[60], children[60] = [], []
+    own[360:] = [[] for _ in range(40)]
+    r_degree = np.array([len(own[r]) + sum(len(own[c]) for c in children[r]) for r in range(R)], np.int64)
+    v2r = [list(rng.integers(100, 340, int(rng.integers(0, 3)))) if v > 4 else [] for v in range(V)]
+    v2r[0], v2r[2], v2r[3] = list(range(300)), list(range(300, 330)), list(range(360, 400)) * 2
+    v2v = [list(rng.integers(0, V, int(rng.integers(0, 30)))) for _ in range(V)]
+    v2v[3] = [7, 8]
+    r_degree[60] = -1
+    v_degree = np.array([len(v2v[v]) + sum(int(r_degree[r]) for r in v2r[v]) for v in range(V)], np.int64)
+    v2v[4], v_degree[4] = list(range(20, 60)), 1
+    b = dict(v2v=csr(v2v), v2r=csr(v2r), r2v=csr(own), r2r=[csr(children)], v_degree=v_degree, r_degree=r_degree)
+    dev = on_device(b)
+    for inp in ([0, 1, 0, 2], [3, 1], [4, 0], np.arange(5, V), rng.integers(5, V, 1024 * 64 // max(fan[0], 1) + 1)):
+        check(b, dev, np.asarray(inp, np.int64), fan, seed=int(rng.integers(0, 10 ** 9)))
+
+
+def test_layers_of_many_chunks():
+    """More slots than the workgroup that ranks them sums up in one step."""
+    rng = np.random.default_rng(32)
+    b = dict(v2v=(np.arange(3001, dtype=np.int64) * 70, rng.integers(0, 3000, 210000)))
+    inp = rng.integers(0, 3000, 34000)
+    t = lambda a: torch.from_numpy(a).to(DEV)
+    import compressgnn_sample as sampler
+    got = sampler.neighbor_sample_ori_impl(t(b["v2v"][0]), t(b["v2v"][1]), t(inp), [64], seed=5)
+    for a, w in zip(got, oracle.neighbor_sample(b, inp, [64], seed=5, plain=True)):
+        assert np.array_equal(a.cpu().numpy(), w)
