@@ -21,7 +21,7 @@ EXPORTS = [
     "cgnn_spmm_static_scratch_bytes", "cgnn_spmm_static_init", "cgnn_spmm_static",
     "cgnn_csr_prepare_i64", "cgnn_csr_expand_rows", "cgnn_narrow_ids", "cgnn_csr_compose_columns",
     "cgnn_csr_transpose_workspace_bytes", "cgnn_csr_transpose_device",
-    "cgnn_compress_batch_workspace_bytes", "cgnn_compress_csr_batch_device",
+    "cgnn_compress_batch_workspace_bytes", "cgnn_compress_csr_batch_device", "cgnn_compress_batch_rows", "cgnn_compress_batch_feed", "cgnn_compress_batch_rounds",
     "cgnn_lsh_scan_workspace_bytes", "cgnn_lsh_hash", "cgnn_lsh_scan", "cgnn_lsh_finish",
     "cgnn_lsh_group_workspace_bytes", "cgnn_lsh_group", "cgnn_lsh_group_small_rows", "cgnn_cluster_sums_workspace_bytes",
     "cgnn_cluster_sums", "cgnn_column_sums_workspace_bytes", "cgnn_column_sums",

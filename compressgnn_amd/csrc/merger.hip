@@ -4,29 +4,37 @@
 // (src/offline/bindings/batch_cuda.cpp:3-9, module compressgnn_batch_cuda; its
 // kernels are not part of the reference tree).
 //
-// A round, on the sequence of all rows laid end to end (L entries):
-//   1. key[e] = (seq[e], seq[e+1]) for every e that is not the last entry of its row;
-//      the keys are sorted and run-length encoded, the pairs that occur at least
-//      min_pair_frequency times are the candidates, in ascending key order.
+// A round, on the sequence of all rows laid end to end (L entries; the last entry of a row carries a flag bit):
+//   1. The pairs (seq[e], seq[e+1]) within the rows that occur at least min_pair_frequency times are the
+//      candidates, in ascending order.
 //   2. Greedy left-to-right parse of every row with all candidates.  A position is
 //      "matched" if its pair is a candidate; the greedy parse takes the 1st, 3rd, 5th ...
 //      position of every maximal stretch of matched positions (the last entry of a row
-//      is never matched, so stretches do not cross rows).  With lz[e] = the last
-//      unmatched position <= e (a running maximum), position e is taken iff it is matched
-//      and e - lz[e] is odd: no sequential walk of a row, however long.
+//      is never matched, so stretches do not cross rows): no sequential walk of a row, however long.
 //   3. Candidates taken at least twice become rules, numbered in key order.
-//   4. The parse is repeated with the rules only; taken positions emit the rule, the
-//      position behind a taken one emits nothing, all others emit their entry; output
-//      positions are a prefix sum, and the new row starts are the output positions of
-//      the old ones.
-// Sorting, run-length encoding, selection and the prefix scans are rocPRIM's (through
-// hipCUB); their results do not depend on timing, the counters of step 2 are integer
-// sums, so the arrays are the same run to run and equal the host routine's.
+//   4. The parse is repeated with the rules only; a taken position becomes the rule, the position behind it goes.
 //
-// Offline work: the entry point waits for the device three times per round (three
-// counts decide how the round goes on).
+// What bounds a round is how often it goes over the sequence and at what price, so each step keeps fewer positions:
+//   - Only the pairs that can be candidates are looked at: in the first round all, later those with a rule of the round
+//     before in them and those that were candidates in it.  (Another pair was there before and was no candidate, and a
+//     round makes no pair of old entries more frequent.)
+//   - These are counted in a table by their hash alone, an upper bound of how often they occur; the counters stop at
+//     min_pair_frequency, so that a pair met a thousand times costs its counter no thousand atomics one after the other.
+//   - The positions that pass (one in seven of a web graph at 16) are listed in order, and their pairs
+//     counted exactly in a table of keys.  The candidates are sorted, nothing else is.
+//   - Both parses run over the list.  Positions taken are bits of a map, whose prefix sums move the entries
+//     and the row starts.
+// Sorting all pairs in every round (eight passes over 64-bit keys, run-length encoding, selection, a binary search per
+// position, scans over all positions) took 1,950 us of the device for the three rounds of 325,557 rows and 3.2 million
+// entries; this takes 700 us, 220 of them while the sequence still arrives (cgnn_compress_batch_feed).
+//
+// Timing decides where an atomic lands, never what comes of it: counts and sums are whole numbers, lists are in
+// order of position or sorted, so the arrays are the same run to run and equal the host routine's.
+//
+// Offline work: the entry point waits for the device twice per round (the number of candidates, the new length).
 #include <hipcub/hipcub.hpp>
 
+#include <chrono>
 #include <utility>
 
 #include "common.h"
@@ -34,11 +42,43 @@
 namespace cgnn {
 namespace {
 
-constexpr uint64_t kNoPair = ~0ull;
 constexpr int64_t kMergerLimit = (int64_t)INT32_MAX - 65536;
+constexpr uint32_t kLast = 0x80000000u;   // of an entry of the sequence: the last one of its row
+constexpr uint64_t kEmpty = ~0ull;
+constexpr int kItems = 8;
+constexpr int kTile = kItems * kBlock;    // positions per workgroup
+constexpr int kTileWords = kTile / 64;
+constexpr int kScanBlock = 1024;
+// Up to this many candidates are ranked by comparing all with all (10,821: 5 us); the radix sort's launches
+// alone take 40 us, and at 16,384 the comparisons do, too.
+constexpr int32_t kRankAll = 16384;
 
-struct MaxOp {
-    __device__ __forceinline__ int32_t operator()(int32_t a, int32_t b) const { return a > b ? a : b; }
+enum Scalar { kBad, kActive, kListed, kCandidates, kAdded, kTakenTotal, kNextActive, kScalars = 8 };
+
+struct Merger {
+    int64_t V;
+    int32_t L, min_frequency, rules;   // rules: numbered before this round
+    int32_t listed, candidates;        // once the host has read them
+    int key_bits;                      // of one entry
+    bool first;
+    uint32_t *seq, *next_seq;
+    int32_t *ptr, *next_ptr;
+    uint8_t *active, *next_active;     // [L] of all rounds but the first
+    uint32_t *filter;                  // counters by hash; the same memory as table_key
+    uint32_t *frequent;                // a bit for each: it got to min_frequency
+    uint64_t *words;                   // [L / 64] positions that pass the filter
+    int32_t *tile;                     // [tiles] sums in front of a tile, or its last start of a stretch
+    int32_t *tile_start;
+    int32_t *position, *slot, *candidate;  // [listed] slot of the table; -1: the pair is no candidate
+    uint64_t *table_key;
+    int32_t *table_count;              // later the rank of the slot's candidate, -1: none
+    uint64_t *cand_key, *sorted_key;   // [candidates] (first entry << key_bits) | second
+    int32_t *cand_slot, *sorted_slot, *cand_rank;
+    int32_t *uses, *rule_of;           // [candidates] in order
+    uint64_t *matched, *taken;         // [L / 64]
+    int32_t *word_sum;                 // [L / 64] taken positions of the tile in front of a word
+    int32_t *children;
+    int32_t *scalar;                   // [kScalars]
 };
 
 unsigned merger_grid(int64_t n) {
@@ -46,149 +86,533 @@ unsigned merger_grid(int64_t n) {
     return (unsigned)(b > 262144 ? 262144 : (b < 1 ? 1 : b));
 }
 
+unsigned tiles_of(int64_t n) { return (unsigned)(n < 1 ? 1 : ceil_div(n, kTile)); }
+
 #define CGNN_GRID_LOOP(i, n) \
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < (n); i += (int64_t)gridDim.x * blockDim.x)
 
-__global__ void merger_init_kernel(const int64_t *__restrict__ vlist, const int64_t *__restrict__ elist, int64_t V,
-                                   int64_t E, int32_t *__restrict__ ptr, int32_t *__restrict__ seq,
-                                   int32_t *__restrict__ bad) {
-    CGNN_GRID_LOOP(i, (V + 1 > E ? V + 1 : E)) {
-        if (i <= V) {
-            const int64_t p = vlist[i];
-            if (p < 0 || p > E || (i > 0 && p < vlist[i - 1]) || (i == 0 && p != 0) || (i == V && p != E)) *bad = 1;
-            ptr[i] = (int32_t)p;
+__device__ __forceinline__ int64_t ceil_div_dev(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+__device__ __forceinline__ uint64_t pair_hash(uint64_t k) {
+    k ^= k >> 33;
+    k *= 0xff51afd7ed558ccdULL;
+    k ^= k >> 33;
+    return k * 0x9e3779b97f4a7c15ULL;
+}
+
+// Bits of a table with more than n entries.
+__device__ __forceinline__ int table_bits(int32_t n) { return n <= 0 ? 1 : 32 - __clz(n); }
+
+__device__ __forceinline__ int load_now(const int32_t *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Exclusive sums over the workgroup.
+template <int BLOCK>
+__device__ __forceinline__ int block_scan(int v, int *total) {
+    __shared__ int wave_sum[BLOCK / kWave];
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    int sum = v;
+#pragma unroll
+    for (int s = 1; s < kWave; s <<= 1) {
+        const int up = __shfl_up(sum, s, kWave);
+        if (lane >= s) sum += up;
+    }
+    __syncthreads();
+    if (lane == kWave - 1) wave_sum[wave] = sum;
+    __syncthreads();
+    int before = sum - v, all = 0;
+#pragma unroll
+    for (int w = 0; w < BLOCK / kWave; ++w) {
+        if (w < wave) before += wave_sum[w];
+        all += wave_sum[w];
+    }
+    *total = all;
+    return before;
+}
+
+// Row starts, where rows end (bits of `taken`, which the first round has no other use for yet) and the counters.
+template <typename In>
+__global__ void merger_rows_kernel(Merger m, const In *__restrict__ vlist, int64_t E) {
+    CGNN_GRID_LOOP(i, m.V + 1) {
+        const int64_t p = vlist[i], before = i > 0 ? (int64_t)vlist[i - 1] : 0;
+        if (p < before || p > E || (i == 0 && p != 0) || (i == m.V && p != E)) m.scalar[kBad] = 1;
+        m.ptr[i] = (int32_t)(p < 0 || p > E ? 0 : p);
+        if (p > before && p <= E && before >= 0)
+            atomicOr(reinterpret_cast<unsigned long long *>(m.taken + (p - 1) / 64), 1ull << ((p - 1) % 64));
+    }
+}
+
+// Where the round begins: the counters, and scalars of this round.
+__global__ void merger_begin_kernel(Merger m) {
+    const int32_t n = m.first ? m.L : m.scalar[kNextActive];
+    const int64_t counters = (int64_t)2 << table_bits(n), words = ((int64_t)m.L + kTile - 1) / kTile * kTileWords;
+    CGNN_GRID_LOOP(i, counters / 4) reinterpret_cast<int4 *>(m.filter)[i] = make_int4(0, 0, 0, 0);
+    CGNN_GRID_LOOP(i, ceil_div_dev(counters, 32)) m.frequent[i] = 0;
+    if (m.first) CGNN_GRID_LOOP(i, words) m.taken[i] = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        m.scalar[kActive] = n;
+        m.scalar[kCandidates] = 0;
+        if (m.first) m.scalar[kBad] = 0;
+    }
+}
+
+// A counter goes up unless it got to min_frequency, as far as the caller has seen.
+__device__ __forceinline__ void count_pair(const Merger &m, uint64_t counter, uint32_t seen) {
+    if (seen < (uint32_t)m.min_frequency && atomicAdd(m.filter + counter, 1u) == (uint32_t)m.min_frequency - 1)
+        atomicOr(m.frequent + counter / 32, 1u << (counter % 32));
+}
+
+// Entries [from, from + n) of the first round's sequence, and the pairs that end there.
+template <typename In>
+__global__ __launch_bounds__(kBlock) void merger_feed_kernel(Merger m, const In *__restrict__ elist, int64_t from, int64_t n) {
+    const int shift = 63 - table_bits(m.L);
+    const int64_t i0 = from + (int64_t)blockIdx.x * kTile + threadIdx.x, end = from + n;
+    uint64_t counter[kItems];
+    uint32_t seen[kItems];
+#pragma unroll
+    for (int u = 0; u < kItems; ++u) {
+        const int64_t i = i0 + u * kBlock;
+        counter[u] = kEmpty;
+        if (i >= end) continue;
+        int64_t c = elist[i], before = i > 0 ? (int64_t)elist[i - 1] : 0;
+        if (c < 0 || c >= m.V) {
+            m.scalar[kBad] = 1;
+            c = 0;
         }
-        if (i < E) {
-            const int64_t c = elist[i];
-            if (c < 0 || c >= V) *bad = 1;
-            seq[i] = (int32_t)c;
+        if (before < 0 || before >= m.V) before = 0;
+        const bool last = m.taken[i / 64] >> (i % 64) & 1;
+        m.seq[i] = (uint32_t)c | (last ? kLast : 0);
+        if (i > 0 && !(m.taken[(i - 1) / 64] >> ((i - 1) % 64) & 1))
+            counter[u] = pair_hash((uint64_t)before << 32 | (uint64_t)c) >> shift;
+    }
+#pragma unroll
+    for (int u = 0; u < kItems; ++u)
+        if (counter[u] != kEmpty) seen[u] = __hip_atomic_load(m.filter + counter[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int u = 0; u < kItems; ++u)
+        if (counter[u] != kEmpty) count_pair(m, counter[u], seen[u]);
+}
+
+// The pair at e, or kEmpty: none, or none that can be a candidate.
+__device__ __forceinline__ uint64_t pair_at(const Merger &m, int64_t e) {
+    if (e + 1 >= m.L || (!m.first && m.active[e] == 0)) return kEmpty;
+    const uint32_t x = m.seq[e], y = m.seq[e + 1];
+    return (x & kLast) ? kEmpty : (uint64_t)x << 32 | (y & ~kLast);
+}
+
+__global__ __launch_bounds__(kBlock) void merger_count_kernel(Merger m) {
+    const int shift = 63 - table_bits(m.scalar[kActive]);
+    const int64_t e0 = (int64_t)blockIdx.x * kTile + threadIdx.x;
+    uint64_t key[kItems];
+    uint64_t counter[kItems];
+    uint32_t seen[kItems];
+#pragma unroll
+    for (int u = 0; u < kItems; ++u) key[u] = pair_at(m, e0 + u * kBlock);
+#pragma unroll
+    for (int u = 0; u < kItems; ++u)
+        if (key[u] != kEmpty) {
+            counter[u] = pair_hash(key[u]) >> shift;
+            seen[u] = __hip_atomic_load(m.filter + counter[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+#pragma unroll
+    for (int u = 0; u < kItems; ++u)
+        if (key[u] != kEmpty) count_pair(m, counter[u], seen[u]);
+}
+
+__global__ __launch_bounds__(kBlock) void merger_pass_kernel(Merger m) {
+    __shared__ int passed[kBlock / kWave];
+    const int shift = 63 - table_bits(m.scalar[kActive]);
+    const int64_t e0 = (int64_t)blockIdx.x * kTile + threadIdx.x;
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    uint64_t key[kItems];
+    uint32_t seen[kItems];
+#pragma unroll
+    for (int u = 0; u < kItems; ++u) key[u] = pair_at(m, e0 + u * kBlock);
+#pragma unroll
+    for (int u = 0; u < kItems; ++u) {
+        const uint64_t counter = key[u] == kEmpty ? 0 : pair_hash(key[u]) >> shift;
+        seen[u] = m.frequent[counter / 32] >> (counter % 32) & 1;
+    }
+    int count = 0;
+#pragma unroll
+    for (int u = 0; u < kItems; ++u) {
+        const uint64_t word = __ballot(key[u] != kEmpty && seen[u] != 0);
+        if (lane == 0) m.words[(int64_t)blockIdx.x * kTileWords + u * (kBlock / kWave) + wave] = word;
+        count += __popcll(word);
+    }
+    if (lane == 0) passed[wave] = count;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int all = 0;
+        for (int w = 0; w < kBlock / kWave; ++w) all += passed[w];
+        m.tile[blockIdx.x] = all;
+    }
+}
+
+// Sums of the tiles in front of every tile, and the total.
+__global__ __launch_bounds__(kScanBlock) void merger_tile_sums_kernel(int32_t *__restrict__ tile, int32_t tiles,
+                                                                      int32_t *__restrict__ total) {
+    int running = 0;
+    for (int32_t k0 = 0; k0 < tiles; k0 += kScanBlock * kItems) {
+        const int32_t k = k0 + threadIdx.x * kItems;
+        int v[kItems], sum = 0, all;
+#pragma unroll
+        for (int u = 0; u < kItems; ++u) v[u] = k + u < tiles ? tile[k + u] : 0;
+#pragma unroll
+        for (int u = 0; u < kItems; ++u) sum += v[u];
+        int before = running + block_scan<kScanBlock>(sum, &all);
+#pragma unroll
+        for (int u = 0; u < kItems; ++u) {
+            if (k + u < tiles) tile[k + u] = before;
+            before += v[u];
+        }
+        running += all;
+    }
+    if (threadIdx.x == 0) *total = running;
+}
+
+__global__ void merger_clear_table_kernel(Merger m) {
+    const int64_t slots = (int64_t)1 << table_bits(m.scalar[kListed]);
+    CGNN_GRID_LOOP(i, slots / 2) {
+        reinterpret_cast<ulonglong2 *>(m.table_key)[i] = make_ulonglong2(kEmpty, kEmpty);
+        reinterpret_cast<int2 *>(m.table_count)[i] = make_int2(0, 0);
+    }
+}
+
+// The list of positions, and how often their pairs occur.  Tables have more slots than pairs, so every probe ends.
+__global__ __launch_bounds__(kBlock) void merger_collect_kernel(Merger m) {
+    __shared__ int before[kTileWords];
+    const uint64_t *words = m.words + (int64_t)blockIdx.x * kTileWords;
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    if (wave == 0) {
+        const int mine = lane < kTileWords ? __popcll(words[lane]) : 0;
+        int sum = mine;
+#pragma unroll
+        for (int s = 1; s < kTileWords; s <<= 1) {
+            const int up = __shfl_up(sum, s, kWave);
+            if (lane >= s) sum += up;
+        }
+        if (lane < kTileWords) before[lane] = m.tile[blockIdx.x] + sum - mine;
+    }
+    __syncthreads();
+    const int bits = table_bits(m.scalar[kListed]);
+    const uint64_t mask = ((uint64_t)1 << bits) - 1;
+#pragma unroll
+    for (int u = 0; u < kItems; ++u) {
+        const int w = u * (kBlock / kWave) + wave;
+        const uint64_t word = words[w];
+        if (!(word >> lane & 1)) continue;
+        const int64_t e = (int64_t)blockIdx.x * kTile + u * kBlock + threadIdx.x;
+        const uint64_t key = (uint64_t)m.seq[e] << 32 | (m.seq[e + 1] & ~kLast);
+        const int32_t k = before[w] + __popcll(word & (((uint64_t)1 << lane) - 1));
+        uint64_t h = pair_hash(key) >> (64 - bits);
+        for (;;) {
+            uint64_t there = __hip_atomic_load(m.table_key + h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (there == kEmpty) there = atomicCAS(reinterpret_cast<unsigned long long *>(m.table_key + h), kEmpty, key);
+            if (there == kEmpty || there == key) break;
+            h = (h + 1) & mask;
+        }
+        if (load_now(m.table_count + h) < m.min_frequency) atomicAdd(m.table_count + h, 1);
+        m.position[k] = (int32_t)e;
+        m.slot[k] = (int32_t)h;
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void merger_candidates_kernel(Merger m) {
+    __shared__ int base;
+    const int64_t slots = (int64_t)1 << table_bits(m.scalar[kListed]);
+    for (int64_t t0 = (int64_t)blockIdx.x * kTile; t0 < slots; t0 += (int64_t)gridDim.x * kTile) {
+        unsigned is = 0;
+#pragma unroll
+        for (int u = 0; u < kItems; ++u) {
+            const int64_t i = t0 + u * kBlock + threadIdx.x;
+            if (i < slots && m.table_count[i] >= m.min_frequency) is |= 1u << u;
+        }
+        int all;
+        int j = block_scan<kBlock>(__popc(is), &all);
+        if (threadIdx.x == 0) base = all > 0 ? atomicAdd(m.scalar + kCandidates, all) : 0;
+        __syncthreads();
+        j += base;
+#pragma unroll
+        for (int u = 0; u < kItems; ++u) {
+            const int64_t i = t0 + u * kBlock + threadIdx.x;
+            if (is >> u & 1) {
+                const uint64_t key = m.table_key[i];
+                m.cand_key[j] = (key >> 32) << m.key_bits | (uint32_t)key;
+                m.cand_slot[j] = (int32_t)i;
+                m.cand_rank[j++] = 0;
+            } else if (i < slots) {
+                m.table_count[i] = -1;
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// Ranks of a few candidates: a workgroup compares kBlock of them with kBlock others.
+__global__ __launch_bounds__(kBlock) void merger_rank_kernel(Merger m) {
+    __shared__ uint64_t other[kBlock];
+    const int32_t i = blockIdx.x * kBlock + threadIdx.x, j = blockIdx.y * kBlock + threadIdx.x;
+    other[threadIdx.x] = j < m.candidates ? m.cand_key[j] : kEmpty;
+    __syncthreads();
+    if (i >= m.candidates) return;
+    const uint64_t key = m.cand_key[i];
+    int smaller = 0;
+#pragma unroll 8
+    for (int t = 0; t < kBlock; ++t) smaller += other[t] < key;
+    if (smaller > 0) atomicAdd(m.cand_rank + i, smaller);
+}
+
+// The candidates take their places; their uses, the maps of the parses and the count of the next round start at nothing.
+__global__ void merger_place_kernel(Merger m) {
+    const bool ranked = m.candidates <= kRankAll;
+    const int64_t words = ((int64_t)m.L + kTile - 1) / kTile * kTileWords, n = m.candidates > words ? m.candidates : words;
+    if (blockIdx.x == 0 && threadIdx.x == 0) m.scalar[kNextActive] = 0;
+    CGNN_GRID_LOOP(i, n) {
+        if (i < words) m.matched[i] = m.taken[i] = 0;
+        if (i < m.candidates) {
+            const int32_t r = ranked ? m.cand_rank[i] : (int32_t)i;
+            if (ranked) m.sorted_key[r] = m.cand_key[i];
+            m.table_count[ranked ? m.cand_slot[i] : m.sorted_slot[i]] = r;
+            m.uses[i] = 0;
         }
     }
 }
 
-__global__ void merger_fill_kernel(int32_t *__restrict__ a, int32_t value, int64_t n) {
-    CGNN_GRID_LOOP(i, n) a[i] = value;
+// A parse takes the list a tile per workgroup and 64 positions per wave and step.  First half: which positions are
+// matched (RULES: by the rules only), and the last start of a stretch in every tile.
+struct Match {
+    int32_t by, at;  // candidate or rule, -1: none; position
+    bool starts;
+};
+
+template <bool RULES, bool FIND>
+__device__ __forceinline__ Match match_at(const Merger &m, int32_t k) {
+    auto matched_by = [&](int32_t i) {
+        const int32_t c = FIND ? m.table_count[m.slot[i]] : m.candidate[i];
+        return RULES && c >= 0 ? m.rule_of[c] : c;
+    };
+    Match a{-1, -1, false};
+    if (k >= m.listed) return a;
+    a.by = matched_by(k);
+    a.at = m.position[k];
+    if (a.by >= 0) a.starts = k == 0 || m.position[k - 1] != a.at - 1 || matched_by(k - 1) < 0;
+    return a;
 }
 
-// last[e] = 1 for the last entry of every non-empty row.
-__global__ void merger_mark_last_kernel(const int32_t *__restrict__ ptr, int64_t V, int32_t *__restrict__ last) {
-    CGNN_GRID_LOOP(v, V) {
-        if (ptr[v + 1] > ptr[v]) last[ptr[v + 1] - 1] = 1;
-    }
+__device__ __forceinline__ int32_t wave_begin() {
+    return blockIdx.x * kTile + threadIdx.x / kWave * (kItems * kWave);
 }
 
-__global__ void merger_keys_kernel(const int32_t *__restrict__ seq, const int32_t *__restrict__ last, int64_t L,
-                                   uint64_t *__restrict__ keys) {
-    CGNN_GRID_LOOP(e, L) {
-        keys[e] = last[e] ? kNoPair : (((uint64_t)(uint32_t)seq[e] << 32) | (uint32_t)seq[e + 1]);
-    }
-}
-
-__global__ void merger_candidate_flags_kernel(const uint64_t *__restrict__ unique, const int32_t *__restrict__ counts,
-                                              const int32_t *__restrict__ runs, int64_t L, int32_t min_frequency,
-                                              char *__restrict__ flags) {
-    const int64_t n = *runs;
-    CGNN_GRID_LOOP(i, L) flags[i] = (i < n && counts[i] >= min_frequency && unique[i] != kNoPair) ? 1 : 0;
-}
-
-// idx[e] = index of key[e] among the candidates, or -1.
-__global__ void merger_lookup_kernel(const uint64_t *__restrict__ keys, int64_t L,
-                                     const uint64_t *__restrict__ cand, int32_t ncand, int32_t *__restrict__ idx) {
-    CGNN_GRID_LOOP(e, L) {
-        const uint64_t k = keys[e];
-        int32_t lo = 0, hi = ncand;
-        while (lo < hi) {
-            const int32_t mid = (lo + hi) >> 1;
-            if (cand[mid] < k) lo = mid + 1;
-            else hi = mid;
+template <bool RULES>
+__global__ __launch_bounds__(kBlock) void merger_match_kernel(Merger m) {
+    __shared__ int32_t wave_start[kBlock / kWave];
+    const int lane = threadIdx.x % kWave;
+    const int32_t k0 = wave_begin();
+    int32_t last = -1;
+#pragma unroll
+    for (int u = 0; u < kItems; ++u) {
+        const int32_t k = k0 + u * kWave + lane;
+        const Match a = match_at<RULES, !RULES>(m, k);
+        const uint64_t starts = __ballot(a.starts);
+        if (starts != 0) last = k0 + u * kWave + 63 - __clzll(starts);
+        if (!RULES && k < m.listed) {
+            m.candidate[k] = a.by;
+            if (a.by >= 0) atomicOr(reinterpret_cast<unsigned long long *>(m.matched + a.at / 64), 1ull << (a.at % 64));
         }
-        idx[e] = (lo < ncand && cand[lo] == k) ? lo : -1;  // kNoPair is never a candidate
+    }
+    if (lane == 0) wave_start[threadIdx.x / kWave] = last;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 0; w < kBlock / kWave; ++w) last = max(last, wave_start[w]);
+        m.tile_start[blockIdx.x] = last;
     }
 }
 
-// z[e] = e where position e is unmatched, -1 where it is matched (kept == NULL: every candidate counts).
-__global__ void merger_unmatched_kernel(const int32_t *__restrict__ idx, const int32_t *__restrict__ kept,
-                                        int64_t L, int32_t *__restrict__ z) {
-    CGNN_GRID_LOOP(e, L) {
-        const int32_t c = idx[e];
-        const bool matched = c >= 0 && (kept == nullptr || kept[c] != 0);
-        z[e] = matched ? -1 : (int32_t)e;
+// Second half: every other position of a stretch is taken.  Without RULES it counts as a use, of which only
+// the first two matter; with RULES the rule takes its place in the sequence.
+template <bool RULES>
+__global__ __launch_bounds__(kBlock) void merger_take_kernel(Merger m) {
+    __shared__ int32_t wave_start[kBlock / kWave], carried;
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int32_t k0 = wave_begin();
+    Match a[kItems];
+    uint64_t starts[kItems];
+    int32_t last = -1;
+#pragma unroll
+    for (int u = 0; u < kItems; ++u) {
+        a[u] = match_at<RULES, false>(m, k0 + u * kWave + lane);
+        starts[u] = __ballot(a[u].starts);
+        if (starts[u] != 0) last = k0 + u * kWave + 63 - __clzll(starts[u]);
     }
-}
-
-__device__ __forceinline__ bool merger_taken(const int32_t *idx, const int32_t *kept, const int32_t *lz, int64_t e) {
-    const int32_t c = idx[e];
-    if (c < 0 || (kept != nullptr && kept[c] == 0)) return false;
-    return ((e - (int64_t)lz[e]) & 1) != 0;
-}
-
-__global__ void merger_count_uses_kernel(const int32_t *__restrict__ idx, const int32_t *__restrict__ lz, int64_t L,
-                                         int32_t *__restrict__ uses) {
-    CGNN_GRID_LOOP(e, L) {
-        if (merger_taken(idx, nullptr, lz, e)) atomicAdd(&uses[idx[e]], 1);
-    }
-}
-
-__global__ void merger_kept_kernel(const int32_t *__restrict__ uses, int32_t ncand, int32_t *__restrict__ kept) {
-    CGNN_GRID_LOOP(c, ncand) kept[c] = uses[c] >= 2 ? 1 : 0;
-}
-
-// children of the new rules, and the number of rules added (rank[c] = kept candidates before c).
-__global__ void merger_rules_kernel(const uint64_t *__restrict__ cand, const int32_t *__restrict__ kept,
-                                    const int32_t *__restrict__ rank, int32_t ncand, int64_t rules_before,
-                                    int32_t *__restrict__ children, int32_t *__restrict__ added) {
-    CGNN_GRID_LOOP(c, ncand) {
-        if (kept[c]) {
-            const int64_t r = rules_before + rank[c];
-            children[2 * r] = (int32_t)(cand[c] >> 32);
-            children[2 * r + 1] = (int32_t)(cand[c] & 0xffffffffu);
+    if (lane == 0) wave_start[wave] = last;
+    if (wave == 0) {  // the last start in front of the tile
+        int32_t found = -1;
+        for (int32_t b = (int32_t)blockIdx.x; b > 0 && found < 0; b -= kWave) {
+            const int32_t s = b - 1 - lane >= 0 ? m.tile_start[b - 1 - lane] : -1;
+            const uint64_t any = __ballot(s >= 0);
+            if (any != 0) found = __shfl(s, __ffsll((unsigned long long)any) - 1, kWave);
         }
-        if (c == ncand - 1) *added = rank[c] + kept[c];
+        if (lane == 0) carried = found;
+    }
+    __syncthreads();
+    last = carried;
+    for (int w = 0; w < wave; ++w) last = max(last, wave_start[w]);
+#pragma unroll
+    for (int u = 0; u < kItems; ++u) {
+        const int32_t base = k0 + u * kWave;
+        const uint64_t here = starts[u] & (~0ull >> (63 - lane));
+        const int32_t start = here != 0 ? base + 63 - __clzll(here) : last;
+        if (starts[u] != 0) last = base + 63 - __clzll(starts[u]);
+        if (a[u].by < 0 || ((base + lane - start) & 1) != 0) continue;
+        if (!RULES) {
+            if (load_now(m.uses + a[u].by) < 2) atomicAdd(m.uses + a[u].by, 1);
+        } else {
+            atomicOr(reinterpret_cast<unsigned long long *>(m.taken + a[u].at / 64), 1ull << (a[u].at % 64));
+            m.seq[a[u].at] = (uint32_t)a[u].by | (m.seq[a[u].at + 1] & kLast);  // the entry behind it is not taken
+        }
     }
 }
 
-__global__ void merger_emit_kernel(const int32_t *__restrict__ idx, const int32_t *__restrict__ kept,
-                                   const int32_t *__restrict__ lz, int64_t L, int32_t *__restrict__ emit) {
-    CGNN_GRID_LOOP(e, L) {
-        const bool second = e > 0 && merger_taken(idx, kept, lz, e - 1);  // swallowed by the rule at e-1
-        emit[e] = second ? 0 : 1;
+__global__ __launch_bounds__(kBlock) void merger_kept_kernel(Merger m) {
+    const int32_t c0 = (blockIdx.x * kBlock + threadIdx.x) * kItems;
+    int kept = 0, all;
+#pragma unroll
+    for (int u = 0; u < kItems; ++u) kept += c0 + u < m.candidates && m.uses[c0 + u] >= 2;
+    block_scan<kBlock>(kept, &all);
+    if (threadIdx.x == 0) m.tile[blockIdx.x] = all;
+}
+
+// Numbers of the new rules, and their children.
+__global__ __launch_bounds__(kBlock) void merger_rules_kernel(Merger m) {
+    const int32_t c0 = (blockIdx.x * kBlock + threadIdx.x) * kItems;
+    bool is[kItems];
+    int kept = 0, all;
+#pragma unroll
+    for (int u = 0; u < kItems; ++u) {
+        is[u] = c0 + u < m.candidates && m.uses[c0 + u] >= 2;
+        kept += is[u];
+    }
+    int64_t r = m.rules + m.tile[blockIdx.x] + block_scan<kBlock>(kept, &all);
+#pragma unroll
+    for (int u = 0; u < kItems; ++u) {
+        if (c0 + u >= m.candidates) break;
+        m.rule_of[c0 + u] = is[u] ? (int32_t)(m.V + r) : -1;
+        if (!is[u]) continue;
+        const uint64_t key = m.sorted_key[c0 + u];
+        m.children[2 * r] = (int32_t)(key >> m.key_bits);
+        m.children[2 * r + 1] = (int32_t)(key & (((uint64_t)1 << m.key_bits) - 1));
+        ++r;
     }
 }
 
-__global__ void merger_write_kernel(const int32_t *__restrict__ seq, const int32_t *__restrict__ idx,
-                                    const int32_t *__restrict__ kept, const int32_t *__restrict__ rank,
-                                    const int32_t *__restrict__ lz, const int32_t *__restrict__ emit,
-                                    const int32_t *__restrict__ opos, int64_t L, int32_t first_new_rule,
-                                    int32_t *__restrict__ out, int32_t *__restrict__ total) {
-    CGNN_GRID_LOOP(e, L) {
-        if (emit[e]) out[opos[e]] = merger_taken(idx, kept, lz, e) ? first_new_rule + rank[idx[e]] : seq[e];
-        if (e == L - 1) *total = opos[e] + emit[e];
+// Taken positions of the tile in front of every word of the map, and of every tile.
+__global__ __launch_bounds__(kBlock) void merger_taken_sums_kernel(Merger m, int64_t words) {
+    const int64_t w = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const int count = w < words ? __popcll(m.taken[w]) : 0, lane = threadIdx.x % kTileWords;
+    int sum = count;
+#pragma unroll
+    for (int s = 1; s < kTileWords; s <<= 1) {
+        const int up = __shfl_up(sum, s, kTileWords);
+        if (lane >= s) sum += up;
+    }
+    if (w >= words) return;
+    m.word_sum[w] = sum - count;
+    if (lane == kTileWords - 1) m.tile[w / kTileWords] = sum;
+}
+
+// Where position e goes: to the left by the taken ones in front of it.
+__device__ __forceinline__ int32_t moved(const Merger &m, int32_t e) {
+    const uint64_t below = m.taken[e / 64] & (((uint64_t)1 << (e % 64)) - 1);
+    return e - m.tile[e / kTile] - m.word_sum[e / 64] - __popcll(below);
+}
+
+// A wave per kItems words of the map: a word is the same for all lanes.
+__global__ __launch_bounds__(kBlock) void merger_move_kernel(Merger m) {
+    __shared__ int counts[kBlock / kWave];
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int64_t t0 = (int64_t)blockIdx.x * kTile;
+    int active = 0;
+#pragma unroll
+    for (int u = 0; u < kItems; ++u) {
+        const int64_t v = t0 + u * kBlock + threadIdx.x;
+        if (v <= m.V) {
+            const int32_t p = m.ptr[v];
+            m.next_ptr[v] = p < m.L ? moved(m, p) : m.L - m.scalar[kTakenTotal];
+        }
+    }
+    if (t0 < m.L) {
+        const int64_t w0 = blockIdx.x * kTileWords + wave * kItems;
+        const int32_t left = m.tile[blockIdx.x];
+        uint32_t entry[kItems];
+        uint64_t word[kItems], matched[kItems];
+        int32_t sum[kItems];
+#pragma unroll
+        for (int u = 0; u < kItems; ++u) {
+            const int64_t e = (w0 + u) * 64 + lane;
+            entry[u] = e < m.L ? m.seq[e] : 0;
+            word[u] = m.taken[w0 + u];
+            matched[u] = m.matched[w0 + u];
+            sum[u] = m.word_sum[w0 + u];
+        }
+        bool behind = w0 > 0 && m.taken[w0 - 1] >> 63;                       // the position in front is taken
+        const bool next = (w0 + kItems) * 64 < m.L && (m.taken[w0 + kItems] & 1);  // the first behind these words
+#pragma unroll
+        for (int u = 0; u < kItems; ++u) {
+            const int64_t e = (w0 + u) * 64 + lane;
+            const uint64_t gone = word[u] << 1 | (behind ? 1 : 0);
+            behind = word[u] >> 63;
+            if (e >= m.L || (gone >> lane & 1)) continue;
+            const uint64_t follows = word[u] >> 1 | (uint64_t)(u + 1 < kItems ? word[u + 1 < kItems ? u + 1 : u] & 1 : next) << 63;
+            const int32_t to = (int32_t)e - left - sum[u] - __popcll(word[u] & (((uint64_t)1 << lane) - 1));
+            // what can be a candidate next: a pair with a rule of this round in it, or a candidate of this round
+            const bool pair = !(entry[u] & kLast) && ((word[u] | follows | matched[u]) >> lane & 1);
+            m.next_seq[to] = entry[u];
+            m.next_active[to] = pair;
+            active += pair;
+        }
+    }
+#pragma unroll
+    for (int s = kWave / 2; s > 0; s >>= 1) active += __shfl_xor(active, s, kWave);
+    if (lane == 0) counts[wave] = active;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kBlock / kWave; ++w) active += counts[w];
+        if (active > 0) atomicAdd(m.scalar + kNextActive, active);
     }
 }
 
-__global__ void merger_new_ptr_kernel(const int32_t *__restrict__ ptr, int64_t V, int64_t L,
-                                      const int32_t *__restrict__ opos, const int32_t *__restrict__ total,
-                                      int32_t *__restrict__ next_ptr) {
-    CGNN_GRID_LOOP(v, V + 1) next_ptr[v] = ptr[v] < L ? opos[ptr[v]] : *total;
+// The scalars for the host, the flag last.
+__global__ void merger_publish_kernel(const int32_t *__restrict__ scalar, int32_t *__restrict__ host, int32_t flag) {
+    for (int i = 0; i < kScalars; ++i) host[i] = scalar[i];
+    __hip_atomic_store(host + kScalars, flag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // out_ptr = [row starts | starts of the rule rows], out_col = [rows | children of the rules].
-__global__ void merger_finish_kernel(const int32_t *__restrict__ ptr, const int32_t *__restrict__ seq,
+__global__ void merger_finish_kernel(const int32_t *__restrict__ ptr, const uint32_t *__restrict__ seq,
                                      const int32_t *__restrict__ children, int64_t V, int64_t R, int64_t L,
                                      int32_t *__restrict__ out_ptr, int32_t *__restrict__ out_col) {
     const int64_t n = L + 2 * R > V + R + 1 ? L + 2 * R : V + R + 1;
     CGNN_GRID_LOOP(i, n) {
         if (i <= V) out_ptr[i] = ptr[i];
         else if (i <= V + R) out_ptr[i] = (int32_t)(L + 2 * (i - V));
-        if (i < L) out_col[i] = seq[i];
+        if (i < L) out_col[i] = (int32_t)(seq[i] & ~kLast);
         else if (i < L + 2 * R) out_col[i] = children[i - L];
     }
 }
 
 struct MergerWorkspace {
-    size_t seq[3], ptr[2], last, keys[2], counts, flags, cand, idx, z, lz, emit, opos, uses, kept, rank, children,
-        scalars, temp, temp_bytes, total;
+    size_t seq[2], ptr[2], active[2], table_key, table_count, frequent, words, matched, taken, word_sum, tile, tile_start, position,
+        slot, candidate, cand_key, sorted_key, cand_slot, sorted_slot, cand_rank, uses, rule_of, children, scalars, temp,
+        temp_bytes, total;
 };
+
+int bits_of(int64_t n) {  // of the numbers up to n
+    int bits = 1;
+    while ((n >> bits) > 0) ++bits;
+    return bits;
+}
 
 MergerWorkspace merger_workspace(int64_t V, int64_t E) {
     MergerWorkspace w{};
@@ -198,40 +622,31 @@ MergerWorkspace merger_workspace(int64_t V, int64_t E) {
         at += align_up(bytes > 0 ? bytes : 1, 256);
         return here;
     };
-    const size_t n = (size_t)(E > 0 ? E : 1);
+    const size_t n = (size_t)(E > 0 ? E : 1), tiles = tiles_of(E > V ? E : V + 1), words = tiles * kTileWords, c = n / 3 + 1;
+    const size_t slots = (size_t)1 << bits_of((int64_t)n);
     for (auto &s : w.seq) s = take(n * 4);
     for (auto &p : w.ptr) p = take((size_t)(V + 1) * 4);
-    w.last = take(n * 4);
-    for (auto &k : w.keys) k = take(n * 8);  // keys[0]: keys, later the distinct keys; keys[1]: sorted keys
-    w.counts = take(n * 4);
-    w.flags = take(n);
-    w.cand = take(n * 8);
-    w.idx = take(n * 4);
-    w.z = take(n * 4);
-    w.lz = take(n * 4);
-    w.emit = take(n * 4);
-    w.opos = take(n * 4);
-    w.uses = take(n * 4);
-    w.kept = take(n * 4);
-    w.rank = take(n * 4);
+    for (auto &s : w.active) s = take(n);
+    w.table_key = take(slots * 8);  // also the counters by hash, twice as many
+    w.table_count = take(slots * 4);
+    w.frequent = take(slots / 4 + 8);
+    w.words = take(words * 8);
+    w.matched = take(words * 8);
+    w.taken = take(words * 8);
+    w.word_sum = take(words * 4);
+    w.tile = take(tiles * 4);
+    w.tile_start = take(tiles * 4);
+    w.position = take(n * 4);
+    w.slot = take(n * 4);
+    w.candidate = take(n * 4);
+    w.cand_key = take(c * 8);
+    w.sorted_key = take(c * 8);
+    for (auto *a : {&w.cand_slot, &w.sorted_slot, &w.cand_rank, &w.uses, &w.rule_of}) *a = take(c * 4);
     w.children = take(n * 4);
-    w.scalars = take(64);
-    size_t t = 0, best = 0;
-    const int m = (int)n;
-    hipcub::DeviceRadixSort::SortKeys(nullptr, t, (const uint64_t *)nullptr, (uint64_t *)nullptr, m, 0, 64, 0);
-    best = t > best ? t : best;
-    hipcub::DeviceRunLengthEncode::Encode(nullptr, t, (const uint64_t *)nullptr, (uint64_t *)nullptr,
-                                          (int32_t *)nullptr, (int32_t *)nullptr, m, 0);
-    best = t > best ? t : best;
-    hipcub::DeviceSelect::Flagged(nullptr, t, (const uint64_t *)nullptr, (const char *)nullptr, (uint64_t *)nullptr,
-                                  (int32_t *)nullptr, m, 0);
-    best = t > best ? t : best;
-    hipcub::DeviceScan::InclusiveScan(nullptr, t, (const int32_t *)nullptr, (int32_t *)nullptr, MaxOp(), m, 0);
-    best = t > best ? t : best;
-    hipcub::DeviceScan::ExclusiveSum(nullptr, t, (const int32_t *)nullptr, (int32_t *)nullptr, m, 0);
-    best = t > best ? t : best;
-    w.temp_bytes = best;
-    w.temp = take(best);
+    w.scalars = take(kScalars * 4);
+    hipcub::DeviceRadixSort::SortPairs(nullptr, w.temp_bytes, (const uint64_t *)nullptr, (uint64_t *)nullptr,
+                                       (const int32_t *)nullptr, (int32_t *)nullptr, (int)c, 0, 64, 0);
+    w.temp = take(w.temp_bytes);
     w.total = at;
     return w;
 }
@@ -239,6 +654,180 @@ MergerWorkspace merger_workspace(int64_t V, int64_t E) {
 int merger_fail(hipError_t e, const char *what) {
     set_error("cgnn_compress_csr_batch_device: %s: %s", what, hipGetErrorString(e));
     return CGNN_ELAUNCH;
+}
+
+Merger merger_of(int64_t V, int64_t E, int min_pair_frequency, const MergerWorkspace &w, void *workspace) {
+    char *base = static_cast<char *>(workspace);
+    auto i32 = [&](size_t off) { return reinterpret_cast<int32_t *>(base + off); };
+    auto u32 = [&](size_t off) { return reinterpret_cast<uint32_t *>(base + off); };
+    auto u64 = [&](size_t off) { return reinterpret_cast<uint64_t *>(base + off); };
+    auto u8 = [&](size_t off) { return reinterpret_cast<uint8_t *>(base + off); };
+    Merger m{};
+    m.V = V;
+    m.L = (int32_t)E;
+    m.min_frequency = min_pair_frequency;
+    m.first = true;
+    m.seq = u32(w.seq[0]), m.next_seq = u32(w.seq[1]);
+    m.ptr = i32(w.ptr[0]), m.next_ptr = i32(w.ptr[1]);
+    m.active = u8(w.active[0]), m.next_active = u8(w.active[1]);
+    m.table_key = u64(w.table_key), m.table_count = i32(w.table_count);
+    m.filter = u32(w.table_key), m.frequent = u32(w.frequent);
+    m.words = u64(w.words), m.matched = u64(w.matched), m.taken = u64(w.taken), m.word_sum = i32(w.word_sum);
+    m.tile = i32(w.tile), m.tile_start = i32(w.tile_start);
+    m.position = i32(w.position), m.slot = i32(w.slot), m.candidate = i32(w.candidate);
+    m.cand_key = u64(w.cand_key), m.sorted_key = u64(w.sorted_key);
+    m.cand_slot = i32(w.cand_slot), m.sorted_slot = i32(w.sorted_slot), m.cand_rank = i32(w.cand_rank);
+    m.uses = i32(w.uses), m.rule_of = i32(w.rule_of), m.children = i32(w.children), m.scalar = i32(w.scalars);
+    return m;
+}
+
+int merger_check(int64_t V, int64_t E, const void *vlist, const void *elist, int min_pair_frequency, const void *workspace,
+                 size_t workspace_bytes, MergerWorkspace *w) {
+    CGNN_REQUIRE(V >= 0 && E >= 0 && V < kMergerLimit && E < kMergerLimit,
+                 "cgnn_compress_csr_batch_device: V and E must be in [0, 2^31 - 65536)");
+    CGNN_REQUIRE(min_pair_frequency >= 3, "cgnn_compress_csr_batch_device: min_pair_frequency must be at least 3");
+    CGNN_REQUIRE(vlist && (E == 0 || elist), "cgnn_compress_csr_batch_device: null array");
+    *w = merger_workspace(V, E);
+    if (workspace == nullptr || workspace_bytes < w->total) {
+        set_error("cgnn_compress_csr_batch_device: workspace of %zu bytes needed, %zu given", w->total, workspace_bytes);
+        return CGNN_EWORKSPACE;
+    }
+    return CGNN_OK;
+}
+
+// Launches that depend on a count the host has not read cover the most it can be.
+void launch_begin(const Merger &m, int64_t most, hipStream_t stream) {
+    hipLaunchKernelGGL(merger_begin_kernel, dim3(merger_grid(((int64_t)2 << bits_of(most)) / 4)), dim3(kBlock), 0, stream, m);
+}
+
+template <typename In>
+int merger_rows(int64_t V, int64_t E, const In *vlist, int min_pair_frequency, void *workspace, size_t workspace_bytes,
+                hipStream_t stream) {
+    MergerWorkspace w;
+    const int rc = merger_check(V, E, vlist, vlist, min_pair_frequency, workspace, workspace_bytes, &w);
+    if (rc != CGNN_OK) return rc;
+    const Merger m = merger_of(V, E, min_pair_frequency, w, workspace);
+    launch_begin(m, E, stream);
+    hipLaunchKernelGGL(merger_rows_kernel<In>, dim3(merger_grid(V + 1)), dim3(kBlock), 0, stream, m, vlist, E);
+    return check_launch("compress_csr_batch_rows");
+}
+
+template <typename In>
+int merger_feed(int64_t V, int64_t E, const In *elist, int64_t from, int64_t n, int min_pair_frequency, void *workspace,
+                size_t workspace_bytes, hipStream_t stream) {
+    MergerWorkspace w;
+    const int rc = merger_check(V, E, elist, elist, min_pair_frequency, workspace, workspace_bytes, &w);
+    if (rc != CGNN_OK) return rc;
+    CGNN_REQUIRE(from >= 0 && n >= 0 && from + n <= E, "cgnn_compress_csr_batch_device: entries outside [0, E)");
+    if (n == 0) return CGNN_OK;
+    const Merger m = merger_of(V, E, min_pair_frequency, w, workspace);
+    hipLaunchKernelGGL(merger_feed_kernel<In>, dim3(tiles_of(n)), dim3(kBlock), 0, stream, m, elist, from, n);
+    return check_launch("compress_csr_batch_feed");
+}
+
+// The rounds, once all entries were fed.  `pinned`: kScalars + 1 integers of pinned host memory for what the host
+// reads, or NULL.
+int merger_rounds(int64_t V, int64_t E, int rounds, int min_pair_frequency, int32_t *out_ptr, int32_t *out_col,
+                  int64_t *host_summary, int32_t *pinned, void *workspace, size_t workspace_bytes, hipStream_t stream) {
+    CGNN_REQUIRE(rounds >= 1, "cgnn_compress_csr_batch_device: rounds must be positive");
+    CGNN_REQUIRE(host_summary, "cgnn_compress_csr_batch_device: null array");
+    MergerWorkspace w;
+    const int rc = merger_check(V, E, out_ptr, out_col, min_pair_frequency, workspace, workspace_bytes, &w);
+    if (rc != CGNN_OK) return rc;
+    Merger m = merger_of(V, E, min_pair_frequency, w, workspace);
+    const dim3 block(kBlock);
+    int32_t reads = 0, host[kScalars + 1];
+    if (pinned != nullptr) pinned[kScalars] = 0;
+    // What the host needs is written to memory that it looks at for a while, which costs it a few us; a copy and
+    // a wait cost it 40.
+    auto read = [&]() -> hipError_t {
+        if (pinned == nullptr) {
+            hipError_t e = hipMemcpyAsync(host, m.scalar, kScalars * sizeof(int32_t), hipMemcpyDeviceToHost, stream);
+            return e == hipSuccess ? hipStreamSynchronize(stream) : e;
+        }
+        hipLaunchKernelGGL(merger_publish_kernel, dim3(1), dim3(1), 0, stream, m.scalar, pinned, ++reads);
+        const auto patience = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
+        while (__atomic_load_n(pinned + kScalars, __ATOMIC_ACQUIRE) != reads)
+            if (std::chrono::steady_clock::now() > patience) {
+                const hipError_t e = hipStreamSynchronize(stream);
+                if (e != hipSuccess) return e;
+                if (__atomic_load_n(pinned + kScalars, __ATOMIC_ACQUIRE) != reads) return hipErrorUnknown;
+                break;
+            }
+        for (int i = 0; i < kScalars; ++i) host[i] = pinned[i];
+        return hipSuccess;
+    };
+    const int32_t all_tiles = (int32_t)tiles_of(E > V ? E : V + 1);
+    hipError_t err = hipSuccess;
+    bool checked = false;  // the input check is read with the first counts
+    int64_t R = 0, most = E;
+    for (int round = 0; round < rounds && m.L > 1 && most > 0; ++round) {
+        const int32_t tiles = (int32_t)tiles_of(m.L);
+        const dim3 grid((unsigned)tiles);
+        m.key_bits = bits_of(V + R);
+        m.rules = (int32_t)R;
+        if (round > 0) {
+            launch_begin(m, most, stream);
+            hipLaunchKernelGGL(merger_count_kernel, grid, block, 0, stream, m);
+        }
+        hipLaunchKernelGGL(merger_pass_kernel, grid, block, 0, stream, m);
+        hipLaunchKernelGGL(merger_tile_sums_kernel, dim3(1), dim3(kScanBlock), 0, stream, m.tile, tiles, m.scalar + kListed);
+        hipLaunchKernelGGL(merger_clear_table_kernel, dim3(merger_grid(((int64_t)1 << bits_of(most)) / 2)), block, 0, stream, m);
+        hipLaunchKernelGGL(merger_collect_kernel, grid, block, 0, stream, m);
+        hipLaunchKernelGGL(merger_candidates_kernel, dim3(tiles_of((int64_t)1 << bits_of(most))), block, 0, stream, m);
+        if ((err = read()) != hipSuccess) return merger_fail(err, "reading the candidate count");
+        if (!checked && host[kBad])
+            return fail(CGNN_EINVAL, "cgnn_compress_csr_batch_device: malformed CSR (row starts or columns out of range)");
+        checked = true;
+        m.listed = host[kListed], m.candidates = host[kCandidates];
+        if (m.candidates == 0) break;
+        if (m.candidates <= kRankAll) {
+            const unsigned side = (unsigned)ceil_div(m.candidates, kBlock);
+            hipLaunchKernelGGL(merger_rank_kernel, dim3(side, side), block, 0, stream, m);
+        } else {
+            size_t tb = w.temp_bytes;
+            err = hipcub::DeviceRadixSort::SortPairs(static_cast<char *>(workspace) + w.temp, tb, m.cand_key, m.sorted_key,
+                                                     m.cand_slot, m.sorted_slot, m.candidates, 0, 2 * m.key_bits, stream);
+            if (err != hipSuccess) return merger_fail(err, "sort");
+        }
+        const int64_t words = (int64_t)tiles * kTileWords;
+        const dim3 list(tiles_of(m.listed)), rules(tiles_of(m.candidates));
+        const int64_t places = m.candidates > words ? m.candidates : words;
+        hipLaunchKernelGGL(merger_place_kernel, dim3(merger_grid(places)), block, 0, stream, m);
+        hipLaunchKernelGGL(merger_match_kernel<false>, list, block, 0, stream, m);
+        hipLaunchKernelGGL(merger_take_kernel<false>, list, block, 0, stream, m);
+        hipLaunchKernelGGL(merger_kept_kernel, rules, block, 0, stream, m);
+        hipLaunchKernelGGL(merger_tile_sums_kernel, dim3(1), dim3(kScanBlock), 0, stream, m.tile, (int32_t)rules.x,
+                           m.scalar + kAdded);
+        hipLaunchKernelGGL(merger_rules_kernel, rules, block, 0, stream, m);
+        hipLaunchKernelGGL(merger_match_kernel<true>, list, block, 0, stream, m);
+        hipLaunchKernelGGL(merger_take_kernel<true>, list, block, 0, stream, m);
+        hipLaunchKernelGGL(merger_taken_sums_kernel, dim3(merger_grid(words)), block, 0, stream, m, words);
+        hipLaunchKernelGGL(merger_tile_sums_kernel, dim3(1), dim3(kScanBlock), 0, stream, m.tile, tiles, m.scalar + kTakenTotal);
+        hipLaunchKernelGGL(merger_move_kernel, dim3((unsigned)all_tiles), block, 0, stream, m);
+        if ((err = read()) != hipSuccess) return merger_fail(err, "reading the new length");
+        const int32_t added = host[kAdded];
+        if (added == 0) break;  // and nothing was taken
+        if (V + R + added >= kMergerLimit) return fail(CGNN_EUNSUPPORTED, "cgnn_compress_csr_batch_device: node ids exceed int32");
+        std::swap(m.seq, m.next_seq);
+        std::swap(m.ptr, m.next_ptr);
+        std::swap(m.active, m.next_active);
+        m.L -= host[kTakenTotal];
+        m.first = false;
+        most = host[kNextActive];
+        R += added;
+    }
+    if (!checked) {
+        if ((err = read()) != hipSuccess) return merger_fail(err, "reading the input check");
+        if (host[kBad])
+            return fail(CGNN_EINVAL, "cgnn_compress_csr_batch_device: malformed CSR (row starts or columns out of range)");
+    }
+    const int64_t L = m.L;
+    hipLaunchKernelGGL(merger_finish_kernel, dim3(merger_grid(L + 2 * R > V + R + 1 ? L + 2 * R : V + R + 1)), block, 0,
+                       stream, m.ptr, m.seq, m.children, V, R, L, out_ptr, out_col);
+    host_summary[0] = R;
+    host_summary[1] = L + 2 * R;
+    return check_launch("compress_csr_batch_device");
 }
 
 }  // namespace
@@ -255,110 +844,31 @@ extern "C" int cgnn_compress_csr_batch_device(int64_t V, int64_t E, const int64_
                                               int rounds, int min_pair_frequency, int32_t *out_ptr,
                                               int32_t *out_col, int64_t *host_summary, void *workspace,
                                               size_t workspace_bytes, cgnn_stream_t stream) {
-    CGNN_REQUIRE(V >= 0 && E >= 0 && V < kMergerLimit && E < kMergerLimit,
-                 "cgnn_compress_csr_batch_device: V and E must be in [0, 2^31 - 65536)");
-    CGNN_REQUIRE(rounds >= 1, "cgnn_compress_csr_batch_device: rounds must be positive");
-    CGNN_REQUIRE(min_pair_frequency >= 3, "cgnn_compress_csr_batch_device: min_pair_frequency must be at least 3");
-    CGNN_REQUIRE(vlist && out_ptr && host_summary && (E == 0 || (elist && out_col)),
-                 "cgnn_compress_csr_batch_device: null array");
-    const MergerWorkspace w = merger_workspace(V, E);
-    if (workspace == nullptr || workspace_bytes < w.total) {
-        set_error("cgnn_compress_csr_batch_device: workspace of %zu bytes needed, %zu given", w.total, workspace_bytes);
-        return CGNN_EWORKSPACE;
-    }
-    char *base = static_cast<char *>(workspace);
-    auto i32 = [&](size_t off) { return reinterpret_cast<int32_t *>(base + off); };
-    auto u64 = [&](size_t off) { return reinterpret_cast<uint64_t *>(base + off); };
-    int32_t *seq = i32(w.seq[0]), *next_seq = i32(w.seq[1]);
-    int32_t *ptr = i32(w.ptr[0]), *next_ptr = i32(w.ptr[1]);
-    int32_t *last = i32(w.last), *counts = i32(w.counts), *idx = i32(w.idx), *z = i32(w.z), *lz = i32(w.lz);
-    int32_t *emit = i32(w.emit), *opos = i32(w.opos), *uses = i32(w.uses), *kept = i32(w.kept), *rank = i32(w.rank);
-    int32_t *children = i32(w.children);
-    uint64_t *keys = u64(w.keys[0]), *sorted = u64(w.keys[1]), *cand = u64(w.cand);
-    char *flags = base + w.flags;
-    // device scalars: [0] bad input, [1] distinct keys, [2] candidates, [3] rules added, [4] new length
-    int32_t *scalars = i32(w.scalars);
-    void *temp = base + w.temp;
-    const dim3 block(kBlock);
-    auto read = [&](int k, int32_t *value) {
-        hipError_t e = hipMemcpyAsync(value, scalars + k, sizeof(int32_t), hipMemcpyDeviceToHost, stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(stream);
-        return e;
-    };
-    hipLaunchKernelGGL(merger_fill_kernel, dim3(1), block, 0, stream, scalars, 0, (int64_t)16);
-    hipLaunchKernelGGL(merger_init_kernel, dim3(merger_grid(V + 1 > E ? V + 1 : E)), block, 0, stream, vlist, elist, V,
-                       E, ptr, seq, scalars);
-    int32_t bad = 0;
-    hipError_t err = read(0, &bad);
-    if (err != hipSuccess) return merger_fail(err, "reading the input check");
-    if (bad) return fail(CGNN_EINVAL, "cgnn_compress_csr_batch_device: malformed CSR (row starts or columns out of range)");
-    int64_t L = E, R = 0;
-    for (int round = 0; round < rounds && L > 1; ++round) {
-        const int n = (int)L;
-        size_t tb = w.temp_bytes;
-        hipLaunchKernelGGL(merger_fill_kernel, dim3(merger_grid(L)), block, 0, stream, last, 0, L);
-        hipLaunchKernelGGL(merger_mark_last_kernel, dim3(merger_grid(V)), block, 0, stream, ptr, V, last);
-        hipLaunchKernelGGL(merger_keys_kernel, dim3(merger_grid(L)), block, 0, stream, seq, last, L, keys);
-        err = hipcub::DeviceRadixSort::SortKeys(temp, tb, keys, sorted, n, 0, 64, stream);
-        if (err != hipSuccess) return merger_fail(err, "sort");
-        uint64_t *unique = cand;  // the distinct keys; the candidates then go where the sorted keys were
-        tb = w.temp_bytes;
-        err = hipcub::DeviceRunLengthEncode::Encode(temp, tb, sorted, unique, counts, scalars + 1, n, stream);
-        if (err != hipSuccess) return merger_fail(err, "run-length encoding");
-        hipLaunchKernelGGL(merger_candidate_flags_kernel, dim3(merger_grid(L)), block, 0, stream, unique, counts,
-                           scalars + 1, L, (int32_t)min_pair_frequency, flags);
-        tb = w.temp_bytes;
-        err = hipcub::DeviceSelect::Flagged(temp, tb, unique, flags, sorted, scalars + 2, n, stream);
-        if (err != hipSuccess) return merger_fail(err, "selection");
-        int32_t ncand = 0;
-        if ((err = read(2, &ncand)) != hipSuccess) return merger_fail(err, "reading the candidate count");
-        if (ncand == 0) break;
-        const uint64_t *candidates = sorted;  // ascending
-        hipLaunchKernelGGL(merger_lookup_kernel, dim3(merger_grid(L)), block, 0, stream, keys, L, candidates, ncand,
-                           idx);
-        // pass 1: every candidate
-        hipLaunchKernelGGL(merger_unmatched_kernel, dim3(merger_grid(L)), block, 0, stream, idx,
-                           (const int32_t *)nullptr, L, z);
-        tb = w.temp_bytes;
-        err = hipcub::DeviceScan::InclusiveScan(temp, tb, z, lz, MaxOp(), n, stream);
-        if (err != hipSuccess) return merger_fail(err, "scan");
-        hipLaunchKernelGGL(merger_fill_kernel, dim3(merger_grid(ncand)), block, 0, stream, uses, 0, (int64_t)ncand);
-        hipLaunchKernelGGL(merger_count_uses_kernel, dim3(merger_grid(L)), block, 0, stream, idx, lz, L, uses);
-        hipLaunchKernelGGL(merger_kept_kernel, dim3(merger_grid(ncand)), block, 0, stream, uses, ncand, kept);
-        tb = w.temp_bytes;
-        err = hipcub::DeviceScan::ExclusiveSum(temp, tb, kept, rank, ncand, stream);
-        if (err != hipSuccess) return merger_fail(err, "scan");
-        hipLaunchKernelGGL(merger_rules_kernel, dim3(merger_grid(ncand)), block, 0, stream, candidates, kept, rank,
-                           ncand, R, children, scalars + 3);
-        int32_t added = 0;
-        if ((err = read(3, &added)) != hipSuccess) return merger_fail(err, "reading the rule count");
-        if (added == 0) break;
-        if (V + R + added >= kMergerLimit) return fail(CGNN_EUNSUPPORTED, "cgnn_compress_csr_batch_device: node ids exceed int32");
-        // pass 2: the rules only
-        hipLaunchKernelGGL(merger_unmatched_kernel, dim3(merger_grid(L)), block, 0, stream, idx, kept, L, z);
-        tb = w.temp_bytes;
-        err = hipcub::DeviceScan::InclusiveScan(temp, tb, z, lz, MaxOp(), n, stream);
-        if (err != hipSuccess) return merger_fail(err, "scan");
-        hipLaunchKernelGGL(merger_emit_kernel, dim3(merger_grid(L)), block, 0, stream, idx, kept, lz, L, emit);
-        tb = w.temp_bytes;
-        err = hipcub::DeviceScan::ExclusiveSum(temp, tb, emit, opos, n, stream);
-        if (err != hipSuccess) return merger_fail(err, "scan");
-        hipLaunchKernelGGL(merger_write_kernel, dim3(merger_grid(L)), block, 0, stream, seq, idx, kept, rank, lz, emit,
-                           opos, L, (int32_t)(V + R), next_seq, scalars + 4);
-        hipLaunchKernelGGL(merger_new_ptr_kernel, dim3(merger_grid(V + 1)), block, 0, stream, ptr, V, L, opos,
-                           scalars + 4, next_ptr);
-        int32_t total = 0;
-        if ((err = read(4, &total)) != hipSuccess) return merger_fail(err, "reading the new length");
-        std::swap(seq, next_seq);
-        std::swap(ptr, next_ptr);
-        L = total;
-        R += added;
-    }
-    hipLaunchKernelGGL(merger_finish_kernel, dim3(merger_grid(L + 2 * R > V + R + 1 ? L + 2 * R : V + R + 1)), block, 0,
-                       stream, ptr, seq, children, V, R, L, out_ptr, out_col);
-    err = hipStreamSynchronize(stream);
-    if (err != hipSuccess) return merger_fail(err, "finishing");
-    host_summary[0] = R;
-    host_summary[1] = L + 2 * R;
-    return check_launch("compress_csr_batch_device");
+    CGNN_REQUIRE(out_ptr && host_summary && (E == 0 || out_col), "cgnn_compress_csr_batch_device: null array");
+    int rc = merger_rows(V, E, vlist, min_pair_frequency, workspace, workspace_bytes, stream);
+    if (rc == CGNN_OK && E > 0) rc = merger_feed(V, E, elist, 0, E, min_pair_frequency, workspace, workspace_bytes, stream);
+    if (rc == CGNN_OK)
+        rc = merger_rounds(V, E, rounds, min_pair_frequency, out_ptr, out_col, host_summary, nullptr, workspace, workspace_bytes,
+                           stream);
+    if (rc != CGNN_OK) return rc;
+    const hipError_t err = hipStreamSynchronize(stream);
+    return err == hipSuccess ? CGNN_OK : merger_fail(err, "finishing");
+}
+
+extern "C" int cgnn_compress_batch_rows(int64_t V, int64_t E, const int32_t *vlist, int min_pair_frequency, void *workspace,
+                                        size_t workspace_bytes, cgnn_stream_t stream) {
+    return merger_rows(V, E, vlist, min_pair_frequency, workspace, workspace_bytes, stream);
+}
+
+extern "C" int cgnn_compress_batch_feed(int64_t V, int64_t E, const int32_t *elist, int64_t from, int64_t n,
+                                        int min_pair_frequency, void *workspace, size_t workspace_bytes,
+                                        cgnn_stream_t stream) {
+    return merger_feed(V, E, elist, from, n, min_pair_frequency, workspace, workspace_bytes, stream);
+}
+
+extern "C" int cgnn_compress_batch_rounds(int64_t V, int64_t E, int rounds, int min_pair_frequency, int32_t *out_ptr,
+                                          int32_t *out_col, int64_t *host_summary, int32_t *pinned, void *workspace,
+                                          size_t workspace_bytes, cgnn_stream_t stream) {
+    return merger_rounds(V, E, rounds, min_pair_frequency, out_ptr, out_col, host_summary, pinned, workspace, workspace_bytes,
+                         stream);
 }

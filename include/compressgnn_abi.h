@@ -232,12 +232,23 @@ int cgnn_csr_transpose_device(int64_t rows, int64_t cols, int64_t nnz, const int
  * (capacity V + E/2 + 2) holds the V + R + 1 row starts, out_col (capacity E) the vertex
  * rows written with vertex and rule ids, followed by the two children of every rule;
  * host_summary[0] = R, host_summary[1] = entries of out_col.  Offline work: the call waits
- * for the device (three small reads per round) and returns when the arrays are complete. */
+ * for the device (two small reads per round) and returns when the arrays are complete.
+ * The same from int32 arrays that arrive in parts: cgnn_compress_batch_rows takes the row starts, cgnn_compress_batch_feed
+ * entries [from, from + n) of elist (in order, all of them in the end), cgnn_compress_batch_rounds does the rest and does
+ * not wait for its last launch; pinned (9 integers of pinned host memory, or NULL) makes its reads cheaper.  All
+ * with the same V, E, min_pair_frequency and workspace, on one stream. */
 size_t cgnn_compress_batch_workspace_bytes(int64_t V, int64_t E);
 int cgnn_compress_csr_batch_device(int64_t V, int64_t E, const int64_t *vlist, const int64_t *elist,
                                    int rounds, int min_pair_frequency, int32_t *out_ptr,
                                    int32_t *out_col, int64_t *host_summary, void *workspace,
                                    size_t workspace_bytes, cgnn_stream_t stream);
+int cgnn_compress_batch_rows(int64_t V, int64_t E, const int32_t *vlist, int min_pair_frequency, void *workspace,
+                             size_t workspace_bytes, cgnn_stream_t stream);
+int cgnn_compress_batch_feed(int64_t V, int64_t E, const int32_t *elist, int64_t from, int64_t n, int min_pair_frequency,
+                             void *workspace, size_t workspace_bytes, cgnn_stream_t stream);
+int cgnn_compress_batch_rounds(int64_t V, int64_t E, int rounds, int min_pair_frequency, int32_t *out_ptr, int32_t *out_col,
+                               int64_t *host_summary, int32_t *pinned, void *workspace, size_t workspace_bytes,
+                               cgnn_stream_t stream);
 
 /* ------------------------------------------------- transformation compression -- */
 

@@ -124,3 +124,23 @@ def test_loader_gives_the_same_dataset_on_either_backend():
             assert p.dtype == q.dtype and np.array_equal(p.cpu().numpy(), q.cpu().numpy())
     assert np.array_equal(a.vertex_degree.numpy(), b.vertex_degree.numpy())
     assert np.array_equal(a.rule_degree.numpy(), b.rule_degree.numpy())
+
+
+@pytest.mark.parametrize("entries, freq", [(2047, 3), (2048, 3), (2049, 3), (4097, 64), (1 << 19, 5), ((1 << 19) + 1, 3)])
+def test_gpu_compressor_at_the_edges_of_its_tiles(entries, freq):
+    """Sequences around the tiles of the kernels and the chunks that cross to the device; one row as long as all others
+    together, of which most is one stretch; int32 and int64 input.  The largest has more candidates than are
+    ranked by comparing all with all."""
+    rng = np.random.default_rng(entries)
+    half, V = entries // 2, max(64, entries // 8)
+    long_row = rng.integers(0, 3, half)
+    long_row[half // 4:] = 5  # a stretch over several tiles
+    others = entries - half
+    pool = rng.integers(0, V, (max(1, others // 16), 4))
+    rest = pool[rng.integers(0, len(pool), others // 4 + 1)].ravel()[:others]
+    cuts = np.sort(rng.integers(0, others + 1, V - 2))
+    v = np.concatenate([[0, half], half + cuts, [entries]]).astype(np.int64)
+    e = np.concatenate([long_row, rest]).astype(np.int64)
+    got = both(v, e, 12, freq)
+    assert got[3] > 0
+    assert all(np.array_equal(a, b) for a, b in zip(got, both(v.astype(np.int32), e.astype(np.int32), 12, freq)))
