@@ -16,7 +16,7 @@
 //
 // What bounds a round is how often it goes over the sequence and at what price, so each step keeps fewer positions:
 //   - Only the pairs that can be candidates are looked at: in the first round all, later those with a rule of the round
-//     before in them and those that were candidates in it.  (Another pair was there before and was no candidate, and a
+//     before in them and those that could be candidates in it.  (Another pair was there before and was no candidate, and a
 //     round makes no pair of old entries more frequent.)
 //   - These are counted in a table by their hash alone, an upper bound of how often they occur; the counters stop at
 //     min_pair_frequency, so that a pair met a thousand times costs its counter no thousand atomics one after the other.
@@ -26,7 +26,7 @@
 //     and the row starts.
 // Sorting all pairs in every round (eight passes over 64-bit keys, run-length encoding, selection, a binary search per
 // position, scans over all positions) took 1,950 us of the device for the three rounds of 325,557 rows and 3.2 million
-// entries; this takes 700 us, 220 of them while the sequence still arrives (cgnn_compress_batch_feed).
+// entries; this takes 620 us, 210 of them while the sequence still arrives (cgnn_compress_batch_feed).
 //
 // Timing decides where an atomic lands, never what comes of it: counts and sums are whole numbers, lists are in
 // order of position or sorted, so the arrays are the same run to run and equal the host routine's.
@@ -53,11 +53,12 @@ constexpr int kScanBlock = 1024;
 // alone take 40 us, and at 16,384 the comparisons do, too.
 constexpr int32_t kRankAll = 16384;
 
-enum Scalar { kBad, kActive, kListed, kCandidates, kAdded, kTakenTotal, kNextActive, kScalars = 8 };
+enum Scalar { kBad, kListed, kCandidates, kAdded, kTakenTotal, kScalars = 8 };
 
 struct Merger {
     int64_t V;
     int32_t L, min_frequency, rules;   // rules: numbered before this round
+    int32_t most;                      // pairs that can be candidates
     int32_t listed, candidates;        // once the host has read them
     int key_bits;                      // of one entry
     bool first;
@@ -74,8 +75,9 @@ struct Merger {
     int32_t *table_count;              // later the rank of the slot's candidate, -1: none
     uint64_t *cand_key, *sorted_key;   // [candidates] (first entry << key_bits) | second
     int32_t *cand_slot, *sorted_slot, *cand_rank;
-    int32_t *uses, *rule_of;           // [candidates] in order
-    uint64_t *matched, *taken;         // [L / 64]
+    int32_t *use, *rule_of;            // [candidates] in order
+    uint64_t *used;                    // [listed / 64] taken when all candidates were
+    uint64_t *taken;                   // [L / 64] taken by a rule
     int32_t *word_sum;                 // [L / 64] taken positions of the tile in front of a word
     int32_t *children;
     int32_t *scalar;                   // [kScalars]
@@ -145,13 +147,11 @@ __global__ void merger_rows_kernel(Merger m, const In *__restrict__ vlist, int64
 
 // Where the round begins: the counters, and scalars of this round.
 __global__ void merger_begin_kernel(Merger m) {
-    const int32_t n = m.first ? m.L : m.scalar[kNextActive];
-    const int64_t counters = (int64_t)2 << table_bits(n), words = ((int64_t)m.L + kTile - 1) / kTile * kTileWords;
+    const int64_t counters = (int64_t)2 << table_bits(m.most), words = ((int64_t)m.L + kTile - 1) / kTile * kTileWords;
     CGNN_GRID_LOOP(i, counters / 4) reinterpret_cast<int4 *>(m.filter)[i] = make_int4(0, 0, 0, 0);
     CGNN_GRID_LOOP(i, ceil_div_dev(counters, 32)) m.frequent[i] = 0;
     if (m.first) CGNN_GRID_LOOP(i, words) m.taken[i] = 0;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        m.scalar[kActive] = n;
         m.scalar[kCandidates] = 0;
         if (m.first) m.scalar[kBad] = 0;
     }
@@ -166,7 +166,7 @@ __device__ __forceinline__ void count_pair(const Merger &m, uint64_t counter, ui
 // Entries [from, from + n) of the first round's sequence, and the pairs that end there.
 template <typename In>
 __global__ __launch_bounds__(kBlock) void merger_feed_kernel(Merger m, const In *__restrict__ elist, int64_t from, int64_t n) {
-    const int shift = 63 - table_bits(m.L);
+    const int shift = 63 - table_bits(m.most);
     const int64_t i0 = from + (int64_t)blockIdx.x * kTile + threadIdx.x, end = from + n;
     uint64_t counter[kItems];
     uint32_t seen[kItems];
@@ -202,7 +202,7 @@ __device__ __forceinline__ uint64_t pair_at(const Merger &m, int64_t e) {
 }
 
 __global__ __launch_bounds__(kBlock) void merger_count_kernel(Merger m) {
-    const int shift = 63 - table_bits(m.scalar[kActive]);
+    const int shift = 63 - table_bits(m.most);
     const int64_t e0 = (int64_t)blockIdx.x * kTile + threadIdx.x;
     uint64_t key[kItems];
     uint64_t counter[kItems];
@@ -222,7 +222,7 @@ __global__ __launch_bounds__(kBlock) void merger_count_kernel(Merger m) {
 
 __global__ __launch_bounds__(kBlock) void merger_pass_kernel(Merger m) {
     __shared__ int passed[kBlock / kWave];
-    const int shift = 63 - table_bits(m.scalar[kActive]);
+    const int shift = 63 - table_bits(m.most);
     const int64_t e0 = (int64_t)blockIdx.x * kTile + threadIdx.x;
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     uint64_t key[kItems];
@@ -364,89 +364,92 @@ __global__ __launch_bounds__(kBlock) void merger_rank_kernel(Merger m) {
     if (smaller > 0) atomicAdd(m.cand_rank + i, smaller);
 }
 
-// The candidates take their places; their uses, the maps of the parses and the count of the next round start at nothing.
+// The candidates take their places; none is used twice yet, and nothing is taken.
 __global__ void merger_place_kernel(Merger m) {
     const bool ranked = m.candidates <= kRankAll;
     const int64_t words = ((int64_t)m.L + kTile - 1) / kTile * kTileWords, n = m.candidates > words ? m.candidates : words;
-    if (blockIdx.x == 0 && threadIdx.x == 0) m.scalar[kNextActive] = 0;
     CGNN_GRID_LOOP(i, n) {
-        if (i < words) m.matched[i] = m.taken[i] = 0;
+        if (i < words) m.taken[i] = 0;
         if (i < m.candidates) {
             const int32_t r = ranked ? m.cand_rank[i] : (int32_t)i;
             if (ranked) m.sorted_key[r] = m.cand_key[i];
             m.table_count[ranked ? m.cand_slot[i] : m.sorted_slot[i]] = r;
-            m.uses[i] = 0;
+            m.rule_of[i] = 0;
         }
     }
 }
 
-// A parse takes the list a tile per workgroup and 64 positions per wave and step.  First half: which positions are
-// matched (RULES: by the rules only), and the last start of a stretch in every tile.
-struct Match {
-    int32_t by, at;  // candidate or rule, -1: none; position
-    bool starts;
-};
-
-template <bool RULES, bool FIND>
-__device__ __forceinline__ Match match_at(const Merger &m, int32_t k) {
-    auto matched_by = [&](int32_t i) {
-        const int32_t c = FIND ? m.table_count[m.slot[i]] : m.candidate[i];
-        return RULES && c >= 0 ? m.rule_of[c] : c;
-    };
-    Match a{-1, -1, false};
-    if (k >= m.listed) return a;
-    a.by = matched_by(k);
-    a.at = m.position[k];
-    if (a.by >= 0) a.starts = k == 0 || m.position[k - 1] != a.at - 1 || matched_by(k - 1) < 0;
-    return a;
-}
-
+// A parse takes the list a tile per workgroup and 64 positions per wave and step.
 __device__ __forceinline__ int32_t wave_begin() {
     return blockIdx.x * kTile + threadIdx.x / kWave * (kItems * kWave);
 }
 
+struct Matches {
+    int32_t by[kItems], at[kItems];  // candidate or rule (-1: none), position
+    uint64_t starts[kItems];         // of a stretch
+    int32_t last;                    // the last one of the wave, -1: none
+};
+
+// Which positions are matched (RULES: by the rules only; FIND: the candidates are still in the table).
+template <bool RULES, bool FIND>
+__device__ __forceinline__ Matches matches(const Merger &m, int32_t k0, int lane) {
+    auto matched_by = [&](int32_t k) {
+        const int32_t c = FIND ? m.table_count[m.slot[k]] : m.candidate[k];
+        return RULES && c >= 0 ? m.rule_of[c] : c;
+    };
+    Matches a;
+#pragma unroll
+    for (int u = 0; u < kItems; ++u) {
+        const int32_t k = k0 + u * kWave + lane;
+        a.by[u] = k < m.listed ? matched_by(k) : -1;
+        a.at[u] = k < m.listed ? m.position[k] : -1;
+    }
+    // a stretch goes on where the position in front is matched, too
+    int32_t before = k0 > 0 && k0 < m.listed && matched_by(k0 - 1) >= 0 ? m.position[k0 - 1] : -2;
+    a.last = -1;
+#pragma unroll
+    for (int u = 0; u < kItems; ++u) {
+        const int32_t mine = a.by[u] >= 0 ? a.at[u] : -2;
+        const int32_t up = __shfl_up(mine, 1, kWave);
+        a.starts[u] = __ballot(a.by[u] >= 0 && (lane == 0 ? before : up) != mine - 1);
+        before = __shfl(mine, kWave - 1, kWave);
+        if (a.starts[u] != 0) a.last = k0 + u * kWave + 63 - __clzll(a.starts[u]);
+    }
+    return a;
+}
+
+// First half of a parse: the last start of a stretch in every tile.
 template <bool RULES>
 __global__ __launch_bounds__(kBlock) void merger_match_kernel(Merger m) {
     __shared__ int32_t wave_start[kBlock / kWave];
     const int lane = threadIdx.x % kWave;
     const int32_t k0 = wave_begin();
-    int32_t last = -1;
+    const Matches a = matches<RULES, !RULES>(m, k0, lane);
+    if (!RULES)
 #pragma unroll
-    for (int u = 0; u < kItems; ++u) {
-        const int32_t k = k0 + u * kWave + lane;
-        const Match a = match_at<RULES, !RULES>(m, k);
-        const uint64_t starts = __ballot(a.starts);
-        if (starts != 0) last = k0 + u * kWave + 63 - __clzll(starts);
-        if (!RULES && k < m.listed) {
-            m.candidate[k] = a.by;
-            if (a.by >= 0) atomicOr(reinterpret_cast<unsigned long long *>(m.matched + a.at / 64), 1ull << (a.at % 64));
+        for (int u = 0; u < kItems; ++u) {
+            const int32_t k = k0 + u * kWave + lane;
+            if (k < m.listed) m.candidate[k] = a.by[u];
         }
-    }
-    if (lane == 0) wave_start[threadIdx.x / kWave] = last;
+    if (lane == 0) wave_start[threadIdx.x / kWave] = a.last;
     __syncthreads();
     if (threadIdx.x == 0) {
+        int32_t last = -1;
         for (int w = 0; w < kBlock / kWave; ++w) last = max(last, wave_start[w]);
         m.tile_start[blockIdx.x] = last;
     }
 }
 
-// Second half: every other position of a stretch is taken.  Without RULES it counts as a use, of which only
-// the first two matter; with RULES the rule takes its place in the sequence.
+// Second half: every other position of a stretch is taken.  Without RULES it leaves its name as a use of the candidate
+// (any of them may stay; merger_again_kernel finds out whether there are two); with RULES the rule takes its
+// place in the sequence.
 template <bool RULES>
 __global__ __launch_bounds__(kBlock) void merger_take_kernel(Merger m) {
     __shared__ int32_t wave_start[kBlock / kWave], carried;
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     const int32_t k0 = wave_begin();
-    Match a[kItems];
-    uint64_t starts[kItems];
-    int32_t last = -1;
-#pragma unroll
-    for (int u = 0; u < kItems; ++u) {
-        a[u] = match_at<RULES, false>(m, k0 + u * kWave + lane);
-        starts[u] = __ballot(a[u].starts);
-        if (starts[u] != 0) last = k0 + u * kWave + 63 - __clzll(starts[u]);
-    }
-    if (lane == 0) wave_start[wave] = last;
+    const Matches a = matches<RULES, false>(m, k0, lane);
+    if (lane == 0) wave_start[wave] = a.last;
     if (wave == 0) {  // the last start in front of the tile
         int32_t found = -1;
         for (int32_t b = (int32_t)blockIdx.x; b > 0 && found < 0; b -= kWave) {
@@ -457,21 +460,36 @@ __global__ __launch_bounds__(kBlock) void merger_take_kernel(Merger m) {
         if (lane == 0) carried = found;
     }
     __syncthreads();
-    last = carried;
+    int32_t last = carried;
     for (int w = 0; w < wave; ++w) last = max(last, wave_start[w]);
 #pragma unroll
     for (int u = 0; u < kItems; ++u) {
         const int32_t base = k0 + u * kWave;
-        const uint64_t here = starts[u] & (~0ull >> (63 - lane));
+        const uint64_t here = a.starts[u] & (~0ull >> (63 - lane));
         const int32_t start = here != 0 ? base + 63 - __clzll(here) : last;
-        if (starts[u] != 0) last = base + 63 - __clzll(starts[u]);
-        if (a[u].by < 0 || ((base + lane - start) & 1) != 0) continue;
+        if (a.starts[u] != 0) last = base + 63 - __clzll(a.starts[u]);
+        const bool taken = a.by[u] >= 0 && ((base + lane - start) & 1) == 0;
         if (!RULES) {
-            if (load_now(m.uses + a[u].by) < 2) atomicAdd(m.uses + a[u].by, 1);
-        } else {
-            atomicOr(reinterpret_cast<unsigned long long *>(m.taken + a[u].at / 64), 1ull << (a[u].at % 64));
-            m.seq[a[u].at] = (uint32_t)a[u].by | (m.seq[a[u].at + 1] & kLast);  // the entry behind it is not taken
+            const uint64_t word = __ballot(taken);
+            if (lane == 0 && base < m.listed) m.used[base / 64] = word;
+            if (taken) m.use[a.by[u]] = base + lane;
+        } else if (taken) {
+            atomicOr(reinterpret_cast<unsigned long long *>(m.taken + a.at[u] / 64), 1ull << (a.at[u] % 64));
+            m.seq[a.at[u]] = (uint32_t)a.by[u] | (m.seq[a.at[u] + 1] & kLast);  // the entry behind it is not taken
         }
+    }
+}
+
+// A position whose candidate has the name of another use: the candidate becomes a rule.  Counting the uses with
+// atomics took 42 us for the 305,000 of a web graph, because a few candidates have most of them; the names and this take 12.
+__global__ __launch_bounds__(kBlock) void merger_again_kernel(Merger m) {
+    const int32_t k0 = wave_begin() + threadIdx.x % kWave;
+#pragma unroll
+    for (int u = 0; u < kItems; ++u) {
+        const int32_t k = k0 + u * kWave;
+        if (k >= m.listed || !(m.used[k / 64] >> (k % 64) & 1)) continue;
+        const int32_t c = m.candidate[k];
+        if (m.use[c] != k) m.rule_of[c] = 1;
     }
 }
 
@@ -479,32 +497,34 @@ __global__ __launch_bounds__(kBlock) void merger_kept_kernel(Merger m) {
     const int32_t c0 = (blockIdx.x * kBlock + threadIdx.x) * kItems;
     int kept = 0, all;
 #pragma unroll
-    for (int u = 0; u < kItems; ++u) kept += c0 + u < m.candidates && m.uses[c0 + u] >= 2;
+    for (int u = 0; u < kItems; ++u) kept += c0 + u < m.candidates ? m.rule_of[c0 + u] : 0;
     block_scan<kBlock>(kept, &all);
     if (threadIdx.x == 0) m.tile[blockIdx.x] = all;
 }
 
-// Numbers of the new rules, and their children.
-__global__ __launch_bounds__(kBlock) void merger_rules_kernel(Merger m) {
-    const int32_t c0 = (blockIdx.x * kBlock + threadIdx.x) * kItems;
-    bool is[kItems];
-    int kept = 0, all;
+// Numbers of the new rules, and their children: kItems candidates a thread.  ALONE: one workgroup has them all; otherwise
+// `tile` holds the sums of the workgroups in front.
+template <int BLOCK, bool ALONE>
+__global__ __launch_bounds__(BLOCK) void merger_rules_kernel(Merger m) {
+    const int32_t c0 = (blockIdx.x * BLOCK + threadIdx.x) * kItems;
+    int kept[kItems], sum = 0, all;
 #pragma unroll
     for (int u = 0; u < kItems; ++u) {
-        is[u] = c0 + u < m.candidates && m.uses[c0 + u] >= 2;
-        kept += is[u];
+        kept[u] = c0 + u < m.candidates ? m.rule_of[c0 + u] : 0;
+        sum += kept[u];
     }
-    int64_t r = m.rules + m.tile[blockIdx.x] + block_scan<kBlock>(kept, &all);
+    int64_t r = m.rules + (ALONE ? 0 : m.tile[blockIdx.x]) + block_scan<BLOCK>(sum, &all);
 #pragma unroll
     for (int u = 0; u < kItems; ++u) {
         if (c0 + u >= m.candidates) break;
-        m.rule_of[c0 + u] = is[u] ? (int32_t)(m.V + r) : -1;
-        if (!is[u]) continue;
+        m.rule_of[c0 + u] = kept[u] ? (int32_t)(m.V + r) : -1;
+        if (!kept[u]) continue;
         const uint64_t key = m.sorted_key[c0 + u];
         m.children[2 * r] = (int32_t)(key >> m.key_bits);
         m.children[2 * r + 1] = (int32_t)(key & (((uint64_t)1 << m.key_bits) - 1));
         ++r;
     }
+    if (ALONE && threadIdx.x == 0) m.scalar[kAdded] = all;
 }
 
 // Taken positions of the tile in front of every word of the map, and of every tile.
@@ -530,10 +550,8 @@ __device__ __forceinline__ int32_t moved(const Merger &m, int32_t e) {
 
 // A wave per kItems words of the map: a word is the same for all lanes.
 __global__ __launch_bounds__(kBlock) void merger_move_kernel(Merger m) {
-    __shared__ int counts[kBlock / kWave];
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     const int64_t t0 = (int64_t)blockIdx.x * kTile;
-    int active = 0;
 #pragma unroll
     for (int u = 0; u < kItems; ++u) {
         const int64_t v = t0 + u * kBlock + threadIdx.x;
@@ -546,14 +564,14 @@ __global__ __launch_bounds__(kBlock) void merger_move_kernel(Merger m) {
         const int64_t w0 = blockIdx.x * kTileWords + wave * kItems;
         const int32_t left = m.tile[blockIdx.x];
         uint32_t entry[kItems];
-        uint64_t word[kItems], matched[kItems];
+        uint64_t word[kItems], passed[kItems];
         int32_t sum[kItems];
 #pragma unroll
         for (int u = 0; u < kItems; ++u) {
             const int64_t e = (w0 + u) * 64 + lane;
             entry[u] = e < m.L ? m.seq[e] : 0;
             word[u] = m.taken[w0 + u];
-            matched[u] = m.matched[w0 + u];
+            passed[u] = m.words[w0 + u];
             sum[u] = m.word_sum[w0 + u];
         }
         bool behind = w0 > 0 && m.taken[w0 - 1] >> 63;                       // the position in front is taken
@@ -566,20 +584,10 @@ __global__ __launch_bounds__(kBlock) void merger_move_kernel(Merger m) {
             if (e >= m.L || (gone >> lane & 1)) continue;
             const uint64_t follows = word[u] >> 1 | (uint64_t)(u + 1 < kItems ? word[u + 1 < kItems ? u + 1 : u] & 1 : next) << 63;
             const int32_t to = (int32_t)e - left - sum[u] - __popcll(word[u] & (((uint64_t)1 << lane) - 1));
-            // what can be a candidate next: a pair with a rule of this round in it, or a candidate of this round
-            const bool pair = !(entry[u] & kLast) && ((word[u] | follows | matched[u]) >> lane & 1);
+            // what can be a candidate next: a pair with a rule of this round in it, or one that passed the filter
             m.next_seq[to] = entry[u];
-            m.next_active[to] = pair;
-            active += pair;
+            m.next_active[to] = !(entry[u] & kLast) && ((word[u] | follows | passed[u]) >> lane & 1);
         }
-    }
-#pragma unroll
-    for (int s = kWave / 2; s > 0; s >>= 1) active += __shfl_xor(active, s, kWave);
-    if (lane == 0) counts[wave] = active;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < kBlock / kWave; ++w) active += counts[w];
-        if (active > 0) atomicAdd(m.scalar + kNextActive, active);
     }
 }
 
@@ -603,8 +611,8 @@ __global__ void merger_finish_kernel(const int32_t *__restrict__ ptr, const uint
 }
 
 struct MergerWorkspace {
-    size_t seq[2], ptr[2], active[2], table_key, table_count, frequent, words, matched, taken, word_sum, tile, tile_start, position,
-        slot, candidate, cand_key, sorted_key, cand_slot, sorted_slot, cand_rank, uses, rule_of, children, scalars, temp,
+    size_t seq[2], ptr[2], active[2], table_key, table_count, frequent, words, used, taken, word_sum, tile, tile_start, position,
+        slot, candidate, cand_key, sorted_key, cand_slot, sorted_slot, cand_rank, use, rule_of, children, scalars, temp,
         temp_bytes, total;
 };
 
@@ -631,7 +639,7 @@ MergerWorkspace merger_workspace(int64_t V, int64_t E) {
     w.table_count = take(slots * 4);
     w.frequent = take(slots / 4 + 8);
     w.words = take(words * 8);
-    w.matched = take(words * 8);
+    w.used = take(words * 8);
     w.taken = take(words * 8);
     w.word_sum = take(words * 4);
     w.tile = take(tiles * 4);
@@ -641,7 +649,7 @@ MergerWorkspace merger_workspace(int64_t V, int64_t E) {
     w.candidate = take(n * 4);
     w.cand_key = take(c * 8);
     w.sorted_key = take(c * 8);
-    for (auto *a : {&w.cand_slot, &w.sorted_slot, &w.cand_rank, &w.uses, &w.rule_of}) *a = take(c * 4);
+    for (auto *a : {&w.cand_slot, &w.sorted_slot, &w.cand_rank, &w.use, &w.rule_of}) *a = take(c * 4);
     w.children = take(n * 4);
     w.scalars = take(kScalars * 4);
     hipcub::DeviceRadixSort::SortPairs(nullptr, w.temp_bytes, (const uint64_t *)nullptr, (uint64_t *)nullptr,
@@ -667,17 +675,18 @@ Merger merger_of(int64_t V, int64_t E, int min_pair_frequency, const MergerWorks
     m.L = (int32_t)E;
     m.min_frequency = min_pair_frequency;
     m.first = true;
+    m.most = (int32_t)E;
     m.seq = u32(w.seq[0]), m.next_seq = u32(w.seq[1]);
     m.ptr = i32(w.ptr[0]), m.next_ptr = i32(w.ptr[1]);
     m.active = u8(w.active[0]), m.next_active = u8(w.active[1]);
     m.table_key = u64(w.table_key), m.table_count = i32(w.table_count);
     m.filter = u32(w.table_key), m.frequent = u32(w.frequent);
-    m.words = u64(w.words), m.matched = u64(w.matched), m.taken = u64(w.taken), m.word_sum = i32(w.word_sum);
+    m.words = u64(w.words), m.used = u64(w.used), m.taken = u64(w.taken), m.word_sum = i32(w.word_sum);
     m.tile = i32(w.tile), m.tile_start = i32(w.tile_start);
     m.position = i32(w.position), m.slot = i32(w.slot), m.candidate = i32(w.candidate);
     m.cand_key = u64(w.cand_key), m.sorted_key = u64(w.sorted_key);
     m.cand_slot = i32(w.cand_slot), m.sorted_slot = i32(w.sorted_slot), m.cand_rank = i32(w.cand_rank);
-    m.uses = i32(w.uses), m.rule_of = i32(w.rule_of), m.children = i32(w.children), m.scalar = i32(w.scalars);
+    m.use = i32(w.use), m.rule_of = i32(w.rule_of), m.children = i32(w.children), m.scalar = i32(w.scalars);
     return m;
 }
 
@@ -696,8 +705,8 @@ int merger_check(int64_t V, int64_t E, const void *vlist, const void *elist, int
 }
 
 // Launches that depend on a count the host has not read cover the most it can be.
-void launch_begin(const Merger &m, int64_t most, hipStream_t stream) {
-    hipLaunchKernelGGL(merger_begin_kernel, dim3(merger_grid(((int64_t)2 << bits_of(most)) / 4)), dim3(kBlock), 0, stream, m);
+void launch_begin(const Merger &m, hipStream_t stream) {
+    hipLaunchKernelGGL(merger_begin_kernel, dim3(merger_grid(((int64_t)2 << bits_of(m.most)) / 4)), dim3(kBlock), 0, stream, m);
 }
 
 template <typename In>
@@ -707,7 +716,7 @@ int merger_rows(int64_t V, int64_t E, const In *vlist, int min_pair_frequency, v
     const int rc = merger_check(V, E, vlist, vlist, min_pair_frequency, workspace, workspace_bytes, &w);
     if (rc != CGNN_OK) return rc;
     const Merger m = merger_of(V, E, min_pair_frequency, w, workspace);
-    launch_begin(m, E, stream);
+    launch_begin(m, stream);
     hipLaunchKernelGGL(merger_rows_kernel<In>, dim3(merger_grid(V + 1)), dim3(kBlock), 0, stream, m, vlist, E);
     return check_launch("compress_csr_batch_rows");
 }
@@ -760,21 +769,21 @@ int merger_rounds(int64_t V, int64_t E, int rounds, int min_pair_frequency, int3
     const int32_t all_tiles = (int32_t)tiles_of(E > V ? E : V + 1);
     hipError_t err = hipSuccess;
     bool checked = false;  // the input check is read with the first counts
-    int64_t R = 0, most = E;
-    for (int round = 0; round < rounds && m.L > 1 && most > 0; ++round) {
+    int64_t R = 0;
+    for (int round = 0; round < rounds && m.L > 1; ++round) {
         const int32_t tiles = (int32_t)tiles_of(m.L);
         const dim3 grid((unsigned)tiles);
         m.key_bits = bits_of(V + R);
         m.rules = (int32_t)R;
         if (round > 0) {
-            launch_begin(m, most, stream);
+            launch_begin(m, stream);
             hipLaunchKernelGGL(merger_count_kernel, grid, block, 0, stream, m);
         }
         hipLaunchKernelGGL(merger_pass_kernel, grid, block, 0, stream, m);
         hipLaunchKernelGGL(merger_tile_sums_kernel, dim3(1), dim3(kScanBlock), 0, stream, m.tile, tiles, m.scalar + kListed);
-        hipLaunchKernelGGL(merger_clear_table_kernel, dim3(merger_grid(((int64_t)1 << bits_of(most)) / 2)), block, 0, stream, m);
+        hipLaunchKernelGGL(merger_clear_table_kernel, dim3(merger_grid(((int64_t)1 << bits_of(m.most)) / 2)), block, 0, stream, m);
         hipLaunchKernelGGL(merger_collect_kernel, grid, block, 0, stream, m);
-        hipLaunchKernelGGL(merger_candidates_kernel, dim3(tiles_of((int64_t)1 << bits_of(most))), block, 0, stream, m);
+        hipLaunchKernelGGL(merger_candidates_kernel, dim3(tiles_of((int64_t)1 << bits_of(m.most))), block, 0, stream, m);
         if ((err = read()) != hipSuccess) return merger_fail(err, "reading the candidate count");
         if (!checked && host[kBad])
             return fail(CGNN_EINVAL, "cgnn_compress_csr_batch_device: malformed CSR (row starts or columns out of range)");
@@ -796,10 +805,15 @@ int merger_rounds(int64_t V, int64_t E, int rounds, int min_pair_frequency, int3
         hipLaunchKernelGGL(merger_place_kernel, dim3(merger_grid(places)), block, 0, stream, m);
         hipLaunchKernelGGL(merger_match_kernel<false>, list, block, 0, stream, m);
         hipLaunchKernelGGL(merger_take_kernel<false>, list, block, 0, stream, m);
-        hipLaunchKernelGGL(merger_kept_kernel, rules, block, 0, stream, m);
-        hipLaunchKernelGGL(merger_tile_sums_kernel, dim3(1), dim3(kScanBlock), 0, stream, m.tile, (int32_t)rules.x,
-                           m.scalar + kAdded);
-        hipLaunchKernelGGL(merger_rules_kernel, rules, block, 0, stream, m);
+        hipLaunchKernelGGL(merger_again_kernel, list, block, 0, stream, m);
+        if (m.candidates <= kScanBlock * kItems) {  // a step of one workgroup costs less than three launches
+            hipLaunchKernelGGL((merger_rules_kernel<kScanBlock, true>), dim3(1), dim3(kScanBlock), 0, stream, m);
+        } else {
+            hipLaunchKernelGGL(merger_kept_kernel, rules, block, 0, stream, m);
+            hipLaunchKernelGGL(merger_tile_sums_kernel, dim3(1), dim3(kScanBlock), 0, stream, m.tile, (int32_t)rules.x,
+                               m.scalar + kAdded);
+            hipLaunchKernelGGL((merger_rules_kernel<kBlock, false>), rules, block, 0, stream, m);
+        }
         hipLaunchKernelGGL(merger_match_kernel<true>, list, block, 0, stream, m);
         hipLaunchKernelGGL(merger_take_kernel<true>, list, block, 0, stream, m);
         hipLaunchKernelGGL(merger_taken_sums_kernel, dim3(merger_grid(words)), block, 0, stream, m, words);
@@ -812,9 +826,11 @@ int merger_rounds(int64_t V, int64_t E, int rounds, int min_pair_frequency, int3
         std::swap(m.seq, m.next_seq);
         std::swap(m.ptr, m.next_ptr);
         std::swap(m.active, m.next_active);
+        // at most the pairs around every new rule, and those listed before
+        const int64_t most = 2 * (int64_t)host[kTakenTotal] + m.listed;
         m.L -= host[kTakenTotal];
+        m.most = (int32_t)(most < m.L ? most : m.L);
         m.first = false;
-        most = host[kNextActive];
         R += added;
     }
     if (!checked) {

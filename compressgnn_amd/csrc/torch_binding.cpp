@@ -1500,10 +1500,9 @@ std::tuple<Tensor, Tensor, Tensor> neighbor_sample_ori_impl(Tensor colptr, Tenso
 // The 28 MB of int64 of a graph of 3.2 million edges took 0.4 ms to check and 0.7 ms to cross from pageable memory, and
 // the 13 MB of result 0.95 ms; the link takes 0.25 ms either way.  kSlots chunks are in flight at most,
 // whatever the size of the graph, and the pinned memory is the allocator's again after the call.
-// Chunks take turns on two streams, because a copy and the event behind it leave the link idle for a quarter of
-// the time that 2 MB take it.
+// Chunks take turns on two streams: behind a copy and its event the link is idle for 10 us if nothing else is there for it.
 struct Link {
-    static constexpr int64_t kChunk = 1 << 19, kSlots = 8;  // 2 MB: 38 us of the link, three times what they cost the host
+    static constexpr int64_t kChunk = 1 << 20, kSlots = 4;  // 4 MB: 76 us of the link, four times what they cost the host
     Tensor slots;
     hipStream_t streams[2];
     hipEvent_t sent[kSlots] = {}, ready = nullptr;
