@@ -843,7 +843,7 @@ def main():
         "dtype": "f32", "data": "synthetic",
         "config": workload,
         "frac_of_hbm_peak": value / HBM_PEAK_GBPS,
-        "roofline": {"bound": "hbm", "kernel": "cgnn_spmm_dual, forward vertex stage [v2v | v2r]: spmm_nnz_kernel<float,4,32,1,dual> + its fix-up pass",
+        "roofline": {"bound": "hbm", "kernel": "cgnn_spmm_dual, forward vertex stage [v2v | v2r]: spmm_nnz_kernel<float,4,32,1,dual,workgroup runs>",
                      "achieved": dom_gbps, "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": dom_gbps / HBM_PEAK_GBPS,
                      "traffic": traffic, "traffic_note": traffic_note, "ms": dom, "bytes": dom_bytes,
                      "event_samples": len(dom_samples)},
