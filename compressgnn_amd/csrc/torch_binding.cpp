@@ -51,6 +51,13 @@ void require_gpu(const Tensor &t, const char *name) {
     TORCH_CHECK(t.is_cuda(), name, " must be a GPU tensor: this build of compressgnn_runtime has no CPU operators");
 }
 
+// Whether what is launched on this stream is recorded into a graph: contents made now exist from a replay on only.
+bool capturing(const Tensor &like) {
+    hipStream_t stream = reinterpret_cast<hipStream_t>(current_stream(like));
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return stream != nullptr && hipStreamIsCapturing(stream, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
+}
+
 // Counters of the kernels whose last workgroup to arrive finishes a row (cgnn_csr.arrivals): every launch
 // leaves them at zero, so the launches of one stream share one set, and streams, which may overlap, each have
 // their own.  At most kStreams sets are held; the one used longest ago goes back to the allocator when another
@@ -68,9 +75,7 @@ struct ArrivalPool {
     Tensor get(int64_t n, const Tensor &like) {
         auto options = like.options().dtype(torch::kInt32).requires_grad(false);
         hipStream_t stream = reinterpret_cast<hipStream_t>(current_stream(like));
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        if (stream != nullptr && hipStreamIsCapturing(stream, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone)
-            return torch::zeros({n}, options);
+        if (capturing(like)) return torch::zeros({n}, options);
         std::lock_guard<std::mutex> hold(lock);
         const int device = like.device().index();
         auto it = std::find_if(sets.begin(), sets.end(), [&](const Set &s) { return s.device == device && s.stream == stream; });
@@ -108,7 +113,12 @@ struct Scratch {
             buf = torch::empty({(int64_t)std::max<size_t>(bytes, 1)}, like.options().dtype(torch::kUInt8));
         return buf;
     }
+    Tensor captured;  // those of the product recorded last: a graph has its own and zeroes them in every replay
     int32_t *counters(int64_t n, const Tensor &like) {
+        if (capturing(like)) {
+            captured = torch::zeros({std::max<int64_t>(n, 1)}, like.options().dtype(torch::kInt32));
+            return captured.data_ptr<int32_t>();
+        }
         if (!arrivals.defined() || arrivals.numel() < n || arrivals.device() != like.device())
             arrivals = torch::zeros({std::max<int64_t>(n, 1)}, like.options().dtype(torch::kInt32));
         return arrivals.data_ptr<int32_t>();
@@ -136,6 +146,7 @@ struct DeviceCsr {
         Tensor table;
     };
     std::vector<WgRuns> wg_runs;
+    Tensor captured_runs;  // the table of the product recorded last, where it was not there before: the graph fills it
 
     cgnn_csr view() const {
         cgnn_csr a{};
@@ -213,9 +224,10 @@ struct DeviceCsr {
                 Tensor table = torch::empty({(nnz + a.wg_len - 1) / a.wg_len * a.wg_groups + 1}, rowptr.options());
                 ok(cgnn_spmm_wg_runs(&a, a.wg_groups, a.wg_len, table.data_ptr<int32_t>(), current_stream(rowptr)),
                    "spmm_wg_runs");
-                found = wg_runs.insert(wg_runs.end(), WgRuns{a.wg_groups, a.wg_len, table});
+                if (capturing(rowptr)) captured_runs = table;
+                else found = wg_runs.insert(wg_runs.end(), WgRuns{a.wg_groups, a.wg_len, table});
             }
-            a.wg_runs = found->table.data_ptr<int32_t>();
+            a.wg_runs = (found != wg_runs.end() ? found->table : captured_runs).data_ptr<int32_t>();
             a.arrivals = scratch->counters(arrivals, rowptr);
         }
         *bytes = cgnn_spmm_workspace_bytes(&a, F, dtype, kernel);

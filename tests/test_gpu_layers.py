@@ -317,6 +317,28 @@ def test_propagation_replays_from_a_captured_graph():
         assert torch.equal(out_graph, out_eager) and torch.equal(gx_graph, gx_eager)
 
 
+def test_eager_products_before_the_first_replay():
+    """What a capture makes for a width that no product had before belongs to the graph: an eager product between
+    the capture and its first replay, when none of it has run, makes its own."""
+    data, _ = _make_data("copy", 64, True, 3, seed=4)
+    data.to(DEV)
+    plan = data.edge_index.plan()
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(10)
+    narrow, wide = (torch.randn(data.vertex_cnt, F, device=DEV, generator=gen) for F in (20, 250))
+    plan.forward(narrow), plan.backward(narrow)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out_graph, gx_graph = plan.forward(wide), plan.backward(wide)
+    out_eager, gx_eager = plan.forward(wide), plan.backward(wide)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out_graph, out_eager) and torch.equal(gx_graph, gx_eager)
+        assert torch.equal(plan.forward(wide), out_eager)
+
+
 def test_spmm_func_int64_api():
     """The reference's raw operator on int64 CSR tensors, all accepted method strings."""
     import compressgnn_runtime as rt
