@@ -110,6 +110,8 @@ struct SpmmArgs {
     int32_t keep;               // ... a row of at most this many entries is never divided, whatever the lengths
     int32_t find_empty;         // ... the rows without entries are found from rowptr, not from a list
     int32_t mean;               // MODE_UNIT, plain runs: every row is divided by its number of entries
+    const int32_t *span;        // WGRUNS_COMPUTED: {entries, where the first of them stands in val}, known on the device
+                                // only (cgnn_spmm_once); NULL: nnz entries from the start of val on
 };
 
 // An entry of the table of workgroup runs is the first non-zero of a run, with this bit set when the row
@@ -117,12 +119,15 @@ struct SpmmArgs {
 constexpr int32_t kRowGoesOn = INT32_MIN;
 
 // Where lane group g of workgroup w begins, as such an entry (the rule stands at cgnn_csr.wg_runs).
-__device__ __forceinline__ int32_t wg_run_begin(const int32_t *rowptr, const int32_t *rowidx, int32_t nnz, int32_t wg_len,
-                                                int32_t groups, int32_t keep, int64_t w, int g) {
+// held: length of rowidx, of which the first nnz entries count.
+__device__ __forceinline__ int32_t wg_run_begin(const int32_t *rowptr, const int32_t *rowidx, int32_t held, int32_t nnz,
+                                                int32_t wg_len, int32_t groups, int32_t keep, int64_t w, int g) {
     // e moved back to the start of its row when the row has at most `whole` entries
     auto begin_of = [&](int64_t e, int whole) -> int32_t {
+        if (e >= held) return nnz;
+        const int r = rowidx[e];  // asked for before nnz, which may come from memory too, is looked at
         if (e >= nnz) return nnz;
-        const int r = rowidx[e], s0 = rowptr[r];
+        const int s0 = rowptr[r];
         return rowptr[r + 1] - s0 <= whole ? s0 : (s0 < e ? (int32_t)e | kRowGoesOn : (int32_t)e);
     };
     const int run_len = wg_len / groups;
@@ -676,6 +681,12 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
     const int block = logical_block(a);
     int seg = block * GPB + grp;
     if constexpr (LPR == kWave) seg = __builtin_amdgcn_readfirstlane(seg);
+    int32_t dealt = a.nnz;
+    if constexpr (WGRUNS == WGRUNS_COMPUTED && MODE == MODE_VAL)
+        if (a.span != nullptr) {
+            dealt = a.span[0];
+            if (a.val != nullptr) a.val += a.span[1];
+        }
     int e0 = 0, e1 = 0;
     bool continues = false;    // the last row of the run goes on in the next one
     bool open = false;         // WGRUNS: the row at hand began before the run
@@ -687,7 +698,7 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                 r0 = a.run_start[seg], r1 = a.run_start[seg + 1];
             } else {
                 auto begin_of = [&](int w, int g) {
-                    return wg_run_begin(a.rowptr, a.rowidx, a.nnz, a.wg_len, GPB, a.keep, w, g);
+                    return wg_run_begin(a.rowptr, a.rowidx, a.nnz, dealt, a.wg_len, GPB, a.keep, w, g);
                 };
                 wg_begin = begin_of(block, 0), wg_behind = begin_of(block + 1, 0);
                 r0 = begin_of(block, grp), r1 = grp + 1 < GPB ? begin_of(block, grp + 1) : wg_behind;
@@ -1605,7 +1616,7 @@ __global__ void run_starts_kernel(const int32_t *__restrict__ rowptr, const int3
 __global__ void wg_runs_kernel(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ rowidx, int32_t nnz,
                                int32_t wg_len, int32_t groups, int64_t n, int32_t *__restrict__ runs) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) runs[i] = wg_run_begin(rowptr, rowidx, nnz, wg_len, groups, 0, i / groups, (int)(i % groups));
+    if (i < n) runs[i] = wg_run_begin(rowptr, rowidx, nnz, nnz, wg_len, groups, 0, i / groups, (int)(i % groups));
 }
 
 // rowidx[e] = largest r with rowptr[r] <= e (rows without entries are skipped).
@@ -1630,15 +1641,19 @@ __global__ void expand_rows_kernel(const P *__restrict__ rowptr, int64_t rows, i
 // workgroup per 16 rows took 41 us for 100,003 rows of 1.0 M entries of a web graph, whose hubs are neighbours) nor the
 // thousands of empty rows of the youngest vertices (2,048 entries per workgroup: 22 us) keep one longer than the others.
 // It looks for the two ends of its stretch with all its threads at once (256 row pointers a step), marks the entries
-// that rows begin at and spreads the marks by a running maximum: 8.6 us.  Row pointers and columns narrowed apart and a
+// that rows begin at and spreads the marks by a running maximum: 9.0 us.  Row pointers and columns narrowed apart and a
 // binary search per entry were three launches of 25 us, behind 26 us for the length of the longest row and its
 // way to the host.
+// The rows hold the entries [rowptr64[0], rowptr64[rows]) of the arrays: a slice of the row pointers of a larger block
+// comes with all its entries, and a list may be padded behind the last row.  Only these entries are taken over, and the
+// int32 arrays count from the first of them: span = {how many, where the first stands}.
 constexpr int kOnceItems = 8;
 constexpr int kOncePlaces = kOnceItems * kBlock;
 
 __global__ __launch_bounds__(kBlock) void csr_once_kernel(const int64_t *__restrict__ rowptr64, const int64_t *__restrict__ col64,
                                                           int64_t rows, int64_t nnz, int32_t *__restrict__ rowptr,
-                                                          int32_t *__restrict__ col, int32_t *__restrict__ rowidx) {
+                                                          int32_t *__restrict__ col, int32_t *__restrict__ rowidx,
+                                                          int32_t *__restrict__ span) {
     __shared__ int32_t begins[kOncePlaces];  // the row that begins at an entry of the stretch, or -1
     __shared__ int waves[2][kBlock / kWave];
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
@@ -1671,18 +1686,20 @@ __global__ __launch_bounds__(kBlock) void csr_once_kernel(const int64_t *__restr
         }
         __syncthreads();
     }
+    // the entries that belong to rows; row pointers that are none must not lead out of the arrays
+    const int64_t first = max((int64_t)0, min(nnz, rowptr64[0])), last = max(first, min(nnz, rowptr64[rows]));
+    auto inside = [&](int64_t e) { return max(first, min(last, e)); };
+    if (blockIdx.x == 0 && threadIdx.x == 0) span[0] = (int32_t)(last - first), span[1] = (int32_t)first;
     // first entry and first row of the stretch, and those behind it
     int64_t entry[2], row[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
         const int64_t start = rowptr64[lo[k]];
         const bool on_row = start + lo[k] >= places[k];  // the place is that of the row itself
-        entry[k] = on_row ? start : places[k] - lo[k] - 1;
+        entry[k] = inside(on_row ? start : places[k] - lo[k] - 1);
         row[k] = on_row ? lo[k] : lo[k] + 1;
-        // row pointers that are none must not lead out of the arrays
-        entry[k] = max((int64_t)0, min(nnz, entry[k]));
     }
-    if (places[1] == rows + nnz) entry[1] = nnz, row[1] = rows;
+    if (places[1] == rows + nnz) entry[1] = last, row[1] = rows;
     const int64_t e0 = entry[0];
     const int held = (int)max((int64_t)0, min((int64_t)kOncePlaces, entry[1] - e0));
     int64_t c[kOnceItems], at[kOnceItems], end[kOnceItems];
@@ -1691,15 +1708,18 @@ __global__ __launch_bounds__(kBlock) void csr_once_kernel(const int64_t *__restr
         const int k = u * kBlock + threadIdx.x;
         const int64_t r = row[0] + k;
         c[u] = k < held ? col64[e0 + k] : 0;
-        at[u] = r < row[1] ? rowptr64[r] : 0;
-        end[u] = r < row[1] ? rowptr64[r + 1] : 0;
+        // without a condition, on which the limits below would be worked out beside each load, the next one
+        // waiting behind them (11.1 us instead of 9.0)
+        at[u] = rowptr64[min(r, rows - 1)];
+        end[u] = rowptr64[min(r, rows - 1) + 1];
     }
 #pragma unroll
     for (int u = 0; u < kOnceItems; ++u) {
         const int64_t r = row[0] + u * kBlock + threadIdx.x;
         if (r >= row[1]) break;
-        rowptr[r] = (int32_t)at[u];
-        if (r == rows - 1) rowptr[rows] = (int32_t)end[u];
+        at[u] = inside(at[u]), end[u] = inside(end[u]);
+        rowptr[r] = (int32_t)(at[u] - first);
+        if (r == rows - 1) rowptr[rows] = (int32_t)(end[u] - first);
         // rows without entries begin where another does: not marked, so one row a mark
         const int64_t k = at[u] - e0;
         if (end[u] > at[u] && k >= 0 && k < held) begins[k] = (int32_t)r;
@@ -1734,8 +1754,8 @@ __global__ __launch_bounds__(kBlock) void csr_once_kernel(const int64_t *__restr
     for (int u = 0; u < kOnceItems; ++u) {
         const int k = u * kBlock + threadIdx.x;
         if (k < held) {
-            col[e0 + k] = (int32_t)c[u];
-            rowidx[e0 + k] = begins[k];
+            col[e0 - first + k] = (int32_t)c[u];
+            rowidx[e0 - first + k] = begins[k];
         }
     }
 }
@@ -1891,7 +1911,7 @@ extern "C" int cgnn_spmm_run_length(const cgnn_csr *A) { return A == nullptr ? 0
 namespace {
 
 struct OnceLayout {
-    size_t rowptr, col, rowidx, pieces, total;
+    size_t span, rowptr, col, rowidx, pieces, total;
     int groups, wg_len;
     int64_t workgroups;
 };
@@ -1905,8 +1925,9 @@ OnceLayout once_layout(int64_t rows, int64_t nnz, int64_t F, int dtype) {
     L.groups = kBlock / shape_of(F, dtype).lpr;
     L.wg_len = wg_run_len(&A, L.groups) * L.groups;
     L.workgroups = ceil_div(nnz, L.wg_len);
-    L.rowptr = 0;
-    L.col = align_up((size_t)(rows + 1) * sizeof(int32_t), 256);
+    L.span = 0;
+    L.rowptr = 256;
+    L.col = L.rowptr + align_up((size_t)(rows + 1) * sizeof(int32_t), 256);
     L.rowidx = L.col + align_up((size_t)nnz * sizeof(int32_t), 256);
     L.pieces = L.rowidx + align_up((size_t)nnz * sizeof(int32_t), 256);
     L.total = L.pieces + wg_piece_bytes(L.workgroups, F, dtype == CGNN_F64 ? 8 : 4);
@@ -1930,6 +1951,7 @@ int spmm_once(const OnceLayout &L, int64_t rows, int64_t nnz, const void *val, i
     a.nseg = (int32_t)(L.workgroups * L.groups);
     a.carry = reinterpret_cast<T *>(ws + L.pieces);
     a.find_empty = 1;
+    a.span = reinterpret_cast<const int32_t *>(ws + L.span);
     return launch<T>(KIND_NNZ, MODE_VAL, pick_shape<T>(F, true), a, a.nseg, stream);
 }
 
@@ -1955,7 +1977,7 @@ extern "C" int cgnn_spmm_once(int64_t rows, int64_t nnz, const int64_t *rowptr, 
     char *ws = static_cast<char *>(workspace);
     hipLaunchKernelGGL(csr_once_kernel, dim3((unsigned)ceil_div(rows + nnz, kOncePlaces)), dim3(kBlock), 0, stream,
                        rowptr, col, rows, nnz, reinterpret_cast<int32_t *>(ws + L.rowptr), reinterpret_cast<int32_t *>(ws + L.col),
-                       reinterpret_cast<int32_t *>(ws + L.rowidx));
+                       reinterpret_cast<int32_t *>(ws + L.rowidx), reinterpret_cast<int32_t *>(ws + L.span));
     int rc = check_launch("csr_once");
     if (rc != CGNN_OK) return rc;
     if (dtype == CGNN_F32)

@@ -280,8 +280,21 @@ std::shared_ptr<DeviceCsr> make_csr(Tensor rowptr, Tensor col, c10::optional<Ten
         blk->rowmap = rowmap->to(device).to(torch::kInt32).contiguous();
     }
     if (rows > 0) {
+        // one host read per block, at build time: the longest row, and which entries of the arrays the rows hold
         Tensor lens = blk->rowptr.slice(0, 1, rows + 1) - blk->rowptr.slice(0, 0, rows);
-        blk->max_row_nnz = lens.max().item<int32_t>();  // one host read per block, at build time
+        Tensor found = torch::stack({lens.max(), blk->rowptr[0], blk->rowptr[rows]}).cpu();
+        blk->max_row_nnz = found.data_ptr<int32_t>()[0];
+        const int64_t first = found.data_ptr<int32_t>()[1], held = found.data_ptr<int32_t>()[2] - first;
+        if (first != 0 || held != blk->nnz) {
+            // a slice of a larger block's row pointers, or a list that is padded behind its last row: the schedules
+            // deal the entries 0 ... nnz, so the block keeps the ones in use and counts from the first of them
+            TORCH_CHECK(held == 0 || (first >= 0 && held > 0 && first + held <= blk->nnz),
+                        "rowptr names entries that col does not have");
+            blk->rowptr = blk->rowptr - first;
+            blk->colidx = blk->colidx.narrow(0, held == 0 ? 0 : first, held).clone();
+            if (blk->val.defined()) blk->val = blk->val.narrow(0, held == 0 ? 0 : first, held).clone();
+            blk->nnz = held;
+        }
     }
     if (with_row_lists) blk->list_rows();
     return blk;

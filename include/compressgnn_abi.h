@@ -54,7 +54,7 @@ typedef struct cgnn_csr {
     int64_t rows;
     int64_t cols;
     int64_t nnz;
-    const int32_t *rowptr; /* [rows+1] */
+    const int32_t *rowptr; /* [rows+1]; rowptr[0] = 0 and rowptr[rows] = nnz (the NNZ schedule deals the entries 0 ... nnz) */
     const int32_t *colidx; /* [nnz]    */
     const int32_t *rowidx; /* [nnz] or NULL */
     const void *val;       /* [nnz] of the call's dtype, or NULL */
@@ -131,7 +131,9 @@ size_t cgnn_spmm_workspace_bytes(const cgnn_csr *A, int64_t F, int dtype, int ke
  * has made once: the arrays are narrowed by the call (one launch), the schedule is the NNZ one with workgroup runs
  * whatever the rows look like, and nothing is read by the host.  A row of at most 64 entries is summed in
  * ascending order.  arrivals: counters as in cgnn_csr, as many as the size query reports.  rows, nnz and F must
- * be positive; the columns must lie in X (not checked).
+ * be positive; the row pointers must ascend and the columns of the rows must lie in X (not checked).  nnz is the length of
+ * col and val; the rows hold the entries [rowptr[0], rowptr[rows]) of them (a slice of a larger block's row pointers, or
+ * a list padded behind its last row), and no other entry is read.
  * Replaces spmm_func: src/runtime/csrc/sparse/spmm.cpp:11-22. */
 size_t cgnn_spmm_once_workspace_bytes(int64_t rows, int64_t nnz, int64_t F, int dtype, int64_t *arrivals);
 int cgnn_spmm_once(int64_t rows, int64_t nnz, const int64_t *rowptr, const int64_t *col, const void *val, int dtype,

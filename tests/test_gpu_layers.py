@@ -833,3 +833,39 @@ def test_spmm_func_on_blocks_of_every_shape(shape, accumulate):
         assert_within(got, want, rtol=1e-5, atol=2e-5)
     short = lens <= 64
     assert np.array_equal(got[short], oracle.spmm(vlist, elist, value, x, out0.copy())[short])
+
+
+@pytest.mark.parametrize("method", ["auto", "row_schedule", "nnz_schedule"])
+@pytest.mark.parametrize("hubs", [False, True])
+@pytest.mark.parametrize("rows", [(0, 3000), (1, 3000), (0, 2999), (1234, 1235), (700, 2900)])
+def test_spmm_func_on_a_slice_of_the_rows(rows, hubs, method):
+    """Row pointers sliced out of a larger block, with all its entries, and lists padded behind the last row: the rows
+    of the whole product, bit for bit where a row is never divided.  Entries outside the rows are NaN: none is used."""
+    import compressgnn_runtime as rt
+    rng = np.random.default_rng(23)
+    lens = rng.integers(0, 9, 3000)
+    if hubs:
+        lens[::500] = 3000
+    vlist = np.concatenate([[0], np.cumsum(lens)])
+    cols, F = 700, 20
+    elist = rng.integers(0, cols, int(vlist[-1]))
+    value = (rng.standard_normal(len(elist)) * 0.3 / np.sqrt(np.maximum(np.repeat(lens, lens), 1))).astype(np.float32)
+    x = rng.standard_normal((cols, F)).astype(np.float32)
+    t = lambda a: torch.from_numpy(a).to(DEV)
+    whole = np.zeros((len(lens), F))
+    np.add.at(whole, np.repeat(np.arange(len(lens)), lens), value[:, None].astype(np.float64) * x[elist])
+    sequential = oracle.spmm(vlist, elist, value, x)
+    a, b = rows
+    outside = np.ones(len(elist) + 777, bool)
+    outside[vlist[a]:vlist[b]] = False
+    padded = np.concatenate([value, np.zeros(777, np.float32)])
+    padded[outside] = np.nan
+    args = t(vlist[a:b + 1].copy()), t(np.concatenate([elist, np.zeros(777, np.int64)])), t(padded)
+    got = rt.spmm_func(*args, t(x), method, None).cpu().numpy()
+    assert_within(got, whole[a:b], rtol=1e-5, atol=2e-5)
+    short = lens[a:b] <= 64
+    assert np.array_equal(got[short], sequential[a:b][short])
+    added = rt.spmm_func(*args, t(x), method, torch.ones(b - a, F, device=DEV)).cpu().numpy()
+    assert_within(added, whole[a:b] + 1, rtol=1e-5, atol=2e-5)
+    wide = rt.spmm_func(args[0], args[1], args[2].double(), t(x).double(), method, None).cpu().numpy()
+    np.testing.assert_allclose(wide, whole[a:b], rtol=1e-12, atol=1e-12)
