@@ -58,6 +58,26 @@ bool capturing(const Tensor &like) {
     return stream != nullptr && hipStreamIsCapturing(stream, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
 }
 
+// A lock over what the products of a block or a plan share.  The gradient of a native step runs on a thread of the
+// autograd engine, without the interpreter's lock, while the program's own threads may be in another product of the
+// same plan; the launches of both are ordered by their stream, the host objects behind them by this.  A thread that
+// has to wait lets go of the interpreter, so that the one that holds the lock may need it (a dispatch mode's torch.empty);
+// recursive for the same reason: such a mode may run a product of its own.
+class Hold {
+    std::unique_lock<std::recursive_mutex> lock;
+
+public:
+    explicit Hold(std::recursive_mutex &m) : lock(m, std::try_to_lock) {
+        if (lock.owns_lock()) return;
+        if (PyGILState_Check()) {
+            pybind11::gil_scoped_release others;
+            lock.lock();
+        } else {
+            lock.lock();
+        }
+    }
+};
+
 // Counters of the kernels whose last workgroup to arrive finishes a row (cgnn_csr.arrivals): every launch
 // leaves them at zero, so the launches of one stream share one set, and streams, which may overlap, each have
 // their own.  At most kStreams sets are held; the one used longest ago goes back to the allocator when another
@@ -106,6 +126,9 @@ ArrivalPool &arrival_pool() {
 // scratch at the same time would overwrite each other's carries: a caller who does that
 // gives each stream a plan (or a block) of its own.
 struct Scratch {
+    // Held from DeviceCsr::prepare to the launch of the product: over this scratch and over the tables that the blocks
+    // with this scratch make on their first product.
+    std::recursive_mutex lock;
     Tensor buf;
     Tensor arrivals;  // counters that every product leaves at zero
     const Tensor &get(size_t bytes, const Tensor &like) {
@@ -209,7 +232,8 @@ struct DeviceCsr {
         run_start = starts;
     }
 
-    // The block as a product of width F reads it, and the scratch for that product.
+    // The block as a product of width F reads it, and the scratch for that product; the caller holds scratch->lock until
+    // the product is launched.
     cgnn_csr prepare(int64_t F, int dtype, int kernel, void **ws, size_t *bytes) {
         ensure_rowidx(kernel);
         cgnn_csr a = view();
@@ -235,6 +259,13 @@ struct DeviceCsr {
         return a;
     }
 };
+
+// A tensor of the block that a product on another thread may be making.
+Tensor locked(DeviceCsr &A, Tensor DeviceCsr::*made) {
+    const std::shared_ptr<Scratch> scratch = A.scratch;
+    Hold hold(scratch->lock);
+    return A.*made;
+}
 
 // rowptr/col: int64 or int32 tensors on any device; value: float tensor or undefined.
 std::shared_ptr<DeviceCsr> make_csr(Tensor rowptr, Tensor col, c10::optional<Tensor> value, int64_t rows,
@@ -346,6 +377,8 @@ Tensor block_spmm(DeviceCsr &A, const Tensor &mat, c10::optional<Tensor> optiona
     if (A.rows == 0 || F == 0) return out;
     size_t bytes = 0;
     void *ws = nullptr;
+    const std::shared_ptr<Scratch> scratch = A.scratch;
+    Hold hold(scratch->lock);
     cgnn_csr a = A.prepare(F, dtype, kernel, &ws, &bytes);
     ok(cgnn_spmm(&a, dtype, mat.data_ptr(), out.data_ptr(), F, accumulate, kernel, ws, bytes,
                  current_stream(mat)),
@@ -471,6 +504,7 @@ struct PropagationPlan {
     bool fuse_final = true;  // last two stages in one pass (cgnn_spmm_dual)
     int kernel = CGNN_SPMM_AUTO;
     std::shared_ptr<Scratch> scratch = std::make_shared<Scratch>();
+    std::recursive_mutex lock;  // held for a chain of products: over the timer and the composed blocks
     StageTimer timer;
     // The forward blocks with their vertex columns sent through a cluster assignment
     // (propagate_forward_gathered), kept for the index tensors they were made for: an
@@ -515,6 +549,8 @@ Tensor final_stage(PropagationPlan &p, const std::string &prefix, DeviceCsr *mer
         const int dtype = dtype_code(x);
         size_t bytes = 0;
         void *ws = nullptr;
+        const std::shared_ptr<Scratch> scratch = merged->scratch;
+        Hold hold(scratch->lock);
         cgnn_csr a = merged->prepare(F, dtype, p.kernel, &ws, &bytes);
         hipStream_t stream = reinterpret_cast<hipStream_t>(current_stream(x));
         const int id = p.timer.open(prefix + "final", stream);
@@ -536,6 +572,7 @@ Tensor propagate_forward(PropagationPlan &p, Tensor x) {
     TORCH_CHECK(x.dim() == 2 && x.size(0) == p.V, "x must be [vertex_cnt, F]");
     x = x.contiguous();
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    Hold hold(p.lock);
     Tensor rule_out = timed_spmm(p, "fwd.rules", *p.r2v, x, c10::nullopt);
     for (size_t i = 0; i < p.r2r.size(); ++i)
         rule_out = timed_spmm(p, "fwd.level" + std::to_string(i), *p.r2r[i], rule_out, rule_out);
@@ -545,6 +582,8 @@ Tensor propagate_forward(PropagationPlan &p, Tensor x) {
 // A copy of a block that shares everything but the column numbers: the columns below
 // `first_cols` go through `index` (cgnn_csr_compose_columns).
 std::shared_ptr<DeviceCsr> compose_block(const DeviceCsr &A, const Tensor &narrow, int64_t first_cols, int64_t cols) {
+    const std::shared_ptr<Scratch> scratch = A.scratch;
+    Hold hold(scratch->lock);
     auto blk = std::make_shared<DeviceCsr>(A);
     blk->cols = cols;
     if (A.nnz > 0) {
@@ -573,6 +612,7 @@ Tensor propagate_forward_gathered(PropagationPlan &p, Tensor reps, Tensor index)
     reps = reps.contiguous();
     c10::hip::HIPGuardMasqueradingAsCUDA guard(reps.device());
     const int64_t groups = reps.size(0), F = reps.size(1);
+    Hold hold(p.lock);
     std::shared_ptr<DeviceCsr> rules, stage;
     for (auto it = p.composed.begin(); it != p.composed.end();) {
         if (it->index.expired()) {
@@ -610,6 +650,8 @@ Tensor propagate_forward_gathered(PropagationPlan &p, Tensor reps, Tensor index)
     const int dtype = dtype_code(reps);
     size_t bytes = 0;
     void *ws = nullptr;
+    const std::shared_ptr<Scratch> scratch = stage->scratch;
+    Hold products(scratch->lock);
     cgnn_csr a = stage->prepare(F, dtype, p.kernel, &ws, &bytes);
     hipStream_t stream = reinterpret_cast<hipStream_t>(current_stream(reps));
     const int id = p.timer.open("fwd.final", stream);
@@ -627,6 +669,7 @@ Tensor propagate_backward(PropagationPlan &p, Tensor grad) {
     TORCH_CHECK(grad.dim() == 2 && grad.size(0) == p.V, "grad must be [vertex_cnt, F]");
     grad = grad.contiguous();
     c10::hip::HIPGuardMasqueradingAsCUDA guard(grad.device());
+    Hold hold(p.lock);
     Tensor rule_g = timed_spmm(p, "bwd.rules", *p.v2r_t, grad, c10::nullopt);
     for (size_t i = p.r2r_t.size(); i-- > 0;)
         rule_g = timed_spmm(p, "bwd.level" + std::to_string(i), *p.r2r_t[i], rule_g, rule_g);
@@ -1710,18 +1753,20 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         .def_readonly("max_row_nnz", &DeviceCsr::max_row_nnz)
         .def_property("seg_nnz", [](DeviceCsr &self) { return self.seg_nnz; },
                       [](DeviceCsr &self, int32_t seg) {
+                          const std::shared_ptr<Scratch> scratch = self.scratch;
+                          Hold hold(scratch->lock);
                           self.seg_nnz = seg;
                           self.run_start = Tensor();  // made again by the next product, like the workgroup runs
                           self.wg_runs.clear();
                           if (self.cut_rows.defined()) self.list_rows();  // the lists belong to a run length
                       })
         .def_readwrite("workgroup_runs", &DeviceCsr::workgroup_runs)
-        .def_readonly("cut_rows", &DeviceCsr::cut_rows)
-        .def_readonly("run_start", &DeviceCsr::run_start)
-        .def_readonly("empty_rows", &DeviceCsr::empty_rows)
+        .def_property_readonly("cut_rows", [](DeviceCsr &self) { return locked(self, &DeviceCsr::cut_rows); })
+        .def_property_readonly("run_start", [](DeviceCsr &self) { return locked(self, &DeviceCsr::run_start); })
+        .def_property_readonly("empty_rows", [](DeviceCsr &self) { return locked(self, &DeviceCsr::empty_rows); })
         .def_readonly("rowptr", &DeviceCsr::rowptr)
         .def_readonly("colidx", &DeviceCsr::colidx)
-        .def_readonly("rowidx", &DeviceCsr::rowidx)
+        .def_property_readonly("rowidx", [](DeviceCsr &self) { return locked(self, &DeviceCsr::rowidx); })
         .def_readonly("val", &DeviceCsr::val)
         .def("spmm",
              [](DeviceCsr &self, Tensor mat, c10::optional<Tensor> out, std::string method) {
@@ -1749,12 +1794,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                  TORCH_CHECK(fwd && bwd && fwd->rows == p.V && bwd->rows == p.V && fwd->cols == p.V + p.R &&
                                  bwd->cols == p.V + p.R,
                              "a vertex stage is [vertex_cnt, vertex_cnt + rule_cnt]");
+                 Hold hold(p.lock);
                  p.vertex_stage = fwd; p.vertex_stage_t = bwd;
                  p.adopt(fwd); p.adopt(bwd);
              })
         .def("set_split_blocks",
              [](PropagationPlan &p, std::shared_ptr<DeviceCsr> v2v, std::shared_ptr<DeviceCsr> v2r,
                 std::shared_ptr<DeviceCsr> v2v_t, std::shared_ptr<DeviceCsr> r2v_t) {
+                 Hold hold(p.lock);
                  p.v2v = v2v; p.v2r = v2r; p.v2v_t = v2v_t; p.r2v_t = r2v_t;
                  p.adopt(v2v); p.adopt(v2r); p.adopt(v2v_t); p.adopt(r2v_t);
                  p.require_split_blocks();
@@ -1763,24 +1810,43 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                       [](PropagationPlan &p, bool fuse) {
                           if (!fuse) p.require_split_blocks();
                           else TORCH_CHECK(p.vertex_stage && p.vertex_stage_t, "this plan has no fused vertex stages");
+                          Hold hold(p.lock);
                           p.fuse_final = fuse;
                       })
         .def_readonly("vertex_stage", &PropagationPlan::vertex_stage)
         .def_readonly("vertex_stage_t", &PropagationPlan::vertex_stage_t)
         .def_property_readonly("scratch_bytes",
-                               [](PropagationPlan &p) { return p.scratch->buf.defined() ? p.scratch->buf.numel() : 0; })
+                               [](PropagationPlan &p) {
+                                   Hold hold(p.scratch->lock);
+                                   return p.scratch->buf.defined() ? p.scratch->buf.numel() : 0;
+                               })
         .def_property("method",
                       [](PropagationPlan &p) { return p.kernel == CGNN_SPMM_ROW ? "row_schedule" : p.kernel == CGNN_SPMM_NNZ ? "nnz_schedule" : "auto"; },
-                      [](PropagationPlan &p, std::string mth) { p.kernel = kernel_of_method(mth); })
-        .def_property("timed_stages", [](PropagationPlan &p) { return p.timer.timed; },
-                      [](PropagationPlan &p, std::vector<std::string> names) { p.timer.timed = names; })
+                      [](PropagationPlan &p, std::string mth) {
+                          Hold hold(p.lock);
+                          p.kernel = kernel_of_method(mth);
+                      })
+        .def_property("timed_stages",
+                      [](PropagationPlan &p) {
+                          Hold hold(p.lock);
+                          return p.timer.timed;
+                      },
+                      [](PropagationPlan &p, std::vector<std::string> names) {
+                          Hold hold(p.lock);
+                          p.timer.timed = names;
+                      })
         .def_property("timed_every", [](PropagationPlan &p) { return p.timer.every; },
                       [](PropagationPlan &p, int64_t n) {
                           TORCH_CHECK(n >= 1, "timed_every must be at least 1");
+                          Hold hold(p.lock);
                           p.timer.every = n;
                           p.timer.passes.clear();
                       })
-        .def("take_stage_times", [](PropagationPlan &p) { return p.timer.take(); })
+        .def("take_stage_times",
+             [](PropagationPlan &p) {
+                 Hold hold(p.lock);
+                 return p.timer.take();
+             })
         .def_readonly("v2v", &PropagationPlan::v2v)
         .def_readonly("v2r", &PropagationPlan::v2r)
         .def_readonly("r2v", &PropagationPlan::r2v)

@@ -869,3 +869,50 @@ def test_spmm_func_on_a_slice_of_the_rows(rows, hubs, method):
     assert_within(added, whole[a:b] + 1, rtol=1e-5, atol=2e-5)
     wide = rt.spmm_func(args[0], args[1], args[2].double(), t(x).double(), method, None).cpu().numpy()
     np.testing.assert_allclose(wide, whole[a:b], rtol=1e-12, atol=1e-12)
+
+
+def test_products_of_one_plan_from_several_threads():
+    """Forward in one thread, forward and gradient (which runs on the engine's thread) in others, all over one plan and one
+    stream, at widths that make each product ask for other scratch, counters and tables: every result is that of a
+    program with one thread, and the timer keeps its records whole."""
+    import threading
+    from KPropagate import KPropagate
+    data, _ = _make_data("copy", 8, True, 3, seed=4)
+    data.to(DEV)
+    graph, hop = data.edge_index, KPropagate()
+    plan = graph.plan()
+    plan.timed_stages = ["bwd.final"]
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(12)
+    widths = [5, 250, 16, 130, 33, 64]
+    inputs = {F: torch.randn(data.vertex_cnt, F, device=DEV, generator=gen) for F in widths}
+
+    def step(x, F):
+        x = x.detach().requires_grad_()
+        out = hop(x, graph, None, data.vertex_cnt, data.rule_cnt)
+        return out.detach(), torch.autograd.grad(out, x, inputs[F])[0]
+
+    failures, rounds = [], 12
+    results = [[] for _ in range(3)]
+
+    def work(k):
+        try:
+            for r in range(rounds):
+                F = widths[(r + 2 * k) % len(widths)]
+                results[k].append((F,) + (step(inputs[F], F) if k else (plan.forward(inputs[F]),)))
+        except Exception as e:  # reported by the test's own thread
+            failures.append(e)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures, failures
+    times = plan.take_stage_times()
+    assert len(times) == 2 * rounds and all(name == "bwd.final" and ms > 0 for name, ms in times)
+    plan.timed_stages = []
+    for k in range(3):
+        for F, *got in results[k]:
+            want = step(inputs[F], F)
+            assert all(torch.equal(a, b) for a, b in zip(got, want))
