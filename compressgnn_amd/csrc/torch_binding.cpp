@@ -7,11 +7,13 @@
 // are rejected with an error.
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <hip/hip_runtime_api.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/extension.h>
 
 #include <algorithm>
@@ -676,21 +678,53 @@ Tensor propagate_backward(PropagationPlan &p, Tensor grad) {
     return final_stage(p, "bwd.", p.vertex_stage_t.get(), p.r2v_t, rule_g, p.v2v_t, grad);
 }
 
+// Where a native step of autograd does not do what an autograd function of Python does: under torch.jit.trace, which
+// records a function as an operation on its inputs but the result of a native call as a constant; for inputs with a
+// forward-mode tangent and under the transforms of torch.func, which a function without the rules for them refuses.
+// The layers ask and take their function there; the steps themselves refuse.
+bool needs_function(const Tensor &a, const c10::optional<Tensor> &b) {
+    return torch::jit::tracer::isTracing() || a._fw_grad(0).defined() || (b.has_value() && b->defined() && b->_fw_grad(0).defined()) ||
+           c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
+
+void require_plain(const char *op, const Tensor &a, const c10::optional<Tensor> &b = c10::nullopt) {
+    TORCH_CHECK_NOT_IMPLEMENTED(!needs_function(a, b), op, ": a native step has no forward-mode gradient and is not recorded by "
+                                "torch.jit.trace or torch.func; the layers' autograd functions are for those");
+}
+
+// A gradient asked for with create_graph, of a step that has first-order gradients only: it cannot be differentiated
+// again and says so.
+torch::autograd::variable_list first_order(torch::autograd::variable_list grads, bool recorded) {
+    if (!recorded) return grads;
+    auto refuse = std::make_shared<torch::autograd::DelayedError>(
+        "trying to differentiate twice a function that has first-order gradients only (once_differentiable)", 1);
+    for (Tensor &g : grads)
+        if (g.defined()) g = (*refuse)({g.requires_grad() ? g : g.detach().requires_grad_()})[0];
+    return grads;
+}
+
 // One propagation as a step of autograd.  The node is native, so a training step takes neither the
 // interpreter nor its lock on the way back (the engine's thread and the caller's would pass the lock to each
 // other): forward and gradient over 2,708 vertices took 69 us through a Python function and take 54 us so, 29
 // of them the engine's own.
 struct PropagateBackward : torch::autograd::Node {
     std::shared_ptr<PropagationPlan> plan;
+    bool once = false;  // whether a second differentiation is refused (else the gradient counts as a constant there)
     torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
         if (!grads[0].defined()) return {Tensor()};
-        at::NoGradGuard no_grad;
-        return {propagate_backward(*plan, grads[0])};
+        const bool recorded = once && at::GradMode::is_enabled();
+        Tensor out;
+        {
+            at::NoGradGuard no_grad;
+            out = propagate_backward(*plan, grads[0]);
+        }
+        return first_order({out}, recorded);
     }
     std::string name() const override { return "PropagateBackward"; }
 };
 
-Tensor propagate(const std::shared_ptr<PropagationPlan> &plan, const Tensor &x) {
+Tensor propagate(const std::shared_ptr<PropagationPlan> &plan, const Tensor &x, bool once_differentiable) {
+    require_plain("propagate", x);
     const bool differentiable = at::GradMode::is_enabled() && x.requires_grad();
     Tensor out;
     {
@@ -700,6 +734,7 @@ Tensor propagate(const std::shared_ptr<PropagationPlan> &plan, const Tensor &x) 
     if (differentiable) {
         std::shared_ptr<PropagateBackward> node(new PropagateBackward(), torch::autograd::deleteNode);
         node->plan = plan;
+        node->once = once_differentiable;
         node->set_next_edges(torch::autograd::collect_next_edges(x));
         torch::autograd::set_history(out, node);
     }
@@ -1197,17 +1232,8 @@ Tensor cluster_reconstruct_backward_signs(Tensor grad, Tensor index, Tensor sign
 
 // ------------------------------------------------------ the layers' autograd steps ----
 //
-// Native nodes, for the reason given at PropagateBackward.  They give first-order gradients (as the reference's
-// functions do): a gradient asked for with create_graph cannot be differentiated again and says so.
-
-torch::autograd::variable_list first_order(torch::autograd::variable_list grads, bool recorded) {
-    if (!recorded) return grads;
-    auto refuse = std::make_shared<torch::autograd::DelayedError>(
-        "trying to differentiate twice a function that has first-order gradients only (once_differentiable)", 1);
-    for (Tensor &g : grads)
-        if (g.defined()) g = (*refuse)({g.requires_grad() ? g : g.detach().requires_grad_()})[0];
-    return grads;
-}
+// Native nodes, for the reason given at PropagateBackward.  They give first-order gradients, as the reference's
+// functions do.
 
 template <typename Node>
 std::shared_ptr<Node> node_over(const Tensor &a, const Tensor &b = Tensor()) {
@@ -1252,6 +1278,7 @@ void attach_mean(Tensor &reps, const Tensor &x, const Tensor &index, const Tenso
 // lengths of its lists).
 Tensor cluster_representatives(Tensor x, Tensor index, Tensor counts, std::vector<Tensor> members) {
     const char *op = "cluster_mean";
+    require_plain(op, x);
     Tensor reps;
     {
         at::AutoDispatchBelowADInplaceOrView plain;
@@ -1269,6 +1296,7 @@ Tensor cluster_representatives(Tensor x, Tensor index, Tensor counts, std::vecto
 
 // A refresh: (representatives, ids, counts, active, member lists).
 std::tuple<Tensor, Tensor, Tensor, int64_t, std::vector<Tensor>> cluster_refresh(Tensor x, Tensor planes, int64_t bits) {
+    require_plain("cluster_refresh", x);
     Assigned a;
     {
         at::AutoDispatchBelowADInplaceOrView plain;
@@ -1328,6 +1356,7 @@ struct ReconstructBackward : torch::autograd::Node {
 // per element, written by the kernel that produces the rows (the reference keeps the rows themselves:
 // layer/CompressgnnReconstruct.py:16-22); without a ReLU nothing of the [N, F] output is needed again.
 Tensor reconstruct(Tensor reps, Tensor index, c10::optional<Tensor> bias, bool relu, Members members) {
+    require_plain("reconstruct", reps, bias);
     Tensor rows, signs, ids;
     {
         at::AutoDispatchBelowADInplaceOrView plain;
@@ -1736,7 +1765,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("reconstruct", &reconstruct, "act(reps[index] + bias) with its gradients", py::arg("reps"), py::arg("index"),
           py::arg("bias"), py::arg("relu"), py::arg("members") = py::none());
     m.def("column_sums", &column_sums, "sum over the rows of a matrix");
-    m.def("propagate", &propagate, "plan.forward(x) with plan.backward as its gradient", py::arg("plan"), py::arg("x"));
+    m.def("propagate", &propagate, "plan.forward(x) with plan.backward as its gradient", py::arg("plan"), py::arg("x"),
+          py::arg("once_differentiable") = false);
+    m.def("needs_function", &needs_function, "whether a step on these inputs has to be an autograd function: the native steps "
+          "(propagate, cluster_refresh, cluster_representatives, reconstruct) refuse them", py::arg("a"), py::arg("b") = py::none());
     m.def("version", []() { return std::string(cgnn_version()); });
     py::class_<DeviceCsr, std::shared_ptr<DeviceCsr>>(m, "DeviceCsr")
         .def(py::init([](Tensor rowptr, Tensor col, c10::optional<Tensor> value, int64_t rows, int64_t cols,

@@ -215,9 +215,9 @@ class CooPropagateFunction(torch.autograd.Function):
 
 def coo_propagate(plan, x):
     """plan.forward(x) with its gradient; a chain's step of autograd is native."""
-    if plan.chain is None or x.dim() != 2 or x.size(0) != plan.V:
+    if plan.chain is None or x.dim() != 2 or x.size(0) != plan.V or _native.needs_function(x):
         return CooPropagateFunction.apply(plan, x)
-    return _native.propagate(plan.chain, x)
+    return _native.propagate(plan.chain, x, once_differentiable=True)
 
 
 class CooPlanCache:

@@ -916,3 +916,62 @@ def test_products_of_one_plan_from_several_threads():
         for F, *got in results[k]:
             want = step(inputs[F], F)
             assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def _steps_of_every_layer():
+    """(name, function of one tensor, rows, width) of each layer's differentiable step."""
+    from CompressgnnCluster import Compressgnn_Cluster
+    from CompressgnnReconstruct import Compressgnn_Reconstruct
+    from KPropagate import KPropagate
+    data, _ = _make_data("copy", 8, True, 3, seed=4)
+    data.to(DEV)
+    V, hop = data.vertex_cnt, KPropagate()
+    edges = torch.randint(0, V, (2, 4 * V), device=DEV)
+    torch.manual_seed(6)
+    fresh = Compressgnn_Cluster(12, 5, training=True, device=DEV, cache=False)
+    held = Compressgnn_Cluster(12, 5, training=True, device=DEV, refresh_interval=5)
+    with torch.no_grad():
+        held(torch.randn(V, 12, device=DEV), epoch=0)
+    index = torch.randint(0, 30, (V,), device=DEV)
+    bias = torch.randn(12, device=DEV)
+    return [("csr", lambda x: hop(x, data.edge_index, None, V, data.rule_cnt), V, 12),
+            ("coo", lambda x: hop.propagate(edges, x), V, 12),
+            ("cluster_fresh", lambda x: fresh(x)[0], V, 12),
+            ("cluster_held", lambda x: held(x, epoch=1)[0], V, 12),
+            ("reconstruct", lambda x: Compressgnn_Reconstruct()(x, index, bias, "relu"), 30, 12)]
+
+
+@pytest.mark.filterwarnings("ignore")
+def test_steps_where_a_native_one_would_be_lost():
+    """torch.jit.trace records a layer as an operation on its input; tangents and torch.func transforms are refused (no
+    layer has rules for them) and never dropped; all but the propagation of a CompressGraph refuse a second differentiation."""
+    import torch.autograd.forward_ad as forward_mode
+    import compressgnn_runtime as rt
+    for name, step, rows, width in _steps_of_every_layer():
+        x, y = (torch.randn(rows, width, device=DEV) for _ in range(2))
+        with forward_mode.dual_level():
+            with pytest.raises(NotImplementedError):
+                step(forward_mode.make_dual(x, y))
+        with pytest.raises(RuntimeError):
+            torch.func.grad(lambda t: step(t).sum())(x)
+        with pytest.raises(RuntimeError):
+            torch.func.vmap(step)(torch.stack([x, y]))
+        if name == "cluster_fresh":  # a trace cannot hold an assignment that is made anew
+            with pytest.raises(RuntimeError):
+                torch.jit.trace(step, (x,), check_trace=False)
+        else:
+            traced = torch.jit.trace(step, (x,), check_trace=False)
+            assert torch.equal(traced(x), step(x)) and torch.equal(traced(y), step(y)), name
+        z = x.clone().requires_grad_()
+        first, = torch.autograd.grad(step(z).square().sum(), z, create_graph=True)
+        again = (first * y).sum() + (z * y).sum()
+        if name == "csr":  # no second-order term, as Compressgnn_SPMM_Function has none
+            again.backward()
+            assert torch.equal(z.grad, y)
+        else:
+            with pytest.raises(RuntimeError, match="twice"):
+                again.backward()
+    with forward_mode.dual_level():
+        dual = forward_mode.make_dual(x, y)
+        with pytest.raises(NotImplementedError):
+            rt.reconstruct(dual, torch.zeros(5, dtype=torch.int64, device=DEV), None, False)
