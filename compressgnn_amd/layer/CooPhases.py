@@ -49,12 +49,12 @@ class _Edges:
 
     def __init__(self, edge_index, edge_weight, V, R):
         self.V, self.R, self.phases = V, R, len(edge_index)
-        ends = torch.cat([e.detach() for e in edge_index], 1).to(torch.int64)
+        device = edge_index[0].device  # where the others are taken to
+        ends = torch.cat([e.detach().to(device) for e in edge_index], 1).to(torch.int64)
         self.src, self.dst = ends[0].contiguous(), ends[1].contiguous()
         counts = [e.size(1) for e in edge_index]
-        device = self.src.device
         self.weight = torch.cat([torch.ones(n, device=device) if edge_weight is None or edge_weight[k] is None
-                                 else edge_weight[k].detach().to(device, torch.float32).reshape(-1)
+                                 else edge_weight[k].detach().to(device, torch.float32)
                                  for k, n in enumerate(counts)])
         self.phase = torch.repeat_interleave(torch.arange(self.phases, device=device),
                                              torch.tensor(counts, device=device), output_size=sum(counts))
@@ -63,7 +63,7 @@ class _Edges:
         """(vertices are sources of phase 0 only and rules of the others, and every rule is complete before it is
         a source; whether there are edges from rule to rule).  One host read."""
         V, R, late = self.V, self.R, self.phase > 0
-        if self.src.numel() == 0 or self.weight.numel() != self.src.numel():
+        if self.src.numel() == 0:
             return False, False
         from_rule, to_rule = self.src >= V, self.dst >= V
         in_range = ((self.src >= 0) & (self.dst >= 0) & (self.src < V + R) & (self.dst < V + R)).all()
@@ -79,14 +79,15 @@ class _Edges:
         chain, levels = torch.stack([in_range & ruled & ordered, (from_rule & to_rule).any()]).tolist()
         return chain, levels
 
-    def plan(self, levels):
+    def plan(self, levels, dtype=torch.float32):
+        """The chain as a PropagationPlan for features of `dtype` (levels, as is_chain() reports)."""
         V, R, device = self.V, self.R, self.src.device
         forward = _grouped(self.dst, V + R, self.src, self.weight)
         # the gradient of a vertex: from its vertex targets first, then from its rule targets
         order = torch.cat([torch.nonzero(self.dst < V).flatten(), torch.nonzero(self.dst >= V).flatten()])
         src, dst, weight = (t.index_select(0, order) for t in (self.src, self.dst, self.weight))
         backward = _grouped(src, V + R, dst, weight)
-        csr = _native.DeviceCsr
+        csr = lambda ptr, other, value, *rest: _native.DeviceCsr(ptr, other, value.to(dtype), *rest)
         cut = torch.stack([forward[0][V], backward[0][V]]).tolist()
 
         def vertex_rows(grouped, n):
@@ -141,12 +142,16 @@ class CooPhasePlan:
         self.in_place = []  # per phase: no node is both a source and a destination of the phase
         # keeps the tensors (and so their addresses) alive for as long as the plan is cached
         self.sources = (list(edge_index), None if edge_weight is None else list(edge_weight))
-        for edges in edge_index:
+        for k, edges in enumerate(edge_index):
             if edges.dim() != 2 or edges.size(0) != 2:
                 raise ValueError("every phase must be a [2, E] edge tensor")
+            if edge_weight is not None and edge_weight[k] is not None and edge_weight[k].shape != edges[0].shape:
+                raise ValueError("edge_weight[%d] must have one value per edge" % k)
         edges = _Edges(edge_index, edge_weight, self.V, self.R)
-        is_chain, levels = edges.is_chain()
-        self.chain = edges.plan(levels) if is_chain else None
+        is_chain, self._levels = edges.is_chain()
+        self.chain = edges.plan(self._levels) if is_chain else None
+        # weights are of 32 bits; without any the sums take features of either precision
+        self._wide_chain, self._weighted = None, edge_weight is not None and any(w is not None for w in edge_weight)
         if self.chain is not None:
             return
         t = torch.from_numpy
@@ -156,8 +161,6 @@ class CooPhasePlan:
             w = None
             if edge_weight is not None and edge_weight[k] is not None:
                 w = edge_weight[k].detach().cpu().numpy().astype(np.float32)
-                if w.shape != src.shape:
-                    raise ValueError("edge_weight[%d] must have one value per edge" % k)
             cols = self.V if k == 0 else total  # phase 0 gathers from x
             rows_back = cols
             if src.size and (src.min() < 0 or src.max() >= cols or dst.min() < 0 or dst.max() >= total):
@@ -177,12 +180,20 @@ class CooPhasePlan:
             self.backward_blocks.append(_native.DeviceCsr(t(sp), t(np.ascontiguousarray(s_col)), wt(s_val),
                                                           rows_back, total, device))
 
+    def chain_for(self, dtype):
+        """The chain for features of this type: an unweighted list holds a one of the type for every edge."""
+        if dtype != torch.float64 or self._weighted:
+            return self.chain
+        if self._wide_chain is None:
+            self._wide_chain = _Edges(self.sources[0], None, self.V, self.R).plan(self._levels, dtype)
+        return self._wide_chain
+
     def forward(self, x):
         x = x.contiguous()
         if x.dim() != 2 or x.size(0) != self.V:
             raise ValueError("x must be [vertex_cnt, F]")
         if self.chain is not None:
-            return self.chain.forward(x)
+            return self.chain_for(x.dtype).forward(x)
         out = self.forward_blocks[0].spmm(x)
         for block, in_place in zip(self.forward_blocks[1:], self.in_place[1:]):
             out = block.spmm(out, out) if in_place else out + block.spmm(out)
@@ -191,7 +202,7 @@ class CooPhasePlan:
     def backward(self, grad):
         grad = grad.contiguous()
         if self.chain is not None:
-            return self.chain.backward(grad)
+            return self.chain_for(grad.dtype).backward(grad)
         if len(self.backward_blocks) == 1:
             full = grad if self.R == 0 else torch.cat([grad, grad.new_zeros((self.R, grad.size(1)))])
             return self.backward_blocks[0].spmm(full)
@@ -217,7 +228,7 @@ def coo_propagate(plan, x):
     """plan.forward(x) with its gradient; a chain's step of autograd is native."""
     if plan.chain is None or x.dim() != 2 or x.size(0) != plan.V or _native.needs_function(x):
         return CooPropagateFunction.apply(plan, x)
-    return _native.propagate(plan.chain, x, once_differentiable=True)
+    return _native.propagate(plan.chain_for(x.dtype), x, once_differentiable=True)
 
 
 class CooPlanCache:

@@ -975,3 +975,50 @@ def test_steps_where_a_native_one_would_be_lost():
         dual = forward_mode.make_dual(x, y)
         with pytest.raises(NotImplementedError):
             rt.reconstruct(dual, torch.zeros(5, dtype=torch.int64, device=DEV), None, False)
+
+
+@pytest.mark.parametrize("kind", ["chain", "levels", "no_rules", "vertex_source_late"])
+def test_edge_lists_of_either_precision_and_from_several_devices(kind):
+    """Without weights the features may be float64, in lists that run as a chain and in others; with weights (32 bits)
+    they may not.  Edges and weights may lie elsewhere than the first phase; a weight per edge is asked for phase by phase."""
+    from CooPhases import CooPhasePlan, coo_propagate
+    rng = np.random.default_rng(8)
+    V, R, F = 300, 0 if kind == "no_rules" else 40, 11
+    vert = lambda n: rng.integers(0, V, n)
+    phases = [np.stack([vert(900), np.concatenate([vert(700), V + rng.integers(0, 10, 200) if R else vert(200)])])]
+    if kind == "levels":
+        phases += [np.stack([V + rng.integers(0, 10, 10), V + rng.integers(10, 20, 10)])]
+    if R:
+        phases += [np.stack([V + rng.integers(10 if kind == "levels" else 0, 20 if kind == "levels" else 10, 60), vert(60)])]
+    if kind == "vertex_source_late":
+        phases += [np.stack([vert(9), vert(9)])]
+    x, g = rng.standard_normal((V, F)), rng.standard_normal((V, F))
+    full, back, gx = np.zeros((V + R, F)), np.concatenate([g, np.zeros((R, F))]), np.zeros((V, F))
+    for k, (s, d) in enumerate(phases):
+        source = x if k == 0 else full.copy()
+        np.add.at(full, d, source[s])
+    for k in range(len(phases) - 1, -1, -1):
+        s, d = phases[k]
+        moved = back[d]
+        np.add.at(gx if k == 0 else back, s, moved)
+    edges = [torch.from_numpy(p).to(DEV if k == 0 else "cpu") for k, p in enumerate(phases)]
+    plan = CooPhasePlan(edges, None, V, R)
+    assert (plan.chain is not None) == (kind != "vertex_source_late")
+    for dtype, tol in ((torch.float64, 1e-12), (torch.float32, 1e-4), (torch.float64, 1e-12)):
+        X = torch.from_numpy(x).to(DEV, dtype).requires_grad_()
+        out = coo_propagate(plan, X)
+        (got,) = torch.autograd.grad(out, X, torch.from_numpy(g).to(DEV, dtype))
+        assert out.dtype == got.dtype == dtype
+        np.testing.assert_allclose(out.detach().cpu().numpy(), full[:V], rtol=tol, atol=tol * np.abs(full).max())
+        np.testing.assert_allclose(got.cpu().numpy(), gx, rtol=tol, atol=tol * np.abs(gx).max())
+    with pytest.raises(RuntimeError):
+        coo_propagate(plan, X.detach().half())
+    ones = [torch.ones(p.shape[1], dtype=torch.float64) for p in phases]
+    weighted = CooPhasePlan(edges, ones, V, R)
+    np.testing.assert_allclose(coo_propagate(weighted, X.detach().float()).cpu().numpy(), full[:V], rtol=1e-4,
+                               atol=1e-4 * np.abs(full).max())
+    with pytest.raises(RuntimeError):
+        coo_propagate(weighted, X.detach())
+    for wrong in ([ones[0][:, None]] + ones[1:], [ones[0][:-1]] + [torch.ones(len(w) + 1) for w in ones[1:]]):
+        with pytest.raises(ValueError):
+            CooPhasePlan(edges, wrong, V, R)
