@@ -101,7 +101,7 @@ def build_runtime():
     for p in ce.include_paths() + [sysconfig.get_paths()["include"], INCLUDE, "/opt/rocm/include"]:
         inc += ["-I", p]
     torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fopenmp", "-shared",
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fopenmp-simd", "-shared",
            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=compressgnn_runtime",
            "-DTORCH_API_INCLUDE_EXTENSION_H", "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
            "-Wno-deprecated-declarations", "-Wno-unused-result"] + inc + [

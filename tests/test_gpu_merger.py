@@ -144,3 +144,44 @@ def test_gpu_compressor_at_the_edges_of_its_tiles(entries, freq):
     got = both(v, e, 12, freq)
     assert got[3] > 0
     assert all(np.array_equal(a, b) for a, b in zip(got, both(v.astype(np.int32), e.astype(np.int32), 12, freq)))
+
+
+@pytest.mark.parametrize("entries", [(1 << 14) - 1, (1 << 14) + 1, (1 << 20) + (1 << 14), (9 << 19) + 3])
+def test_gpu_compressor_from_several_threads(entries):
+    """The host's passes are dealt out in blocks, to as many helpers as there are or to none: alone, with one thread
+    allowed, and in three calls at once the arrays are the same; a value out of range in the last block ends a call and
+    leaves the next one whole."""
+    import threading
+    import torch
+    import compressgnn_batch_cuda as gpu
+    rng = np.random.default_rng(entries)
+    V = 5000
+    pool = rng.integers(0, V, (entries // 64 + 1, 4))
+    e = pool[rng.integers(0, len(pool), entries // 4 + 1)].ravel()[:entries].astype(np.int64)
+    v = np.concatenate([[0], np.sort(rng.integers(0, entries + 1, V - 1)), [entries]]).astype(np.int64)
+    run = lambda: gpu.compress_csr_batch(v, e, rounds=3, min_pair_frequency=16)
+    same = lambda a, b: a[2:] == b[2:] and np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+    want = both(v, e, 3, 16) if entries < 1 << 21 else run()
+    assert want[3] > 0
+    threads = torch.get_num_threads()
+    try:
+        torch.set_num_threads(1)
+        assert same(run(), want)
+    finally:
+        torch.set_num_threads(threads)
+    got = [None] * 3
+
+    def call(k):
+        got[k] = run()
+
+    calls = [threading.Thread(target=call, args=(k,)) for k in range(3)]
+    for t in calls:
+        t.start()
+    for t in calls:
+        t.join()
+    assert all(g is not None and same(g, want) for g in got)
+    wrong = e.copy()
+    wrong[-1] = -1
+    with pytest.raises(ValueError):
+        gpu.compress_csr_batch(v, wrong, rounds=3, min_pair_frequency=16)
+    assert same(run(), want)
