@@ -164,7 +164,7 @@ struct DeviceCsr {
     int32_t max_row_nnz = 0;
     int32_t seg_nnz = 0;
     Tensor cut_rows, empty_rows;  // the rows the runs of the nnz schedule cut / the rows without entries
-    Tensor run_start;  // nnz schedule: where every run begins (made with rowidx)
+    Tensor run_start;  // plain runs of the nnz schedule: where every run begins
     std::shared_ptr<Scratch> scratch = std::make_shared<Scratch>();
     // Whether AUTO may take workgroup runs, which divide long rows at other places than the nnz schedule
     // of the C ABI does (a plan's blocks do; a block on its own keeps the sums of the C ABI unless asked).
@@ -175,7 +175,7 @@ struct DeviceCsr {
         Tensor table;
     };
     std::vector<WgRuns> wg_runs;
-    Tensor captured_runs;  // the table of the product recorded last, where it was not there before: the graph fills it
+    Tensor captured_rowidx, captured_runs;  // those of the product recorded last, where they were not there before
 
     cgnn_csr view() const {
         cgnn_csr a{};
@@ -218,47 +218,44 @@ struct DeviceCsr {
         empty_rows = pad(none.contiguous());
     }
 
-    // rowidx (the row of every non-zero, as large as colidx) is read by the nnz schedule only:
-    // it is made when a product first resolves to that schedule, on the product's stream.
-    // So is the table of run starts, which belongs to a run length as the row lists do.
-    void ensure_rowidx(int kernel) {
-        if (nnz == 0 || (rowidx.defined() && run_start.defined())) return;
-        if (cgnn_spmm_schedule(rows, nnz, max_row_nnz, kernel) != CGNN_SPMM_NNZ) return;
-        auto stream = reinterpret_cast<cgnn_stream_t>(
-            c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(rowptr.device().index()).stream());
-        if (!rowidx.defined()) {
-            rowidx = torch::empty({nnz}, rowptr.options());
-            ok(cgnn_csr_expand_rows(rows, nnz, rowptr.data_ptr<int32_t>(), rowidx.data_ptr<int32_t>(), stream),
-               "csr_expand_rows");
-        }
-        cgnn_csr a = view();
-        const int64_t K = cgnn_spmm_run_length(&a);
-        Tensor starts = torch::empty({(nnz + K - 1) / K + 1}, rowptr.options());
-        ok(cgnn_spmm_run_starts(&a, starts.data_ptr<int32_t>(), stream), "spmm_run_starts");
-        run_start = starts;
-    }
-
     // The block as a product of width F reads it, and the scratch for that product; the caller holds scratch->lock until
     // the product is launched.
+    // What the nnz schedule reads beside the block is made when a product first resolves to it, on the product's
+    // stream: rowidx (the row of every non-zero, as large as colidx), and the run starts of the plain runs or the table of
+    // the workgroup runs for a lane layout.  Recorded into a graph they are the graph's, which fills them with every replay:
+    // there is nothing in them before, so no eager product may find them.
     cgnn_csr prepare(int64_t F, int dtype, int kernel, void **ws, size_t *bytes) {
-        ensure_rowidx(kernel);
         cgnn_csr a = view();
-        if (workgroup_runs && kernel == CGNN_SPMM_AUTO && nnz > 0 && empty_rows.defined() &&
-            cgnn_spmm_schedule(rows, nnz, max_row_nnz, kernel) == CGNN_SPMM_NNZ) {
-            int64_t arrivals = 0;
-            ok(cgnn_spmm_wg_shape(&a, F, dtype, &a.wg_groups, &a.wg_len, &arrivals), "spmm_wg_shape");
-            auto found = std::find_if(wg_runs.begin(), wg_runs.end(), [&](const WgRuns &r) {
-                return r.groups == a.wg_groups && r.len == a.wg_len;
-            });
-            if (found == wg_runs.end()) {
-                Tensor table = torch::empty({(nnz + a.wg_len - 1) / a.wg_len * a.wg_groups + 1}, rowptr.options());
-                ok(cgnn_spmm_wg_runs(&a, a.wg_groups, a.wg_len, table.data_ptr<int32_t>(), current_stream(rowptr)),
-                   "spmm_wg_runs");
-                if (capturing(rowptr)) captured_runs = table;
-                else found = wg_runs.insert(wg_runs.end(), WgRuns{a.wg_groups, a.wg_len, table});
+        if (nnz > 0 && cgnn_spmm_schedule(rows, nnz, max_row_nnz, kernel) == CGNN_SPMM_NNZ) {
+            const auto stream = current_stream(rowptr);
+            const bool recorded = capturing(rowptr);
+            if (!rowidx.defined()) {
+                Tensor made = torch::empty({nnz}, rowptr.options());
+                ok(cgnn_csr_expand_rows(rows, nnz, rowptr.data_ptr<int32_t>(), made.data_ptr<int32_t>(), stream), "csr_expand_rows");
+                a.rowidx = made.data_ptr<int32_t>();
+                (recorded ? captured_rowidx : rowidx) = made;
             }
-            a.wg_runs = (found != wg_runs.end() ? found->table : captured_runs).data_ptr<int32_t>();
-            a.arrivals = scratch->counters(arrivals, rowptr);
+            if (workgroup_runs && kernel == CGNN_SPMM_AUTO && empty_rows.defined()) {
+                int64_t arrivals = 0;
+                ok(cgnn_spmm_wg_shape(&a, F, dtype, &a.wg_groups, &a.wg_len, &arrivals), "spmm_wg_shape");
+                auto found = std::find_if(wg_runs.begin(), wg_runs.end(), [&](const WgRuns &r) {
+                    return r.groups == a.wg_groups && r.len == a.wg_len;
+                });
+                if (found == wg_runs.end()) {
+                    Tensor table = torch::empty({(nnz + a.wg_len - 1) / a.wg_len * a.wg_groups + 1}, rowptr.options());
+                    ok(cgnn_spmm_wg_runs(&a, a.wg_groups, a.wg_len, table.data_ptr<int32_t>(), stream), "spmm_wg_runs");
+                    if (recorded) captured_runs = table;
+                    else found = wg_runs.insert(wg_runs.end(), WgRuns{a.wg_groups, a.wg_len, table});
+                }
+                a.wg_runs = (found != wg_runs.end() ? found->table : captured_runs).data_ptr<int32_t>();
+                a.arrivals = scratch->counters(arrivals, rowptr);
+            } else if (!run_start.defined()) {
+                const int64_t K = cgnn_spmm_run_length(&a);
+                Tensor starts = torch::empty({(nnz + K - 1) / K + 1}, rowptr.options());
+                ok(cgnn_spmm_run_starts(&a, starts.data_ptr<int32_t>(), stream), "spmm_run_starts");
+                a.run_start = starts.data_ptr<int32_t>();
+                (recorded ? captured_runs : run_start) = starts;
+            }
         }
         *bytes = cgnn_spmm_workspace_bytes(&a, F, dtype, kernel);
         *ws = *bytes ? scratch->get(*bytes, rowptr).data_ptr() : nullptr;

@@ -339,6 +339,35 @@ def test_eager_products_before_the_first_replay():
         assert torch.equal(plan.forward(wide), out_eager)
 
 
+def test_first_products_of_a_plan_under_capture():
+    """A plan whose first products are recorded: row numbers and run tables made on the way are the graph's too, so eager
+    products (AUTO and the plain runs) between the capture and its first replay make their own."""
+    data, _ = _make_data("copy", 64, True, 3, seed=4)
+    data.to(DEV)
+    plan = data.edge_index.plan()
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(11)
+    x = torch.randn(data.vertex_cnt, 40, device=DEV, generator=gen)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out_graph, gx_graph = plan.forward(x), plan.backward(x)
+        plan.method = "nnz_schedule"
+        plain_graph = plan.forward(x)
+        plan.method = "auto"
+    out_eager, gx_eager = plan.forward(x), plan.backward(x)
+    plan.method = "nnz_schedule"
+    plain_eager = plan.forward(x)
+    plan.method = "auto"
+    fresh = _make_data("copy", 64, True, 3, seed=4)[0].to(DEV)  # a plan that was never recorded
+    assert torch.equal(fresh.edge_index.plan().forward(x), out_eager)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out_graph, out_eager) and torch.equal(gx_graph, gx_eager) and torch.equal(plain_graph, plain_eager)
+        assert torch.equal(plan.forward(x), out_eager) and torch.equal(plan.backward(x), gx_eager)
+
+
 def test_spmm_func_int64_api():
     """The reference's raw operator on int64 CSR tensors, all accepted method strings."""
     import compressgnn_runtime as rt
