@@ -943,8 +943,11 @@ struct BoundedLayout {
     int64_t samples_cap;
 };
 
-// The most slots a call may have in all its layers: 512 MB of them.
-constexpr int64_t kMostSlots = int64_t(1) << 27;
+// The most slots a call may have in all its layers: 128 MB of them.  They are for the longest lists that the fan-outs
+// allow, and are written and ranked however short the lists are.  With lists of two entries over 2 million vertices,
+// the worst case, this form takes 132 us at 2^25 slots (16,384 seeds, fan-outs 64 and 32: 100,000 edges; layer by layer
+// 311 us), 204 at 2^26 (303) and 348 at 2^27 (346), but holds 160, 294 and 525 MB where the layers take 23, 23 and 30.
+constexpr int64_t kMostSlots = int64_t(1) << 25;
 
 // false: the fan-outs do not bound the call well enough, or it has too many layers
 bool bounded_layout(int64_t vertex_cnt, int64_t n_input, int layers, const int64_t *fanouts, BoundedLayout *L) {

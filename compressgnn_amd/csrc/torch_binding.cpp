@@ -1461,8 +1461,15 @@ std::tuple<Tensor, Tensor, Tensor> run_sampler(SampleGraph &G, const Tensor &inp
         TORCH_CHECK(code != CGNN_SAMPLE_TOO_MANY, op, ": a layer of more than 2^31 - 2 neighbours");
     };
     const int layers = (int)std::min<size_t>(num_neighbors.size(), INT_MAX);
-    if (const size_t bytes = cgnn_sample_layers_workspace_bytes(g.vertex_cnt, n_input, layers, num_neighbors.data())) {
-        Tensor ws = torch::empty({(int64_t)bytes}, u8);
+    const size_t bounded = cgnn_sample_layers_workspace_bytes(g.vertex_cnt, n_input, layers, num_neighbors.data());
+    Tensor slots;
+    try {
+        if (bounded > 0) slots = torch::empty({(int64_t)bounded}, u8);
+    } catch (const c10::OutOfMemoryError &) {  // room for the longest lists there could be: the layers take what they are
+    }
+    if (slots.defined()) {
+        const Tensor &ws = slots;
+        const size_t bytes = bounded;
         Tensor summary = torch::empty({4}, torch::TensorOptions().dtype(torch::kInt32).pinned_memory(true));
         ok(cgnn_sample_layers(&g, n_input, input.data_ptr<int64_t>(), layers, num_neighbors.data(), (uint64_t)seed,
                               summary.data_ptr<int32_t>(), ws.data_ptr(), bytes, stream),

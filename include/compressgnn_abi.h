@@ -467,7 +467,7 @@ int cgnn_sample_relabel(int64_t total, const int64_t *neighbors, int64_t base, i
  * if the full list of a vertex is not bounded by its degree, in which case the entries above have to be used, and, written
  * last, before the stream has come to its end, 1.  cgnn_sample_layers_write, with the same arguments and workspace,
  * writes samples[samples], and per edge the position of its vertex and of the neighbour among them.  Size
- * query: 0 if the fan-outs do not bound the call. */
+ * query: 0 if the fan-outs do not bound the call, or only to more than 2^25 neighbours in all layers. */
 #define CGNN_SAMPLE_MAX_BOUNDED 8
 size_t cgnn_sample_layers_workspace_bytes(int64_t vertex_cnt, int64_t n_input, int layers, const int64_t *fanouts);
 int cgnn_sample_layers(const cgnn_sample_graph *graph, int64_t n_input, const int64_t *input, int layers,

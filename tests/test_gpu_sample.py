@@ -270,3 +270,31 @@ def test_layers_of_many_chunks():
     got = sampler.neighbor_sample_ori_impl(t(b["v2v"][0]), t(b["v2v"][1]), t(inp), [64], seed=5)
     for a, w in zip(got, oracle.neighbor_sample(b, inp, [64], seed=5, plain=True)):
         assert np.array_equal(a.cpu().numpy(), w)
+
+
+@pytest.mark.parametrize("rows", [1 << 19, (1 << 19) + 1])
+def test_layers_at_the_limit_of_the_slots_and_without_room_for_them(rows):
+    """As many slots as a call with one host read may have, and one vertex more; and a call that finds no room for its
+    slots, which goes layer by layer as one without a bound does."""
+    import compressgnn_sample as sampler
+    rng = np.random.default_rng(33)
+    V = 6000
+    b = dict(v2v=(np.arange(V + 1, dtype=np.int64) * 2, rng.integers(0, V, 2 * V)))
+    t = lambda a: torch.from_numpy(a).to(DEV)
+    ptr, col = t(b["v2v"][0]), t(b["v2v"][1])
+
+    def check_call(inp, fan):
+        got = sampler.neighbor_sample_ori_impl(ptr, col, t(inp), fan, seed=5)
+        for a, w in zip(got, oracle.neighbor_sample(b, inp, fan, seed=5, plain=True)):
+            assert np.array_equal(a.cpu().numpy(), w)
+
+    check_call(rng.integers(0, V, rows), [64])
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    before = torch.cuda.memory_stats()["num_ooms"]
+    try:  # 90 MB beside what is held; the slots of this call would be 102 MB
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (90 << 20)) / total)
+        check_call(rng.integers(0, V, 400000), [64])
+        assert torch.cuda.memory_stats()["num_ooms"] == before + 1
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
