@@ -1750,6 +1750,8 @@ std::tuple<Tensor, Tensor, int64_t> compress_csr_batch(const Tensor &vlist, cons
     };
     std::vector<int64_t> entries;
     const std::vector<Part> there = chunks_of(V + 1, E, &entries);
+    // gone in the reverse order, also where an error ends the call: the helpers, the copies, what they copy
+    Tensor dev[2], out_ptr, out_col, ws, result[2];
     std::unique_ptr<Link> up, down;
     std::atomic<bool> fits{true};
     // the helpers are on their way while the rest is made ready
@@ -1765,9 +1767,9 @@ std::tuple<Tensor, Tensor, int64_t> compress_csr_batch(const Tensor &vlist, cons
     auto compute = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device.index()).stream();
     auto stream = reinterpret_cast<cgnn_stream_t>(compute);
     const size_t bytes = cgnn_compress_batch_workspace_bytes(V, E);
-    Tensor dev[2] = {torch::empty({V + 1}, i32), torch::empty({std::max<int64_t>(E, 1)}, i32)};
-    Tensor out_ptr = torch::empty({V + E / 2 + 2}, i32), out_col = torch::empty({std::max<int64_t>(E, 1)}, i32);
-    Tensor ws = torch::empty({(int64_t)std::max<size_t>(bytes, 1)}, i32.dtype(torch::kUInt8));
+    dev[0] = torch::empty({V + 1}, i32), dev[1] = torch::empty({std::max<int64_t>(E, 1)}, i32);
+    out_ptr = torch::empty({V + E / 2 + 2}, i32), out_col = torch::empty({std::max<int64_t>(E, 1)}, i32);
+    ws = torch::empty({(int64_t)std::max<size_t>(bytes, 1)}, i32.dtype(torch::kUInt8));
     up = std::make_unique<Link>(V + 1 + E + Link::kChunk, device.index(), compute);
     sender.open(std::min<int64_t>(there.size(), Link::kSlots));
     for (int64_t k = 0; k < (int64_t)there.size(); ++k) {
@@ -1789,7 +1791,6 @@ std::tuple<Tensor, Tensor, int64_t> compress_csr_batch(const Tensor &vlist, cons
     done(cgnn_compress_batch_rounds(V, E, passes, frequency, out_ptr.data_ptr<int32_t>(), out_col.data_ptr<int32_t>(), summary,
                                     pinned.data_ptr<int32_t>(), ws.data_ptr(), bytes, stream));
     const std::vector<Part> back = chunks_of(V + summary[0] + 1, summary[1], &entries);
-    Tensor result[2];
     const Tensor *from[2] = {&out_ptr, &out_col};
     Crew receiver(std::move(entries), [&](int64_t k, int64_t at, int64_t n) {
         std::memcpy(result[back[k].array].data_ptr<int32_t>() + back[k].at + at, down->slot(k) + at, n * sizeof(int32_t));
