@@ -868,9 +868,19 @@ Assigned assign(Tensor input, Tensor planes, int64_t bits, bool with_reps) {
     Tensor summary = direct ? torch::empty({2}, torch::TensorOptions().dtype(torch::kInt32).pinned_memory(true))
                             : torch::empty({2}, ints);
     auto stream = current_stream(input);
+    // The pool of pinned memory knows nothing of the launch that writes `summary`: an error before the host read (no
+    // room for the representatives) waits for it.
+    struct Settle {
+        hipStream_t stream;
+        bool pending = false;
+        ~Settle() {
+            if (pending) (void)hipStreamSynchronize(stream);
+        }
+    } settle{reinterpret_cast<hipStream_t>(stream)};
     ok(cgnn_lsh_hash(N, F, (int)bits, dtype_code(input), input.data_ptr(), planes.data_ptr(), raw, nullptr, stream), "lsh_hash");
     const size_t bytes = cgnn_lsh_group_workspace_bytes(N, (int)bits);
     Tensor ws = torch::empty({(int64_t)std::max<size_t>(bytes, 1)}, input.options().dtype(torch::kUInt8));
+    settle.pending = direct;
     ok(cgnn_lsh_group(N, (int)bits, raw, a.ids.data_ptr<int64_t>(), offsets.data_ptr<int32_t>(), perm.data_ptr<int32_t>(),
                       sorted_id.data_ptr<int32_t>(), counts.data_ptr<int32_t>(), summary.data_ptr<int32_t>(), ws.data_ptr(), bytes,
                       stream),
@@ -880,6 +890,7 @@ Assigned assign(Tensor input, Tensor planes, int64_t bits, bool with_reps) {
     if (early) a.reps = member_means("cluster_mean", input, nullptr, wide_lists, cap + 1, N);
     // the one host read of a refresh
     if (direct) {
+        settle.pending = false;
         TORCH_CHECK(hipStreamSynchronize(reinterpret_cast<hipStream_t>(stream)) == hipSuccess, op, ": the stream reported an error");
     } else {
         summary = summary.cpu();

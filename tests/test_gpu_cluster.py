@@ -410,3 +410,24 @@ def test_column_sums(rows, width, dtype):
     for _ in range(2):
         got = rt.column_sums(x).double()
         assert float((got - want).abs().max()) <= tol * max(1.0, float(x.double().abs().sum(0).max()))
+
+
+def test_a_refresh_without_room_for_its_representatives():
+    """The sums of a refresh are launched before the host reads how many clusters there are; where there is no room
+    for them the error is torch's own, and the next refresh is whole."""
+    from CompressgnnCluster import Compressgnn_Cluster
+    torch.manual_seed(3)
+    x = torch.randn(8000, 520, device=DEV)
+    cluster = Compressgnn_Cluster(520, 12, training=True, device=DEV, cache=False)
+    reps, index = (t.clone() for t in cluster(x))
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:  # 4,097 representatives are 8.5 MB, in a segment of 20; the rest of a refresh is in segments of 2
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (12 << 20)) / total)
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            cluster(x)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    again, ids = cluster(x)
+    assert torch.equal(again, reps) and torch.equal(ids, index)
