@@ -490,3 +490,30 @@ def test_workgroup_runs(F, accumulate):
         assert np.array_equal(got, product(X).cpu().numpy())
         if dtype == np.float32:
             assert np.array_equal(got[whole], sequential[whole])
+
+
+@pytest.mark.parametrize("F", [1, 3, 8, 16, 19, 33, 47, 64, 130, 256, 258, 600])
+@pytest.mark.parametrize("rows, longest", [(1, 64), (118, 5), (118, 64), (509, 33), (8192, 40)])
+def test_row_schedule_with_lanes_beside_the_width(rows, longest, F):
+    """Launches of few rows take lane groups as wide as their longest row; the layout does not show in the result: the bits
+    of the sequential sum, from one source and from two, fresh and accumulating."""
+    rng = np.random.default_rng(rows + longest + F)
+    cols, lens = 700, rng.integers(0, longest + 1, rows)
+    lens[0] = longest
+    vlist = np.concatenate([[0], np.cumsum(lens)])
+    elist = rng.integers(0, cols, int(vlist[-1]))
+    value = rng.standard_normal(len(elist)).astype(np.float32)
+    x = rng.standard_normal((cols, F)).astype(np.float32)
+    want = oracle.spmm(vlist, elist, value, x)
+    assert np.array_equal(_run(vlist, elist, value, x, abi.SPMM_ROW), want)
+    out0 = rng.standard_normal((rows, F)).astype(np.float32)
+    assert np.array_equal(_run(vlist, elist, value, x, abi.SPMM_ROW, out0), oracle.spmm(vlist, elist, value, x, out0.copy()))
+    # rows of two sources hold the entries of the first in front
+    split, row_of = 600, np.repeat(np.arange(rows), lens)
+    order = np.lexsort((elist >= split, row_of))
+    e2, v2 = elist[order], value[order]
+    pick = lambda keep, shift: (np.concatenate([[0], np.cumsum(np.bincount(row_of[order][keep], minlength=rows))]), e2[keep] - shift, v2[keep])
+    want2 = oracle.spmm(*pick(e2 < split, 0), x[:split], oracle.spmm(*pick(e2 >= split, split), x[split:]))
+    A, X = abi.DeviceCsr.from_host(rows, cols, vlist, e2, v2, DEV), torch.from_numpy(x).to(DEV)
+    got = abi.spmm_dual(A, split, X[:split].contiguous(), X[split:].contiguous(), None, abi.SPMM_ROW).cpu().numpy()
+    assert np.array_equal(got, want2)
