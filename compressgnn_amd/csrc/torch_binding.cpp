@@ -682,15 +682,10 @@ Tensor propagate_backward(PropagationPlan &p, Tensor grad) {
 // Where a native step of autograd does not do what an autograd function of Python does: under torch.jit.trace, which
 // records a function as an operation on its inputs but the result of a native call as a constant; for inputs with a
 // forward-mode tangent and under the transforms of torch.func, which a function without the rules for them refuses.
-// The layers ask and take their function there; the steps themselves refuse.
-bool needs_function(const Tensor &a, const c10::optional<Tensor> &b) {
+// There a native step does nothing and returns None, and the layer calls its function.
+bool needs_function(const Tensor &a, const c10::optional<Tensor> &b = c10::nullopt) {
     return torch::jit::tracer::isTracing() || a._fw_grad(0).defined() || (b.has_value() && b->defined() && b->_fw_grad(0).defined()) ||
            c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
-}
-
-void require_plain(const char *op, const Tensor &a, const c10::optional<Tensor> &b = c10::nullopt) {
-    TORCH_CHECK_NOT_IMPLEMENTED(!needs_function(a, b), op, ": a native step has no forward-mode gradient and is not recorded by "
-                                "torch.jit.trace or torch.func; the layers' autograd functions are for those");
 }
 
 // A gradient asked for with create_graph, of a step that has first-order gradients only: it cannot be differentiated
@@ -724,8 +719,8 @@ struct PropagateBackward : torch::autograd::Node {
     std::string name() const override { return "PropagateBackward"; }
 };
 
-Tensor propagate(const std::shared_ptr<PropagationPlan> &plan, const Tensor &x, bool once_differentiable) {
-    require_plain("propagate", x);
+c10::optional<Tensor> propagate(const std::shared_ptr<PropagationPlan> &plan, const Tensor &x, bool once_differentiable) {
+    if (needs_function(x)) return c10::nullopt;
     const bool differentiable = at::GradMode::is_enabled() && x.requires_grad();
     Tensor out;
     {
@@ -1288,9 +1283,9 @@ void attach_mean(Tensor &reps, const Tensor &x, const Tensor &index, const Tenso
 
 // Representatives of an assignment that is held: the means of x over its clusters (the counts are the
 // lengths of its lists).
-Tensor cluster_representatives(Tensor x, Tensor index, Tensor counts, std::vector<Tensor> members) {
+c10::optional<Tensor> cluster_representatives(Tensor x, Tensor index, Tensor counts, std::vector<Tensor> members) {
     const char *op = "cluster_mean";
-    require_plain(op, x);
+    if (needs_function(x)) return c10::nullopt;
     Tensor reps;
     {
         at::AutoDispatchBelowADInplaceOrView plain;
@@ -1307,15 +1302,16 @@ Tensor cluster_representatives(Tensor x, Tensor index, Tensor counts, std::vecto
 }
 
 // A refresh: (representatives, ids, counts, active, member lists).
-std::tuple<Tensor, Tensor, Tensor, int64_t, std::vector<Tensor>> cluster_refresh(Tensor x, Tensor planes, int64_t bits) {
-    require_plain("cluster_refresh", x);
+c10::optional<std::tuple<Tensor, Tensor, Tensor, int64_t, std::vector<Tensor>>> cluster_refresh(Tensor x, Tensor planes,
+                                                                                              int64_t bits) {
+    if (needs_function(x)) return c10::nullopt;
     Assigned a;
     {
         at::AutoDispatchBelowADInplaceOrView plain;
         a = assign(x.contiguous(), planes.contiguous(), bits, true);
     }
     attach_mean(a.reps, x, a.ids, a.counts, a.members);
-    return {a.reps, a.ids, a.counts, a.active, a.members};
+    return std::make_tuple(a.reps, a.ids, a.counts, a.active, a.members);
 }
 
 // Column sums of a [rows, F] matrix: the gradient of a bias.
@@ -1367,8 +1363,8 @@ struct ReconstructBackward : torch::autograd::Node {
 // rows[i] = act(reps[index[i]] + bias) with its gradients.  The ReLU mask of the gradient is kept as one bit
 // per element, written by the kernel that produces the rows (the reference keeps the rows themselves:
 // layer/CompressgnnReconstruct.py:16-22); without a ReLU nothing of the [N, F] output is needed again.
-Tensor reconstruct(Tensor reps, Tensor index, c10::optional<Tensor> bias, bool relu, Members members) {
-    require_plain("reconstruct", reps, bias);
+c10::optional<Tensor> reconstruct(Tensor reps, Tensor index, c10::optional<Tensor> bias, bool relu, Members members) {
+    if (needs_function(reps, bias)) return c10::nullopt;
     Tensor rows, signs, ids;
     {
         at::AutoDispatchBelowADInplaceOrView plain;
@@ -1863,6 +1859,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("signs"), py::arg("groups"), py::arg("members") = py::none());
     m.def("csr_transpose", &csr_transpose, "CSR -> CSC of an int64 block on the GPU, SparseTensor.csc() order",
           py::arg("rowptr"), py::arg("col"), py::arg("value"), py::arg("cols"));
+    // the native steps of the layers: None under torch.jit.trace, for inputs with a tangent and under torch.func
     m.def("cluster_refresh", &cluster_refresh,
           "(representatives, ids, counts, active, [offsets, perm, sorted_id]) of an assignment refresh, with the gradient of "
           "the representatives", py::arg("x"), py::arg("planes"), py::arg("bits"));
@@ -1873,8 +1870,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("column_sums", &column_sums, "sum over the rows of a matrix");
     m.def("propagate", &propagate, "plan.forward(x) with plan.backward as its gradient", py::arg("plan"), py::arg("x"),
           py::arg("once_differentiable") = false);
-    m.def("needs_function", &needs_function, "whether a step on these inputs has to be an autograd function: the native steps "
-          "(propagate, cluster_refresh, cluster_representatives, reconstruct) refuse them", py::arg("a"), py::arg("b") = py::none());
     m.def("version", []() { return std::string(cgnn_version()); });
     py::class_<DeviceCsr, std::shared_ptr<DeviceCsr>>(m, "DeviceCsr")
         .def(py::init([](Tensor rowptr, Tensor col, c10::optional<Tensor> value, int64_t rows, int64_t cols,

@@ -7,7 +7,7 @@ import _paths  # noqa: F401
 import torch
 from torch import Tensor
 
-from compressgnn_runtime import needs_function, propagate, spmm_func
+from compressgnn_runtime import propagate, spmm_func
 from compress_graph import CompressGraph
 
 
@@ -56,6 +56,6 @@ class Compressgnn_SPMM(torch.nn.Module):
     def forward(self, edge_index: CompressGraph, x_j: Tensor) -> Tensor:
         # the same step as Compressgnn_SPMM_Function, with its gradient in the operator module
         _check(edge_index, x_j)
-        if needs_function(x_j):  # a trace records the function; forward mode and torch.func are refused by it
-            return Compressgnn_SPMM_Function.apply(edge_index, x_j)
-        return propagate(edge_index.plan(), x_j)
+        out = propagate(edge_index.plan(), x_j)
+        # None: a trace records the function; tangents and torch.func are refused by it
+        return Compressgnn_SPMM_Function.apply(edge_index, x_j) if out is None else out

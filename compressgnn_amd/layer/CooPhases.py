@@ -226,9 +226,10 @@ class CooPropagateFunction(torch.autograd.Function):
 
 def coo_propagate(plan, x):
     """plan.forward(x) with its gradient; a chain's step of autograd is native."""
-    if plan.chain is None or x.dim() != 2 or x.size(0) != plan.V or _native.needs_function(x):
+    if plan.chain is None or x.dim() != 2 or x.size(0) != plan.V:
         return CooPropagateFunction.apply(plan, x)
-    return _native.propagate(plan.chain_for(x.dtype), x, once_differentiable=True)
+    out = _native.propagate(plan.chain_for(x.dtype), x, once_differentiable=True)
+    return CooPropagateFunction.apply(plan, x) if out is None else out
 
 
 class CooPlanCache:
