@@ -1482,15 +1482,28 @@ size_t wg_piece_bytes(int64_t workgroups, int64_t F, size_t elt) { return 2 * (s
 // Non-zeros per lane group of the workgroup runs: as short as fills the card (lane groups resident at
 // once: 7 workgroups per compute unit), since a run is a chain of dependent rounds of gathers and a small
 // product is nothing but the time of its longest chain; not under 8 (two rounds: below that the ends of a
-// run cost more than its entries), not over the block's run length.
+// run cost more than its entries); where they would be longer than `most`, the block's run length, of which several fill
+// the card one after the other.
 constexpr int64_t kResidentWorkgroups = 256 * 7;
 
-int wg_run_len(const cgnn_csr *A, int groups) {
+int wg_run_len(const cgnn_csr *A, int groups, int most) {
     const int64_t fill = ceil_div(ceil_div(A->nnz, kResidentWorkgroups * groups), kUnroll) * kUnroll;
     const int longest = seg_len(A);
     if (fill < 8) return longest < 8 ? longest : 8;
-    return (int)(fill <= 2 * longest ? fill : longest);
+    return (int)(fill <= most ? fill : longest);
 }
+
+// Blocks of a plan: the run length, where two rounds of runs end more evenly than one of longer runs (forward vertex stage
+// of web graphs, runs of 52 to 64 entries against 32: 80 -> 71 us for 100,000 vertices of 128 features, 89 -> 78 for 200,000
+// of 64, 96 -> 87 for 200,000 of 47; of 36 to 44: 53 -> 51, 57 -> 56 and 61 -> 59 us for 47 features); rows of less than a
+// cache line, whose runs are quicker, take runs a little longer (16 features, 40 and 44 entries: 28 and 31 us against 31
+// and 33 of 32; 48: 39 against 34).
+int most_per_run(const cgnn_csr *A, int64_t row_bytes) { return row_bytes < 128 ? seg_len(A) * 11 / 8 : seg_len(A); }
+
+// Blocks that are new with every call: up to twice the run length.  Out-lists, near-regular rows in their natural order,
+// gain from it (runs of 36 to 44 entries against 32: 42 against 50 us for 100,003 rows of 64 features), in-lists lose less
+// (44 to 56 entries: 69 against 67 us for 120,000 rows, 89 against 83 for 160,000), and which a block is nobody has looked.
+int most_per_new_run(const cgnn_csr *A) { return 2 * seg_len(A); }
 
 // The layout of the row schedule.  A lane group takes its entries as many at a time as it has lanes, each time behind a
 // load of their columns, and a launch that leaves the card idle takes as long as its longest row: there, lanes beside
@@ -1838,7 +1851,7 @@ int spmm_member_runs(const cgnn_csr *A, int dtype, const void *X, const void *M,
     auto run = [&](auto zero) {
         typedef decltype(zero) T;
         const Shape s = pick_shape<T>(F, true);
-        const int groups = kBlock / s.lpr, wg_len = wg_run_len(A, groups) * groups;
+        const int groups = kBlock / s.lpr, wg_len = wg_run_len(A, groups, most_per_new_run(A)) * groups;
         const int64_t workgroups = ceil_div(A->nnz, wg_len);
         if (ws == nullptr || ws_bytes < wg_piece_bytes(workgroups, F, sizeof(T)))
             return fail(CGNN_EWORKSPACE, "member sums: workspace too small");
@@ -1868,7 +1881,7 @@ size_t spmm_member_runs_bytes(const cgnn_csr *A, int64_t F, int dtype, int64_t *
     const int groups = kBlock / s.lpr;
     *arrivals = 0;
     if (A->nnz > kResidentWorkgroups * groups * kDefaultSeg) return 0;
-    const int64_t workgroups = ceil_div(A->nnz, wg_run_len(A, groups) * groups);
+    const int64_t workgroups = ceil_div(A->nnz, wg_run_len(A, groups, most_per_new_run(A)) * groups);
     *arrivals = workgroups * s.grid_y;
     return wg_piece_bytes(workgroups, F, dtype == CGNN_F64 ? 8 : 4);
 }
@@ -1940,7 +1953,7 @@ OnceLayout once_layout(int64_t rows, int64_t nnz, int64_t F, int dtype) {
     A.seg_nnz = 32;  // as for the blocks of a plan
     OnceLayout L;
     L.groups = kBlock / shape_of(F, dtype).lpr;
-    L.wg_len = wg_run_len(&A, L.groups) * L.groups;
+    L.wg_len = wg_run_len(&A, L.groups, most_per_new_run(&A)) * L.groups;
     L.workgroups = ceil_div(nnz, L.wg_len);
     L.span = 0;
     L.rowptr = 256;
@@ -2009,7 +2022,7 @@ extern "C" int cgnn_spmm_wg_shape(const cgnn_csr *A, int64_t F, int dtype, int32
     CGNN_REQUIRE(groups && wg_len && arrivals && F >= 1, "cgnn_spmm_wg_shape: bad argument");
     const Shape s = shape_of(F, dtype);
     *groups = kBlock / s.lpr;
-    *wg_len = wg_run_len(A, *groups) * *groups;
+    *wg_len = wg_run_len(A, *groups, most_per_run(A, F * (dtype == CGNN_F64 ? 8 : 4))) * *groups;
     *arrivals = ceil_div(A->nnz, *wg_len) * s.grid_y;
     return CGNN_OK;
 }

@@ -517,3 +517,29 @@ def test_row_schedule_with_lanes_beside_the_width(rows, longest, F):
     A, X = abi.DeviceCsr.from_host(rows, cols, vlist, e2, v2, DEV), torch.from_numpy(x).to(DEV)
     got = abi.spmm_dual(A, split, X[:split].contiguous(), X[split:].contiguous(), None, abi.SPMM_ROW).cpu().numpy()
     assert np.array_equal(got, want2)
+
+
+@pytest.mark.parametrize("F", [16, 47, 128])
+@pytest.mark.parametrize("share", [31, 32, 33, 44, 45, 65])
+def test_workgroup_runs_where_the_card_is_filled_once(share, F):
+    """Blocks of as many entries as give every resident lane group a run about as long as the block's run length, and of one
+    entry more: runs of that length or two rounds of them, rows over several runs, against float64."""
+    import scipy.sparse as sp
+    import compressgnn_runtime as rt
+    rng = np.random.default_rng(share + F)
+    cols, rows = 5000, 40000
+    lane_groups = 256 * 7 * (16 if F <= 64 else 8)
+    for nnz in (lane_groups * share, lane_groups * share + 1):
+        cuts = np.sort((nnz * rng.random(rows - 1) ** 3).astype(np.int64))
+        vlist = np.concatenate([[0], cuts, [nnz]])
+        elist = rng.integers(0, cols, nnz)
+        lens = np.diff(vlist)
+        value = (rng.standard_normal(nnz) * 0.3 / np.sqrt(np.repeat(np.maximum(lens, 1), lens))).astype(np.float32)
+        x = rng.standard_normal((cols, F)).astype(np.float32)
+        t = lambda a: torch.from_numpy(a).to(DEV)
+        A = rt.DeviceCsr(t(vlist), t(elist), t(value), rows, cols, torch.device(DEV), 32)
+        A.workgroup_runs = True
+        want = sp.csr_matrix((value.astype(np.float64), elist, vlist), (rows, cols)) @ x.astype(np.float64)
+        got = A.spmm(t(x)).cpu().numpy()
+        np.testing.assert_allclose(got, want, rtol=2e-5, atol=2e-5)
+        assert np.array_equal(got, A.spmm(t(x)).cpu().numpy())
