@@ -1505,21 +1505,25 @@ int most_per_run(const cgnn_csr *A, int64_t row_bytes) { return row_bytes < 128 
 // (44 to 56 entries: 69 against 67 us for 120,000 rows, 89 against 83 for 160,000), and which a block is nobody has looked.
 int most_per_new_run(const cgnn_csr *A) { return 2 * seg_len(A); }
 
-// The layout of the row schedule.  A lane group takes its entries as many at a time as it has lanes, each time behind a
-// load of their columns, and a launch that leaves the card idle takes as long as its longest row: there, lanes beside
-// the width cost nothing and shorten that chain.  So lanes are added as long as a row is longer than a group and the
-// launch stays within kFewLanes, a quarter of what the card holds at once.  (118 rules of up to 64 vertices, 19 features:
-// 27.5 us with 8 lanes a row, 20 with 64; one forward propagation over their graph of 3,774 vertices 37.8 -> 31.3, of 16
-// features 36.9 -> 30.0, of 128 33.7 -> 30.8; over 2,708 vertices and one rule 15.0 -> 14.6.)
-constexpr int64_t kFewLanes = int64_t(1) << 17;
+// The layout of the row schedule.  Wide packs are for launches that fill the card several times over, where a row's
+// share of the memory instructions counts.  A launch that all of it fits the card at once takes as long as its longest
+// row, and that chain is shorter with more lanes: a lane group takes its entries as many at a time as it has lanes, each
+// time behind a load of their columns, and a lane adds up as many features of every entry as its packs have.  There a
+// row has the narrowest packs that a wave holds and as many lanes as the longest row has entries.  (118 rules of up to
+// 64 vertices, 19 features: 27.5 us with packs of four on 8 lanes, 20 with 64 lanes, 17 with one feature a lane on 64;
+// forward propagations over web graphs, 6,000 vertices: 8 features 36 -> 31 us, 19 38 -> 32, 47 38 -> 33, 128 38 -> 34, the
+// backward vertex stage 10.3 -> 9.2; with twice the lanes the same stage of 14,000 vertices took 10.8 us instead of 9.0.)
+constexpr int64_t kResidentLanes = 256 * 32 * kWave;
 
 template <typename T>
 Shape row_shape(int64_t F, int64_t rows, int32_t max_row_nnz) {
-    Shape s = pick_shape<T>(F, false);
-    if (sizeof(T) != 4 || s.tiles != 1 || s.grid_y != 1) return s;
-    const int factor = s.vec == 4 ? 2 : 4;  // the layouts there are
-    while (s.lpr < kWave && s.lpr < max_row_nnz && rows * s.lpr * factor <= kFewLanes) s.lpr *= factor;
-    return s;
+    const Shape wide = pick_shape<T>(F, false);
+    if (sizeof(T) != 4 || wide.tiles != 1 || wide.grid_y != 1) return wide;
+    Shape s = wide;
+    s.vec = F <= kWave ? 1 : (F <= 2 * kWave ? 2 : 4);
+    s.lpr = s.vec == 4 ? kWave : (F <= 4 * s.vec ? 4 : (F <= 16 * s.vec ? 16 : kWave));  // the layouts there are
+    while (s.lpr < kWave && s.lpr < max_row_nnz) s.lpr *= 4;
+    return rows * s.lpr <= kResidentLanes ? s : wide;
 }
 
 // mean (may be NULL; MODE_UNIT): whether the rows are wanted divided by their numbers of entries; false on return

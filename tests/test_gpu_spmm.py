@@ -492,11 +492,12 @@ def test_workgroup_runs(F, accumulate):
             assert np.array_equal(got[whole], sequential[whole])
 
 
-@pytest.mark.parametrize("F", [1, 3, 8, 16, 19, 33, 47, 64, 130, 256, 258, 600])
-@pytest.mark.parametrize("rows, longest", [(1, 64), (118, 5), (118, 64), (509, 33), (8192, 40)])
-def test_row_schedule_with_lanes_beside_the_width(rows, longest, F):
-    """Launches of few rows take lane groups as wide as their longest row; the layout does not show in the result: the bits
-    of the sequential sum, from one source and from two, fresh and accumulating."""
+@pytest.mark.parametrize("F", [1, 3, 4, 5, 16, 17, 19, 47, 64, 65, 100, 128, 129, 256, 258, 600])
+@pytest.mark.parametrize("rows, longest", [(1, 64), (118, 5), (118, 64), (8192, 40), (8193, 40)])
+def test_row_schedule_in_every_layout(rows, longest, F):
+    """Launches that fit the card at once take narrow packs and lane groups as wide as their longest row, others wide
+    packs; the layout does not show in the result: the bits of the sequential sum, from one source and from two, fresh
+    and accumulating."""
     rng = np.random.default_rng(rows + longest + F)
     cols, lens = 700, rng.integers(0, longest + 1, rows)
     lens[0] = longest
