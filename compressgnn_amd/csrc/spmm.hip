@@ -1834,6 +1834,66 @@ __global__ void compose_columns_kernel(const int32_t *__restrict__ col, int64_t 
     }
 }
 
+// A block with the columns from split on multiplied out (cgnn_csr_expand_columns), a wave per row: made once for a
+// plan, so what counts is that a hub's entries are taken 64 at a time.
+__global__ __launch_bounds__(kBlock) void expand_count_kernel(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col,
+                                                              int32_t rows, int32_t split, const int32_t *__restrict__ rule_ptr,
+                                                              int32_t *__restrict__ counts) {
+    const int64_t row = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
+    if (row >= rows) return;
+    const int lane = threadIdx.x % kWave;
+    const int32_t e1 = rowptr[row + 1];
+    int64_t n = 0;
+    for (int64_t e = rowptr[row] + lane; e < e1; e += kWave) {
+        const int32_t c = col[e];
+        n += c < split ? 1 : rule_ptr[c - split + 1] - rule_ptr[c - split];
+    }
+#pragma unroll
+    for (int s = kWave / 2; s > 0; s >>= 1) n += __shfl_xor(n, s, kWave);
+    if (lane == 0) counts[row] = (int32_t)min(n, (int64_t)INT32_MAX);
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) void expand_columns_kernel(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col,
+                                                                const T *__restrict__ val, int32_t rows, int32_t split,
+                                                                const int32_t *__restrict__ rule_ptr,
+                                                                const int32_t *__restrict__ rule_col, const T *__restrict__ rule_val,
+                                                                const int32_t *__restrict__ out_ptr, int32_t *__restrict__ out_col,
+                                                                T *__restrict__ out_val) {
+    const int64_t row = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
+    if (row >= rows) return;
+    const int lane = threadIdx.x % kWave;
+    const int32_t e0 = rowptr[row], e1 = rowptr[row + 1];
+    int32_t out = out_ptr[row];
+    for (int64_t base = e0; base < e1; base += kWave) {
+        const int64_t e = base + lane;
+        int32_t c = 0, from = 0, n = 0;
+        T w = T(0);
+        if (e < e1) {
+            c = col[e];
+            w = val[e];
+            if (c >= split) from = rule_ptr[c - split];
+            n = c < split ? 1 : rule_ptr[c - split + 1] - from;
+        }
+        int32_t upto = n;
+#pragma unroll
+        for (int s = 1; s < kWave; s <<= 1) {
+            const int32_t below = __shfl_up(upto, s, kWave);
+            if (lane >= s) upto += below;
+        }
+        const int32_t at = out + upto - n;
+        if (c < split) {
+            if (n > 0) out_col[at] = c, out_val[at] = w;
+        } else {
+            for (int32_t k = 0; k < n; ++k) {
+                out_col[at + k] = rule_col[from + k];
+                out_val[at + k] = rule_val != nullptr ? w * rule_val[from + k] : w;
+            }
+        }
+        out += __shfl(upto, kWave - 1, kWave);
+    }
+}
+
 }  // namespace
 
 // Entry used by the cluster reductions (mean: as for spmm_typed; unit values; mask: 0 none, 1 the rows of M, where M <= 0 drops
@@ -2178,6 +2238,48 @@ extern "C" int cgnn_spmm_run_starts(const cgnn_csr *A, int32_t *run_start, cgnn_
     hipLaunchKernelGGL(run_starts_kernel, dim3((unsigned)ceil_div(n, kBlock)), dim3(kBlock), 0, stream, A->rowptr,
                        A->rowidx, (int32_t)A->nnz, seg, n, run_start);
     return check_launch("spmm_run_starts");
+}
+
+namespace {
+
+int check_expand(const cgnn_csr *A, int64_t split, const cgnn_csr *rules) {
+    int rc = check_csr(A, "cgnn_csr_expand");
+    if (rc == CGNN_OK) rc = check_csr(rules, "cgnn_csr_expand");
+    if (rc != CGNN_OK) return rc;
+    CGNN_REQUIRE(split >= 0 && split <= A->cols && A->cols - split <= rules->rows,
+                 "cgnn_csr_expand: every column from split on has to be a row of the rules");
+    return CGNN_OK;
+}
+
+}  // namespace
+
+extern "C" int cgnn_csr_expand_count(const cgnn_csr *A, int64_t split, const cgnn_csr *rules, int32_t *counts,
+                                     cgnn_stream_t stream) {
+    int rc = check_expand(A, split, rules);
+    if (rc != CGNN_OK) return rc;
+    if (A->rows == 0) return CGNN_OK;
+    CGNN_REQUIRE(counts != nullptr, "cgnn_csr_expand_count: counts is null");
+    hipLaunchKernelGGL(expand_count_kernel, dim3((unsigned)ceil_div(A->rows, kBlock / kWave)), dim3(kBlock), 0, stream,
+                       A->rowptr, A->colidx, (int32_t)A->rows, (int32_t)split, rules->rowptr, counts);
+    return check_launch("csr_expand_count");
+}
+
+extern "C" int cgnn_csr_expand_columns(const cgnn_csr *A, int64_t split, const cgnn_csr *rules, int dtype, const int32_t *rowptr,
+                                       int32_t *colidx, void *val, cgnn_stream_t stream) {
+    int rc = check_expand(A, split, rules);
+    if (rc != CGNN_OK) return rc;
+    CGNN_REQUIRE(dtype == CGNN_F32 || dtype == CGNN_F64, "cgnn_csr_expand_columns: dtype must be f32 or f64");
+    if (A->rows == 0 || A->nnz == 0) return CGNN_OK;
+    CGNN_REQUIRE(A->val && rowptr && colidx && val, "cgnn_csr_expand_columns: null array");
+    auto run = [&](auto zero) {
+        typedef decltype(zero) T;
+        hipLaunchKernelGGL(expand_columns_kernel<T>, dim3((unsigned)ceil_div(A->rows, kBlock / kWave)), dim3(kBlock), 0, stream,
+                           A->rowptr, A->colidx, static_cast<const T *>(A->val), (int32_t)A->rows, (int32_t)split, rules->rowptr,
+                           rules->colidx, static_cast<const T *>(rules->val), rowptr, colidx, static_cast<T *>(val));
+    };
+    if (dtype == CGNN_F32) run(0.0f);
+    else run(0.0);
+    return check_launch("csr_expand_columns");
 }
 
 extern "C" int cgnn_csr_expand_rows(int64_t rows, int64_t nnz, const int32_t *rowptr, int32_t *rowidx,

@@ -500,6 +500,9 @@ struct PropagationPlan {
     std::vector<std::shared_ptr<DeviceCsr>> r2r, r2r_t;
     // [v2v | v2r] and [v2v^T | r2v^T]: the vertex stage of forward / backward in one pass
     std::shared_ptr<DeviceCsr> vertex_stage, vertex_stage_t;
+    // The vertex stages with the rules multiplied out ([vertex_cnt, vertex_cnt], the same stored rows): a propagation
+    // in one launch where the compressed form does not save what its second launch costs (takes_whole).  NULL: never.
+    std::shared_ptr<DeviceCsr> whole, whole_t;
     // the four blocks of the vertex stages on their own: only for the two-launch form
     // (fuse_final = false); a plan without them holds the graph once
     std::shared_ptr<DeviceCsr> v2v, v2r, v2v_t, r2v_t;
@@ -516,7 +519,7 @@ struct PropagationPlan {
         c10::weak_intrusive_ptr<c10::TensorImpl> index;
         uint32_t version;
         int64_t groups;
-        std::shared_ptr<DeviceCsr> rules, stage;
+        std::shared_ptr<DeviceCsr> rules, stage, whole;
     };
     std::deque<Composed> composed;
 
@@ -532,6 +535,58 @@ struct PropagationPlan {
                     "r2v_t blocks (graph.keep_split_blocks = True before graph.plan())");
     }
 };
+
+// A propagation with the rules multiplied out.  The rule stage is a launch that the vertex stage waits for: 3 to 12 us
+// however few entries it holds, 20 where the few rules of a small graph have long rows.  Multiplied out, the vertex stage
+// is a launch alone and gathers what the rules had saved it; on web graphs of 20,000 to 325,557 vertices both
+// forms take the same time where that is 45 to 60 MB more than the two stages move, and 75 to 90 MB in the row schedule,
+// whose stored neighbours share most of what they gather (forward + gradient, us, two stages against one: 64 features over
+// 2,708 vertices 25 / 16, 10,000 41 / 14, 50,001 49 / 37, 100,003 81 / 69, 200,000 of degree 5 100 / 89; beyond the line
+// 128 features over 325,557 vertices 365 / 388).
+constexpr int64_t kRuleStageBytes = int64_t(48) << 20, kRuleStageBytesRowSchedule = int64_t(72) << 20;
+
+// No more entries than this are kept beside the stages: beyond, a propagation takes so long that a launch is nothing to
+// it, and the device would hold a large graph twice.
+constexpr int64_t kMaxWholeEntries = int64_t(1) << 22;
+
+// Whether a product whose rows take row_bytes is as fast with the `entries` of the multiplied-out stage.
+bool takes_whole(int64_t entries, const DeviceCsr &stage, const DeviceCsr &rules, int64_t row_bytes) {
+    const int64_t index_bytes = 12;  // column, value, row
+    const int64_t more = (entries - stage.nnz - rules.nnz) * (row_bytes + index_bytes) - 2 * rules.rows * row_bytes;
+    const bool row_schedule = cgnn_spmm_schedule(stage.rows, stage.nnz, stage.max_row_nnz, CGNN_SPMM_AUTO) == CGNN_SPMM_ROW;
+    return more <= (row_schedule ? kRuleStageBytesRowSchedule : kRuleStageBytes);
+}
+
+// [vertices | rules] with the rules multiplied out, or NULL where no product would take it.
+std::shared_ptr<DeviceCsr> multiplied_out(const DeviceCsr &stage, const DeviceCsr &rules, int64_t V) {
+    if (stage.rows == 0 || stage.nnz == 0 || rules.nnz == 0 || !stage.val.defined() || stage.nnz > kMaxWholeEntries ||
+        (rules.val.defined() && rules.val.scalar_type() != stage.val.scalar_type()) || capturing(stage.rowptr))
+        return nullptr;
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(stage.rowptr.device());
+    const auto stream = current_stream(stage.rowptr);
+    const cgnn_csr a = stage.view(), r = rules.view();
+    Tensor counts = torch::empty({stage.rows}, stage.rowptr.options()), starts = torch::empty({stage.rows + 1}, stage.rowptr.options());
+    Tensor ws = torch::empty({(int64_t)cgnn_exclusive_sum_workspace_bytes(stage.rows)}, stage.rowptr.options().dtype(torch::kUInt8));
+    ok(cgnn_csr_expand_count(&a, V, &r, counts.data_ptr<int32_t>(), stream), "csr_expand_count");
+    ok(cgnn_exclusive_sum_i32(stage.rows, counts.data_ptr<int32_t>(), starts.data_ptr<int32_t>(), nullptr, ws.data_ptr(), ws.numel(),
+                              stream),
+       "exclusive_sum");
+    const int64_t entries = starts[stage.rows].item<int32_t>();
+    if (entries > kMaxWholeEntries || !takes_whole(entries, stage, rules, stage.val.element_size())) return nullptr;
+    Tensor col = torch::empty({entries}, stage.colidx.options()), val = torch::empty({entries}, stage.val.options());
+    ok(cgnn_csr_expand_columns(&a, V, &r, dtype_code(stage.val), starts.data_ptr<int32_t>(), col.data_ptr<int32_t>(), val.data_ptr(),
+                               stream),
+       "csr_expand_columns");
+    c10::optional<Tensor> rowmap;
+    if (stage.rowmap.defined()) rowmap = stage.rowmap;
+    return make_csr(starts, col, val, stage.rows, V, stage.rowptr.device(), stage.seg_nnz, rowmap);
+}
+
+// The multiplied-out stage where a product with x takes it.  A forced schedule and the two-launch form run the stages.
+bool use_whole(const PropagationPlan &p, const DeviceCsr *whole, const DeviceCsr &stage, const DeviceCsr &rules, const Tensor &x) {
+    return whole != nullptr && p.fuse_final && p.kernel == CGNN_SPMM_AUTO && x.scalar_type() == whole->val.scalar_type() &&
+           takes_whole(whole->nnz, stage, rules, x.size(1) * x.element_size());
+}
 
 Tensor timed_spmm(PropagationPlan &p, const std::string &stage, DeviceCsr &A, const Tensor &mat,
                   c10::optional<Tensor> out) {
@@ -569,13 +624,14 @@ Tensor final_stage(PropagationPlan &p, const std::string &prefix, DeviceCsr *mer
 }
 
 // layer/CompressgnnSPMM.py:43-62 of the reference.  Stage names: fwd.rules (r2v),
-// fwd.level<i>, fwd.final (v2r + v2v fused) or fwd.from_rules / fwd.from_vertices.
+// fwd.level<i>, fwd.final (v2r + v2v fused; alone where the rules are multiplied out) or fwd.from_rules / fwd.from_vertices.
 Tensor propagate_forward(PropagationPlan &p, Tensor x) {
     require_gpu(x, "x");
     TORCH_CHECK(x.dim() == 2 && x.size(0) == p.V, "x must be [vertex_cnt, F]");
     x = x.contiguous();
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
     Hold hold(p.lock);
+    if (p.whole && use_whole(p, p.whole.get(), *p.vertex_stage, *p.r2v, x)) return timed_spmm(p, "fwd.final", *p.whole, x, c10::nullopt);
     Tensor rule_out = timed_spmm(p, "fwd.rules", *p.r2v, x, c10::nullopt);
     for (size_t i = 0; i < p.r2r.size(); ++i)
         rule_out = timed_spmm(p, "fwd.level" + std::to_string(i), *p.r2r[i], rule_out, rule_out);
@@ -616,7 +672,7 @@ Tensor propagate_forward_gathered(PropagationPlan &p, Tensor reps, Tensor index)
     c10::hip::HIPGuardMasqueradingAsCUDA guard(reps.device());
     const int64_t groups = reps.size(0), F = reps.size(1);
     Hold hold(p.lock);
-    std::shared_ptr<DeviceCsr> rules, stage;
+    std::shared_ptr<DeviceCsr> rules, stage, whole;
     for (auto it = p.composed.begin(); it != p.composed.end();) {
         if (it->index.expired()) {
             it = p.composed.erase(it);
@@ -626,6 +682,7 @@ Tensor propagate_forward_gathered(PropagationPlan &p, Tensor reps, Tensor index)
             it->groups == groups) {
             rules = it->rules;
             stage = it->stage;
+            whole = it->whole;
             break;
         }
         ++it;
@@ -638,13 +695,15 @@ Tensor propagate_forward_gathered(PropagationPlan &p, Tensor reps, Tensor index)
            "narrow_ids");
         rules = compose_block(*p.r2v, narrow, p.V, groups);
         stage = compose_block(*p.vertex_stage, narrow, p.V, p.vertex_stage->cols);
+        if (p.whole) whole = compose_block(*p.whole, narrow, p.V, groups);
         TORCH_CHECK(bad.item<int32_t>() == 0, "propagation from representatives: the index holds a cluster id outside [0, ", groups, ")");
         if (!index.is_inference()) {
             p.composed.push_front(PropagationPlan::Composed{c10::weak_intrusive_ptr<c10::TensorImpl>(index.getIntrusivePtr()),
-                                                           index._version(), groups, rules, stage});
+                                                           index._version(), groups, rules, stage, whole});
             while (p.composed.size() > 4) p.composed.pop_back();
         }
     }
+    if (whole && use_whole(p, whole.get(), *stage, *rules, reps)) return timed_spmm(p, "fwd.final", *whole, reps, c10::nullopt);
     Tensor rule_out = timed_spmm(p, "fwd.rules", *rules, reps, c10::nullopt);
     for (size_t i = 0; i < p.r2r.size(); ++i)
         rule_out = timed_spmm(p, "fwd.level" + std::to_string(i), *p.r2r[i], rule_out, rule_out);
@@ -673,6 +732,8 @@ Tensor propagate_backward(PropagationPlan &p, Tensor grad) {
     grad = grad.contiguous();
     c10::hip::HIPGuardMasqueradingAsCUDA guard(grad.device());
     Hold hold(p.lock);
+    if (p.whole_t && use_whole(p, p.whole_t.get(), *p.vertex_stage_t, *p.v2r_t, grad))
+        return timed_spmm(p, "bwd.final", *p.whole_t, grad, c10::nullopt);
     Tensor rule_g = timed_spmm(p, "bwd.rules", *p.v2r_t, grad, c10::nullopt);
     for (size_t i = p.r2r_t.size(); i-- > 0;)
         rule_g = timed_spmm(p, "bwd.level" + std::to_string(i), *p.r2r_t[i], rule_g, rule_g);
@@ -1927,9 +1988,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                  TORCH_CHECK(fwd && bwd && fwd->rows == p.V && bwd->rows == p.V && fwd->cols == p.V + p.R &&
                                  bwd->cols == p.V + p.R,
                              "a vertex stage is [vertex_cnt, vertex_cnt + rule_cnt]");
+                 const bool folded = p.r2r.empty();  // no levels, or all of them in the rule stages
+                 auto whole = folded ? multiplied_out(*fwd, *p.r2v, p.V) : nullptr;
+                 auto whole_t = folded ? multiplied_out(*bwd, *p.v2r_t, p.V) : nullptr;
                  Hold hold(p.lock);
                  p.vertex_stage = fwd; p.vertex_stage_t = bwd;
+                 p.whole = whole; p.whole_t = whole_t;
                  p.adopt(fwd); p.adopt(bwd);
+                 p.adopt(whole); p.adopt(whole_t);
              })
         .def("set_split_blocks",
              [](PropagationPlan &p, std::shared_ptr<DeviceCsr> v2v, std::shared_ptr<DeviceCsr> v2r,

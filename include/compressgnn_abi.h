@@ -208,6 +208,16 @@ int cgnn_narrow_ids(int64_t n, const int64_t *ids, int64_t groups, int32_t *narr
 int cgnn_csr_compose_columns(int64_t nnz, const int32_t *colidx, int64_t first_cols, const int32_t *narrow_ids,
                              int32_t *out, cgnn_stream_t stream);
 
+/* A block with the columns from `split` on multiplied out: an entry (c, w) with c >= split becomes the entries
+ * (k, w * v) of row c - split of `rules` (values of the block's type; without values v is 1), in their order and in its
+ * place; the other entries stay.  cgnn_csr_expand_count writes the entries every row of A comes to (INT32_MAX if more
+ * do not fit), cgnn_csr_expand_columns the new columns and values for the row starts that these sum up to
+ * (cgnn_exclusive_sum_i32; no sum may have overflowed).  A needs values; its rowidx and rowmap are not looked at.
+ * The product of the vertex stage of layer/CompressgnnSPMM.py:59-60 with its rule stage (:54) as one matrix. */
+int cgnn_csr_expand_count(const cgnn_csr *A, int64_t split, const cgnn_csr *rules, int32_t *counts, cgnn_stream_t stream);
+int cgnn_csr_expand_columns(const cgnn_csr *A, int64_t split, const cgnn_csr *rules, int dtype, const int32_t *rowptr,
+                            int32_t *colidx, void *val, cgnn_stream_t stream);
+
 /* rowidx[e] = row of non-zero e, from an int32 rowptr. */
 int cgnn_csr_expand_rows(int64_t rows, int64_t nnz, const int32_t *rowptr,
                          int32_t *rowidx, cgnn_stream_t stream);

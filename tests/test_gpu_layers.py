@@ -245,6 +245,34 @@ def test_plan_feature_sweep(F, method, fold, fuse):
             other.to(DEV)
             other.edge_index.plan().fuse_final = False
 
+@pytest.mark.parametrize("F,one_launch", [(8, (True, True)), (128, (True, True)), (384, (False, True)), (1024, (False, False))])
+def test_rules_multiplied_out_or_in_stages(F, one_launch):
+    """A web graph of 60,000 vertices on both sides of the line from which a propagation runs its rule stage: AUTO against
+    the stages themselves (a forced schedule runs them), forward and gradient, and the propagation from representatives
+    gives the bits of the plain one on either side."""
+    import compressgnn_offline as off
+    from CompressgnnData import CompressgnnData
+    v, e = off.gen_copy_model(60000, 9.8, 0.7, 3)
+    V, mask = len(v) - 1, np.ones(len(v) - 1, bool)
+    data = CompressgnnData(np.zeros((V, 1), np.float32), (v, e), np.zeros(V, np.int64), mask, mask, mask, graph_type="csr")
+    data.to(DEV)
+    plan = data.edge_index.plan()
+    gen = torch.Generator(device=DEV).manual_seed(F)
+    x, g = (torch.randn(V, F, device=DEV, generator=gen) for _ in range(2))
+    plan.timed_stages = ["*"]
+    out, grad = plan.forward(x), plan.backward(g)
+    torch.cuda.synchronize()
+    names = [name for name, _ in plan.take_stage_times()]
+    assert names == [n for way, alone in zip(("fwd", "bwd"), one_launch) for n in ([] if alone else [way + ".rules"]) + [way + ".final"]]
+    plan.timed_stages = []
+    index = torch.randint(0, 900, (V,), device=DEV, generator=gen)
+    reps = torch.randn(900, F, device=DEV, generator=gen)
+    assert torch.equal(plan.forward_gathered(reps, index), plan.forward(reps.index_select(0, index)))
+    plan.method = "nnz_schedule"
+    # the same products in another order, and one more rounding of a weight: 2^-24 of the sum of absolute values per step
+    assert_within(out.cpu().numpy(), plan.forward(x).cpu().numpy(), rtol=1e-5, atol=1e-6)
+    assert_within(grad.cpu().numpy(), plan.backward(g).cpu().numpy(), rtol=1e-5, atol=1e-6)
+
 
 def test_rule_levels_are_stored_without_their_padding():
     """One launch per level (the form kept for hierarchies too deep to fold): the reference pads

@@ -544,3 +544,43 @@ def test_workgroup_runs_where_the_card_is_filled_once(share, F):
         got = A.spmm(t(x)).cpu().numpy()
         np.testing.assert_allclose(got, want, rtol=2e-5, atol=2e-5)
         assert np.array_equal(got, A.spmm(t(x)).cpu().numpy())
+
+
+@pytest.mark.parametrize("with_values", [True, False])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("rows", [1, 3, 4, 5, 130])
+def test_columns_multiplied_out(rows, dtype, with_values):
+    """cgnn_csr_expand_count / _columns against numpy: rows without entries, with rules only, and of 63 to 130 entries
+    (a wave takes 64 at a time), rules without entries and of up to 70.  A value is one product, so the arrays are the same."""
+    import ctypes
+    rng = np.random.default_rng(rows)
+    split, rules = 50, 9
+    lens = np.resize([0, 65, 1, 130, 63, 2, 64], rows)
+    rule_lens = np.array([0, 1, 2, 70, 3, 0, 64, 5, 65])
+    ptr = lambda n: np.concatenate([[0], np.cumsum(n)]).astype(np.int64)
+    vlist, rptr = ptr(lens), ptr(rule_lens)
+    # mostly plain columns, one row of rules alone
+    elist = np.where(rng.random(vlist[-1]) < 0.2, rng.integers(split, split + rules, vlist[-1]), rng.integers(0, split, vlist[-1]))
+    elist[vlist[0]:vlist[min(2, rows)]] = rng.integers(split, split + rules, vlist[min(2, rows)] - vlist[0])
+    value = rng.standard_normal(vlist[-1]).astype(dtype)
+    rcol, rval = rng.integers(0, split, rptr[-1]), rng.standard_normal(rptr[-1]).astype(dtype)
+    A = abi.DeviceCsr.from_host(rows, split + rules, vlist, elist, value, DEV)
+    B = abi.DeviceCsr.from_host(rules, split, rptr, rcol, rval if with_values else None, DEV)
+    want_ptr, want_col, want_val = [0], [], []
+    for r in range(rows):
+        for c, w in zip(elist[vlist[r]:vlist[r + 1]], value[vlist[r]:vlist[r + 1]]):
+            own = slice(rptr[c - split], rptr[c - split + 1]) if c >= split else None
+            want_col.extend([c] if own is None else rcol[own])
+            want_val.extend([w] if own is None else w * (rval[own] if with_values else np.ones(own.stop - own.start, dtype)))
+        want_ptr.append(len(want_col))
+    a, b, stream = A.struct(), B.struct(), abi.stream_of(A.rowptr)
+    counts = torch.empty(rows, dtype=torch.int32, device=DEV)
+    abi.check(abi.lib().cgnn_csr_expand_count(ctypes.byref(a), abi.i64(split), ctypes.byref(b), abi.ptr(counts), stream))
+    assert np.array_equal(counts.cpu().numpy(), np.diff(want_ptr))
+    starts = torch.tensor(want_ptr, dtype=torch.int32, device=DEV)
+    col = torch.full((max(1, len(want_col)),), -1, dtype=torch.int32, device=DEV)
+    val = torch.zeros(max(1, len(want_col)), dtype=A.val.dtype, device=DEV)
+    abi.check(abi.lib().cgnn_csr_expand_columns(ctypes.byref(a), abi.i64(split), ctypes.byref(b), abi.dtype_code(val.dtype),
+                                                abi.ptr(starts), abi.ptr(col), abi.ptr(val), stream))
+    assert np.array_equal(col.cpu().numpy()[:len(want_col)], np.array(want_col, np.int64))
+    assert np.array_equal(val.cpu().numpy()[:len(want_val)], np.array(want_val, dtype))
