@@ -123,6 +123,7 @@ struct LshArgs {
     int32_t stride_v;  // LDS row stride in units of VEC elements (odd)
     int32_t wstride;   // matrix-unit kernel, 16-byte rows: LDS stride of a plane in floats
     uint32_t magic;    // floor(2^32 / slab_v) + 1: i / slab_v == mulhi(i, magic) for i < 2^16
+    uint32_t hmagic;   // the same for bits
 };
 
 template <typename T, int VEC>
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(kLshRows) void lsh_hash_kernel(LshArgs<T> a) {
 // the current one out of LDS.  W is staged with zero columns beyond `bits`; NG = 2 covers
 // 17..30 planes with two instructions per k.  lsh_hash_mfma_kernel is the general form
 // (any F, several passes per tile); lsh_hash_mfma_flat_kernel below is the form for
-// 16-byte-aligned rows of at most 128 columns.
+// rows of at most 256 columns.
 
 typedef float lsh_acc_t __attribute__((ext_vector_type(16)));
 typedef float lsh_f4_t __attribute__((ext_vector_type(4)));
@@ -368,55 +369,64 @@ __global__ __launch_bounds__(kLshRows) void lsh_hash_mfma_kernel(LshArgs<float> 
     counter.flush(sink, lane);
 }
 
-// Whole rows per pass (F <= 128, 16-byte packs): the 64 rows of a tile are one contiguous
-// range of X, so pack p = lane + 64*u of the tile needs no index arithmetic on the way in
-// and a lane moves exactly F/4 packs per tile.  XP >= F/4 packs are loaded without any
+// Whole rows per tile (F <= 256): the 64 rows of a tile are one contiguous range of X whose length is a whole
+// number of 16-byte packs whatever F is, so pack p = lane + 64*u of the tile needs no index arithmetic on the way in
+// and a lane moves ceil(F/4) packs per tile.  XP >= F/4 packs are loaded without any
 // branch (offsets clamped to the last pack of the tile, which also covers the partial last
-// tile: the rows such loads fill are not written out); only the LDS writes are guarded, by
-// a wave-uniform condition.  The code of a tile is stored (and its bucket counted) only
-// after the next tile has been committed to LDS, so that no wait for the loads also waits
+// tile: the rows such loads fill are not written out); only the LDS writes are guarded.  The code of a tile is stored
+// (and its bucket counted) only after the next tile has been committed to LDS, so that no wait for the loads also waits
 // for that atomic.
 //
-// The tiles of a workgroup (those a static deal would give its waves) are handed out by a
+// PACKED: rows are whole packs and get an odd number of them in LDS, read 16 bytes at a time.  Otherwise the tile stands in
+// LDS as it does in memory and a lane reads its row element by element: four reads of 4 bytes against one of 16 for
+// 128 cycles of the matrix unit.  Such rows, and those of 129 to 256 columns, went through the general form, a wave per
+// workgroup that walks them 32 or 128 columns a pass and stages the planes with each (16 planes, us, general form / here:
+// 47 features, 71,981 rows 16.8 / 6.0 and 2,449,029 rows 309 / 77; 111 features, 20,011 rows 28.7 / 7.0 and 2,449,029
+// rows 1085 / 176, 6.2 TB/s; 136, 71,981 rows 33.7 / 15.5; 256, 1,000,003 rows 880 / 254).
+//
+// Workgroup b has tiles b, b + workgroups, ..., so that few rows are spread over as many compute units as they have
+// tiles; all waves of a workgroup stage the planes, those without a tile too.  The tiles of a workgroup are handed out by a
 // counter in LDS, one at a time: six waves on four SIMDs means two SIMDs carry two waves
-// and two carry one, and a wave that has a SIMD to itself gets through its tiles faster.
+// and two carry one, and a wave that has a SIMD to itself gets through its tiles faster.  The first tile of a wave is
+// asked for before the planes are staged: with few rows a wave has one tile, and the launch is these two latencies
+// (2,708 rows of 100 features: 8.3 us with the tiles of a workgroup next to each other, 5.8 so).
 constexpr int kLshFlatMaxWaves = 8;
+constexpr int kLshFlatMaxCols = 256;
 constexpr int kLshQueueBytes = 16;  // the counter, padded so that the tiles stay 16-byte aligned
 
-template <int NG, int XP>
-__global__ __launch_bounds__(kLshRows *kLshFlatMaxWaves) void lsh_hash_mfma_flat_kernel(LshArgs<float> a,
-                                                                                       int64_t tiles) {
-    // LDS: the planes, shared by the waves of the workgroup, then one X tile per wave.
-    // The waves are independent after the planes have been staged.
+// Rows of the planes in LDS: 16 for each group of the matrix instruction; beside tiles of long rows, which leave less
+// room, those there are and one of zeros.
+__host__ __device__ constexpr int lsh_plane_rows(int groups, int F, int bits) {
+    return (F + 3) / 4 <= kLshMfmaSlab / 4 ? 16 * groups : bits + 1;
+}
+
+typedef float lsh_f4_unaligned_t __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int NG, int XP, bool PACKED>
+__global__ __launch_bounds__(kLshRows *(XP > 32 ? 2 : kLshFlatMaxWaves)) void lsh_hash_mfma_flat_kernel(LshArgs<float> a,
+                                                                                                       int64_t tiles) {
+    // LDS: the planes, shared by the waves of the workgroup, then one X tile per wave.  The waves are independent after
+    // the planes have been staged.
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+    constexpr bool kPadded = XP <= kLshMfmaSlab / 4;
     const int lane = threadIdx.x & (kLshRows - 1);
-    const int wave = threadIdx.x / kLshRows;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLshRows);
     const int waves = blockDim.x / kLshRows;
+    const int H = a.bits;
     float *wtile = reinterpret_cast<float *>(lds_raw);
-    const size_t plane_bytes = (size_t)a.wstride * 16 * NG * sizeof(float);
+    const size_t plane_bytes = (size_t)a.wstride * lsh_plane_rows(NG, a.F, H) * sizeof(float);
     int *queue = reinterpret_cast<int *>(lds_raw + plane_bytes);
     lsh_f4_t *tile = reinterpret_cast<lsh_f4_t *>(lds_raw + plane_bytes + kLshQueueBytes) +
-                     (size_t)wave * kLshRows * a.stride_v;
-    const int H = a.bits;
-    const int ks_v = a.F / 4;  // packs per row = packs per lane and tile
-    const lsh_f4_t *X4 = reinterpret_cast<const lsh_f4_t *>(a.X);
-    const int64_t first = (int64_t)blockIdx.x * waves;
-    const int64_t step = (int64_t)gridDim.x * waves;
+                     (size_t)wave * (PACKED ? kLshRows * a.stride_v : kLshRows / 4 * a.F);
+    const int ks_v = PACKED ? a.F / 4 : (a.F + 3) / 4;  // packs per lane and tile
     const GlobalSink sink{a.bucket_count};
-
-    for (int e = threadIdx.x; e < a.F * 16 * NG; e += blockDim.x) {  // planes as [plane][k]
-        const int kk = e / (16 * NG), j = e % (16 * NG);
-        wtile[j * a.wstride + kk] = j < H ? a.W[(int64_t)kk * H + j] : 0.f;
-    }
-    if (threadIdx.x == 0) *queue = 0;
-    __syncthreads();
     // the j-th tile of this workgroup; grows with j, so a wave that draws one beyond the
     // end is done, and so is every later draw
+    auto nth = [&](int j) { return (int64_t)j * gridDim.x + blockIdx.x; };
     auto take = [&]() -> int64_t {
         int j = 0;
         if (lane == 0) j = atomicAdd(queue, 1);
-        j = __builtin_amdgcn_readfirstlane(j);
-        return (int64_t)(j / waves) * step + first + j % waves;
+        return nth(__builtin_amdgcn_readfirstlane(j));
     };
 
     lsh_acc_t acc[NG];
@@ -426,27 +436,55 @@ __global__ __launch_bounds__(kLshRows *kLshFlatMaxWaves) void lsh_hash_mfma_flat
         for (int v = 0; v < 16; ++v) acc[g][v] = 0.f;
 
     lsh_f4_t xr[XP];
+    auto floats_of = [&](int64_t t) { return (int)min((int64_t)kLshRows, a.N - t * kLshRows) * a.F; };
     auto fetch = [&](int64_t t) {
-        const int64_t row0 = t * kLshRows;
-        const lsh_f4_t *src = X4 + row0 * ks_v;
-        const int top = (int)min((int64_t)kLshRows, a.N - row0) * ks_v - 1;
+        const lsh_f4_unaligned_t *src = reinterpret_cast<const lsh_f4_unaligned_t *>(a.X + t * kLshRows * a.F);
+        const int top = floats_of(t) / 4 - 1;
+        if (!PACKED && top < 0) return;  // fewer than four floats in all: commit() takes them one by one
 #pragma unroll
         for (int u = 0; u < XP; ++u) xr[u] = __builtin_nontemporal_load(src + min(lane + u * kLshRows, top));
     };
+    int64_t t = nth(wave);
+    if (t < tiles) fetch(t);
+
+    if constexpr (kPadded) {  // planes as [plane][k], zero beyond bits
+#pragma unroll 4
+        for (int e = threadIdx.x; e < a.F * 16 * NG; e += blockDim.x) {
+            const int kk = e / (16 * NG), j = e % (16 * NG);
+            wtile[j * a.wstride + kk] = j < H ? a.W[(int64_t)kk * H + j] : 0.f;
+        }
+    } else {  // the planes there are and one row of zeros for the lanes beyond: element e of W is W[e / H][e % H]
+#pragma unroll 4
+        for (int e = threadIdx.x; e < a.F * H; e += blockDim.x) {
+            const int kk = H > 1 ? (int)__umulhi((uint32_t)e, a.hmagic) : e;
+            wtile[(e - kk * H) * a.wstride + kk] = a.W[e];
+        }
+        for (int k = threadIdx.x; k < a.wstride; k += blockDim.x) wtile[H * a.wstride + k] = 0.f;
+    }
+    if (threadIdx.x == 0) *queue = waves;
+    __syncthreads();
+
     // slot of pack p: row * stride_v + column pack = p + row * (stride_v - ks_v)
-    const bool padded = a.stride_v != ks_v;
+    const bool padded = PACKED && a.stride_v != ks_v;
     const int myv = 4 * (lane >> 4) + (lane & 3);
     const int shift = 16 * ((lane & 15) >> 2);
     const lsh_f4_t *mine = tile + lane * a.stride_v;
-    const lsh_f4_t *wq = reinterpret_cast<const lsh_f4_t *>(wtile + (lane & 15) * a.wstride);
-    const int gstep = 4 * a.wstride;  // 16 planes further, in 16-byte units
+    const float *mine1 = reinterpret_cast<const float *>(tile) + lane * a.F;
+    const lsh_f4_t *wq = reinterpret_cast<const lsh_f4_t *>(wtile + (kPadded ? lane & 15 : min(lane & 15, H)) * a.wstride);
+    // 16 planes further, in 16-byte units
+    const int gstep = (kPadded ? 16 : min((lane & 15) + 16, H) - min(lane & 15, H)) * (a.wstride / 4);
 
     auto multiply = [&](int c, auto count) {
         constexpr int n = decltype(count)::value;
         lsh_f4_t x[n], w[NG][n];
 #pragma unroll
         for (int i = 0; i < n; ++i) {
-            x[i] = mine[c + i];
+            if constexpr (PACKED) {
+                x[i] = mine[c + i];
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) x[i][k] = mine1[4 * (c + i) + k];
+            }
 #pragma unroll
             for (int g = 0; g < NG; ++g) w[g][i] = wq[g * gstep + c + i];
         }
@@ -465,14 +503,21 @@ __global__ __launch_bounds__(kLshRows *kLshFlatMaxWaves) void lsh_hash_mfma_flat
     WaveCodeCounter counter;
     int pending_code = 0;
     int64_t pending_row = -1;
-    int64_t t = take();
-    if (t < tiles) fetch(t);
     while (t < tiles) {
         wave_lds_sync();  // the previous tile has been consumed
 #pragma unroll
         for (int u = 0; u < XP; ++u) {
             const int p = lane + u * kLshRows;
-            if (u < ks_v) tile[p + (padded ? (int)__umulhi((uint32_t)p, a.magic) : 0)] = xr[u];
+            if constexpr (PACKED) {
+                if (u < ks_v) tile[p + (padded ? (int)__umulhi((uint32_t)p, a.magic) : 0)] = xr[u];
+            } else {
+                if (p < kLshRows / 4 * a.F) tile[p] = xr[u];
+            }
+        }
+        if constexpr (!PACKED) {
+            // the last tile may end inside a pack
+            const int n = floats_of(t), held = n / 4 * 4;
+            if (lane < n - held) reinterpret_cast<float *>(tile)[held + lane] = a.X[t * kLshRows * a.F + held + lane];
         }
         wave_lds_sync();
         if (pending_row >= 0 && pending_row < a.N) a.raw_code[pending_row] = pending_code;
@@ -480,15 +525,26 @@ __global__ __launch_bounds__(kLshRows *kLshFlatMaxWaves) void lsh_hash_mfma_flat
         const int64_t t_next = take();
         if (t_next < tiles) fetch(t_next);
 
-        // eight column packs at a time: all sixteen LDS reads are issued before the first
-        // multiply, so their latency is paid once per 32 matrix instructions
+        // Column packs of 32 matrix instructions at a time: all their LDS reads are issued before the first multiply,
+        // so their latency is paid once for these (and with two groups of planes the registers hold no more than that).
+        const int whole = a.F / 4;
         int c = 0;
-        for (; c + 8 <= ks_v; c += 8) multiply(c, std::integral_constant<int, 8>{});
-        if (c + 4 <= ks_v) {
-            multiply(c, std::integral_constant<int, 4>{});
-            c += 4;
+        if constexpr (NG == 1) {
+            for (; c + 8 <= whole; c += 8) multiply(c, std::integral_constant<int, 8>{});
+            if (c + 4 <= whole) {
+                multiply(c, std::integral_constant<int, 4>{});
+                c += 4;
+            }
+        } else {
+            for (; c + 4 <= whole; c += 4) multiply(c, std::integral_constant<int, 4>{});
         }
-        for (; c < ks_v; ++c) multiply(c, std::integral_constant<int, 1>{});
+        for (; c < whole; ++c) multiply(c, std::integral_constant<int, 1>{});
+        if constexpr (!PACKED) {
+            for (int k = 4 * whole; k < a.F; ++k)
+#pragma unroll
+                for (int g = 0; g < NG; ++g)
+                    acc[g] = __builtin_amdgcn_mfma_f32_16x16x1f32(mine1[k], reinterpret_cast<const float *>(wq + g * gstep)[k], acc[g], 0, 0, 0);
+        }
 
         unsigned long long sel[NG];
 #pragma unroll
@@ -559,31 +615,44 @@ int compute_units() {
 template <typename Kernel>
 int launch_lsh_persistent(Kernel kernel, int waves, size_t lds, const LshArgs<float> &a, hipStream_t stream) {
     const int64_t tiles = ceil_div(a.N, kLshRows);
-    // exactly as many workgroups as are resident at once, each wave walking its share of
-    // the tiles
+    // exactly as many workgroups as are resident at once, each walking its share of the tiles
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kLshRows * waves, lds) != hipSuccess ||
         per_cu < 1)
         per_cu = 1;
     int64_t blocks = (int64_t)per_cu * compute_units();
-    if (blocks > ceil_div(tiles, waves)) blocks = ceil_div(tiles, waves);
+    if (blocks > tiles) blocks = tiles;
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kLshRows * waves), lds, stream, a, tiles);
     return check_launch("lsh_hash");
 }
 
 constexpr size_t kLdsPerCu = 160 * 1024;
 constexpr size_t kLdsDefaultLimit = 64 * 1024;  // larger workgroups must be allowed per kernel
+constexpr int kLshNoFlat = -1;                  // ... and this one is not: the general form serves
 
-template <int NG, int XP>
+// How many waves of the flat form a compute unit's LDS holds beside one copy of the planes.
+struct LshFlat {
+    size_t fixed_bytes, tile_bytes;
+    int waves;
+};
+
+LshFlat lsh_flat(const LshArgs<float> &a) {
+    LshFlat f;
+    const bool packed = a.F % 4 == 0;
+    f.tile_bytes = (size_t)kLshRows * (packed ? a.stride_v * sizeof(lsh_f4_t) : a.F * sizeof(float));
+    f.fixed_bytes = (size_t)a.wstride * lsh_plane_rows(a.bits > 16 ? 2 : 1, a.F, a.bits) * sizeof(float) + kLshQueueBytes;
+    // two per SIMD at most, one wave on two of them for rows of more than 512 bytes (registers)
+    const int most = a.F > kLshMfmaSlab ? 2 : kLshFlatMaxWaves;
+    const int fit = f.fixed_bytes < kLdsPerCu ? (int)((kLdsPerCu - f.fixed_bytes) / f.tile_bytes) : 0;
+    f.waves = fit > most ? most : fit;
+    return f;
+}
+
+template <int NG, int XP, bool PACKED>
 int launch_lsh_flat(const LshArgs<float> &a, hipStream_t stream) {
-    const size_t tile_bytes = (size_t)kLshRows * a.stride_v * sizeof(lsh_f4_t);
-    const size_t plane_bytes = (size_t)a.wstride * 16 * NG * sizeof(float);
-    // as many waves as fit beside one copy of the planes; two per SIMD at most (registers)
-    const size_t fixed_bytes = plane_bytes + kLshQueueBytes;
-    int waves = (int)((kLdsPerCu - fixed_bytes) / tile_bytes);
-    waves = waves < 1 ? 1 : (waves > kLshFlatMaxWaves ? kLshFlatMaxWaves : waves);
-    auto kernel = lsh_hash_mfma_flat_kernel<NG, XP>;
-    size_t lds = fixed_bytes + waves * tile_bytes;
+    const LshFlat f = lsh_flat(a);
+    auto kernel = lsh_hash_mfma_flat_kernel<NG, XP, PACKED>;
+    const size_t lds = f.fixed_bytes + f.waves * f.tile_bytes;
     if (lds > kLdsDefaultLimit) {
         static bool allowed = false, refused = false;  // per kernel instantiation
         if (!allowed && !refused) {
@@ -595,28 +664,52 @@ int launch_lsh_flat(const LshArgs<float> &a, hipStream_t stream) {
                 (void)hipGetLastError();
             }
         }
-        if (!allowed) {
-            waves = (int)((kLdsDefaultLimit - fixed_bytes) / tile_bytes);
-            waves = waves < 1 ? 1 : waves;
-            lds = fixed_bytes + waves * tile_bytes;
-        }
+        if (!allowed) return kLshNoFlat;
     }
-    return launch_lsh_persistent(kernel, waves, lds, a, stream);
+    return launch_lsh_persistent(kernel, f.waves, lds, a, stream);
+}
+
+// 16-byte rows of up to 512 bytes in the steps that the registers come in; others in steps of 32 columns.
+template <int NG>
+int dispatch_lsh_flat(const LshArgs<float> &a, hipStream_t stream) {
+    const int packs = (a.F + 3) / 4;
+    if (a.F % 4 == 0) {
+        if (packs <= 4) return launch_lsh_flat<NG, 4, true>(a, stream);
+        if (packs <= 8) return launch_lsh_flat<NG, 8, true>(a, stream);
+        if (packs <= 12) return launch_lsh_flat<NG, 12, true>(a, stream);
+        if (packs <= 16) return launch_lsh_flat<NG, 16, true>(a, stream);
+        if (packs <= 20) return launch_lsh_flat<NG, 20, true>(a, stream);
+        if (packs <= 24) return launch_lsh_flat<NG, 24, true>(a, stream);
+        if (packs == 25) return launch_lsh_flat<NG, 25, true>(a, stream);
+        if (packs <= 28) return launch_lsh_flat<NG, 28, true>(a, stream);
+        if (packs <= 32) return launch_lsh_flat<NG, 32, true>(a, stream);
+        if (packs <= 40) return launch_lsh_flat<NG, 40, true>(a, stream);
+        if (packs <= 48) return launch_lsh_flat<NG, 48, true>(a, stream);
+        return launch_lsh_flat<NG, 64, true>(a, stream);
+    }
+    if (packs <= 8) return launch_lsh_flat<NG, 8, false>(a, stream);
+    if (packs <= 16) return launch_lsh_flat<NG, 16, false>(a, stream);
+    if (packs <= 24) return launch_lsh_flat<NG, 24, false>(a, stream);
+    if (packs <= 32) return launch_lsh_flat<NG, 32, false>(a, stream);
+    if (packs <= 48) return launch_lsh_flat<NG, 48, false>(a, stream);
+    return launch_lsh_flat<NG, 64, false>(a, stream);
 }
 
 template <int VEC, int NG>
 int launch_lsh_mfma(const LshArgs<float> &a, hipStream_t stream) {
-    if (VEC == 4 && a.slab == a.F) {  // whole rows per pass
-        const int packs = a.F / 4;
-        if (packs <= 4) return launch_lsh_flat<NG, 4>(a, stream);
-        if (packs <= 8) return launch_lsh_flat<NG, 8>(a, stream);
-        if (packs <= 12) return launch_lsh_flat<NG, 12>(a, stream);
-        if (packs <= 16) return launch_lsh_flat<NG, 16>(a, stream);
-        if (packs <= 20) return launch_lsh_flat<NG, 20>(a, stream);
-        if (packs <= 24) return launch_lsh_flat<NG, 24>(a, stream);
-        if (packs == 25) return launch_lsh_flat<NG, 25>(a, stream);
-        if (packs <= 28) return launch_lsh_flat<NG, 28>(a, stream);
-        return launch_lsh_flat<NG, 32>(a, stream);
+    // A tile of whole rows where at least two fit a compute unit (rows of up to 1 KB, and the planes beside them);
+    // longer rows go column slab by column slab.
+    if (a.F <= kLshFlatMaxCols) {
+        LshArgs<float> flat = a;
+        const int packs = (a.F + 3) / 4;
+        flat.stride_v = packs | 1;
+        flat.wstride = (packs | 1) * 4;
+        flat.magic = packs > 1 ? (uint32_t)((1ull << 32) / (uint32_t)packs) + 1u : 0u;
+        flat.hmagic = (uint32_t)((1ull << 32) / (uint32_t)a.bits) + 1u;
+        if (lsh_flat(flat).waves >= 2) {
+            const int rc = dispatch_lsh_flat<NG>(flat, stream);
+            if (rc != kLshNoFlat) return rc;
+        }
     }
     const size_t x_bytes = (size_t)kLshRows * a.stride_v * VEC * sizeof(float);
     return launch_lsh_persistent(lsh_hash_mfma_kernel<VEC, NG>, 1,

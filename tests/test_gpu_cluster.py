@@ -34,6 +34,35 @@ def pack_signs(out):
     return packed.astype(np.uint32).view(np.int32)
 
 
+@pytest.mark.parametrize("bits", [1, 16, 17, 22])
+@pytest.mark.parametrize("width", [1, 2, 3, 5, 30, 64, 127, 129, 160, 193, 250, 256, 257])
+@pytest.mark.parametrize("rows", [1, 64, 65, 4003])
+def test_hash_of_rows_of_any_width(rows, width, bits):
+    """Ids against the oracle on both sides of the widths at which the hash kernel changes its form, for rows that are whole
+    16-byte packs and others, tiles that end inside a pack, and features that begin anywhere in memory; a row with NaN or
+    infinities leaves the rows beside it alone."""
+    rng = np.random.default_rng(rows * 1000 + width)
+    x = rng.standard_normal((rows, width)).astype(np.float32)
+    if rows > 64:
+        x[::37, 0], x[5::41, width - 1] = np.nan, np.inf
+    w = rng.standard_normal((width, bits)).astype(np.float32)
+    want, _, active = oracle.assign(x, w, bits)
+    shifted = torch.empty(rows * width + 1, device=DEV)[1:].view(rows, width)
+    shifted.copy_(_t(x))
+    for features in (_t(x), shifted):
+        ids, _, n, _ = abi.lsh_assign_grouped(features, _t(w), bits)
+        assert n == active and np.array_equal(ids.cpu().numpy(), want)
+
+
+def test_hash_tiles_are_drawn_in_turn():
+    """More tiles than all waves of the card hold at once, rows that are no whole packs."""
+    rng = np.random.default_rng(7)
+    x, w = rng.standard_normal((300007, 6)).astype(np.float32), rng.standard_normal((6, 9)).astype(np.float32)
+    want, _, active = oracle.assign(x, w, 9)
+    ids, _, n, _ = abi.lsh_assign_grouped(_t(x), _t(w), 9)
+    assert n == active and np.array_equal(ids.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("width", [0, 1, 31, 33, 100, 128, 602])
 @pytest.mark.parametrize("n,bits", [(1, 0), (67, 8), (257, 16), (1000, 5), (5000, 12), (300, 20)])
