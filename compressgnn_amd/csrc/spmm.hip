@@ -213,6 +213,73 @@ __device__ __forceinline__ void feature_offsets(int64_t F, int lane, int64_t fof
     }
 }
 
+// What a gather of one feature tile brings: the pack of X, and what decides which of its elements count.  Loads only: they
+// stand in a branch of their own (no gathers behind the end of a row), and what used the loaded values there would have to
+// wait for them before the next gather of the round is asked for -- four waits one after the other, which doubled the time of
+// sums that are a chain of rounds (with sign words, us, so / as it stands: 30,011 rows of 256 features 43 / 27, 100,003 of 100
+// 41 / 28, 1,000,003 of 188 211 / 188; without a mask 23, 23 and 177).
+template <typename T, int VEC, int MODE>
+struct Gathered {
+    Pack<T, VEC> x;
+    Pack<T, MODE == MODE_RELU_MASK ? VEC : 1> m;  // MODE_RELU_MASK: the rows that decide
+    uint32_t word, next;                          // MODE_SIGN_MASK: the word the pack's bits begin in, and the one behind
+
+    // the pack, zeroed where the mask drops an element
+    __device__ __forceinline__ Pack<T, VEC> masked(int64_t foff) const {
+        Pack<T, VEC> o = x;
+        if constexpr (MODE == MODE_SIGN_MASK) {
+            const uint32_t bits = __builtin_amdgcn_alignbit(next, word, (uint32_t)foff & 31u);
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) o.v[i] = ((bits >> i) & 1u) ? o.v[i] : T(0);
+        }
+        if constexpr (MODE == MODE_RELU_MASK)
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) o.v[i] = (m.v[i] <= T(0)) ? T(0) : o.v[i];
+        return o;
+    }
+};
+
+// kRowBytes: what the lanes of a row span.  Gather one feature tile of column c (source chosen by `src` in MODE_DUAL).
+template <typename T, int VEC, int MODE, int kRowBytes>
+__device__ __forceinline__ Gathered<T, VEC, MODE> gather(const SpmmArgs<T> &a, int c, int src, int64_t foff) {
+    Gathered<T, VEC, MODE> g;
+    if (foff < 0) {
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) g.x.v[i] = T(0);
+        if constexpr (MODE == MODE_SIGN_MASK) g.word = g.next = 0;
+        if constexpr (MODE == MODE_RELU_MASK) g.m = g.x;
+        return g;
+    }
+    const T *base = a.X;
+    if constexpr (MODE == MODE_DUAL) {
+        // both pointers are read first and chosen between as values (a choice between the two
+        // fields of the argument block becomes a vector load of the chosen field, and a wait)
+        const T *first = a.X, *second = a.X1;
+        base = src ? second : first;
+        c -= src ? a.split : 0;
+    }
+    const int64_t off = (int64_t)c * (int32_t)a.F + foff;  // F < 2^31: one 32 x 32 -> 64 bit multiply
+    // Rows that are gathered once (member lists, which the modes without values exist for) are not kept in the
+    // caches -- unless they are shorter than a cache line, whose other half is a row that is still to come (16
+    // features, 10^6 rows: 44 us so, 32 us kept).  A choice at compile time: the compiler merges the two loads of a
+    // branch into one that is kept.  Kept rows cost the kernel that writes next most: behind the means of 2.4 M rows
+    // the spread of 256 features took 725 us for 485 and the gradient of the means 283 us for 175.
+    if constexpr ((MODE == MODE_RELU_MASK || MODE == MODE_SIGN_MASK || MODE == MODE_UNIT) && kRowBytes > 128)
+        g.x = load_pack_stream<T, VEC>(base + off);
+    else
+        g.x = load_pack<T, VEC>(base + off);
+    if constexpr (MODE == MODE_SIGN_MASK) {
+        const uint32_t *words = a.signs + (int64_t)c * a.sign_words;
+        const int at = (int)(foff >> 5);
+        g.word = words[at];
+        g.next = 0;  // not a copy of the word, which would have to be waited for
+        // VEC divides 32, so the bits of one pack lie in one word, unless the pack was moved back
+        if (VEC > 1 && (a.F & (VEC - 1)) != 0) g.next = words[min(at + 1, a.sign_words - 1)];
+    }
+    if constexpr (MODE == MODE_RELU_MASK) g.m = load_pack_stream<T, VEC>(a.M + off);
+    return g;
+}
+
 // Accumulator of one output row.  MODE_DUAL keeps the sums over the two sources apart: the
 // entries of a row are sorted by column, so those of the first source come first; when the
 // first entry of the second source arrives the running sum is put aside and started anew.
@@ -232,8 +299,8 @@ struct Acc {
                 if constexpr (MODE == MODE_DUAL) a1[t].v[i] = T(0);
             }
     }
-    // entry with gathered tiles x, value w, from source `src` (0 or 1)
-    __device__ __forceinline__ void add(const Pack<T, VEC> x[TILES], T w, int src) {
+    // entry with gathered tiles g at features foff, value w, from source `src` (0 or 1)
+    __device__ __forceinline__ void add(const Gathered<T, VEC, MODE> g[TILES], const int64_t foff[TILES], T w, int src) {
         if constexpr (MODE == MODE_DUAL) {
             // At most once per row, so the whole wave jumps over it nearly always.  Written
             // with value selects under a wave-uniform branch: a branch per lane would be
@@ -251,12 +318,14 @@ struct Acc {
             }
         }
 #pragma unroll
-        for (int t = 0; t < TILES; ++t)
+        for (int t = 0; t < TILES; ++t) {
+            const Pack<T, VEC> x = g[t].masked(foff[t]);
 #pragma unroll
             for (int i = 0; i < VEC; ++i) {
-                if constexpr (MODE == MODE_VAL || MODE == MODE_DUAL) a0[t].v[i] = a0[t].v[i] + x[t].v[i] * w;
-                else a0[t].v[i] = a0[t].v[i] + x[t].v[i];
+                if constexpr (MODE == MODE_VAL || MODE == MODE_DUAL) a0[t].v[i] = a0[t].v[i] + x.v[i] * w;
+                else a0[t].v[i] = a0[t].v[i] + x.v[i];
             }
+        }
     }
     // the row's value on top of `base`: (base + sum1) + sum0 in MODE_DUAL, base + sum otherwise
     __device__ __forceinline__ T total(T base, int t, int i) const {
@@ -297,51 +366,6 @@ __device__ __forceinline__ void write_row(T *Y, int64_t F, int row, const int64_
         if (accumulate) store_pack<T, VEC>(yrow + foff[t], o);
         else store_pack_stream<T, VEC>(yrow + foff[t], o);
     }
-}
-
-// kRowBytes: what the lanes of a row span.  Gather one feature tile of column c (source chosen by `src` in MODE_DUAL, masked by
-// M in MODE_RELU_MASK and by the bits of `signs` in MODE_SIGN_MASK).
-template <typename T, int VEC, int MODE, int kRowBytes>
-__device__ __forceinline__ Pack<T, VEC> gather(const SpmmArgs<T> &a, int c, int src, int64_t foff) {
-    Pack<T, VEC> x;
-    if (foff < 0) {
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) x.v[i] = T(0);
-        return x;
-    }
-    const T *base = a.X;
-    if constexpr (MODE == MODE_DUAL) {
-        // both pointers are read first and chosen between as values (a choice between the two
-        // fields of the argument block becomes a vector load of the chosen field, and a wait)
-        const T *first = a.X, *second = a.X1;
-        base = src ? second : first;
-        c -= src ? a.split : 0;
-    }
-    const int64_t off = (int64_t)c * (int32_t)a.F + foff;  // F < 2^31: one 32 x 32 -> 64 bit multiply
-    // Rows that are gathered once (member lists, which the modes without values exist for) are not kept in the
-    // caches -- unless they are shorter than a cache line, whose other half is a row that is still to come (16
-    // features, 10^6 rows: 44 us so, 32 us kept).  A choice at compile time: the compiler merges the two loads of a
-    // branch into one that is kept.  Kept rows cost the kernel that writes next most: behind the means of 2.4 M rows
-    // the spread of 256 features took 725 us for 485 and the gradient of the means 283 us for 175.
-    if constexpr ((MODE == MODE_RELU_MASK || MODE == MODE_SIGN_MASK || MODE == MODE_UNIT) && kRowBytes > 128)
-        x = load_pack_stream<T, VEC>(base + off);
-    else
-        x = load_pack<T, VEC>(base + off);
-    if constexpr (MODE == MODE_SIGN_MASK) {
-        const uint32_t *words = a.signs + (int64_t)c * a.sign_words;
-        uint32_t bits = words[foff >> 5] >> (foff & 31);
-        // VEC divides 32, so the bits of one pack lie in one word, unless the pack was moved back
-        if (VEC > 1 && (a.F & (VEC - 1)) != 0 && (foff & 31) > 32 - VEC)
-            bits |= words[(foff >> 5) + 1] << (32 - (foff & 31));
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) x.v[i] = ((bits >> i) & 1u) ? x.v[i] : T(0);
-    }
-    if constexpr (MODE == MODE_RELU_MASK) {
-        Pack<T, VEC> m = load_pack_stream<T, VEC>(a.M + off);
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) x.v[i] = (m.v[i] <= T(0)) ? T(0) : x.v[i];
-    }
-    return x;
 }
 
 // Row of Y that stored row r stands for.
@@ -448,7 +472,7 @@ __global__ __launch_bounds__(kBlock) void spmm_row_kernel(SpmmArgs<T> a) {
                 }
                 auto gather_and_add = [&](auto plain) {
                     constexpr bool kPlain = decltype(plain)::value;  // every entry from the first source
-                    Pack<T, VEC> x[RU][TILES];
+                    Gathered<T, VEC, MODE> x[RU][TILES];
 #pragma unroll
                     for (int u = 0; u < RU; ++u)
                         if (u0 + u < cnt) {  // no gathers behind the row's end: repeated ones still cost issue slots
@@ -458,7 +482,7 @@ __global__ __launch_bounds__(kBlock) void spmm_row_kernel(SpmmArgs<T> a) {
                         }
 #pragma unroll
                     for (int u = 0; u < RU; ++u)
-                        if (u0 + u < cnt) acc.add(x[u], w[u], kPlain ? 0 : c[u] >= a.split);
+                        if (u0 + u < cnt) acc.add(x[u], fld, w[u], kPlain ? 0 : c[u] >= a.split);
                 };
                 if (MODE != MODE_DUAL || __ballot(second) == 0) gather_and_add(std::true_type{});
                 else gather_and_add(std::false_type{});
@@ -468,7 +492,7 @@ __global__ __launch_bounds__(kBlock) void spmm_row_kernel(SpmmArgs<T> a) {
         for (int e = e0; e < e1; e += kRowUnroll) {
             int c[kRowUnroll];
             T w[kRowUnroll];
-            Pack<T, VEC> x[kRowUnroll][TILES];
+            Gathered<T, VEC, MODE> x[kRowUnroll][TILES];
 #pragma unroll
             for (int u = 0; u < kRowUnroll; ++u) {
                 const int idx = min(e + u, e1 - 1);
@@ -483,7 +507,7 @@ __global__ __launch_bounds__(kBlock) void spmm_row_kernel(SpmmArgs<T> a) {
                 }
 #pragma unroll
             for (int u = 0; u < kRowUnroll; ++u)
-                if (e + u < e1) acc.add(x[u], w[u], c[u] >= a.split);
+                if (e + u < e1) acc.add(x[u], foff, w[u], c[u] >= a.split);
         }
     }
     write_row<T, VEC, TILES, MODE>(a.Y, a.F, row, foff, acc, a.accumulate);
@@ -814,7 +838,7 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                     }
                     auto gather_and_add = [&](auto plain) {
                         constexpr bool kPlain = decltype(plain)::value;  // every entry from the first source
-                        Pack<T, VEC> x[kUnroll][TILES];
+                        Gathered<T, VEC, MODE> x[kUnroll][TILES];
                         // Up to 64 bytes per lane group and gather, a position behind the last entry gathers
                         // like the others (column 0, see above): the branches around four small loads cost
                         // more than the loads.  Wider rows skip it: there the extra row is what costs.
@@ -836,7 +860,7 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                                     acc.clear();
                                     cur_out = o[u];
                                 }
-                                acc.add(x[u], w[u], kPlain ? 0 : c[u] >= a.split);
+                                acc.add(x[u], fld, w[u], kPlain ? 0 : c[u] >= a.split);
                             }
                         }
                     };
@@ -855,7 +879,7 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
             for (int e = e0; e < e1; e += kUnroll) {
                 int o[kUnroll], c[kUnroll];
                 T w[kUnroll];
-                Pack<T, VEC> x[kUnroll][TILES];
+                Gathered<T, VEC, MODE> x[kUnroll][TILES];
 #pragma unroll
                 for (int u = 0; u < kUnroll; ++u) {
                     const int idx = min(e + u, e1 - 1);
@@ -882,7 +906,7 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                             acc.clear();
                             cur_out = o[u];
                         }
-                        acc.add(x[u], w[u], c[u] >= a.split);
+                        acc.add(x[u], foff, w[u], c[u] >= a.split);
                     }
                 }
             }
