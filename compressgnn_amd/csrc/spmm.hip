@@ -38,7 +38,7 @@
 //     per workgroup in memory; the workgroup that finds itself the last to arrive at the row adds the pieces
 //     up, in ascending order, so the sum does not depend on which one that is.
 //
-// Modes: VAL (stored values), UNIT (all values 1: member lists, whose rows are gathered once), RELU_MASK (unit values, gathered
+// Modes: VAL (stored values), ADD (the same, added to what Y holds), UNIT (all values 1: member lists, whose rows are gathered once), RELU_MASK (unit values, gathered
 // rows zeroed where a second matrix is <= 0), DUAL (columns below `split` gather from
 // X, the others from X1; the two partial sums are kept apart and combined as
 // (0 + sum1) + sum0, which is what two successive accumulating products give).
@@ -64,7 +64,8 @@ constexpr int kDefaultSeg = 64;   // non-zeros per lane group in the nnz schedul
 // workgroup runs, or the same rule worked out by every lane group (blocks that are new with every call -- member
 // lists, cgnn_spmm_once: a launch for their table would cost more than the few dependent loads).
 enum { WGRUNS_NONE = 0, WGRUNS_TABLE = 1, WGRUNS_COMPUTED = 2 };
-enum { MODE_VAL = 0, MODE_UNIT = 1, MODE_RELU_MASK = 2, MODE_DUAL = 3, MODE_SIGN_MASK = 4 };
+enum { MODE_VAL = 0, MODE_UNIT = 1, MODE_RELU_MASK = 2, MODE_DUAL = 3, MODE_SIGN_MASK = 4, MODE_ADD = 5 };
+constexpr bool has_values(int mode) { return mode == MODE_VAL || mode == MODE_ADD; }
 
 template <typename T, int VEC>
 struct alignas(sizeof(T) * VEC) Pack {
@@ -322,7 +323,7 @@ struct Acc {
             const Pack<T, VEC> x = g[t].masked(foff[t]);
 #pragma unroll
             for (int i = 0; i < VEC; ++i) {
-                if constexpr (MODE == MODE_VAL || MODE == MODE_DUAL) a0[t].v[i] = a0[t].v[i] + x.v[i] * w;
+                if constexpr (has_values(MODE) || MODE == MODE_DUAL) a0[t].v[i] = a0[t].v[i] + x.v[i] * w;
                 else a0[t].v[i] = a0[t].v[i] + x.v[i];
             }
         }
@@ -339,15 +340,14 @@ struct Acc {
     }
 };
 
-// Y[row] = (accumulate ? Y[row] : 0) + acc
+// Y[row] = (MODE_ADD ? Y[row] : 0) + acc
 template <typename T, int VEC, int TILES, int MODE>
 __device__ __forceinline__ void write_row(T *Y, int64_t F, int row, const int64_t foff[TILES],
-                                          const Acc<T, VEC, TILES, MODE> &acc, int accumulate, T divisor = T(1)) {
+                                          const Acc<T, VEC, TILES, MODE> &acc, T divisor = T(1)) {
     T *yrow = Y + (int64_t)row * F;
-    // Only the plain product (MODE_VAL) can add to an existing Y.  The other modes write every row once, and
-    // knowing that at compile time keeps a load of Y out of the block that closes a row inside a run of the
-    // nnz schedule, where the compiler would have to wait for it on every path behind the block.
-    if constexpr (MODE != MODE_VAL) accumulate = 0;
+    // Whether the row is added to is known at compile time: a load of Y in the block that closes a row inside a run of
+    // the nnz schedule would have to be waited for, with everything asked for before it, on every path behind the block.
+    constexpr bool accumulate = MODE == MODE_ADD;
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
         if (foff[t] < 0) continue;
@@ -363,7 +363,10 @@ __device__ __forceinline__ void write_row(T *Y, int64_t F, int row, const int64_
         if constexpr (MODE == MODE_UNIT)
 #pragma unroll
             for (int i = 0; i < VEC; ++i) o.v[i] = o.v[i] / divisor;
-        if (accumulate) store_pack<T, VEC>(yrow + foff[t], o);
+        // Rows of the plain product that go out element by element are short or no whole lines, and the few of a small
+        // graph are read next: kept (8 features over 4,000 vertices 4.1 us streaming, 3.7 kept; in packs 64
+        // features over 50,001 vertices 12.3 us kept, 11.4 streaming).
+        if constexpr (accumulate || (MODE == MODE_VAL && VEC == 1)) store_pack<T, VEC>(yrow + foff[t], o);
         else store_pack_stream<T, VEC>(yrow + foff[t], o);
     }
 }
@@ -433,7 +436,7 @@ __global__ __launch_bounds__(kBlock) void spmm_row_kernel(SpmmArgs<T> a) {
     Acc<T, VEC, TILES, MODE> acc;
     acc.clear();
     if (e0 == e1) {
-        if (!a.accumulate) write_row<T, VEC, TILES, MODE>(a.Y, a.F, row, foff, acc, 0);
+        if constexpr (MODE != MODE_ADD) write_row<T, VEC, TILES, MODE>(a.Y, a.F, row, foff, acc);
         return;
     }
     if constexpr (sizeof(T) == 4) {
@@ -510,7 +513,7 @@ __global__ __launch_bounds__(kBlock) void spmm_row_kernel(SpmmArgs<T> a) {
                 if (e + u < e1) acc.add(x[u], foff, w[u], c[u] >= a.split);
         }
     }
-    write_row<T, VEC, TILES, MODE>(a.Y, a.F, row, foff, acc, a.accumulate);
+    write_row<T, VEC, TILES, MODE>(a.Y, a.F, row, foff, acc);
 }
 
 // ---------------------------------------------------------------- nnz schedule --
@@ -518,6 +521,26 @@ __global__ __launch_bounds__(kBlock) void spmm_row_kernel(SpmmArgs<T> a) {
 // that falls inside a row of at most K entries is moved back to the start of that row,
 // so such rows are never split (and are summed in the same order as the row schedule);
 // only rows longer than K are cut, at multiples of K.  Runs hold fewer than 2K entries.
+// Says that a loaded value is used here, so that the wait for it stands here and not at its first use.  In the run loop the
+// first uses lie behind branches in which rows are stored; loads and stores are counted together, so a wait there
+// also waits for the store to be acknowledged by memory.  With the waits in front -- one for the entries of a batch, one for
+// the gathers of a round -- the store of a row that ended is under way together with the next round's gathers (forward
+// + gradient with the rules multiplied out, us: 64 features over 50,001 vertices 36.9 -> 34.5, 32 over 100,003 45 -> 44).
+// The two-source product of large graphs is bound by its traffic and took 364 us for 362 so: it keeps the waits where the
+// compiler puts them.
+__device__ __forceinline__ void arrive(int &v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void arrive(uint32_t &v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void arrive(float &v) { asm volatile("" : "+v"(v)); }
+template <typename T, int VEC, int MODE>
+__device__ __forceinline__ void arrive(Gathered<T, VEC, MODE> &g) {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) arrive(g.x.v[i]);
+    if constexpr (MODE == MODE_SIGN_MASK) arrive(g.word), arrive(g.next);
+    if constexpr (MODE == MODE_RELU_MASK)
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) arrive(g.m.v[i]);
+}
+
 template <typename T>
 __device__ __forceinline__ int run_boundary(const SpmmArgs<T> &a, int e) {
     if (e >= a.nnz) return a.nnz;
@@ -553,7 +576,7 @@ __device__ __forceinline__ void join_rows(const SpmmArgs<T> &a, int block, int l
     }
     __syncthreads();
     const int64_t groups = (int64_t)a.blocks * GPB;
-    if (!a.accumulate) {  // rows without entries
+    if constexpr (MODE != MODE_ADD) {  // rows without entries
         const int candidates = a.find_empty ? a.rows : a.n_empty_rows;
 #pragma unroll 1
         for (int64_t item = (int64_t)block * GPB + grp; item < candidates; item += groups) {
@@ -604,12 +627,11 @@ __device__ __forceinline__ void join_rows(const SpmmArgs<T> &a, int block, int l
         for (int t = 0; t < TILES; ++t) {
             if (foff[t] < 0) continue;
             Pack<T, VEC> o = sum[t];
-            if constexpr (MODE == MODE_VAL)
-                if (a.accumulate) {
-                    const Pack<T, VEC> base = load_pack<T, VEC>(y + foff[t]);
+            if constexpr (MODE == MODE_ADD) {
+                const Pack<T, VEC> base = load_pack<T, VEC>(y + foff[t]);
 #pragma unroll
-                    for (int i = 0; i < VEC; ++i) o.v[i] = base.v[i] + o.v[i];
-                }
+                for (int i = 0; i < VEC; ++i) o.v[i] = base.v[i] + o.v[i];
+            }
             store_pack<T, VEC>(y + foff[t], o);
         }
     };
@@ -706,7 +728,7 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
     int seg = block * GPB + grp;
     if constexpr (LPR == kWave) seg = __builtin_amdgcn_readfirstlane(seg);
     int32_t dealt = a.nnz;
-    if constexpr (WGRUNS == WGRUNS_COMPUTED && MODE == MODE_VAL)
+    if constexpr (WGRUNS == WGRUNS_COMPUTED && has_values(MODE))
         if (a.span != nullptr) {
             dealt = a.span[0];
             if (a.val != nullptr) a.val += a.span[1];
@@ -761,7 +783,7 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                 return;
             }
         }
-        write_row<T, VEC, TILES, MODE>(a.Y, a.F, y_row, foff, acc, a.accumulate,
+        write_row<T, VEC, TILES, MODE>(a.Y, a.F, y_row, foff, acc,
                                        MODE == MODE_UNIT && a.mean && !(began_before && row_e0 == e0) ? (T)(end - row_e0) : T(1));
     };
     // the names of rows: see below
@@ -797,10 +819,11 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                 int my_o = 0, my_c = 0;
                 T my_w = T(1);
                 if (e + lane < e1) {
-                    my_o = named(a.rowidx[e + lane]);
+                    const int row = a.rowidx[e + lane];
                     my_c = a.colidx[e + lane];
                     if constexpr (MODE == MODE_DUAL) my_w = a.val[e + lane];
-                    if constexpr (MODE == MODE_VAL) my_w = a.val != nullptr ? a.val[e + lane] : T(1);
+                    if constexpr (has_values(MODE)) my_w = a.val != nullptr ? a.val[e + lane] : T(1);
+                    my_o = named(row);  // behind the others: it waits for the row
                 }
                 if constexpr (kNamesRowsOfY) {
                     // with every batch of entries, so that no load of the run waits for another but
@@ -813,6 +836,8 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                     const int batch_first = __builtin_amdgcn_ds_bpermute(group_lane0, my_o);
                     if (e == e0) cur_out = batch_first;
                 }
+                if constexpr (MODE != MODE_DUAL) arrive(my_o), arrive(my_c);
+                if constexpr (has_values(MODE)) arrive(my_w);
                 const int cnt = min(e1 - e, LPR);
                 for (int u0 = 0; u0 < cnt; u0 += kUnroll) {
                     int o[kUnroll], c[kUnroll];
@@ -822,7 +847,7 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                         const int from = group_lane0 + 4 * (u0 + u);
                         o[u] = __builtin_amdgcn_ds_bpermute(from, my_o);
                         c[u] = __builtin_amdgcn_ds_bpermute(from, my_c);
-                        if constexpr (MODE == MODE_VAL || MODE == MODE_DUAL)
+                        if constexpr (has_values(MODE) || MODE == MODE_DUAL)
                             w[u] = __builtin_bit_cast(T, __builtin_amdgcn_ds_bpermute(from, __builtin_bit_cast(int, my_w)));
                         else
                             w[u] = T(1);
@@ -850,6 +875,11 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                                 for (int t = 0; t < TILES; ++t)
                                     x[u][t] = gather<T, VEC, MODE, (int)(VEC * LPR * sizeof(T))>(a, c[u], kPlain ? 0 : c[u] >= a.split, fld[t]);
                             }
+                        if constexpr (MODE != MODE_DUAL)
+#pragma unroll
+                            for (int u = 0; u < kUnroll; ++u)
+#pragma unroll
+                                for (int t = 0; t < TILES; ++t) arrive(x[u][t]);
 #pragma unroll
                         for (int u = 0; u < kUnroll; ++u) {
                             if (u0 + u < cnt) {
@@ -886,7 +916,7 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                     o[u] = named(a.rowidx[idx]);
                     c[u] = a.colidx[idx];
                     if constexpr (MODE == MODE_DUAL) w[u] = a.val[idx];
-                    else if constexpr (MODE == MODE_VAL) w[u] = a.val != nullptr ? a.val[idx] : T(1);
+                    else if constexpr (has_values(MODE)) w[u] = a.val != nullptr ? a.val[idx] : T(1);
                     else w[u] = T(1);
                 }
 #pragma unroll
@@ -1328,6 +1358,8 @@ int launch_shape(int kind, int mode, const SpmmArgs<T> &args, int64_t items, int
         case KIND_ROW:
             if (mode == MODE_DUAL)
                 hipLaunchKernelGGL((spmm_row_kernel<T, VEC, LPR, TILES, MODE_DUAL>), grid, block, 0, stream, a);
+            else if (a.accumulate)
+                hipLaunchKernelGGL((spmm_row_kernel<T, VEC, LPR, TILES, MODE_ADD>), grid, block, 0, stream, a);
             else
                 hipLaunchKernelGGL((spmm_row_kernel<T, VEC, LPR, TILES, MODE_VAL>), grid, block, 0, stream, a);
             break;
@@ -1335,6 +1367,8 @@ int launch_shape(int kind, int mode, const SpmmArgs<T> &args, int64_t items, int
             if (a.arrivals != nullptr && a.run_start == nullptr) {
                 if (mode == MODE_UNIT)
                     hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_UNIT, WGRUNS_COMPUTED>), grid, block, 0, stream, a);
+                else if (mode == MODE_VAL && a.accumulate)
+                    hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_ADD, WGRUNS_COMPUTED>), grid, block, 0, stream, a);
                 else if (mode == MODE_VAL)
                     hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_VAL, WGRUNS_COMPUTED>), grid, block, 0, stream, a);
                 else if (mode == MODE_SIGN_MASK)
@@ -1343,8 +1377,12 @@ int launch_shape(int kind, int mode, const SpmmArgs<T> &args, int64_t items, int
                     hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_RELU_MASK, WGRUNS_COMPUTED>), grid, block, 0, stream, a);
             } else if (a.arrivals != nullptr && mode == MODE_DUAL)
                 hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_DUAL, WGRUNS_TABLE>), grid, block, 0, stream, a);
+            else if (a.arrivals != nullptr && a.accumulate)
+                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_ADD, WGRUNS_TABLE>), grid, block, 0, stream, a);
             else if (a.arrivals != nullptr)
                 hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_VAL, WGRUNS_TABLE>), grid, block, 0, stream, a);
+            else if (mode == MODE_VAL && a.accumulate)
+                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_ADD, WGRUNS_NONE>), grid, block, 0, stream, a);
             else if (mode == MODE_VAL)
                 hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_VAL, WGRUNS_NONE>), grid, block, 0, stream, a);
             else if (mode == MODE_UNIT)
