@@ -969,63 +969,165 @@ __global__ __launch_bounds__(kBlock) void gather_rows_kernel(GatherArgs<T> a) {
     }
 }
 
-// Both gathers in natural row order over rows that are not whole cache lines (and, for the
-// reconstruct, without sign words): the output is walked as one array of 16-byte packs, so every store instruction of a wave covers 64
+// Both gathers in natural row order over rows that are not whole cache lines: the output is walked as one array of
+// 16-byte packs, so every store instruction of a wave covers 64
 // consecutive packs -- whole 128-byte lines -- wherever the rows begin and end.  A workgroup
 // takes a multiple of 64 rows (a whole number of lines whatever F is), enough of them for
 // every thread to have four packs; pack l of them lies in row l / packs_per_row, by
 // multiplication (exact for l < 2^16).
+//
+// WHOLE: a row is a whole number of packs.  Otherwise a pack may hold the end of one row and the beginning of the next: both
+// are read as a pack of their row (the last VEC elements of the one, the first of the other) and shifted
+// together; such rows went out an element a lane (1,000,003 rows, us: 47 features 76, 48 so; 111 184, 95 so; 300,007 of 254
+// 141, 61 so).
+//
+// Sign words: 64 packs of a wave are 64 * VEC consecutive bits, VEC ballots of them, which eight lanes (at VEC = 4) put in
+// order and leave in LDS; the words of a row are then cut out of the workgroup's string of bits and written side by side
+// (rows without whole lines wrote their words through the row form; 1,000,003 rows, us: 20 features 36, 17.5 so; 47 95, 57
+// so; 100 88 to 104, 69 to 75 so).
 constexpr int kFlatRows = 64;
 constexpr int kFlatItems = 4;  // packs of a thread in flight together
 
-template <typename T, int VEC, int OP>
-__global__ __launch_bounds__(kBlock) void gather_flat_kernel(GatherArgs<T> a, int ppr, uint32_t magic,
+template <typename T, int VEC>
+__device__ __forceinline__ LPack<T, VEC> load_anywhere(const T *p) {
+    typedef T vec_t __attribute__((ext_vector_type(VEC), aligned(sizeof(T))));
+    const vec_t v = *reinterpret_cast<const vec_t *>(p);
+    LPack<T, VEC> x;
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) x.v[i] = v[i];
+    return x;
+}
+
+// elements s ... s + VEC - 1 of the two packs in a row
+template <typename T, int VEC>
+__device__ __forceinline__ LPack<T, VEC> funnel(const LPack<T, VEC> &x, const LPack<T, VEC> &y, int s) {
+    LPack<T, VEC> o = x;
+#pragma unroll
+    for (int k = 1; k < VEC; ++k)
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) o.v[i] = s == k ? (i + k < VEC ? x.v[i + k] : y.v[i + k - VEC]) : o.v[i];
+    return o;
+}
+
+// bit i of the byte to bit VEC * i
+template <int VEC>
+__device__ __forceinline__ uint32_t spread_bits(uint32_t x) {
+    if constexpr (VEC == 4) {
+        x = (x | x << 12) & 0x000f000fu;
+        x = (x | x << 6) & 0x03030303u;
+        return (x | x << 3) & 0x11111111u;
+    } else {  // VEC == 2, sixteen bits
+        x = (x | x << 8) & 0x00ff00ffu;
+        x = (x | x << 4) & 0x0f0f0f0fu;
+        x = (x | x << 2) & 0x33333333u;
+        return (x | x << 1) & 0x55555555u;
+    }
+}
+
+// per: packs of a row (WHOLE), else its elements; magic: floor(2^32 / per) + 1
+template <typename T, int VEC, int OP, bool WHOLE, bool SIGNS>
+__global__ __launch_bounds__(kBlock) void gather_flat_kernel(GatherArgs<T> a, int per, uint32_t magic,
                                                              int rows_per_group) {
+    extern __shared__ uint32_t sign_bits[];  // one bit per element of the workgroup's rows, and a word behind them
     const int64_t row0 = (int64_t)blockIdx.x * rows_per_group;
     const int rows = (int)min((int64_t)rows_per_group, a.N - row0);
-    const int packs = rows * ppr;
-    const LPack<T, VEC> *src = reinterpret_cast<const LPack<T, VEC> *>(a.src);
+    const int F = (int)a.F, total = rows * F;
+    const int packs = WHOLE ? rows * per : (total + VEC - 1) / VEC;
     T *out = a.out + row0 * a.F;
-    for (int l0 = threadIdx.x; l0 < packs; l0 += kFlatItems * kBlock) {
-        int col[kFlatItems];
-        int64_t g[kFlatItems];
+    const int64_t *ids = a.ids + row0;
+    // an id that names no row of src is moved to the nearest row that exists and reported
+    auto check = [&](int64_t &g) {
+        if (g < 0 || g >= a.groups) {
+            g = g < 0 ? 0 : a.groups - 1;
+            if (a.bad_id) *a.bad_id = 1;  // every writer stores the same value
+        }
+    };
+    LPack<T, VEC> bias_begin;
+    if constexpr (OP == GATHER_RECONSTRUCT && !WHOLE)
+        if (a.bias) bias_begin = load_anywhere<T, VEC>(a.bias);
+    // without ballots a thread is done with its last pack
+    for (int l0 = threadIdx.x; SIGNS ? l0 - (int)threadIdx.x < packs : l0 < packs; l0 += kFlatItems * kBlock) {
+        // first element in its row (WHOLE: pack); how many of the pack's elements belong to the next row
+        int col[kFlatItems], cut[kFlatItems];
+        int64_t g[kFlatItems], h[kFlatItems];
 #pragma unroll
         for (int u = 0; u < kFlatItems; ++u) {
             const int l = min(l0 + u * kBlock, packs - 1);
-            const int r = (int)__umulhi((uint32_t)l, magic);
-            col[u] = l - r * ppr;
-            g[u] = a.ids[row0 + r];
+            const int r = (int)__umulhi((uint32_t)(WHOLE ? l : l * VEC), magic);
+            col[u] = (WHOLE ? l : l * VEC) - r * per;
+            cut[u] = WHOLE ? 0 : max(0, col[u] + VEC - F);
+            g[u] = ids[r];
+            if constexpr (!WHOLE) h[u] = ids[min(r + 1, rows - 1)];
         }
-        T denom[kFlatItems];
-        LPack<T, VEC> x[kFlatItems];
+        T denom[kFlatItems], denom_next[kFlatItems];
+        LPack<T, VEC> x[kFlatItems], y[kFlatItems];
 #pragma unroll
         for (int u = 0; u < kFlatItems; ++u) {
-            // an id that names no row of src is moved to the nearest row that exists and reported
-            if (g[u] < 0 || g[u] >= a.groups) {
-                g[u] = g[u] < 0 ? 0 : a.groups - 1;
-                if (a.bad_id) *a.bad_id = 1;  // every writer stores the same value
-            }
+            check(g[u]);
             if constexpr (OP == GATHER_MEAN_GRAD) denom[u] = (T)max(a.counts[g[u]], 1);
-            x[u] = src[g[u] * ppr + col[u]];
+            if constexpr (WHOLE) x[u] = reinterpret_cast<const LPack<T, VEC> *>(a.src)[g[u] * per + col[u]];
+            else x[u] = load_anywhere<T, VEC>(a.src + g[u] * a.F + (col[u] - cut[u]));
+            if constexpr (!WHOLE)
+                if (cut[u] > 0) {
+                    check(h[u]);
+                    y[u] = load_anywhere<T, VEC>(a.src + h[u] * a.F);
+                    if constexpr (OP == GATHER_MEAN_GRAD) denom_next[u] = (T)max(a.counts[h[u]], 1);
+                }
         }
 #pragma unroll
         for (int u = 0; u < kFlatItems; ++u) {
             const int l = l0 + u * kBlock;
-            if (l >= packs) break;
+            const bool on = l < packs;
+            LPack<T, VEC> o = x[u];
+            if constexpr (!WHOLE) o = funnel<T, VEC>(x[u], y[u], cut[u]);
             if constexpr (OP == GATHER_MEAN_GRAD) {
 #pragma unroll
-                for (int i = 0; i < VEC; ++i) x[u].v[i] = x[u].v[i] / denom[u];
+                for (int i = 0; i < VEC; ++i) o.v[i] = o.v[i] / (!WHOLE && i >= VEC - cut[u] ? denom_next[u] : denom[u]);
             } else {
-                LPack<T, VEC> b;
-                if (a.bias) b = reinterpret_cast<const LPack<T, VEC> *>(a.bias)[col[u]];
+                if (a.bias) {
+                    LPack<T, VEC> b;
+                    if constexpr (WHOLE) b = reinterpret_cast<const LPack<T, VEC> *>(a.bias)[col[u]];
+                    else b = funnel<T, VEC>(load_anywhere<T, VEC>(a.bias + (col[u] - cut[u])), bias_begin, cut[u]);
 #pragma unroll
-                for (int i = 0; i < VEC; ++i) {
-                    T v = x[u].v[i];
-                    if (a.bias) v = v + b.v[i];
-                    x[u].v[i] = (a.relu && v < T(0)) ? T(0) : v;
+                    for (int i = 0; i < VEC; ++i) o.v[i] = o.v[i] + b.v[i];
+                }
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) o.v[i] = (a.relu && o.v[i] < T(0)) ? T(0) : o.v[i];
+                if constexpr (SIGNS) {
+                    unsigned long long kept[VEC];
+#pragma unroll
+                    for (int i = 0; i < VEC; ++i) kept[i] = __ballot(on && !(o.v[i] <= T(0)));
+                    // lane k < 2 * VEC: word k of the wave's 64 * VEC bits
+                    const int lane = threadIdx.x % kWave, word = (l - lane) * VEC / 32 + lane;
+                    uint32_t w = 0;
+#pragma unroll
+                    for (int i = 0; i < VEC; ++i)
+                        w |= spread_bits<VEC>((uint32_t)(kept[i] >> (lane % (2 * VEC) * (32 / VEC))) & ((1u << 32 / VEC) - 1)) << i;
+                    if (lane < 2 * VEC && 32 * word < total) sign_bits[word] = w;
                 }
             }
-            store_stream<T, VEC>(out + (int64_t)l * VEC, x[u]);
+            if constexpr (!SIGNS)
+                if (!on) break;
+            if (!on) continue;  // the ballots want all lanes
+            if (WHOLE || (l + 1) * VEC <= total) {
+                store_stream<T, VEC>(out + (int64_t)l * VEC, o);
+            } else {  // the last pack of the array ends inside
+#pragma unroll
+                for (int i = 0; i < VEC; ++i)
+                    if (l * VEC + i < total) out[(int64_t)l * VEC + i] = o.v[i];
+            }
+        }
+    }
+    if constexpr (SIGNS) {
+        __syncthreads();
+        const int words = rows * a.sign_words;
+        uint32_t *signs = a.signs + row0 * a.sign_words;
+        const int last = (total - 1) / 32;
+        for (int i = threadIdx.x; i < words; i += kBlock) {
+            const int r = i / a.sign_words, w = i - r * a.sign_words;
+            const int bit = r * F + 32 * w, left = F - 32 * w;
+            const uint32_t v = __builtin_amdgcn_alignbit(sign_bits[min(bit / 32 + 1, last)], sign_bits[bit / 32], (uint32_t)bit % 32u);
+            signs[i] = left < 32 ? v & ((1u << left) - 1u) : v;
         }
     }
 }
@@ -1056,14 +1158,34 @@ int launch_gather(const GatherArgs<T> &a, hipStream_t stream) {
     constexpr int WIDE = 16 / sizeof(T);
     auto al = [](const void *p) { return p == nullptr || reinterpret_cast<uintptr_t>(p) % 16 == 0; };
     const bool wide = a.F % WIDE == 0 && al(a.src) && al(a.out) && al(a.bias);
-    const int64_t ppr = a.F / WIDE;
-    if (wide && a.perm == nullptr && a.signs == nullptr && (a.F * (int64_t)sizeof(T)) % 128 != 0 && ppr > 1 &&
-        kFlatRows * ppr < (1 << 16) && ceil_div(a.N, kFlatRows) < ((int64_t)1 << 31)) {
-        const uint32_t magic = (uint32_t)((1ull << 32) / (uint32_t)ppr) + 1u;
-        // 64 rows, or as many times 64 as give the threads their four packs each
-        const int rows = kFlatRows * (int)std::max<int64_t>(1, kFlatItems * kBlock / (kFlatRows * ppr));
-        hipLaunchKernelGGL((gather_flat_kernel<T, WIDE, OP>), dim3((unsigned)ceil_div(a.N, rows)), dim3(kBlock), 0,
-                           stream, a, (int)ppr, magic, rows);
+    // Rows that are whole lines go row by row, in the order of the member lists where there is one; the others as one
+    // array, which begins on a line.  Packs that span two rows take a second id and a second load, which pays from some
+    // 16 MB on (us, row by row / as one array: 30,011 rows of 47 features 4.9 / 5.1, of 111 6.5 / 6.9, 100,003 of 47 10.3
+    // / 8.2), and sign words of whole packs from some 200,000 rows on (100,003 rows of 100 11.0 / 12.5, 300,007 31 / 25).
+    const int64_t ppr = ceil_div(a.F, WIDE), per = wide ? ppr : a.F;
+    const bool pays = wide ? a.signs == nullptr || a.N >= 200000 : a.N * a.F * (int64_t)sizeof(T) >= ((int64_t)1 << 24);
+    if (pays && a.perm == nullptr && (a.F * (int64_t)sizeof(T)) % 128 != 0 && a.F >= WIDE && per > 1 && al(a.out) &&
+        kFlatRows * per < (1 << 16) && ceil_div(a.N, kFlatRows) < ((int64_t)1 << 31)) {
+        const uint32_t magic = (uint32_t)((1ull << 32) / (uint32_t)per) + 1u;
+        // 64 rows, or as many times 64 as give the threads their four packs each; where that is fewer than four workgroups
+        // per compute unit, as many rows as give a thread four packs or fewer, a multiple of four (which begins on a
+        // pack): 2,708 rows of 100 features 3.9 us with 64 rows, 3.1 with 40; 30,011 of 188 6.9 and 5.9.
+        int rows = kFlatRows * (int)std::max<int64_t>(1, kFlatItems * kBlock / (kFlatRows * ppr));
+        if (ceil_div(a.N, rows) < 4 * (int64_t)compute_units()) rows = std::max(4, (int)(kFlatItems * kBlock / ppr) / 4 * 4);
+        const size_t lds = a.signs != nullptr ? ((size_t)rows * a.F / 32 + 2) * sizeof(uint32_t) : 0;
+        const dim3 grid((unsigned)ceil_div(a.N, rows)), block(kBlock);
+        if constexpr (OP == GATHER_RECONSTRUCT)
+            if (a.signs != nullptr) {
+                if (wide)
+                    hipLaunchKernelGGL((gather_flat_kernel<T, WIDE, OP, true, true>), grid, block, lds, stream, a, (int)per, magic, rows);
+                else
+                    hipLaunchKernelGGL((gather_flat_kernel<T, WIDE, OP, false, true>), grid, block, lds, stream, a, (int)per, magic, rows);
+                return check_launch("gather_flat");
+            }
+        if (wide)
+            hipLaunchKernelGGL((gather_flat_kernel<T, WIDE, OP, true, false>), grid, block, 0, stream, a, (int)per, magic, rows);
+        else
+            hipLaunchKernelGGL((gather_flat_kernel<T, WIDE, OP, false, false>), grid, block, 0, stream, a, (int)per, magic, rows);
         return check_launch("gather_flat");
     }
     if (wide) return launch_gather_lpr<T, WIDE, OP>(a, stream);

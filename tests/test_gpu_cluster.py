@@ -141,6 +141,36 @@ def test_assign_shapes(width, bits):
     assert np.array_equal(counts.cpu().numpy(), want_counts)
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("width", [4, 5, 7, 20, 33, 47, 100, 111, 254, 255])
+def test_gathers_as_one_array(width, dtype):
+    """The gathers whose output is walked as one array: rows that are whole packs and others (a pack then holds the end of a row and
+    the beginning of the next, the last one of the array ends inside), with and without sign words, values that are NaN and
+    zeros of both signs, enough rows that the form is taken; a view that begins inside a pack takes the other form."""
+    n, groups = max(200003, 2 ** 22 // width + 5), 301
+    rng = np.random.default_rng(width)
+    ids = rng.integers(0, groups, n)
+    counts = np.bincount(ids, minlength=groups).astype(np.int32)
+    src = rng.standard_normal((groups, width)).astype(dtype)
+    src[::7, ::3], src[1::7, ::5], src[2::7, width - 1] = 0.0, -0.0, np.nan
+    bias = rng.standard_normal(width).astype(dtype)
+    bias[::4] = 0.0
+    dsrc, dids, dcounts = _t(src), _t(ids), _t(counts)
+    assert np.array_equal(abi.cluster_mean_backward(dsrc, dids, dcounts).cpu().numpy(),
+                          oracle.cluster_mean_backward(src, ids, counts), equal_nan=True)
+    shifted = torch.empty(groups * width + 1, dtype=dsrc.dtype, device=DEV)[1:].view(groups, width)
+    shifted.copy_(dsrc)
+    for b in (None, bias):
+        db = None if b is None else _t(b)
+        want = oracle.reconstruct(src, ids, b, False)
+        assert np.array_equal(abi.reconstruct(dsrc, dids, db, False).cpu().numpy(), want, equal_nan=True)
+        assert np.array_equal(abi.reconstruct(shifted, dids, db, False).cpu().numpy(), want, equal_nan=True)
+        want = oracle.reconstruct(src, ids, b, True)
+        rows, signs = abi.reconstruct_signs(dsrc, dids, db, None)
+        assert np.array_equal(rows.cpu().numpy(), want, equal_nan=True)
+        assert np.array_equal(signs.cpu().numpy(), pack_signs(want))
+
+
 @pytest.mark.parametrize("width,bits", [(100, 16), (64, 16), (128, 20)])
 def test_assign_many_tiles_a_wave(width, bits):
     """A million rows: every wave of the projection kernel takes some six to ten tiles from
