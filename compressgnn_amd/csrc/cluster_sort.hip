@@ -1,8 +1,8 @@
 // Member lists of the clusters: rows sorted by cluster id, ties in ascending row order.
 //
 // The sort is a stable LSD radix sort written for this job (8-bit digits, keys of at most 30
-// bits, the row number as payload): per pass a digit histogram per tile of 4,096 keys, a scan
-// of the histograms, and a scatter that ranks the keys of a tile in index order with wave
+// bits, the row number as payload): per pass a digit histogram per tile of 1,024 to 4,096 keys, a
+// scan of the histograms (few tiles: in the scatter), and a scatter that ranks the keys of a tile in index order with wave
 // ballots, so the order of equal keys is kept without any atomic on global memory.  The first
 // pass takes the row numbers from the positions (no index array is written or read first).
 // It runs once per assignment refresh, not per training step.
@@ -24,22 +24,43 @@ namespace {
 // ------------------------------------------------------------------- radix sort --
 constexpr int kDigitBits = 8;
 constexpr int kDigits = 1 << kDigitBits;           // one per thread of a workgroup
-constexpr int kSortItems = 16;                     // keys per thread
-constexpr int kSortTile = kBlock * kSortItems;     // keys per workgroup
 static_assert(kDigits == kBlock, "one digit per thread");
+
+// How the keys are dealt out: `items` per thread of a workgroup's tile, and whether the workgroups of a scatter add up the
+// histograms of the tiles for themselves (`own_scan`) or a launch in between does.  Up to 128 tiles the former costs four
+// rounds of loads that hit the L2s, no more than the launch and its dependence; few keys take small tiles, since a
+// tile is ranked 64 keys a wave and step, one step after the other, and 4,096 keys a tile leave most of the card idle.
+// Hashing and grouping rows of 24 columns by 16 planes, us, with tiles of 4,096, a launch for the scan and a copy of
+// the group count / so: 9,000 rows 76 / 58, 30,011 73 / 58, 100,003 74 / 66, 200,000 77 / 71, 300,007 79 / 81,
+// 450,000 86 / 89 (kernels alone at 300,007: 69 / 65).  More keys keep the launch and the large tiles:
+// 2,048 a tile 0.301 against 0.293 ms for a refresh of 2.4 M rows.
+struct SortShape {
+    int items, tiles;
+    bool own_scan;
+};
+
+constexpr int kOwnScanTiles = 128;
+
+SortShape sort_shape(int64_t N) {
+    const int64_t n = N < 1 ? 1 : N;
+    for (int items = 4; items <= 16; items *= 2)
+        if (ceil_div(n, (int64_t)items * kBlock) <= kOwnScanTiles) return {items, (int)ceil_div(n, (int64_t)items * kBlock), true};
+    return {16, (int)ceil_div(n, (int64_t)16 * kBlock), false};
+}
 
 __device__ __forceinline__ int digit_of(int32_t key, int shift) { return (key >> shift) & (kDigits - 1); }
 
-// hist[d * tiles + tile] = number of keys of the tile with digit d (digit-major: the scan over a
-// digit's tiles is a scan over consecutive entries).  THREADS: the workgroup's size, a multiple
-// of kDigits; the loads of a thread are all issued before the first count.
-template <int THREADS>
+// The number of keys of the tile with digit d: hist[d * tiles + tile], digit-major, since the scan over a
+// digit's tiles is a scan over consecutive entries; hist[tile * kDigits + d] where the scatter adds them up itself, a thread
+// per digit (ITEMS: keys per thread of a workgroup of kBlock; own_scan: as in SortShape).  THREADS: the workgroup's size, a multiple
+// of kBlock.
+template <int THREADS, int ITEMS>
 __device__ __forceinline__ void tile_histogram(const int32_t *__restrict__ keys, int64_t N, int shift,
-                                               int32_t *__restrict__ hist, int tiles, int tile, int *count) {
-    constexpr int kItems = kSortTile / THREADS;
+                                               int32_t *__restrict__ hist, int tiles, bool own_scan, int tile, int *count) {
+    constexpr int kTile = ITEMS * kBlock, kItems = (kTile + THREADS - 1) / THREADS;
     if (threadIdx.x < kDigits) count[threadIdx.x] = 0;
     __syncthreads();
-    const int64_t base = (int64_t)tile * kSortTile;
+    const int64_t base = (int64_t)tile * kTile;
     int32_t key[kItems];
 #pragma unroll
     for (int it = 0; it < kItems; ++it) {
@@ -52,19 +73,24 @@ __device__ __forceinline__ void tile_histogram(const int32_t *__restrict__ keys,
         if (i < N) atomicAdd(&count[digit_of(key[it], shift)], 1);  // LDS, integer: the sum does not depend on the order
     }
     __syncthreads();
-    if (threadIdx.x < kDigits) hist[(int64_t)threadIdx.x * tiles + tile] = count[threadIdx.x];
+    if (threadIdx.x < kDigits)
+        hist[own_scan ? (int64_t)tile * kDigits + threadIdx.x : (int64_t)threadIdx.x * tiles + tile] = count[threadIdx.x];
 }
 
 // `clear` (optional, first pass): a table of clear_n entries that this launch sets to zero, for
-// the scatter of the same pass to mark.
+// the scatter of the same pass to mark; `state` (optional): kGroupState counters likewise.
+constexpr int kGroupState = 4;
+
+template <int ITEMS>
 __global__ __launch_bounds__(kBlock) void radix_hist_kernel(const int32_t *__restrict__ keys, int64_t N, int shift,
-                                                           int32_t *__restrict__ hist, int tiles,
-                                                           int32_t *__restrict__ clear, int clear_n) {
+                                                           int32_t *__restrict__ hist, int tiles, bool own_scan,
+                                                           int32_t *__restrict__ clear, int clear_n, int32_t *__restrict__ state) {
     __shared__ int count[kDigits];
     if (clear)
         for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < clear_n; i += (int64_t)gridDim.x * kBlock)
             clear[i] = 0;
-    tile_histogram<kBlock>(keys, N, shift, hist, tiles, blockIdx.x, count);
+    if (state && blockIdx.x == 0 && threadIdx.x < kGroupState) state[threadIdx.x] = 0;
+    tile_histogram<kBlock, ITEMS>(keys, N, shift, hist, tiles, own_scan, blockIdx.x, count);
 }
 
 // One wave per digit: within[d * tiles + t] = keys with digit d in the tiles before t, and
@@ -113,6 +139,8 @@ __device__ __forceinline__ unsigned long long same_digit(int d, unsigned long lo
 // every key, the table the dense ranks of the hash codes are made from (the mask keeps a code
 // beyond the table, a caller's mistake, inside it).  `remap` (optional, last pass): the keys are
 // written as remap[key & seen_mask], an order-preserving renaming (the rank of the code).
+// OWN_SCAN: `within` holds the tiles' histograms (tile_histogram), `total` is not read.
+template <int ITEMS, bool OWN_SCAN>
 __global__ __launch_bounds__(kBlock) void radix_scatter_kernel(const int32_t *__restrict__ keys,
                                                               const int32_t *__restrict__ vals, int64_t N, int shift,
                                                               const int32_t *__restrict__ within,
@@ -122,31 +150,48 @@ __global__ __launch_bounds__(kBlock) void radix_scatter_kernel(const int32_t *__
                                                               int32_t *__restrict__ seen, int seen_mask,
                                                               const int32_t *__restrict__ remap) {
     constexpr int kWaves = kBlock / kWave;
-    constexpr int kPerWave = kSortTile / kWaves;
+    constexpr int kTile = ITEMS * kBlock, kPerWave = kTile / kWaves;
     __shared__ int digit_start[kDigits];         // output position of the tile's first key of a digit, minus tile_start
     __shared__ int tile_start[kDigits];          // position of that key in the ordered tile
     __shared__ int wave_count[kWaves][kDigits];  // keys of a digit seen by a wave so far; then: by the waves before it
     __shared__ int scan_tmp[2][kWaves];
-    __shared__ int32_t tile_key[kSortTile], tile_val[kSortTile];
+    __shared__ int32_t tile_key[kTile], tile_val[kTile];
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-    const int mine = total[threadIdx.x];  // thread = digit
-    const int my_within = within[(int64_t)threadIdx.x * tiles + blockIdx.x];
+    int mine = 0, my_within = 0;  // thread = digit
+    if constexpr (!OWN_SCAN) {
+        mine = total[threadIdx.x];
+        my_within = within[(int64_t)threadIdx.x * tiles + blockIdx.x];
+    }
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) wave_count[w][threadIdx.x] = 0;
     __syncthreads();
-    const int64_t base = (int64_t)blockIdx.x * kSortTile + (int64_t)wave * kPerWave;
-    int32_t key[kSortItems], val[kSortItems];
-    int rank[kSortItems];
+    const int64_t base = (int64_t)blockIdx.x * kTile + (int64_t)wave * kPerWave;
+    int32_t key[ITEMS], val[ITEMS];
+    int rank[ITEMS];
     const unsigned long long below = (1ull << lane) - 1ull;
 #pragma unroll
-    for (int it = 0; it < kSortItems; ++it) {
+    for (int it = 0; it < ITEMS; ++it) {
         const int64_t i = base + (int64_t)it * kWave + lane;
         const bool live = i < N;
         key[it] = live ? keys[i] : 0;
         val[it] = live ? (vals ? vals[i] : (int32_t)i) : 0;
     }
+    if constexpr (OWN_SCAN) {
+        constexpr int kBatch = 32;
+#pragma unroll 1
+        for (int t0 = 0; t0 < tiles; t0 += kBatch) {
+            int v[kBatch];
 #pragma unroll
-    for (int it = 0; it < kSortItems; ++it) {
+            for (int u = 0; u < kBatch; ++u) v[u] = within[min(t0 + u, tiles - 1) * kDigits + threadIdx.x];
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+                mine += t0 + u < tiles ? v[u] : 0;
+                my_within += t0 + u < (int)blockIdx.x ? v[u] : 0;
+            }
+        }
+    }
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it) {
         const int64_t i = base + (int64_t)it * kWave + lane;
         const bool live = i < N;
         const int d = digit_of(key[it], shift);
@@ -199,7 +244,7 @@ __global__ __launch_bounds__(kBlock) void radix_scatter_kernel(const int32_t *__
     }
     __syncthreads();
 #pragma unroll
-    for (int it = 0; it < kSortItems; ++it) {
+    for (int it = 0; it < ITEMS; ++it) {
         const int64_t i = base + (int64_t)it * kWave + lane;
         if (i < N) {
             const int d = digit_of(key[it], shift);
@@ -209,10 +254,10 @@ __global__ __launch_bounds__(kBlock) void radix_scatter_kernel(const int32_t *__
         }
     }
     __syncthreads();
-    const int64_t left = N - (int64_t)blockIdx.x * kSortTile;
-    const int in_this_tile = left < kSortTile ? (int)left : kSortTile;
+    const int64_t left = N - (int64_t)blockIdx.x * kTile;
+    const int in_this_tile = left < kTile ? (int)left : kTile;
 #pragma unroll
-    for (int it = 0; it < kSortItems; ++it) {
+    for (int it = 0; it < ITEMS; ++it) {
         const int at = it * kBlock + threadIdx.x;
         if (at < in_this_tile) {
             const int32_t k = tile_key[at];
@@ -224,11 +269,12 @@ __global__ __launch_bounds__(kBlock) void radix_scatter_kernel(const int32_t *__
 }
 
 int radix_passes(int bits) { return bits <= kDigitBits ? 1 : (bits + kDigitBits - 1) / kDigitBits; }
-int64_t radix_tiles(int64_t N) { return ceil_div(N < 1 ? 1 : N, kSortTile); }
 
-// hist, within (kDigits x tiles each) and total (kDigits)
+// hist, within (kDigits x tiles each) and total (kDigits); never less than fewer keys take, which may be dealt in more tiles
 size_t radix_counter_bytes(int64_t N) {
-    return 2 * align_up((size_t)kDigits * (size_t)radix_tiles(N) * sizeof(int32_t), 256) + align_up(kDigits * sizeof(int32_t), 256);
+    const int64_t small_tiles = std::min<int64_t>(ceil_div(N, (int64_t)4 * kBlock), kOwnScanTiles);
+    const int64_t tiles = std::max<int64_t>(sort_shape(N).tiles, small_tiles);
+    return 2 * align_up((size_t)kDigits * (size_t)tiles * sizeof(int32_t), 256) + align_up(kDigits * sizeof(int32_t), 256);
 }
 
 // ------------------------------------------------------------------ member lists --
@@ -377,9 +423,10 @@ __global__ __launch_bounds__(kRankThreads) void code_rank_kernel(int32_t *__rest
 // The histograms of a later pass and the ranks of the codes in one launch: neither needs the
 // other, both need the scatter of the first pass (its keys; the codes it has marked), and the
 // sixteen workgroups of the ranks are over before the histograms are.
+template <int ITEMS>
 __global__ __launch_bounds__(kRankThreads) void radix_hist_rank_kernel(const int32_t *__restrict__ keys, int64_t N,
                                                                        int shift, int32_t *__restrict__ hist, int tiles,
-                                                                       int32_t *__restrict__ table, int codes,
+                                                                       bool own_scan, int32_t *__restrict__ table, int codes,
                                                                        int32_t *__restrict__ summary) {
     __shared__ int count[kDigits];
     __shared__ int wave_before[kRankWaves], wave_mine[kRankWaves];
@@ -387,7 +434,7 @@ __global__ __launch_bounds__(kRankThreads) void radix_hist_rank_kernel(const int
     if ((int)blockIdx.x < parts)  // first, so that they are not the tail of the launch
         code_rank_stretch(table, codes, summary, blockIdx.x, parts, wave_before, wave_mine);
     else
-        tile_histogram<kRankThreads>(keys, N, shift, hist, tiles, (int)blockIdx.x - parts, count);
+        tile_histogram<kRankThreads, ITEMS>(keys, N, shift, hist, tiles, own_scan, (int)blockIdx.x - parts, count);
 }
 
 // Stable sort of (keys[i], i) by the low `bits` bits of the keys into (keys_out, vals_out).
@@ -397,17 +444,16 @@ __global__ __launch_bounds__(kRankThreads) void radix_hist_rank_kernel(const int
 // a single pass, else part of the second pass's histogram launch) then turns it into the ranks
 // of the keys (summary as there), and with more than one pass the last pass writes the ranks
 // in place of the keys (*ranked = true).
-int radix_sort_by_key(const int32_t *keys, int64_t N, int bits, int32_t *keys_out, int32_t *vals_out, int32_t *tmp_keys,
-                      int32_t *tmp_vals, void *counters, int32_t *table, int seen_mask, int32_t *summary, bool *ranked,
-                      hipStream_t stream) {
-    if (ranked) *ranked = false;
-    if (N <= 0) return CGNN_OK;
+// state (optional): kGroupState counters that the first launch clears.
+template <int ITEMS, bool OWN_SCAN>
+int radix_sort_tiles(const int32_t *keys, int64_t N, int bits, int32_t *keys_out, int32_t *vals_out, int32_t *tmp_keys,
+                     int32_t *tmp_vals, void *counters, int32_t *table, int seen_mask, int32_t *summary, bool *ranked, int32_t *state,
+                     int tiles, hipStream_t stream) {
     const int passes = radix_passes(bits);
-    const int tiles = (int)radix_tiles(N);
     char *cbase = static_cast<char *>(counters);
     const size_t tbytes = align_up((size_t)kDigits * (size_t)tiles * sizeof(int32_t), 256);
     int32_t *hist = reinterpret_cast<int32_t *>(cbase);
-    int32_t *within = reinterpret_cast<int32_t *>(cbase + tbytes);
+    int32_t *within = OWN_SCAN ? hist : reinterpret_cast<int32_t *>(cbase + tbytes);
     int32_t *total = reinterpret_cast<int32_t *>(cbase + 2 * tbytes);
     const int32_t *in_keys = keys, *in_vals = nullptr;
     for (int p = 0; p < passes; ++p) {
@@ -420,15 +466,16 @@ int radix_sort_by_key(const int32_t *keys, int64_t N, int bits, int32_t *keys_ou
         const int rank_parts = (int)ceil_div(seen_mask + 1, kRankStretch);
         const bool rank_here = table && p == 1;  // the marks are complete after the first scatter
         if (rank_here)
-            hipLaunchKernelGGL(radix_hist_rank_kernel, dim3((unsigned)(tiles + rank_parts)), dim3(kRankThreads), 0,
-                               stream, in_keys, N, shift, hist, tiles, table, seen_mask + 1, summary);
+            hipLaunchKernelGGL(radix_hist_rank_kernel<ITEMS>, dim3((unsigned)(tiles + rank_parts)), dim3(kRankThreads), 0,
+                               stream, in_keys, N, shift, hist, tiles, OWN_SCAN, table, seen_mask + 1, summary);
         else
-            hipLaunchKernelGGL(radix_hist_kernel, dim3((unsigned)tiles), dim3(kBlock), 0, stream, in_keys, N, shift,
-                               hist, tiles, first ? table : nullptr, seen_mask + 1);
-        hipLaunchKernelGGL(radix_scan_kernel, dim3(kDigits / (kBlock / kWave)), dim3(kBlock), 0, stream, hist, tiles,
-                           within, total);
-        hipLaunchKernelGGL(radix_scatter_kernel, dim3((unsigned)tiles), dim3(kBlock), 0, stream, in_keys, in_vals, N,
-                           shift, within, total, tiles, out_keys, out_vals, first ? table : nullptr, seen_mask, remap);
+            hipLaunchKernelGGL(radix_hist_kernel<ITEMS>, dim3((unsigned)tiles), dim3(kBlock), 0, stream, in_keys, N, shift,
+                               hist, tiles, OWN_SCAN, first ? table : nullptr, seen_mask + 1, first ? state : nullptr);
+        if (!OWN_SCAN)
+            hipLaunchKernelGGL(radix_scan_kernel, dim3(kDigits / (kBlock / kWave)), dim3(kBlock), 0, stream, hist, tiles,
+                               within, total);
+        hipLaunchKernelGGL((radix_scatter_kernel<ITEMS, OWN_SCAN>), dim3((unsigned)tiles), dim3(kBlock), 0, stream, in_keys, in_vals,
+                           N, shift, within, total, tiles, out_keys, out_vals, first ? table : nullptr, seen_mask, remap);
         if (table && first && last)  // with a second pass its histogram launch makes the ranks
             hipLaunchKernelGGL(code_rank_kernel, dim3((unsigned)rank_parts), dim3(kRankThreads), 0, stream, table,
                                seen_mask + 1, summary);
@@ -437,6 +484,19 @@ int radix_sort_by_key(const int32_t *keys, int64_t N, int bits, int32_t *keys_ou
         in_vals = out_vals;
     }
     return check_launch("radix_sort");
+}
+
+int radix_sort_by_key(const int32_t *keys, int64_t N, int bits, int32_t *keys_out, int32_t *vals_out, int32_t *tmp_keys,
+                      int32_t *tmp_vals, void *counters, int32_t *table, int seen_mask, int32_t *summary, bool *ranked,
+                      int32_t *state, hipStream_t stream) {
+    if (ranked) *ranked = false;
+    if (N <= 0) return CGNN_OK;
+    const SortShape s = sort_shape(N);
+    const auto sort = !s.own_scan ? radix_sort_tiles<16, false>
+                                  : (s.items == 4 ? radix_sort_tiles<4, true>
+                                                  : (s.items == 8 ? radix_sort_tiles<8, true> : radix_sort_tiles<16, true>));
+    return sort(keys, N, bits, keys_out, vals_out, tmp_keys, tmp_vals, counters, table, seen_mask, summary, ranked, state, s.tiles,
+                stream);
 }
 
 // The rest of an assignment from the rank table: ids in row order; in sorted order the id of
@@ -483,11 +543,23 @@ __global__ __launch_bounds__(kBlock) void group_table_finish_kernel(int64_t N, c
     }
 }
 
-// summary[0] = number of groups, summary[1] = largest group (cleared before this kernel).
-__global__ void group_counts_kernel(const int32_t *__restrict__ offsets, int32_t *__restrict__ summary,
-                                    int32_t *__restrict__ counts, int64_t capacity) {
-    const int64_t groups = min((int64_t)summary[0], capacity) + 1;
+// The number of groups and the size of the largest, which may lie in pinned host memory: the number is written last, and a
+// host that finds it there finds both.  Two stores past the caches with a wait between: a release would write back the
+// whole L2.
+__device__ __forceinline__ void write_summary(int32_t *summary, int32_t groups, int32_t largest) {
+    __hip_atomic_store(summary + 1, largest, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0);
+    __hip_atomic_store(summary, groups, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// state[0] = number of groups; state[1] and state[2] are zero: the largest group so far, and the workgroups that are done.
+// The last of them writes the summary.
+__global__ void group_counts_kernel(const int32_t *__restrict__ offsets, int32_t *__restrict__ state,
+                                    int32_t *__restrict__ counts, int64_t capacity, int32_t *__restrict__ summary) {
+    const int64_t found = state[0], groups = min(found, capacity) + 1;
     int largest = 0;
+#pragma unroll 4
     for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < groups;
          g += (int64_t)gridDim.x * blockDim.x) {
         const int c = g == 0 ? 0 : offsets[g + 1] - offsets[g];
@@ -502,12 +574,20 @@ __global__ void group_counts_kernel(const int32_t *__restrict__ offsets, int32_t
     if (threadIdx.x == 0) {
 #pragma unroll
         for (int w = 1; w < kBlock / kWave; ++w) largest = max(largest, wave_largest[w]);
-        if (largest > 0) atomicMax(summary + 1, largest);  // one per workgroup: integer maximum, any order
+        // one per workgroup: integer maximum, any order
+        if (largest > 0) __hip_atomic_fetch_max(state + 1, largest, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // the maximum has reached memory before the arrival is counted
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_waitcnt(0);
+        const int done = __hip_atomic_fetch_add(state + 2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (done == (int)gridDim.x - 1) {
+            write_summary(summary, (int32_t)found, __hip_atomic_load(state + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        }
     }
 }
 
 // The whole grouping of a small assignment in one workgroup: the sort, the ids, the member lists, the sizes
-// and the summary (which may lie in pinned host memory: plain stores).  The passes above are eight
+// and the summary.  The passes above are six
 // launches of 2 to 9 us each whatever they hold; this one takes 11 us for 2,708 rows and 8 bits.  Up to
 // kSmallRows rows: keys and row numbers of two passes then fit the LDS of a compute unit, and a key is ranked
 // eight steps into its wave's share.
@@ -643,15 +723,14 @@ __global__ __launch_bounds__(kSmallThreads) void group_small_kernel(const int32_
         offsets[0] = 0;
         counts[0] = 0;
         offsets[groups + 1] = N;
-        summary[0] = groups;
-        summary[1] = largest;
+        write_summary(summary, groups, largest);
     }
 }
 
 __global__ void group_empty_kernel(int32_t *offsets, int32_t *counts, int32_t *summary) {
     offsets[0] = offsets[1] = 0;
     counts[0] = 0;
-    summary[0] = summary[1] = 0;
+    write_summary(summary, 0, 0);
 }
 
 int key_bits(int64_t groups) {
@@ -662,7 +741,8 @@ int key_bits(int64_t groups) {
 
 struct GroupLayout {
     size_t col, counters, table, scan;
-    size_t total() const { return 3 * col + counters + table + scan; }
+    static constexpr size_t state = 256;  // kGroupState counters
+    size_t total() const { return 3 * col + counters + state + table + scan; }
 };
 
 }  // namespace
@@ -673,7 +753,7 @@ size_t radix_sort_counter_bytes(int64_t N) { return radix_counter_bytes(N); }
 int radix_sort_positions(const int32_t *keys, int64_t N, int bits, int32_t *keys_out, int32_t *pos_out,
                          int32_t *tmp_keys, int32_t *tmp_pos, void *counters, hipStream_t stream) {
     return radix_sort_by_key(keys, N, bits, keys_out, pos_out, tmp_keys, tmp_pos, counters, nullptr, 0, nullptr, nullptr,
-                             stream);
+                             nullptr, stream);
 }
 
 size_t occupancy_scan_bytes(int64_t n);
@@ -730,12 +810,14 @@ extern "C" int cgnn_lsh_group(int64_t N, int bits, const int32_t *raw_code, int6
     int32_t *tmp_keys = reinterpret_cast<int32_t *>(base + L.col);
     int32_t *tmp_vals = reinterpret_cast<int32_t *>(base + 2 * L.col);
     void *counters = base + 3 * L.col;
-    char *rest = base + 3 * L.col + L.counters;
+    int32_t *state = reinterpret_cast<int32_t *>(base + 3 * L.col + L.counters);
+    char *rest = base + 3 * L.col + L.counters + GroupLayout::state;
     int64_t blocks = ceil_div(N, kBlock);
     if (blocks > 8192) blocks = 8192;
     const int64_t capacity = std::min<int64_t>(N, (int64_t)1 << bits);
     int64_t cblocks = ceil_div(capacity + 1, kBlock);
-    if (cblocks > 4096) cblocks = 4096;
+    // the arrivals are counted one by one, 12 ns each: few workgroups, or up to eight groups a thread
+    if (cblocks > 64) cblocks = std::min<int64_t>(std::max<int64_t>(64, ceil_div(cblocks, 8)), 4096);
     int rc;
     if (bits <= kTableBits) {
         const int codes = 1 << bits;
@@ -743,8 +825,8 @@ extern "C" int cgnn_lsh_group(int64_t N, int bits, const int32_t *raw_code, int6
         // with two passes the last one writes the ids straight into sorted_id
         bool ranked = false;
         int32_t *sorted = radix_passes(bits) > 1 ? sorted_id : sorted_code;
-        rc = radix_sort_by_key(raw_code, N, bits, sorted, perm, tmp_keys, tmp_vals, counters, table, codes - 1, summary,
-                               &ranked, stream);
+        rc = radix_sort_by_key(raw_code, N, bits, sorted, perm, tmp_keys, tmp_vals, counters, table, codes - 1, state,
+                               &ranked, state, stream);
         if (rc != CGNN_OK) return rc;
         int64_t fblocks = ceil_div(N, 4 * kBlock);  // four positions a thread
         if (fblocks > 8192) fblocks = 8192;
@@ -754,17 +836,17 @@ extern "C" int cgnn_lsh_group(int64_t N, int bits, const int32_t *raw_code, int6
         int32_t *head = reinterpret_cast<int32_t *>(rest);
         void *scan_scratch = rest + L.col;
         rc = radix_sort_by_key(raw_code, N, bits, sorted_code, perm, tmp_keys, tmp_vals, counters, nullptr, 0, nullptr,
-                               nullptr, stream);
+                               nullptr, state, stream);
         if (rc != CGNN_OK) return rc;
         hipLaunchKernelGGL(group_heads_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, stream, sorted_code, N, head,
-                           summary);
+                           state);
         rc = occupancy_scan(head, N, sorted_id, scan_scratch, stream);
         if (rc != CGNN_OK) return rc;
         hipLaunchKernelGGL(group_finish_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, stream, N, sorted_id, head,
-                           perm, ids, offsets, summary);
+                           perm, ids, offsets, state);
     }
-    hipLaunchKernelGGL(group_counts_kernel, dim3((unsigned)cblocks), dim3(kBlock), 0, stream, offsets, summary,
-                       counts, capacity);
+    hipLaunchKernelGGL(group_counts_kernel, dim3((unsigned)cblocks), dim3(kBlock), 0, stream, offsets, state,
+                       counts, capacity, summary);
     return check_launch("lsh_group");
 }
 
@@ -796,7 +878,7 @@ extern "C" int cgnn_cluster_members(int64_t N, int64_t groups, const int64_t *id
         hipLaunchKernelGGL(members_keys_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, stream, ids, keys, N, groups,
                            bad_id);
         int rc = radix_sort_by_key(keys, N, key_bits(groups), sorted_id, perm, tmp_keys, tmp_vals, base + 3 * col,
-                                   nullptr, 0, nullptr, nullptr, stream);
+                                   nullptr, 0, nullptr, nullptr, nullptr, stream);
         if (rc != CGNN_OK) return rc;
     }
     hipLaunchKernelGGL(members_offsets_kernel, dim3((unsigned)oblocks), dim3(kBlock), 0, stream,

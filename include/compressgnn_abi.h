@@ -313,12 +313,13 @@ int cgnn_cluster_members(int64_t N, int64_t groups, const int64_t *ids, int32_t 
  * counters): rows are sorted by code (stable), a run of equal codes is a group, and the
  * 1-based id of a group is the rank of its code.  Produces what cgnn_lsh_scan +
  * cgnn_lsh_finish + cgnn_cluster_members produce -- ids[N], counts[active+1] (entry 0 = 0),
- * offsets[active+2], perm[N], sorted_id[N] -- and summary[2] (device): summary[0] = active,
+ * offsets[active+2], perm[N], sorted_id[N] -- and summary[2]: summary[0] = active,
  * the number of groups, summary[1] = the size of the largest group.  counts needs room for min(N, 2^bits)+1 entries and offsets for one more; entries
  * beyond active+1 (active+2) are left untouched.  Replaces cluster_kernel.cu:143-150 and
  * the atomics of hash_ids (cluster_kernel.cu:41-59). */
-/* Up to cgnn_lsh_group_small_rows() rows the whole of it is one launch that needs no workspace and writes the
- * summary with plain stores, so that it may lie in pinned host memory. */
+/* Up to cgnn_lsh_group_small_rows() rows the whole of it is one launch that needs no workspace.  The summary may lie in
+ * pinned host memory; summary[0] is the last word that the call writes, so a host that finds it there finds all of
+ * the summary, and the arrays as soon as the stream is done with the call. */
 int64_t cgnn_lsh_group_small_rows(void);
 size_t cgnn_lsh_group_workspace_bytes(int64_t N, int bits);
 int cgnn_lsh_group(int64_t N, int bits, const int32_t *raw_code, int64_t *ids, int32_t *offsets,

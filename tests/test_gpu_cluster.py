@@ -240,6 +240,27 @@ def test_grouped_assign_matches_counter_path(shape, bits):
     assert members[3] == int(want_counts.max())
 
 
+@pytest.mark.parametrize("bits", [5, 16, 20])
+@pytest.mark.parametrize("n", [8193, 131072, 131073, 262145, 524288, 524289])
+def test_grouped_assign_of_any_length(n, bits):
+    """On both sides of the lengths at which the sort deals its keys differently: ids, counts, member lists and the largest
+    group of an assignment are whole numbers and come out as the oracle's, also on a second call."""
+    rng = np.random.default_rng(n + bits)
+    x = rng.standard_normal((n, 2)).astype(np.float32)  # few directions: the groups are of very different sizes
+    w = rng.standard_normal((2, bits)).astype(np.float32)
+    want, counts, active = oracle.assign(x, w, bits)
+    features, planes = _t(x), _t(w)
+    for _ in range(2):
+        ids, got_counts, got_active, members = abi.lsh_assign_grouped(features, planes, bits)
+        assert got_active == active
+        assert np.array_equal(ids.cpu().numpy(), want)
+        assert np.array_equal(got_counts.cpu().numpy(), counts)
+        offsets, perm, sorted_id = (m.cpu().numpy() for m in members[:3])
+        assert np.array_equal(perm, np.argsort(want, kind="stable"))
+        assert np.array_equal(sorted_id, want[perm])
+        assert np.array_equal(offsets, np.concatenate([[0], np.cumsum(counts)]))
+
+
 def test_grouped_assign_empty():
     ids, counts, active, members = abi.lsh_assign_grouped(torch.zeros(0, 8, device=DEV), torch.randn(8, 8, device=DEV), 8)
     assert ids.numel() == 0 and active == 0 and counts.tolist() == [0] and members[0].tolist() == [0, 0]
