@@ -285,15 +285,26 @@ __global__ __launch_bounds__(kBlock) void sample_fill_kernel(LayerArgs a) {
 // was given.  Smaller is final, so that claims are atomic minima that never touch a number.
 constexpr int32_t kClaim = 1 << 30;
 constexpr int kChunkItems = 4;
-constexpr int kChunk = kChunkItems * kBlock;  // slots per workgroup when they are ranked
+constexpr int kChunk = kChunkItems * kBlock;  // most slots per workgroup when they are ranked
 constexpr int kTail = 8;                      // chunks a thread sums up when all are counted
 constexpr int kRegPicks = kWave;              // fan-outs up to this keep the chosen positions in registers, one a lane
+// Layers of up to this many chunks are counted while they are filled: a claim that is taken over moves its vertex from one
+// chunk to another, and the workgroups that rank the slots sum up the chunks in front of theirs.  A launch of 5 to 7 us
+// less a layer (and one pass less over the slots, 15 us where there are 5 million), 1 to 2 us more in the fill: 1,024 seeds
+// with 25 and 10 61 -> 57 us, 8,192 with 10 and 10 76 -> 70, 16,384 with 25 and 15 109 -> 93, with 25 and 25 (8,139 chunks)
+// 123 -> 99.  Beyond, what they read of each other's counts (256 MB at this limit) grows with the square, and a launch of
+// its own counts the slots and sums them up once.
+constexpr int64_t kCountedChunks = 8192;
 
 struct BoundedLayer {
     int64_t fanout, n_cap;   // most vertices of the frontier
+    int32_t chunk;           // slots of a chunk: those of as many workgroups of bounded_fill_kernel as kChunk holds
     int32_t *slots;          // [n_cap * fanout] neighbours, -1 behind the last
-    uint64_t *before;        // [chunks] neighbours, and << 32 vertices they introduce, in the chunks in front
+    uint64_t *counts;        // [chunks] neighbours, and << 32 vertices they introduce; NULL: counted by bounded_count_kernel
+    uint64_t *before;        // [chunks] the same in the chunks in front
 };
+
+__host__ __device__ __forceinline__ int bounded_lanes(int64_t fanout) { return fanout <= 16 ? 16 : fanout <= 32 ? 32 : kWave; }
 
 // state of a layer: position of its frontier among the samples, vertices in it, edges of the layers before, chunks
 // ranked so far
@@ -315,6 +326,9 @@ struct BoundedArgs {
 __global__ __launch_bounds__(kBlock) void bounded_begin_kernel(BoundedArgs a) {
     const int64_t stride = (int64_t)gridDim.x * kBlock, t0 = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     for (int64_t v = t0; v < a.g.vertex_cnt; v += stride) a.number_of[v] = kUnseen;
+    for (int k = 0; k < a.layers; ++k)
+        if (a.at[k].counts != nullptr)
+            for (int64_t c = t0; c < a.first_chunk[k + 1] - a.first_chunk[k]; c += stride) a.at[k].counts[c] = 0;
     if (t0 < 4 * (a.layers + 1)) a.state[t0] = t0 == 1 ? (int32_t)a.n_input : 0;
     if (t0 < 2) a.status[t0] = CGNN_SAMPLE_OK;
 }
@@ -385,92 +399,125 @@ __device__ __forceinline__ int64_t neighbors_at(const Graph &g, int64_t node, in
 
 // LANES lanes per frontier vertex (as many as the fan-out asks for: a step waits for one load after another, and
 // with a wave per vertex most lanes of it wait for nothing), into the vertex's slots.  The first layer also
-// numbers the input, a vertex given twice by its first position.
-template <int LANES>
+// numbers the input, a vertex given twice by its first position.  COUNTED: adds to the counts of the workgroup's chunk how
+// many neighbours it found and how many vertices they introduce as far as is known; a claim that it takes from a slot
+// further back, or that a number takes from a slot, is taken off that slot's chunk.
+template <int LANES, bool COUNTED>
 __global__ __launch_bounds__(kBlock) void bounded_fill_kernel(BoundedArgs a) {
     const BoundedLayer &l = a.at[a.layer];
-    const int lane = threadIdx.x % LANES;
-    const int64_t i = (int64_t)blockIdx.x * (kBlock / LANES) + threadIdx.x / LANES;
     const int32_t first = a.state[4 * a.layer], n = a.state[4 * a.layer + 1];
-    if (i >= n) return;
-    const Graph &g = a.g;
-    const int fanout = (int)l.fanout;
-    const int64_t node = a.layer == 0 ? a.input[i] : a.samples[first + i], slot0 = i * fanout;
-    auto put = [&](int t, int64_t neighbor) {
-        if (neighbor < 0 || neighbor >= g.vertex_cnt) {
-            atomicCAS(a.status, CGNN_SAMPLE_OK, neighbor == -1 ? CGNN_SAMPLE_OUT_OF_RANGE : CGNN_SAMPLE_BAD_VERTEX);
-            neighbor = 0;
-        }
-        l.slots[slot0 + t] = (int32_t)neighbor;
-        const int32_t claim = kClaim + (int32_t)(slot0 + t);
-        if (a.number_of[neighbor] > claim) atomicMin(&a.number_of[neighbor], claim);
+    const int64_t i0 = (int64_t)blockIdx.x * (kBlock / LANES);
+    if (i0 >= n) return;
+    int live = 0, fresh = 0;
+    auto displaced = [&](int32_t claim) {
+        if (claim >= kClaim && claim != kUnseen)
+            __hip_atomic_fetch_add(l.counts + (claim - kClaim) / l.chunk, ~uint64_t(0) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
-    auto full_list = [&]() -> int {  // its length, or -1: longer than the fan-out (or by rules that lead nowhere)
-        const int64_t v2v_start = g.v2v_ptr[node], v2v_count = g.v2v_ptr[node + 1] - v2v_start;
-        if (v2v_count > fanout) return -1;
-        if (lane < v2v_count) put(lane, g.v2v_idx[v2v_start + lane]);
-        int count = (int)v2v_count;
-        if (g.v2r_ptr == nullptr) return count;
-        // Depth by depth, a rule a lane, in the order in which a walk in pre-order meets the rules of a depth.  Sizes
-        // are cut off where they are too large in any case, so that two sums fit into one.
-        const int64_t v2r_start = g.v2r_ptr[node], v2r_count = g.v2r_ptr[node + 1] - v2r_start;
-        if (v2r_count > LANES) return -1;
-        auto cut = [](int64_t size) { return (int)(size < 0 ? 0 : size > LANES ? LANES + 1 : size); };
-        int rules = (int)v2r_count;
-        int64_t rule = lane < rules ? g.v2r_idx[v2r_start + lane] : 0;
-        for (int depth = 0; rules > 0; ++depth) {
-            int64_t own_start = 0, child_start = 0;
-            int own = 0, children = 0;
-            if (lane < rules) {
-                own_start = g.r2v_ptr[rule];
-                own = cut(g.r2v_ptr[rule + 1] - own_start);
-                if (depth < g.levels) {
-                    child_start = g.r2r_ptr[depth][rule];
-                    children = cut(g.r2r_ptr[depth][rule + 1] - child_start);
+    auto fill = [&](int64_t i, int lane) {
+        const Graph &g = a.g;
+        const int fanout = (int)l.fanout;
+        const int64_t node = a.layer == 0 ? a.input[i] : a.samples[first + i], slot0 = i * fanout;
+        auto put = [&](int t, int64_t neighbor) {
+            if (neighbor < 0 || neighbor >= g.vertex_cnt) {
+                atomicCAS(a.status, CGNN_SAMPLE_OK, neighbor == -1 ? CGNN_SAMPLE_OUT_OF_RANGE : CGNN_SAMPLE_BAD_VERTEX);
+                neighbor = 0;
+            }
+            l.slots[slot0 + t] = (int32_t)neighbor;
+            const int32_t claim = kClaim + (int32_t)(slot0 + t);
+            if (a.number_of[neighbor] > claim) {
+                const int32_t was = atomicMin(&a.number_of[neighbor], claim);
+                if (COUNTED && was > claim) {
+                    ++fresh;
+                    displaced(was);
                 }
             }
-            const int sums = inclusive_sum<LANES>(own | children << 16, lane), all = __shfl(sums, LANES - 1, LANES);
-            const int owns = sums & 0xffff, all_own = all & 0xffff, descend = sums >> 16, all_descend = all >> 16;
-            if (count + all_own > fanout || all_descend > LANES) return -1;
-            const int p = first_above<LANES>(owns, lane);
-            const int64_t from = __shfl(own_start - (owns - own), p, LANES);
-            if (lane < all_own) put(count + lane, g.r2v_idx[from + lane]);
-            count += all_own;
-            rules = all_descend;
-            const int q = first_above<LANES>(descend, lane);
-            const int64_t child = __shfl(child_start - (descend - children), q, LANES);
-            if (lane < rules) rule = g.r2r_idx[depth][child + lane];
+        };
+        auto full_list = [&]() -> int {  // its length, or -1: longer than the fan-out (or by rules that lead nowhere)
+            const int64_t v2v_start = g.v2v_ptr[node], v2v_count = g.v2v_ptr[node + 1] - v2v_start;
+            if (v2v_count > fanout) return -1;
+            if (lane < v2v_count) put(lane, g.v2v_idx[v2v_start + lane]);
+            int count = (int)v2v_count;
+            if (g.v2r_ptr == nullptr) return count;
+            // Depth by depth, a rule a lane, in the order in which a walk in pre-order meets the rules of a depth.  Sizes
+            // are cut off where they are too large in any case, so that two sums fit into one.
+            const int64_t v2r_start = g.v2r_ptr[node], v2r_count = g.v2r_ptr[node + 1] - v2r_start;
+            if (v2r_count > LANES) return -1;
+            auto cut = [](int64_t size) { return (int)(size < 0 ? 0 : size > LANES ? LANES + 1 : size); };
+            int rules = (int)v2r_count;
+            int64_t rule = lane < rules ? g.v2r_idx[v2r_start + lane] : 0;
+            for (int depth = 0; rules > 0; ++depth) {
+                int64_t own_start = 0, child_start = 0;
+                int own = 0, children = 0;
+                if (lane < rules) {
+                    own_start = g.r2v_ptr[rule];
+                    own = cut(g.r2v_ptr[rule + 1] - own_start);
+                    if (depth < g.levels) {
+                        child_start = g.r2r_ptr[depth][rule];
+                        children = cut(g.r2r_ptr[depth][rule + 1] - child_start);
+                    }
+                }
+                const int sums = inclusive_sum<LANES>(own | children << 16, lane), all = __shfl(sums, LANES - 1, LANES);
+                const int owns = sums & 0xffff, all_own = all & 0xffff, descend = sums >> 16, all_descend = all >> 16;
+                if (count + all_own > fanout || all_descend > LANES) return -1;
+                const int p = first_above<LANES>(owns, lane);
+                const int64_t from = __shfl(own_start - (owns - own), p, LANES);
+                if (lane < all_own) put(count + lane, g.r2v_idx[from + lane]);
+                count += all_own;
+                rules = all_descend;
+                const int q = first_above<LANES>(descend, lane);
+                const int64_t child = __shfl(child_start - (descend - children), q, LANES);
+                if (lane < rules) rule = g.r2r_idx[depth][child + lane];
+            }
+            return count;
+        };
+        int count = 0;
+        if (node < 0 || node >= g.vertex_cnt) {
+            atomicCAS(a.status, CGNN_SAMPLE_OK, CGNN_SAMPLE_BAD_VERTEX);
+        } else {
+            if (a.layer == 0 && lane == 0) {
+                const int32_t was = atomicMin(&a.number_of[node], (int32_t)i);
+                if (COUNTED) displaced(was);
+            }
+            const int64_t degree = degree_of(g, node);
+            if (degree > fanout) {
+                // The selection loop of sample_fill_kernel with a step per lane: the draws do not depend on each other, only
+                // whether a drawn position was taken before does.
+                count = fanout;
+                const int64_t j = degree - count + lane;
+                int64_t pick = lane < count ? draw(a.seed, a.layer, first + i, j, j) : -1;
+                for (int s = 1; s < count; ++s) {
+                    const int64_t rnd = __shfl(pick, s, LANES);
+                    const bool taken = any_lane<LANES>(lane < s && pick == rnd);
+                    if (lane == s && taken) pick = j;
+                }
+                const int64_t neighbor = neighbors_at<LANES>(g, node, pick, lane < count, lane);
+                if (lane < count) put(lane, neighbor);
+            } else if (degree > 0) {
+                count = full_list();
+                if (count < 0) {  // the call is done again layer by layer
+                    a.status[1] = 1;
+                    count = 0;
+                }
+            }
         }
-        return count;
+        for (int t = count + lane; t < fanout; t += LANES) l.slots[slot0 + t] = -1;
+        if (lane == 0) live = count;
     };
-    int count = 0;
-    if (node < 0 || node >= g.vertex_cnt) {
-        atomicCAS(a.status, CGNN_SAMPLE_OK, CGNN_SAMPLE_BAD_VERTEX);
-    } else {
-        if (a.layer == 0 && lane == 0) atomicMin(&a.number_of[node], (int32_t)i);
-        const int64_t degree = degree_of(g, node);
-        if (degree > fanout) {
-            // The selection loop of sample_fill_kernel with a step per lane: the draws do not depend on each other, only
-            // whether a drawn position was taken before does.
-            count = fanout;
-            const int64_t j = degree - count + lane;
-            int64_t pick = lane < count ? draw(a.seed, a.layer, first + i, j, j) : -1;
-            for (int s = 1; s < count; ++s) {
-                const int64_t rnd = __shfl(pick, s, LANES);
-                const bool taken = any_lane<LANES>(lane < s && pick == rnd);
-                if (lane == s && taken) pick = j;
-            }
-            const int64_t neighbor = neighbors_at<LANES>(g, node, pick, lane < count, lane);
-            if (lane < count) put(lane, neighbor);
-        } else if (degree > 0) {
-            count = full_list();
-            if (count < 0) {  // the call is done again layer by layer
-                a.status[1] = 1;
-                count = 0;
-            }
+    const int64_t mine = i0 + threadIdx.x / LANES;
+    if (mine < n) fill(mine, threadIdx.x % LANES);
+    if constexpr (COUNTED) {  // at most 256 of each a workgroup
+        __shared__ int sums[kBlock / kWave];
+        const int sum = inclusive_sum<kWave>(live | fresh << 16, (int)(threadIdx.x % kWave));
+        if (threadIdx.x % kWave == kWave - 1) sums[threadIdx.x / kWave] = sum;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            int all = 0;
+#pragma unroll
+            for (int w = 0; w < kBlock / kWave; ++w) all += sums[w];
+            __hip_atomic_fetch_add(l.counts + i0 * l.fanout / l.chunk, (uint64_t)(all >> 16) << 32 | (uint64_t)(all & 0xffff),
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
-    for (int t = count + lane; t < fanout; t += LANES) l.slots[slot0 + t] = -1;
 }
 
 // The slots of a thread in a chunk of a layer with `slots` of them: neighbours (or -1), and which introduce a vertex.
@@ -483,7 +530,8 @@ struct ChunkSlots {
 __device__ __forceinline__ ChunkSlots chunk_slots(const BoundedArgs &a, const BoundedLayer &l, int64_t slots, int64_t chunk,
                                                   bool ranks) {
     ChunkSlots c;
-    const int64_t s0 = chunk * kChunk + threadIdx.x * kChunkItems;
+    const int64_t s0 = chunk * l.chunk + threadIdx.x * kChunkItems;
+    slots = min(slots, (chunk + 1) * l.chunk);
     if (s0 + kChunkItems <= slots) {
         const int4 four = *reinterpret_cast<const int4 *>(l.slots + s0);
         c.v[0] = four.x, c.v[1] = four.y, c.v[2] = four.z, c.v[3] = four.w;
@@ -532,12 +580,23 @@ __device__ __forceinline__ int2 chunk_sums(int live, int fresh, int2 *total) {
     return before;
 }
 
+// The sizes of a call, in pinned host memory: the last word last, past the caches with a wait between (a release would write
+// back the whole L2).
+__device__ __forceinline__ void bounded_summary(const BoundedArgs &a, int32_t samples, int32_t edges) {
+    const int32_t words[3] = {samples, edges, a.status[1] ? -1 : a.status[0]};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) __hip_atomic_store(a.summary + k, words[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0);
+    __hip_atomic_store(a.summary + 3, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // How many neighbours a chunk holds and how many vertices they introduce; the last chunk to be counted sums the
 // chunks up and sets the state of the next layer.
 __global__ __launch_bounds__(kBlock) void bounded_count_kernel(BoundedArgs a) {
     const BoundedLayer &l = a.at[a.layer];
     int32_t *state = a.state + 4 * a.layer;
-    const int64_t n = state[1], held = ceil_div_dev(n * l.fanout, kChunk), chunks = held < 1 ? 1 : held;
+    const int64_t n = state[1], held = ceil_div_dev(n * l.fanout, l.chunk), chunks = held < 1 ? 1 : held;
     if (blockIdx.x >= chunks) return;
     const ChunkSlots c = chunk_slots(a, l, n * l.fanout, blockIdx.x, true);
     int2 total;
@@ -575,24 +634,52 @@ __global__ __launch_bounds__(kBlock) void bounded_count_kernel(BoundedArgs a) {
         state[4] = end;
         state[5] = running.y;
         state[6] = state[2] + running.x;
-        if (a.layer == a.layers - 1) {
-            a.summary[0] = end + running.y;
-            a.summary[1] = state[2] + running.x;
-            a.summary[2] = a.status[1] ? -1 : a.status[0];
-            __hip_atomic_store(a.summary + 3, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
+        if (a.layer == a.layers - 1) bounded_summary(a, end + running.y, state[2] + running.x);
     }
 }
 
-// The vertices that a layer introduces take the numbers behind its frontier, in the order of their slots.
+// The vertices that a layer introduces take the numbers behind its frontier, in the order of their slots.  COUNTED: every
+// workgroup sums up the counts of the chunks, and the first sets the state of the next layer.
+template <bool COUNTED>
 __global__ __launch_bounds__(kBlock) void bounded_assign_kernel(BoundedArgs a) {
     const BoundedLayer &l = a.at[a.layer];
-    const int32_t *state = a.state + 4 * a.layer;
-    const int64_t n = state[1];
-    if ((int64_t)blockIdx.x * kChunk >= n * l.fanout) return;
-    const ChunkSlots c = chunk_slots(a, l, n * l.fanout, blockIdx.x, true);
+    int32_t *state = a.state + 4 * a.layer;
+    const int64_t n = state[1], slots = n * l.fanout;
+    if (blockIdx.x > 0 && (int64_t)blockIdx.x * l.chunk >= slots) return;
+    const int32_t end = state[0] + (int32_t)n;
+    int32_t fresh_before;
+    if constexpr (COUNTED) {
+        const int64_t chunks = ceil_div_dev(slots, l.chunk);
+        uint64_t before = 0, behind = 0;  // only the first workgroup needs what stands behind
+        for (int64_t c0 = threadIdx.x; c0 < (blockIdx.x == 0 ? chunks : blockIdx.x); c0 += kTail * kBlock) {
+            uint64_t pair[kTail];
+#pragma unroll
+            for (int u = 0; u < kTail; ++u) pair[u] = c0 + u * kBlock < chunks ? l.counts[c0 + u * kBlock] : 0;
+#pragma unroll
+            for (int u = 0; u < kTail; ++u) {
+                if (c0 + u * kBlock < blockIdx.x) before += pair[u];
+                else behind += pair[u];
+            }
+        }
+        int2 all_before, all_behind;
+        chunk_sums((int)(uint32_t)before, (int)(before >> 32), &all_before);
+        chunk_sums((int)(uint32_t)behind, (int)(behind >> 32), &all_behind);
+        if (threadIdx.x == 0) {
+            l.before[blockIdx.x] = (uint64_t)all_before.y << 32 | (uint32_t)all_before.x;
+            if (blockIdx.x == 0) {
+                state[4] = end;
+                state[5] = all_behind.y;
+                state[6] = state[2] + all_behind.x;
+                if (a.layer == a.layers - 1) bounded_summary(a, end + all_behind.y, state[2] + all_behind.x);
+            }
+        }
+        fresh_before = all_before.y;
+    } else {
+        fresh_before = (int32_t)(l.before[blockIdx.x] >> 32);
+    }
+    const ChunkSlots c = chunk_slots(a, l, slots, blockIdx.x, true);
     int2 total;
-    int32_t number = state[4] + (int32_t)(l.before[blockIdx.x] >> 32) + chunk_sums(c.live, c.fresh, &total).y;
+    int32_t number = end + fresh_before + chunk_sums(c.live, c.fresh, &total).y;
 #pragma unroll
     for (int u = 0; u < kChunkItems; ++u)
         if (c.introduces >> u & 1u) {
@@ -615,11 +702,12 @@ __global__ __launch_bounds__(kBlock) void bounded_write_kernel(BoundedArgs a) {
     const BoundedLayer &l = a.at[layer];
     const int32_t *state = a.state + 4 * layer;
     const int64_t chunk = blockIdx.x - a.first_chunk[layer], n = state[1];
-    if (chunk * kChunk >= n * l.fanout) return;
+    if (chunk * l.chunk >= n * l.fanout) return;
     const ChunkSlots c = chunk_slots(a, l, n * l.fanout, chunk, false);
     int2 total;
     int64_t e = (int64_t)state[2] + (int32_t)l.before[chunk] + chunk_sums(c.live, 0, &total).x;
-    int64_t i = (chunk * kChunk + threadIdx.x * kChunkItems) / l.fanout, t = chunk * kChunk + threadIdx.x * kChunkItems - i * l.fanout;
+    const int64_t s0 = chunk * l.chunk + threadIdx.x * kChunkItems;
+    int64_t i = s0 / l.fanout, t = s0 - i * l.fanout;
 #pragma unroll
     for (int u = 0; u < kChunkItems; ++u) {
         if (c.v[u] >= 0) {
@@ -938,8 +1026,9 @@ namespace {
 
 struct BoundedLayout {
     size_t number_of, samples, state, status, total;
-    size_t slots[CGNN_SAMPLE_MAX_BOUNDED], before[CGNN_SAMPLE_MAX_BOUNDED];
+    size_t slots[CGNN_SAMPLE_MAX_BOUNDED], counts[CGNN_SAMPLE_MAX_BOUNDED], before[CGNN_SAMPLE_MAX_BOUNDED];
     int64_t n_cap[CGNN_SAMPLE_MAX_BOUNDED], chunks[CGNN_SAMPLE_MAX_BOUNDED];
+    int32_t chunk[CGNN_SAMPLE_MAX_BOUNDED];
     int64_t samples_cap;
 };
 
@@ -969,8 +1058,11 @@ bool bounded_layout(int64_t vertex_cnt, int64_t n_input, int layers, const int64
         all += slots;
         if (all > kMostSlots) return false;
         L->n_cap[k] = n;
-        L->chunks[k] = ceil_div(slots, kChunk);
+        const int64_t workgroup = kBlock / bounded_lanes(fanouts[k]) * fanouts[k];  // a multiple of four slots, at most 256
+        L->chunk[k] = (int32_t)(kChunk / workgroup * workgroup);
+        L->chunks[k] = ceil_div(slots, L->chunk[k]);
         L->slots[k] = take(slots);
+        L->counts[k] = L->chunks[k] <= kCountedChunks ? take(2 * L->chunks[k]) : 0;
         L->before[k] = take(2 * L->chunks[k]);
         n = slots < vertex_cnt ? slots : vertex_cnt;  // a layer adds every vertex once
         L->samples_cap += n;
@@ -994,7 +1086,9 @@ BoundedArgs bounded_args(const cgnn_sample_graph *graph, int64_t n_input, const 
     a.seed = seed;
     a.layers = layers;
     for (int k = 0; k < layers; ++k) {
-        a.at[k] = BoundedLayer{fanouts[k], L.n_cap[k], ints(L.slots[k]), reinterpret_cast<uint64_t *>(base + L.before[k])};
+        a.at[k] = BoundedLayer{fanouts[k], L.n_cap[k], L.chunk[k], ints(L.slots[k]),
+                               L.chunks[k] <= kCountedChunks ? reinterpret_cast<uint64_t *>(base + L.counts[k]) : nullptr,
+                               reinterpret_cast<uint64_t *>(base + L.before[k])};
         a.first_chunk[k + 1] = a.first_chunk[k] + L.chunks[k];
     }
     return a;
@@ -1023,13 +1117,15 @@ extern "C" int cgnn_sample_layers(const cgnn_sample_graph *graph, int64_t n_inpu
     hipLaunchKernelGGL(bounded_begin_kernel, dim3(blocks_for(graph->vertex_cnt)), dim3(kBlock), 0, stream, a);
     for (int k = 0; k < layers; ++k) {
         a.layer = k;
-        const int lanes = fanouts[k] <= 16 ? 16 : fanouts[k] <= 32 ? 32 : kWave;
-        const dim3 grid((unsigned)ceil_div(L.n_cap[k], kBlock / lanes));
-        if (lanes == 16) hipLaunchKernelGGL((bounded_fill_kernel<16>), grid, dim3(kBlock), 0, stream, a);
-        else if (lanes == 32) hipLaunchKernelGGL((bounded_fill_kernel<32>), grid, dim3(kBlock), 0, stream, a);
-        else hipLaunchKernelGGL((bounded_fill_kernel<kWave>), grid, dim3(kBlock), 0, stream, a);
-        hipLaunchKernelGGL(bounded_count_kernel, dim3((unsigned)L.chunks[k]), dim3(kBlock), 0, stream, a);
-        hipLaunchKernelGGL(bounded_assign_kernel, dim3((unsigned)L.chunks[k]), dim3(kBlock), 0, stream, a);
+        const int lanes = bounded_lanes(fanouts[k]);
+        const bool counted = a.at[k].counts != nullptr;
+        const auto fill = lanes == 16   ? (counted ? bounded_fill_kernel<16, true> : bounded_fill_kernel<16, false>)
+                          : lanes == 32 ? (counted ? bounded_fill_kernel<32, true> : bounded_fill_kernel<32, false>)
+                                        : (counted ? bounded_fill_kernel<kWave, true> : bounded_fill_kernel<kWave, false>);
+        const dim3 chunks((unsigned)L.chunks[k]);
+        hipLaunchKernelGGL(fill, dim3((unsigned)ceil_div(L.n_cap[k], kBlock / lanes)), dim3(kBlock), 0, stream, a);
+        if (!counted) hipLaunchKernelGGL(bounded_count_kernel, chunks, dim3(kBlock), 0, stream, a);
+        hipLaunchKernelGGL(counted ? bounded_assign_kernel<true> : bounded_assign_kernel<false>, chunks, dim3(kBlock), 0, stream, a);
     }
     return check_launch("sample_layers");
 }

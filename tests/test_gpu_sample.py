@@ -272,6 +272,25 @@ def test_layers_of_many_chunks():
         assert np.array_equal(a.cpu().numpy(), w)
 
 
+@pytest.mark.parametrize("seeds, fan", [(131072, [64]), (131073, [64]), (13653, [15, 3]), (68, [15, 15]), (69, [15, 15]), (1, [25, 1, 40])])
+def test_layers_counted_while_they_are_filled(seeds, fan):
+    """On both sides of the number of chunks up to which the fill counts them (8,192), and with ragged last chunks: a few
+    vertices stand in most lists and among the seeds, so that claims pass from chunk to chunk and to the seeds' numbers."""
+    import compressgnn_sample as sampler
+    rng = np.random.default_rng(seeds + len(fan))
+    V = 20000
+    lengths = rng.integers(0, 80, V)
+    ptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64)
+    idx = np.where(rng.random(ptr[-1]) < 0.5, rng.integers(0, 50, ptr[-1]), rng.integers(0, V, ptr[-1]))
+    inp = np.where(rng.random(seeds) < 0.2, rng.integers(0, 60, seeds), rng.integers(0, V, seeds))
+    t = lambda a: torch.from_numpy(a).to(DEV)
+    want = oracle.neighbor_sample(dict(v2v=(ptr, idx)), inp, fan, seed=9, plain=True)
+    for _ in range(3):
+        got = sampler.neighbor_sample_ori_impl(t(ptr), t(idx), t(inp), fan, seed=9)
+        for a, w in zip(got, want):
+            assert np.array_equal(a.cpu().numpy(), w)
+
+
 @pytest.mark.parametrize("rows", [1 << 19, (1 << 19) + 1])
 def test_layers_at_the_limit_of_the_slots_and_without_room_for_them(rows):
     """As many slots as a call with one host read may have, and one vertex more; and a call that finds no room for its
