@@ -1734,55 +1734,49 @@ __global__ void expand_rows_kernel(const P *__restrict__ rowptr, int64_t rows, i
 
 // The int32 form of a block that is given as int64 arrays for one product: row pointers, columns and the row of
 // every entry, in one launch.  Rows and entries are walked as one list -- every row in front of its entries, row r at
-// position rowptr[r] + r -- and a workgroup takes kOnceItems * kBlock consecutive places of it, so neither hubs (a
+// position rowptr[r] + r -- and a workgroup takes ITEMS * kBlock consecutive places of it, so neither hubs (a
 // workgroup per 16 rows took 41 us for 100,003 rows of 1.0 M entries of a web graph, whose hubs are neighbours) nor the
 // thousands of empty rows of the youngest vertices (2,048 entries per workgroup: 22 us) keep one longer than the others.
-// It looks for the two ends of its stretch with all its threads at once (256 row pointers a step), marks the entries
-// that rows begin at and spreads the marks by a running maximum: 9.0 us.  Row pointers and columns narrowed apart and a
-// binary search per entry were three launches of 25 us, behind 26 us for the length of the longest row and its
-// way to the host.
+// Two of its waves look for the two ends of its stretch, 64 row pointers a step, and its threads mark the entries that rows
+// begin at and spread the marks by a running maximum: 7.4 us.  With all threads at the search, 256 row pointers a step, the
+// card spent its time on requests for row pointers: 9.0 us (1,024 a step: 13).  Row pointers and columns narrowed apart and
+// a binary search per entry were three launches of 25 us, behind 26 us for the length of the longest row and its way to the
+// host.
 // The rows hold the entries [rowptr64[0], rowptr64[rows]) of the arrays: a slice of the row pointers of a larger block
 // comes with all its entries, and a list may be padded behind the last row.  Only these entries are taken over, and the
 // int32 arrays count from the first of them: span = {how many, where the first stands}.
-constexpr int kOnceItems = 8;
-constexpr int kOncePlaces = kOnceItems * kBlock;
+// 1,024 places a workgroup while that is about a round of workgroups, whose searches then wait beside each other (a product
+// over 8,000 rows 20.1 -> 19.4 us), and 2,048 beyond, where the searches cost (325,557 rows 92.7 -> 90.3).
+int once_items(int64_t places) { return places <= (int64_t)4 * kBlock * 1536 ? 4 : 8; }
 
+template <int ITEMS>
 __global__ __launch_bounds__(kBlock) void csr_once_kernel(const int64_t *__restrict__ rowptr64, const int64_t *__restrict__ col64,
                                                           int64_t rows, int64_t nnz, int32_t *__restrict__ rowptr,
                                                           int32_t *__restrict__ col, int32_t *__restrict__ rowidx,
                                                           int32_t *__restrict__ span) {
-    __shared__ int32_t begins[kOncePlaces];  // the row that begins at an entry of the stretch, or -1
+    constexpr int kPlaces = ITEMS * kBlock;
+    __shared__ int32_t begins[kPlaces];  // the row that begins at an entry of the stretch, or -1
     __shared__ int waves[2][kBlock / kWave];
-    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-    const int64_t places[2] = {(int64_t)blockIdx.x * kOncePlaces, min(rows + nnz, (int64_t)(blockIdx.x + 1) * kOncePlaces)};
+    __shared__ int64_t found[2];
+    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int64_t places[2] = {(int64_t)blockIdx.x * kPlaces, min(rows + nnz, (int64_t)(blockIdx.x + 1) * kPlaces)};
 #pragma unroll
-    for (int u = 0; u < kOnceItems; ++u) begins[u * kBlock + threadIdx.x] = -1;
-    // the largest row at or before each of the two places lies in [lo, hi); row lo does throughout
-    int64_t lo[2] = {0, 0}, hi[2] = {rows, rows};
-    while (hi[0] - lo[0] > 1 || hi[1] - lo[1] > 1) {
-        int64_t step[2], at[2];
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            step[k] = (hi[k] - lo[k] + kBlock - 1) / kBlock;
-            const int64_t r = lo[k] + step[k] * threadIdx.x;
-            at[k] = r < hi[k] ? rowptr64[r] + r : INT64_MAX;
+    for (int u = 0; u < ITEMS; ++u) begins[u * kBlock + threadIdx.x] = -1;
+    // The largest row at or before each of the two places: a wave looks for one of them, 64 row pointers a step
+    // (it lies in [from, to), and row `from` does throughout).
+    if (wave < 2) {
+        int64_t from = 0, to = rows;
+        const int64_t place = places[wave];
+        while (to - from > 1) {
+            const int64_t step = (to - from + kWave - 1) / kWave, r = from + step * lane;
+            const bool at_or_before = lane == 0 || (r < to && rowptr64[r] + r <= place);
+            from += step * (__popcll(__ballot(at_or_before)) - 1);
+            to = min(to, from + step);
         }
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const int n = __popcll(__ballot(threadIdx.x == 0 || at[k] <= places[k]));
-            if (lane == 0) waves[k][wave] = n;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            int below = 0;
-#pragma unroll
-            for (int w = 0; w < kBlock / kWave; ++w) below += waves[k][w];
-            lo[k] += step[k] * (below - 1);
-            hi[k] = min(hi[k], lo[k] + step[k]);
-        }
-        __syncthreads();
+        if (lane == 0) found[wave] = from;
     }
+    __syncthreads();
+    const int64_t lo[2] = {found[0], found[1]};
     // the entries that belong to rows; row pointers that are none must not lead out of the arrays
     const int64_t first = max((int64_t)0, min(nnz, rowptr64[0])), last = max(first, min(nnz, rowptr64[rows]));
     auto inside = [&](int64_t e) { return max(first, min(last, e)); };
@@ -1798,10 +1792,10 @@ __global__ __launch_bounds__(kBlock) void csr_once_kernel(const int64_t *__restr
     }
     if (places[1] == rows + nnz) entry[1] = last, row[1] = rows;
     const int64_t e0 = entry[0];
-    const int held = (int)max((int64_t)0, min((int64_t)kOncePlaces, entry[1] - e0));
-    int64_t c[kOnceItems], at[kOnceItems], end[kOnceItems];
+    const int held = (int)max((int64_t)0, min((int64_t)kPlaces, entry[1] - e0));
+    int64_t c[ITEMS], at[ITEMS], end[ITEMS];
 #pragma unroll
-    for (int u = 0; u < kOnceItems; ++u) {
+    for (int u = 0; u < ITEMS; ++u) {
         const int k = u * kBlock + threadIdx.x;
         const int64_t r = row[0] + k;
         c[u] = k < held ? col64[e0 + k] : 0;
@@ -1811,7 +1805,7 @@ __global__ __launch_bounds__(kBlock) void csr_once_kernel(const int64_t *__restr
         end[u] = rowptr64[min(r, rows - 1) + 1];
     }
 #pragma unroll
-    for (int u = 0; u < kOnceItems; ++u) {
+    for (int u = 0; u < ITEMS; ++u) {
         const int64_t r = row[0] + u * kBlock + threadIdx.x;
         if (r >= row[1]) break;
         at[u] = inside(at[u]), end[u] = inside(end[u]);
@@ -1822,15 +1816,15 @@ __global__ __launch_bounds__(kBlock) void csr_once_kernel(const int64_t *__restr
         if (end[u] > at[u] && k >= 0 && k < held) begins[k] = (int32_t)r;
     }
     __syncthreads();
-    // thread t spreads the marks over entries t * kOnceItems ...; what comes before the first mark belongs to the
+    // thread t spreads the marks over entries t * ITEMS ...; what comes before the first mark belongs to the
     // row in front of the stretch
-    int32_t mark[kOnceItems];
+    int32_t mark[ITEMS];
 #pragma unroll
-    for (int u = 0; u < kOnceItems; ++u) {
-        mark[u] = begins[threadIdx.x * kOnceItems + u];
+    for (int u = 0; u < ITEMS; ++u) {
+        mark[u] = begins[threadIdx.x * ITEMS + u];
         if (u > 0) mark[u] = max(mark[u], mark[u - 1]);
     }
-    int upto = mark[kOnceItems - 1];
+    int upto = mark[ITEMS - 1];
 #pragma unroll
     for (int s = 1; s < kWave; s <<= 1) {
         const int n = __shfl_up(upto, s, kWave);
@@ -1845,10 +1839,10 @@ __global__ __launch_bounds__(kBlock) void csr_once_kernel(const int64_t *__restr
     for (int w = 0; w < kBlock / kWave; ++w)
         if (w < wave) before = max(before, waves[0][w]);
 #pragma unroll
-    for (int u = 0; u < kOnceItems; ++u) begins[threadIdx.x * kOnceItems + u] = max(mark[u], before);
+    for (int u = 0; u < ITEMS; ++u) begins[threadIdx.x * ITEMS + u] = max(mark[u], before);
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < kOnceItems; ++u) {
+    for (int u = 0; u < ITEMS; ++u) {
         const int k = u * kBlock + threadIdx.x;
         if (k < held) {
             col[e0 - first + k] = (int32_t)c[u];
@@ -2132,9 +2126,11 @@ extern "C" int cgnn_spmm_once(int64_t rows, int64_t nnz, const int64_t *rowptr, 
     const OnceLayout L = once_layout(rows, nnz, F, dtype);
     if (workspace == nullptr || workspace_bytes < L.total) return fail(CGNN_EWORKSPACE, "cgnn_spmm_once: workspace too small");
     char *ws = static_cast<char *>(workspace);
-    hipLaunchKernelGGL(csr_once_kernel, dim3((unsigned)ceil_div(rows + nnz, kOncePlaces)), dim3(kBlock), 0, stream,
-                       rowptr, col, rows, nnz, reinterpret_cast<int32_t *>(ws + L.rowptr), reinterpret_cast<int32_t *>(ws + L.col),
-                       reinterpret_cast<int32_t *>(ws + L.rowidx), reinterpret_cast<int32_t *>(ws + L.span));
+    const int items = once_items(rows + nnz);
+    hipLaunchKernelGGL(items == 4 ? csr_once_kernel<4> : csr_once_kernel<8>, dim3((unsigned)ceil_div(rows + nnz, items * kBlock)),
+                       dim3(kBlock), 0, stream, rowptr, col, rows, nnz, reinterpret_cast<int32_t *>(ws + L.rowptr),
+                       reinterpret_cast<int32_t *>(ws + L.col), reinterpret_cast<int32_t *>(ws + L.rowidx),
+                       reinterpret_cast<int32_t *>(ws + L.span));
     int rc = check_launch("csr_once");
     if (rc != CGNN_OK) return rc;
     if (dtype == CGNN_F32)

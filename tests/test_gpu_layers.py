@@ -892,6 +892,27 @@ def test_spmm_func_on_blocks_of_every_shape(shape, accumulate):
     assert np.array_equal(got[short], oracle.spmm(vlist, elist, value, x, out0.copy())[short])
 
 
+@pytest.mark.parametrize("rows, nnz", [(1, 5), (63, 1), (64, 4033), (65, 4096 - 65), (4097, 9999), (400000, 1172864), (400000, 1172865),
+                                       (1572000, 1000)])
+def test_spmm_func_of_any_length(rows, nnz):
+    """Blocks on both sides of the rows and entries that a workgroup and its search for them take, with a hub, a stretch of
+    empty rows and an empty last row.  Whole numbers, so every order of the sums gives the same bits."""
+    import compressgnn_runtime as rt
+    rng = np.random.default_rng(rows + nnz)
+    ends = np.sort(np.concatenate([rng.integers(0, nnz + 1, rows - rows // 3), np.full(rows // 3, nnz // 2)]))
+    vlist = np.concatenate([[0], ends]).astype(np.int64)
+    vlist[-2:] = nnz
+    vlist[0] = 0
+    elist = rng.integers(0, 500, nnz).astype(np.int64)
+    value = rng.integers(-3, 4, nnz).astype(np.float32)
+    x = rng.integers(-3, 4, (500, 4)).astype(np.float32)
+    sums = np.concatenate([np.zeros((1, 4)), np.cumsum(value[:, None] * x[elist].astype(np.float64), 0)])
+    want = (sums[vlist[1:]] - sums[vlist[:-1]]).astype(np.float32)
+    t = lambda a: torch.from_numpy(a).to(DEV)
+    for _ in range(2):
+        assert np.array_equal(rt.spmm_func(t(vlist), t(elist), t(value), t(x), "auto", None).cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("method", ["auto", "row_schedule", "nnz_schedule"])
 @pytest.mark.parametrize("hubs", [False, True])
 @pytest.mark.parametrize("rows", [(0, 3000), (1, 3000), (0, 2999), (1234, 1235), (700, 2900)])
