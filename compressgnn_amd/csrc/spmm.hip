@@ -56,6 +56,8 @@ namespace {
 
 constexpr int kUnroll = 4;        // gathers in flight per lane and tile, nnz schedule (with 7 waves per SIMD;
                                   // 8 in flight with 5 waves measured the same)
+constexpr int kMidRound = 8, kDeepRound = 16;  // ... where a launch has few workgroups (launch_nnz)
+constexpr int64_t kResidentWorkgroups = 256 * 7;  // of the nnz kernel on the card at once, with kUnroll
 constexpr int kRowUnroll = 4;     // same for the row schedule (8: 9 % slower on web-graph out-lists, 2: 13 %, 16: 38 %)
 constexpr int kXcds = 8;          // accelerator dies of an MI355X, each with its own L2
 constexpr int kDefaultSeg = 64;   // non-zeros per lane group in the nnz schedule
@@ -718,9 +720,11 @@ __device__ __forceinline__ void join_rows(const SpmmArgs<T> &a, int block, int l
     }
 }
 
-template <typename T, int VEC, int LPR, int TILES, int MODE, int WGRUNS>
-__global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spmm_nnz_kernel(SpmmArgs<T> a) {
+template <typename T, int VEC, int LPR, int TILES, int MODE, int WGRUNS, int ROUND>
+__global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRound ? 5 : (TILES == 1 && LPR >= 16) ? 7 : 1) void spmm_nnz_kernel(SpmmArgs<T> a) {
     constexpr int GPB = kBlock / LPR;
+    static_assert(LPR % ROUND == 0 || ROUND == kUnroll, "a round's entries come from one batch");
+    constexpr bool kAhead = ROUND == kDeepRound;  // the entries of the next batch are asked for before the gathers of this one
     __shared__ int wg_row[GPB];
     __shared__ Pack<T, VEC> wg_carry[TILES][kBlock];
     __shared__ Pack<T, VEC> wg_head[WGRUNS != WGRUNS_NONE ? TILES : 1][WGRUNS != WGRUNS_NONE ? kBlock : 1];
@@ -816,16 +820,20 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
             int64_t fld[TILES];  // lanes beyond the width gather feature 0 again (never stored)
 #pragma unroll
             for (int t = 0; t < TILES; ++t) fld[t] = foff[t] < 0 ? 0 : foff[t];
+            int my_row = 0, my_c = 0;
+            T my_w = T(1);
+            auto load_entry = [&](int e) {  // this lane's of the batch from e on
+                my_row = 0, my_c = 0, my_w = T(1);
+                if (e + lane >= e1) return;
+                my_row = a.rowidx[e + lane];
+                my_c = a.colidx[e + lane];
+                if constexpr (MODE == MODE_DUAL) my_w = a.val[e + lane];
+                if constexpr (has_values(MODE)) my_w = a.val != nullptr ? a.val[e + lane] : T(1);
+            };
+            if constexpr (kAhead) load_entry(e0);
             for (int e = e0; e < e1; e += LPR) {
-                int my_o = 0, my_c = 0;
-                T my_w = T(1);
-                if (e + lane < e1) {
-                    const int row = a.rowidx[e + lane];
-                    my_c = a.colidx[e + lane];
-                    if constexpr (MODE == MODE_DUAL) my_w = a.val[e + lane];
-                    if constexpr (has_values(MODE)) my_w = a.val != nullptr ? a.val[e + lane] : T(1);
-                    my_o = named(row);  // behind the others: it waits for the row
-                }
+                if constexpr (!kAhead) load_entry(e);
+                int my_o = e + lane < e1 ? named(my_row) : 0;  // behind the others: it waits for the row
                 if constexpr (kNamesRowsOfY) {
                     // with every batch of entries, so that no load of the run waits for another but
                     // the row numbers for their rows (the same two words each time)
@@ -840,16 +848,19 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                 if constexpr (MODE != MODE_DUAL) arrive(my_o), arrive(my_c);
                 if constexpr (has_values(MODE)) arrive(my_w);
                 const int cnt = min(e1 - e, LPR);
-                for (int u0 = 0; u0 < cnt; u0 += kUnroll) {
-                    int o[kUnroll], c[kUnroll];
-                    T w[kUnroll];
+                const int this_c = my_c;
+                const T this_w = my_w;
+                if constexpr (kAhead) load_entry(e + LPR);
+                for (int u0 = 0; u0 < cnt; u0 += ROUND) {
+                    int o[ROUND], c[ROUND];
+                    T w[ROUND];
 #pragma unroll
-                    for (int u = 0; u < kUnroll; ++u) {
+                    for (int u = 0; u < ROUND; ++u) {
                         const int from = group_lane0 + 4 * (u0 + u);
                         o[u] = __builtin_amdgcn_ds_bpermute(from, my_o);
-                        c[u] = __builtin_amdgcn_ds_bpermute(from, my_c);
+                        c[u] = __builtin_amdgcn_ds_bpermute(from, this_c);
                         if constexpr (has_values(MODE) || MODE == MODE_DUAL)
-                            w[u] = __builtin_bit_cast(T, __builtin_amdgcn_ds_bpermute(from, __builtin_bit_cast(int, my_w)));
+                            w[u] = __builtin_bit_cast(T, __builtin_amdgcn_ds_bpermute(from, __builtin_bit_cast(int, this_w)));
                         else
                             w[u] = T(1);
                     }
@@ -860,17 +871,17 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                     bool second = false;
                     if constexpr (MODE == MODE_DUAL) {
 #pragma unroll
-                        for (int u = 0; u < kUnroll; ++u) second = second | (c[u] >= a.split);
+                        for (int u = 0; u < ROUND; ++u) second = second | (c[u] >= a.split);
                     }
                     auto gather_and_add = [&](auto plain) {
                         constexpr bool kPlain = decltype(plain)::value;  // every entry from the first source
-                        Gathered<T, VEC, MODE> x[kUnroll][TILES];
+                        Gathered<T, VEC, MODE> x[ROUND][TILES];
                         // Up to 64 bytes per lane group and gather, a position behind the last entry gathers
                         // like the others (column 0, see above): the branches around four small loads cost
                         // more than the loads.  Wider rows skip it: there the extra row is what costs.
                         constexpr bool kGatherAll = VEC * LPR * sizeof(T) <= 64;
 #pragma unroll
-                        for (int u = 0; u < kUnroll; ++u)
+                        for (int u = 0; u < ROUND; ++u)
                             if (kGatherAll || u0 + u < cnt) {
 #pragma unroll
                                 for (int t = 0; t < TILES; ++t)
@@ -878,11 +889,11 @@ __global__ __launch_bounds__(kBlock, (TILES == 1 && LPR >= 16) ? 7 : 1) void spm
                             }
                         if constexpr (MODE != MODE_DUAL && !(kGatherAll && !has_values(MODE)))
 #pragma unroll
-                            for (int u = 0; u < kUnroll; ++u)
+                            for (int u = 0; u < ROUND; ++u)
 #pragma unroll
                                 for (int t = 0; t < TILES; ++t) arrive(x[u][t]);
 #pragma unroll
-                        for (int u = 0; u < kUnroll; ++u) {
+                        for (int u = 0; u < ROUND; ++u) {
                             if (u0 + u < cnt) {
                                 if (o[u] != cur_out) {
                                     // the row ends inside this run: finish it here
@@ -1343,6 +1354,76 @@ Shape shape_of(int64_t F, int dtype) { return dtype == CGNN_F64 ? pick_shape<dou
 
 enum { KIND_ROW = 0, KIND_NNZ = 1, KIND_FIXUP = 2, KIND_REDUCE = 3, KIND_FIXUP_ROWS = 4 };
 
+// How many gathers a lane of the nnz schedule has in flight.  A row of up to kDefaultSeg entries is added by one lane group,
+// and where a launch has few workgroups its time is that of the longest run: a batch of entries, then its gathers
+// kUnroll at a time, each round waiting for memory.  With kDeepRound the gathers of 16 entries are one round, and the next
+// batch of entries is on its way meanwhile; the registers for that leave two workgroups a compute unit.  us, with kUnroll / so:
+// means of 30,011 rows of 64 columns in 7,584 groups 37.8 / 31.3, sums 16.8 / 12.9, masked sums 20.9 / 17.3; 9,000 rows of
+// 100: 35.2 / 30.4, 18.3 / 14.5, 21.3 / 18.2; 2,708 of 64: 23.2 / 21.6, 11.0 / 10.1, 15.3 / 14.8.  Beyond 512 workgroups the means,
+// whose runs are 64 entries long, would wait for a second round of workgroups (300,007 rows of 100 36.2, with kMidRound 34.8,
+// with kUnroll 39.0); the runs of the others are as short as fills the card, and they gain up to 1,024 (sums of 100,003
+// rows of 64 21.5 / 17.8, masked 25.5 / 22.0; a product over 8,000 rows with hubs 19.6 / 18.7).  Unmasked sums take kMidRound where
+// the card holds all workgroups at once, up to 3 * 2^18 entries (300,007 rows of 64 27.4 / 25.0, 600,000 38.5 / 36.3, means
+// 40.7 / 38.5; at 1,000,003, where enough lane groups gather in any case, 49.3 / 51.0 and 49.2 / 50.2); masked ones do not gain by it
+// (100,003 rows of 100 28.5 / 29.7), nor do the products of a plan with kDeepRound (5,000 rows of 64 9.4 / 10.1).
+template <int MODE, int WGRUNS>
+constexpr bool kGoesDeep = MODE == MODE_UNIT || MODE == MODE_SIGN_MASK || (has_values(MODE) && WGRUNS == WGRUNS_COMPUTED);
+
+template <int MODE, int WGRUNS>
+int round_of(int64_t workgroups, int64_t entries) {
+    if (kGoesDeep<MODE, WGRUNS> && workgroups <= (WGRUNS == WGRUNS_NONE ? 512 : 1024)) return kDeepRound;
+    return MODE == MODE_UNIT && workgroups <= kResidentWorkgroups && entries <= 3 << 18 ? kMidRound : kUnroll;
+}
+
+template <typename T, int VEC, int LPR, int TILES>
+void launch_nnz(int mode, const SpmmArgs<T> &a, dim3 grid, hipStream_t stream) {
+    auto go = [&](auto m, auto runs) {
+        constexpr int kMode = decltype(m)::value, kRuns = decltype(runs)::value;
+        const dim3 block(kBlock);
+        if constexpr (sizeof(T) == 4 && LPR >= kDeepRound && TILES == 1) {
+            const int round = round_of<kMode, kRuns>((int64_t)grid.x * grid.y, a.nnz);
+            if constexpr (kGoesDeep<kMode, kRuns>)
+                if (round == kDeepRound) {
+                    hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, kMode, kRuns, kDeepRound>), grid, block, 0, stream, a);
+                    return;
+                }
+            if constexpr (kMode == MODE_UNIT)
+                if (round == kMidRound) {
+                    hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, kMode, kRuns, kMidRound>), grid, block, 0, stream, a);
+                    return;
+                }
+        }
+        hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, kMode, kRuns, kUnroll>), grid, block, 0, stream, a);
+    };
+    const std::integral_constant<int, MODE_VAL> val;
+    const std::integral_constant<int, MODE_ADD> add;
+    const std::integral_constant<int, MODE_UNIT> unit;
+    const std::integral_constant<int, MODE_DUAL> dual;
+    const std::integral_constant<int, MODE_SIGN_MASK> sign_mask;
+    const std::integral_constant<int, MODE_RELU_MASK> relu_mask;
+    if (a.arrivals != nullptr && a.run_start == nullptr) {
+        const std::integral_constant<int, WGRUNS_COMPUTED> computed;
+        if (mode == MODE_UNIT) go(unit, computed);
+        else if (mode == MODE_VAL && a.accumulate) go(add, computed);
+        else if (mode == MODE_VAL) go(val, computed);
+        else if (mode == MODE_SIGN_MASK) go(sign_mask, computed);
+        else go(relu_mask, computed);
+    } else if (a.arrivals != nullptr) {
+        const std::integral_constant<int, WGRUNS_TABLE> table;
+        if (mode == MODE_DUAL) go(dual, table);
+        else if (a.accumulate) go(add, table);
+        else go(val, table);
+    } else {
+        const std::integral_constant<int, WGRUNS_NONE> none;
+        if (mode == MODE_VAL && a.accumulate) go(add, none);
+        else if (mode == MODE_VAL) go(val, none);
+        else if (mode == MODE_UNIT) go(unit, none);
+        else if (mode == MODE_DUAL) go(dual, none);
+        else if (mode == MODE_SIGN_MASK) go(sign_mask, none);
+        else go(relu_mask, none);
+    }
+}
+
 template <typename T, int VEC, int LPR, int TILES>
 int launch_shape(int kind, int mode, const SpmmArgs<T> &args, int64_t items, int grid_y, hipStream_t stream) {
     constexpr int GPB = kBlock / LPR;
@@ -1365,35 +1446,7 @@ int launch_shape(int kind, int mode, const SpmmArgs<T> &args, int64_t items, int
                 hipLaunchKernelGGL((spmm_row_kernel<T, VEC, LPR, TILES, MODE_VAL>), grid, block, 0, stream, a);
             break;
         case KIND_NNZ:
-            if (a.arrivals != nullptr && a.run_start == nullptr) {
-                if (mode == MODE_UNIT)
-                    hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_UNIT, WGRUNS_COMPUTED>), grid, block, 0, stream, a);
-                else if (mode == MODE_VAL && a.accumulate)
-                    hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_ADD, WGRUNS_COMPUTED>), grid, block, 0, stream, a);
-                else if (mode == MODE_VAL)
-                    hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_VAL, WGRUNS_COMPUTED>), grid, block, 0, stream, a);
-                else if (mode == MODE_SIGN_MASK)
-                    hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_SIGN_MASK, WGRUNS_COMPUTED>), grid, block, 0, stream, a);
-                else
-                    hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_RELU_MASK, WGRUNS_COMPUTED>), grid, block, 0, stream, a);
-            } else if (a.arrivals != nullptr && mode == MODE_DUAL)
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_DUAL, WGRUNS_TABLE>), grid, block, 0, stream, a);
-            else if (a.arrivals != nullptr && a.accumulate)
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_ADD, WGRUNS_TABLE>), grid, block, 0, stream, a);
-            else if (a.arrivals != nullptr)
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_VAL, WGRUNS_TABLE>), grid, block, 0, stream, a);
-            else if (mode == MODE_VAL && a.accumulate)
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_ADD, WGRUNS_NONE>), grid, block, 0, stream, a);
-            else if (mode == MODE_VAL)
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_VAL, WGRUNS_NONE>), grid, block, 0, stream, a);
-            else if (mode == MODE_UNIT)
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_UNIT, WGRUNS_NONE>), grid, block, 0, stream, a);
-            else if (mode == MODE_DUAL)
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_DUAL, WGRUNS_NONE>), grid, block, 0, stream, a);
-            else if (mode == MODE_SIGN_MASK)
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_SIGN_MASK, WGRUNS_NONE>), grid, block, 0, stream, a);
-            else
-                hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, MODE_RELU_MASK, WGRUNS_NONE>), grid, block, 0, stream, a);
+            launch_nnz<T, VEC, LPR, TILES>(mode, a, grid, stream);
             break;
         case KIND_FIXUP: {  // a lane group per carry, and (when not accumulating) a thread per row
             const int64_t for_rows = a.accumulate ? 0 : ceil_div((int64_t)a.rows, kBlock);
@@ -1547,7 +1600,6 @@ size_t wg_piece_bytes(int64_t workgroups, int64_t F, size_t elt) { return 2 * (s
 // product is nothing but the time of its longest chain; not under 8 (two rounds: below that the ends of a
 // run cost more than its entries); where they would be longer than `most`, the block's run length, of which several fill
 // the card one after the other.
-constexpr int64_t kResidentWorkgroups = 256 * 7;
 
 int wg_run_len(const cgnn_csr *A, int groups, int most) {
     const int64_t fill = ceil_div(ceil_div(A->nnz, kResidentWorkgroups * groups), kUnroll) * kUnroll;

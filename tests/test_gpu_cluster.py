@@ -261,6 +261,31 @@ def test_grouped_assign_of_any_length(n, bits):
         assert np.array_equal(offsets, np.concatenate([[0], np.cumsum(counts)]))
 
 
+@pytest.mark.parametrize("n, width", [(300, 47), (2049, 64), (30011, 256), (131072, 64), (131073, 64), (262145, 128), (524288, 64), (524289, 64),
+                                      (524289, 16), (786432, 64), (786433, 64), (1835009, 16)])
+def test_means_and_sums_with_any_number_of_workgroups(n, width):
+    """Lists whose launches have few, some and many workgroups (their lanes then have more or fewer gathers in flight), with
+    groups from one row to a tenth of them.  Whole numbers: the sums are exact in any order."""
+    import compressgnn_runtime as rt
+    gen = torch.Generator(device=DEV).manual_seed(n)
+    ids = torch.randint(0, 3000, (n,), device=DEV, generator=gen)
+    ids[torch.randint(0, n, (n // 8,), device=DEV, generator=gen)] = 7
+    ids = torch.unique(ids, return_inverse=True)[1]
+    groups = int(ids.max()) + 1
+    x = torch.randint(-4, 5, (n, width), device=DEV, generator=gen).float()
+    index = ids, abi.cluster_members(ids, groups)
+    counts = torch.bincount(ids, minlength=groups)
+    sums = torch.zeros(groups, width, device=DEV).index_add_(0, ids, x)
+    biased = torch.randint(-1, 2, (groups, width), device=DEV, generator=gen).float()
+    out, signs = rt.cluster_reconstruct_signs(biased, ids, torch.zeros(width, device=DEV), list(index[1]))
+    masked = torch.zeros(groups, width, device=DEV).index_add_(0, ids, x * (out > 0))
+    for _ in range(2):
+        mean = rt.cluster_mean(x, ids, counts.int(), list(index[1]))
+        assert torch.equal(mean, sums / counts[:, None])
+        assert torch.equal(rt.cluster_reconstruct_backward(x, ids, x, groups, False, list(index[1])), sums)
+        assert torch.equal(rt.cluster_reconstruct_backward_signs(x, ids, signs, groups, list(index[1])), masked)
+
+
 def test_grouped_assign_empty():
     ids, counts, active, members = abi.lsh_assign_grouped(torch.zeros(0, 8, device=DEV), torch.randn(8, 8, device=DEV), 8)
     assert ids.numel() == 0 and active == 0 and counts.tolist() == [0] and members[0].tolist() == [0, 0]
