@@ -591,6 +591,11 @@ __device__ __forceinline__ void bounded_summary(const BoundedArgs &a, int32_t sa
     __hip_atomic_store(a.summary + 3, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// The vertices in the next layer's frontier.  None once a list did not fit its degree: its slots were cleared behind its
+// claims, which no slot of this layer answers to, and the next layer would take them off counts that are not theirs.  The
+// call is done again layer by layer in any case.
+__device__ __forceinline__ int32_t bounded_frontier(const BoundedArgs &a, int32_t introduced) { return a.status[1] ? 0 : introduced; }
+
 // How many neighbours a chunk holds and how many vertices they introduce; the last chunk to be counted sums the
 // chunks up and sets the state of the next layer.
 __global__ __launch_bounds__(kBlock) void bounded_count_kernel(BoundedArgs a) {
@@ -632,7 +637,7 @@ __global__ __launch_bounds__(kBlock) void bounded_count_kernel(BoundedArgs a) {
     if (threadIdx.x == 0) {
         const int32_t end = state[0] + (int32_t)n;
         state[4] = end;
-        state[5] = running.y;
+        state[5] = bounded_frontier(a, running.y);
         state[6] = state[2] + running.x;
         if (a.layer == a.layers - 1) bounded_summary(a, end + running.y, state[2] + running.x);
     }
@@ -668,7 +673,7 @@ __global__ __launch_bounds__(kBlock) void bounded_assign_kernel(BoundedArgs a) {
             l.before[blockIdx.x] = (uint64_t)all_before.y << 32 | (uint32_t)all_before.x;
             if (blockIdx.x == 0) {
                 state[4] = end;
-                state[5] = all_behind.y;
+                state[5] = bounded_frontier(a, all_behind.y);
                 state[6] = state[2] + all_behind.x;
                 if (a.layer == a.layers - 1) bounded_summary(a, end + all_behind.y, state[2] + all_behind.x);
             }

@@ -291,6 +291,25 @@ def test_layers_counted_while_they_are_filled(seeds, fan):
             assert np.array_equal(a.cpu().numpy(), w)
 
 
+@pytest.mark.parametrize("seeds", [40, 4096, 140000])
+def test_layers_behind_a_list_that_does_not_fit_its_degree(seeds):
+    """The claims of a list that turns out longer than its degree stay with the vertices it names, at slots that the next
+    layer, here of one chunk, does not have: that layer has to be left out, and the call done again layer by layer.  In
+    counted layers and in one that a launch of its own counts in front of a counted one (140,000 seeds with 64)."""
+    rng = np.random.default_rng(seeds)
+    V, R = 300, 70
+    csr = lambda lists: (np.concatenate([[0], np.cumsum([len(x) for x in lists])]).astype(np.int64),
+                         np.array([y for x in lists for y in x], np.int64))
+    v2v = [list(rng.integers(100, 200, 12)) if v < 100 else list(rng.integers(200, 210, 3)) for v in range(V)]
+    v2v[0] = list(range(200, 210))
+    v2r = [list(range(R)) if v == 0 else [] for v in range(V)]  # more rules than lanes, all of them empty
+    b = dict(v2v=csr(v2v), v2r=csr(v2r), r2v=csr([[] for _ in range(R)]), r2r=[],
+             v_degree=np.array([len(x) for x in v2v], np.int64), r_degree=np.zeros(R, np.int64))
+    inp = np.concatenate([rng.integers(1, 100, seeds - 1), [0]])
+    for fan in ([16, 1], [64, 1, 2]):
+        check(b, on_device(b), inp, fan, seed=seeds)
+
+
 @pytest.mark.parametrize("rows", [1 << 19, (1 << 19) + 1])
 def test_layers_at_the_limit_of_the_slots_and_without_room_for_them(rows):
     """As many slots as a call with one host read may have, and one vertex more; and a call that finds no room for its
