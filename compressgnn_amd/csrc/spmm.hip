@@ -1362,16 +1362,18 @@ enum { KIND_ROW = 0, KIND_NNZ = 1, KIND_FIXUP = 2, KIND_REDUCE = 3, KIND_FIXUP_R
 // 100: 35.2 / 30.4, 18.3 / 14.5, 21.3 / 18.2; 2,708 of 64: 23.2 / 21.6, 11.0 / 10.1, 15.3 / 14.8.  Beyond 512 workgroups the means,
 // whose runs are 64 entries long, would wait for a second round of workgroups (300,007 rows of 100 36.2, with kMidRound 34.8,
 // with kUnroll 39.0); the runs of the others are as short as fills the card, and they gain up to 1,024 (sums of 100,003
-// rows of 64 21.5 / 17.8, masked 25.5 / 22.0; a product over 8,000 rows with hubs 19.6 / 18.7).  Unmasked sums take kMidRound where
+// rows of 64 21.5 / 17.8, masked 25.5 / 22.0).  Unmasked sums take kMidRound where
 // the card holds all workgroups at once, up to 3 * 2^18 entries (300,007 rows of 64 27.4 / 25.0, 600,000 38.5 / 36.3, means
 // 40.7 / 38.5; at 1,000,003, where enough lane groups gather in any case, 49.3 / 51.0 and 49.2 / 50.2); masked ones do not gain by it
-// (100,003 rows of 100 28.5 / 29.7), nor do the products of a plan with kDeepRound (5,000 rows of 64 9.4 / 10.1).
-template <int MODE, int WGRUNS>
-constexpr bool kGoesDeep = MODE == MODE_UNIT || MODE == MODE_SIGN_MASK || (has_values(MODE) && WGRUNS == WGRUNS_COMPUTED);
+// (100,003 rows of 100 28.5 / 29.7), nor do the products of a plan with kDeepRound (5,000 rows of 64 9.4 / 10.1).  Those of a
+// block that is new with the call gain where hubs make long runs (8,000 rows 19.6 / 18.7) and lose where rows are short
+// (out-lists of 5,463 vertices, 208 features, the whole pass 14.3 / 16.7), which nothing tells apart before the launch.
+template <int MODE>
+constexpr bool kGoesDeep = MODE == MODE_UNIT || MODE == MODE_SIGN_MASK;
 
 template <int MODE, int WGRUNS>
 int round_of(int64_t workgroups, int64_t entries) {
-    if (kGoesDeep<MODE, WGRUNS> && workgroups <= (WGRUNS == WGRUNS_NONE ? 512 : 1024)) return kDeepRound;
+    if (kGoesDeep<MODE> && workgroups <= (WGRUNS == WGRUNS_NONE ? 512 : 1024)) return kDeepRound;
     return MODE == MODE_UNIT && workgroups <= kResidentWorkgroups && entries <= 3 << 18 ? kMidRound : kUnroll;
 }
 
@@ -1382,7 +1384,7 @@ void launch_nnz(int mode, const SpmmArgs<T> &a, dim3 grid, hipStream_t stream) {
         const dim3 block(kBlock);
         if constexpr (sizeof(T) == 4 && LPR >= kDeepRound && TILES == 1) {
             const int round = round_of<kMode, kRuns>((int64_t)grid.x * grid.y, a.nnz);
-            if constexpr (kGoesDeep<kMode, kRuns>)
+            if constexpr (kGoesDeep<kMode>)
                 if (round == kDeepRound) {
                     hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, kMode, kRuns, kDeepRound>), grid, block, 0, stream, a);
                     return;
