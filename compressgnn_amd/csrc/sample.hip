@@ -30,8 +30,8 @@
 // frontier vertex i stand in slots i * fan-out ..., whose order is the order of the list, so that nothing is summed up
 // before they are drawn; the sizes stay on the device, every launch covers the most there can be, and the
 // host reads once, when the outputs have to be allocated.  One mini-batch of 1,024 seeds with fan-outs 25 and 10
-// took 47 launches and four host reads (256 us) layer by layer; it takes eight and one (60 us);
-// 16,384 seeds with 25 and 15 went from 384 to 105 us, most of it the chains of loads through the rules.
+// took 47 launches and four host reads (256 us) layer by layer; it takes six and one (57 us);
+// 16,384 seeds with 25 and 15 went from 384 to 93 us, most of it the chains of loads through the rules.
 #include "common.h"
 
 namespace cgnn {
