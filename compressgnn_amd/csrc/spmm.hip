@@ -1966,6 +1966,57 @@ __global__ __launch_bounds__(kBlock) void expand_count_kernel(const int32_t *__r
     if (lane == 0) counts[row] = (int32_t)min(n, (int64_t)INT32_MAX);
 }
 
+// The magnitudes of a value as bits, in whose order they are.
+__device__ __forceinline__ uint64_t magnitude(float v) { return __float_as_uint(v) & 0x7fffffffu; }
+__device__ __forceinline__ uint64_t magnitude(double v) { return (uint64_t)__double_as_longlong(v) & 0x7fffffffffffffffull; }
+
+__global__ void expand_range_begin_kernel(uint64_t *__restrict__ out) {
+    if (threadIdx.x < 4) out[threadIdx.x] = threadIdx.x % 2 == 0 ? 0 : ~uint64_t(0);
+}
+
+// out: largest and smallest non-zero magnitude of the values that stand for rules, and of the rules' values
+// (cgnn_csr_expand_range).  Integer extremes, any order.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void expand_range_kernel(const int32_t *__restrict__ col, const T *__restrict__ val, int64_t nnz,
+                                                              int32_t split, const T *__restrict__ rule_val, int64_t rule_nnz,
+                                                              unsigned long long *__restrict__ out) {
+    constexpr int kWaves = kBlock / kWave;
+    __shared__ unsigned long long found[4][kWaves];
+    unsigned long long most[2] = {0, 0}, least[2] = {~0ull, ~0ull};
+    auto look = [&](int k, T v) {
+        const unsigned long long m = magnitude(v);
+        most[k] = max(most[k], m);
+        if (m != 0) least[k] = min(least[k], m);
+    };
+    const int64_t stride = (int64_t)gridDim.x * kBlock, t0 = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+#pragma unroll 4
+    for (int64_t e = t0; e < nnz; e += stride)
+        if (col[e] >= split) look(0, val[e]);
+    if (rule_val != nullptr)
+#pragma unroll 4
+        for (int64_t e = t0; e < rule_nnz; e += stride) look(1, rule_val[e]);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+#pragma unroll
+        for (int s = kWave / 2; s > 0; s >>= 1) {
+            most[k] = max(most[k], (unsigned long long)__shfl_xor(most[k], s, kWave));
+            least[k] = min(least[k], (unsigned long long)__shfl_xor(least[k], s, kWave));
+        }
+        if (threadIdx.x % kWave == 0) found[2 * k][threadIdx.x / kWave] = most[k], found[2 * k + 1][threadIdx.x / kWave] = least[k];
+    }
+    __syncthreads();
+    if (threadIdx.x < 4) {
+        unsigned long long v = found[threadIdx.x][0];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) {
+            const unsigned long long other = found[threadIdx.x][w];
+            v = threadIdx.x % 2 == 0 ? max(v, other) : min(v, other);
+        }
+        if (threadIdx.x % 2 == 0) atomicMax(out + threadIdx.x, v);
+        else atomicMin(out + threadIdx.x, v);
+    }
+}
+
 template <typename T>
 __global__ __launch_bounds__(kBlock) void expand_columns_kernel(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col,
                                                                 const T *__restrict__ val, int32_t rows, int32_t split,
@@ -2381,6 +2432,27 @@ extern "C" int cgnn_csr_expand_count(const cgnn_csr *A, int64_t split, const cgn
     hipLaunchKernelGGL(expand_count_kernel, dim3((unsigned)ceil_div(A->rows, kBlock / kWave)), dim3(kBlock), 0, stream,
                        A->rowptr, A->colidx, (int32_t)A->rows, (int32_t)split, rules->rowptr, counts);
     return check_launch("csr_expand_count");
+}
+
+extern "C" int cgnn_csr_expand_range(const cgnn_csr *A, int64_t split, const cgnn_csr *rules, int dtype, uint64_t *magnitudes,
+                                     cgnn_stream_t stream) {
+    int rc = check_expand(A, split, rules);
+    if (rc != CGNN_OK) return rc;
+    CGNN_REQUIRE(dtype == CGNN_F32 || dtype == CGNN_F64, "cgnn_csr_expand_range: dtype must be f32 or f64");
+    CGNN_REQUIRE(magnitudes != nullptr && (A->nnz == 0 || A->val != nullptr), "cgnn_csr_expand_range: null array");
+    hipLaunchKernelGGL(expand_range_begin_kernel, dim3(1), dim3(kWave), 0, stream, magnitudes);
+    const int64_t entries = std::max(A->nnz, rules->val != nullptr ? rules->nnz : 0);
+    if (entries == 0) return check_launch("csr_expand_range");
+    const dim3 grid((unsigned)std::min<int64_t>(ceil_div(entries, 4 * kBlock), 256));
+    auto run = [&](auto zero) {
+        typedef decltype(zero) T;
+        hipLaunchKernelGGL(expand_range_kernel<T>, grid, dim3(kBlock), 0, stream, A->colidx, static_cast<const T *>(A->val), A->nnz,
+                           (int32_t)split, static_cast<const T *>(rules->val), rules->nnz,
+                           reinterpret_cast<unsigned long long *>(magnitudes));
+    };
+    if (dtype == CGNN_F32) run(0.0f);
+    else run(0.0);
+    return check_launch("csr_expand_range");
 }
 
 extern "C" int cgnn_csr_expand_columns(const cgnn_csr *A, int64_t split, const cgnn_csr *rules, int dtype, const int32_t *rowptr,

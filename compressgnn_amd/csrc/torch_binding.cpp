@@ -21,9 +21,11 @@
 #include <atomic>
 #include <chrono>
 #include <climits>
+#include <cmath>
 #include <cstring>
 #include <deque>
 #include <functional>
+#include <limits>
 #include <memory>
 #include <mutex>
 #include <sstream>
@@ -557,7 +559,23 @@ bool takes_whole(int64_t entries, const DeviceCsr &stage, const DeviceCsr &rules
     return more <= (row_schedule ? kRuleStageBytesRowSchedule : kRuleStageBytes);
 }
 
-// [vertices | rules] with the rules multiplied out, or NULL where no product would take it.
+// Whether every product of a value that stands for a rule and a value of the rules has a place in the type T, by the
+// extremes of both (cgnn_csr_expand_range).  A multiplied-out block stores these products; the stages multiply through
+// the sums of the rules, and factors like 1e-25 and 1e-25, or 1e25 and 1e25, are theirs.
+template <typename T>
+bool products_in_range(const uint64_t *magnitudes) {
+    long double of[4];
+    for (int k = 0; k < 4; ++k) {
+        if (magnitudes[k] == UINT64_MAX) return true;  // all zero, or none
+        T v;
+        std::memcpy(&v, &magnitudes[k], sizeof(T));  // the low half comes first
+        of[k] = v;
+    }
+    return std::isfinite(of[0]) && std::isfinite(of[2]) && of[0] * of[2] <= std::numeric_limits<T>::max() &&
+           of[1] * of[3] >= std::numeric_limits<T>::min();
+}
+
+// [vertices | rules] with the rules multiplied out, or NULL where no product would take it or a value has no place in it.
 std::shared_ptr<DeviceCsr> multiplied_out(const DeviceCsr &stage, const DeviceCsr &rules, int64_t V) {
     if (stage.rows == 0 || stage.nnz == 0 || rules.nnz == 0 || !stage.val.defined() || stage.nnz > kMaxWholeEntries ||
         (rules.val.defined() && rules.val.scalar_type() != stage.val.scalar_type()) || capturing(stage.rowptr))
@@ -571,8 +589,16 @@ std::shared_ptr<DeviceCsr> multiplied_out(const DeviceCsr &stage, const DeviceCs
     ok(cgnn_exclusive_sum_i32(stage.rows, counts.data_ptr<int32_t>(), starts.data_ptr<int32_t>(), nullptr, ws.data_ptr(), ws.numel(),
                               stream),
        "exclusive_sum");
-    const int64_t entries = starts[stage.rows].item<int32_t>();
+    Tensor found = torch::empty({5}, stage.rowptr.options().dtype(torch::kInt64));
+    ok(cgnn_csr_expand_range(&a, V, &r, dtype_code(stage.val), reinterpret_cast<uint64_t *>(found.data_ptr<int64_t>() + 1), stream),
+       "csr_expand_range");
+    found.narrow(0, 0, 1).copy_(starts.narrow(0, stage.rows, 1));
+    found = found.cpu();
+    const int64_t entries = found.data_ptr<int64_t>()[0];
     if (entries > kMaxWholeEntries || !takes_whole(entries, stage, rules, stage.val.element_size())) return nullptr;
+    const uint64_t *magnitudes = reinterpret_cast<const uint64_t *>(found.data_ptr<int64_t>() + 1);
+    if (!(stage.val.scalar_type() == torch::kFloat32 ? products_in_range<float>(magnitudes) : products_in_range<double>(magnitudes)))
+        return nullptr;
     Tensor col = torch::empty({entries}, stage.colidx.options()), val = torch::empty({entries}, stage.val.options());
     ok(cgnn_csr_expand_columns(&a, V, &r, dtype_code(stage.val), starts.data_ptr<int32_t>(), col.data_ptr<int32_t>(), val.data_ptr(),
                                stream),

@@ -213,8 +213,16 @@ int cgnn_csr_compose_columns(int64_t nnz, const int32_t *colidx, int64_t first_c
  * place; the other entries stay.  cgnn_csr_expand_count writes the entries every row of A comes to (INT32_MAX if more
  * do not fit), cgnn_csr_expand_columns the new columns and values for the row starts that these sum up to
  * (cgnn_exclusive_sum_i32; no sum may have overflowed).  A needs values; its rowidx and rowmap are not looked at.
- * The product of the vertex stage of layer/CompressgnnSPMM.py:59-60 with its rule stage (:54) as one matrix. */
+ * The product of the vertex stage of layer/CompressgnnSPMM.py:59-60 with its rule stage (:54) as one matrix.
+ *
+ * w * v is rounded to the block's type before it meets a row of features, where the two stages multiply through the sum
+ * over the rule: factors whose product the type does not hold give zeros, infinities and NaN where the stages have finite
+ * sums.  cgnn_csr_expand_range writes magnitudes[4]: the largest and the smallest non-zero |w| of the entries with c >=
+ * split, as the bits of the type (in the low half where that is float32), and the same of the values of `rules`; 0 and
+ * UINT64_MAX where there are none.  The order of the bits is that of the magnitudes, with infinity and NaN above all others. */
 int cgnn_csr_expand_count(const cgnn_csr *A, int64_t split, const cgnn_csr *rules, int32_t *counts, cgnn_stream_t stream);
+int cgnn_csr_expand_range(const cgnn_csr *A, int64_t split, const cgnn_csr *rules, int dtype, uint64_t *magnitudes,
+                          cgnn_stream_t stream);
 int cgnn_csr_expand_columns(const cgnn_csr *A, int64_t split, const cgnn_csr *rules, int dtype, const int32_t *rowptr,
                             int32_t *colidx, void *val, cgnn_stream_t stream);
 

@@ -274,6 +274,69 @@ def test_rules_multiplied_out_or_in_stages(F, one_launch):
     assert_within(grad.cpu().numpy(), plan.backward(g).cpu().numpy(), rtol=1e-5, atol=1e-6)
 
 
+def _plan_over(dtype, near, far, rules):
+    """A propagation plan over device arrays of its own, [near | far] its vertex stage and `rules` its rule stage (scipy
+    matrices): (plan, the values of the rule stage, of its transpose, of the vertex stage, of its transpose)."""
+    import scipy.sparse as sp
+    import compressgnn_runtime as rt
+    (R, V), values, blocks = rules.shape, [], []
+    for m in (rules, far.T, sp.hstack([near, far]), sp.hstack([near.T, rules.T])):
+        m = m.tocsr()
+        m.sort_indices()
+        rowptr, col, val = (torch.from_numpy(a.astype(kind)).to(DEV)
+                            for a, kind in ((m.indptr, np.int32), (m.indices, np.int32), (m.data, dtype)))
+        values.append(val)
+        blocks.append(rt.DeviceCsr(rowptr, col, val, m.shape[0], m.shape[1], torch.device(DEV), 32))
+    plan = rt.PropagationPlan(V, R, blocks[0], [], blocks[1], [])
+    plan.set_vertex_stages(blocks[2], blocks[3])
+    return plan, values
+
+
+def _random_stages(seed, near_is=None, far_is=None, rules_is=None, V=300, R=24):
+    import scipy.sparse as sp
+    rng = np.random.default_rng(seed)
+    made = []
+    for shape, density, value in (((V, V), 0.02, near_is), ((V, R), 0.1, far_is), ((R, V), 0.05, rules_is)):
+        m = sp.random(*shape, density, "csr", random_state=rng, dtype=np.float64)
+        if value is not None:
+            m.data[:] = value
+        made.append(m)
+    return made
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("factors", ["small", "large", "infinite", "far_apart", "ordinary"])
+def test_weights_whose_products_leave_the_range(dtype, factors):
+    """Values of two stages whose products have no place in the type, though the sums of the stages have: such a plan runs
+    its stages, others a launch alone, forward and gradient."""
+    tiny, huge = (1e-25, 1e25) if dtype == np.float32 else (1e-180, 1e180)
+    w, v, scale = dict(small=(tiny, tiny, huge), large=(huge, huge, tiny), infinite=(np.inf, tiny, huge),
+                       far_apart=(tiny, huge, 1.0), ordinary=(0.3, 0.7, 1.0))[factors]
+    in_range = factors in ("far_apart", "ordinary")
+    near, far, rules = _random_stages(5, None if in_range else 0.0, w, v)
+    plan, _ = _plan_over(dtype, near, far, rules)
+    plan.timed_stages = ["*"]
+    x_np = ((0.5 + np.random.default_rng(3).random((300, 12))) * scale).astype(dtype)
+    x = torch.from_numpy(x_np).to(DEV)
+    chains = ((near, far, rules), (near.T, rules.T, far.T))
+    for got, (vertices, second, first) in zip((plan.forward(x), plan.backward(x)), chains):
+        got = got.cpu().numpy()
+        if in_range:  # sums of up to 40 positive terms, three roundings each
+            want = vertices @ x_np.astype(np.float64) + second @ (first @ x_np.astype(np.float64))
+            np.testing.assert_allclose(got, want, rtol=64 * np.finfo(dtype).eps)
+            continue
+        ones = lambda m: (m != 0).astype(np.float64)
+        paths = (ones(second) @ (ones(first) @ np.ones(300)))[:, None]
+        if factors == "infinite":
+            assert np.isinf(got[paths[:, 0] > 0]).all()
+            continue
+        # every term is w * v * x with x in [0.5, 1.5] scale
+        size = float(w) * (float(v) * scale)
+        assert (got >= 0.49 * size * paths).all() and (got <= 1.51 * size * paths).all() and paths.any()
+    names = [name for name, _ in plan.take_stage_times()]
+    assert names == (["fwd.final", "bwd.final"] if in_range else ["fwd.rules", "fwd.final", "bwd.rules", "bwd.final"])
+
+
 def test_rule_levels_are_stored_without_their_padding():
     """One launch per level (the form kept for hierarchies too deep to fold): the reference pads
     every level to all R rule rows (src/offline/csrc/partition.h:175-203); the device form of a level

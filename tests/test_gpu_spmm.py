@@ -584,3 +584,39 @@ def test_columns_multiplied_out(rows, dtype, with_values):
                                                 abi.ptr(starts), abi.ptr(col), abi.ptr(val), stream))
     assert np.array_equal(col.cpu().numpy()[:len(want_col)], np.array(want_col, np.int64))
     assert np.array_equal(val.cpu().numpy()[:len(want_val)], np.array(want_val, dtype))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("kind", ["ordinary", "zeros", "special", "no_rule_columns", "no_rule_values", "one_entry", "many"])
+def test_range_of_the_factors_of_multiplied_out_columns(kind, dtype):
+    """cgnn_csr_expand_range against numpy, over values that are zero, subnormal, infinite and NaN, and over more entries
+    than a launch has threads; columns below the split do not count."""
+    import ctypes
+    rng = np.random.default_rng(len(kind))
+    bits = np.uint32 if dtype == np.float32 else np.uint64
+    split, rules, rows = 50, 9, 30
+    n, m = dict(one_entry=(1, 1), many=(600001, 300007)).get(kind, (301, 77))
+    elist = rng.integers(0, split if kind == "no_rule_columns" else split + rules, n)
+    if kind == "one_entry":
+        elist[:] = split
+    value, rval = rng.standard_normal(n).astype(dtype), rng.standard_normal(m).astype(dtype)
+    value[elist < split] *= dtype(1e30)
+    if kind == "zeros":
+        value[:], rval[::3] = -0.0, 0.0
+    if kind == "special":
+        value[elist >= split] = np.resize(np.array([np.finfo(dtype).tiny / 8, -np.inf, np.nan, 0.0], dtype), (elist >= split).sum())
+        rval[5] = -np.finfo(dtype).max
+    ptr = lambda k, n: np.linspace(0, n, k + 1).astype(np.int64)
+    A = abi.DeviceCsr.from_host(rows, split + rules, ptr(rows, n), elist, value, DEV)
+    B = abi.DeviceCsr.from_host(rules, split, ptr(rules, m), rng.integers(0, split, m), None if kind == "no_rule_values" else rval, DEV)
+
+    def extremes(v):
+        v = np.abs(v).view(bits)
+        return [int(v.max(initial=0)), int(v[v > 0].min(initial=np.iinfo(bits).max)) if (v > 0).any() else 2 ** 64 - 1]
+
+    want = extremes(value[elist >= split]) + extremes(rval[:0] if kind == "no_rule_values" else rval)
+    out = torch.full((4,), 7, dtype=torch.int64, device=DEV)
+    a, b = A.struct(), B.struct()
+    abi.check(abi.lib().cgnn_csr_expand_range(ctypes.byref(a), abi.i64(split), ctypes.byref(b), abi.dtype_code(A.val.dtype),
+                                              abi.ptr(out), abi.stream_of(A.rowptr)))
+    assert [int(x) for x in out.cpu().numpy().view(np.uint64)] == want
