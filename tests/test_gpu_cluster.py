@@ -142,12 +142,15 @@ def test_assign_shapes(width, bits):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("width", [4, 5, 7, 20, 33, 47, 100, 111, 254, 255])
-def test_gathers_as_one_array(width, dtype):
+@pytest.mark.parametrize("width,n", [(width, None) for width in (4, 5, 7, 20, 33, 47, 100, 111, 254, 255)] +
+                         [(255, 20011), (254, 17003), (257, 16401), (513, 8229), (1021, 4123), (1023, 8192)])
+def test_gathers_as_one_array(width, n, dtype):
     """The gathers whose output is walked as one array: rows that are whole packs and others (a pack then holds the end of a row and
     the beginning of the next, the last one of the array ends inside), with and without sign words, values that are NaN and
-    zeros of both signs, enough rows that the form is taken; a view that begins inside a pack takes the other form."""
-    n, groups = max(200003, 2 ** 22 // width + 5), 301
+    zeros of both signs, enough rows that the form is taken; a view that begins inside a pack takes the other form.  The row
+    counts that are given, from 16 MB on, leave few workgroups of 64 rows: those take 4 to 16 rows instead, and the last one
+    fewer."""
+    n, groups = n or max(200003, 2 ** 22 // width + 5), 301
     rng = np.random.default_rng(width)
     ids = rng.integers(0, groups, n)
     counts = np.bincount(ids, minlength=groups).astype(np.int32)
