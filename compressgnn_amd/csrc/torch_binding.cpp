@@ -18,6 +18,7 @@
 #include <torch/extension.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <chrono>
 #include <climits>
@@ -494,6 +495,21 @@ struct StageTimer {
     }
 };
 
+// What a multiplied-out block is made of, by version counter: the columns and values of a vertex stage and its rules.
+// They may be tensors of the caller's (DeviceCsr takes int32 and float arrays as they are), and the stages read them
+// with every product.  Writes to inference tensors are not counted; those are taken as they were.
+std::array<uint32_t, 4> written(const DeviceCsr &stage, const DeviceCsr &rules) {
+    auto version = [](const Tensor &t) { return t.defined() && !t.is_inference() ? (uint32_t)t._version() : 0u; };
+    return {version(stage.colidx), version(stage.val), version(rules.colidx), version(rules.val)};
+}
+
+// A vertex stage with its rules multiplied out ([vertex_cnt, vertex_cnt], the same stored rows): a propagation in one
+// launch where the compressed form does not save what its second launch costs (takes_whole).
+struct MultipliedOut {
+    std::shared_ptr<DeviceCsr> block;  // NULL: never
+    std::array<uint32_t, 4> made_of{};
+};
+
 // The device form of a CompressGraph (loader/compress_graph.py:6-43 of the reference):
 // the three vertex/rule blocks, the rule levels and their transposes.
 struct PropagationPlan {
@@ -502,9 +518,7 @@ struct PropagationPlan {
     std::vector<std::shared_ptr<DeviceCsr>> r2r, r2r_t;
     // [v2v | v2r] and [v2v^T | r2v^T]: the vertex stage of forward / backward in one pass
     std::shared_ptr<DeviceCsr> vertex_stage, vertex_stage_t;
-    // The vertex stages with the rules multiplied out ([vertex_cnt, vertex_cnt], the same stored rows): a propagation
-    // in one launch where the compressed form does not save what its second launch costs (takes_whole).  NULL: never.
-    std::shared_ptr<DeviceCsr> whole, whole_t;
+    MultipliedOut whole, whole_t;
     // the four blocks of the vertex stages on their own: only for the two-launch form
     // (fuse_final = false); a plan without them holds the graph once
     std::shared_ptr<DeviceCsr> v2v, v2r, v2v_t, r2v_t;
@@ -575,11 +589,11 @@ bool products_in_range(const uint64_t *magnitudes) {
            of[1] * of[3] >= std::numeric_limits<T>::min();
 }
 
-// [vertices | rules] with the rules multiplied out, or NULL where no product would take it or a value has no place in it.
-std::shared_ptr<DeviceCsr> multiplied_out(const DeviceCsr &stage, const DeviceCsr &rules, int64_t V) {
+// [vertices | rules] with the rules multiplied out; no block where no product would take it or a value has no place in it.
+MultipliedOut multiplied_out(const DeviceCsr &stage, const DeviceCsr &rules, int64_t V) {
     if (stage.rows == 0 || stage.nnz == 0 || rules.nnz == 0 || !stage.val.defined() || stage.nnz > kMaxWholeEntries ||
         (rules.val.defined() && rules.val.scalar_type() != stage.val.scalar_type()) || capturing(stage.rowptr))
-        return nullptr;
+        return {};
     c10::hip::HIPGuardMasqueradingAsCUDA guard(stage.rowptr.device());
     const auto stream = current_stream(stage.rowptr);
     const cgnn_csr a = stage.view(), r = rules.view();
@@ -595,23 +609,25 @@ std::shared_ptr<DeviceCsr> multiplied_out(const DeviceCsr &stage, const DeviceCs
     found.narrow(0, 0, 1).copy_(starts.narrow(0, stage.rows, 1));
     found = found.cpu();
     const int64_t entries = found.data_ptr<int64_t>()[0];
-    if (entries > kMaxWholeEntries || !takes_whole(entries, stage, rules, stage.val.element_size())) return nullptr;
+    if (entries > kMaxWholeEntries || !takes_whole(entries, stage, rules, stage.val.element_size())) return {};
     const uint64_t *magnitudes = reinterpret_cast<const uint64_t *>(found.data_ptr<int64_t>() + 1);
     if (!(stage.val.scalar_type() == torch::kFloat32 ? products_in_range<float>(magnitudes) : products_in_range<double>(magnitudes)))
-        return nullptr;
+        return {};
     Tensor col = torch::empty({entries}, stage.colidx.options()), val = torch::empty({entries}, stage.val.options());
     ok(cgnn_csr_expand_columns(&a, V, &r, dtype_code(stage.val), starts.data_ptr<int32_t>(), col.data_ptr<int32_t>(), val.data_ptr(),
                                stream),
        "csr_expand_columns");
     c10::optional<Tensor> rowmap;
     if (stage.rowmap.defined()) rowmap = stage.rowmap;
-    return make_csr(starts, col, val, stage.rows, V, stage.rowptr.device(), stage.seg_nnz, rowmap);
+    return {make_csr(starts, col, val, stage.rows, V, stage.rowptr.device(), stage.seg_nnz, rowmap), written(stage, rules)};
 }
 
-// The multiplied-out stage where a product with x takes it.  A forced schedule and the two-launch form run the stages.
-bool use_whole(const PropagationPlan &p, const DeviceCsr *whole, const DeviceCsr &stage, const DeviceCsr &rules, const Tensor &x) {
-    return whole != nullptr && p.fuse_final && p.kernel == CGNN_SPMM_AUTO && x.scalar_type() == whole->val.scalar_type() &&
-           takes_whole(whole->nnz, stage, rules, x.size(1) * x.element_size());
+// Whether a product with x takes the multiplied-out stage.  A forced schedule and the two-launch form run the stages, and so
+// does every product once one of their arrays was written to.  (A graph replays what it recorded: after such a write it has to
+// be captured again.)
+bool use_whole(const PropagationPlan &p, const MultipliedOut &whole, const DeviceCsr &stage, const DeviceCsr &rules, const Tensor &x) {
+    return whole.block && p.fuse_final && p.kernel == CGNN_SPMM_AUTO && x.scalar_type() == whole.block->val.scalar_type() &&
+           takes_whole(whole.block->nnz, stage, rules, x.size(1) * x.element_size()) && whole.made_of == written(stage, rules);
 }
 
 Tensor timed_spmm(PropagationPlan &p, const std::string &stage, DeviceCsr &A, const Tensor &mat,
@@ -657,7 +673,7 @@ Tensor propagate_forward(PropagationPlan &p, Tensor x) {
     x = x.contiguous();
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
     Hold hold(p.lock);
-    if (p.whole && use_whole(p, p.whole.get(), *p.vertex_stage, *p.r2v, x)) return timed_spmm(p, "fwd.final", *p.whole, x, c10::nullopt);
+    if (p.whole.block && use_whole(p, p.whole, *p.vertex_stage, *p.r2v, x)) return timed_spmm(p, "fwd.final", *p.whole.block, x, c10::nullopt);
     Tensor rule_out = timed_spmm(p, "fwd.rules", *p.r2v, x, c10::nullopt);
     for (size_t i = 0; i < p.r2r.size(); ++i)
         rule_out = timed_spmm(p, "fwd.level" + std::to_string(i), *p.r2r[i], rule_out, rule_out);
@@ -721,7 +737,7 @@ Tensor propagate_forward_gathered(PropagationPlan &p, Tensor reps, Tensor index)
            "narrow_ids");
         rules = compose_block(*p.r2v, narrow, p.V, groups);
         stage = compose_block(*p.vertex_stage, narrow, p.V, p.vertex_stage->cols);
-        if (p.whole) whole = compose_block(*p.whole, narrow, p.V, groups);
+        if (p.whole.block) whole = compose_block(*p.whole.block, narrow, p.V, groups);
         TORCH_CHECK(bad.item<int32_t>() == 0, "propagation from representatives: the index holds a cluster id outside [0, ", groups, ")");
         if (!index.is_inference()) {
             p.composed.push_front(PropagationPlan::Composed{c10::weak_intrusive_ptr<c10::TensorImpl>(index.getIntrusivePtr()),
@@ -729,7 +745,7 @@ Tensor propagate_forward_gathered(PropagationPlan &p, Tensor reps, Tensor index)
             while (p.composed.size() > 4) p.composed.pop_back();
         }
     }
-    if (whole && use_whole(p, whole.get(), *stage, *rules, reps)) return timed_spmm(p, "fwd.final", *whole, reps, c10::nullopt);
+    if (whole && use_whole(p, p.whole, *p.vertex_stage, *p.r2v, reps)) return timed_spmm(p, "fwd.final", *whole, reps, c10::nullopt);
     Tensor rule_out = timed_spmm(p, "fwd.rules", *rules, reps, c10::nullopt);
     for (size_t i = 0; i < p.r2r.size(); ++i)
         rule_out = timed_spmm(p, "fwd.level" + std::to_string(i), *p.r2r[i], rule_out, rule_out);
@@ -758,8 +774,8 @@ Tensor propagate_backward(PropagationPlan &p, Tensor grad) {
     grad = grad.contiguous();
     c10::hip::HIPGuardMasqueradingAsCUDA guard(grad.device());
     Hold hold(p.lock);
-    if (p.whole_t && use_whole(p, p.whole_t.get(), *p.vertex_stage_t, *p.v2r_t, grad))
-        return timed_spmm(p, "bwd.final", *p.whole_t, grad, c10::nullopt);
+    if (p.whole_t.block && use_whole(p, p.whole_t, *p.vertex_stage_t, *p.v2r_t, grad))
+        return timed_spmm(p, "bwd.final", *p.whole_t.block, grad, c10::nullopt);
     Tensor rule_g = timed_spmm(p, "bwd.rules", *p.v2r_t, grad, c10::nullopt);
     for (size_t i = p.r2r_t.size(); i-- > 0;)
         rule_g = timed_spmm(p, "bwd.level" + std::to_string(i), *p.r2r_t[i], rule_g, rule_g);
@@ -2017,13 +2033,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                                  bwd->cols == p.V + p.R,
                              "a vertex stage is [vertex_cnt, vertex_cnt + rule_cnt]");
                  const bool folded = p.r2r.empty();  // no levels, or all of them in the rule stages
-                 auto whole = folded ? multiplied_out(*fwd, *p.r2v, p.V) : nullptr;
-                 auto whole_t = folded ? multiplied_out(*bwd, *p.v2r_t, p.V) : nullptr;
+                 const MultipliedOut whole = folded ? multiplied_out(*fwd, *p.r2v, p.V) : MultipliedOut();
+                 const MultipliedOut whole_t = folded ? multiplied_out(*bwd, *p.v2r_t, p.V) : MultipliedOut();
                  Hold hold(p.lock);
                  p.vertex_stage = fwd; p.vertex_stage_t = bwd;
                  p.whole = whole; p.whole_t = whole_t;
                  p.adopt(fwd); p.adopt(bwd);
-                 p.adopt(whole); p.adopt(whole_t);
+                 p.adopt(whole.block); p.adopt(whole_t.block);
              })
         .def("set_split_blocks",
              [](PropagationPlan &p, std::shared_ptr<DeviceCsr> v2v, std::shared_ptr<DeviceCsr> v2r,

@@ -337,6 +337,24 @@ def test_weights_whose_products_leave_the_range(dtype, factors):
     assert names == (["fwd.final", "bwd.final"] if in_range else ["fwd.rules", "fwd.final", "bwd.rules", "bwd.final"])
 
 
+@pytest.mark.parametrize("which", [0, 1, 2, 3])
+def test_values_written_after_the_plan_was_made(which):
+    """The values of a plan's blocks may be the caller's own tensors.  A product behind a write to one of them uses what
+    stands there then, also where the products before it ran as one launch."""
+    near, far, rules = _random_stages(6)
+    plan, values = _plan_over(np.float32, near, far, rules)
+    x_np = np.random.default_rng(4).standard_normal((300, 12)).astype(np.float32)
+    x = torch.from_numpy(x_np).to(DEV)
+    plan.forward(x), plan.backward(x)
+    values[which].mul_(3.0)
+    by = [3.0 if k == which else 1.0 for k in range(4)]
+    want = by[2] * (near @ x_np + far @ (by[0] * (rules @ x_np)))
+    want_g = by[3] * (near.T @ x_np + rules.T @ (by[1] * (far.T @ x_np)))
+    for _ in range(2):
+        assert_within(plan.forward(x).cpu().numpy(), want, rtol=1e-5, atol=2e-5)
+        assert_within(plan.backward(x).cpu().numpy(), want_g, rtol=1e-5, atol=2e-5)
+
+
 def test_rule_levels_are_stored_without_their_padding():
     """One launch per level (the form kept for hierarchies too deep to fold): the reference pads
     every level to all R rule rows (src/offline/csrc/partition.h:175-203); the device form of a level
