@@ -1970,51 +1970,62 @@ __global__ __launch_bounds__(kBlock) void expand_count_kernel(const int32_t *__r
 __device__ __forceinline__ uint64_t magnitude(float v) { return __float_as_uint(v) & 0x7fffffffu; }
 __device__ __forceinline__ uint64_t magnitude(double v) { return (uint64_t)__double_as_longlong(v) & 0x7fffffffffffffffull; }
 
-__global__ void expand_range_begin_kernel(uint64_t *__restrict__ out) {
-    if (threadIdx.x < 4) out[threadIdx.x] = threadIdx.x % 2 == 0 ? 0 : ~uint64_t(0);
+// words of a summary that are sums, and smallest values; the others are largest ones
+__host__ __device__ constexpr bool is_sum(int word) { return word == 0 || word == 2; }
+__host__ __device__ constexpr bool is_least(int word) { return word == 4 || word == 6; }
+
+__global__ void expand_summary_begin_kernel(uint64_t *__restrict__ out) {
+    if (threadIdx.x < CGNN_EXPAND_SUMMARY) out[threadIdx.x] = is_least(threadIdx.x) ? ~uint64_t(0) : 0;
 }
 
-// out: largest and smallest non-zero magnitude of the values that stand for rules, and of the rules' values
-// (cgnn_csr_expand_range).  Integer extremes, any order.
+// cgnn_csr_expand_summary: integer sums and extremes, any order.
 template <typename T>
-__global__ __launch_bounds__(kBlock) void expand_range_kernel(const int32_t *__restrict__ col, const T *__restrict__ val, int64_t nnz,
-                                                              int32_t split, const T *__restrict__ rule_val, int64_t rule_nnz,
-                                                              unsigned long long *__restrict__ out) {
-    constexpr int kWaves = kBlock / kWave;
-    __shared__ unsigned long long found[4][kWaves];
-    unsigned long long most[2] = {0, 0}, least[2] = {~0ull, ~0ull};
-    auto look = [&](int k, T v) {
-        const unsigned long long m = magnitude(v);
-        most[k] = max(most[k], m);
-        if (m != 0) least[k] = min(least[k], m);
+__global__ __launch_bounds__(kBlock) void expand_summary_kernel(const int32_t *__restrict__ counts, int64_t rows,
+                                                                const int32_t *__restrict__ col, const T *__restrict__ val, int64_t nnz,
+                                                                int32_t split, const T *__restrict__ rule_val, int64_t rule_nnz,
+                                                                unsigned long long *__restrict__ out) {
+    constexpr int kWaves = kBlock / kWave, kWords = CGNN_EXPAND_SUMMARY;
+    __shared__ unsigned long long found[kWords][kWaves];
+    unsigned long long v[kWords];
+#pragma unroll
+    for (int k = 0; k < kWords; ++k) v[k] = is_least(k) ? ~0ull : 0;
+    auto look = [&](int k, T value) {
+        const unsigned long long m = magnitude(value);
+        v[k] = max(v[k], m);
+        if (m != 0) v[k + 1] = min(v[k + 1], m);
     };
     const int64_t stride = (int64_t)gridDim.x * kBlock, t0 = (int64_t)blockIdx.x * kBlock + threadIdx.x;
 #pragma unroll 4
+    for (int64_t r = t0; r < rows; r += stride) {
+        const int32_t n = counts[r];
+        v[0] += n;
+        v[1] = max(v[1], (unsigned long long)n);
+        v[2] += n == 0;
+    }
+#pragma unroll 4
     for (int64_t e = t0; e < nnz; e += stride)
-        if (col[e] >= split) look(0, val[e]);
+        if (col[e] >= split) look(3, val[e]);
     if (rule_val != nullptr)
 #pragma unroll 4
-        for (int64_t e = t0; e < rule_nnz; e += stride) look(1, rule_val[e]);
+        for (int64_t e = t0; e < rule_nnz; e += stride) look(5, rule_val[e]);
+    auto join = [](int k, unsigned long long a, unsigned long long b) {
+        return is_sum(k) ? a + b : is_least(k) ? min(a, b) : max(a, b);
+    };
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
+    for (int k = 0; k < kWords; ++k) {
 #pragma unroll
-        for (int s = kWave / 2; s > 0; s >>= 1) {
-            most[k] = max(most[k], (unsigned long long)__shfl_xor(most[k], s, kWave));
-            least[k] = min(least[k], (unsigned long long)__shfl_xor(least[k], s, kWave));
-        }
-        if (threadIdx.x % kWave == 0) found[2 * k][threadIdx.x / kWave] = most[k], found[2 * k + 1][threadIdx.x / kWave] = least[k];
+        for (int s = kWave / 2; s > 0; s >>= 1) v[k] = join(k, v[k], (unsigned long long)__shfl_xor(v[k], s, kWave));
+        if (threadIdx.x % kWave == 0) found[k][threadIdx.x / kWave] = v[k];
     }
     __syncthreads();
-    if (threadIdx.x < 4) {
-        unsigned long long v = found[threadIdx.x][0];
+    const int k = threadIdx.x;
+    if (k >= kWords) return;
+    unsigned long long all = found[k][0];
 #pragma unroll
-        for (int w = 1; w < kWaves; ++w) {
-            const unsigned long long other = found[threadIdx.x][w];
-            v = threadIdx.x % 2 == 0 ? max(v, other) : min(v, other);
-        }
-        if (threadIdx.x % 2 == 0) atomicMax(out + threadIdx.x, v);
-        else atomicMin(out + threadIdx.x, v);
-    }
+    for (int w = 1; w < kWaves; ++w) all = join(k, all, found[k][w]);
+    if (is_sum(k)) atomicAdd(out + k, all);
+    else if (is_least(k)) atomicMin(out + k, all);
+    else atomicMax(out + k, all);
 }
 
 template <typename T>
@@ -2434,25 +2445,26 @@ extern "C" int cgnn_csr_expand_count(const cgnn_csr *A, int64_t split, const cgn
     return check_launch("csr_expand_count");
 }
 
-extern "C" int cgnn_csr_expand_range(const cgnn_csr *A, int64_t split, const cgnn_csr *rules, int dtype, uint64_t *magnitudes,
-                                     cgnn_stream_t stream) {
+extern "C" int cgnn_csr_expand_summary(const cgnn_csr *A, int64_t split, const cgnn_csr *rules, int dtype, const int32_t *counts,
+                                       uint64_t *summary, cgnn_stream_t stream) {
     int rc = check_expand(A, split, rules);
     if (rc != CGNN_OK) return rc;
-    CGNN_REQUIRE(dtype == CGNN_F32 || dtype == CGNN_F64, "cgnn_csr_expand_range: dtype must be f32 or f64");
-    CGNN_REQUIRE(magnitudes != nullptr && (A->nnz == 0 || A->val != nullptr), "cgnn_csr_expand_range: null array");
-    hipLaunchKernelGGL(expand_range_begin_kernel, dim3(1), dim3(kWave), 0, stream, magnitudes);
-    const int64_t entries = std::max(A->nnz, rules->val != nullptr ? rules->nnz : 0);
-    if (entries == 0) return check_launch("csr_expand_range");
-    const dim3 grid((unsigned)std::min<int64_t>(ceil_div(entries, 4 * kBlock), 256));
+    CGNN_REQUIRE(dtype == CGNN_F32 || dtype == CGNN_F64, "cgnn_csr_expand_summary: dtype must be f32 or f64");
+    CGNN_REQUIRE(summary && (A->rows == 0 || counts) && (A->nnz == 0 || A->val), "cgnn_csr_expand_summary: null array");
+    hipLaunchKernelGGL(expand_summary_begin_kernel, dim3(1), dim3(kWave), 0, stream, summary);
+    const int64_t items = std::max(A->rows, std::max(A->nnz, rules->val != nullptr ? rules->nnz : 0));
+    if (items == 0) return check_launch("csr_expand_summary");
+    // as many workgroups as there are compute units: each adds seven words to the summary
+    const dim3 grid((unsigned)std::min<int64_t>(ceil_div(items, 4 * kBlock), 256));
     auto run = [&](auto zero) {
         typedef decltype(zero) T;
-        hipLaunchKernelGGL(expand_range_kernel<T>, grid, dim3(kBlock), 0, stream, A->colidx, static_cast<const T *>(A->val), A->nnz,
-                           (int32_t)split, static_cast<const T *>(rules->val), rules->nnz,
-                           reinterpret_cast<unsigned long long *>(magnitudes));
+        hipLaunchKernelGGL(expand_summary_kernel<T>, grid, dim3(kBlock), 0, stream, counts, A->rows, A->colidx,
+                           static_cast<const T *>(A->val), A->nnz, (int32_t)split, static_cast<const T *>(rules->val), rules->nnz,
+                           reinterpret_cast<unsigned long long *>(summary));
     };
     if (dtype == CGNN_F32) run(0.0f);
     else run(0.0);
-    return check_launch("csr_expand_range");
+    return check_launch("csr_expand_summary");
 }
 
 extern "C" int cgnn_csr_expand_columns(const cgnn_csr *A, int64_t split, const cgnn_csr *rules, int dtype, const int32_t *rowptr,

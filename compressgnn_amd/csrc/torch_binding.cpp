@@ -506,8 +506,10 @@ std::array<uint32_t, 4> written(const DeviceCsr &stage, const DeviceCsr &rules) 
 // A vertex stage with its rules multiplied out ([vertex_cnt, vertex_cnt], the same stored rows): a propagation in one
 // launch where the compressed form does not save what its second launch costs (takes_whole).
 struct MultipliedOut {
-    std::shared_ptr<DeviceCsr> block;  // NULL: never
+    int64_t entries = 0;  // 0: never
+    int32_t longest = 0;  // its longest row
     std::array<uint32_t, 4> made_of{};
+    std::shared_ptr<DeviceCsr> block;  // made for the first product that takes it
 };
 
 // The device form of a CompressGraph (loader/compress_graph.py:6-43 of the reference):
@@ -530,14 +532,14 @@ struct PropagationPlan {
     StageTimer timer;
     // The forward blocks with their vertex columns sent through a cluster assignment
     // (propagate_forward_gathered), kept for the index tensors they were made for: an
-    // assignment lasts until the next refresh, and a model may hold one per layer.
+    // assignment lasts until the next refresh, and a model may hold one per layer.  Either form, or both, as products ask.
     struct Composed {
         c10::weak_intrusive_ptr<c10::TensorImpl> index;
         uint32_t version;
         int64_t groups;
         std::shared_ptr<DeviceCsr> rules, stage, whole;
     };
-    std::deque<Composed> composed;
+    std::deque<std::shared_ptr<Composed>> composed;
 
     void adopt(const std::shared_ptr<DeviceCsr> &block) {
         if (!block) return;
@@ -574,7 +576,7 @@ bool takes_whole(int64_t entries, const DeviceCsr &stage, const DeviceCsr &rules
 }
 
 // Whether every product of a value that stands for a rule and a value of the rules has a place in the type T, by the
-// extremes of both (cgnn_csr_expand_range).  A multiplied-out block stores these products; the stages multiply through
+// extremes of both (cgnn_csr_expand_summary).  A multiplied-out block stores these products; the stages multiply through
 // the sums of the rules, and factors like 1e-25 and 1e-25, or 1e25 and 1e25, are theirs.
 template <typename T>
 bool products_in_range(const uint64_t *magnitudes) {
@@ -589,45 +591,108 @@ bool products_in_range(const uint64_t *magnitudes) {
            of[1] * of[3] >= std::numeric_limits<T>::min();
 }
 
-// [vertices | rules] with the rules multiplied out; no block where no product would take it or a value has no place in it.
-MultipliedOut multiplied_out(const DeviceCsr &stage, const DeviceCsr &rules, int64_t V) {
-    if (stage.rows == 0 || stage.nnz == 0 || rules.nnz == 0 || !stage.val.defined() || stage.nnz > kMaxWholeEntries ||
-        (rules.val.defined() && rules.val.scalar_type() != stage.val.scalar_type()) || capturing(stage.rowptr))
-        return {};
-    c10::hip::HIPGuardMasqueradingAsCUDA guard(stage.rowptr.device());
-    const auto stream = current_stream(stage.rowptr);
-    const cgnn_csr a = stage.view(), r = rules.view();
-    Tensor counts = torch::empty({stage.rows}, stage.rowptr.options()), starts = torch::empty({stage.rows + 1}, stage.rowptr.options());
-    Tensor ws = torch::empty({(int64_t)cgnn_exclusive_sum_workspace_bytes(stage.rows)}, stage.rowptr.options().dtype(torch::kUInt8));
-    ok(cgnn_csr_expand_count(&a, V, &r, counts.data_ptr<int32_t>(), stream), "csr_expand_count");
-    ok(cgnn_exclusive_sum_i32(stage.rows, counts.data_ptr<int32_t>(), starts.data_ptr<int32_t>(), nullptr, ws.data_ptr(), ws.numel(),
-                              stream),
-       "exclusive_sum");
-    Tensor found = torch::empty({5}, stage.rowptr.options().dtype(torch::kInt64));
-    ok(cgnn_csr_expand_range(&a, V, &r, dtype_code(stage.val), reinterpret_cast<uint64_t *>(found.data_ptr<int64_t>() + 1), stream),
-       "csr_expand_range");
-    found.narrow(0, 0, 1).copy_(starts.narrow(0, stage.rows, 1));
-    found = found.cpu();
-    const int64_t entries = found.data_ptr<int64_t>()[0];
-    if (entries > kMaxWholeEntries || !takes_whole(entries, stage, rules, stage.val.element_size())) return {};
-    const uint64_t *magnitudes = reinterpret_cast<const uint64_t *>(found.data_ptr<int64_t>() + 1);
-    if (!(stage.val.scalar_type() == torch::kFloat32 ? products_in_range<float>(magnitudes) : products_in_range<double>(magnitudes)))
-        return {};
-    Tensor col = torch::empty({entries}, stage.colidx.options()), val = torch::empty({entries}, stage.val.options());
-    ok(cgnn_csr_expand_columns(&a, V, &r, dtype_code(stage.val), starts.data_ptr<int32_t>(), col.data_ptr<int32_t>(), val.data_ptr(),
-                               stream),
-       "csr_expand_columns");
-    c10::optional<Tensor> rowmap;
-    if (stage.rowmap.defined()) rowmap = stage.rowmap;
-    return {make_csr(starts, col, val, stage.rows, V, stage.rowptr.device(), stage.seg_nnz, rowmap), written(stage, rules)};
+// What the vertex stages [vertices | rules] of both directions come to with their rules multiplied out; no entries where no
+// product would take that, or a value has no place in it.  One host read.
+std::array<MultipliedOut, 2> surveyed(const std::array<std::pair<DeviceCsr *, DeviceCsr *>, 2> &stages, int64_t V) {
+    std::array<MultipliedOut, 2> found;
+    const Tensor like = stages[0].first->rowptr;
+    if (capturing(like)) return found;
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(like.device());
+    const auto stream = current_stream(like);
+    Tensor summaries;
+    bool wanted[2];
+    for (int k = 0; k < 2; ++k) {
+        const DeviceCsr &stage = *stages[k].first, &rules = *stages[k].second;
+        const std::shared_ptr<Scratch> scratch = stage.scratch, of_rules = rules.scratch;
+        Hold hold(scratch->lock), hold_rules(of_rules->lock);
+        wanted[k] = stage.empty_rows.defined() && rules.nnz > 0 && stage.val.defined() && stage.nnz <= kMaxWholeEntries &&
+                    (!rules.val.defined() || rules.val.scalar_type() == stage.val.scalar_type()) &&
+                    stage.rowptr.device() == like.device() && rules.rowptr.device() == like.device();
+        if (!wanted[k]) continue;
+        found[k].made_of = written(stage, rules);
+        if (!summaries.defined()) summaries = torch::empty({2, CGNN_EXPAND_SUMMARY}, like.options().dtype(torch::kInt64));
+        const cgnn_csr a = stage.view(), r = rules.view();
+        Tensor counts = torch::empty({stage.rows}, like.options());
+        ok(cgnn_csr_expand_count(&a, V, &r, counts.data_ptr<int32_t>(), stream), "csr_expand_count");
+        ok(cgnn_csr_expand_summary(&a, V, &r, dtype_code(stage.val), counts.data_ptr<int32_t>(),
+                                   reinterpret_cast<uint64_t *>(summaries[k].data_ptr<int64_t>()), stream),
+           "csr_expand_summary");
+    }
+    if (!summaries.defined()) return found;
+    summaries = summaries.cpu();
+    for (int k = 0; k < 2; ++k) {
+        if (!wanted[k]) continue;
+        const uint64_t *s = reinterpret_cast<const uint64_t *>(summaries.data_ptr<int64_t>()) + k * CGNN_EXPAND_SUMMARY;
+        const DeviceCsr &stage = *stages[k].first;
+        const bool in_range = stage.val.scalar_type() == torch::kFloat32 ? products_in_range<float>(s + 3) : products_in_range<double>(s + 3);
+        // (a row that only rules without entries stand in would be one that the stage's list of empty rows does not have)
+        if (s[0] > (uint64_t)kMaxWholeEntries || s[2] != (uint64_t)stage.empty_rows.numel() || !in_range) continue;
+        found[k].entries = (int64_t)s[0];
+        found[k].longest = (int32_t)s[1];
+    }
+    return found;
 }
 
-// Whether a product with x takes the multiplied-out stage.  A forced schedule and the two-launch form run the stages, and so
-// does every product once one of their arrays was written to.  (A graph replays what it recorded: after such a write it has to
-// be captured again.)
-bool use_whole(const PropagationPlan &p, const MultipliedOut &whole, const DeviceCsr &stage, const DeviceCsr &rules, const Tensor &x) {
-    return whole.block && p.fuse_final && p.kernel == CGNN_SPMM_AUTO && x.scalar_type() == whole.block->val.scalar_type() &&
-           takes_whole(whole.block->nnz, stage, rules, x.size(1) * x.element_size()) && whole.made_of == written(stage, rules);
+// Waits for the stream; the interpreter's other threads run meanwhile.
+bool synchronized(cgnn_stream_t stream) {
+    auto wait = [&] { return hipStreamSynchronize(reinterpret_cast<hipStream_t>(stream)) == hipSuccess; };
+    if (!PyGILState_Check()) return wait();
+    pybind11::gil_scoped_release others;
+    return wait();
+}
+
+// The multiplied-out stage where a product with x takes it, else NULL.  A forced schedule and the two-launch form run the
+// stages, and so does every product once one of their arrays was written to.  (A graph replays what it recorded: after such a
+// write it has to be captured again.)  Made for the first product that takes it, so that a plan whose products are all wide
+// holds the graph once, and finished when that product is launched, whatever stream the next one runs on; no array
+// needs a host read to be made, so under a capture it is the graph's, which makes it with every replay (a program that runs a
+// product first captures the finished one).  The caller holds the plan's lock.
+std::shared_ptr<DeviceCsr> multiplied_out(PropagationPlan &p, MultipliedOut &whole, const std::shared_ptr<DeviceCsr> &stage,
+                                          const std::shared_ptr<DeviceCsr> &rules, const Tensor &x) {
+    if (whole.entries == 0 || !p.fuse_final || p.kernel != CGNN_SPMM_AUTO || x.scalar_type() != stage->val.scalar_type() ||
+        x.size(1) == 0 || x.device() != stage->rowptr.device() ||
+        !takes_whole(whole.entries, *stage, *rules, x.size(1) * x.element_size()))
+        return nullptr;
+    if (whole.made_of != written(*stage, *rules)) {
+        whole = MultipliedOut();
+        return nullptr;
+    }
+    if (whole.block) return whole.block;
+    const auto stream = current_stream(x);
+    const auto ints = stage->rowptr.options();
+    auto blk = std::make_shared<DeviceCsr>();
+    blk->rows = blk->out_rows = stage->rows;
+    blk->cols = p.V;
+    blk->nnz = whole.entries;
+    blk->max_row_nnz = whole.longest;
+    blk->seg_nnz = stage->seg_nnz;
+    blk->rowmap = stage->rowmap;
+    blk->rowptr = torch::empty({stage->rows + 1}, ints);
+    blk->colidx = torch::empty({whole.entries}, ints);
+    blk->val = torch::empty({whole.entries}, stage->val.options());
+    // The plan's AUTO products run the row schedule or workgroup runs: neither asks which rows plain runs would cut.
+    blk->cut_rows = torch::empty({1}, ints).narrow(0, 0, 0);
+    blk->empty_rows = locked(*stage, &DeviceCsr::empty_rows);
+    p.adopt(blk);
+    Tensor counts = torch::empty({stage->rows}, ints);
+    const size_t bytes = cgnn_exclusive_sum_workspace_bytes(stage->rows);
+    Tensor ws = torch::empty({(int64_t)bytes}, ints.dtype(torch::kUInt8));
+    {
+        const std::shared_ptr<Scratch> scratch = stage->scratch, of_rules = rules->scratch;
+        Hold hold(scratch->lock), hold_rules(of_rules->lock);
+        const cgnn_csr a = stage->view(), r = rules->view();
+        ok(cgnn_csr_expand_count(&a, p.V, &r, counts.data_ptr<int32_t>(), stream), "csr_expand_count");
+        ok(cgnn_exclusive_sum_i32(stage->rows, counts.data_ptr<int32_t>(), blk->rowptr.data_ptr<int32_t>(), nullptr, ws.data_ptr(), bytes,
+                                  stream),
+           "exclusive_sum");
+        ok(cgnn_csr_expand_columns(&a, p.V, &r, dtype_code(x), blk->rowptr.data_ptr<int32_t>(), blk->colidx.data_ptr<int32_t>(),
+                                   blk->val.data_ptr(), stream),
+           "csr_expand_columns");
+    }
+    if (capturing(x)) return blk;
+    TORCH_CHECK(synchronized(stream), "propagate: the stream reported an error");
+    whole.block = blk;
+    return blk;
 }
 
 Tensor timed_spmm(PropagationPlan &p, const std::string &stage, DeviceCsr &A, const Tensor &mat,
@@ -673,7 +738,7 @@ Tensor propagate_forward(PropagationPlan &p, Tensor x) {
     x = x.contiguous();
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
     Hold hold(p.lock);
-    if (p.whole.block && use_whole(p, p.whole, *p.vertex_stage, *p.r2v, x)) return timed_spmm(p, "fwd.final", *p.whole.block, x, c10::nullopt);
+    if (auto whole = multiplied_out(p, p.whole, p.vertex_stage, p.r2v, x)) return timed_spmm(p, "fwd.final", *whole, x, c10::nullopt);
     Tensor rule_out = timed_spmm(p, "fwd.rules", *p.r2v, x, c10::nullopt);
     for (size_t i = 0; i < p.r2r.size(); ++i)
         rule_out = timed_spmm(p, "fwd.level" + std::to_string(i), *p.r2r[i], rule_out, rule_out);
@@ -700,8 +765,8 @@ std::shared_ptr<DeviceCsr> compose_block(const DeviceCsr &A, const Tensor &narro
 // propagate_forward on blocks whose vertex columns name the representative of the vertex.
 // reps: [groups, F]; index: int64 [vertex_cnt] with values in [0, groups).  The same sums in the
 // same order as propagate_forward(reps.index_select(0, index)): the same bits.  The composed
-// blocks are made on the first call for an index tensor (one host read: the ids are checked)
-// and kept until that tensor is written to or freed.  Stage names: fwd.rules, fwd.level<i>, fwd.final.
+// blocks that the width takes are made on the first call for an index tensor (one host read: the ids are
+// checked) and kept until that tensor is written to or freed.  Stage names: fwd.rules, fwd.level<i>, fwd.final.
 Tensor propagate_forward_gathered(PropagationPlan &p, Tensor reps, Tensor index) {
     require_gpu(reps, "reps");
     require_gpu(index, "index");
@@ -714,38 +779,47 @@ Tensor propagate_forward_gathered(PropagationPlan &p, Tensor reps, Tensor index)
     c10::hip::HIPGuardMasqueradingAsCUDA guard(reps.device());
     const int64_t groups = reps.size(0), F = reps.size(1);
     Hold hold(p.lock);
-    std::shared_ptr<DeviceCsr> rules, stage, whole;
-    for (auto it = p.composed.begin(); it != p.composed.end();) {
-        if (it->index.expired()) {
+    const std::shared_ptr<DeviceCsr> whole = multiplied_out(p, p.whole, p.vertex_stage, p.r2v, reps);
+    std::shared_ptr<PropagationPlan::Composed> known;
+    for (auto it = p.composed.begin(); it != p.composed.end() && !known;) {
+        if ((*it)->index.expired()) {
             it = p.composed.erase(it);
             continue;
         }
-        if (it->index._unsafe_get_target() == index.unsafeGetTensorImpl() && it->version == index._version() &&
-            it->groups == groups) {
-            rules = it->rules;
-            stage = it->stage;
-            whole = it->whole;
-            break;
-        }
+        if ((*it)->index._unsafe_get_target() == index.unsafeGetTensorImpl() && (*it)->version == index._version() &&
+            (*it)->groups == groups)
+            known = *it;
         ++it;
     }
-    if (!stage) {
+    std::shared_ptr<DeviceCsr> rules, stage, composed_whole;
+    if (known) rules = known->rules, stage = known->stage, composed_whole = known->whole;
+    if (whole ? !composed_whole : !stage) {
         Tensor bad = torch::zeros({1}, index.options().dtype(torch::kInt32));
         Tensor narrow = torch::empty({p.V}, index.options().dtype(torch::kInt32));
         ok(cgnn_narrow_ids(p.V, index.data_ptr<int64_t>(), groups, narrow.data_ptr<int32_t>(), bad.data_ptr<int32_t>(),
                            current_stream(index)),
            "narrow_ids");
-        rules = compose_block(*p.r2v, narrow, p.V, groups);
-        stage = compose_block(*p.vertex_stage, narrow, p.V, p.vertex_stage->cols);
-        if (p.whole.block) whole = compose_block(*p.whole.block, narrow, p.V, groups);
-        TORCH_CHECK(bad.item<int32_t>() == 0, "propagation from representatives: the index holds a cluster id outside [0, ", groups, ")");
-        if (!index.is_inference()) {
-            p.composed.push_front(PropagationPlan::Composed{c10::weak_intrusive_ptr<c10::TensorImpl>(index.getIntrusivePtr()),
-                                                           index._version(), groups, rules, stage, whole});
+        if (whole) {
+            composed_whole = compose_block(*whole, narrow, p.V, groups);
+        } else {
+            rules = compose_block(*p.r2v, narrow, p.V, groups);
+            stage = compose_block(*p.vertex_stage, narrow, p.V, p.vertex_stage->cols);
+        }
+        if (known) {  // the ids were checked; what a capture makes is the graph's
+            if (!capturing(index)) {
+                TORCH_CHECK(synchronized(current_stream(index)), "propagate: the stream reported an error");
+                known->rules = rules, known->stage = stage, known->whole = composed_whole;
+            }
+        } else {
+            TORCH_CHECK(bad.item<int32_t>() == 0, "propagation from representatives: the index holds a cluster id outside [0, ", groups, ")");
+        }
+        if (!known && !index.is_inference()) {
+            p.composed.push_front(std::make_shared<PropagationPlan::Composed>(PropagationPlan::Composed{
+                c10::weak_intrusive_ptr<c10::TensorImpl>(index.getIntrusivePtr()), index._version(), groups, rules, stage, composed_whole}));
             while (p.composed.size() > 4) p.composed.pop_back();
         }
     }
-    if (whole && use_whole(p, p.whole, *p.vertex_stage, *p.r2v, reps)) return timed_spmm(p, "fwd.final", *whole, reps, c10::nullopt);
+    if (whole) return timed_spmm(p, "fwd.final", *composed_whole, reps, c10::nullopt);
     Tensor rule_out = timed_spmm(p, "fwd.rules", *rules, reps, c10::nullopt);
     for (size_t i = 0; i < p.r2r.size(); ++i)
         rule_out = timed_spmm(p, "fwd.level" + std::to_string(i), *p.r2r[i], rule_out, rule_out);
@@ -774,8 +848,8 @@ Tensor propagate_backward(PropagationPlan &p, Tensor grad) {
     grad = grad.contiguous();
     c10::hip::HIPGuardMasqueradingAsCUDA guard(grad.device());
     Hold hold(p.lock);
-    if (p.whole_t.block && use_whole(p, p.whole_t, *p.vertex_stage_t, *p.v2r_t, grad))
-        return timed_spmm(p, "bwd.final", *p.whole_t.block, grad, c10::nullopt);
+    if (auto whole = multiplied_out(p, p.whole_t, p.vertex_stage_t, p.v2r_t, grad))
+        return timed_spmm(p, "bwd.final", *whole, grad, c10::nullopt);
     Tensor rule_g = timed_spmm(p, "bwd.rules", *p.v2r_t, grad, c10::nullopt);
     for (size_t i = p.r2r_t.size(); i-- > 0;)
         rule_g = timed_spmm(p, "bwd.level" + std::to_string(i), *p.r2r_t[i], rule_g, rule_g);
@@ -2032,14 +2106,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                  TORCH_CHECK(fwd && bwd && fwd->rows == p.V && bwd->rows == p.V && fwd->cols == p.V + p.R &&
                                  bwd->cols == p.V + p.R,
                              "a vertex stage is [vertex_cnt, vertex_cnt + rule_cnt]");
-                 const bool folded = p.r2r.empty();  // no levels, or all of them in the rule stages
-                 const MultipliedOut whole = folded ? multiplied_out(*fwd, *p.r2v, p.V) : MultipliedOut();
-                 const MultipliedOut whole_t = folded ? multiplied_out(*bwd, *p.v2r_t, p.V) : MultipliedOut();
+                 std::array<MultipliedOut, 2> whole;
+                 if (p.r2r.empty())  // no levels, or all of them in the rule stages
+                     whole = surveyed({std::make_pair(fwd.get(), p.r2v.get()), std::make_pair(bwd.get(), p.v2r_t.get())}, p.V);
                  Hold hold(p.lock);
                  p.vertex_stage = fwd; p.vertex_stage_t = bwd;
-                 p.whole = whole; p.whole_t = whole_t;
+                 p.whole = whole[0]; p.whole_t = whole[1];
+                 p.composed.clear();
                  p.adopt(fwd); p.adopt(bwd);
-                 p.adopt(whole.block); p.adopt(whole_t.block);
              })
         .def("set_split_blocks",
              [](PropagationPlan &p, std::shared_ptr<DeviceCsr> v2v, std::shared_ptr<DeviceCsr> v2r,

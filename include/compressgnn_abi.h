@@ -217,12 +217,15 @@ int cgnn_csr_compose_columns(int64_t nnz, const int32_t *colidx, int64_t first_c
  *
  * w * v is rounded to the block's type before it meets a row of features, where the two stages multiply through the sum
  * over the rule: factors whose product the type does not hold give zeros, infinities and NaN where the stages have finite
- * sums.  cgnn_csr_expand_range writes magnitudes[4]: the largest and the smallest non-zero |w| of the entries with c >=
- * split, as the bits of the type (in the low half where that is float32), and the same of the values of `rules`; 0 and
- * UINT64_MAX where there are none.  The order of the bits is that of the magnitudes, with infinity and NaN above all others. */
+ * sums.  cgnn_csr_expand_summary writes what there is to know of a block before it is made: summary[0] its entries, [1] its
+ * longest row and [2] its rows without entries, from the counts of cgnn_csr_expand_count; [3] and [4] the largest and the
+ * smallest non-zero |w| of the entries with c >= split, as the bits of the type (in the low half where that is float32), [5]
+ * and [6] the same of the values of `rules`; 0 and UINT64_MAX where there are none.  The order of the bits is that of the
+ * magnitudes, with infinity and NaN above all others. */
+#define CGNN_EXPAND_SUMMARY 7
 int cgnn_csr_expand_count(const cgnn_csr *A, int64_t split, const cgnn_csr *rules, int32_t *counts, cgnn_stream_t stream);
-int cgnn_csr_expand_range(const cgnn_csr *A, int64_t split, const cgnn_csr *rules, int dtype, uint64_t *magnitudes,
-                          cgnn_stream_t stream);
+int cgnn_csr_expand_summary(const cgnn_csr *A, int64_t split, const cgnn_csr *rules, int dtype, const int32_t *counts,
+                            uint64_t *summary, cgnn_stream_t stream);
 int cgnn_csr_expand_columns(const cgnn_csr *A, int64_t split, const cgnn_csr *rules, int dtype, const int32_t *rowptr,
                             int32_t *colidx, void *val, cgnn_stream_t stream);
 

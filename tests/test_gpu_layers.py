@@ -355,6 +355,66 @@ def test_values_written_after_the_plan_was_made(which):
         assert_within(plan.backward(x).cpu().numpy(), want_g, rtol=1e-5, atol=2e-5)
 
 
+def _requested():
+    return torch.cuda.memory_stats()["requested_bytes.all.current"]
+
+
+def _web_graph_plan(vertices):
+    import compressgnn_offline as off
+    from CompressgnnData import CompressgnnData
+    v, e = off.gen_copy_model(vertices, 9.8, 0.7, 3)
+    V, mask = len(v) - 1, np.ones(len(v) - 1, bool)
+    data = CompressgnnData(np.zeros((V, 1), np.float32), (v, e), np.zeros(V, np.int64), mask, mask, mask, graph_type="csr")
+    return data.to(DEV).edge_index.plan()
+
+
+def test_multiplied_out_blocks_are_made_for_the_products_that_take_them():
+    """A plan holds its stages alone until a product takes the multiplied-out form, whose columns and values are 8 bytes an
+    entry."""
+    plan = _web_graph_plan(60000)
+    wide, narrow = torch.randn(plan.vertex_stage.rows, 1024, device=DEV), torch.randn(plan.vertex_stage.rows, 8, device=DEV)
+    entries = plan.vertex_stage.nnz + plan.vertex_stage_t.nnz
+    plan.forward(wide), plan.backward(wide)  # with the tables of the stages
+    before = _requested()
+    first = plan.forward(narrow), plan.backward(narrow)
+    assert _requested() - before >= 8 * entries
+    assert all(torch.equal(a, b) for a, b in zip(first, (plan.forward(narrow), plan.backward(narrow))))
+    other = torch.cuda.Stream()  # the blocks are finished: a stream that waits for nothing may use them
+    with torch.cuda.stream(other):
+        got = plan.forward(narrow)
+    torch.cuda.synchronize()
+    assert torch.equal(got, first[0])
+
+
+@pytest.mark.parametrize("F", [1024, 8])
+def test_representatives_compose_the_blocks_that_their_width_takes(F):
+    """A new index sends the columns of the stages or of the multiplied-out block through it, 4 bytes an entry, and not of
+    both; a product of the other width over the same index, also one that is recorded, has the bits of the plain one."""
+    plan = _web_graph_plan(60000)
+    V = plan.vertex_stage.rows
+    index = torch.randint(0, 900, (V,), device=DEV)
+    reps, other = torch.randn(900, F, device=DEV), torch.randn(900, 1032 - F, device=DEV)
+    want, want_other = (plan.forward(r.index_select(0, index)) for r in (reps, other))
+    torch.cuda.synchronize()
+    before = _requested()
+    got = plan.forward_gathered(reps, index)
+    held = _requested() - before - 4 * got.numel()
+    assert torch.equal(got, want)
+    # the multiplied-out block has 1.05 entries for one of the stages
+    assert held < 1.3 * 4 * (plan.r2v.nnz + plan.vertex_stage.nnz)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        recorded = plan.forward_gathered(other, index)
+    for _ in range(3):
+        assert torch.equal(plan.forward_gathered(other, index), want_other)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(recorded, want_other)
+    with pytest.raises(RuntimeError, match="outside"):
+        plan.forward_gathered(reps, torch.full((V,), 900, device=DEV))
+
+
 def test_rule_levels_are_stored_without_their_padding():
     """One launch per level (the form kept for hierarchies too deep to fold): the reference pads
     every level to all R rule rows (src/offline/csrc/partition.h:175-203); the device form of a level

@@ -588,13 +588,14 @@ def test_columns_multiplied_out(rows, dtype, with_values):
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("kind", ["ordinary", "zeros", "special", "no_rule_columns", "no_rule_values", "one_entry", "many"])
-def test_range_of_the_factors_of_multiplied_out_columns(kind, dtype):
-    """cgnn_csr_expand_range against numpy, over values that are zero, subnormal, infinite and NaN, and over more entries
-    than a launch has threads; columns below the split do not count."""
+def test_summary_of_multiplied_out_columns(kind, dtype):
+    """cgnn_csr_expand_summary against numpy, over values that are zero, subnormal, infinite and NaN, and over more entries
+    than a launch has threads; the values of columns below the split do not count."""
     import ctypes
     rng = np.random.default_rng(len(kind))
     bits = np.uint32 if dtype == np.float32 else np.uint64
-    split, rules, rows = 50, 9, 30
+    split, rules = 50, 9
+    rows = 70003 if kind == "many" else 30
     n, m = dict(one_entry=(1, 1), many=(600001, 300007)).get(kind, (301, 77))
     elist = rng.integers(0, split if kind == "no_rule_columns" else split + rules, n)
     if kind == "one_entry":
@@ -615,8 +616,12 @@ def test_range_of_the_factors_of_multiplied_out_columns(kind, dtype):
         return [int(v.max(initial=0)), int(v[v > 0].min(initial=np.iinfo(bits).max)) if (v > 0).any() else 2 ** 64 - 1]
 
     want = extremes(value[elist >= split]) + extremes(rval[:0] if kind == "no_rule_values" else rval)
-    out = torch.full((4,), 7, dtype=torch.int64, device=DEV)
-    a, b = A.struct(), B.struct()
-    abi.check(abi.lib().cgnn_csr_expand_range(ctypes.byref(a), abi.i64(split), ctypes.byref(b), abi.dtype_code(A.val.dtype),
-                                              abi.ptr(out), abi.stream_of(A.rowptr)))
-    assert [int(x) for x in out.cpu().numpy().view(np.uint64)] == want
+    counts = rng.integers(0, 5, rows).astype(np.int32)
+    counts[0] = 2 ** 31 - 1
+    want = [int(counts.astype(np.int64).sum()), 2 ** 31 - 1, int((counts == 0).sum())] + want
+    out = torch.full((len(want),), 7, dtype=torch.int64, device=DEV)
+    a, b, dcounts = A.struct(), B.struct(), torch.from_numpy(counts).to(DEV)
+    for _ in range(2):
+        abi.check(abi.lib().cgnn_csr_expand_summary(ctypes.byref(a), abi.i64(split), ctypes.byref(b), abi.dtype_code(A.val.dtype),
+                                                    abi.ptr(dcounts), abi.ptr(out), abi.stream_of(A.rowptr)))
+        assert [int(x) for x in out.cpu().numpy().view(np.uint64)] == want
