@@ -29,6 +29,7 @@
 #include <limits>
 #include <memory>
 #include <mutex>
+#include <optional>
 #include <sstream>
 #include <map>
 #include <string>
@@ -999,18 +1000,24 @@ std::vector<Tensor> cluster_workspace(Tensor input, int64_t bits) {
 int64_t largest_group(const std::vector<Tensor> &m) { return m.size() == 4 ? m[3].item<int64_t>() : 0; }
 
 // Waits until a word of pinned memory is no longer `not_yet`.  The last thing that a launch writes is there while what
-// stands behind it still runs: look for it as long as a stream with a training step ahead takes, and otherwise wait for the
-// stream, which also reports its errors.  A copy behind the launch takes the host 24 us, a refresh of 60,000 rows and its
-// products 262 us with it and 220 so; waiting for the stream after 200 us already makes a step of 3.77 ms 20 us longer.
-void await(const int32_t *word, int32_t not_yet, cgnn_stream_t stream, const char *op) {
-    const auto patience = std::chrono::steady_clock::now() + std::chrono::milliseconds(5);
-    while (__atomic_load_n(word, __ATOMIC_ACQUIRE) == not_yet)
-        if (std::chrono::steady_clock::now() > patience) {
-            TORCH_CHECK(hipStreamSynchronize(reinterpret_cast<hipStream_t>(stream)) == hipSuccess, op,
-                        ": the stream reported an error");
-            TORCH_CHECK(__atomic_load_n(word, __ATOMIC_ACQUIRE) != not_yet, op, ": the sizes were not written");
-            return;
-        }
+// stands behind it still runs: look for it as long as `patience`, and otherwise wait for the stream, which also reports its
+// errors.  After kShortWait the interpreter's other threads may run.  (Not before: a thread that lets go of the lock has it back
+// when the one that took it gives it up, after 5 ms if that one computes.)
+constexpr std::chrono::microseconds kShortWait(200);
+
+void await(const int32_t *word, int32_t not_yet, std::chrono::microseconds patience, cgnn_stream_t stream, const char *op) {
+    const auto begin = std::chrono::steady_clock::now();
+    auto arrives_within = [&](std::chrono::microseconds wait) {
+        while (__atomic_load_n(word, __ATOMIC_ACQUIRE) == not_yet)
+            if (std::chrono::steady_clock::now() - begin > wait) return false;
+        return true;
+    };
+    if (arrives_within(std::min(patience, kShortWait))) return;
+    std::optional<pybind11::gil_scoped_release> others;
+    if (PyGILState_Check()) others.emplace();
+    if (patience > kShortWait && arrives_within(patience)) return;
+    TORCH_CHECK(hipStreamSynchronize(reinterpret_cast<hipStream_t>(stream)) == hipSuccess, op, ": the stream reported an error");
+    TORCH_CHECK(__atomic_load_n(word, __ATOMIC_ACQUIRE) != not_yet, op, ": the sizes were not written");
 }
 
 struct Assigned {
@@ -1075,8 +1082,10 @@ Assigned assign(Tensor input, Tensor planes, int64_t bits, bool with_reps) {
     const std::vector<Tensor> wide_lists = {offsets, perm, sorted_id};
     const bool early = with_reps && F > 0 && (cap + 1) * F <= kSmallReps && N <= kSmallClusters;
     if (early) a.reps = member_means("cluster_mean", input, nullptr, wide_lists, cap + 1, N);
-    // the one host read of a refresh
-    await(summary.data_ptr<int32_t>(), kNotYet, stream, op);
+    // The one host read of a refresh, in a stream with a training step ahead.  A copy behind the launch takes the host
+    // 24 us, a refresh of 60,000 rows and its products 262 us with it and 220 so; waiting for the stream after 200 us already
+    // makes a step of 3.77 ms 20 us longer.
+    await(summary.data_ptr<int32_t>(), kNotYet, std::chrono::milliseconds(5), stream, op);
     settle.pending = false;
     a.active = summary.data_ptr<int32_t>()[0];
     a.counts = counts.narrow(0, 0, a.active + 1);
@@ -1670,7 +1679,8 @@ std::tuple<Tensor, Tensor, Tensor> run_sampler(SampleGraph &G, const Tensor &inp
                               summary.data_ptr<int32_t>(), ws.data_ptr(), bytes, stream),
            op);
         const int32_t *sizes = summary.data_ptr<int32_t>();
-        await(sizes + 3, 0, stream, op);
+        // a stream with little work ahead has them within this time
+        await(sizes + 3, 0, kShortWait, stream, op);
         if (sizes[2] != -1) {  // -1: degrees that do not bound the lists; the layers then go one by one
             raise_on(sizes[2]);
             Tensor samples = torch::empty({sizes[0]}, i64), source = torch::empty({sizes[1]}, i64), neighbor = torch::empty({sizes[1]}, i64);

@@ -1240,3 +1240,52 @@ def test_edge_lists_of_either_precision_and_from_several_devices(kind):
     for wrong in ([ones[0][:, None]] + ones[1:], [ones[0][:-1]] + [torch.ones(len(w) + 1) for w in ones[1:]]):
         with pytest.raises(ValueError):
             CooPhasePlan(edges, wrong, V, R)
+
+
+@pytest.mark.parametrize("call", ["assignment", "sampler"])
+def test_other_threads_run_while_a_call_waits_for_the_stream(call):
+    """The host read of an assignment and of a sampled batch stands behind what the stream has still to do; the other
+    threads of the interpreter go on meanwhile."""
+    import threading
+    import time
+    import compressgnn_runtime as rt
+    import compressgnn_sample as sampler
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(13)
+    if call == "assignment":
+        x, planes = (torch.randn(n, m, device=DEV, generator=gen) for n, m in ((40000, 32), (32, 12)))
+        run = lambda: rt.cluster_assign_members(x, planes, 12)[0]
+    else:
+        ptr = torch.arange(0, 3 * 5000 + 1, 3, device=DEV)
+        col, seeds = (torch.randint(0, 5000, (n,), device=DEV, generator=gen) for n in (15000, 64))
+        run = lambda: sampler.neighbor_sample_ori_impl(ptr, col, seeds, [5, 5], seed=2)[0]
+    a = torch.randn(8192, 8192, device=DEV, generator=gen)
+    out = torch.empty_like(a)
+    want = run().clone()
+    torch.mm(a, a, out=out)
+    torch.cuda.synchronize()
+    stamps, stop = [], threading.Event()
+
+    def tick():
+        while not stop.is_set():
+            stamps.append(time.perf_counter())
+            time.sleep(0.0005)
+
+    ticker = threading.Thread(target=tick)
+    ticker.start()
+    try:
+        time.sleep(0.02)
+        for _ in range(16):  # 1.1 TFLOP each
+            torch.mm(a, a, out=out)
+        begin = time.perf_counter()
+        got = run()
+        end = time.perf_counter()
+        time.sleep(0.02)
+    finally:
+        stop.set()
+        ticker.join()
+    assert torch.equal(got, want)
+    assert end - begin > 0.03, "the stream was not busy"
+    inside = [begin] + [t for t in stamps if begin < t < end] + [end]
+    longest = max(later - earlier for earlier, later in zip(inside, inside[1:]))
+    assert longest < 0.5 * (end - begin)
