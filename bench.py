@@ -746,8 +746,18 @@ def main():
             xs = torch.randn(C1_VERTICES, Fs, device=dev, generator=gen)
             gs = torch.randn(C1_VERTICES, Fs, device=dev, generator=gen)
             ms = time_loop(lambda: (plan.forward(xs), plan.backward(gs)), args.steps, 2, torch)
-            nbytes = sum(t["bytes"] for t in graph_accounting(graph, Fs).values())
-            sweep[str(Fs)] = dict(ms_per_step=ms, bytes=nbytes, GBps=nbytes / (ms * 1e-3) / 1e9,
+            plan.timed_stages = ["*"]
+            plan.forward(xs), plan.backward(gs)
+            torch.cuda.synchronize()
+            ran = [name for name, _ in plan.take_stage_times()]
+            plan.timed_stages = []
+            # A direction without its rule stage went over the graph with the rules multiplied out, whose entries are
+            # those of the uncompressed product.
+            staged, nbytes = graph_accounting(graph, Fs), 0
+            for way, ptr, col in (("fwd", cp, row), ("bwd", v2, e2)):
+                nbytes += (sum(a["bytes"] for k, a in staged.items() if k.startswith(way)) if way + ".rules" in ran
+                           else block_bytes(ptr, col, C1_VERTICES, Fs, 0)["bytes"])
+            sweep[str(Fs)] = dict(ms_per_step=ms, launches=ran, bytes=nbytes, GBps=nbytes / (ms * 1e-3) / 1e9,
                                   frac_of_hbm_peak=nbytes / (ms * 1e-3) / 1e9 / HBM_PEAK_GBPS)
             del xs, gs
         detail["feature_sweep_C2"] = sweep

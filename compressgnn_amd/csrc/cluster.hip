@@ -973,8 +973,8 @@ __global__ __launch_bounds__(kBlock) void gather_rows_kernel(GatherArgs<T> a) {
 // 16-byte packs, so every store instruction of a wave covers 64
 // consecutive packs -- whole 128-byte lines -- wherever the rows begin and end.  A workgroup
 // takes a multiple of 64 rows (a whole number of lines whatever F is), enough of them for
-// every thread to have four packs; pack l of them lies in row l / packs_per_row, by
-// multiplication (exact for l < 2^16).
+// every thread to have four packs, or, where that makes few workgroups, a multiple of four (whole packs, lines that two
+// workgroups may share); pack l of them lies in row l / packs_per_row, by multiplication (exact for l < 2^16).
 //
 // WHOLE: a row is a whole number of packs.  Otherwise a pack may hold the end of one row and the beginning of the next: both
 // are read as a pack of their row (the last VEC elements of the one, the first of the other) and shifted

@@ -57,7 +57,9 @@ namespace {
 constexpr int kUnroll = 4;        // gathers in flight per lane and tile, nnz schedule (with 7 waves per SIMD;
                                   // 8 in flight with 5 waves measured the same)
 constexpr int kMidRound = 8, kDeepRound = 16;  // ... where a launch has few workgroups (launch_nnz)
-constexpr int64_t kResidentWorkgroups = 256 * 7;  // of the nnz kernel on the card at once, with kUnroll
+// Of the nnz kernel on an MI355X at once, with kUnroll.  Not asked of the device: run lengths follow from it, and with them
+// the workspaces of a product and where its sums are divided, which callers plan without a device as well.
+constexpr int64_t kResidentWorkgroups = 256 * 7;
 constexpr int kRowUnroll = 4;     // same for the row schedule (8: 9 % slower on web-graph out-lists, 2: 13 %, 16: 38 %)
 constexpr int kXcds = 8;          // accelerator dies of an MI355X, each with its own L2
 constexpr int kDefaultSeg = 64;   // non-zeros per lane group in the nnz schedule
@@ -1810,7 +1812,7 @@ __global__ __launch_bounds__(kBlock) void csr_once_kernel(const int64_t *__restr
                                                           int32_t *__restrict__ span) {
     constexpr int kPlaces = ITEMS * kBlock;
     __shared__ int32_t begins[kPlaces];  // the row that begins at an entry of the stretch, or -1
-    __shared__ int waves[2][kBlock / kWave];
+    __shared__ int waves[kBlock / kWave];
     __shared__ int64_t found[2];
     const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int64_t places[2] = {(int64_t)blockIdx.x * kPlaces, min(rows + nnz, (int64_t)(blockIdx.x + 1) * kPlaces)};
@@ -1884,14 +1886,14 @@ __global__ __launch_bounds__(kBlock) void csr_once_kernel(const int64_t *__restr
         const int n = __shfl_up(upto, s, kWave);
         if (lane >= s) upto = max(upto, n);
     }
-    if (lane == kWave - 1) waves[0][wave] = upto;
+    if (lane == kWave - 1) waves[wave] = upto;
     int before = __shfl_up(upto, 1, kWave);
     if (lane == 0) before = -1;
     __syncthreads();
     before = max(before, (int)row[0] - 1);
 #pragma unroll
     for (int w = 0; w < kBlock / kWave; ++w)
-        if (w < wave) before = max(before, waves[0][w]);
+        if (w < wave) before = max(before, waves[w]);
 #pragma unroll
     for (int u = 0; u < ITEMS; ++u) begins[threadIdx.x * ITEMS + u] = max(mark[u], before);
     __syncthreads();
@@ -1978,7 +1980,8 @@ __global__ void expand_summary_begin_kernel(uint64_t *__restrict__ out) {
     if (threadIdx.x < CGNN_EXPAND_SUMMARY) out[threadIdx.x] = is_least(threadIdx.x) ? ~uint64_t(0) : 0;
 }
 
-// cgnn_csr_expand_summary: integer sums and extremes, any order.
+// cgnn_csr_expand_summary: integer sums and extremes, any order.  Once per plan and direction; a launch and its few rounds of
+// loads (17 us for 50,001 rows of 545,000 entries), so a workgroup joins its words in LDS before it adds them to the summary.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void expand_summary_kernel(const int32_t *__restrict__ counts, int64_t rows,
                                                                 const int32_t *__restrict__ col, const T *__restrict__ val, int64_t nnz,

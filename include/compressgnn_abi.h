@@ -328,7 +328,8 @@ int cgnn_cluster_members(int64_t N, int64_t groups, const int64_t *ids, int32_t 
  * the number of groups, summary[1] = the size of the largest group.  counts needs room for min(N, 2^bits)+1 entries and offsets for one more; entries
  * beyond active+1 (active+2) are left untouched.  Replaces cluster_kernel.cu:143-150 and
  * the atomics of hash_ids (cluster_kernel.cu:41-59). */
-/* Up to cgnn_lsh_group_small_rows() rows the whole of it is one launch that needs no workspace.  The summary may lie in
+/* Up to cgnn_lsh_group_small_rows() rows the whole of it is one launch that needs no workspace (for callers that keep
+ * workspaces or count launches; the summary is written the same way for any number of rows).  The summary may lie in
  * pinned host memory; summary[0] is the last word that the call writes, so a host that finds it there finds all of
  * the summary, and the arrays as soon as the stream is done with the call. */
 int64_t cgnn_lsh_group_small_rows(void);
