@@ -126,6 +126,28 @@ def graph_accounting(graph, F):
     return acct
 
 
+def stage_names(plan, step, torch):
+    """The launches of a step, by their stages' names."""
+    plan.timed_stages = ["*"]
+    step()
+    torch.cuda.synchronize()
+    names = [name for name, _ in plan.take_stage_times()]
+    plan.timed_stages = []
+    return names
+
+
+def accounting_of(names, staged, plain):
+    """The figures of the stages that ran.  A direction without its rule stage went over the graph with the rules
+    multiplied out, whose entries are those of the uncompressed product."""
+    acct = {}
+    for way, block in plain.items():
+        if way + ".rules" in names:
+            acct.update((name, a) for name, a in staged.items() if name.startswith(way + "."))
+        else:
+            acct[way + ".final"] = block
+    return acct
+
+
 def build_c1(F):
     import compressgnn_offline as off
     from CompressgnnData import CompressgnnData
@@ -639,7 +661,7 @@ def main():
     dev = torch.device("cuda:0")
     data, (v_raw, e_raw) = build_c1(F)
     graph = data.edge_index
-    acct = graph_accounting(graph, F)
+    staged = graph_accounting(graph, F)
     data.to(dev)
     plan = graph.plan()
     gen = torch.Generator(device=dev)
@@ -696,6 +718,8 @@ def main():
     err = (out - ref_out).abs().max().item()
     early["max_abs_diff_vs_plain_csr"] = err
 
+    acct = accounting_of(stage_names(plan, step, torch), staged, dict(fwd=pb_f, bwd=pb_b))
+
     # The timed region: K steps, with a pair of HIP events around the dominant kernel on four of
     # them, evenly spread.  (An event pair leaves the stream idle for some 5 us on either side of the
     # launch, by the kernel trace; around every step that is 11 us of a 0.41 ms step that the workload
@@ -746,17 +770,9 @@ def main():
             xs = torch.randn(C1_VERTICES, Fs, device=dev, generator=gen)
             gs = torch.randn(C1_VERTICES, Fs, device=dev, generator=gen)
             ms = time_loop(lambda: (plan.forward(xs), plan.backward(gs)), args.steps, 2, torch)
-            plan.timed_stages = ["*"]
-            plan.forward(xs), plan.backward(gs)
-            torch.cuda.synchronize()
-            ran = [name for name, _ in plan.take_stage_times()]
-            plan.timed_stages = []
-            # A direction without its rule stage went over the graph with the rules multiplied out, whose entries are
-            # those of the uncompressed product.
-            staged, nbytes = graph_accounting(graph, Fs), 0
-            for way, ptr, col in (("fwd", cp, row), ("bwd", v2, e2)):
-                nbytes += (sum(a["bytes"] for k, a in staged.items() if k.startswith(way)) if way + ".rules" in ran
-                           else block_bytes(ptr, col, C1_VERTICES, Fs, 0)["bytes"])
+            ran = stage_names(plan, lambda: (plan.forward(xs), plan.backward(gs)), torch)
+            nbytes = sum(a["bytes"] for a in accounting_of(ran, graph_accounting(graph, Fs), dict(
+                fwd=block_bytes(cp, row, C1_VERTICES, Fs, 0), bwd=block_bytes(v2, e2, C1_VERTICES, Fs, 0))).values())
             sweep[str(Fs)] = dict(ms_per_step=ms, launches=ran, bytes=nbytes, GBps=nbytes / (ms * 1e-3) / 1e9,
                                   frac_of_hbm_peak=nbytes / (ms * 1e-3) / 1e9 / HBM_PEAK_GBPS)
             del xs, gs
