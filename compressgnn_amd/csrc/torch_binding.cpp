@@ -523,7 +523,7 @@ struct PropagationPlan {
     std::shared_ptr<DeviceCsr> vertex_stage, vertex_stage_t;
     MultipliedOut whole, whole_t;
     // the four blocks of the vertex stages on their own: only for the two-launch form
-    // (fuse_final = false); a plan without them holds the graph once
+    // (fuse_final = false); a plan without them holds its stages once
     std::shared_ptr<DeviceCsr> v2v, v2r, v2v_t, r2v_t;
     int64_t V = 0, R = 0;
     bool fuse_final = true;  // last two stages in one pass (cgnn_spmm_dual)

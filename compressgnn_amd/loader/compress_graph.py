@@ -184,7 +184,8 @@ class CompressGraph():
             backward_blocks = (host(self.v2v_graph.csc()), host(self.r2v_graph.csc()))
             # From here on the kernels read the plan's own int32 arrays: the int64 blocks go
             # back to host memory (csr()/csc() still deliver device tensors, as copies), so the
-            # device holds the graph once.  keep_device_blocks = True keeps them resident.
+            # device holds the stages alone (and, once a product takes it, the multiplied-out form
+            # of a graph of up to 4 M entries).  keep_device_blocks = True keeps the blocks resident.
             if not getattr(self, "keep_device_blocks", False):
                 for block in self.blocks():
                     block.offload()

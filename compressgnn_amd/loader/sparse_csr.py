@@ -7,7 +7,7 @@ host by the host library.  Both give the same arrays.
 
 offload(): a block that belongs to a GPU can keep its int64 arrays in host memory; csr() and
 csc() then upload a copy per call.  CompressGraph does that once its propagation plan (int32
-arrays of its own) is built, so that the device holds the graph once."""
+arrays of its own) is built, so that the device does not hold the blocks twice."""
 import _paths  # noqa: F401
 import numpy as np
 import torch
