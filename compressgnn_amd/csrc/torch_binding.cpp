@@ -607,6 +607,7 @@ std::array<MultipliedOut, 2> surveyed(const std::array<std::pair<DeviceCsr *, De
         const std::shared_ptr<Scratch> scratch = stage.scratch, of_rules = rules.scratch;
         Hold hold(scratch->lock), hold_rules(of_rules->lock);
         wanted[k] = stage.empty_rows.defined() && rules.nnz > 0 && stage.val.defined() && stage.nnz <= kMaxWholeEntries &&
+                    (stage.val.scalar_type() == torch::kFloat32 || stage.val.scalar_type() == torch::kFloat64) &&
                     (!rules.val.defined() || rules.val.scalar_type() == stage.val.scalar_type()) &&
                     stage.rowptr.device() == like.device() && rules.rowptr.device() == like.device();
         if (!wanted[k]) continue;

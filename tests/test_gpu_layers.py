@@ -355,6 +355,15 @@ def test_values_written_after_the_plan_was_made(which):
         assert_within(plan.backward(x).cpu().numpy(), want_g, rtol=1e-5, atol=2e-5)
 
 
+def test_plans_over_values_of_other_types():
+    """Values of a type that no product takes are refused by the product, as ever, and not while the plan is made."""
+    plan, _ = _plan_over(np.float16, *_random_stages(7))
+    x = torch.randn(300, 12, device=DEV)
+    for mat in (x, x.half()):
+        with pytest.raises(RuntimeError):
+            plan.forward(mat)
+
+
 def _requested():
     return torch.cuda.memory_stats()["requested_bytes.all.current"]
 
