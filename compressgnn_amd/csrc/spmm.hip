@@ -2043,6 +2043,7 @@ __global__ __launch_bounds__(kBlock) void expand_columns_kernel(const int32_t *_
     const int lane = threadIdx.x % kWave;
     const int32_t e0 = rowptr[row], e1 = rowptr[row + 1];
     int32_t out = out_ptr[row];
+    const int32_t end = out_ptr[row + 1];  // nothing behind it is this row's, whatever its columns have become since they were counted
     for (int64_t base = e0; base < e1; base += kWave) {
         const int64_t e = base + lane;
         int32_t c = 0, from = 0, n = 0;
@@ -2068,7 +2069,7 @@ __global__ __launch_bounds__(kBlock) void expand_columns_kernel(const int32_t *_
                 if (__shfl(upto, k + s - 1, kWave) <= p) k += s;
             const int32_t of = __shfl(c, k, kWave), at = __shfl(from, k, kWave) + p - __shfl(before, k, kWave);
             const T by = __shfl(w, k, kWave);
-            if (p >= total) continue;
+            if (p >= total || out + p >= end) continue;
             out_col[out + p] = of < split ? of : rule_col[at];
             out_val[out + p] = of >= split && rule_val != nullptr ? by * rule_val[at] : by;
         }

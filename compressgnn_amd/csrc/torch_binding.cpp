@@ -509,6 +509,7 @@ std::array<uint32_t, 4> written(const DeviceCsr &stage, const DeviceCsr &rules) 
 struct MultipliedOut {
     int64_t entries = 0;  // 0: never
     int32_t longest = 0;  // its longest row
+    Tensor starts;        // its row pointers
     std::array<uint32_t, 4> made_of{};
     std::shared_ptr<DeviceCsr> block;  // made for the first product that takes it
 };
@@ -592,6 +593,13 @@ bool products_in_range(const uint64_t *magnitudes) {
            of[1] * of[3] >= std::numeric_limits<T>::min();
 }
 
+// The block as a kernel reads it, beside a product on another thread that makes tables of it.
+cgnn_csr viewed(const DeviceCsr &A) {
+    const std::shared_ptr<Scratch> scratch = A.scratch;
+    Hold hold(scratch->lock);
+    return A.view();
+}
+
 // What the vertex stages [vertices | rules] of both directions come to with their rules multiplied out; no entries where no
 // product would take that, or a value has no place in it.  One host read.
 std::array<MultipliedOut, 2> surveyed(const std::array<std::pair<DeviceCsr *, DeviceCsr *>, 2> &stages, int64_t V) {
@@ -600,25 +608,31 @@ std::array<MultipliedOut, 2> surveyed(const std::array<std::pair<DeviceCsr *, De
     if (capturing(like)) return found;
     c10::hip::HIPGuardMasqueradingAsCUDA guard(like.device());
     const auto stream = current_stream(like);
-    Tensor summaries;
+    Tensor summaries, starts[2];
     bool wanted[2];
+    uint64_t empty[2] = {0, 0};
     for (int k = 0; k < 2; ++k) {
         const DeviceCsr &stage = *stages[k].first, &rules = *stages[k].second;
-        const std::shared_ptr<Scratch> scratch = stage.scratch, of_rules = rules.scratch;
-        Hold hold(scratch->lock), hold_rules(of_rules->lock);
-        wanted[k] = stage.empty_rows.defined() && rules.nnz > 0 && stage.val.defined() && stage.nnz <= kMaxWholeEntries &&
+        const Tensor empty_rows = locked(*stages[k].first, &DeviceCsr::empty_rows);
+        wanted[k] = empty_rows.defined() && rules.nnz > 0 && stage.val.defined() && stage.nnz <= kMaxWholeEntries &&
                     (stage.val.scalar_type() == torch::kFloat32 || stage.val.scalar_type() == torch::kFloat64) &&
                     (!rules.val.defined() || rules.val.scalar_type() == stage.val.scalar_type()) &&
                     stage.rowptr.device() == like.device() && rules.rowptr.device() == like.device();
         if (!wanted[k]) continue;
+        empty[k] = (uint64_t)empty_rows.numel();
         found[k].made_of = written(stage, rules);
         if (!summaries.defined()) summaries = torch::empty({2, CGNN_EXPAND_SUMMARY}, like.options().dtype(torch::kInt64));
-        const cgnn_csr a = stage.view(), r = rules.view();
+        const cgnn_csr a = viewed(stage), r = viewed(rules);
         Tensor counts = torch::empty({stage.rows}, like.options());
         ok(cgnn_csr_expand_count(&a, V, &r, counts.data_ptr<int32_t>(), stream), "csr_expand_count");
         ok(cgnn_csr_expand_summary(&a, V, &r, dtype_code(stage.val), counts.data_ptr<int32_t>(),
                                    reinterpret_cast<uint64_t *>(summaries[k].data_ptr<int64_t>()), stream),
            "csr_expand_summary");
+        starts[k] = torch::empty({stage.rows + 1}, like.options());
+        const size_t bytes = cgnn_exclusive_sum_workspace_bytes(stage.rows);
+        Tensor ws = torch::empty({(int64_t)bytes}, like.options().dtype(torch::kUInt8));
+        ok(cgnn_exclusive_sum_i32(stage.rows, counts.data_ptr<int32_t>(), starts[k].data_ptr<int32_t>(), nullptr, ws.data_ptr(), bytes, stream),
+           "exclusive_sum");
     }
     if (!summaries.defined()) return found;
     summaries = summaries.cpu();
@@ -628,9 +642,10 @@ std::array<MultipliedOut, 2> surveyed(const std::array<std::pair<DeviceCsr *, De
         const DeviceCsr &stage = *stages[k].first;
         const bool in_range = stage.val.scalar_type() == torch::kFloat32 ? products_in_range<float>(s + 3) : products_in_range<double>(s + 3);
         // (a row that only rules without entries stand in would be one that the stage's list of empty rows does not have)
-        if (s[0] > (uint64_t)kMaxWholeEntries || s[2] != (uint64_t)stage.empty_rows.numel() || !in_range) continue;
+        if (s[0] > (uint64_t)kMaxWholeEntries || s[2] != empty[k] || !in_range) continue;
         found[k].entries = (int64_t)s[0];
         found[k].longest = (int32_t)s[1];
+        found[k].starts = starts[k];
     }
     return found;
 }
@@ -656,7 +671,7 @@ std::shared_ptr<DeviceCsr> multiplied_out(PropagationPlan &p, MultipliedOut &who
         !takes_whole(whole.entries, *stage, *rules, x.size(1) * x.element_size()))
         return nullptr;
     if (whole.made_of != written(*stage, *rules)) {
-        whole = MultipliedOut();
+        whole.entries = 0;  // the block stays until the plan goes: a product on another stream may still read it
         return nullptr;
     }
     if (whole.block) return whole.block;
@@ -669,28 +684,20 @@ std::shared_ptr<DeviceCsr> multiplied_out(PropagationPlan &p, MultipliedOut &who
     blk->max_row_nnz = whole.longest;
     blk->seg_nnz = stage->seg_nnz;
     blk->rowmap = stage->rowmap;
-    blk->rowptr = torch::empty({stage->rows + 1}, ints);
-    blk->colidx = torch::empty({whole.entries}, ints);
-    blk->val = torch::empty({whole.entries}, stage->val.options());
+    blk->rowptr = whole.starts;
+    // A graph that recorded the making may be replayed after the columns were written to, and rows then come to more or fewer
+    // entries than they have room for: they are cut off, or keep entries (0, 0), so that the arrays are the block that the
+    // starts say whatever the columns are, and no product reads or writes outside them.
+    blk->colidx = torch::zeros({whole.entries}, ints);
+    blk->val = torch::zeros({whole.entries}, stage->val.options());
     // The plan's AUTO products run the row schedule or workgroup runs: neither asks which rows plain runs would cut.
     blk->cut_rows = torch::empty({1}, ints).narrow(0, 0, 0);
     blk->empty_rows = locked(*stage, &DeviceCsr::empty_rows);
     p.adopt(blk);
-    Tensor counts = torch::empty({stage->rows}, ints);
-    const size_t bytes = cgnn_exclusive_sum_workspace_bytes(stage->rows);
-    Tensor ws = torch::empty({(int64_t)bytes}, ints.dtype(torch::kUInt8));
-    {
-        const std::shared_ptr<Scratch> scratch = stage->scratch, of_rules = rules->scratch;
-        Hold hold(scratch->lock), hold_rules(of_rules->lock);
-        const cgnn_csr a = stage->view(), r = rules->view();
-        ok(cgnn_csr_expand_count(&a, p.V, &r, counts.data_ptr<int32_t>(), stream), "csr_expand_count");
-        ok(cgnn_exclusive_sum_i32(stage->rows, counts.data_ptr<int32_t>(), blk->rowptr.data_ptr<int32_t>(), nullptr, ws.data_ptr(), bytes,
-                                  stream),
-           "exclusive_sum");
-        ok(cgnn_csr_expand_columns(&a, p.V, &r, dtype_code(x), blk->rowptr.data_ptr<int32_t>(), blk->colidx.data_ptr<int32_t>(),
-                                   blk->val.data_ptr(), stream),
-           "csr_expand_columns");
-    }
+    const cgnn_csr a = viewed(*stage), r = viewed(*rules);
+    ok(cgnn_csr_expand_columns(&a, p.V, &r, dtype_code(x), blk->rowptr.data_ptr<int32_t>(), blk->colidx.data_ptr<int32_t>(),
+                               blk->val.data_ptr(), stream),
+       "csr_expand_columns");
     if (capturing(x)) return blk;
     TORCH_CHECK(synchronized(stream), "propagate: the stream reported an error");
     whole.block = blk;

@@ -212,7 +212,8 @@ int cgnn_csr_compose_columns(int64_t nnz, const int32_t *colidx, int64_t first_c
  * (k, w * v) of row c - split of `rules` (values of the block's type; without values v is 1), in their order and in its
  * place; the other entries stay.  cgnn_csr_expand_count writes the entries every row of A comes to (INT32_MAX if more
  * do not fit), cgnn_csr_expand_columns the new columns and values for the row starts that these sum up to
- * (cgnn_exclusive_sum_i32; no sum may have overflowed).  A needs values; its rowidx and rowmap are not looked at.
+ * (cgnn_exclusive_sum_i32; no sum may have overflowed; a row that comes to more than its starts leave it is cut off there).
+ * A needs values; its rowidx and rowmap are not looked at.
  * The product of the vertex stage of layer/CompressgnnSPMM.py:59-60 with its rule stage (:54) as one matrix.
  *
  * w * v is rounded to the block's type before it meets a row of features, where the two stages multiply through the sum

@@ -355,6 +355,32 @@ def test_values_written_after_the_plan_was_made(which):
         assert_within(plan.backward(x).cpu().numpy(), want_g, rtol=1e-5, atol=2e-5)
 
 
+def test_columns_written_between_the_replays_of_a_recorded_making():
+    """A graph whose capture holds a plan's first product of the multiplied-out form makes the block with every replay.  Where
+    the columns have changed meanwhile, so that it comes to more or fewer entries than there is room for, it stays inside its
+    arrays; and with the columns as they were its replays are right again."""
+    near, far, rules = _random_stages(8)
+    plan, _ = _plan_over(np.float32, near, far, rules)
+    x = torch.randn(300, 12, device=DEV)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        recorded = plan.forward(x), plan.backward(x)
+    want = plan.forward(x), plan.backward(x)
+    columns = plan.vertex_stage.colidx
+    kept = columns.clone()
+    for fewer in (None, True, False):
+        if fewer is not None:  # vertices alone; rules alone
+            columns.copy_(torch.randint(0, 300, kept.shape, device=DEV) if fewer else torch.randint(300, 324, kept.shape, device=DEV))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert recorded[0].shape == want[0].shape
+        columns.copy_(kept)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(recorded, want))
+
+
 def test_plans_over_values_of_other_types():
     """Values of a type that no product takes are refused by the product, as ever, and not while the plan is made."""
     plan, _ = _plan_over(np.float16, *_random_stages(7))
