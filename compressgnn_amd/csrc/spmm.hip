@@ -726,7 +726,14 @@ template <typename T, int VEC, int LPR, int TILES, int MODE, int WGRUNS, int ROU
 __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRound ? 5 : (TILES == 1 && LPR >= 16) ? 7 : 1) void spmm_nnz_kernel(SpmmArgs<T> a) {
     constexpr int GPB = kBlock / LPR;
     static_assert(LPR % ROUND == 0 || ROUND == kUnroll, "a round's entries come from one batch");
-    constexpr bool kAhead = ROUND == kDeepRound;  // the entries of the next batch are asked for before the gathers of this one
+    // What a lane group waits for between two batches of entries.  The entries of the next batch are asked for before the
+    // gathers of this one, and the rows of Y they go to (rowmap, a look-up that needs the entry) are waited for behind the
+    // gathers, which do not need them: a chain of entries -> gathers a batch, where it was entries -> rows -> gathers, one batch
+    // behind the other.  A launch that fits the card at once is little but that chain (web graphs, forward, us, before / so:
+    // 50,001 vertices of 47 features 23.5 / 22.2, 100,003 of 32 31.1 / 29.0, 200,003 of 16 45.7 / 42.7).  The two-source product
+    // of large graphs is bound by its traffic and sits at its register limit, the masked sums spill: neither reads ahead.
+    constexpr bool kAhead = ROUND == kDeepRound || has_values(MODE) || MODE == MODE_UNIT;
+    constexpr bool kRowsBehindGathers = MODE != MODE_DUAL;
     __shared__ int wg_row[GPB];
     __shared__ Pack<T, VEC> wg_carry[TILES][kBlock];
     __shared__ Pack<T, VEC> wg_head[WGRUNS != WGRUNS_NONE ? TILES : 1][WGRUNS != WGRUNS_NONE ? kBlock : 1];
@@ -835,7 +842,9 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
             if constexpr (kAhead) load_entry(e0);
             for (int e = e0; e < e1; e += LPR) {
                 if constexpr (!kAhead) load_entry(e);
-                int my_o = e + lane < e1 ? named(my_row) : 0;  // behind the others: it waits for the row
+                if constexpr (MODE != MODE_DUAL) arrive(my_c), arrive(my_row);
+                if constexpr (has_values(MODE)) arrive(my_w);
+                int my_o = e + lane < e1 ? named(my_row) : 0;
                 if constexpr (kNamesRowsOfY) {
                     // with every batch of entries, so that no load of the run waits for another but
                     // the row numbers for their rows (the same two words each time)
@@ -844,11 +853,11 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
                         row_behind = e1 < a.nnz ? a.rowidx[e1] : -1;
                     }
                     // the run begins with the row of its first entry
-                    const int batch_first = __builtin_amdgcn_ds_bpermute(group_lane0, my_o);
-                    if (e == e0) cur_out = batch_first;
+                    if constexpr (!kRowsBehindGathers) {
+                        const int batch_first = __builtin_amdgcn_ds_bpermute(group_lane0, my_o);
+                        if (e == e0) cur_out = batch_first;
+                    }
                 }
-                if constexpr (MODE != MODE_DUAL) arrive(my_o), arrive(my_c);
-                if constexpr (has_values(MODE)) arrive(my_w);
                 const int cnt = min(e1 - e, LPR);
                 const int this_c = my_c;
                 const T this_w = my_w;
@@ -859,7 +868,7 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
 #pragma unroll
                     for (int u = 0; u < ROUND; ++u) {
                         const int from = group_lane0 + 4 * (u0 + u);
-                        o[u] = __builtin_amdgcn_ds_bpermute(from, my_o);
+                        if constexpr (!kRowsBehindGathers) o[u] = __builtin_amdgcn_ds_bpermute(from, my_o);
                         c[u] = __builtin_amdgcn_ds_bpermute(from, this_c);
                         if constexpr (has_values(MODE) || MODE == MODE_DUAL)
                             w[u] = __builtin_bit_cast(T, __builtin_amdgcn_ds_bpermute(from, __builtin_bit_cast(int, this_w)));
@@ -889,6 +898,13 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
                                 for (int t = 0; t < TILES; ++t)
                                     x[u][t] = gather<T, VEC, MODE, (int)(VEC * LPR * sizeof(T))>(a, c[u], kPlain ? 0 : c[u] >= a.split, fld[t]);
                             }
+                        if constexpr (kRowsBehindGathers) {
+                            // the names of the rows are waited for behind the gathers, which do not need them
+                            if (u0 == 0) arrive(my_o);
+#pragma unroll
+                            for (int u = 0; u < ROUND; ++u) o[u] = __builtin_amdgcn_ds_bpermute(group_lane0 + 4 * (u0 + u), my_o);
+                            if (u0 == 0 && e == e0) cur_out = o[0];  // the run begins with the row of its first entry
+                        }
                         if constexpr (MODE != MODE_DUAL && !(kGatherAll && !has_values(MODE)))
 #pragma unroll
                             for (int u = 0; u < ROUND; ++u)
