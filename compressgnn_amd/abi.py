@@ -28,7 +28,7 @@ EXPORTS = [
     "cgnn_cluster_members_workspace_bytes", "cgnn_cluster_members",
     "cgnn_cluster_mean_workspace_bytes", "cgnn_cluster_mean", "cgnn_cluster_mean_backward",
     "cgnn_reconstruct", "cgnn_reconstruct_backward", "cgnn_sign_words", "cgnn_reconstruct_signs",
-    "cgnn_reconstruct_backward_signs", "cgnn_copy_bytes", "cgnn_read_bytes", "cgnn_fill_bytes",
+    "cgnn_reconstruct_backward_signs", "cgnn_reconstruct_masks", "cgnn_reconstruct_backward_masks", "cgnn_copy_bytes", "cgnn_read_bytes", "cgnn_fill_bytes",
     "cgnn_exclusive_sum_workspace_bytes", "cgnn_exclusive_sum_i32", "cgnn_sample_count", "cgnn_sample_fill",
     "cgnn_sample_relabel_begin", "cgnn_sample_relabel_workspace_bytes", "cgnn_sample_relabel", "cgnn_sample_layers_workspace_bytes", "cgnn_sample_layers", "cgnn_sample_layers_write",
 ]

@@ -871,6 +871,7 @@ struct GatherArgs {
     T *__restrict__ out;             // [N x F]
     int32_t *bad_id;                 // set to 1 when an id lies outside [0, groups), or NULL
     uint32_t *signs;                 // reconstruct: bit f % 32 of word [i, f / 32] = !(out[i, f] <= 0), or NULL
+    int32_t signs_by_group;          // ... of word [ids[i], f / 32]: the rows of a group are the same row
     int64_t N, F, groups;
     int32_t relu;
     int32_t sign_words;              // words per row of signs: ceil(F / 32)
@@ -959,10 +960,11 @@ __global__ __launch_bounds__(kBlock) void gather_rows_kernel(GatherArgs<T> a) {
 #pragma unroll
                 for (int r = 0; r < kGatherRows; ++r) {
                     if (first + r >= a.N) break;  // the same for all lanes of the row
+                    if (a.signs_by_group && r > 0 && g[r] == g[r - 1]) continue;  // and this; the word is written
                     uint32_t w = bits[r] << (f & 31);
 #pragma unroll
                     for (int d = 1; d < R; d <<= 1) w |= __shfl_xor(w, d);
-                    if (on && lane % R == 0) a.signs[row[r] * a.sign_words + (f >> 5)] = w;
+                    if (on && lane % R == 0) a.signs[(a.signs_by_group ? g[r] : row[r]) * a.sign_words + (f >> 5)] = w;
                 }
             }
         }
@@ -1121,13 +1123,17 @@ __global__ __launch_bounds__(kBlock) void gather_flat_kernel(GatherArgs<T> a, in
     if constexpr (SIGNS) {
         __syncthreads();
         const int words = rows * a.sign_words;
-        uint32_t *signs = a.signs + row0 * a.sign_words;
         const int last = (total - 1) / 32;
         for (int i = threadIdx.x; i < words; i += kBlock) {
             const int r = i / a.sign_words, w = i - r * a.sign_words;
             const int bit = r * F + 32 * w, left = F - 32 * w;
             const uint32_t v = __builtin_amdgcn_alignbit(sign_bits[min(bit / 32 + 1, last)], sign_bits[bit / 32], (uint32_t)bit % 32u);
-            signs[i] = left < 32 ? v & ((1u << left) - 1u) : v;
+            int64_t to = row0 + r;
+            if (a.signs_by_group) {
+                to = ids[r];
+                check(to);
+            }
+            a.signs[to * a.sign_words + w] = left < 32 ? v & ((1u << left) - 1u) : v;
         }
     }
 }
@@ -1481,7 +1487,7 @@ extern "C" int cgnn_cluster_sums(int64_t N, int64_t F, int64_t groups, int dtype
                                  void *workspace, size_t workspace_bytes, int32_t *arrivals, cgnn_stream_t stream) {
     CGNN_REQUIRE(N > 0 && F > 0 && groups > 0 && N < INT32_MAX - 65536, "cgnn_cluster_sums: bad size");
     CGNN_REQUIRE(dtype == CGNN_F32 || dtype == CGNN_F64, "cgnn_cluster_sums: dtype must be f32 or f64");
-    CGNN_REQUIRE(mask >= 0 && mask <= 2, "cgnn_cluster_sums: mask must be 0, 1 or 2");
+    CGNN_REQUIRE(mask >= 0 && mask <= 3, "cgnn_cluster_sums: mask must be 0, 1, 2 or 3");
     CGNN_REQUIRE(X && offsets && perm && sorted_id && sums && arrivals && (mask == 0 || M), "cgnn_cluster_sums: null array");
     cgnn_csr A = members_csr(N, groups, offsets, perm, sorted_id);
     int64_t n = 0;
@@ -1529,9 +1535,10 @@ extern "C" int cgnn_column_sums(int64_t rows, int64_t F, int dtype, const void *
 template <typename T, int OP>
 static int gather_typed(int64_t N, int64_t F, int64_t groups, const void *src, const int64_t *ids,
                         const int32_t *counts, const int32_t *perm, const void *bias, int relu, void *out,
-                        int32_t *bad_id, hipStream_t stream, uint32_t *signs = nullptr) {
+                        int32_t *bad_id, hipStream_t stream, uint32_t *signs = nullptr, bool signs_by_group = false) {
     GatherArgs<T> a{};
     a.signs = signs;
+    a.signs_by_group = signs_by_group;
     a.sign_words = (int32_t)ceil_div(F, 32);
     a.src = static_cast<const T *>(src);
     a.ids = ids;
@@ -1620,6 +1627,33 @@ extern "C" int cgnn_reconstruct_backward_signs(int64_t N, int64_t F, int64_t gro
     CGNN_REQUIRE(N == 0 || (grad && perm && sorted_id && signs), "cgnn_reconstruct_backward_signs: null array");
     cgnn_csr A = members_csr(N, groups, offsets, perm, sorted_id, max_members);
     return spmm_members(&A, dtype, grad, signs, reps_grad, F, 2, workspace, workspace_bytes, stream);
+}
+
+extern "C" int cgnn_reconstruct_masks(int64_t N, int64_t F, int64_t groups, int dtype, const void *reps, const int64_t *ids,
+                                      const int32_t *perm, const void *bias, void *out, uint32_t *masks, int32_t *bad_id,
+                                      cgnn_stream_t stream) {
+    CGNN_REQUIRE(N >= 0 && F >= 0 && groups >= 0, "cgnn_reconstruct_masks: bad size");
+    CGNN_REQUIRE(N == 0 || F == 0 || groups >= 1, "cgnn_reconstruct_masks: rows to reconstruct but no representatives");
+    if (N == 0 || F == 0) return CGNN_OK;
+    CGNN_REQUIRE(reps && ids && out && masks, "cgnn_reconstruct_masks: null array");
+    if (dtype == CGNN_F32)
+        return gather_typed<float, GATHER_RECONSTRUCT>(N, F, groups, reps, ids, nullptr, perm, bias, 1, out, bad_id, stream, masks, true);
+    if (dtype == CGNN_F64)
+        return gather_typed<double, GATHER_RECONSTRUCT>(N, F, groups, reps, ids, nullptr, perm, bias, 1, out, bad_id, stream, masks, true);
+    return fail(CGNN_EUNSUPPORTED, "cgnn_reconstruct_masks: dtype must be f32 or f64");
+}
+
+extern "C" int cgnn_reconstruct_backward_masks(int64_t N, int64_t F, int64_t groups, int64_t max_members, int dtype,
+                                               const void *grad, const uint32_t *masks, const int32_t *offsets,
+                                               const int32_t *perm, const int32_t *sorted_id, void *reps_grad,
+                                               void *workspace, size_t workspace_bytes, cgnn_stream_t stream) {
+    CGNN_REQUIRE(N >= 0 && F >= 0 && groups >= 0, "cgnn_reconstruct_backward_masks: bad size");
+    CGNN_REQUIRE(dtype == CGNN_F32 || dtype == CGNN_F64, "cgnn_reconstruct_backward_masks: dtype must be f32 or f64");
+    if (F == 0 || groups == 0) return CGNN_OK;
+    CGNN_REQUIRE(offsets && reps_grad, "cgnn_reconstruct_backward_masks: null array");
+    CGNN_REQUIRE(N == 0 || (grad && perm && sorted_id && masks), "cgnn_reconstruct_backward_masks: null array");
+    cgnn_csr A = members_csr(N, groups, offsets, perm, sorted_id, max_members);
+    return spmm_members(&A, dtype, grad, masks, reps_grad, F, 3, workspace, workspace_bytes, stream);
 }
 
 extern "C" int cgnn_read_bytes(const void *src, size_t n, void *sink, cgnn_stream_t stream) {

@@ -39,7 +39,8 @@
 //     up, in ascending order, so the sum does not depend on which one that is.
 //
 // Modes: VAL (stored values), ADD (the same, added to what Y holds), UNIT (all values 1: member lists, whose rows are gathered once), RELU_MASK (unit values, gathered
-// rows zeroed where a second matrix is <= 0), DUAL (columns below `split` gather from
+// rows zeroed where a second matrix is <= 0), SIGN_MASK (the same, the mask a bit per element), ROW_MASK (unit values, the finished
+// rows of Y zeroed by a bit per element), DUAL (columns below `split` gather from
 // X, the others from X1; the two partial sums are kept apart and combined as
 // (0 + sum1) + sum0, which is what two successive accumulating products give).
 //
@@ -68,7 +69,7 @@ constexpr int kDefaultSeg = 64;   // non-zeros per lane group in the nnz schedul
 // workgroup runs, or the same rule worked out by every lane group (blocks that are new with every call -- member
 // lists, cgnn_spmm_once: a launch for their table would cost more than the few dependent loads).
 enum { WGRUNS_NONE = 0, WGRUNS_TABLE = 1, WGRUNS_COMPUTED = 2 };
-enum { MODE_VAL = 0, MODE_UNIT = 1, MODE_RELU_MASK = 2, MODE_DUAL = 3, MODE_SIGN_MASK = 4, MODE_ADD = 5 };
+enum { MODE_VAL = 0, MODE_UNIT = 1, MODE_RELU_MASK = 2, MODE_DUAL = 3, MODE_SIGN_MASK = 4, MODE_ADD = 5, MODE_ROW_MASK = 6 };
 constexpr bool has_values(int mode) { return mode == MODE_VAL || mode == MODE_ADD; }
 
 template <typename T, int VEC>
@@ -87,6 +88,7 @@ struct SpmmArgs {
     const T *X1;  // MODE_DUAL: source of the columns >= split
     const T *M;   // MODE_RELU_MASK: rows of X are zeroed where M <= 0
     const uint32_t *signs;  // MODE_SIGN_MASK: the same with one bit per element (set: keep), sign_words words per row
+    const uint32_t *row_signs;  // MODE_ROW_MASK: such words for the rows of Y; also asked by the passes that add carries
     int32_t sign_words;
     T *Y;
     int32_t *carry_row;  // [nseg] row a run carries into, or -1
@@ -269,7 +271,7 @@ __device__ __forceinline__ Gathered<T, VEC, MODE> gather(const SpmmArgs<T> &a, i
     // features, 10^6 rows: 44 us so, 32 us kept).  A choice at compile time: the compiler merges the two loads of a
     // branch into one that is kept.  Kept rows cost the kernel that writes next most: behind the means of 2.4 M rows
     // the spread of 256 features took 725 us for 485 and the gradient of the means 283 us for 175.
-    if constexpr ((MODE == MODE_RELU_MASK || MODE == MODE_SIGN_MASK || MODE == MODE_UNIT) && kRowBytes > 128)
+    if constexpr ((MODE == MODE_RELU_MASK || MODE == MODE_SIGN_MASK || MODE == MODE_UNIT || MODE == MODE_ROW_MASK) && kRowBytes > 128)
         g.x = load_pack_stream<T, VEC>(base + off);
     else
         g.x = load_pack<T, VEC>(base + off);
@@ -284,6 +286,29 @@ __device__ __forceinline__ Gathered<T, VEC, MODE> gather(const SpmmArgs<T> &a, i
     if constexpr (MODE == MODE_RELU_MASK) g.m = load_pack_stream<T, VEC>(a.M + off);
     return g;
 }
+
+// MODE_ROW_MASK: the bits of a row of Y for one pack.  A row whose members are all masked alike (the gradient of a ReLU behind rows
+// that are copies of one representative) is summed unmasked and masked once: the same value, element by element, and the words are
+// one row per row of Y instead of one per member, which is a cache line a member however few of its bytes count (2,449,029 rows of
+// 256 features into 41,000: 503 us with a mask per member, 462 us so; the rows and their words 494, 483).
+template <int VEC>
+struct RowMask {
+    uint32_t word = ~0u, next = ~0u;
+
+    __device__ __forceinline__ void load(const uint32_t *signs, int32_t sign_words, int64_t F, int row, int64_t f) {
+        const uint32_t *words = signs + (int64_t)row * sign_words;
+        const int at = (int)(f >> 5);
+        word = words[at];
+        next = 0;  // as in gather()
+        if (VEC > 1 && (F & (VEC - 1)) != 0) next = words[min(at + 1, sign_words - 1)];
+    }
+    template <typename T>
+    __device__ __forceinline__ void apply(Pack<T, VEC> &x, int64_t f) const {
+        const uint32_t bits = __builtin_amdgcn_alignbit(next, word, (uint32_t)f & 31u);
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) x.v[i] = ((bits >> i) & 1u) ? x.v[i] : T(0);
+    }
+};
 
 // Accumulator of one output row.  MODE_DUAL keeps the sums over the two sources apart: the
 // entries of a row are sorted by column, so those of the first source come first; when the
@@ -347,7 +372,8 @@ struct Acc {
 // Y[row] = (MODE_ADD ? Y[row] : 0) + acc
 template <typename T, int VEC, int TILES, int MODE>
 __device__ __forceinline__ void write_row(T *Y, int64_t F, int row, const int64_t foff[TILES],
-                                          const Acc<T, VEC, TILES, MODE> &acc, T divisor = T(1)) {
+                                          const Acc<T, VEC, TILES, MODE> &acc, T divisor = T(1),
+                                          const RowMask<VEC> *mask = nullptr) {
     T *yrow = Y + (int64_t)row * F;
     // Whether the row is added to is known at compile time: a load of Y in the block that closes a row inside a run of
     // the nnz schedule would have to be waited for, with everything asked for before it, on every path behind the block.
@@ -367,6 +393,7 @@ __device__ __forceinline__ void write_row(T *Y, int64_t F, int row, const int64_
         if constexpr (MODE == MODE_UNIT)
 #pragma unroll
             for (int i = 0; i < VEC; ++i) o.v[i] = o.v[i] / divisor;
+        if constexpr (MODE == MODE_ROW_MASK) mask[t].template apply<T>(o, foff[t]);
         // Rows of the plain product that go out element by element are short or no whole lines, and the few of a small
         // graph are read next: kept (8 features over 4,000 vertices 4.1 us streaming, 3.7 kept; in packs 64
         // features over 50,001 vertices 12.3 us kept, 11.4 streaming).
@@ -637,6 +664,11 @@ __device__ __forceinline__ void join_rows(const SpmmArgs<T> &a, int block, int l
 #pragma unroll
                 for (int i = 0; i < VEC; ++i) o.v[i] = base.v[i] + o.v[i];
             }
+            if constexpr (MODE == MODE_ROW_MASK) {
+                RowMask<VEC> mask;
+                mask.load(a.row_signs, a.sign_words, a.F, row, foff[t]);
+                mask.template apply<T>(o, foff[t]);
+            }
             store_pack<T, VEC>(y + foff[t], o);
         }
     };
@@ -732,7 +764,7 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
     // behind the other.  A launch that fits the card at once is little but that chain (web graphs, forward, us, before / so:
     // 50,001 vertices of 47 features 23.5 / 22.2, 100,003 of 32 31.1 / 29.0, 200,003 of 16 45.7 / 42.7).  The two-source product
     // of large graphs is bound by its traffic and sits at its register limit, the masked sums spill: neither reads ahead.
-    constexpr bool kAhead = ROUND == kDeepRound || has_values(MODE) || MODE == MODE_UNIT;
+    constexpr bool kAhead = ROUND == kDeepRound || has_values(MODE) || MODE == MODE_UNIT || MODE == MODE_ROW_MASK;
     constexpr bool kRowsBehindGathers = MODE != MODE_DUAL;
     __shared__ int wg_row[GPB];
     __shared__ Pack<T, VEC> wg_carry[TILES][kBlock];
@@ -783,6 +815,7 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
     acc.clear();
     int cur = -1;
     int cur_out = -1;
+    RowMask<VEC> mask[TILES];
     // A row ends inside the run: it is written, or (the part of it that lies in this run) put aside
     // for the lane group where the row began.
     int row_e0 = e0;  // where the row at hand begins in the run
@@ -798,7 +831,13 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
             }
         }
         write_row<T, VEC, TILES, MODE>(a.Y, a.F, y_row, foff, acc,
-                                       MODE == MODE_UNIT && a.mean && !(began_before && row_e0 == e0) ? (T)(end - row_e0) : T(1));
+                                       MODE == MODE_UNIT && a.mean && !(began_before && row_e0 == e0) ? (T)(end - row_e0) : T(1), mask);
+    };
+    // A row's mask is asked for where the row begins and used where it ends, behind the gathers in between.
+    auto begin_row = [&](int y_row) {
+        if constexpr (MODE == MODE_ROW_MASK)
+#pragma unroll
+            for (int t = 0; t < TILES; ++t) mask[t].load(a.row_signs, a.sign_words, a.F, y_row, foff[t] < 0 ? 0 : foff[t]);
     };
     // the names of rows: see below
     constexpr bool kNamesRowsOfY = !(MODE == MODE_DUAL && VEC * LPR * sizeof(T) >= 512);
@@ -903,7 +942,10 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
                             if (u0 == 0) arrive(my_o);
 #pragma unroll
                             for (int u = 0; u < ROUND; ++u) o[u] = __builtin_amdgcn_ds_bpermute(group_lane0 + 4 * (u0 + u), my_o);
-                            if (u0 == 0 && e == e0) cur_out = o[0];  // the run begins with the row of its first entry
+                            if (u0 == 0 && e == e0) {  // the run begins with the row of its first entry
+                                cur_out = o[0];
+                                begin_row(cur_out);
+                            }
                         }
                         if constexpr (MODE != MODE_DUAL && !(kGatherAll && !has_values(MODE)))
 #pragma unroll
@@ -919,6 +961,7 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
                                     row_e0 = e + u0 + u;
                                     acc.clear();
                                     cur_out = o[u];
+                                    begin_row(cur_out);
                                 }
                                 acc.add(x[u], fld, w[u], kPlain ? 0 : c[u] >= a.split);
                             }
@@ -931,6 +974,7 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
         } else {
             if constexpr (kNamesRowsOfY) {
                 cur_out = named(a.rowidx[e0]);
+                begin_row(cur_out);
                 if constexpr (WGRUNS == WGRUNS_NONE) {
                     last_row = a.rowidx[e1 - 1];
                     row_behind = e1 < a.nnz ? a.rowidx[e1] : -1;
@@ -965,6 +1009,7 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
                             row_e0 = e + u;
                             acc.clear();
                             cur_out = o[u];
+                            begin_row(cur_out);
                         }
                         acc.add(x[u], foff, w[u], c[u] >= a.split);
                     }
@@ -1083,6 +1128,11 @@ __global__ __launch_bounds__(kBlock) void spmm_carry_reduce_kernel(SpmmArgs<T> a
                 // last run has stored its part already), so its result does not depend on
                 // timing; sent as an atomic only so that the lane need not wait for Y.
                 T *y = a.Y + (int64_t)out_row(a, cur) * a.F + f;
+                if (a.row_signs != nullptr) {  // the row's last run has masked its part
+                    RowMask<VEC> mask;
+                    mask.load(a.row_signs, a.sign_words, a.F, cur, f);
+                    mask.template apply<T>(acc, f);
+                }
 #pragma unroll
                 for (int i = 0; i < VEC; ++i)
                     if (f + i >= nominal) unsafeAtomicAdd(y + i, acc.v[i]);  // the elements before are the lane's before
@@ -1223,6 +1273,11 @@ __global__ __launch_bounds__(kBlock) void spmm_fixup_kernel(SpmmArgs<T> a) {
             }
             T *y = a.Y + (int64_t)out_row(a, row) * a.F + f;
             Pack<T, VEC> o = load_pack<T, VEC>(y);
+            if (a.row_signs != nullptr) {  // the row's last run has masked its part
+                RowMask<VEC> mask;
+                mask.load(a.row_signs, a.sign_words, a.F, row, f);
+                mask.template apply<T>(acc, f);
+            }
 #pragma unroll
             for (int i = 0; i < VEC; ++i) o.v[i] = o.v[i] + acc.v[i];
             if (MERGED && a.mean) {
@@ -1387,12 +1442,12 @@ enum { KIND_ROW = 0, KIND_NNZ = 1, KIND_FIXUP = 2, KIND_REDUCE = 3, KIND_FIXUP_R
 // block that is new with the call gain where hubs make long runs (8,000 rows 19.6 / 18.7) and lose where rows are short
 // (out-lists of 5,463 vertices, 208 features, the whole pass 14.3 / 16.7), which nothing tells apart before the launch.
 template <int MODE>
-constexpr bool kGoesDeep = MODE == MODE_UNIT || MODE == MODE_SIGN_MASK;
+constexpr bool kGoesDeep = MODE == MODE_UNIT || MODE == MODE_SIGN_MASK || MODE == MODE_ROW_MASK;
 
 template <int MODE, int WGRUNS>
 int round_of(int64_t workgroups, int64_t entries) {
     if (kGoesDeep<MODE> && workgroups <= (WGRUNS == WGRUNS_NONE ? 512 : 1024)) return kDeepRound;
-    return MODE == MODE_UNIT && workgroups <= kResidentWorkgroups && entries <= 3 << 18 ? kMidRound : kUnroll;
+    return (MODE == MODE_UNIT || MODE == MODE_ROW_MASK) && workgroups <= kResidentWorkgroups && entries <= 3 << 18 ? kMidRound : kUnroll;
 }
 
 template <typename T, int VEC, int LPR, int TILES>
@@ -1407,7 +1462,7 @@ void launch_nnz(int mode, const SpmmArgs<T> &a, dim3 grid, hipStream_t stream) {
                     hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, kMode, kRuns, kDeepRound>), grid, block, 0, stream, a);
                     return;
                 }
-            if constexpr (kMode == MODE_UNIT)
+            if constexpr (kMode == MODE_UNIT || kMode == MODE_ROW_MASK)
                 if (round == kMidRound) {
                     hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, kMode, kRuns, kMidRound>), grid, block, 0, stream, a);
                     return;
@@ -1421,12 +1476,14 @@ void launch_nnz(int mode, const SpmmArgs<T> &a, dim3 grid, hipStream_t stream) {
     const std::integral_constant<int, MODE_DUAL> dual;
     const std::integral_constant<int, MODE_SIGN_MASK> sign_mask;
     const std::integral_constant<int, MODE_RELU_MASK> relu_mask;
+    const std::integral_constant<int, MODE_ROW_MASK> row_mask;
     if (a.arrivals != nullptr && a.run_start == nullptr) {
         const std::integral_constant<int, WGRUNS_COMPUTED> computed;
         if (mode == MODE_UNIT) go(unit, computed);
         else if (mode == MODE_VAL && a.accumulate) go(add, computed);
         else if (mode == MODE_VAL) go(val, computed);
         else if (mode == MODE_SIGN_MASK) go(sign_mask, computed);
+        else if (mode == MODE_ROW_MASK) go(row_mask, computed);
         else go(relu_mask, computed);
     } else if (a.arrivals != nullptr) {
         const std::integral_constant<int, WGRUNS_TABLE> table;
@@ -1440,6 +1497,7 @@ void launch_nnz(int mode, const SpmmArgs<T> &a, dim3 grid, hipStream_t stream) {
         else if (mode == MODE_UNIT) go(unit, none);
         else if (mode == MODE_DUAL) go(dual, none);
         else if (mode == MODE_SIGN_MASK) go(sign_mask, none);
+        else if (mode == MODE_ROW_MASK) go(row_mask, none);
         else go(relu_mask, none);
     }
 }
@@ -1669,9 +1727,9 @@ int spmm_typed(const cgnn_csr *A, const void *X, const void *X1, int64_t split, 
     if (A->rows == 0 || F == 0) return CGNN_OK;
     if (mode != MODE_DUAL) split = INT32_MAX;  // every column comes from X
     SpmmArgs<T> a = make_args<T>(A, X, X1, split, M, Y, F, accumulate);
-    const bool masked = mode == MODE_RELU_MASK || mode == MODE_SIGN_MASK;
-    if (mode == MODE_SIGN_MASK) {  // M holds bits, not rows
-        a.signs = static_cast<const uint32_t *>(M);
+    const bool masked = mode == MODE_RELU_MASK || mode == MODE_SIGN_MASK || mode == MODE_ROW_MASK;
+    if (mode == MODE_SIGN_MASK || mode == MODE_ROW_MASK) {  // M holds bits, not rows
+        (mode == MODE_SIGN_MASK ? a.signs : a.row_signs) = static_cast<const uint32_t *>(M);
         a.sign_words = (int32_t)ceil_div(F, 32);
         a.M = nullptr;
         M = nullptr;
@@ -2096,10 +2154,14 @@ __global__ __launch_bounds__(kBlock) void expand_columns_kernel(const int32_t *_
 }  // namespace
 
 // Entry used by the cluster reductions (mean: as for spmm_typed; unit values; mask: 0 none, 1 the rows of M, where M <= 0 drops
-// the element, 2 M holds ceil(F / 32) words of bits per row, where a clear bit drops it).
+// the element, 2 M holds ceil(F / 32) words of bits per row, where a clear bit drops it, 3 such words per sum).
+static int member_mode(int mask) {
+    return mask == 3 ? MODE_ROW_MASK : (mask == 2 ? MODE_SIGN_MASK : (mask == 1 ? MODE_RELU_MASK : MODE_UNIT));
+}
+
 int spmm_members(const cgnn_csr *A, int dtype, const void *X, const void *M, void *Y, int64_t F,
                  int mask, void *ws, size_t ws_bytes, hipStream_t stream, bool *mean) {
-    const int mode = mask == 2 ? MODE_SIGN_MASK : (mask == 1 ? MODE_RELU_MASK : MODE_UNIT);
+    const int mode = member_mode(mask);
     if (dtype == CGNN_F32)
         return spmm_typed<float>(A, X, nullptr, 0, M, Y, F, 0, CGNN_SPMM_NNZ, mode, ws, ws_bytes, stream, mean);
     if (dtype == CGNN_F64)
@@ -2119,8 +2181,9 @@ int spmm_member_runs(const cgnn_csr *A, int dtype, const void *X, const void *M,
         if (ws == nullptr || ws_bytes < wg_piece_bytes(workgroups, F, sizeof(T)))
             return fail(CGNN_EWORKSPACE, "member sums: workspace too small");
         SpmmArgs<T> a = make_args<T>(A, X, nullptr, INT32_MAX, M, Y, F, 0);
-        if (mask == 2) {
-            a.signs = static_cast<const uint32_t *>(M);
+        const int mode = member_mode(mask);
+        if (mode == MODE_SIGN_MASK || mode == MODE_ROW_MASK) {
+            (mode == MODE_SIGN_MASK ? a.signs : a.row_signs) = static_cast<const uint32_t *>(M);
             a.sign_words = (int32_t)ceil_div(F, 32);
         }
         a.arrivals = arrivals;
@@ -2129,7 +2192,7 @@ int spmm_member_runs(const cgnn_csr *A, int dtype, const void *X, const void *M,
         a.nseg = (int32_t)(workgroups * groups);
         a.carry = static_cast<T *>(ws);
         a.find_empty = 1;
-        return launch<T>(KIND_NNZ, mask == 2 ? MODE_SIGN_MASK : (mask == 1 ? MODE_RELU_MASK : MODE_UNIT), s, a, a.nseg, stream);
+        return launch<T>(KIND_NNZ, mode, s, a, a.nseg, stream);
     };
     return dtype == CGNN_F32 ? run(0.0f) : run(0.0);
 }

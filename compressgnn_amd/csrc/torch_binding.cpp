@@ -1272,9 +1272,10 @@ Tensor member_sums(const char *op, const Tensor &rows, int mask, const void *M, 
         ok(cgnn_cluster_sums(N, F, groups, dtype, rows.data_ptr(), mask, M, offsets, perm, sorted_id, out.data_ptr(), ws.data_ptr(),
                              bytes, counters.data_ptr<int32_t>(), stream),
            op);
-    } else if (mask == 2) {
-        ok(cgnn_reconstruct_backward_signs(N, F, groups, largest_group(m), dtype, rows.data_ptr(), static_cast<const uint32_t *>(M),
-                                           offsets, perm, sorted_id, out.data_ptr(), ws.data_ptr(), bytes, stream),
+    } else if (mask >= 2) {
+        const auto run = mask == 3 ? cgnn_reconstruct_backward_masks : cgnn_reconstruct_backward_signs;
+        ok(run(N, F, groups, largest_group(m), dtype, rows.data_ptr(), static_cast<const uint32_t *>(M), offsets, perm, sorted_id,
+               out.data_ptr(), ws.data_ptr(), bytes, stream),
            op);
     } else {
         ok(cgnn_reconstruct_backward(N, F, groups, largest_group(m), dtype, rows.data_ptr(), M, offsets, perm, sorted_id, mask,
@@ -1396,11 +1397,11 @@ Tensor cluster_reconstruct_backward(Tensor grad, Tensor index, Tensor output, in
 }
 
 // The ReLU form of cluster_reconstruct that also returns the sign of every output element as one
-// bit: (rows [N, F], signs int32 [N, ceil(F / 32)]).  A layer keeps the signs for its backward pass
-// instead of the rows (the reference keeps the rows: layer/CompressgnnReconstruct.py:16-22).
-std::tuple<Tensor, Tensor> cluster_reconstruct_signs(Tensor reps, Tensor index, c10::optional<Tensor> bias,
-                                                     c10::optional<std::vector<Tensor>> members) {
-    const char *op = "cluster_reconstruct_signs";
+// bit: (rows [N, F], signs int32 [N, ceil(F / 32)]), or, by group, masks int32 [groups, ceil(F / 32)]: the rows
+// of a group are copies of one representative and have the same signs.
+std::tuple<Tensor, Tensor> reconstruct_with_signs(const char *op, const Tensor &reps, const Tensor &index,
+                                                  const c10::optional<Tensor> &bias, const c10::optional<std::vector<Tensor>> &members,
+                                                  bool by_group) {
     expect(op, reps, {{Role::Features, "representatives", &reps}, {Role::Ids, "index", &index}});
     if (bias.has_value()) {
         expect(op, reps, {{Role::Bias, "bias", &*bias}});
@@ -1410,36 +1411,57 @@ std::tuple<Tensor, Tensor> cluster_reconstruct_signs(Tensor reps, Tensor index, 
     c10::hip::HIPGuardMasqueradingAsCUDA guard(reps.device());
     const int64_t N = index.numel(), F = reps.size(1);
     Tensor out = torch::empty({N, F}, reps.options());
-    Tensor signs = torch::empty({N, cgnn_sign_words(F)}, reps.options().dtype(torch::kInt32));
+    Tensor signs = torch::empty({by_group ? reps.size(0) : N, cgnn_sign_words(F)}, reps.options().dtype(torch::kInt32));
     if (out.numel() == 0) return {out, signs};
     std::vector<Tensor> held;
     const int32_t *perm = production_order(op, members, index, reps.size(0), &held);
     c10::optional<IdFlag> bad;
     if (perm == nullptr) bad.emplace(index);
-    ok(cgnn_reconstruct_signs(N, F, reps.size(0), dtype_code(reps), reps.data_ptr(), index.data_ptr<int64_t>(), perm,
-                              bias.has_value() ? bias->data_ptr() : nullptr, out.data_ptr(),
-                              reinterpret_cast<uint32_t *>(signs.data_ptr<int32_t>()), bad ? bad->ptr() : nullptr,
-                              current_stream(reps)),
+    const auto run = by_group ? cgnn_reconstruct_masks : cgnn_reconstruct_signs;
+    ok(run(N, F, reps.size(0), dtype_code(reps), reps.data_ptr(), index.data_ptr<int64_t>(), perm,
+           bias.has_value() ? bias->data_ptr() : nullptr, out.data_ptr(), reinterpret_cast<uint32_t *>(signs.data_ptr<int32_t>()),
+           bad ? bad->ptr() : nullptr, current_stream(reps)),
        op);
     if (bad) remember_checked_index(op, *bad, index, reps.size(0));
     return {out, signs};
 }
 
-// cluster_reconstruct_backward with relu = true, the mask taken from the signs above.
-Tensor cluster_reconstruct_backward_signs(Tensor grad, Tensor index, Tensor signs, int64_t groups,
-                                          c10::optional<std::vector<Tensor>> members) {
-    const char *op = "cluster_reconstruct_backward_signs";
+// cluster_reconstruct_backward with relu = true, the mask taken from the words above.
+Tensor reconstruct_backward_with_signs(const char *op, const Tensor &grad, const Tensor &index, const Tensor &signs, int64_t groups,
+                                       const c10::optional<std::vector<Tensor>> &members, bool by_group) {
     expect(op, grad, {{Role::Features, "grad", &grad}, {Role::Ids, "index", &index}});
     TORCH_CHECK(groups >= 0, op, ": groups = ", groups);
     TORCH_CHECK(index.numel() == grad.size(0), op, ": ", grad.size(0), " rows but ", index.numel(), " cluster ids");
-    const int64_t N = grad.size(0), F = grad.size(1);
+    const int64_t N = grad.size(0), F = grad.size(1), of = by_group ? groups : N;
     TORCH_CHECK(signs.device() == grad.device() && signs.scalar_type() == torch::kInt32 && signs.is_contiguous() &&
-                    signs.dim() == 2 && signs.size(0) == N && signs.size(1) == cgnn_sign_words(F),
-                op, ": signs must be a contiguous int32 tensor [", N, ", ", cgnn_sign_words(F), "] on the device of grad");
+                    signs.dim() == 2 && signs.size(0) == of && signs.size(1) == cgnn_sign_words(F),
+                op, by_group ? ": masks" : ": signs", " must be a contiguous int32 tensor [", of, ", ", cgnn_sign_words(F),
+                "] on the device of grad");
     c10::hip::HIPGuardMasqueradingAsCUDA guard(grad.device());
     if (grad.numel() == 0 || groups == 0) return torch::zeros({groups, F}, grad.options());
     auto m = members_or_build(op, members, index, groups);
-    return member_sums(op, grad, 2, signs.data_ptr<int32_t>(), m, groups);
+    return member_sums(op, grad, by_group ? 3 : 2, signs.data_ptr<int32_t>(), m, groups);
+}
+
+std::tuple<Tensor, Tensor> cluster_reconstruct_signs(Tensor reps, Tensor index, c10::optional<Tensor> bias,
+                                                     c10::optional<std::vector<Tensor>> members) {
+    return reconstruct_with_signs("cluster_reconstruct_signs", reps, index, bias, members, false);
+}
+
+Tensor cluster_reconstruct_backward_signs(Tensor grad, Tensor index, Tensor signs, int64_t groups,
+                                          c10::optional<std::vector<Tensor>> members) {
+    return reconstruct_backward_with_signs("cluster_reconstruct_backward_signs", grad, index, signs, groups, members, false);
+}
+
+// By group: what a layer keeps for its backward pass (the reference keeps the rows: layer/CompressgnnReconstruct.py:16-22).
+std::tuple<Tensor, Tensor> cluster_reconstruct_masks(Tensor reps, Tensor index, c10::optional<Tensor> bias,
+                                                     c10::optional<std::vector<Tensor>> members) {
+    return reconstruct_with_signs("cluster_reconstruct_masks", reps, index, bias, members, true);
+}
+
+Tensor cluster_reconstruct_backward_masks(Tensor grad, Tensor index, Tensor masks, int64_t groups,
+                                          c10::optional<std::vector<Tensor>> members) {
+    return reconstruct_backward_with_signs("cluster_reconstruct_backward_masks", grad, index, masks, groups, members, true);
 }
 
 // ------------------------------------------------------ the layers' autograd steps ----
@@ -1538,7 +1560,7 @@ Tensor column_sums(const Tensor &x) {
 }
 
 struct ReconstructBackward : torch::autograd::Node {
-    torch::autograd::SavedVariable index, signs;  // signs: one bit per element, where the rows went through a ReLU
+    torch::autograd::SavedVariable index, masks;  // masks: one bit per element of a representative, where the rows went through a ReLU
     Members members;
     int64_t groups = 0;
     bool relu = false, with_bias = false;
@@ -1551,7 +1573,7 @@ struct ReconstructBackward : torch::autograd::Node {
             at::NoGradGuard no_grad;
             const Tensor d_rows = grads[0].contiguous(), ids = index.unpack();
             // without a ReLU the operator does not read the rows it is given as output
-            out.push_back(relu ? cluster_reconstruct_backward_signs(d_rows, ids, signs.unpack(), groups, members)
+            out.push_back(relu ? cluster_reconstruct_backward_masks(d_rows, ids, masks.unpack(), groups, members)
                                : cluster_reconstruct_backward(d_rows, ids, d_rows, groups, false, members));
             if (with_bias) out.push_back(task_should_compute_output(1) ? column_sums(out[0]) : Tensor());
         }
@@ -1559,31 +1581,31 @@ struct ReconstructBackward : torch::autograd::Node {
     }
     void release_variables() override {
         index.reset_data();
-        signs.reset_data();
+        masks.reset_data();
         members.reset();
     }
     std::string name() const override { return "ReconstructBackward"; }
 };
 
 // rows[i] = act(reps[index[i]] + bias) with its gradients.  The ReLU mask of the gradient is kept as one bit
-// per element, written by the kernel that produces the rows (the reference keeps the rows themselves:
+// per element of a representative, written by the kernel that produces the rows (the reference keeps the rows themselves:
 // layer/CompressgnnReconstruct.py:16-22); without a ReLU nothing of the [N, F] output is needed again.
 c10::optional<Tensor> reconstruct(Tensor reps, Tensor index, c10::optional<Tensor> bias, bool relu, Members members) {
     if (needs_function(reps, bias)) return c10::nullopt;
-    Tensor rows, signs, ids;
+    Tensor rows, masks, ids;
     {
         at::AutoDispatchBelowADInplaceOrView plain;
         ids = index.contiguous();
         c10::optional<Tensor> b;
         if (bias.has_value() && bias->defined()) b = bias->contiguous();
-        if (relu) std::tie(rows, signs) = cluster_reconstruct_signs(reps.contiguous(), ids, b, members);
+        if (relu) std::tie(rows, masks) = cluster_reconstruct_masks(reps.contiguous(), ids, b, members);
         else rows = cluster_reconstruct(reps.contiguous(), ids, b, false, members);
     }
     const bool with_bias = bias.has_value() && bias->defined();
     if (at::GradMode::is_enabled() && (reps.requires_grad() || (with_bias && bias->requires_grad()))) {
         auto node = with_bias ? node_over<ReconstructBackward>(reps, *bias) : node_over<ReconstructBackward>(reps);
         node->index = torch::autograd::SavedVariable(ids, false);
-        if (relu) node->signs = torch::autograd::SavedVariable(signs, false);
+        if (relu) node->masks = torch::autograd::SavedVariable(masks, false);
         node->members = std::move(members);
         node->groups = reps.size(0);
         node->relu = relu;
@@ -2054,6 +2076,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("cluster_reconstruct_backward_signs", &cluster_reconstruct_backward_signs,
           "cluster_reconstruct_backward with ReLU, masked by the sign bits", py::arg("grad"), py::arg("index"),
           py::arg("signs"), py::arg("groups"), py::arg("members") = py::none());
+    m.def("cluster_reconstruct_masks", &cluster_reconstruct_masks,
+          "cluster_reconstruct with ReLU -> (rows, one sign bit per element of a representative)", py::arg("reps"),
+          py::arg("index"), py::arg("bias"), py::arg("members") = py::none());
+    m.def("cluster_reconstruct_backward_masks", &cluster_reconstruct_backward_masks,
+          "cluster_reconstruct_backward with ReLU, masked by the representatives' sign bits", py::arg("grad"), py::arg("index"),
+          py::arg("masks"), py::arg("groups"), py::arg("members") = py::none());
     m.def("csr_transpose", &csr_transpose, "CSR -> CSC of an int64 block on the GPU, SparseTensor.csc() order",
           py::arg("rowptr"), py::arg("col"), py::arg("value"), py::arg("cols"));
     // the native steps of the layers: None under torch.jit.trace, for inputs with a tangent and under torch.func

@@ -341,7 +341,8 @@ int cgnn_lsh_group(int64_t N, int bits, const int32_t *raw_code, int64_t *ids, i
 
 /* The sums over the members of every group in one launch, the form the gradients use: sums[g,:] = the sum over
  * members i of group g of X[i,:]; mask 1: elements dropped where M[N x F] <= 0, mask 2: where a bit of
- * M[N x ceil(F / 32)] is clear (as in cgnn_reconstruct_backward and its _signs form).  A group of at most 64
+ * M[N x ceil(F / 32)] is clear (as in cgnn_reconstruct_backward and its _signs form), mask 3: sums dropped where a
+ * bit of M[groups x ceil(F / 32)] is clear (its _masks form).  A group of at most 64
  * members is summed in ascending order; a larger one in an order that depends on the sizes alone.
  * arrivals: counters (as many as the size query reports), zero before and after the call, as in cgnn_csr.
  * N > 0 and F > 0.  No counters reported: there are so many rows that cgnn_reconstruct_backward and its _signs form
@@ -406,6 +407,19 @@ int cgnn_reconstruct_signs(int64_t N, int64_t F, int64_t groups, int dtype, cons
                            uint32_t *signs, int32_t *bad_id, cgnn_stream_t stream);
 int cgnn_reconstruct_backward_signs(int64_t N, int64_t F, int64_t groups, int64_t max_members, int dtype,
                                     const void *grad, const uint32_t *signs, const int32_t *offsets,
+                                    const int32_t *perm, const int32_t *sorted_id, void *reps_grad,
+                                    void *workspace, size_t workspace_bytes, cgnn_stream_t stream);
+
+/* The same pair with one mask per group: the rows of a group are copies of one representative, so they are masked
+ * alike.  cgnn_reconstruct_masks is cgnn_reconstruct with relu = 1 that also writes masks[ids[i] * W + f / 32], the
+ * words above, for every group that occurs in ids (the words of other groups are left untouched, and not read).
+ * cgnn_reconstruct_backward_masks sums the members and drops the sums whose bit is clear: the values of
+ * cgnn_reconstruct_backward bit for bit. */
+int cgnn_reconstruct_masks(int64_t N, int64_t F, int64_t groups, int dtype, const void *reps,
+                           const int64_t *ids, const int32_t *perm, const void *bias, void *out,
+                           uint32_t *masks, int32_t *bad_id, cgnn_stream_t stream);
+int cgnn_reconstruct_backward_masks(int64_t N, int64_t F, int64_t groups, int64_t max_members, int dtype,
+                                    const void *grad, const uint32_t *masks, const int32_t *offsets,
                                     const int32_t *perm, const int32_t *sorted_id, void *reps_grad,
                                     void *workspace, size_t workspace_bytes, cgnn_stream_t stream);
 

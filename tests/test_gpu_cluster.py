@@ -403,6 +403,46 @@ def test_sign_bits_of_special_values():
     assert np.array_equal(got, oracle.reconstruct_backward(go, ids, want, 3, True))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("n,width,clusters", [(1, 1, 1), (70, 33, 9), (2708, 16, 90), (9001, 47, 3), (30011, 100, 700), (200003, 31, 40),
+                                              (250007, 20, 3000), (250007, 256, 2), (520001, 5, 1), (60011, 520, 41)])
+def test_one_mask_per_representative(n, width, clusters, dtype):
+    """Masks of representatives against the masks of their rows, bit for bit: rows, words and gradients, where the sums are one
+    launch, runs with carries, and carries of several levels; NaN, infinities and zeros of both signs among the
+    representatives, infinities and NaN in the gradient.  An unused group has no members and a gradient of zero."""
+    import compressgnn_runtime as rt
+    gen = torch.Generator(device=DEV).manual_seed(n + width)
+    ids = (torch.rand(n, device=DEV, generator=gen) ** 3 * clusters).long()
+    ids[:min(n, clusters)] = torch.arange(min(n, clusters), device=DEV)
+    groups = clusters + 1
+    reps = torch.randn(groups, width, device=DEV, generator=gen, dtype=dtype)
+    reps.view(-1)[::11], reps.view(-1)[5::13], reps.view(-1)[7::17], reps.view(-1)[3::19] = 0.0, -0.0, float("nan"), -float("inf")
+    bias = torch.randn(width, device=DEV, generator=gen, dtype=dtype)
+    bias[::3] = 0.0
+    grad = torch.randn(n, width, device=DEV, generator=gen, dtype=dtype)
+    grad.view(-1)[::101], grad.view(-1)[50::103] = float("inf"), float("nan")
+    lists = list(abi.cluster_members(ids, groups))
+    for members in (lists, None):
+        rows, signs = rt.cluster_reconstruct_signs(reps, ids, bias, members)
+        same, masks = rt.cluster_reconstruct_masks(reps, ids, bias, members)
+        assert torch.equal(rows.view(torch.uint8), same.view(torch.uint8))
+        assert torch.equal(masks[ids], signs)
+        want = rt.cluster_reconstruct_backward_signs(grad, ids, signs, groups, members)
+        got = rt.cluster_reconstruct_backward_masks(grad, ids, masks, groups, members)
+        assert torch.equal(torch.nan_to_num(got, nan=3.0), torch.nan_to_num(want, nan=3.0))
+        assert torch.equal(got[clusters], torch.zeros(width, device=DEV, dtype=dtype))
+
+
+def test_masks_of_the_wrong_shape_are_refused():
+    import compressgnn_runtime as rt
+    ids = torch.tensor([0, 1, 1], device=DEV)
+    grad = torch.zeros(3, 40, device=DEV)
+    for bad in (torch.zeros(3, 2, device=DEV, dtype=torch.int32), torch.zeros(2, 1, device=DEV, dtype=torch.int32),
+                torch.zeros(2, 2, device=DEV), torch.zeros(2, 2, dtype=torch.int32), torch.zeros(4, 2, device=DEV, dtype=torch.int32)[::2]):
+        with pytest.raises(RuntimeError, match="masks"):
+            rt.cluster_reconstruct_backward_masks(grad, ids, bad, 2)
+
+
 def test_memory_probes_move_what_they_say():
     """The calibration kernels: the copy reproduces its source, the fill writes zeros over exactly n bytes."""
     import ctypes
