@@ -27,49 +27,49 @@ constexpr int kDigits = 1 << kDigitBits;           // one per thread of a workgr
 static_assert(kDigits == kBlock, "one digit per thread");
 
 // How the keys are dealt out: `items` per thread of a workgroup's tile, and whether the workgroups of a scatter add up the
-// histograms of the tiles for themselves (`own_scan`) or a launch in between does.  Up to 128 tiles the former costs four
-// rounds of loads that hit the L2s, no more than the launch and its dependence; few keys take small tiles, since a
-// tile is ranked 64 keys a wave and step, one step after the other, and 4,096 keys a tile leave most of the card idle.
-// Hashing and grouping rows of 24 columns by 16 planes, us, with tiles of 4,096, a launch for the scan and a copy of
-// the group count / so: 9,000 rows 76 / 58, 30,011 73 / 58, 100,003 74 / 66, 200,000 77 / 71, 300,007 79 / 81,
-// 450,000 86 / 89 (kernels alone at 300,007: 69 / 65).  More keys keep the launch and the large tiles:
-// 2,048 a tile 0.301 against 0.293 ms for a refresh of 2.4 M rows.
+// histograms of the tiles for themselves (`own_scan`) or a launch in between does.  Up to 128 tiles the former is one round
+// of loads that hit the L2s, up to 256 tiles two, no more than the launch and its dependence (hashing and grouping rows of 24
+// columns by 16 planes, us, scan launch / own scan: 524,289 rows 74.6 / 71.8, 700,001 79.2 / 76.8, 1,000,003 87.9 / 87.9); few
+// keys take small tiles, since a tile's time is a chain and 4,096 keys a tile leave most of the card idle (tiles of 4,096 and a
+// launch for the scan / smaller tiles and own scans, both with 256 threads a tile: 9,000 rows 76 / 58, 100,003 74 / 66).  More keys
+// keep the launch and the large tiles: 2,048 a tile 0.301 against 0.293 ms for a refresh of 2.4 M rows.
 struct SortShape {
     int items, tiles;
     bool own_scan;
 };
 
 constexpr int kOwnScanTiles = 128;
+constexpr int kSortThreads = 1024;  // a tile's, in the scatter and the histograms: one key each in the smallest
 
 SortShape sort_shape(int64_t N) {
     const int64_t n = N < 1 ? 1 : N;
-    for (int items = 4; items <= 16; items *= 2)
-        if (ceil_div(n, (int64_t)items * kBlock) <= kOwnScanTiles) return {items, (int)ceil_div(n, (int64_t)items * kBlock), true};
-    return {16, (int)ceil_div(n, (int64_t)16 * kBlock), false};
+    for (int items = 1; items <= 4; items *= 2)
+        if (ceil_div(n, (int64_t)items * kSortThreads) <= kOwnScanTiles) return {items, (int)ceil_div(n, (int64_t)items * kSortThreads), true};
+    const int64_t large = ceil_div(n, (int64_t)4 * kSortThreads);
+    return {4, (int)large, large <= 2 * kOwnScanTiles};
 }
 
 __device__ __forceinline__ int digit_of(int32_t key, int shift) { return (key >> shift) & (kDigits - 1); }
 
 // The number of keys of the tile with digit d: hist[d * tiles + tile], digit-major, since the scan over a
 // digit's tiles is a scan over consecutive entries; hist[tile * kDigits + d] where the scatter adds them up itself, a thread
-// per digit (ITEMS: keys per thread of a workgroup of kBlock; own_scan: as in SortShape).  THREADS: the workgroup's size, a multiple
-// of kBlock.
-template <int THREADS, int ITEMS>
+// per digit (ITEMS: keys per thread of a workgroup of kSortThreads; own_scan: as in SortShape).
+template <int ITEMS>
 __device__ __forceinline__ void tile_histogram(const int32_t *__restrict__ keys, int64_t N, int shift,
                                                int32_t *__restrict__ hist, int tiles, bool own_scan, int tile, int *count) {
-    constexpr int kTile = ITEMS * kBlock, kItems = (kTile + THREADS - 1) / THREADS;
+    constexpr int kTile = ITEMS * kSortThreads;
     if (threadIdx.x < kDigits) count[threadIdx.x] = 0;
     __syncthreads();
     const int64_t base = (int64_t)tile * kTile;
-    int32_t key[kItems];
+    int32_t key[ITEMS];
 #pragma unroll
-    for (int it = 0; it < kItems; ++it) {
-        const int64_t i = base + (int64_t)it * THREADS + threadIdx.x;
+    for (int it = 0; it < ITEMS; ++it) {
+        const int64_t i = base + (int64_t)it * kSortThreads + threadIdx.x;
         key[it] = i < N ? keys[i] : 0;
     }
 #pragma unroll
-    for (int it = 0; it < kItems; ++it) {
-        const int64_t i = base + (int64_t)it * THREADS + threadIdx.x;
+    for (int it = 0; it < ITEMS; ++it) {
+        const int64_t i = base + (int64_t)it * kSortThreads + threadIdx.x;
         if (i < N) atomicAdd(&count[digit_of(key[it], shift)], 1);  // LDS, integer: the sum does not depend on the order
     }
     __syncthreads();
@@ -82,15 +82,15 @@ __device__ __forceinline__ void tile_histogram(const int32_t *__restrict__ keys,
 constexpr int kGroupState = 4;
 
 template <int ITEMS>
-__global__ __launch_bounds__(kBlock) void radix_hist_kernel(const int32_t *__restrict__ keys, int64_t N, int shift,
+__global__ __launch_bounds__(kSortThreads) void radix_hist_kernel(const int32_t *__restrict__ keys, int64_t N, int shift,
                                                            int32_t *__restrict__ hist, int tiles, bool own_scan,
                                                            int32_t *__restrict__ clear, int clear_n, int32_t *__restrict__ state) {
     __shared__ int count[kDigits];
     if (clear)
-        for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < clear_n; i += (int64_t)gridDim.x * kBlock)
+        for (int64_t i = (int64_t)blockIdx.x * kSortThreads + threadIdx.x; i < clear_n; i += (int64_t)gridDim.x * kSortThreads)
             clear[i] = 0;
     if (state && blockIdx.x == 0 && threadIdx.x < kGroupState) state[threadIdx.x] = 0;
-    tile_histogram<kBlock, ITEMS>(keys, N, shift, hist, tiles, own_scan, blockIdx.x, count);
+    tile_histogram<ITEMS>(keys, N, shift, hist, tiles, own_scan, blockIdx.x, count);
 }
 
 // One wave per digit: within[d * tiles + t] = keys with digit d in the tiles before t, and
@@ -103,17 +103,23 @@ __global__ __launch_bounds__(kBlock) void radix_scan_kernel(const int32_t *__res
     const int32_t *row = hist + (int64_t)d * tiles;
     int32_t *out = within + (int64_t)d * tiles;
     int running = 0;
-    for (int t0 = 0; t0 < tiles; t0 += kWave) {
-        const int t = t0 + lane;
-        const int v = t < tiles ? row[t] : 0;
-        int inc = v;
+    constexpr int kAhead = 10;  // 640 tiles, 2.6 M keys, in one round of loads (2,449,029 keys, us: one by one 7.3, 5.1 so)
+    for (int t0 = 0; t0 < tiles; t0 += kAhead * kWave) {
+        int v[kAhead];
 #pragma unroll
-        for (int s = 1; s < kWave; s <<= 1) {
-            const int n = __shfl_up(inc, s, kWave);
-            if (lane >= s) inc += n;
+        for (int u = 0; u < kAhead; ++u) v[u] = t0 + u * kWave + lane < tiles ? row[t0 + u * kWave + lane] : 0;
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const int t = t0 + u * kWave + lane;
+            int inc = v[u];
+#pragma unroll
+            for (int s = 1; s < kWave; s <<= 1) {
+                const int n = __shfl_up(inc, s, kWave);
+                if (lane >= s) inc += n;
+            }
+            if (t < tiles) out[t] = running + inc - v[u];
+            running += __shfl(inc, kWave - 1, kWave);
         }
-        if (t < tiles) out[t] = running + inc - v;
-        running += __shfl(inc, kWave - 1, kWave);
     }
     if (lane == 0) total[d] = running;
 }
@@ -140,8 +146,14 @@ __device__ __forceinline__ unsigned long long same_digit(int d, unsigned long lo
 // beyond the table, a caller's mistake, inside it).  `remap` (optional, last pass): the keys are
 // written as remap[key & seen_mask], an order-preserving renaming (the rank of the code).
 // OWN_SCAN: `within` holds the tiles' histograms (tile_histogram), `total` is not read.
+//
+// A tile is dealt to kSortThreads threads, ITEMS keys each: its time is a chain -- loads, a step of ballots and one look at LDS
+// per 64 keys of a wave, three barriers, stores -- and all tiles of a launch are resident at once, so the launch takes as long as
+// one of them.  With 256 threads a wave ranked 1,024 keys in sixteen steps (us a pass, so / with 1,024 threads: 2,449,029 keys
+// 22.6 / 20.7, 1,000,003 15.1 / 13.0; hashing and grouping rows of 24 columns by 16 planes: 100,003 rows 58.6 / 54.0, 262,145
+// 73.9 / 64.4, 450,000 80.2 / 69.8).
 template <int ITEMS, bool OWN_SCAN>
-__global__ __launch_bounds__(kBlock) void radix_scatter_kernel(const int32_t *__restrict__ keys,
+__global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(const int32_t *__restrict__ keys,
                                                               const int32_t *__restrict__ vals, int64_t N, int shift,
                                                               const int32_t *__restrict__ within,
                                                               const int32_t *__restrict__ total, int tiles,
@@ -149,21 +161,25 @@ __global__ __launch_bounds__(kBlock) void radix_scatter_kernel(const int32_t *__
                                                               int32_t *__restrict__ vals_out,
                                                               int32_t *__restrict__ seen, int seen_mask,
                                                               const int32_t *__restrict__ remap) {
-    constexpr int kWaves = kBlock / kWave;
-    constexpr int kTile = ITEMS * kBlock, kPerWave = kTile / kWaves;
+    constexpr int kWaves = kSortThreads / kWave, kDigitWaves = kDigits / kWave;
+    constexpr int kTile = ITEMS * kSortThreads, kPerWave = kTile / kWaves;
     __shared__ int digit_start[kDigits];         // output position of the tile's first key of a digit, minus tile_start
     __shared__ int tile_start[kDigits];          // position of that key in the ordered tile
     __shared__ int wave_count[kWaves][kDigits];  // keys of a digit seen by a wave so far; then: by the waves before it
-    __shared__ int scan_tmp[2][kWaves];
+    __shared__ int scan_tmp[2][kDigitWaves];
     __shared__ int32_t tile_key[kTile], tile_val[kTile];
+    __shared__ int share_sums[OWN_SCAN ? 2 : 1][OWN_SCAN ? kSortThreads : 1];
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-    int mine = 0, my_within = 0;  // thread = digit
+    int mine = 0, my_within = 0;  // thread = digit (the first kDigits threads)
+    const bool of_digit = threadIdx.x < kDigits;
     if constexpr (!OWN_SCAN) {
-        mine = total[threadIdx.x];
-        my_within = within[(int64_t)threadIdx.x * tiles + blockIdx.x];
+        if (of_digit) {
+            mine = total[threadIdx.x];
+            my_within = within[(int64_t)threadIdx.x * tiles + blockIdx.x];
+        }
     }
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) wave_count[w][threadIdx.x] = 0;
+    for (int k = threadIdx.x; k < kWaves * kDigits; k += kSortThreads) (&wave_count[0][0])[k] = 0;
     __syncthreads();
     const int64_t base = (int64_t)blockIdx.x * kTile + (int64_t)wave * kPerWave;
     int32_t key[ITEMS], val[ITEMS];
@@ -177,18 +193,21 @@ __global__ __launch_bounds__(kBlock) void radix_scatter_kernel(const int32_t *__
         val[it] = live ? (vals ? vals[i] : (int32_t)i) : 0;
     }
     if constexpr (OWN_SCAN) {
-        constexpr int kBatch = 32;
+        // a thread adds up a digit over a share of the tiles, the shares meet below
+        constexpr int kShares = kSortThreads / kDigits, kBatch = kOwnScanTiles / kShares;
+        const int share = threadIdx.x / kDigits, d = threadIdx.x % kDigits;
 #pragma unroll 1
-        for (int t0 = 0; t0 < tiles; t0 += kBatch) {
+        for (int t0 = share * kBatch; t0 < tiles; t0 += kOwnScanTiles) {
             int v[kBatch];
 #pragma unroll
-            for (int u = 0; u < kBatch; ++u) v[u] = within[min(t0 + u, tiles - 1) * kDigits + threadIdx.x];
+            for (int u = 0; u < kBatch; ++u) v[u] = within[min(t0 + u, tiles - 1) * kDigits + d];
 #pragma unroll
             for (int u = 0; u < kBatch; ++u) {
                 mine += t0 + u < tiles ? v[u] : 0;
                 my_within += t0 + u < (int)blockIdx.x ? v[u] : 0;
             }
         }
+        share_sums[0][threadIdx.x] = mine, share_sums[1][threadIdx.x] = my_within;
     }
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
@@ -209,38 +228,50 @@ __global__ __launch_bounds__(kBlock) void radix_scatter_kernel(const int32_t *__
     __syncthreads();
     {   // per digit (thread = digit): what the waves before a wave hold, and the tile's count
         int running = 0;
+        if (of_digit) {
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) {
-            const int c = wave_count[w][threadIdx.x];
-            wave_count[w][threadIdx.x] = running;
-            running += c;
+            for (int w = 0; w < kWaves; ++w) {
+                const int c = wave_count[w][threadIdx.x];
+                wave_count[w][threadIdx.x] = running;
+                running += c;
+            }
+            if constexpr (OWN_SCAN)
+#pragma unroll
+                for (int k = 1; k < kSortThreads / kDigits; ++k) {
+                    mine += share_sums[0][k * kDigits + threadIdx.x];
+                    my_within += share_sums[1][k * kDigits + threadIdx.x];
+                }
         }
         // exclusive scans over the digits: of the tile's counts (places in the ordered tile) and of
         // the totals (places in the output)
         int inc_tile = running, inc_all = mine;
+        if (of_digit) {
 #pragma unroll
-        for (int s = 1; s < kWave; s <<= 1) {
-            const int a = __shfl_up(inc_tile, s, kWave), b = __shfl_up(inc_all, s, kWave);
-            if (lane >= s) {
-                inc_tile += a;
-                inc_all += b;
+            for (int s = 1; s < kWave; s <<= 1) {
+                const int a = __shfl_up(inc_tile, s, kWave), b = __shfl_up(inc_all, s, kWave);
+                if (lane >= s) {
+                    inc_tile += a;
+                    inc_all += b;
+                }
             }
-        }
-        if (lane == kWave - 1) {
-            scan_tmp[0][wave] = inc_tile;
-            scan_tmp[1][wave] = inc_all;
+            if (lane == kWave - 1) {
+                scan_tmp[0][wave] = inc_tile;
+                scan_tmp[1][wave] = inc_all;
+            }
         }
         __syncthreads();
-        int before_tile = 0, before_all = 0;
+        if (of_digit) {
+            int before_tile = 0, before_all = 0;
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w)
-            if (w < wave) {
-                before_tile += scan_tmp[0][w];
-                before_all += scan_tmp[1][w];
-            }
-        const int in_tile = before_tile + inc_tile - running;
-        tile_start[threadIdx.x] = in_tile;
-        digit_start[threadIdx.x] = before_all + inc_all - mine + my_within - in_tile;
+            for (int w = 0; w < kDigitWaves; ++w)
+                if (w < wave) {
+                    before_tile += scan_tmp[0][w];
+                    before_all += scan_tmp[1][w];
+                }
+            const int in_tile = before_tile + inc_tile - running;
+            tile_start[threadIdx.x] = in_tile;
+            digit_start[threadIdx.x] = before_all + inc_all - mine + my_within - in_tile;
+        }
     }
     __syncthreads();
 #pragma unroll
@@ -258,7 +289,7 @@ __global__ __launch_bounds__(kBlock) void radix_scatter_kernel(const int32_t *__
     const int in_this_tile = left < kTile ? (int)left : kTile;
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
-        const int at = it * kBlock + threadIdx.x;
+        const int at = it * kSortThreads + threadIdx.x;
         if (at < in_this_tile) {
             const int32_t k = tile_key[at];
             const int64_t pos = (int64_t)digit_start[digit_of(k, shift)] + at;
@@ -272,7 +303,7 @@ int radix_passes(int bits) { return bits <= kDigitBits ? 1 : (bits + kDigitBits 
 
 // hist, within (kDigits x tiles each) and total (kDigits); never less than fewer keys take, which may be dealt in more tiles
 size_t radix_counter_bytes(int64_t N) {
-    const int64_t small_tiles = std::min<int64_t>(ceil_div(N, (int64_t)4 * kBlock), kOwnScanTiles);
+    const int64_t small_tiles = std::min<int64_t>(ceil_div(N, (int64_t)kSortThreads), kOwnScanTiles);
     const int64_t tiles = std::max<int64_t>(sort_shape(N).tiles, small_tiles);
     return 2 * align_up((size_t)kDigits * (size_t)tiles * sizeof(int32_t), 256) + align_up(kDigits * sizeof(int32_t), 256);
 }
@@ -342,7 +373,7 @@ __global__ void group_finish_kernel(int64_t N, const int32_t *__restrict__ rank,
 // thread, and counts for itself the codes that occur before its stretch (the table is 256 KB
 // at most, so reading it again costs less than a second launch would); all loads of a thread
 // are in flight together.
-constexpr int kRankThreads = 1024;
+constexpr int kRankThreads = kSortThreads;  // the ranks ride in a launch of histograms
 constexpr int kRankStretch = 4 * kRankThreads;
 constexpr int kTableBits = 16;  // up to this many hyperplanes the ranks come from a table over all codes
 constexpr int kRankStretches = (1 << kTableBits) / kRankStretch;
@@ -434,7 +465,7 @@ __global__ __launch_bounds__(kRankThreads) void radix_hist_rank_kernel(const int
     if ((int)blockIdx.x < parts)  // first, so that they are not the tail of the launch
         code_rank_stretch(table, codes, summary, blockIdx.x, parts, wave_before, wave_mine);
     else
-        tile_histogram<kRankThreads, ITEMS>(keys, N, shift, hist, tiles, own_scan, (int)blockIdx.x - parts, count);
+        tile_histogram<ITEMS>(keys, N, shift, hist, tiles, own_scan, (int)blockIdx.x - parts, count);
 }
 
 // Stable sort of (keys[i], i) by the low `bits` bits of the keys into (keys_out, vals_out).
@@ -469,12 +500,12 @@ int radix_sort_tiles(const int32_t *keys, int64_t N, int bits, int32_t *keys_out
             hipLaunchKernelGGL(radix_hist_rank_kernel<ITEMS>, dim3((unsigned)(tiles + rank_parts)), dim3(kRankThreads), 0,
                                stream, in_keys, N, shift, hist, tiles, OWN_SCAN, table, seen_mask + 1, summary);
         else
-            hipLaunchKernelGGL(radix_hist_kernel<ITEMS>, dim3((unsigned)tiles), dim3(kBlock), 0, stream, in_keys, N, shift,
+            hipLaunchKernelGGL(radix_hist_kernel<ITEMS>, dim3((unsigned)tiles), dim3(kSortThreads), 0, stream, in_keys, N, shift,
                                hist, tiles, OWN_SCAN, first ? table : nullptr, seen_mask + 1, first ? state : nullptr);
         if (!OWN_SCAN)
             hipLaunchKernelGGL(radix_scan_kernel, dim3(kDigits / (kBlock / kWave)), dim3(kBlock), 0, stream, hist, tiles,
                                within, total);
-        hipLaunchKernelGGL((radix_scatter_kernel<ITEMS, OWN_SCAN>), dim3((unsigned)tiles), dim3(kBlock), 0, stream, in_keys, in_vals,
+        hipLaunchKernelGGL((radix_scatter_kernel<ITEMS, OWN_SCAN>), dim3((unsigned)tiles), dim3(kSortThreads), 0, stream, in_keys, in_vals,
                            N, shift, within, total, tiles, out_keys, out_vals, first ? table : nullptr, seen_mask, remap);
         if (table && first && last)  // with a second pass its histogram launch makes the ranks
             hipLaunchKernelGGL(code_rank_kernel, dim3((unsigned)rank_parts), dim3(kRankThreads), 0, stream, table,
@@ -492,9 +523,9 @@ int radix_sort_by_key(const int32_t *keys, int64_t N, int bits, int32_t *keys_ou
     if (ranked) *ranked = false;
     if (N <= 0) return CGNN_OK;
     const SortShape s = sort_shape(N);
-    const auto sort = !s.own_scan ? radix_sort_tiles<16, false>
-                                  : (s.items == 4 ? radix_sort_tiles<4, true>
-                                                  : (s.items == 8 ? radix_sort_tiles<8, true> : radix_sort_tiles<16, true>));
+    const auto sort = !s.own_scan ? radix_sort_tiles<4, false>
+                                  : (s.items == 1 ? radix_sort_tiles<1, true>
+                                                  : (s.items == 2 ? radix_sort_tiles<2, true> : radix_sort_tiles<4, true>));
     return sort(keys, N, bits, keys_out, vals_out, tmp_keys, tmp_vals, counters, table, seen_mask, summary, ranked, state, s.tiles,
                 stream);
 }

@@ -264,6 +264,12 @@ def test_grouped_assign_of_any_length(n, bits):
         assert np.array_equal(offsets, np.concatenate([[0], np.cumsum(counts)]))
 
 
+@pytest.mark.parametrize("n,bits", [(1048576, 16), (1048577, 16), (1048577, 8)])
+def test_grouped_assign_where_the_scan_becomes_a_launch(n, bits):
+    """256 tiles of 4,096 keys, whose histograms the scatter adds up itself, and one more."""
+    test_grouped_assign_of_any_length(n, bits)
+
+
 @pytest.mark.parametrize("n, width", [(300, 47), (2049, 64), (30011, 256), (131072, 64), (131073, 64), (262145, 128), (524288, 64), (524289, 64),
                                       (524289, 16), (786432, 64), (786433, 64), (1835009, 16)])
 def test_means_and_sums_with_any_number_of_workgroups(n, width):
