@@ -53,7 +53,8 @@ constexpr int kScanBlock = 1024;
 // alone take 40 us, and at 16,384 the comparisons do, too.
 constexpr int32_t kRankAll = 16384;
 
-enum Scalar { kBad, kListed, kCandidates, kAdded, kTakenTotal, kScalars = 8 };
+enum Scalar { kBad, kListed, kCandidates, kAdded, kTakenTotal, kArrived, kScalars = 8 };  // kArrived: three counters (Arrival)
+enum Arrival { kPassed, kCounted, kTaken };
 
 struct Merger {
     int64_t V;
@@ -81,6 +82,7 @@ struct Merger {
     int32_t *word_sum;                 // [L / 64] taken positions of the tile in front of a word
     int32_t *children;
     int32_t *scalar;                   // [kScalars]
+    int32_t *host, flag;               // pinned memory for the scalars and this flag behind them, or NULL
 };
 
 unsigned merger_grid(int64_t n) {
@@ -133,6 +135,78 @@ __device__ __forceinline__ int block_scan(int v, int *total) {
     return before;
 }
 
+// Sums of the tiles in front of every tile; returns the total.  FRESH: written by other workgroups of this launch.
+template <int BLOCK, bool FRESH>
+__device__ __forceinline__ int scan_tiles(int32_t *__restrict__ tile, int32_t tiles) {
+    int running = 0;
+    for (int32_t k0 = 0; k0 < tiles; k0 += BLOCK * kItems) {
+        const int32_t k = k0 + threadIdx.x * kItems;
+        int v[kItems], sum = 0, all;
+#pragma unroll
+        for (int u = 0; u < kItems; ++u) v[u] = k + u < tiles ? (FRESH ? load_now(tile + k + u) : tile[k + u]) : 0;
+#pragma unroll
+        for (int u = 0; u < kItems; ++u) sum += v[u];
+        int before = running + block_scan<BLOCK>(sum, &all);
+#pragma unroll
+        for (int u = 0; u < kItems; ++u) {
+            if (k + u < tiles) tile[k + u] = before;
+            before += v[u];
+        }
+        running += all;
+    }
+    return running;
+}
+
+__global__ __launch_bounds__(kScanBlock) void merger_tile_sums_kernel(int32_t *__restrict__ tile, int32_t tiles,
+                                                                      int32_t *__restrict__ total) {
+    const int all = scan_tiles<kScanBlock, false>(tile, tiles);
+    if (threadIdx.x == 0) *total = all;
+}
+
+// What the last workgroup to get here may do for the others instead of a launch behind them (3 to 5 us of the device and as
+// much of the host; 14,530 vertices of degree 8.9 at a frequency of 4, twenty launches a round 636 us a call, sixteen 583; 14,163
+// of 13 at 16 480, 456): true in that one, for all its threads.  What the others have left is past their L2s -- stored with
+// store_now or added with an atomic -- and read with load_now: a release would write back the whole L2.  The arrivals come one
+// after the other, some 12 ns each, so this is for launches of up to kFew workgroups (1,600: 32 us instead of 12).
+constexpr unsigned kFew = 256;
+__device__ __forceinline__ void store_now(int32_t *p, int32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+__device__ __forceinline__ bool arrives_last(const Merger &m, Arrival at) {
+    __shared__ bool last;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0);  // of every wave: its stores have arrived
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int32_t before = __hip_atomic_fetch_add(m.scalar + kArrived + at, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last = before == (int32_t)gridDim.x - 1;
+    }
+    __syncthreads();
+    return last;
+}
+
+// The scalars for the host (one thread), the flag last, when the others have arrived.
+__device__ __forceinline__ void publish(const int32_t *scalar, int32_t *host, int32_t flag) {
+    int32_t v[kScalars];
+#pragma unroll
+    for (int i = 0; i < kScalars; ++i) v[i] = load_now(scalar + i);
+#pragma unroll
+    for (int i = 0; i < kScalars; ++i) __hip_atomic_store(host + i, v[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0);
+    __hip_atomic_store(host + kScalars, flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Tables of up to this many slots (12 MB) are cleared for as many pairs as there can be, in a launch that there is anyway; larger
+// ones for as many as are listed, one in seven of a first round.
+constexpr int64_t kClearedAhead = (int64_t)1 << 20;
+
+__device__ __forceinline__ void clear_table(const Merger &m, int64_t slots) {
+    CGNN_GRID_LOOP(i, slots / 2) {
+        reinterpret_cast<ulonglong2 *>(m.table_key)[i] = make_ulonglong2(kEmpty, kEmpty);
+        reinterpret_cast<int2 *>(m.table_count)[i] = make_int2(0, 0);
+    }
+}
+
 // Row starts, where rows end (bits of `taken`, which the first round has no other use for yet) and the counters.
 template <typename In>
 __global__ void merger_rows_kernel(Merger m, const In *__restrict__ vlist, int64_t E) {
@@ -153,6 +227,7 @@ __global__ void merger_begin_kernel(Merger m) {
     if (m.first) CGNN_GRID_LOOP(i, words) m.taken[i] = 0;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         m.scalar[kCandidates] = 0;
+        for (int i = 0; i < 3; ++i) m.scalar[kArrived + i] = 0;
         if (m.first) m.scalar[kBad] = 0;
     }
 }
@@ -220,7 +295,9 @@ __global__ __launch_bounds__(kBlock) void merger_count_kernel(Merger m) {
         if (key[u] != kEmpty) count_pair(m, counter[u], seen[u]);
 }
 
-__global__ __launch_bounds__(kBlock) void merger_pass_kernel(Merger m) {
+// The positions that pass, their number in front of every tile, and (`clear`) an empty table: the counters by hash, in whose
+// memory it lies, have been read.
+__global__ __launch_bounds__(kBlock) void merger_pass_kernel(Merger m, bool clear) {
     __shared__ int passed[kBlock / kWave];
     const int shift = 63 - table_bits(m.most);
     const int64_t e0 = (int64_t)blockIdx.x * kTile + threadIdx.x;
@@ -246,39 +323,15 @@ __global__ __launch_bounds__(kBlock) void merger_pass_kernel(Merger m) {
     if (threadIdx.x == 0) {
         int all = 0;
         for (int w = 0; w < kBlock / kWave; ++w) all += passed[w];
-        m.tile[blockIdx.x] = all;
+        store_now(m.tile + blockIdx.x, all);
     }
+    if (clear) clear_table(m, (int64_t)1 << table_bits(m.most));
+    if (gridDim.x > kFew || !arrives_last(m, kPassed)) return;
+    const int all = scan_tiles<kBlock, true>(m.tile, (int32_t)gridDim.x);
+    if (threadIdx.x == 0) m.scalar[kListed] = all;
 }
 
-// Sums of the tiles in front of every tile, and the total.
-__global__ __launch_bounds__(kScanBlock) void merger_tile_sums_kernel(int32_t *__restrict__ tile, int32_t tiles,
-                                                                      int32_t *__restrict__ total) {
-    int running = 0;
-    for (int32_t k0 = 0; k0 < tiles; k0 += kScanBlock * kItems) {
-        const int32_t k = k0 + threadIdx.x * kItems;
-        int v[kItems], sum = 0, all;
-#pragma unroll
-        for (int u = 0; u < kItems; ++u) v[u] = k + u < tiles ? tile[k + u] : 0;
-#pragma unroll
-        for (int u = 0; u < kItems; ++u) sum += v[u];
-        int before = running + block_scan<kScanBlock>(sum, &all);
-#pragma unroll
-        for (int u = 0; u < kItems; ++u) {
-            if (k + u < tiles) tile[k + u] = before;
-            before += v[u];
-        }
-        running += all;
-    }
-    if (threadIdx.x == 0) *total = running;
-}
-
-__global__ void merger_clear_table_kernel(Merger m) {
-    const int64_t slots = (int64_t)1 << table_bits(m.scalar[kListed]);
-    CGNN_GRID_LOOP(i, slots / 2) {
-        reinterpret_cast<ulonglong2 *>(m.table_key)[i] = make_ulonglong2(kEmpty, kEmpty);
-        reinterpret_cast<int2 *>(m.table_count)[i] = make_int2(0, 0);
-    }
-}
+__global__ void merger_clear_table_kernel(Merger m) { clear_table(m, (int64_t)1 << table_bits(m.scalar[kListed])); }
 
 // The list of positions, and how often their pairs occur.  Tables have more slots than pairs, so every probe ends.
 __global__ __launch_bounds__(kBlock) void merger_collect_kernel(Merger m) {
@@ -348,6 +401,7 @@ __global__ __launch_bounds__(kBlock) void merger_candidates_kernel(Merger m) {
         }
         __syncthreads();
     }
+    if (m.host != nullptr && gridDim.x <= kFew && arrives_last(m, kCounted) && threadIdx.x == 0) publish(m.scalar, m.host, m.flag);
 }
 
 // Ranks of a few candidates: a workgroup compares kBlock of them with kBlock others.
@@ -527,7 +581,8 @@ __global__ __launch_bounds__(BLOCK) void merger_rules_kernel(Merger m) {
     if (ALONE && threadIdx.x == 0) m.scalar[kAdded] = all;
 }
 
-// Taken positions of the tile in front of every word of the map, and of every tile.
+// Taken positions of the tile in front of every word of the map, those in front of every tile, and all of them: with it the
+// host knows the new length, while the entries still move.
 __global__ __launch_bounds__(kBlock) void merger_taken_sums_kernel(Merger m, int64_t words) {
     const int64_t w = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     const int count = w < words ? __popcll(m.taken[w]) : 0, lane = threadIdx.x % kTileWords;
@@ -537,9 +592,17 @@ __global__ __launch_bounds__(kBlock) void merger_taken_sums_kernel(Merger m, int
         const int up = __shfl_up(sum, s, kTileWords);
         if (lane >= s) sum += up;
     }
-    if (w >= words) return;
-    m.word_sum[w] = sum - count;
-    if (lane == kTileWords - 1) m.tile[w / kTileWords] = sum;
+    if (w < words) {
+        m.word_sum[w] = sum - count;
+        if (lane == kTileWords - 1) store_now(m.tile + w / kTileWords, sum);
+    }
+    if (gridDim.x > kFew || !arrives_last(m, kTaken)) return;
+    const int all = scan_tiles<kBlock, true>(m.tile, (int32_t)(words / kTileWords));
+    if (threadIdx.x == 0) {
+        store_now(m.scalar + kTakenTotal, all);
+        __builtin_amdgcn_s_waitcnt(0);
+        if (m.host != nullptr) publish(m.scalar, m.host, m.flag);
+    }
 }
 
 // Where position e goes: to the left by the taken ones in front of it.
@@ -591,11 +654,7 @@ __global__ __launch_bounds__(kBlock) void merger_move_kernel(Merger m) {
     }
 }
 
-// The scalars for the host, the flag last.
-__global__ void merger_publish_kernel(const int32_t *__restrict__ scalar, int32_t *__restrict__ host, int32_t flag) {
-    for (int i = 0; i < kScalars; ++i) host[i] = scalar[i];
-    __hip_atomic_store(host + kScalars, flag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
+__global__ void merger_publish_kernel(const int32_t *scalar, int32_t *host, int32_t flag) { publish(scalar, host, flag); }
 
 // out_ptr = [row starts | starts of the rule rows], out_col = [rows | children of the rules].
 __global__ void merger_finish_kernel(const int32_t *__restrict__ ptr, const uint32_t *__restrict__ seq,
@@ -747,14 +806,14 @@ int merger_rounds(int64_t V, int64_t E, int rounds, int min_pair_frequency, int3
     const dim3 block(kBlock);
     int32_t reads = 0, host[kScalars + 1];
     if (pinned != nullptr) pinned[kScalars] = 0;
-    // What the host needs is written to memory that it looks at for a while, which costs it a few us; a copy and
-    // a wait cost it 40.
+    m.host = pinned;
+    // What the host needs is written, by the launch that has it last, to memory that it looks at for a while, which costs it a
+    // few us; a copy and a wait cost it 40.  The launch is given the number of the read as its flag (m.flag).
     auto read = [&]() -> hipError_t {
         if (pinned == nullptr) {
             hipError_t e = hipMemcpyAsync(host, m.scalar, kScalars * sizeof(int32_t), hipMemcpyDeviceToHost, stream);
             return e == hipSuccess ? hipStreamSynchronize(stream) : e;
         }
-        hipLaunchKernelGGL(merger_publish_kernel, dim3(1), dim3(1), 0, stream, m.scalar, pinned, ++reads);
         const auto patience = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
         while (__atomic_load_n(pinned + kScalars, __ATOMIC_ACQUIRE) != reads)
             if (std::chrono::steady_clock::now() > patience) {
@@ -765,6 +824,9 @@ int merger_rounds(int64_t V, int64_t E, int rounds, int min_pair_frequency, int3
             }
         for (int i = 0; i < kScalars; ++i) host[i] = pinned[i];
         return hipSuccess;
+    };
+    auto publish_now = [&] {
+        if (pinned != nullptr) hipLaunchKernelGGL(merger_publish_kernel, dim3(1), dim3(1), 0, stream, m.scalar, pinned, m.flag);
     };
     const int32_t all_tiles = (int32_t)tiles_of(E > V ? E : V + 1);
     hipError_t err = hipSuccess;
@@ -779,11 +841,17 @@ int merger_rounds(int64_t V, int64_t E, int rounds, int min_pair_frequency, int3
             launch_begin(m, stream);
             hipLaunchKernelGGL(merger_count_kernel, grid, block, 0, stream, m);
         }
-        hipLaunchKernelGGL(merger_pass_kernel, grid, block, 0, stream, m);
-        hipLaunchKernelGGL(merger_tile_sums_kernel, dim3(1), dim3(kScanBlock), 0, stream, m.tile, tiles, m.scalar + kListed);
-        hipLaunchKernelGGL(merger_clear_table_kernel, dim3(merger_grid(((int64_t)1 << bits_of(m.most)) / 2)), block, 0, stream, m);
+        const int64_t slots = (int64_t)1 << bits_of(m.most);
+        const bool clear_here = slots <= kClearedAhead;
+        hipLaunchKernelGGL(merger_pass_kernel, grid, block, 0, stream, m, clear_here);
+        if (grid.x > kFew)
+            hipLaunchKernelGGL(merger_tile_sums_kernel, dim3(1), dim3(kScanBlock), 0, stream, m.tile, tiles, m.scalar + kListed);
+        if (!clear_here) hipLaunchKernelGGL(merger_clear_table_kernel, dim3(merger_grid(slots / 2)), block, 0, stream, m);
         hipLaunchKernelGGL(merger_collect_kernel, grid, block, 0, stream, m);
-        hipLaunchKernelGGL(merger_candidates_kernel, dim3(tiles_of((int64_t)1 << bits_of(m.most))), block, 0, stream, m);
+        m.flag = ++reads;
+        const dim3 table(tiles_of(slots));
+        hipLaunchKernelGGL(merger_candidates_kernel, table, block, 0, stream, m);
+        if (table.x > kFew) publish_now();
         if ((err = read()) != hipSuccess) return merger_fail(err, "reading the candidate count");
         if (!checked && host[kBad])
             return fail(CGNN_EINVAL, "cgnn_compress_csr_batch_device: malformed CSR (row starts or columns out of range)");
@@ -816,13 +884,21 @@ int merger_rounds(int64_t V, int64_t E, int rounds, int min_pair_frequency, int3
         }
         hipLaunchKernelGGL(merger_match_kernel<true>, list, block, 0, stream, m);
         hipLaunchKernelGGL(merger_take_kernel<true>, list, block, 0, stream, m);
-        hipLaunchKernelGGL(merger_taken_sums_kernel, dim3(merger_grid(words)), block, 0, stream, m, words);
-        hipLaunchKernelGGL(merger_tile_sums_kernel, dim3(1), dim3(kScanBlock), 0, stream, m.tile, tiles, m.scalar + kTakenTotal);
+        m.flag = ++reads;
+        const dim3 maps((unsigned)ceil_div(words, kBlock));
+        hipLaunchKernelGGL(merger_taken_sums_kernel, maps, block, 0, stream, m, words);
+        if (maps.x > kFew) {
+            hipLaunchKernelGGL(merger_tile_sums_kernel, dim3(1), dim3(kScanBlock), 0, stream, m.tile, tiles, m.scalar + kTakenTotal);
+            publish_now();
+        }
         hipLaunchKernelGGL(merger_move_kernel, dim3((unsigned)all_tiles), block, 0, stream, m);
         if ((err = read()) != hipSuccess) return merger_fail(err, "reading the new length");
         const int32_t added = host[kAdded];
         if (added == 0) break;  // and nothing was taken
-        if (V + R + added >= kMergerLimit) return fail(CGNN_EUNSUPPORTED, "cgnn_compress_csr_batch_device: node ids exceed int32");
+        if (V + R + added >= kMergerLimit) {
+            hipStreamSynchronize(stream);  // the entries still move
+            return fail(CGNN_EUNSUPPORTED, "cgnn_compress_csr_batch_device: node ids exceed int32");
+        }
         std::swap(m.seq, m.next_seq);
         std::swap(m.ptr, m.next_ptr);
         std::swap(m.active, m.next_active);
@@ -834,6 +910,8 @@ int merger_rounds(int64_t V, int64_t E, int rounds, int min_pair_frequency, int3
         R += added;
     }
     if (!checked) {
+        m.flag = ++reads;
+        publish_now();
         if ((err = read()) != hipSuccess) return merger_fail(err, "reading the input check");
         if (host[kBad])
             return fail(CGNN_EINVAL, "cgnn_compress_csr_batch_device: malformed CSR (row starts or columns out of range)");

@@ -146,6 +146,12 @@ def test_gpu_compressor_at_the_edges_of_its_tiles(entries, freq):
     assert all(np.array_equal(a, b) for a, b in zip(got, both(v.astype(np.int32), e.astype(np.int32), 12, freq)))
 
 
+@pytest.mark.parametrize("entries, freq", [((1 << 20) - 1, 16), (1 << 20, 16), (1 << 22, 64), ((1 << 22) + 1, 64)])
+def test_gpu_compressor_where_launches_grow_too_large_for_their_last_workgroup(entries, freq):
+    """Around the lengths from which tables are cleared by a launch of their own, and sums over the tiles are one."""
+    test_gpu_compressor_at_the_edges_of_its_tiles(entries, freq)
+
+
 @pytest.mark.parametrize("entries", [(1 << 14) - 1, (1 << 14) + 1, (1 << 20) + (1 << 14), (9 << 19) + 3])
 def test_gpu_compressor_from_several_threads(entries):
     """The host's passes are dealt out in blocks, to as many helpers as there are or to none: alone, with one thread
