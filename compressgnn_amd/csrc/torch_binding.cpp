@@ -1398,10 +1398,10 @@ Tensor cluster_reconstruct_backward(Tensor grad, Tensor index, Tensor output, in
 
 // The ReLU form of cluster_reconstruct that also returns the sign of every output element as one
 // bit: (rows [N, F], signs int32 [N, ceil(F / 32)]), or, by group, masks int32 [groups, ceil(F / 32)]: the rows
-// of a group are copies of one representative and have the same signs.
+// of a group are copies of one representative and have the same signs.  room: as many rows of words at least.
 std::tuple<Tensor, Tensor> reconstruct_with_signs(const char *op, const Tensor &reps, const Tensor &index,
                                                   const c10::optional<Tensor> &bias, const c10::optional<std::vector<Tensor>> &members,
-                                                  bool by_group) {
+                                                  bool by_group, int64_t room = 0) {
     expect(op, reps, {{Role::Features, "representatives", &reps}, {Role::Ids, "index", &index}});
     if (bias.has_value()) {
         expect(op, reps, {{Role::Bias, "bias", &*bias}});
@@ -1411,7 +1411,7 @@ std::tuple<Tensor, Tensor> reconstruct_with_signs(const char *op, const Tensor &
     c10::hip::HIPGuardMasqueradingAsCUDA guard(reps.device());
     const int64_t N = index.numel(), F = reps.size(1);
     Tensor out = torch::empty({N, F}, reps.options());
-    Tensor signs = torch::empty({by_group ? reps.size(0) : N, cgnn_sign_words(F)}, reps.options().dtype(torch::kInt32));
+    Tensor signs = torch::empty({by_group ? std::max(reps.size(0), room) : N, cgnn_sign_words(F)}, reps.options().dtype(torch::kInt32));
     if (out.numel() == 0) return {out, signs};
     std::vector<Tensor> held;
     const int32_t *perm = production_order(op, members, index, reps.size(0), &held);
@@ -1453,10 +1453,12 @@ Tensor cluster_reconstruct_backward_signs(Tensor grad, Tensor index, Tensor sign
     return reconstruct_backward_with_signs("cluster_reconstruct_backward_signs", grad, index, signs, groups, members, false);
 }
 
-// By group: what a layer keeps for its backward pass (the reference keeps the rows: layer/CompressgnnReconstruct.py:16-22).
+// By group: what a layer keeps for its backward pass (the reference keeps the rows: layer/CompressgnnReconstruct.py:16-22).  A layer
+// keeps it in a tensor with a row of words per row of its output, of which the groups have the first: what hooks on saved
+// tensors are shown has the shape of signs.
 std::tuple<Tensor, Tensor> cluster_reconstruct_masks(Tensor reps, Tensor index, c10::optional<Tensor> bias,
-                                                     c10::optional<std::vector<Tensor>> members) {
-    return reconstruct_with_signs("cluster_reconstruct_masks", reps, index, bias, members, true);
+                                                     c10::optional<std::vector<Tensor>> members, int64_t room) {
+    return reconstruct_with_signs("cluster_reconstruct_masks", reps, index, bias, members, true, room);
 }
 
 Tensor cluster_reconstruct_backward_masks(Tensor grad, Tensor index, Tensor masks, int64_t groups,
@@ -1573,7 +1575,7 @@ struct ReconstructBackward : torch::autograd::Node {
             at::NoGradGuard no_grad;
             const Tensor d_rows = grads[0].contiguous(), ids = index.unpack();
             // without a ReLU the operator does not read the rows it is given as output
-            out.push_back(relu ? cluster_reconstruct_backward_masks(d_rows, ids, masks.unpack(), groups, members)
+            out.push_back(relu ? cluster_reconstruct_backward_masks(d_rows, ids, masks.unpack().narrow(0, 0, groups), groups, members)
                                : cluster_reconstruct_backward(d_rows, ids, d_rows, groups, false, members));
             if (with_bias) out.push_back(task_should_compute_output(1) ? column_sums(out[0]) : Tensor());
         }
@@ -1598,7 +1600,7 @@ c10::optional<Tensor> reconstruct(Tensor reps, Tensor index, c10::optional<Tenso
         ids = index.contiguous();
         c10::optional<Tensor> b;
         if (bias.has_value() && bias->defined()) b = bias->contiguous();
-        if (relu) std::tie(rows, masks) = cluster_reconstruct_masks(reps.contiguous(), ids, b, members);
+        if (relu) std::tie(rows, masks) = cluster_reconstruct_masks(reps.contiguous(), ids, b, members, ids.numel());
         else rows = cluster_reconstruct(reps.contiguous(), ids, b, false, members);
     }
     const bool with_bias = bias.has_value() && bias->defined();
@@ -2078,7 +2080,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("signs"), py::arg("groups"), py::arg("members") = py::none());
     m.def("cluster_reconstruct_masks", &cluster_reconstruct_masks,
           "cluster_reconstruct with ReLU -> (rows, one sign bit per element of a representative)", py::arg("reps"),
-          py::arg("index"), py::arg("bias"), py::arg("members") = py::none());
+          py::arg("index"), py::arg("bias"), py::arg("members") = py::none(), py::arg("room") = 0);
     m.def("cluster_reconstruct_backward_masks", &cluster_reconstruct_backward_masks,
           "cluster_reconstruct_backward with ReLU, masked by the representatives' sign bits", py::arg("grad"), py::arg("index"),
           py::arg("masks"), py::arg("groups"), py::arg("members") = py::none());
