@@ -47,6 +47,7 @@
 // X may alias Y when accumulating (rule levels are updated in place, reference
 // layer/CompressgnnSPMM.py:56-58), so X and Y carry no __restrict__; a row that is
 // written is never gathered in the same launch (levels only read earlier levels).
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -66,9 +67,10 @@ constexpr int kXcds = 8;          // accelerator dies of an MI355X, each with it
 constexpr int kDefaultSeg = 64;   // non-zeros per lane group in the nnz schedule
 
 // Where the runs of the nnz kernel come from: positions that are multiples of the run length, the table of
-// workgroup runs, or the same rule worked out by every lane group (blocks that are new with every call -- member
-// lists, cgnn_spmm_once: a launch for their table would cost more than the few dependent loads).
-enum { WGRUNS_NONE = 0, WGRUNS_TABLE = 1, WGRUNS_COMPUTED = 2 };
+// workgroup runs, or the same rule worked out by every lane group (member lists, which are new with every call: a launch for
+// their table would cost more than the few dependent loads) or by every workgroup from 64-bit arrays, the rows of its entries
+// with it (cgnn_spmm_once).
+enum { WGRUNS_NONE = 0, WGRUNS_TABLE = 1, WGRUNS_COMPUTED = 2, WGRUNS_ONCE = 3 };
 enum { MODE_VAL = 0, MODE_UNIT = 1, MODE_RELU_MASK = 2, MODE_DUAL = 3, MODE_SIGN_MASK = 4, MODE_ADD = 5, MODE_ROW_MASK = 6 };
 constexpr bool has_values(int mode) { return mode == MODE_VAL || mode == MODE_ADD; }
 
@@ -117,8 +119,7 @@ struct SpmmArgs {
     int32_t keep;               // ... a row of at most this many entries is never divided, whatever the lengths
     int32_t find_empty;         // ... the rows without entries are found from rowptr, not from a list
     int32_t mean;               // MODE_UNIT, plain runs: every row is divided by its number of entries
-    const int32_t *span;        // WGRUNS_COMPUTED: {entries, where the first of them stands in val}, known on the device
-                                // only (cgnn_spmm_once); NULL: nnz entries from the start of val on
+    const int64_t *rowptr64, *col64;  // WGRUNS_ONCE: in place of rowptr, colidx and rowidx; nnz is the length of col64
 };
 
 // An entry of the table of workgroup runs is the first non-zero of a run, with this bit set when the row
@@ -126,14 +127,12 @@ struct SpmmArgs {
 constexpr int32_t kRowGoesOn = INT32_MIN;
 
 // Where lane group g of workgroup w begins, as such an entry (the rule stands at cgnn_csr.wg_runs).
-// held: length of rowidx, of which the first nnz entries count.
-__device__ __forceinline__ int32_t wg_run_begin(const int32_t *rowptr, const int32_t *rowidx, int32_t held, int32_t nnz,
-                                                int32_t wg_len, int32_t groups, int32_t keep, int64_t w, int g) {
+__device__ __forceinline__ int32_t wg_run_begin(const int32_t *rowptr, const int32_t *rowidx, int32_t nnz, int32_t wg_len,
+                                                int32_t groups, int32_t keep, int64_t w, int g) {
     // e moved back to the start of its row when the row has at most `whole` entries
     auto begin_of = [&](int64_t e, int whole) -> int32_t {
-        if (e >= held) return nnz;
-        const int r = rowidx[e];  // asked for before nnz, which may come from memory too, is looked at
         if (e >= nnz) return nnz;
+        const int r = rowidx[e];
         const int s0 = rowptr[r];
         return rowptr[r + 1] - s0 <= whole ? s0 : (s0 < e ? (int32_t)e | kRowGoesOn : (int32_t)e);
     };
@@ -581,6 +580,120 @@ __device__ __forceinline__ int run_boundary(const SpmmArgs<T> &a, int e) {
     return (a.rowptr[r + 1] - s0 <= a.seg_nnz) ? s0 : e;
 }
 
+// The rows of a block given as 64-bit row pointers: entries count from rowptr[0], and pointers that are none do not lead out
+// of the arrays.
+struct WideRows {
+    const int64_t *rowptr;
+    int64_t first, last;  // the entries that belong to rows
+    __device__ __forceinline__ int32_t at(int64_t r) const { return (int32_t)(max(first, min(last, rowptr[r])) - first); }
+};
+
+// Room for the entries of workgroup w: its wg_len, and those of a row that is moved to it as a whole.
+inline __host__ __device__ int32_t once_room(int32_t wg_len, int32_t keep) { return wg_len + (wg_len > keep ? wg_len : keep); }
+
+// Where workgroup w of WGRUNS_ONCE begins and the next one, as in the table, and row_of[e - begin]: the rows of the entries
+// between.  A wave looks for the row at the first of its wg_len positions, 64 row pointers a step, until kNear rows are left;
+// these and those behind them are read by all threads, which finds the rows at both ends, and mark their first entries;
+// a running maximum spreads the marks.  pivot: row pointer lane * search_step(rows), asked for with the first loads there are.
+//
+// In place of a launch that made int32 arrays of the block, which the product then waited for: that cost 7.5 us, the launch
+// boundary, and five dependent loads in front of a run (two now, of lines just read).  Web graphs, us, in-lists and out-lists,
+// before / so: 6,000 vertices of 16 features 16.9 / 13.9 and 11.9 / 8.7, 50,001 of 16 23.5 / 19.3 and 21.8 / 15.9, 100,003 of 64
+// 52.3 / 45.4 and 36.4 / 29.4, 325,557 of 128 264 / 253 and 197 / 181, of 8, whose few workgroups hold 2,048 entries each, 83.5 /
+// 82.9 and 72.2 / 63.2.  A search for each end of a stretch, down to the row, instead: in-lists of 325,557 vertices 266 us at
+// 128 features; 16 row pointers a step 278.
+constexpr int kNear = kBlock / 2;
+__device__ __forceinline__ int search_step(int rows) { return (rows + kWave - 1) / kWave; }
+
+template <typename T>
+__device__ __forceinline__ void once_stretch(const SpmmArgs<T> &a, const WideRows &rows, int64_t w, int64_t pivot, int *row_of,
+                                             int32_t &begin, int32_t &behind) {
+    __shared__ int found[2], wave_count[2][kBlock / kWave], wave_max[kBlock / kWave];
+    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int64_t dealt = rows.last - rows.first;
+    const int32_t room = once_room(a.wg_len, a.keep);
+    // the last row that begins at or before the place lies in [from, to), and row `from` does throughout
+    int from = 0, to = a.rows;
+    auto halve = [&](int step, int64_t start, int64_t place) {
+        const bool at_or_before = lane == 0 || (from + (int64_t)step * lane < to && start - rows.first <= place);
+        from += step * (__popcll(__ballot(at_or_before)) - 1);
+        to = to - from > step ? from + step : to;
+    };
+    auto look = [&](int64_t place, int near) {
+        while (to - from > near) {
+            const int step = search_step(to - from);
+            halve(step, rows.rowptr[min((int64_t)a.rows, from + (int64_t)step * lane)], place);
+        }
+        if (lane == 0) found[0] = from, found[1] = to;
+    };
+    const int64_t places[2] = {w * a.wg_len, (w + 1) * a.wg_len};
+    if (wave == 0) {
+        if (places[0] >= dealt) from = a.rows - 1;
+        else if (to > kNear) halve(search_step(to), pivot, places[0]);
+        look(places[0], kNear);
+    }
+    for (int k = threadIdx.x; k < room; k += kBlock) row_of[k] = -1;
+    __syncthreads();
+    from = found[0], to = found[1];
+    int64_t r = (int64_t)from + threadIdx.x;
+    int32_t s = r < a.rows ? rows.at(r) : 0, e = r < a.rows ? rows.at(r + 1) : 0;
+    const unsigned long long before_first = __ballot(r < to && s <= places[0]), before_last = __ballot(r < a.rows && s <= places[1] && s < dealt);
+    if (lane == 0) wave_count[0][wave] = __popcll(before_first), wave_count[1][wave] = __popcll(before_last);
+    __syncthreads();
+    int ahead[2] = {0, 0};
+#pragma unroll
+    for (int v = 0; v < kBlock / kWave; ++v) ahead[0] += wave_count[0][v], ahead[1] += wave_count[1][v];
+    const int r0 = from + max(ahead[0], 1) - 1;
+    int r1 = max(r0, from + ahead[1] - 1);
+    if (ahead[1] == kBlock) {  // short rows, or many without entries
+        if (wave == 0) {
+            from = r1, to = a.rows;
+            look(min(places[1], dealt - 1), 1);
+        }
+        __syncthreads();
+        r1 = found[0];
+    }
+    const int32_t whole = a.wg_len > a.keep ? a.wg_len : a.keep;
+    auto begin_of = [&](int64_t place, int row) -> int32_t {
+        const int32_t s0 = rows.at(row), end = rows.at((int64_t)row + 1);
+        if (place >= dealt) return (int32_t)dealt;
+        // (pointers that are none would take it further back than there is room)
+        if (end - s0 <= whole && place - s0 <= whole) return min(s0, (int32_t)place);
+        return s0 < place ? (int32_t)place | kRowGoesOn : (int32_t)place;
+    };
+    begin = begin_of(places[0], r0), behind = begin_of(places[1], r1);
+    const int32_t b0 = begin & ~kRowGoesOn, count = min((behind & ~kRowGoesOn) - b0, room);
+    while (r <= r1) {  // r1 < rows
+        // rows without entries begin where another does: not marked, so one row a mark
+        if (r > r0 && e > s && s > b0 && s - b0 < count) row_of[s - b0] = (int)r;
+        r += kBlock;
+        if (r <= r1) s = rows.at(r), e = rows.at(r + 1);
+    }
+    if (threadIdx.x == 0) row_of[0] = r0;
+    __syncthreads();
+    // thread t spreads the marks over entries t * each ...
+    const int each = (count + kBlock - 1) / kBlock, k0 = threadIdx.x * each, k1 = min(k0 + each, count);
+    int upto = -1;
+    for (int k = k0; k < k1; ++k) upto = max(upto, row_of[k]);
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+        const int n = __shfl_up(upto, d, kWave);
+        if (lane >= d) upto = max(upto, n);
+    }
+    if (lane == kWave - 1) wave_max[wave] = upto;
+    int before = __shfl_up(upto, 1, kWave);
+    if (lane == 0) before = -1;
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < kBlock / kWave; ++v)
+        if (v < wave) before = max(before, wave_max[v]);
+    for (int k = k0; k < k1; ++k) {
+        before = max(before, row_of[k]);
+        row_of[k] = before;
+    }
+    __syncthreads();
+}
+
 // What a workgroup's runs left of the rows that are divided among them, put together: the end of the
 // kernel below for workgroup runs.  Every lane group holds the sum of the row that goes on behind its run
 // (`continues`, in acc) and in `heads` the part of a row that came into its run and ended there; still
@@ -588,11 +701,12 @@ __device__ __forceinline__ int run_boundary(const SpmmArgs<T> &a, int e) {
 // and of the next.  The lane group a row begins in adds the parts of those behind it, in
 // ascending order.  Slots of 2 * workgroups rows of a.carry hold the pieces of the rows that pass from one
 // workgroup to the next: 2 * w for the row that comes into workgroup w, 2 * w + 1 for one that begins in it.
-template <typename T, int VEC, int LPR, int TILES, int MODE>
+// end_row(e, which): the row of the workgroup's first entry (0) or its last (1); row_start(r): the first entry of row r.
+template <typename T, int VEC, int LPR, int TILES, int MODE, int WGRUNS, typename EndRow, typename RowStart>
 __device__ __forceinline__ void join_rows(const SpmmArgs<T> &a, int block, int lane, int grp, const int64_t foff[TILES],
                                           const Acc<T, VEC, TILES, MODE> &acc, bool continues, bool open, int y_row,
                                           int32_t begin, int32_t behind, int *flags, Pack<T, VEC> (*tails)[kBlock],
-                                          Pack<T, VEC> (*heads)[kBlock]) {
+                                          Pack<T, VEC> (*heads)[kBlock], const EndRow &end_row, const RowStart &row_start) {
     constexpr int GPB = kBlock / LPR;
     constexpr int kContinues = 1, kWholeRun = 2;
     Pack<T, VEC> part[TILES];
@@ -608,7 +722,7 @@ __device__ __forceinline__ void join_rows(const SpmmArgs<T> &a, int block, int l
     }
     __syncthreads();
     const int64_t groups = (int64_t)a.blocks * GPB;
-    if constexpr (MODE != MODE_ADD) {  // rows without entries
+    if constexpr (MODE != MODE_ADD && WGRUNS != WGRUNS_ONCE) {  // rows without entries
         const int candidates = a.find_empty ? a.rows : a.n_empty_rows;
 #pragma unroll 1
         for (int64_t item = (int64_t)block * GPB + grp; item < candidates; item += groups) {
@@ -691,12 +805,12 @@ __device__ __forceinline__ void join_rows(const SpmmArgs<T> &a, int block, int l
     if (!comes_in && !goes_out) return;
     // Rows that this workgroup shares with others.
     __shared__ int arrived_last;
-    const int first_row = a.rowidx[begin & ~kRowGoesOn], last_row = a.rowidx[(behind & ~kRowGoesOn) - 1];
+    const int first_row = end_row(begin & ~kRowGoesOn, 0), last_row = end_row((behind & ~kRowGoesOn) - 1, 1);
 #pragma unroll 1
     for (int side = 0; side < 2; ++side) {
         if (side == 0 ? !comes_in : (!goes_out || (comes_in && first_row == last_row))) continue;
         const int row = side == 0 ? first_row : last_row;
-        const int w0 = a.rowptr[row] / a.wg_len, w1 = (a.rowptr[row + 1] - 1) / a.wg_len;
+        const int w0 = min(row_start(row) / a.wg_len, a.blocks - 1), w1 = (row_start(row + 1) - 1) / a.wg_len;
         // every store of the piece has reached memory before the arrival is counted
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __builtin_amdgcn_s_waitcnt(0);
@@ -767,31 +881,59 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
     constexpr bool kAhead = ROUND == kDeepRound || has_values(MODE) || MODE == MODE_UNIT || MODE == MODE_ROW_MASK;
     constexpr bool kRowsBehindGathers = MODE != MODE_DUAL;
     __shared__ int wg_row[GPB];
-    __shared__ Pack<T, VEC> wg_carry[TILES][kBlock];
+    constexpr bool kOnce = WGRUNS == WGRUNS_ONCE;
+    __shared__ Pack<T, VEC> wg_carry[kOnce ? 1 : TILES][kOnce ? 1 : kBlock];
     __shared__ Pack<T, VEC> wg_head[WGRUNS != WGRUNS_NONE ? TILES : 1][WGRUNS != WGRUNS_NONE ? kBlock : 1];
     const int lane = threadIdx.x % LPR, grp = threadIdx.x / LPR;
     const int block = logical_block(a);
     int seg = block * GPB + grp;
     if constexpr (LPR == kWave) seg = __builtin_amdgcn_readfirstlane(seg);
-    int32_t dealt = a.nnz;
-    if constexpr (WGRUNS == WGRUNS_COMPUTED && has_values(MODE))
-        if (a.span != nullptr) {
-            dealt = a.span[0];
-            if (a.val != nullptr) a.val += a.span[1];
-        }
+    // WGRUNS_ONCE: the rows of the workgroup's entries, and when all runs are done what wg_carry holds otherwise
+    extern __shared__ __attribute__((aligned(16))) int row_of[];
+    WideRows wide{};
+    unsigned long long empties = 0;  // WGRUNS_ONCE: rows without entries, one a lane
     int e0 = 0, e1 = 0;
     bool continues = false;    // the last row of the run goes on in the next one
     bool open = false;         // WGRUNS: the row at hand began before the run
     int32_t wg_begin = 0, wg_behind = 0;
-    if (seg < a.nseg) {
+    // WGRUNS_ONCE: every wave looks at an equal share of the rows for those without entries, which are neighbours (the youngest
+    // vertices of a graph's in-lists): zero_rows consecutive ones at a time (64 a wave, so that some have many and most
+    // none: in-lists of 325,557 vertices 282 us at 128 features, 253 so).
+    const int zero_rows = (int)min((int64_t)kWave, (a.rows + (int64_t)a.blocks * (kBlock / kWave) - 1) / ((int64_t)a.blocks * (kBlock / kWave)));
+    const int64_t zero_row0 = ((int64_t)block * (kBlock / kWave) + threadIdx.x / kWave) * zero_rows;
+    if constexpr (WGRUNS == WGRUNS_ONCE) {
+        const int64_t held = a.nnz, looked_at = zero_row0 + threadIdx.x % kWave;
+        wide.rowptr = a.rowptr64;
+        const int64_t p = a.rowptr64[min((int64_t)a.rows, looked_at)], q = a.rowptr64[min((int64_t)a.rows, looked_at + 1)];
+        const int64_t pivot = a.rowptr64[min((int64_t)a.rows, (int64_t)search_step(a.rows) * (threadIdx.x % kWave))];
+        wide.first = max((int64_t)0, min(held, a.rowptr64[0]));
+        wide.last = max(wide.first, min(held, a.rowptr64[a.rows]));
+        if constexpr (MODE != MODE_ADD)
+            empties = __ballot(block < a.blocks && (int)(threadIdx.x % kWave) < zero_rows && looked_at < a.rows && min(p, wide.last) >= max(q, wide.first));
+        if (a.val != nullptr) a.val += wide.first;
+        a.col64 += wide.first;
+        once_stretch(a, wide, block, pivot, row_of, wg_begin, wg_behind);
+        wg_begin = __builtin_amdgcn_readfirstlane(wg_begin), wg_behind = __builtin_amdgcn_readfirstlane(wg_behind);  // no vector registers
+        const int32_t first = wg_begin & ~kRowGoesOn, end = wg_behind & ~kRowGoesOn;
+        const int run_len = a.wg_len / GPB, whole = run_len > a.keep ? run_len : a.keep;
+        auto begin_of = [&](int g) -> int32_t {
+            const int32_t e = first + g * ((end - first + GPB - 1) / GPB);
+            if (g == 0) return wg_begin;
+            if (e >= end) return wg_behind;
+            const int row = row_of[e - first];
+            const int32_t s0 = wide.at(row), behind = wide.at((int64_t)row + 1);
+            return behind - s0 <= whole ? max(first, min(e, s0)) : (s0 < e ? e | kRowGoesOn : e);
+        };
+        const int32_t r0 = begin_of(grp), r1 = begin_of(grp + 1);
+        e0 = r0 & ~kRowGoesOn, e1 = r1 & ~kRowGoesOn;
+        open = r0 < 0, continues = r1 < 0;
+    } else if (seg < a.nseg) {
         if constexpr (WGRUNS != WGRUNS_NONE) {
             int32_t r0, r1;
             if constexpr (WGRUNS == WGRUNS_TABLE) {
                 r0 = a.run_start[seg], r1 = a.run_start[seg + 1];
             } else {
-                auto begin_of = [&](int w, int g) {
-                    return wg_run_begin(a.rowptr, a.rowidx, a.nnz, dealt, a.wg_len, GPB, a.keep, w, g);
-                };
+                auto begin_of = [&](int w, int g) { return wg_run_begin(a.rowptr, a.rowidx, a.nnz, a.wg_len, GPB, a.keep, w, g); };
                 wg_begin = begin_of(block, 0), wg_behind = begin_of(block + 1, 0);
                 r0 = begin_of(block, grp), r1 = grp + 1 < GPB ? begin_of(block, grp + 1) : wg_behind;
             }
@@ -805,6 +947,8 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
             e1 = run_boundary(a, (seg + 1) * a.seg_nnz);
         }
     }
+    auto row_at = [&](int e) -> int { return WGRUNS == WGRUNS_ONCE ? row_of[e - (wg_begin & ~kRowGoesOn)] : a.rowidx[e]; };
+    auto col_at = [&](int e) -> int { return WGRUNS == WGRUNS_ONCE ? (int)a.col64[e] : a.colidx[e]; };
     // e0 >= e1 inside the list cannot happen for a well-formed CSR
     const bool active = e0 < e1;
     // means: a row that began before the run is divided by the pass that adds its carries up
@@ -873,8 +1017,8 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
             auto load_entry = [&](int e) {  // this lane's of the batch from e on
                 my_row = 0, my_c = 0, my_w = T(1);
                 if (e + lane >= e1) return;
-                my_row = a.rowidx[e + lane];
-                my_c = a.colidx[e + lane];
+                my_row = row_at(e + lane);
+                my_c = col_at(e + lane);
                 if constexpr (MODE == MODE_DUAL) my_w = a.val[e + lane];
                 if constexpr (has_values(MODE)) my_w = a.val != nullptr ? a.val[e + lane] : T(1);
             };
@@ -973,7 +1117,7 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
             }
         } else {
             if constexpr (kNamesRowsOfY) {
-                cur_out = named(a.rowidx[e0]);
+                cur_out = named(row_at(e0));
                 begin_row(cur_out);
                 if constexpr (WGRUNS == WGRUNS_NONE) {
                     last_row = a.rowidx[e1 - 1];
@@ -987,8 +1131,8 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
 #pragma unroll
                 for (int u = 0; u < kUnroll; ++u) {
                     const int idx = min(e + u, e1 - 1);
-                    o[u] = named(a.rowidx[idx]);
-                    c[u] = a.colidx[idx];
+                    o[u] = named(row_at(idx));
+                    c[u] = col_at(idx);
                     if constexpr (MODE == MODE_DUAL) w[u] = a.val[idx];
                     else if constexpr (has_values(MODE)) w[u] = a.val != nullptr ? a.val[idx] : T(1);
                     else w[u] = T(1);
@@ -1025,9 +1169,34 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
     if constexpr (WGRUNS != WGRUNS_NONE) {
         if constexpr (WGRUNS == WGRUNS_TABLE)
             if (seg < a.nseg) wg_begin = a.run_start[block * GPB], wg_behind = a.run_start[(block + 1) * GPB];
-        join_rows<T, VEC, LPR, TILES, MODE>(a, block, lane, grp, foff, acc, continues, open,
-                                            continues && active ? row_of_y(cur_out) : -1, wg_begin, wg_behind, wg_row,
-                                            wg_carry, wg_head);
+        if constexpr (WGRUNS == WGRUNS_ONCE && MODE != MODE_ADD) {  // rows without entries, a wave per row
+            for (int64_t row0 = zero_row0;;) {
+                for (; empties != 0; empties &= empties - 1) {
+                    T *y = a.Y + (row0 + __ffsll(empties) - 1) * a.F;
+                    if (blockIdx.y == 0)
+                        for (int64_t f = threadIdx.x % kWave; f < a.F; f += kWave) y[f] = T(0);
+                }
+                row0 += (int64_t)a.blocks * (kBlock / kWave) * zero_rows;
+                if (block >= a.blocks || row0 >= a.rows) break;
+                const int64_t r = row0 + threadIdx.x % kWave;
+                empties = __ballot((int)(threadIdx.x % kWave) < zero_rows && r < a.rows && wide.at(min((int64_t)a.rows - 1, r)) >= wide.at(min((int64_t)a.rows, r + 1)));
+            }
+        }
+        Pack<T, VEC>(*tails)[kBlock];
+        int ends[2] = {0, 0};  // the rows of the workgroup's first entry and of its last
+        if constexpr (kOnce) {
+            const int32_t first = wg_begin & ~kRowGoesOn, end = wg_behind & ~kRowGoesOn;
+            ends[0] = row_of[0], ends[1] = row_of[max(0, end - first - 1)];
+            __syncthreads();
+            tails = reinterpret_cast<Pack<T, VEC>(*)[kBlock]>(row_of);
+        } else {
+            tails = wg_carry;
+        }
+        auto end_row = [&](int32_t e, int which) -> int { return kOnce ? ends[which] : a.rowidx[e]; };
+        auto row_start = [&](int64_t r) -> int32_t { return WGRUNS == WGRUNS_ONCE ? wide.at(r) : a.rowptr[r]; };
+        join_rows<T, VEC, LPR, TILES, MODE, WGRUNS>(a, block, lane, grp, foff, acc, continues, open,
+                                                    continues && active ? row_of_y(cur_out) : -1, wg_begin, wg_behind, wg_row,
+                                                    tails, wg_head, end_row, row_start);
         return;
     }
     // The carries of one row are added per workgroup (or per merge_stride lane groups of it): the first lane
@@ -1468,7 +1637,10 @@ void launch_nnz(int mode, const SpmmArgs<T> &a, dim3 grid, hipStream_t stream) {
                     return;
                 }
         }
-        hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, kMode, kRuns, kUnroll>), grid, block, 0, stream, a);
+        const size_t lds = kRuns != WGRUNS_ONCE ? 0
+                                                : std::max((size_t)once_room(a.wg_len, a.keep) * sizeof(int),
+                                                           sizeof(Pack<T, VEC>) * TILES * kBlock);
+        hipLaunchKernelGGL((spmm_nnz_kernel<T, VEC, LPR, TILES, kMode, kRuns, kUnroll>), grid, block, lds, stream, a);
     };
     const std::integral_constant<int, MODE_VAL> val;
     const std::integral_constant<int, MODE_ADD> add;
@@ -1477,11 +1649,13 @@ void launch_nnz(int mode, const SpmmArgs<T> &a, dim3 grid, hipStream_t stream) {
     const std::integral_constant<int, MODE_SIGN_MASK> sign_mask;
     const std::integral_constant<int, MODE_RELU_MASK> relu_mask;
     const std::integral_constant<int, MODE_ROW_MASK> row_mask;
-    if (a.arrivals != nullptr && a.run_start == nullptr) {
+    if (a.rowptr64 != nullptr) {
+        const std::integral_constant<int, WGRUNS_ONCE> once;
+        if (a.accumulate) go(add, once);
+        else go(val, once);
+    } else if (a.arrivals != nullptr && a.run_start == nullptr) {
         const std::integral_constant<int, WGRUNS_COMPUTED> computed;
         if (mode == MODE_UNIT) go(unit, computed);
-        else if (mode == MODE_VAL && a.accumulate) go(add, computed);
-        else if (mode == MODE_VAL) go(val, computed);
         else if (mode == MODE_SIGN_MASK) go(sign_mask, computed);
         else if (mode == MODE_ROW_MASK) go(row_mask, computed);
         else go(relu_mask, computed);
@@ -1843,7 +2017,7 @@ __global__ void run_starts_kernel(const int32_t *__restrict__ rowptr, const int3
 __global__ void wg_runs_kernel(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ rowidx, int32_t nnz,
                                int32_t wg_len, int32_t groups, int64_t n, int32_t *__restrict__ runs) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) runs[i] = wg_run_begin(rowptr, rowidx, nnz, nnz, wg_len, groups, 0, i / groups, (int)(i % groups));
+    if (i < n) runs[i] = wg_run_begin(rowptr, rowidx, nnz, wg_len, groups, 0, i / groups, (int)(i % groups));
 }
 
 // rowidx[e] = largest r with rowptr[r] <= e (rows without entries are skipped).
@@ -1859,125 +2033,6 @@ __global__ void expand_rows_kernel(const P *__restrict__ rowptr, int64_t rows, i
             else hi = mid;
         }
         rowidx[e] = (int32_t)lo;
-    }
-}
-
-// The int32 form of a block that is given as int64 arrays for one product: row pointers, columns and the row of
-// every entry, in one launch.  Rows and entries are walked as one list -- every row in front of its entries, row r at
-// position rowptr[r] + r -- and a workgroup takes ITEMS * kBlock consecutive places of it, so neither hubs (a
-// workgroup per 16 rows took 41 us for 100,003 rows of 1.0 M entries of a web graph, whose hubs are neighbours) nor the
-// thousands of empty rows of the youngest vertices (2,048 entries per workgroup: 22 us) keep one longer than the others.
-// Two of its waves look for the two ends of its stretch, 64 row pointers a step, and its threads mark the entries that rows
-// begin at and spread the marks by a running maximum: 7.4 us.  With all threads at the search, 256 row pointers a step, the
-// card spent its time on requests for row pointers: 9.0 us (1,024 a step: 13).  Row pointers and columns narrowed apart and
-// a binary search per entry were three launches of 25 us, behind 26 us for the length of the longest row and its way to the
-// host.
-// The rows hold the entries [rowptr64[0], rowptr64[rows]) of the arrays: a slice of the row pointers of a larger block
-// comes with all its entries, and a list may be padded behind the last row.  Only these entries are taken over, and the
-// int32 arrays count from the first of them: span = {how many, where the first stands}.
-// 1,024 places a workgroup while that is about a round of workgroups, whose searches then wait beside each other (a product
-// over 8,000 rows 20.1 -> 19.4 us), and 2,048 beyond, where the searches cost (325,557 rows 92.7 -> 90.3).
-int once_items(int64_t places) { return places <= (int64_t)4 * kBlock * 1536 ? 4 : 8; }
-
-template <int ITEMS>
-__global__ __launch_bounds__(kBlock) void csr_once_kernel(const int64_t *__restrict__ rowptr64, const int64_t *__restrict__ col64,
-                                                          int64_t rows, int64_t nnz, int32_t *__restrict__ rowptr,
-                                                          int32_t *__restrict__ col, int32_t *__restrict__ rowidx,
-                                                          int32_t *__restrict__ span) {
-    constexpr int kPlaces = ITEMS * kBlock;
-    __shared__ int32_t begins[kPlaces];  // the row that begins at an entry of the stretch, or -1
-    __shared__ int waves[kBlock / kWave];
-    __shared__ int64_t found[2];
-    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int64_t places[2] = {(int64_t)blockIdx.x * kPlaces, min(rows + nnz, (int64_t)(blockIdx.x + 1) * kPlaces)};
-#pragma unroll
-    for (int u = 0; u < ITEMS; ++u) begins[u * kBlock + threadIdx.x] = -1;
-    // The largest row at or before each of the two places: a wave looks for one of them, 64 row pointers a step
-    // (it lies in [from, to), and row `from` does throughout).
-    if (wave < 2) {
-        int64_t from = 0, to = rows;
-        const int64_t place = places[wave];
-        while (to - from > 1) {
-            const int64_t step = (to - from + kWave - 1) / kWave, r = from + step * lane;
-            const bool at_or_before = lane == 0 || (r < to && rowptr64[r] + r <= place);
-            from += step * (__popcll(__ballot(at_or_before)) - 1);
-            to = min(to, from + step);
-        }
-        if (lane == 0) found[wave] = from;
-    }
-    __syncthreads();
-    const int64_t lo[2] = {found[0], found[1]};
-    // the entries that belong to rows; row pointers that are none must not lead out of the arrays
-    const int64_t first = max((int64_t)0, min(nnz, rowptr64[0])), last = max(first, min(nnz, rowptr64[rows]));
-    auto inside = [&](int64_t e) { return max(first, min(last, e)); };
-    if (blockIdx.x == 0 && threadIdx.x == 0) span[0] = (int32_t)(last - first), span[1] = (int32_t)first;
-    // first entry and first row of the stretch, and those behind it
-    int64_t entry[2], row[2];
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const int64_t start = rowptr64[lo[k]];
-        const bool on_row = start + lo[k] >= places[k];  // the place is that of the row itself
-        entry[k] = inside(on_row ? start : places[k] - lo[k] - 1);
-        row[k] = on_row ? lo[k] : lo[k] + 1;
-    }
-    if (places[1] == rows + nnz) entry[1] = last, row[1] = rows;
-    const int64_t e0 = entry[0];
-    const int held = (int)max((int64_t)0, min((int64_t)kPlaces, entry[1] - e0));
-    int64_t c[ITEMS], at[ITEMS], end[ITEMS];
-#pragma unroll
-    for (int u = 0; u < ITEMS; ++u) {
-        const int k = u * kBlock + threadIdx.x;
-        const int64_t r = row[0] + k;
-        c[u] = k < held ? col64[e0 + k] : 0;
-        // without a condition, on which the limits below would be worked out beside each load, the next one
-        // waiting behind them (11.1 us instead of 9.0)
-        at[u] = rowptr64[min(r, rows - 1)];
-        end[u] = rowptr64[min(r, rows - 1) + 1];
-    }
-#pragma unroll
-    for (int u = 0; u < ITEMS; ++u) {
-        const int64_t r = row[0] + u * kBlock + threadIdx.x;
-        if (r >= row[1]) break;
-        at[u] = inside(at[u]), end[u] = inside(end[u]);
-        rowptr[r] = (int32_t)(at[u] - first);
-        if (r == rows - 1) rowptr[rows] = (int32_t)(end[u] - first);
-        // rows without entries begin where another does: not marked, so one row a mark
-        const int64_t k = at[u] - e0;
-        if (end[u] > at[u] && k >= 0 && k < held) begins[k] = (int32_t)r;
-    }
-    __syncthreads();
-    // thread t spreads the marks over entries t * ITEMS ...; what comes before the first mark belongs to the
-    // row in front of the stretch
-    int32_t mark[ITEMS];
-#pragma unroll
-    for (int u = 0; u < ITEMS; ++u) {
-        mark[u] = begins[threadIdx.x * ITEMS + u];
-        if (u > 0) mark[u] = max(mark[u], mark[u - 1]);
-    }
-    int upto = mark[ITEMS - 1];
-#pragma unroll
-    for (int s = 1; s < kWave; s <<= 1) {
-        const int n = __shfl_up(upto, s, kWave);
-        if (lane >= s) upto = max(upto, n);
-    }
-    if (lane == kWave - 1) waves[wave] = upto;
-    int before = __shfl_up(upto, 1, kWave);
-    if (lane == 0) before = -1;
-    __syncthreads();
-    before = max(before, (int)row[0] - 1);
-#pragma unroll
-    for (int w = 0; w < kBlock / kWave; ++w)
-        if (w < wave) before = max(before, waves[w]);
-#pragma unroll
-    for (int u = 0; u < ITEMS; ++u) begins[threadIdx.x * ITEMS + u] = max(mark[u], before);
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < ITEMS; ++u) {
-        const int k = u * kBlock + threadIdx.x;
-        if (k < held) {
-            col[e0 - first + k] = (int32_t)c[u];
-            rowidx[e0 - first + k] = begins[k];
-        }
     }
 }
 
@@ -2267,9 +2322,9 @@ extern "C" int cgnn_spmm_run_length(const cgnn_csr *A) { return A == nullptr ? 0
 namespace {
 
 struct OnceLayout {
-    size_t span, rowptr, col, rowidx, pieces, total;
     int groups, wg_len;
     int64_t workgroups;
+    size_t total;  // the pieces
 };
 
 OnceLayout once_layout(int64_t rows, int64_t nnz, int64_t F, int dtype) {
@@ -2281,33 +2336,25 @@ OnceLayout once_layout(int64_t rows, int64_t nnz, int64_t F, int dtype) {
     L.groups = kBlock / shape_of(F, dtype).lpr;
     L.wg_len = wg_run_len(&A, L.groups, most_per_new_run(&A)) * L.groups;
     L.workgroups = ceil_div(nnz, L.wg_len);
-    L.span = 0;
-    L.rowptr = 256;
-    L.col = L.rowptr + align_up((size_t)(rows + 1) * sizeof(int32_t), 256);
-    L.rowidx = L.col + align_up((size_t)nnz * sizeof(int32_t), 256);
-    L.pieces = L.rowidx + align_up((size_t)nnz * sizeof(int32_t), 256);
-    L.total = L.pieces + wg_piece_bytes(L.workgroups, F, dtype == CGNN_F64 ? 8 : 4);
+    L.total = wg_piece_bytes(L.workgroups, F, dtype == CGNN_F64 ? 8 : 4);
     return L;
 }
 
 template <typename T>
-int spmm_once(const OnceLayout &L, int64_t rows, int64_t nnz, const void *val, int dtype, const void *X, void *Y, int64_t F,
-              int accumulate, char *ws, int32_t *arrivals, hipStream_t stream) {
+int spmm_once(const OnceLayout &L, int64_t rows, int64_t nnz, const int64_t *rowptr, const int64_t *col, const void *val,
+              const void *X, void *Y, int64_t F, int accumulate, void *workspace, int32_t *arrivals, hipStream_t stream) {
     cgnn_csr A{};
     A.rows = rows;
     A.nnz = nnz;
-    A.rowptr = reinterpret_cast<const int32_t *>(ws + L.rowptr);
-    A.colidx = reinterpret_cast<const int32_t *>(ws + L.col);
-    A.rowidx = reinterpret_cast<const int32_t *>(ws + L.rowidx);
     A.val = val;
     SpmmArgs<T> a = make_args<T>(&A, X, nullptr, INT32_MAX, nullptr, Y, F, accumulate);
+    a.rowptr64 = rowptr;
+    a.col64 = col;
     a.arrivals = arrivals;
     a.wg_len = L.wg_len;
     a.keep = kDefaultSeg;
     a.nseg = (int32_t)(L.workgroups * L.groups);
-    a.carry = reinterpret_cast<T *>(ws + L.pieces);
-    a.find_empty = 1;
-    a.span = reinterpret_cast<const int32_t *>(ws + L.span);
+    a.carry = static_cast<T *>(workspace);
     return launch<T>(KIND_NNZ, MODE_VAL, pick_shape<T>(F, true), a, a.nseg, stream);
 }
 
@@ -2330,17 +2377,9 @@ extern "C" int cgnn_spmm_once(int64_t rows, int64_t nnz, const int64_t *rowptr, 
     CGNN_REQUIRE(rowptr && col && X && Y && arrivals, "cgnn_spmm_once: null array");
     const OnceLayout L = once_layout(rows, nnz, F, dtype);
     if (workspace == nullptr || workspace_bytes < L.total) return fail(CGNN_EWORKSPACE, "cgnn_spmm_once: workspace too small");
-    char *ws = static_cast<char *>(workspace);
-    const int items = once_items(rows + nnz);
-    hipLaunchKernelGGL(items == 4 ? csr_once_kernel<4> : csr_once_kernel<8>, dim3((unsigned)ceil_div(rows + nnz, items * kBlock)),
-                       dim3(kBlock), 0, stream, rowptr, col, rows, nnz, reinterpret_cast<int32_t *>(ws + L.rowptr),
-                       reinterpret_cast<int32_t *>(ws + L.col), reinterpret_cast<int32_t *>(ws + L.rowidx),
-                       reinterpret_cast<int32_t *>(ws + L.span));
-    int rc = check_launch("csr_once");
-    if (rc != CGNN_OK) return rc;
     if (dtype == CGNN_F32)
-        return spmm_once<float>(L, rows, nnz, val, dtype, X, Y, F, accumulate, ws, arrivals, stream);
-    return spmm_once<double>(L, rows, nnz, val, dtype, X, Y, F, accumulate, ws, arrivals, stream);
+        return spmm_once<float>(L, rows, nnz, rowptr, col, val, X, Y, F, accumulate, workspace, arrivals, stream);
+    return spmm_once<double>(L, rows, nnz, rowptr, col, val, X, Y, F, accumulate, workspace, arrivals, stream);
 }
 
 extern "C" int cgnn_spmm_wg_shape(const cgnn_csr *A, int64_t F, int dtype, int32_t *groups, int32_t *wg_len,

@@ -394,7 +394,7 @@ Tensor block_spmm(DeviceCsr &A, const Tensor &mat, c10::optional<Tensor> optiona
 }
 
 // spmm_func of the reference (src/runtime/csrc/sparse/spmm.cpp:11-22): CSR given as
-// int64 tensors, narrowed on every call.  Graph blocks that are used repeatedly should
+// int64 tensors, whose rows are looked for on every call.  Graph blocks that are used repeatedly should
 // be wrapped in a DeviceCsr once instead.
 Tensor spmm_func(Tensor vlist, Tensor elist, Tensor value, Tensor mat, std::string method,
                  c10::optional<Tensor> optional_out) {

@@ -128,7 +128,7 @@ int cgnn_spmm_wg_runs(const cgnn_csr *A, int32_t groups, int32_t wg_len, int32_t
 size_t cgnn_spmm_workspace_bytes(const cgnn_csr *A, int64_t F, int dtype, int kernel);
 
 /* One product of a block given as int64 arrays, as cgnn_spmm under AUTO but without what a block that is kept
- * has made once: the arrays are narrowed by the call (one launch), the schedule is the NNZ one with workgroup runs
+ * has made once: the launch reads the arrays as they are, the schedule is the NNZ one with workgroup runs
  * whatever the rows look like, and nothing is read by the host.  A row of at most 64 entries is summed in
  * ascending order.  arrivals: counters as in cgnn_csr, as many as the size query reports.  rows, nnz and F must
  * be positive; the row pointers must ascend and the columns of the rows must lie in X (not checked).  nnz is the length of

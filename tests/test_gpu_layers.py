@@ -1324,3 +1324,38 @@ def test_other_threads_run_while_a_call_waits_for_the_stream(call):
     inside = [begin] + [t for t in stamps if begin < t < end] + [end]
     longest = max(later - earlier for earlier, later in zip(inside, inside[1:]))
     assert longest < 0.5 * (end - begin)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("width", [1, 3, 16, 33, 64, 130, 200, 520, 1030])
+def test_products_of_int64_arrays_of_every_shape(width, dtype):
+    """spmm_func looks for the rows of a workgroup's entries itself: numbers of rows around a step of the search and around what
+    the workgroup reads of them at once, rows without entries in front, between and behind, rows at the lengths that are moved
+    or divided, hubs over many workgroups, slices and padded lists.  Whole numbers: the sums are exact in any order."""
+    import compressgnn_runtime as rt
+    rng = np.random.default_rng(width)
+    lengths = [[5], [0, 0, 3], [0] * 300 + [70] + [0] * 700, [1] * 129, [64] * 128, [65] * 64, [63, 64, 65, 0, 31, 32, 33] * 40,
+               [0, 1] * 3000, [5000], [1, 3000, 1, 0, 700] * 9, rng.integers(0, 40, 255).tolist(), rng.integers(0, 3, 8200).tolist(),
+               (rng.pareto(1.2, 4097) * 3).astype(int).clip(0, 4000).tolist(), rng.integers(0, 20, 16385).tolist()]
+    for lens in lengths:
+        cols = 500
+        v = np.concatenate([[0], np.cumsum(lens)])
+        pad = int(rng.integers(0, 3)) * 777  # entries that no row holds
+        first = int(rng.integers(0, 2)) * 130
+        e = torch.from_numpy(rng.integers(0, cols, first + v[-1] + pad)).to(DEV)
+        ptr = torch.from_numpy(v + first).to(DEV)
+        w = torch.from_numpy(rng.integers(-3, 4, len(e))).to(DEV).to(dtype)
+        x = torch.from_numpy(rng.integers(-8, 9, (cols, width))).to(DEV).to(dtype)
+        rows = torch.repeat_interleave(torch.arange(len(lens), device=DEV), torch.tensor(lens, device=DEV))
+        inside = slice(first, first + int(v[-1]))
+        want = torch.zeros(len(lens), width, device=DEV, dtype=dtype)
+        for at in range(0, int(v[-1]), 1 << 14):  # in parts: no array of all products
+            part = slice(inside.start + at, min(inside.stop, inside.start + at + (1 << 14)))
+            want.index_add_(0, rows[at:at + (1 << 14)], x[e[part]] * w[part, None])
+        w[:first], w[inside.stop:] = float("nan"), float("nan")
+        for _ in range(2):
+            assert torch.equal(rt.spmm_func(ptr, e, w, x, "auto", None), want)
+        base = torch.from_numpy(rng.integers(-9, 9, (len(lens), width))).to(DEV).to(dtype)
+        assert torch.equal(rt.spmm_func(ptr, e, w, x, "auto", base.clone()), base + want)
+    nothing = torch.full((1000,), 40, device=DEV, dtype=torch.int64)  # a slice whose rows are all empty
+    assert not rt.spmm_func(nothing, e, w, x, "auto", None).any()
