@@ -219,6 +219,22 @@ __device__ __forceinline__ void feature_offsets(int64_t F, int lane, int64_t fof
     }
 }
 
+// The value of the lane at byte address `from`, through the LDS crossbar.  Doubles cross it as two halves: loading every entry
+// in every lane instead, products of double int64 blocks took, web graphs, us, so / with the crossbar (and in one launch):
+// 6,000 vertices of 14 features, in-lists, 20.2 / 13.9, 50,001 of 32 61 / 36, 325,557 of 64 330 / 252.
+template <typename T>
+__device__ __forceinline__ T from_lane(int from, T v) {
+    if constexpr (sizeof(T) == 4) {
+        return __builtin_bit_cast(T, __builtin_amdgcn_ds_bpermute(from, __builtin_bit_cast(int, v)));
+    } else {
+        struct Halves {
+            int lo, hi;
+        };
+        const Halves h = __builtin_bit_cast(Halves, v);
+        return __builtin_bit_cast(T, Halves{__builtin_amdgcn_ds_bpermute(from, h.lo), __builtin_amdgcn_ds_bpermute(from, h.hi)});
+    }
+}
+
 // What a gather of one feature tile brings: the pack of X, and what decides which of its elements count.  Loads only: they
 // stand in a branch of their own (no gathers behind the end of a row), and what used the loaded values there would have to
 // wait for them before the next gather of the round is asked for -- four waits one after the other, which doubled the time of
@@ -469,78 +485,55 @@ __global__ __launch_bounds__(kBlock) void spmm_row_kernel(SpmmArgs<T> a) {
         if constexpr (MODE != MODE_ADD) write_row<T, VEC, TILES, MODE>(a.Y, a.F, row, foff, acc);
         return;
     }
-    if constexpr (sizeof(T) == 4) {
-        constexpr int RU = LPR < kRowUnroll ? LPR : kRowUnroll;  // entries per round: no more than lanes to stage them
-        // The lanes of the group load one entry each (one coalesced load per array for LPR
-        // entries), and every entry is then handed to all lanes through the LDS crossbar:
-        // no address arithmetic and no memory instruction per entry and lane for the indices.
-        const int group_lane0 = 4 * ((threadIdx.x % kWave) - lane);  // byte address of the group's first lane
-        // lanes beyond the width gather feature 0 again (never stored): no test per gather
-        int64_t fld[TILES];
+    constexpr int RU = LPR < kRowUnroll ? LPR : kRowUnroll;  // entries per round: no more than lanes to stage them
+    // The lanes of the group load one entry each (one coalesced load per array for LPR
+    // entries), and every entry is then handed to all lanes through the LDS crossbar:
+    // no address arithmetic and no memory instruction per entry and lane for the indices.
+    const int group_lane0 = 4 * ((threadIdx.x % kWave) - lane);  // byte address of the group's first lane
+    // lanes beyond the width gather feature 0 again (never stored): no test per gather
+    int64_t fld[TILES];
 #pragma unroll
-        for (int t = 0; t < TILES; ++t) fld[t] = foff[t] < 0 ? 0 : foff[t];
-        for (int e = e0; e < e1; e += LPR) {
-            int my_c = 0;
-            T my_w = T(1);
-            if (e + lane < e1) {
-                my_c = a.colidx[e + lane];
-                if (a.val) my_w = a.val[e + lane];
-            }
-            const int cnt = min(e1 - e, LPR);
-            for (int u0 = 0; u0 < cnt; u0 += RU) {
-                int c[RU];
-                T w[RU];
-#pragma unroll
-                for (int u = 0; u < RU; ++u) {
-                    const int from = group_lane0 + 4 * (u0 + u);
-                    c[u] = __builtin_amdgcn_ds_bpermute(from, my_c);
-                    w[u] = __builtin_bit_cast(T, __builtin_amdgcn_ds_bpermute(from, __builtin_bit_cast(int, my_w)));
-                }
-                // Entries of the second source are rare (columns that stand for rules): when the
-                // wave has none in this round, the gathers need no choice of source per lane.
-                bool second = false;
-                if constexpr (MODE == MODE_DUAL) {
-#pragma unroll
-                    for (int u = 0; u < RU; ++u) second = second || (u0 + u < cnt && c[u] >= a.split);
-                }
-                auto gather_and_add = [&](auto plain) {
-                    constexpr bool kPlain = decltype(plain)::value;  // every entry from the first source
-                    Gathered<T, VEC, MODE> x[RU][TILES];
-#pragma unroll
-                    for (int u = 0; u < RU; ++u)
-                        if (u0 + u < cnt) {  // no gathers behind the row's end: repeated ones still cost issue slots
-#pragma unroll
-                            for (int t = 0; t < TILES; ++t)
-                                x[u][t] = gather<T, VEC, MODE, (int)(VEC * LPR * sizeof(T))>(a, c[u], kPlain ? 0 : c[u] >= a.split, fld[t]);
-                        }
-#pragma unroll
-                    for (int u = 0; u < RU; ++u)
-                        if (u0 + u < cnt) acc.add(x[u], fld, w[u], kPlain ? 0 : c[u] >= a.split);
-                };
-                if (MODE != MODE_DUAL || __ballot(second) == 0) gather_and_add(std::true_type{});
-                else gather_and_add(std::false_type{});
-            }
+    for (int t = 0; t < TILES; ++t) fld[t] = foff[t] < 0 ? 0 : foff[t];
+    for (int e = e0; e < e1; e += LPR) {
+        int my_c = 0;
+        T my_w = T(1);
+        if (e + lane < e1) {
+            my_c = a.colidx[e + lane];
+            if (a.val) my_w = a.val[e + lane];
         }
-    } else {
-        for (int e = e0; e < e1; e += kRowUnroll) {
-            int c[kRowUnroll];
-            T w[kRowUnroll];
-            Gathered<T, VEC, MODE> x[kRowUnroll][TILES];
+        const int cnt = min(e1 - e, LPR);
+        for (int u0 = 0; u0 < cnt; u0 += RU) {
+            int c[RU];
+            T w[RU];
 #pragma unroll
-            for (int u = 0; u < kRowUnroll; ++u) {
-                const int idx = min(e + u, e1 - 1);
-                c[u] = a.colidx[idx];
-                w[u] = a.val ? a.val[idx] : T(1);
+            for (int u = 0; u < RU; ++u) {
+                const int from = group_lane0 + 4 * (u0 + u);
+                c[u] = __builtin_amdgcn_ds_bpermute(from, my_c);
+                w[u] = from_lane(from, my_w);
             }
+            // Entries of the second source are rare (columns that stand for rules): when the
+            // wave has none in this round, the gathers need no choice of source per lane.
+            bool second = false;
+            if constexpr (MODE == MODE_DUAL) {
 #pragma unroll
-            for (int u = 0; u < kRowUnroll; ++u)
-                if (e + u < e1) {
+                for (int u = 0; u < RU; ++u) second = second || (u0 + u < cnt && c[u] >= a.split);
+            }
+            auto gather_and_add = [&](auto plain) {
+                constexpr bool kPlain = decltype(plain)::value;  // every entry from the first source
+                Gathered<T, VEC, MODE> x[RU][TILES];
 #pragma unroll
-                    for (int t = 0; t < TILES; ++t) x[u][t] = gather<T, VEC, MODE, (int)(VEC * LPR * sizeof(T))>(a, c[u], c[u] >= a.split, foff[t]);
-                }
+                for (int u = 0; u < RU; ++u)
+                    if (u0 + u < cnt) {  // no gathers behind the row's end: repeated ones still cost issue slots
 #pragma unroll
-            for (int u = 0; u < kRowUnroll; ++u)
-                if (e + u < e1) acc.add(x[u], foff, w[u], c[u] >= a.split);
+                        for (int t = 0; t < TILES; ++t)
+                            x[u][t] = gather<T, VEC, MODE, (int)(VEC * LPR * sizeof(T))>(a, c[u], kPlain ? 0 : c[u] >= a.split, fld[t]);
+                    }
+#pragma unroll
+                for (int u = 0; u < RU; ++u)
+                    if (u0 + u < cnt) acc.add(x[u], fld, w[u], kPlain ? 0 : c[u] >= a.split);
+            };
+            if (MODE != MODE_DUAL || __ballot(second) == 0) gather_and_add(std::true_type{});
+            else gather_and_add(std::false_type{});
         }
     }
     write_row<T, VEC, TILES, MODE>(a.Y, a.F, row, foff, acc);
@@ -562,6 +555,7 @@ __global__ __launch_bounds__(kBlock) void spmm_row_kernel(SpmmArgs<T> a) {
 __device__ __forceinline__ void arrive(int &v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void arrive(uint32_t &v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void arrive(float &v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void arrive(double &v) { asm volatile("" : "+v"(v)); }
 template <typename T, int VEC, int MODE>
 __device__ __forceinline__ void arrive(Gathered<T, VEC, MODE> &g) {
 #pragma unroll
@@ -871,7 +865,7 @@ __device__ __forceinline__ void join_rows(const SpmmArgs<T> &a, int block, int l
 template <typename T, int VEC, int LPR, int TILES, int MODE, int WGRUNS, int ROUND>
 __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRound ? 5 : (TILES == 1 && LPR >= 16) ? 7 : 1) void spmm_nnz_kernel(SpmmArgs<T> a) {
     constexpr int GPB = kBlock / LPR;
-    static_assert(LPR % ROUND == 0 || ROUND == kUnroll, "a round's entries come from one batch");
+    static_assert(LPR % ROUND == 0, "a round's entries come from one batch");
     // What a lane group waits for between two batches of entries.  The entries of the next batch are asked for before the
     // gathers of this one, and the rows of Y they go to (rowmap, a look-up that needs the entry) are waited for behind the
     // gathers, which do not need them: a chain of entries -> gathers a batch, where it was entries -> rows -> gathers, one batch
@@ -1005,159 +999,113 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
             cur_out = a.rowidx[e0];
             if constexpr (WGRUNS == WGRUNS_NONE) row_behind = e1 < a.nnz ? a.rowidx[e1] : -1;
         }
-        if constexpr (LPR >= kUnroll && sizeof(T) == 4) {
-            // As in the row schedule: the lanes of the group load one entry each, and the
-            // entries reach all lanes through the LDS crossbar.
-            const int group_lane0 = 4 * ((threadIdx.x % kWave) - lane);
-            int64_t fld[TILES];  // lanes beyond the width gather feature 0 again (never stored)
+        // As in the row schedule: the lanes of the group load one entry each, and the
+        // entries reach all lanes through the LDS crossbar.
+        const int group_lane0 = 4 * ((threadIdx.x % kWave) - lane);
+        int64_t fld[TILES];  // lanes beyond the width gather feature 0 again (never stored)
 #pragma unroll
-            for (int t = 0; t < TILES; ++t) fld[t] = foff[t] < 0 ? 0 : foff[t];
-            int my_row = 0, my_c = 0;
-            T my_w = T(1);
-            auto load_entry = [&](int e) {  // this lane's of the batch from e on
-                my_row = 0, my_c = 0, my_w = T(1);
-                if (e + lane >= e1) return;
-                my_row = row_at(e + lane);
-                my_c = col_at(e + lane);
-                if constexpr (MODE == MODE_DUAL) my_w = a.val[e + lane];
-                if constexpr (has_values(MODE)) my_w = a.val != nullptr ? a.val[e + lane] : T(1);
-            };
-            if constexpr (kAhead) load_entry(e0);
-            for (int e = e0; e < e1; e += LPR) {
-                if constexpr (!kAhead) load_entry(e);
-                if constexpr (MODE != MODE_DUAL) arrive(my_c), arrive(my_row);
-                if constexpr (has_values(MODE)) arrive(my_w);
-                int my_o = e + lane < e1 ? named(my_row) : 0;
-                if constexpr (kNamesRowsOfY) {
-                    // with every batch of entries, so that no load of the run waits for another but
-                    // the row numbers for their rows (the same two words each time)
-                    if constexpr (WGRUNS == WGRUNS_NONE) {
-                        last_row = a.rowidx[e1 - 1];
-                        row_behind = e1 < a.nnz ? a.rowidx[e1] : -1;
-                    }
-                    // the run begins with the row of its first entry
-                    if constexpr (!kRowsBehindGathers) {
-                        const int batch_first = __builtin_amdgcn_ds_bpermute(group_lane0, my_o);
-                        if (e == e0) cur_out = batch_first;
-                    }
-                }
-                const int cnt = min(e1 - e, LPR);
-                const int this_c = my_c;
-                const T this_w = my_w;
-                if constexpr (kAhead) load_entry(e + LPR);
-                for (int u0 = 0; u0 < cnt; u0 += ROUND) {
-                    int o[ROUND], c[ROUND];
-                    T w[ROUND];
-#pragma unroll
-                    for (int u = 0; u < ROUND; ++u) {
-                        const int from = group_lane0 + 4 * (u0 + u);
-                        if constexpr (!kRowsBehindGathers) o[u] = __builtin_amdgcn_ds_bpermute(from, my_o);
-                        c[u] = __builtin_amdgcn_ds_bpermute(from, this_c);
-                        if constexpr (has_values(MODE) || MODE == MODE_DUAL)
-                            w[u] = __builtin_bit_cast(T, __builtin_amdgcn_ds_bpermute(from, __builtin_bit_cast(int, this_w)));
-                        else
-                            w[u] = T(1);
-                    }
-                    // Lanes without an entry hold column 0 (a row of X like any other) and value 1, and
-                    // positions behind the last entry of a batch read those: a round may gather for them,
-                    // nothing is added for them.  Only a block without first-source columns sees such a
-                    // position as one of the second source, and takes the slower path for that round.
-                    bool second = false;
-                    if constexpr (MODE == MODE_DUAL) {
-#pragma unroll
-                        for (int u = 0; u < ROUND; ++u) second = second | (c[u] >= a.split);
-                    }
-                    auto gather_and_add = [&](auto plain) {
-                        constexpr bool kPlain = decltype(plain)::value;  // every entry from the first source
-                        Gathered<T, VEC, MODE> x[ROUND][TILES];
-                        // Up to 64 bytes per lane group and gather, a position behind the last entry gathers
-                        // like the others (column 0, see above): the branches around four small loads cost
-                        // more than the loads.  Wider rows skip it: there the extra row is what costs.
-                        constexpr bool kGatherAll = VEC * LPR * sizeof(T) <= 64;
-#pragma unroll
-                        for (int u = 0; u < ROUND; ++u)
-                            if (kGatherAll || u0 + u < cnt) {
-#pragma unroll
-                                for (int t = 0; t < TILES; ++t)
-                                    x[u][t] = gather<T, VEC, MODE, (int)(VEC * LPR * sizeof(T))>(a, c[u], kPlain ? 0 : c[u] >= a.split, fld[t]);
-                            }
-                        if constexpr (kRowsBehindGathers) {
-                            // the names of the rows are waited for behind the gathers, which do not need them
-                            if (u0 == 0) arrive(my_o);
-#pragma unroll
-                            for (int u = 0; u < ROUND; ++u) o[u] = __builtin_amdgcn_ds_bpermute(group_lane0 + 4 * (u0 + u), my_o);
-                            if (u0 == 0 && e == e0) {  // the run begins with the row of its first entry
-                                cur_out = o[0];
-                                begin_row(cur_out);
-                            }
-                        }
-                        if constexpr (MODE != MODE_DUAL && !(kGatherAll && !has_values(MODE)))
-#pragma unroll
-                            for (int u = 0; u < ROUND; ++u)
-#pragma unroll
-                                for (int t = 0; t < TILES; ++t) arrive(x[u][t]);
-#pragma unroll
-                        for (int u = 0; u < ROUND; ++u) {
-                            if (u0 + u < cnt) {
-                                if (o[u] != cur_out) {
-                                    // the row ends inside this run: finish it here
-                                    finish_row(row_of_y(cur_out), e + u0 + u);
-                                    row_e0 = e + u0 + u;
-                                    acc.clear();
-                                    cur_out = o[u];
-                                    begin_row(cur_out);
-                                }
-                                acc.add(x[u], fld, w[u], kPlain ? 0 : c[u] >= a.split);
-                            }
-                        }
-                    };
-                    if (MODE != MODE_DUAL || __ballot(second) == 0) gather_and_add(std::true_type{});
-                    else gather_and_add(std::false_type{});
-                }
-            }
-        } else {
+        for (int t = 0; t < TILES; ++t) fld[t] = foff[t] < 0 ? 0 : foff[t];
+        int my_row = 0, my_c = 0;
+        T my_w = T(1);
+        auto load_entry = [&](int e) {  // this lane's of the batch from e on
+            my_row = 0, my_c = 0, my_w = T(1);
+            if (e + lane >= e1) return;
+            my_row = row_at(e + lane);
+            my_c = col_at(e + lane);
+            if constexpr (MODE == MODE_DUAL) my_w = a.val[e + lane];
+            if constexpr (has_values(MODE)) my_w = a.val != nullptr ? a.val[e + lane] : T(1);
+        };
+        if constexpr (kAhead) load_entry(e0);
+        for (int e = e0; e < e1; e += LPR) {
+            if constexpr (!kAhead) load_entry(e);
+            if constexpr (MODE != MODE_DUAL) arrive(my_c), arrive(my_row);
+            if constexpr (has_values(MODE)) arrive(my_w);
+            int my_o = e + lane < e1 ? named(my_row) : 0;
             if constexpr (kNamesRowsOfY) {
-                cur_out = named(row_at(e0));
-                begin_row(cur_out);
+                // with every batch of entries, so that no load of the run waits for another but
+                // the row numbers for their rows (the same two words each time)
                 if constexpr (WGRUNS == WGRUNS_NONE) {
                     last_row = a.rowidx[e1 - 1];
                     row_behind = e1 < a.nnz ? a.rowidx[e1] : -1;
                 }
-            }
-            for (int e = e0; e < e1; e += kUnroll) {
-                int o[kUnroll], c[kUnroll];
-                T w[kUnroll];
-                Gathered<T, VEC, MODE> x[kUnroll][TILES];
-#pragma unroll
-                for (int u = 0; u < kUnroll; ++u) {
-                    const int idx = min(e + u, e1 - 1);
-                    o[u] = named(row_at(idx));
-                    c[u] = col_at(idx);
-                    if constexpr (MODE == MODE_DUAL) w[u] = a.val[idx];
-                    else if constexpr (has_values(MODE)) w[u] = a.val != nullptr ? a.val[idx] : T(1);
-                    else w[u] = T(1);
+                // the run begins with the row of its first entry
+                if constexpr (!kRowsBehindGathers) {
+                    const int batch_first = __builtin_amdgcn_ds_bpermute(group_lane0, my_o);
+                    if (e == e0) cur_out = batch_first;
                 }
+            }
+            const int cnt = min(e1 - e, LPR);
+            const int this_c = my_c;
+            const T this_w = my_w;
+            if constexpr (kAhead) load_entry(e + LPR);
+            for (int u0 = 0; u0 < cnt; u0 += ROUND) {
+                int o[ROUND], c[ROUND];
+                T w[ROUND];
 #pragma unroll
-                for (int u = 0; u < kUnroll; ++u)
-                    if (e + u < e1) {
+                for (int u = 0; u < ROUND; ++u) {
+                    const int from = group_lane0 + 4 * (u0 + u);
+                    if constexpr (!kRowsBehindGathers) o[u] = __builtin_amdgcn_ds_bpermute(from, my_o);
+                    c[u] = __builtin_amdgcn_ds_bpermute(from, this_c);
+                    if constexpr (has_values(MODE) || MODE == MODE_DUAL)
+                        w[u] = from_lane(from, this_w);
+                    else
+                        w[u] = T(1);
+                }
+                // Lanes without an entry hold column 0 (a row of X like any other) and value 1, and
+                // positions behind the last entry of a batch read those: a round may gather for them,
+                // nothing is added for them.  Only a block without first-source columns sees such a
+                // position as one of the second source, and takes the slower path for that round.
+                bool second = false;
+                if constexpr (MODE == MODE_DUAL) {
 #pragma unroll
-                        for (int t = 0; t < TILES; ++t)
-                            x[u][t] = gather<T, VEC, MODE, (int)(VEC * LPR * sizeof(T))>(a, c[u], c[u] >= a.split, foff[t]);
-                    }
+                    for (int u = 0; u < ROUND; ++u) second = second | (c[u] >= a.split);
+                }
+                auto gather_and_add = [&](auto plain) {
+                    constexpr bool kPlain = decltype(plain)::value;  // every entry from the first source
+                    Gathered<T, VEC, MODE> x[ROUND][TILES];
+                    // Up to 64 bytes per lane group and gather, a position behind the last entry gathers
+                    // like the others (column 0, see above): the branches around four small loads cost
+                    // more than the loads.  Wider rows skip it: there the extra row is what costs.
+                    constexpr bool kGatherAll = VEC * LPR * sizeof(T) <= 64;
 #pragma unroll
-                for (int u = 0; u < kUnroll; ++u) {
-                    if (e + u < e1) {
-                        if (o[u] != cur_out) {
-                            // the row ends inside this run: finish it here
-                            finish_row(row_of_y(cur_out), e + u);
-                            row_e0 = e + u;
-                            acc.clear();
-                            cur_out = o[u];
+                    for (int u = 0; u < ROUND; ++u)
+                        if (kGatherAll || u0 + u < cnt) {
+#pragma unroll
+                            for (int t = 0; t < TILES; ++t)
+                                x[u][t] = gather<T, VEC, MODE, (int)(VEC * LPR * sizeof(T))>(a, c[u], kPlain ? 0 : c[u] >= a.split, fld[t]);
+                        }
+                    if constexpr (kRowsBehindGathers) {
+                        // the names of the rows are waited for behind the gathers, which do not need them
+                        if (u0 == 0) arrive(my_o);
+#pragma unroll
+                        for (int u = 0; u < ROUND; ++u) o[u] = __builtin_amdgcn_ds_bpermute(group_lane0 + 4 * (u0 + u), my_o);
+                        if (u0 == 0 && e == e0) {  // the run begins with the row of its first entry
+                            cur_out = o[0];
                             begin_row(cur_out);
                         }
-                        acc.add(x[u], foff, w[u], c[u] >= a.split);
                     }
-                }
+                    if constexpr (MODE != MODE_DUAL && !(kGatherAll && !has_values(MODE)))
+#pragma unroll
+                        for (int u = 0; u < ROUND; ++u)
+#pragma unroll
+                            for (int t = 0; t < TILES; ++t) arrive(x[u][t]);
+#pragma unroll
+                    for (int u = 0; u < ROUND; ++u) {
+                        if (u0 + u < cnt) {
+                            if (o[u] != cur_out) {
+                                // the row ends inside this run: finish it here
+                                finish_row(row_of_y(cur_out), e + u0 + u);
+                                row_e0 = e + u0 + u;
+                                acc.clear();
+                                cur_out = o[u];
+                                begin_row(cur_out);
+                            }
+                            acc.add(x[u], fld, w[u], kPlain ? 0 : c[u] >= a.split);
+                        }
+                    }
+                };
+                if (MODE != MODE_DUAL || __ballot(second) == 0) gather_and_add(std::true_type{});
+                else gather_and_add(std::false_type{});
             }
         }
         if constexpr (WGRUNS == WGRUNS_NONE) {
