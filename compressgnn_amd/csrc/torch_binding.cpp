@@ -1426,15 +1426,16 @@ std::tuple<Tensor, Tensor> reconstruct_with_signs(const char *op, const Tensor &
     return {out, signs};
 }
 
-// cluster_reconstruct_backward with relu = true, the mask taken from the words above.
+// cluster_reconstruct_backward with relu = true, the mask taken from the words above.  room: there may be more rows of words
+// than are read.
 Tensor reconstruct_backward_with_signs(const char *op, const Tensor &grad, const Tensor &index, const Tensor &signs, int64_t groups,
-                                       const c10::optional<std::vector<Tensor>> &members, bool by_group) {
+                                       const c10::optional<std::vector<Tensor>> &members, bool by_group, bool room = false) {
     expect(op, grad, {{Role::Features, "grad", &grad}, {Role::Ids, "index", &index}});
     TORCH_CHECK(groups >= 0, op, ": groups = ", groups);
     TORCH_CHECK(index.numel() == grad.size(0), op, ": ", grad.size(0), " rows but ", index.numel(), " cluster ids");
     const int64_t N = grad.size(0), F = grad.size(1), of = by_group ? groups : N;
     TORCH_CHECK(signs.device() == grad.device() && signs.scalar_type() == torch::kInt32 && signs.is_contiguous() &&
-                    signs.dim() == 2 && signs.size(0) == of && signs.size(1) == cgnn_sign_words(F),
+                    signs.dim() == 2 && (room ? signs.size(0) >= of : signs.size(0) == of) && signs.size(1) == cgnn_sign_words(F),
                 op, by_group ? ": masks" : ": signs", " must be a contiguous int32 tensor [", of, ", ", cgnn_sign_words(F),
                 "] on the device of grad");
     c10::hip::HIPGuardMasqueradingAsCUDA guard(grad.device());
@@ -1575,7 +1576,8 @@ struct ReconstructBackward : torch::autograd::Node {
             at::NoGradGuard no_grad;
             const Tensor d_rows = grads[0].contiguous(), ids = index.unpack();
             // without a ReLU the operator does not read the rows it is given as output
-            out.push_back(relu ? cluster_reconstruct_backward_masks(d_rows, ids, masks.unpack().narrow(0, 0, groups), groups, members)
+            out.push_back(relu ? reconstruct_backward_with_signs("cluster_reconstruct_backward_masks", d_rows, ids, masks.unpack(), groups,
+                                                                 members, true, true)
                                : cluster_reconstruct_backward(d_rows, ids, d_rows, groups, false, members));
             if (with_bias) out.push_back(task_should_compute_output(1) ? column_sums(out[0]) : Tensor());
         }
