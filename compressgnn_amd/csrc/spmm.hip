@@ -1500,8 +1500,14 @@ struct Shape {
 // wave walks 16 runs at once, each with its own row changes (F = 16: 0.106 -> 0.089 ms for the forward
 // vertex stage of the web graph) -- and so takes the narrowest packs that 16 lanes hold.
 // The row schedule is faster with the widest packs (0.036 against 0.053 ms).
+// two_tiles: rows beyond 64 packs as two tiles of one launch's lanes, which read every entry once for both; otherwise a part of
+// the launch per 64 packs, with fewer registers, more waves and half as wide a working set in the L2s.  That is taken by
+// default where it leaves no lane idle (forward, 512 features, two tiles / so: web graphs of 6,000 vertices 25.5 / 22.6 us, 100,003
+// 301 / 292, 325,557 926 / 914; 1,024 features over 20,000 125 / 119); where lanes idle two tiles stay (264 features over 325,557
+// vertices, forward + gradient 940 / 1,168, 400 1,198 / 1,310).  Rows of few entries cost more than they save in parts
+// (row_shape), and so does the search of a small product of int64 arrays (once_layout).
 template <typename T>
-Shape pick_shape(int64_t F, bool runs) {
+Shape pick_shape(int64_t F, bool runs, bool two_tiles = false) {
     Shape s;
     s.vec = 1;
     if (sizeof(T) == 4) {
@@ -1518,7 +1524,7 @@ Shape pick_shape(int64_t F, bool runs) {
         lpr = lpr <= 4 ? 4 : (lpr <= 16 ? 16 : 64);
     }
     s.lpr = lpr;
-    s.tiles = (lpr == 64 && slots > 64 && sizeof(T) == 4) ? 2 : 1;
+    s.tiles = (lpr == 64 && slots > 64 && sizeof(T) == 4 && (two_tiles || slots % 64 != 0)) ? 2 : 1;
     s.grid_y = (int)ceil_div(slots, (int64_t)s.lpr * s.tiles);
     return s;
 }
@@ -1831,8 +1837,10 @@ int most_per_new_run(const cgnn_csr *A) { return 2 * seg_len(A); }
 constexpr int64_t kResidentLanes = 256 * 32 * kWave;
 
 template <typename T>
-Shape row_shape(int64_t F, int64_t rows, int32_t max_row_nnz) {
-    const Shape wide = pick_shape<T>(F, false);
+Shape row_shape(int64_t F, int64_t rows, int64_t nnz, int32_t max_row_nnz) {
+    // parts of 64 packs for rows of eight entries and more (gradient, 512 features, two tiles / parts: 325,557 vertices of 10.8
+    // entries 567 / 551 us, 200,003 of 8 277 / 280, of 5 226 / 238)
+    const Shape wide = pick_shape<T>(F, false, nnz < 8 * rows);
     if (sizeof(T) != 4 || wide.tiles != 1 || wide.grid_y != 1) return wide;
     Shape s = wide;
     s.vec = F <= kWave ? 1 : (F <= 2 * kWave ? 2 : 4);
@@ -1862,7 +1870,7 @@ int spmm_typed(const cgnn_csr *A, const void *X, const void *X1, int64_t split, 
     if (mode == MODE_DUAL && A->nnz > 0 && A->val == nullptr)
         return fail(CGNN_EINVAL, "spmm: the two-source product needs stored values");
     if (kernel == CGNN_SPMM_ROW) {
-        const Shape s = row_shape<T>(F, A->rows, A->max_row_nnz);
+        const Shape s = row_shape<T>(F, A->rows, A->nnz, A->max_row_nnz);
         return launch<T>(KIND_ROW, mode, s, a, A->rows, stream);
     }
     if (A->nnz > 0 && A->rowidx == nullptr) return fail(CGNN_EINVAL, "spmm: nnz schedule needs rowidx");
@@ -2270,6 +2278,7 @@ extern "C" int cgnn_spmm_run_length(const cgnn_csr *A) { return A == nullptr ? 0
 namespace {
 
 struct OnceLayout {
+    Shape shape;
     int groups, wg_len;
     int64_t workgroups;
     size_t total;  // the pieces
@@ -2281,7 +2290,10 @@ OnceLayout once_layout(int64_t rows, int64_t nnz, int64_t F, int dtype) {
     A.nnz = nnz;
     A.seg_nnz = 32;  // as for the blocks of a plan
     OnceLayout L;
-    L.groups = kBlock / shape_of(F, dtype).lpr;
+    // 512 features, two tiles / parts: out-lists of 6,000 vertices 14.6 / 19.5 us, of 20,000 38.9 / 36.7, 325,557 814 / 745
+    const bool two_tiles = nnz < (1 << 17);
+    L.shape = dtype == CGNN_F64 ? pick_shape<double>(F, true, two_tiles) : pick_shape<float>(F, true, two_tiles);
+    L.groups = kBlock / L.shape.lpr;
     L.wg_len = wg_run_len(&A, L.groups, most_per_new_run(&A)) * L.groups;
     L.workgroups = ceil_div(nnz, L.wg_len);
     L.total = wg_piece_bytes(L.workgroups, F, dtype == CGNN_F64 ? 8 : 4);
@@ -2303,7 +2315,7 @@ int spmm_once(const OnceLayout &L, int64_t rows, int64_t nnz, const int64_t *row
     a.keep = kDefaultSeg;
     a.nseg = (int32_t)(L.workgroups * L.groups);
     a.carry = static_cast<T *>(workspace);
-    return launch<T>(KIND_NNZ, MODE_VAL, pick_shape<T>(F, true), a, a.nseg, stream);
+    return launch<T>(KIND_NNZ, MODE_VAL, L.shape, a, a.nseg, stream);
 }
 
 }  // namespace
@@ -2312,7 +2324,7 @@ extern "C" size_t cgnn_spmm_once_workspace_bytes(int64_t rows, int64_t nnz, int6
     if (arrivals) *arrivals = 0;
     if (rows <= 0 || nnz <= 0 || F <= 0) return 0;
     const OnceLayout L = once_layout(rows, nnz, F, dtype);
-    if (arrivals) *arrivals = L.workgroups * shape_of(F, dtype).grid_y;
+    if (arrivals) *arrivals = L.workgroups * L.shape.grid_y;
     return L.total;
 }
 

@@ -1327,7 +1327,7 @@ def test_other_threads_run_while_a_call_waits_for_the_stream(call):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
-@pytest.mark.parametrize("width", [1, 3, 16, 33, 64, 130, 200, 520, 1030])
+@pytest.mark.parametrize("width", [1, 3, 16, 33, 64, 130, 200, 512, 520, 1030])
 def test_products_of_int64_arrays_of_every_shape(width, dtype):
     """spmm_func looks for the rows of a workgroup's entries itself: numbers of rows around a step of the search and around what
     the workgroup reads of them at once, rows without entries in front, between and behind, rows at the lengths that are moved
