@@ -81,7 +81,7 @@ struct Merger {
     uint64_t *taken;                   // [L / 64] taken by a rule
     int32_t *word_sum;                 // [L / 64] taken positions of the tile in front of a word
     int32_t *children;
-    int32_t *scalar;                   // [kScalars]
+    int32_t *scalar;                   // [kScalars], and the counters of arrives_last, a line each
     int32_t *host, flag;               // pinned memory for the scalars and this flag behind them, or NULL
 };
 
@@ -166,9 +166,13 @@ __global__ __launch_bounds__(kScanBlock) void merger_tile_sums_kernel(int32_t *_
 // What the last workgroup to get here may do for the others instead of a launch behind them (3 to 5 us of the device and as
 // much of the host; 14,530 vertices of degree 8.9 at a frequency of 4, twenty launches a round 636 us a call, sixteen 583; 14,163
 // of 13 at 16 480, 456): true in that one, for all its threads.  What the others have left is past their L2s -- stored with
-// store_now or added with an atomic -- and read with load_now: a release would write back the whole L2.  The arrivals come one
-// after the other, some 12 ns each, so this is for launches of up to kFew workgroups (1,600: 32 us instead of 12).
-constexpr unsigned kFew = 256;
+// store_now or added with an atomic -- and read with load_now: a release would write back the whole L2.  Arrivals at one counter come
+// one after the other, some 12 ns each (1,600: 32 us for a launch of 12), so more than kFew workgroups arrive at one of
+// kArrivalGroups counters first, and the last one there at the one for all.  Beyond kMany the launches behind stay.  (With the
+// launches / one counter up to kFew / so: 121,075 vertices of degree 10.2 at a frequency of 4 1,234 / 1,199 / 1,181 us a call,
+// 325,557 of 9.8 at 16 1,361 / 1,341 / 1,330.)
+constexpr unsigned kFew = 256, kArrivalGroups = 16, kMany = kFew * kArrivalGroups;
+constexpr int kLine = 32;  // integers of a cache line
 __device__ __forceinline__ void store_now(int32_t *p, int32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 __device__ __forceinline__ bool arrives_last(const Merger &m, Arrival at) {
@@ -177,8 +181,13 @@ __device__ __forceinline__ bool arrives_last(const Merger &m, Arrival at) {
     __builtin_amdgcn_s_waitcnt(0);  // of every wave: its stores have arrived
     __syncthreads();
     if (threadIdx.x == 0) {
-        const int32_t before = __hip_atomic_fetch_add(m.scalar + kArrived + at, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        last = before == (int32_t)gridDim.x - 1;
+        auto completes = [](int32_t *count, unsigned of) {
+            return __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int32_t)of - 1;
+        };
+        const unsigned g = blockIdx.x % kArrivalGroups;
+        last = (gridDim.x <= kFew || completes(m.scalar + kScalars + (at * kArrivalGroups + g) * kLine,
+                                               (gridDim.x - g + kArrivalGroups - 1) / kArrivalGroups)) &&
+               completes(m.scalar + kArrived + at, gridDim.x <= kFew ? gridDim.x : kArrivalGroups);
     }
     __syncthreads();
     return last;
@@ -230,6 +239,7 @@ __global__ void merger_begin_kernel(Merger m) {
         for (int i = 0; i < 3; ++i) m.scalar[kArrived + i] = 0;
         if (m.first) m.scalar[kBad] = 0;
     }
+    if (blockIdx.x == 0 && threadIdx.x < 3 * kArrivalGroups) m.scalar[kScalars + threadIdx.x * kLine] = 0;
 }
 
 // A counter goes up unless it got to min_frequency, as far as the caller has seen.
@@ -326,7 +336,7 @@ __global__ __launch_bounds__(kBlock) void merger_pass_kernel(Merger m, bool clea
         store_now(m.tile + blockIdx.x, all);
     }
     if (clear) clear_table(m, (int64_t)1 << table_bits(m.most));
-    if (gridDim.x > kFew || !arrives_last(m, kPassed)) return;
+    if (gridDim.x > kMany || !arrives_last(m, kPassed)) return;
     const int all = scan_tiles<kBlock, true>(m.tile, (int32_t)gridDim.x);
     if (threadIdx.x == 0) m.scalar[kListed] = all;
 }
@@ -401,7 +411,7 @@ __global__ __launch_bounds__(kBlock) void merger_candidates_kernel(Merger m) {
         }
         __syncthreads();
     }
-    if (m.host != nullptr && gridDim.x <= kFew && arrives_last(m, kCounted) && threadIdx.x == 0) publish(m.scalar, m.host, m.flag);
+    if (m.host != nullptr && gridDim.x <= kMany && arrives_last(m, kCounted) && threadIdx.x == 0) publish(m.scalar, m.host, m.flag);
 }
 
 // Ranks of a few candidates: a workgroup compares kBlock of them with kBlock others.
@@ -596,7 +606,7 @@ __global__ __launch_bounds__(kBlock) void merger_taken_sums_kernel(Merger m, int
         m.word_sum[w] = sum - count;
         if (lane == kTileWords - 1) store_now(m.tile + w / kTileWords, sum);
     }
-    if (gridDim.x > kFew || !arrives_last(m, kTaken)) return;
+    if (gridDim.x > kMany || !arrives_last(m, kTaken)) return;
     const int all = scan_tiles<kBlock, true>(m.tile, (int32_t)(words / kTileWords));
     if (threadIdx.x == 0) {
         store_now(m.scalar + kTakenTotal, all);
@@ -710,7 +720,7 @@ MergerWorkspace merger_workspace(int64_t V, int64_t E) {
     w.sorted_key = take(c * 8);
     for (auto *a : {&w.cand_slot, &w.sorted_slot, &w.cand_rank, &w.use, &w.rule_of}) *a = take(c * 4);
     w.children = take(n * 4);
-    w.scalars = take(kScalars * 4);
+    w.scalars = take((kScalars + 3 * kArrivalGroups * kLine) * 4);
     hipcub::DeviceRadixSort::SortPairs(nullptr, w.temp_bytes, (const uint64_t *)nullptr, (uint64_t *)nullptr,
                                        (const int32_t *)nullptr, (int32_t *)nullptr, (int)c, 0, 64, 0);
     w.temp = take(w.temp_bytes);
@@ -844,14 +854,14 @@ int merger_rounds(int64_t V, int64_t E, int rounds, int min_pair_frequency, int3
         const int64_t slots = (int64_t)1 << bits_of(m.most);
         const bool clear_here = slots <= kClearedAhead;
         hipLaunchKernelGGL(merger_pass_kernel, grid, block, 0, stream, m, clear_here);
-        if (grid.x > kFew)
+        if (grid.x > kMany)
             hipLaunchKernelGGL(merger_tile_sums_kernel, dim3(1), dim3(kScanBlock), 0, stream, m.tile, tiles, m.scalar + kListed);
         if (!clear_here) hipLaunchKernelGGL(merger_clear_table_kernel, dim3(merger_grid(slots / 2)), block, 0, stream, m);
         hipLaunchKernelGGL(merger_collect_kernel, grid, block, 0, stream, m);
         m.flag = ++reads;
         const dim3 table(tiles_of(slots));
         hipLaunchKernelGGL(merger_candidates_kernel, table, block, 0, stream, m);
-        if (table.x > kFew) publish_now();
+        if (table.x > kMany) publish_now();
         if ((err = read()) != hipSuccess) return merger_fail(err, "reading the candidate count");
         if (!checked && host[kBad])
             return fail(CGNN_EINVAL, "cgnn_compress_csr_batch_device: malformed CSR (row starts or columns out of range)");
@@ -887,7 +897,7 @@ int merger_rounds(int64_t V, int64_t E, int rounds, int min_pair_frequency, int3
         m.flag = ++reads;
         const dim3 maps((unsigned)ceil_div(words, kBlock));
         hipLaunchKernelGGL(merger_taken_sums_kernel, maps, block, 0, stream, m, words);
-        if (maps.x > kFew) {
+        if (maps.x > kMany) {
             hipLaunchKernelGGL(merger_tile_sums_kernel, dim3(1), dim3(kScanBlock), 0, stream, m.tile, tiles, m.scalar + kTakenTotal);
             publish_now();
         }

@@ -146,7 +146,8 @@ def test_gpu_compressor_at_the_edges_of_its_tiles(entries, freq):
     assert all(np.array_equal(a, b) for a, b in zip(got, both(v.astype(np.int32), e.astype(np.int32), 12, freq)))
 
 
-@pytest.mark.parametrize("entries, freq", [((1 << 20) - 1, 16), (1 << 20, 16), (1 << 22, 64), ((1 << 22) + 1, 64)])
+@pytest.mark.parametrize("entries, freq", [((1 << 20) - 1, 16), (1 << 20, 16), (1 << 22, 64), ((1 << 22) + 1, 64),
+                                           (1 << 23, 64), ((1 << 23) + 1, 64)])
 def test_gpu_compressor_where_launches_grow_too_large_for_their_last_workgroup(entries, freq):
     """Around the lengths from which tables are cleared by a launch of their own, and sums over the tiles are one."""
     test_gpu_compressor_at_the_edges_of_its_tiles(entries, freq)
