@@ -593,10 +593,17 @@ inline __host__ __device__ int32_t once_room(int32_t wg_len, int32_t keep) { ret
 // In place of a launch that made int32 arrays of the block, which the product then waited for: that cost 7.5 us, the launch
 // boundary, and five dependent loads in front of a run (two now, of lines just read).  Web graphs, us, in-lists and out-lists,
 // before / so: 6,000 vertices of 16 features 16.9 / 13.9 and 11.9 / 8.7, 50,001 of 16 23.5 / 19.3 and 21.8 / 15.9, 100,003 of 64
-// 52.3 / 45.4 and 36.4 / 29.4, 325,557 of 128 264 / 253 and 197 / 181, of 8, whose few workgroups hold 2,048 entries each, 83.5 /
-// 82.9 and 72.2 / 63.2.  A search for each end of a stretch, down to the row, instead: in-lists of 325,557 vertices 266 us at
+// 52.3 / 45.4 and 36.4 / 29.4, 325,557 of 128 264 / 253 and 197 / 181, of 8, 512 entries a workgroup, 83.5 / 82.9 and 72.2 /
+// 63.2.  A search for each end of a stretch, down to the row, instead: in-lists of 325,557 vertices 266 us at
 // 128 features; 16 row pointers a step 278.
 constexpr int kNear = kBlock / 2;
+// From this many rows between the two ends on (rows without entries, which may be any number) the rows are found from the entries,
+// a search of them for each: a step of the walk over the rows waits for the one before, a search takes as many steps as the number of
+// rows has bits.  us, all rows walked / so: 10^5 entries on both sides of 987,500 empty rows, 64 features 1,450 / 38; 1,000 in
+// 10^6 rows at random, 1 feature 720 / 13; in-lists of 325,557 vertices of degree 1, 8 features 43 / 23.5, of degree 3 43.5 / 32.
+// Lower bounds (two, four, eight steps) gain nothing there, and eight cost in-lists of 100,003 vertices of degree 9.8 1.5 % at
+// 64 features.
+constexpr int kWalked = 16 * kBlock;
 __device__ __forceinline__ int search_step(int rows) { return (rows + kWave - 1) / kWave; }
 
 template <typename T>
@@ -657,6 +664,26 @@ __device__ __forceinline__ void once_stretch(const SpmmArgs<T> &a, const WideRow
     };
     begin = begin_of(places[0], r0), behind = begin_of(places[1], r1);
     const int32_t b0 = begin & ~kRowGoesOn, count = min((behind & ~kRowGoesOn) - b0, room);
+    if (r1 - r0 >= kWalked) {
+        constexpr int kAtOnce = 4;  // a thread's searches, whose loads do not wait for each other
+        for (int k = threadIdx.x; k < count; k += kAtOnce * kBlock) {
+            int lo[kAtOnce], hi[kAtOnce];
+#pragma unroll
+            for (int u = 0; u < kAtOnce; ++u) lo[u] = r0, hi[u] = r1 + 1;  // as from and to
+            for (int span = r1 + 1 - r0; span > 1; span -= span / 2)
+#pragma unroll
+                for (int u = 0; u < kAtOnce; ++u) {
+                    const int mid = lo[u] + (hi[u] - lo[u]) / 2;
+                    if (rows.at(mid) <= b0 + min(k + u * kBlock, count - 1)) lo[u] = mid;
+                    else hi[u] = max(mid, lo[u] + 1);
+                }
+#pragma unroll
+            for (int u = 0; u < kAtOnce; ++u)
+                if (k + u * kBlock < count) row_of[k + u * kBlock] = lo[u];
+        }
+        __syncthreads();
+        return;
+    }
     while (r <= r1) {  // r1 < rows
         // rows without entries begin where another does: not marked, so one row a mark
         if (r > r0 && e > s && s > b0 && s - b0 < count) row_of[s - b0] = (int)r;
@@ -890,10 +917,11 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
     bool continues = false;    // the last row of the run goes on in the next one
     bool open = false;         // WGRUNS: the row at hand began before the run
     int32_t wg_begin = 0, wg_behind = 0;
-    // WGRUNS_ONCE: every wave looks at an equal share of the rows for those without entries, which are neighbours (the youngest
-    // vertices of a graph's in-lists): zero_rows consecutive ones at a time (64 a wave, so that some have many and most
-    // none: in-lists of 325,557 vertices 282 us at 128 features, 253 so).
-    const int zero_rows = (int)min((int64_t)kWave, (a.rows + (int64_t)a.blocks * (kBlock / kWave) - 1) / ((int64_t)a.blocks * (kBlock / kWave)));
+    // WGRUNS_ONCE: every wave, those without entries of their own among them (kZeroWorkgroups), looks at an equal share of the rows
+    // for those without entries, which are neighbours (the youngest vertices of a graph's in-lists): zero_rows consecutive ones
+    // at a time (64 a wave, so that some have many and most none: in-lists of 325,557 vertices 282 us at 128 features, 253 so).
+    const int64_t waves = (int64_t)gridDim.x * (kBlock / kWave);
+    const int zero_rows = (int)min((int64_t)kWave, (a.rows + waves - 1) / waves);
     const int64_t zero_row0 = ((int64_t)block * (kBlock / kWave) + threadIdx.x / kWave) * zero_rows;
     if constexpr (WGRUNS == WGRUNS_ONCE) {
         const int64_t held = a.nnz, looked_at = zero_row0 + threadIdx.x % kWave;
@@ -903,10 +931,10 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
         wide.first = max((int64_t)0, min(held, a.rowptr64[0]));
         wide.last = max(wide.first, min(held, a.rowptr64[a.rows]));
         if constexpr (MODE != MODE_ADD)
-            empties = __ballot(block < a.blocks && (int)(threadIdx.x % kWave) < zero_rows && looked_at < a.rows && min(p, wide.last) >= max(q, wide.first));
+            empties = __ballot((int)(threadIdx.x % kWave) < zero_rows && looked_at < a.rows && min(p, wide.last) >= max(q, wide.first));
         if (a.val != nullptr) a.val += wide.first;
         a.col64 += wide.first;
-        once_stretch(a, wide, block, pivot, row_of, wg_begin, wg_behind);
+        if (block < a.blocks) once_stretch(a, wide, block, pivot, row_of, wg_begin, wg_behind);
         wg_begin = __builtin_amdgcn_readfirstlane(wg_begin), wg_behind = __builtin_amdgcn_readfirstlane(wg_behind);  // no vector registers
         const int32_t first = wg_begin & ~kRowGoesOn, end = wg_behind & ~kRowGoesOn;
         const int run_len = a.wg_len / GPB, whole = run_len > a.keep ? run_len : a.keep;
@@ -1117,15 +1145,20 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
     if constexpr (WGRUNS != WGRUNS_NONE) {
         if constexpr (WGRUNS == WGRUNS_TABLE)
             if (seg < a.nseg) wg_begin = a.run_start[block * GPB], wg_behind = a.run_start[(block + 1) * GPB];
-        if constexpr (WGRUNS == WGRUNS_ONCE && MODE != MODE_ADD) {  // rows without entries, a wave per row
+        if constexpr (WGRUNS == WGRUNS_ONCE && MODE != MODE_ADD) {  // rows without entries, a wave per stretch of neighbours
+            Pack<T, VEC> zero;
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) zero.v[i] = T(0);
             for (int64_t row0 = zero_row0;;) {
-                for (; empties != 0; empties &= empties - 1) {
-                    T *y = a.Y + (row0 + __ffsll(empties) - 1) * a.F;
-                    if (blockIdx.y == 0)
-                        for (int64_t f = threadIdx.x % kWave; f < a.F; f += kWave) y[f] = T(0);
+                while (empties != 0 && blockIdx.y == 0) {
+                    const int at = __ffsll(empties) - 1, behind = __ffsll(~(empties >> at)) - 1, n = behind < 0 ? kWave : behind;
+                    T *y = a.Y + (row0 + at) * a.F;
+                    for (int64_t i = (int64_t)VEC * (threadIdx.x % kWave), all = n * a.F; i < all; i += VEC * kWave)
+                        store_pack<T, VEC>(y + min(i, all - VEC), zero);
+                    empties = n == kWave ? 0 : empties & ~(((1ull << n) - 1) << at);
                 }
-                row0 += (int64_t)a.blocks * (kBlock / kWave) * zero_rows;
-                if (block >= a.blocks || row0 >= a.rows) break;
+                row0 += waves * zero_rows;
+                if (row0 >= a.rows) break;
                 const int64_t r = row0 + threadIdx.x % kWave;
                 empties = __ballot((int)(threadIdx.x % kWave) < zero_rows && r < a.rows && wide.at(min((int64_t)a.rows - 1, r)) >= wide.at(min((int64_t)a.rows, r + 1)));
             }
@@ -1630,6 +1663,12 @@ void launch_nnz(int mode, const SpmmArgs<T> &a, dim3 grid, hipStream_t stream) {
     }
 }
 
+// Products of int64 arrays that write rows without entries have at least a workgroup per kBlock rows, up to this many (as many as the
+// card holds at once), however few the entries are (1,000 entries in 10^6 rows, us, with the workgroups of the entries alone / so: 1
+// feature 12,500 / 13, 8 3,000 / 19, 64 2,660 / 43; a fill of the result takes 6 at 8 features, 32 at 64).  Plain stores:
+// streaming ones took 49 for 36 at 64 features over 10^6 rows.
+constexpr int kZeroWorkgroups = 2048;
+
 template <typename T, int VEC, int LPR, int TILES>
 int launch_shape(int kind, int mode, const SpmmArgs<T> &args, int64_t items, int grid_y, hipStream_t stream) {
     constexpr int GPB = kBlock / LPR;
@@ -1641,6 +1680,8 @@ int launch_shape(int kind, int mode, const SpmmArgs<T> &args, int64_t items, int
         a.stretch_log2 = stretch_log2_for<GPB>(grid.x);
         a.blocks = (int32_t)grid.x;
         grid.x = (unsigned)(ceil_div((int64_t)grid.x, kXcds) * kXcds);
+        if (a.rowptr64 != nullptr && !a.accumulate)
+            grid.x = std::max(grid.x, (unsigned)std::min<int64_t>(kZeroWorkgroups, ceil_div((int64_t)a.rows, kBlock)));
     }
     switch (kind) {
         case KIND_ROW:

@@ -1359,3 +1359,66 @@ def test_products_of_int64_arrays_of_every_shape(width, dtype):
         assert torch.equal(rt.spmm_func(ptr, e, w, x, "auto", base.clone()), base + want)
     nothing = torch.full((1000,), 40, device=DEV, dtype=torch.int64)  # a slice whose rows are all empty
     assert not rt.spmm_func(nothing, e, w, x, "auto", None).any()
+
+
+def rows_with_entries(rows, taken, rng, cols=300):
+    """Row pointers and columns of a block: taken = {row: entries}, all other rows without entries."""
+    lens = np.zeros(rows, np.int64)
+    for row, n in taken.items():
+        lens[row] = n
+    v = np.concatenate([[0], np.cumsum(lens)])
+    return lens, torch.from_numpy(v).to(DEV), torch.from_numpy(rng.integers(0, cols, int(v[-1]))).to(DEV)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("width", [1, 8, 33, 200, 512])
+def test_products_of_int64_arrays_with_stretches_of_empty_rows(width, dtype):
+    """Rows without entries between those of one workgroup, around the number from which the rows are found from the entries, in
+    blocks with fewer and with more workgroups of entries than of rows to clear.  Whole numbers: the sums are exact in any order."""
+    import compressgnn_runtime as rt
+    rng = np.random.default_rng(width)
+    blocks = [(gap + 2, {0: 3, gap + 1: 2}) for gap in (1790, 2045, 2046, 2047, 2048, 2049, 2304, 40000)]
+    blocks += [(90000, {int(r): int(n) for r, n in zip(rng.choice(90000, 700, replace=False), rng.integers(1, 9, 700))}),
+               (90000, {**{r: 5 for r in range(300)}, **{90000 - 1 - r: 70 for r in range(300)}}),
+               (9000, {**{r: 1 for r in range(0, 9000, 5)}, 4500: 3000}), (70000, {1: 64, 35000: 65, 69998: 2000}),
+               (600000 if width <= 33 else 60000, {0: 1})]
+    for rows, taken in blocks:
+        lens, v, e = rows_with_entries(rows, taken, rng)
+        w = torch.from_numpy(rng.integers(-3, 4, len(e))).to(DEV).to(dtype)
+        x = torch.from_numpy(rng.integers(-8, 9, (300, width))).to(DEV).to(dtype)
+        at = torch.from_numpy(np.repeat(np.arange(rows), lens)).to(DEV)
+        want = torch.zeros(rows, width, device=DEV, dtype=dtype).index_add_(0, at, x[e] * w[:, None])
+        for _ in range(2):
+            torch.full((rows, width), float("nan"), device=DEV, dtype=dtype)  # what the result may be given the memory of
+            assert torch.equal(rt.spmm_func(v, e, w, x, "auto", None), want)
+        base = torch.from_numpy(rng.integers(-9, 9, (rows, width))).to(DEV).to(dtype)
+        assert torch.equal(rt.spmm_func(v, e, w, x, "auto", base.clone()), base + want)
+
+
+@pytest.mark.parametrize("width", [1, 64])
+def test_products_of_int64_arrays_are_not_held_up_by_empty_rows(width):
+    """10^6 rows without entries: in the middle of 10^5 entries they cost what they cost behind them, and with few
+    entries, whose workgroups are few, no more than with a million.  Four times as long is allowed; a workgroup that walks the rows
+    between its entries, or few that clear all rows, take 20 times as long and more."""
+    import compressgnn_runtime as rt
+    rng = np.random.default_rng(1)
+    rows, half = 1000003, 6250
+
+    def time_of(taken):
+        _, v, e = rows_with_entries(rows, taken, rng)
+        w, x = torch.ones(len(e), device=DEV), torch.ones(300, width, device=DEV)
+        times = []
+        for _ in range(9):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            begin.record()
+            for _ in range(4):
+                rt.spmm_func(v, e, w, x, "auto", None)
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end))
+        return sorted(times)[4]
+
+    behind = time_of({r: 8 for r in range(2 * half)})
+    between = time_of({**{r: 8 for r in range(half)}, **{rows - 1 - r: 8 for r in range(half)}})
+    many, few = time_of({r: 1 for r in range(rows)}), time_of({r: 8 for r in range(125)})
+    assert between < 4 * behind and few < 4 * many, (behind, between, many, few)
