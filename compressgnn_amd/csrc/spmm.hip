@@ -2332,10 +2332,22 @@ OnceLayout once_layout(int64_t rows, int64_t nnz, int64_t F, int dtype) {
     A.seg_nnz = 32;  // as for the blocks of a plan
     OnceLayout L;
     // 512 features, two tiles / parts: out-lists of 6,000 vertices 14.6 / 19.5 us, of 20,000 38.9 / 36.7, 325,557 814 / 745
-    const bool two_tiles = nnz < (1 << 17);
+    const bool two_tiles = nnz < (1 << 17);  // a small product
     L.shape = dtype == CGNN_F64 ? pick_shape<double>(F, true, two_tiles) : pick_shape<float>(F, true, two_tiles);
     L.groups = kBlock / L.shape.lpr;
-    L.wg_len = wg_run_len(&A, L.groups, most_per_new_run(&A)) * L.groups;
+    int run = wg_run_len(&A, L.groups, most_per_new_run(&A));
+    // Floats beyond 256 features (a part of the launch per 64 packs or twice that): every part looks for the rows of its entries,
+    // and the parts fill the card together, so runs are as long as that asks for, up to 64 entries of one feature a lane.  Of wider
+    // packs only in small products, where runs would be shortest: in larger ones the search is little beside rows of 1 KB.
+    // (In-lists and out-lists, us, runs that fill the card with one part / so: 5,000 vertices of 257 features 33.6 / 21.9 and
+    // 26.2 / 18.2, of 602 38.6 / 29.7 and 29.9 / 22.9, of 2,048 67 / 67 and 44.8 / 36.4, of 4,096 123 / 115 and 82 / 63; 100,003 of
+    // 513 439 / 409 and 375 / 314; 325,557 of 257 874 / 780 and 750 / 638.  Up to 32 entries whatever the packs: 20,000 vertices
+    // of degree 3 and 2,048 features 63.9 / 68.9; 64 in larger products, too: 20,000 of degree 9.8 and 602 features 85 / 96.)
+    if (dtype == CGNN_F32 && L.shape.grid_y > 1 && (L.shape.vec == 1 || two_tiles)) {
+        const int64_t fill = ceil_div(ceil_div(nnz * L.shape.grid_y, kResidentWorkgroups * L.groups), kUnroll) * kUnroll;
+        run = std::max(run, (int)std::min<int64_t>(fill, 64 / L.shape.vec));
+    }
+    L.wg_len = run * L.groups;
     L.workgroups = ceil_div(nnz, L.wg_len);
     L.total = wg_piece_bytes(L.workgroups, F, dtype == CGNN_F64 ? 8 : 4);
     return L;

@@ -55,6 +55,22 @@ def test_argument_checks_without_a_gpu():
     assert lib.cgnn_lsh_scan_workspace_bytes(16) >= 64
 
 
+@pytest.mark.parametrize("F,nnz,double,parts,groups,run", [
+    (257, 49784, False, 3, 4, 24), (513, 985767, False, 5, 4, 64), (602, 49784, False, 3, 4, 24), (4096, 49784, False, 8, 4, 16),
+    (2048, 131071, False, 4, 4, 20), (2048, 131072, False, 8, 4, 20), (602, 985767, False, 3, 4, 32), (602, 1000, False, 3, 4, 8),
+    (256, 49784, False, 1, 4, 8), (512, 49784, False, 1, 4, 8), (768, 985767, False, 3, 4, 32), (256, 49784, True, 4, 4, 8),
+    (64, 985767, False, 1, 16, 36)])
+def test_entries_per_workgroup_of_products_of_int64_arrays(F, nnz, double, parts, groups, run):
+    """Every part of a wide product looks for the rows of its entries: runs are counted for the parts together, where a search
+    costs much beside what it is for."""
+    from compressgnn_amd import abi
+    arrivals = ctypes.c_int64(-1)
+    total = abi.lib().cgnn_spmm_once_workspace_bytes(abi.i64(1000), abi.i64(nnz), abi.i64(F), int(double), ctypes.byref(arrivals))
+    workgroups = -(-nnz // (groups * run))
+    assert arrivals.value == workgroups * parts
+    assert total == 2 * workgroups * F * (8 if double else 4)
+
+
 def test_runtime_module_has_the_reference_operator_names():
     import compressgnn_runtime as rt
     for name in ["spmm_func", "cluster_forward", "cluster_workspace", "cluster_assign", "cluster_mean",

@@ -1371,7 +1371,7 @@ def rows_with_entries(rows, taken, rng, cols=300):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
-@pytest.mark.parametrize("width", [1, 8, 33, 200, 512])
+@pytest.mark.parametrize("width", [1, 8, 33, 200, 257, 512, 602])
 def test_products_of_int64_arrays_with_stretches_of_empty_rows(width, dtype):
     """Rows without entries between those of one workgroup, around the number from which the rows are found from the entries, in
     blocks with fewer and with more workgroups of entries than of rows to clear.  Whole numbers: the sums are exact in any order."""
