@@ -1398,7 +1398,8 @@ Tensor cluster_reconstruct_backward(Tensor grad, Tensor index, Tensor output, in
 
 // The ReLU form of cluster_reconstruct that also returns the sign of every output element as one
 // bit: (rows [N, F], signs int32 [N, ceil(F / 32)]), or, by group, masks int32 [groups, ceil(F / 32)]: the rows
-// of a group are copies of one representative and have the same signs.  room: as many rows of words at least.
+// of a group are copies of one representative and have the same signs.  Words of groups that do not occur are zero.  room: as
+// many rows of words at least, those behind the groups zero, too.
 std::tuple<Tensor, Tensor> reconstruct_with_signs(const char *op, const Tensor &reps, const Tensor &index,
                                                   const c10::optional<Tensor> &bias, const c10::optional<std::vector<Tensor>> &members,
                                                   bool by_group, int64_t room = 0) {
@@ -1411,7 +1412,9 @@ std::tuple<Tensor, Tensor> reconstruct_with_signs(const char *op, const Tensor &
     c10::hip::HIPGuardMasqueradingAsCUDA guard(reps.device());
     const int64_t N = index.numel(), F = reps.size(1);
     Tensor out = torch::empty({N, F}, reps.options());
-    Tensor signs = torch::empty({by_group ? std::max(reps.size(0), room) : N, cgnn_sign_words(F)}, reps.options().dtype(torch::kInt32));
+    const auto words = reps.options().dtype(torch::kInt32);
+    Tensor signs = by_group ? torch::zeros({std::max(reps.size(0), room), cgnn_sign_words(F)}, words)
+                            : torch::empty({N, cgnn_sign_words(F)}, words);
     if (out.numel() == 0) return {out, signs};
     std::vector<Tensor> held;
     const int32_t *perm = production_order(op, members, index, reps.size(0), &held);
@@ -1454,9 +1457,9 @@ Tensor cluster_reconstruct_backward_signs(Tensor grad, Tensor index, Tensor sign
     return reconstruct_backward_with_signs("cluster_reconstruct_backward_signs", grad, index, signs, groups, members, false);
 }
 
-// By group: what a layer keeps for its backward pass (the reference keeps the rows: layer/CompressgnnReconstruct.py:16-22).  A layer
-// keeps it in a tensor with a row of words per row of its output, of which the groups have the first: what hooks on saved
-// tensors are shown has the shape of signs.
+// By group: what a layer may keep for its backward pass (the reference keeps the rows: layer/CompressgnnReconstruct.py:16-22).  A layer
+// keeps it in a tensor with a row of words per row of its output, of which the groups have the first and the others are
+// zero: what hooks on saved tensors are shown has the shape of signs, and no word of it is left over from other tensors.
 std::tuple<Tensor, Tensor> cluster_reconstruct_masks(Tensor reps, Tensor index, c10::optional<Tensor> bias,
                                                      c10::optional<std::vector<Tensor>> members, int64_t room) {
     return reconstruct_with_signs("cluster_reconstruct_masks", reps, index, bias, members, true, room);
@@ -1563,10 +1566,10 @@ Tensor column_sums(const Tensor &x) {
 }
 
 struct ReconstructBackward : torch::autograd::Node {
-    torch::autograd::SavedVariable index, masks;  // masks: one bit per element of a representative, where the rows went through a ReLU
+    torch::autograd::SavedVariable index, signs;  // signs: one bit per element, where the rows went through a ReLU
     Members members;
     int64_t groups = 0;
-    bool relu = false, with_bias = false;
+    bool relu = false, by_group = false, with_bias = false;  // by_group: bits of the representatives, not of the rows
     torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
         const size_t inputs = with_bias ? 2 : 1;
         if (!grads[0].defined()) return torch::autograd::variable_list(inputs);
@@ -1576,8 +1579,8 @@ struct ReconstructBackward : torch::autograd::Node {
             at::NoGradGuard no_grad;
             const Tensor d_rows = grads[0].contiguous(), ids = index.unpack();
             // without a ReLU the operator does not read the rows it is given as output
-            out.push_back(relu ? reconstruct_backward_with_signs("cluster_reconstruct_backward_masks", d_rows, ids, masks.unpack(), groups,
-                                                                 members, true, true)
+            out.push_back(relu ? reconstruct_backward_with_signs("cluster_reconstruct backward", d_rows, ids, signs.unpack(), groups,
+                                                                 members, by_group, by_group)
                                : cluster_reconstruct_backward(d_rows, ids, d_rows, groups, false, members));
             if (with_bias) out.push_back(task_should_compute_output(1) ? column_sums(out[0]) : Tensor());
         }
@@ -1585,34 +1588,38 @@ struct ReconstructBackward : torch::autograd::Node {
     }
     void release_variables() override {
         index.reset_data();
-        masks.reset_data();
+        signs.reset_data();
         members.reset();
     }
     std::string name() const override { return "ReconstructBackward"; }
 };
 
 // rows[i] = act(reps[index[i]] + bias) with its gradients.  The ReLU mask of the gradient is kept as one bit
-// per element of a representative, written by the kernel that produces the rows (the reference keeps the rows themselves:
-// layer/CompressgnnReconstruct.py:16-22); without a ReLU nothing of the [N, F] output is needed again.
+// per element of a row or of a representative, written by the kernel that produces the rows (the reference keeps the rows themselves:
+// layer/CompressgnnReconstruct.py:16-22), in a tensor with a row of words per row of the output; without a ReLU nothing of the
+// [N, F] output is needed again.
 c10::optional<Tensor> reconstruct(Tensor reps, Tensor index, c10::optional<Tensor> bias, bool relu, Members members) {
     if (needs_function(reps, bias)) return c10::nullopt;
-    Tensor rows, masks, ids;
+    Tensor rows, signs, ids;
+    const bool by_group = reps.size(0) <= index.numel();
     {
         at::AutoDispatchBelowADInplaceOrView plain;
         ids = index.contiguous();
         c10::optional<Tensor> b;
         if (bias.has_value() && bias->defined()) b = bias->contiguous();
-        if (relu) std::tie(rows, masks) = cluster_reconstruct_masks(reps.contiguous(), ids, b, members, ids.numel());
+        if (relu) std::tie(rows, signs) = by_group ? cluster_reconstruct_masks(reps.contiguous(), ids, b, members, ids.numel())
+                                                   : cluster_reconstruct_signs(reps.contiguous(), ids, b, members);
         else rows = cluster_reconstruct(reps.contiguous(), ids, b, false, members);
     }
     const bool with_bias = bias.has_value() && bias->defined();
     if (at::GradMode::is_enabled() && (reps.requires_grad() || (with_bias && bias->requires_grad()))) {
         auto node = with_bias ? node_over<ReconstructBackward>(reps, *bias) : node_over<ReconstructBackward>(reps);
         node->index = torch::autograd::SavedVariable(ids, false);
-        if (relu) node->masks = torch::autograd::SavedVariable(masks, false);
+        if (relu) node->signs = torch::autograd::SavedVariable(signs, false);
         node->members = std::move(members);
         node->groups = reps.size(0);
         node->relu = relu;
+        node->by_group = by_group;
         node->with_bias = with_bias;
         torch::autograd::set_history(rows, node);
     }
@@ -2081,7 +2088,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           "cluster_reconstruct_backward with ReLU, masked by the sign bits", py::arg("grad"), py::arg("index"),
           py::arg("signs"), py::arg("groups"), py::arg("members") = py::none());
     m.def("cluster_reconstruct_masks", &cluster_reconstruct_masks,
-          "cluster_reconstruct with ReLU -> (rows, one sign bit per element of a representative)", py::arg("reps"),
+          "cluster_reconstruct with ReLU -> (rows, one sign bit per element of a representative, zero for those without rows)", py::arg("reps"),
           py::arg("index"), py::arg("bias"), py::arg("members") = py::none(), py::arg("room") = 0);
     m.def("cluster_reconstruct_backward_masks", &cluster_reconstruct_backward_masks,
           "cluster_reconstruct_backward with ReLU, masked by the representatives' sign bits", py::arg("grad"), py::arg("index"),

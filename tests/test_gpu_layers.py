@@ -1422,3 +1422,34 @@ def test_products_of_int64_arrays_are_not_held_up_by_empty_rows(width):
     between = time_of({**{r: 8 for r in range(half)}, **{rows - 1 - r: 8 for r in range(half)}})
     many, few = time_of({r: 1 for r in range(rows)}), time_of({r: 8 for r in range(125)})
     assert between < 4 * behind and few < 4 * many, (behind, between, many, few)
+
+
+@pytest.mark.parametrize("rows,clusters,width,bias", [(6, 5, 100, False), (5, 9, 40, True), (3000, 70, 33, True), (3000, 70, 256, False),
+                                                      (1 << 19, 1 << 14, 32, True), (1 << 18, 1 << 13, 40, False)])
+def test_what_a_reconstruct_keeps_is_written(rows, clusters, width, bias):
+    """One bit per element in a tensor with a row of words per row of the output, whether they are the bits of the rows or of
+    the representatives, and the same words each time, whatever the memory held before."""
+    from CompressgnnReconstruct import Compressgnn_Reconstruct
+    gen = torch.Generator(device=DEV).manual_seed(rows)
+    used = clusters - clusters // 3  # the others have no rows
+    ids = torch.randint(0, used, (rows,), device=DEV, generator=gen)
+    reps = torch.randn(clusters, width, device=DEV, generator=gen, requires_grad=True)
+    add = torch.randn(width, device=DEV, generator=gen, requires_grad=True) if bias else None
+    grad = torch.randn(rows, width, device=DEV, generator=gen)
+    inputs = (reps, add) if bias else (reps,)
+    words, seen = (width + 31) // 32, []
+    for left_over in (-1, 0x55555555):
+        kept = []
+        for n in (rows, clusters):  # what is kept may be given the memory of
+            torch.full((n, words), left_over, device=DEV, dtype=torch.int32)
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: kept.append(t) or t, lambda t: t):
+            out = Compressgnn_Reconstruct()(reps, ids, bias=add, activation="relu")
+        assert sorted((tuple(t.shape), t.dtype) for t in kept) == sorted([((rows,), torch.int64), ((rows, words), torch.int32)])
+        seen += [t for t in kept if t.dtype == torch.int32]
+        got = torch.autograd.grad(out, inputs, grad)
+    assert torch.equal(*seen)
+    want = reps.index_select(0, ids)
+    want = (want if add is None else want + add).relu()
+    assert torch.equal(out, want)
+    for a, b in zip(got, torch.autograd.grad(want, inputs, grad)):
+        torch.testing.assert_close(a, b, atol=1e-5 * float(b.abs().max()), rtol=1e-4)  # sums of up to 2^19 numbers in another order
