@@ -1594,25 +1594,40 @@ struct ReconstructBackward : torch::autograd::Node {
     std::string name() const override { return "ReconstructBackward"; }
 };
 
+// Whether a layer keeps the bits of the representatives or those of the rows.  The former save a cache line a member where the
+// rows are summed; they cost the clearing of the tensor, one more launch, and where rows that follow each other belong to different
+// representatives their words are stored one by one, which costs most where a row ends inside a word.  So they are kept for many rows
+// a representative, of launches that take longer than the host does for them.  (us, a forward and its gradient, bits of the rows / of
+// the representatives: 2,449,029 rows of 41,000 representatives with 7 features 193 / 174, 64 395 / 356, 100 598 / 583, 256
+// 1,083 / 1,033; 1,000,003 of 31,000 with 33 130 / 121, 64 142 / 123, 128 303 / 295; 300,007 of 9,400 with 96 79 / 69, 192
+// 121 / 113, but 48 66 / 71.  A sixteenth as many representatives as rows, 2,449,029 rows with 33 376 / 375, 48 380 / 386, 64
+// 415 / 384; an eighth, 48 411 / 431, 100 729 / 749, 64 439 / 423, 128 810 / 774; a quarter, 300,007 rows with 192 141 / 147;
+// half, 1,000,003 with 33 194 / 204.)
+bool keeps_bits_of_groups(int64_t rows, int64_t groups, int64_t F) {
+    return rows >= (F % 32 == 0 ? 8 : 16) * groups && rows * F >= (1 << 24);
+}
+
 // rows[i] = act(reps[index[i]] + bias) with its gradients.  The ReLU mask of the gradient is kept as one bit
 // per element of a row or of a representative, written by the kernel that produces the rows (the reference keeps the rows themselves:
 // layer/CompressgnnReconstruct.py:16-22), in a tensor with a row of words per row of the output; without a ReLU nothing of the
-// [N, F] output is needed again.
+// [N, F] output is needed again, and without a gradient no bits are (16 features, 10^6 rows: 13.6 us with those of the rows,
+// 16.2 with those of the representatives, 12.5 without).
 c10::optional<Tensor> reconstruct(Tensor reps, Tensor index, c10::optional<Tensor> bias, bool relu, Members members) {
     if (needs_function(reps, bias)) return c10::nullopt;
     Tensor rows, signs, ids;
-    const bool by_group = reps.size(0) <= index.numel();
+    const bool with_bias = bias.has_value() && bias->defined();
+    const bool recorded = at::GradMode::is_enabled() && (reps.requires_grad() || (with_bias && bias->requires_grad()));
+    const bool by_group = reps.dim() == 2 && keeps_bits_of_groups(index.numel(), reps.size(0), reps.size(1));
     {
         at::AutoDispatchBelowADInplaceOrView plain;
         ids = index.contiguous();
         c10::optional<Tensor> b;
-        if (bias.has_value() && bias->defined()) b = bias->contiguous();
-        if (relu) std::tie(rows, signs) = by_group ? cluster_reconstruct_masks(reps.contiguous(), ids, b, members, ids.numel())
+        if (with_bias) b = bias->contiguous();
+        if (relu && recorded) std::tie(rows, signs) = by_group ? cluster_reconstruct_masks(reps.contiguous(), ids, b, members, ids.numel())
                                                    : cluster_reconstruct_signs(reps.contiguous(), ids, b, members);
-        else rows = cluster_reconstruct(reps.contiguous(), ids, b, false, members);
+        else rows = cluster_reconstruct(reps.contiguous(), ids, b, relu, members);
     }
-    const bool with_bias = bias.has_value() && bias->defined();
-    if (at::GradMode::is_enabled() && (reps.requires_grad() || (with_bias && bias->requires_grad()))) {
+    if (recorded) {
         auto node = with_bias ? node_over<ReconstructBackward>(reps, *bias) : node_over<ReconstructBackward>(reps);
         node->index = torch::autograd::SavedVariable(ids, false);
         if (relu) node->signs = torch::autograd::SavedVariable(signs, false);

@@ -1425,7 +1425,7 @@ def test_products_of_int64_arrays_are_not_held_up_by_empty_rows(width):
 
 
 @pytest.mark.parametrize("rows,clusters,width,bias", [(6, 5, 100, False), (5, 9, 40, True), (3000, 70, 33, True), (3000, 70, 256, False),
-                                                      (1 << 19, 1 << 14, 32, True), (1 << 18, 1 << 13, 40, False)])
+                                                      (1 << 19, 1 << 14, 32, True), (1 << 18, 1 << 13, 100, False)])
 def test_what_a_reconstruct_keeps_is_written(rows, clusters, width, bias):
     """One bit per element in a tensor with a row of words per row of the output, whether they are the bits of the rows or of
     the representatives, and the same words each time, whatever the memory held before."""
@@ -1453,3 +1453,39 @@ def test_what_a_reconstruct_keeps_is_written(rows, clusters, width, bias):
     assert torch.equal(out, want)
     for a, b in zip(got, torch.autograd.grad(want, inputs, grad)):
         torch.testing.assert_close(a, b, atol=1e-5 * float(b.abs().max()), rtol=1e-4)  # sums of up to 2^19 numbers in another order
+
+
+@pytest.mark.parametrize("rows,clusters,width,of_groups", [
+    (1 << 19, 1 << 16, 32, True), (1 << 19, (1 << 16) + 1, 32, False), ((1 << 19) - 1, 1 << 13, 32, False), (508401, 7, 33, True),
+    (65537, 200, 256, True), (65535, 200, 256, False), (55925, 3495, 300, True), (55925, 3496, 300, False), (3000, 3, 224, False)])
+def test_which_bits_a_reconstruct_keeps(rows, clusters, width, of_groups):
+    """Those of the representatives from 2^24 elements and 16 rows each on, 8 where a row is whole words, those of the rows
+    otherwise; the gradient is that of the operators with either, bit for bit.  Without a gradient nothing is kept or made."""
+    import compressgnn_runtime as rt
+    from CompressgnnReconstruct import Compressgnn_Reconstruct
+    gen = torch.Generator(device=DEV).manual_seed(rows)
+    ids = torch.randint(0, clusters, (rows,), device=DEV, generator=gen)
+    reps = torch.randn(clusters, width, device=DEV, generator=gen, requires_grad=True)
+    grad = torch.randn(rows, width, device=DEV, generator=gen)
+    out, signs = rt.cluster_reconstruct_signs(reps.detach(), ids, None, None)
+    kept = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: kept.append(t) or t, lambda t: t):
+        layer = Compressgnn_Reconstruct()(reps, ids, activation="relu")
+    kept = [t for t in kept if t.dtype == torch.int32][0]
+    assert torch.equal(layer, out)
+    if of_groups:
+        assert torch.equal(kept[ids], signs) and not kept[clusters:].any()
+    else:
+        assert torch.equal(kept, signs)
+    want = rt.cluster_reconstruct_backward_signs(grad, ids, signs, clusters, None)
+    assert torch.equal(torch.autograd.grad(layer, reps, grad)[0].view(torch.int32), want.view(torch.int32))
+    del layer, kept, signs
+    with torch.no_grad():
+        alone = Compressgnn_Reconstruct()(reps, ids, activation="relu")
+        torch.cuda.synchronize()
+        assert torch.equal(alone, out)
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        again = Compressgnn_Reconstruct()(reps, ids, activation="relu")
+        size = -(-rows * width * 4 // 512) * 512
+        assert torch.cuda.max_memory_allocated() - before < size + rows * 4 and again.numel() == alone.numel()
