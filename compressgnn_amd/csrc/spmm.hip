@@ -898,9 +898,15 @@ __global__ __launch_bounds__(kBlock, ROUND == kDeepRound ? 2 : ROUND == kMidRoun
     // gathers, which do not need them: a chain of entries -> gathers a batch, where it was entries -> rows -> gathers, one batch
     // behind the other.  A launch that fits the card at once is little but that chain (web graphs, forward, us, before / so:
     // 50,001 vertices of 47 features 23.5 / 22.2, 100,003 of 32 31.1 / 29.0, 200,003 of 16 45.7 / 42.7).  The two-source product
-    // of large graphs is bound by its traffic and sits at its register limit, the masked sums spill: neither reads ahead.
-    constexpr bool kAhead = ROUND == kDeepRound || has_values(MODE) || MODE == MODE_UNIT || MODE == MODE_ROW_MASK;
-    constexpr bool kRowsBehindGathers = MODE != MODE_DUAL;
+    // of large graphs is bound by its traffic and sits at its register limit: neither.  Sums of members masked one by one: neither, they
+    // spilled two to four registers with the rows behind the gathers (1,000,003 rows of 100 features, 2,000 sums, by the rows'
+    // signs 242 us, 222 without, by bits 165 and 157; 100,003 of 64 into 1,562 22.5 and 18).  Member lists have no rowmap to wait for, and
+    // rows that end after a few entries were held up (300,007 rows of 32 features into half as many sums 20.5 us, 16.6 without; of
+    // 64 29.0 and 26.5; a thirtieth as many 15.9 and 16.0): behind the gathers only up to 64 bytes a gather (2,449,029 rows of 16
+    // features 121.4 us, 124.5 without), ahead but for rows of a whole wave (200,003 rows of 256 into a quarter 54.3 us, 49.3 without).
+    constexpr bool kAhead = ROUND == kDeepRound || has_values(MODE) || MODE == MODE_ROW_MASK || (MODE == MODE_UNIT && LPR < kWave);
+    constexpr bool kRowsBehindGathers =
+        has_values(MODE) || MODE == MODE_ROW_MASK || (MODE == MODE_UNIT && VEC * LPR * sizeof(T) <= 64);
     __shared__ int wg_row[GPB];
     constexpr bool kOnce = WGRUNS == WGRUNS_ONCE;
     __shared__ Pack<T, VEC> wg_carry[kOnce ? 1 : TILES][kOnce ? 1 : kBlock];

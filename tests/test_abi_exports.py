@@ -4,6 +4,8 @@ the reference's operator names."""
 import ctypes
 import os
 import re
+import shutil
+import subprocess
 import sys
 
 import pytest
@@ -69,6 +71,25 @@ def test_entries_per_workgroup_of_products_of_int64_arrays(F, nnz, double, parts
     workgroups = -(-nnz // (groups * run))
     assert arrivals.value == workgroups * parts
     assert total == 2 * workgroups * F * (8 if double else 4)
+
+
+def test_kernels_spill_no_registers(tmp_path):
+    """What the compiler says of the kernels of the device library: none puts registers aside in memory."""
+    from compressgnn_amd import abi
+    tools = "/opt/rocm/llvm/bin"
+    if not os.path.exists(os.path.join(tools, "llvm-readelf")):
+        pytest.skip("no llvm-readelf")
+    shutil.copy(abi.LIB_PATH, tmp_path / "lib.so")  # the code objects are written beside it
+    subprocess.run([os.path.join(tools, "llvm-objdump"), "--offloading", "lib.so"], cwd=tmp_path, check=True, stdout=subprocess.DEVNULL)
+    kernels, spilled = 0, []
+    for part in sorted(tmp_path.glob("*gfx950")):
+        notes = subprocess.run([os.path.join(tools, "llvm-readelf"), "--notes", str(part)], check=True, stdout=subprocess.PIPE, text=True).stdout
+        for kernel in re.split(r"\n  - ", notes):
+            name, count = re.findall(r"\.symbol:\s+(\S+)", kernel), re.search(r"\.vgpr_spill_count:\s+(\d+)", kernel)
+            if count:
+                kernels += 1
+                spilled += [name[-1]] if int(count[1]) else []
+    assert kernels > 400 and not spilled
 
 
 def test_runtime_module_has_the_reference_operator_names():
