@@ -415,7 +415,8 @@ def test_sign_bits_of_special_values():
 def test_one_mask_per_representative(n, width, clusters, dtype):
     """Masks of representatives against the masks of their rows, bit for bit: rows, words and gradients, where the sums are one
     launch, runs with carries, and carries of several levels; NaN, infinities and zeros of both signs among the
-    representatives, infinities and NaN in the gradient.  An unused group has no members and a gradient of zero."""
+    representatives, infinities and NaN in the gradient, kept sums of nothing but zeros below zero, masked ones of negative numbers.
+    An unused group has no members and a gradient of zero."""
     import compressgnn_runtime as rt
     gen = torch.Generator(device=DEV).manual_seed(n + width)
     ids = (torch.rand(n, device=DEV, generator=gen) ** 3 * clusters).long()
@@ -427,6 +428,16 @@ def test_one_mask_per_representative(n, width, clusters, dtype):
     bias[::3] = 0.0
     grad = torch.randn(n, width, device=DEV, generator=gen, dtype=dtype)
     grad.view(-1)[::101], grad.view(-1)[50::103] = float("inf"), float("nan")
+    kept, dropped = groups - 2, 0  # the last group with members and the first, which has most of them
+    reps[dropped], reps[kept] = -50.0, 50.0
+    grad[ids == dropped] = -grad[ids == dropped].abs()
+    grad[ids == kept] = -0.0
+    bits = torch.int32 if dtype == torch.float32 else torch.int64
+
+    def equal_bits(a, b):  # but those that tell one NaN from another
+        nan = torch.isnan(a)
+        return torch.equal(nan, torch.isnan(b)) and torch.equal(a.view(bits)[~nan], b.view(bits)[~nan])
+
     lists = list(abi.cluster_members(ids, groups))
     for members in (lists, None):
         rows, signs = rt.cluster_reconstruct_signs(reps, ids, bias, members)
@@ -435,8 +446,9 @@ def test_one_mask_per_representative(n, width, clusters, dtype):
         assert torch.equal(masks[ids], signs)
         want = rt.cluster_reconstruct_backward_signs(grad, ids, signs, groups, members)
         got = rt.cluster_reconstruct_backward_masks(grad, ids, masks, groups, members)
-        assert torch.equal(torch.nan_to_num(got, nan=3.0), torch.nan_to_num(want, nan=3.0))
-        assert torch.equal(got[clusters], torch.zeros(width, device=DEV, dtype=dtype))
+        assert equal_bits(got, want) and equal_bits(got, rt.cluster_reconstruct_backward(grad, ids, rows, groups, True, members))
+        for row in (dropped, clusters) if clusters > 1 else (clusters,):
+            assert not got[row].view(bits).any()
 
 
 def test_masks_of_the_wrong_shape_are_refused():
