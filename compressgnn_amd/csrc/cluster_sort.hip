@@ -148,10 +148,11 @@ __device__ __forceinline__ unsigned long long same_digit(int d, unsigned long lo
 // OWN_SCAN: `within` holds the tiles' histograms (tile_histogram), `total` is not read.
 //
 // A tile is dealt to kSortThreads threads, ITEMS keys each: its time is a chain -- loads, a step of ballots and one look at LDS
-// per 64 keys of a wave, three barriers, stores -- and all tiles of a launch are resident at once, so the launch takes as long as
-// one of them.  With 256 threads a wave ranked 1,024 keys in sixteen steps (us a pass, so / with 1,024 threads: 2,449,029 keys
+// per 64 keys of a wave, three barriers, stores -- and up to 512 tiles, two a compute unit, 2,097,152 keys, are resident at once, so
+// the launch takes as long as one of them; with more keys the tiles behind these take a second round, where it gains less.  With
+// 256 threads a wave ranked 1,024 keys in sixteen steps (us a pass, so / with 1,024 threads: 2,449,029 keys, 598 tiles,
 // 22.6 / 20.7, 1,000,003 15.1 / 13.0; hashing and grouping rows of 24 columns by 16 planes: 100,003 rows 58.6 / 54.0, 262,145
-// 73.9 / 64.4, 450,000 80.2 / 69.8).
+// 73.9 / 64.4, 450,000 80.2 / 69.8, 2,100,000 132 / 127, 2,449,029 146 / 141, 4,000,000 199 / 192).
 template <int ITEMS, bool OWN_SCAN>
 __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(const int32_t *__restrict__ keys,
                                                               const int32_t *__restrict__ vals, int64_t N, int shift,

@@ -1885,8 +1885,10 @@ constexpr int64_t kResidentLanes = 256 * 32 * kWave;
 
 template <typename T>
 Shape row_shape(int64_t F, int64_t rows, int64_t nnz, int32_t max_row_nnz) {
-    // parts of 64 packs for rows of eight entries and more (gradient, 512 features, two tiles / parts: 325,557 vertices of 10.8
-    // entries 567 / 551 us, 200,003 of 8 277 / 280, of 5 226 / 238)
+    // parts of 64 packs for rows of eight entries and more (gradient, two tiles / parts: 512 features, 325,557 vertices of 10.8
+    // entries 567 / 551 us, 200,003 of 8 277 / 280, of 5 226 / 238; 10.8 entries, 5,000 vertices of 512, 768, 1,024 and 2,048 features
+    // 9.0 / 9.1, 13.0 / 12.0, 15.7 / 14.8 and 27.0 / 26.0, 20,000 29.2 / 28.1, 44.2 / 39.9, 54.8 / 51.8 and 113 / 108, 100,003
+    // 152 / 149, 264 / 235 and, of 1,024, 324 / 327)
     const Shape wide = pick_shape<T>(F, false, nnz < 8 * rows);
     if (sizeof(T) != 4 || wide.tiles != 1 || wide.grid_y != 1) return wide;
     Shape s = wide;
@@ -2337,7 +2339,9 @@ OnceLayout once_layout(int64_t rows, int64_t nnz, int64_t F, int dtype) {
     A.nnz = nnz;
     A.seg_nnz = 32;  // as for the blocks of a plan
     OnceLayout L;
-    // 512 features, two tiles / parts: out-lists of 6,000 vertices 14.6 / 19.5 us, of 20,000 38.9 / 36.7, 325,557 814 / 745
+    // Two tiles / parts, us: 512 features, out-lists of 6,000 vertices 14.6 / 19.5, of 20,000 38.9 / 36.7, of 325,557 814 / 745.  Of
+    // 768, 1,024 and 2,048 parts are faster in every block of 2^17 entries and more that was looked at, in-lists and out-lists of 20,000 and
+    // 100,003 vertices of degree 5 to 9.8: 1.02 to 1.17 times.
     const bool two_tiles = nnz < (1 << 17);  // a small product
     L.shape = dtype == CGNN_F64 ? pick_shape<double>(F, true, two_tiles) : pick_shape<float>(F, true, two_tiles);
     L.groups = kBlock / L.shape.lpr;
