@@ -6,6 +6,7 @@
 // current stream.  There is no CPU implementation behind these operators: CPU tensors
 // are rejected with an error.
 #include <ATen/Parallel.h>
+#include <ATen/SavedTensorHooks.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
@@ -1398,11 +1399,10 @@ Tensor cluster_reconstruct_backward(Tensor grad, Tensor index, Tensor output, in
 
 // The ReLU form of cluster_reconstruct that also returns the sign of every output element as one
 // bit: (rows [N, F], signs int32 [N, ceil(F / 32)]), or, by group, masks int32 [groups, ceil(F / 32)]: the rows
-// of a group are copies of one representative and have the same signs.  Words of groups that do not occur are zero.  room: as
-// many rows of words at least, those behind the groups zero, too.
+// of a group are copies of one representative and have the same signs.  Words of groups that do not occur are not written.
 std::tuple<Tensor, Tensor> reconstruct_with_signs(const char *op, const Tensor &reps, const Tensor &index,
                                                   const c10::optional<Tensor> &bias, const c10::optional<std::vector<Tensor>> &members,
-                                                  bool by_group, int64_t room = 0) {
+                                                  bool by_group) {
     expect(op, reps, {{Role::Features, "representatives", &reps}, {Role::Ids, "index", &index}});
     if (bias.has_value()) {
         expect(op, reps, {{Role::Bias, "bias", &*bias}});
@@ -1412,9 +1412,7 @@ std::tuple<Tensor, Tensor> reconstruct_with_signs(const char *op, const Tensor &
     c10::hip::HIPGuardMasqueradingAsCUDA guard(reps.device());
     const int64_t N = index.numel(), F = reps.size(1);
     Tensor out = torch::empty({N, F}, reps.options());
-    const auto words = reps.options().dtype(torch::kInt32);
-    Tensor signs = by_group ? torch::zeros({std::max(reps.size(0), room), cgnn_sign_words(F)}, words)
-                            : torch::empty({N, cgnn_sign_words(F)}, words);
+    Tensor signs = torch::empty({by_group ? reps.size(0) : N, cgnn_sign_words(F)}, reps.options().dtype(torch::kInt32));
     if (out.numel() == 0) return {out, signs};
     std::vector<Tensor> held;
     const int32_t *perm = production_order(op, members, index, reps.size(0), &held);
@@ -1429,16 +1427,15 @@ std::tuple<Tensor, Tensor> reconstruct_with_signs(const char *op, const Tensor &
     return {out, signs};
 }
 
-// cluster_reconstruct_backward with relu = true, the mask taken from the words above.  room: there may be more rows of words
-// than are read.
+// cluster_reconstruct_backward with relu = true, the mask taken from the words above.
 Tensor reconstruct_backward_with_signs(const char *op, const Tensor &grad, const Tensor &index, const Tensor &signs, int64_t groups,
-                                       const c10::optional<std::vector<Tensor>> &members, bool by_group, bool room = false) {
+                                       const c10::optional<std::vector<Tensor>> &members, bool by_group) {
     expect(op, grad, {{Role::Features, "grad", &grad}, {Role::Ids, "index", &index}});
     TORCH_CHECK(groups >= 0, op, ": groups = ", groups);
     TORCH_CHECK(index.numel() == grad.size(0), op, ": ", grad.size(0), " rows but ", index.numel(), " cluster ids");
     const int64_t N = grad.size(0), F = grad.size(1), of = by_group ? groups : N;
     TORCH_CHECK(signs.device() == grad.device() && signs.scalar_type() == torch::kInt32 && signs.is_contiguous() &&
-                    signs.dim() == 2 && (room ? signs.size(0) >= of : signs.size(0) == of) && signs.size(1) == cgnn_sign_words(F),
+                    signs.dim() == 2 && signs.size(0) == of && signs.size(1) == cgnn_sign_words(F),
                 op, by_group ? ": masks" : ": signs", " must be a contiguous int32 tensor [", of, ", ", cgnn_sign_words(F),
                 "] on the device of grad");
     c10::hip::HIPGuardMasqueradingAsCUDA guard(grad.device());
@@ -1457,12 +1454,10 @@ Tensor cluster_reconstruct_backward_signs(Tensor grad, Tensor index, Tensor sign
     return reconstruct_backward_with_signs("cluster_reconstruct_backward_signs", grad, index, signs, groups, members, false);
 }
 
-// By group: what a layer may keep for its backward pass (the reference keeps the rows: layer/CompressgnnReconstruct.py:16-22).  A layer
-// keeps it in a tensor with a row of words per row of its output, of which the groups have the first and the others are
-// zero: what hooks on saved tensors are shown has the shape of signs, and no word of it is left over from other tensors.
+// By group: what a layer may keep for its backward pass (the reference keeps the rows: layer/CompressgnnReconstruct.py:16-22).
 std::tuple<Tensor, Tensor> cluster_reconstruct_masks(Tensor reps, Tensor index, c10::optional<Tensor> bias,
-                                                     c10::optional<std::vector<Tensor>> members, int64_t room) {
-    return reconstruct_with_signs("cluster_reconstruct_masks", reps, index, bias, members, true, room);
+                                                     c10::optional<std::vector<Tensor>> members) {
+    return reconstruct_with_signs("cluster_reconstruct_masks", reps, index, bias, members, true);
 }
 
 Tensor cluster_reconstruct_backward_masks(Tensor grad, Tensor index, Tensor masks, int64_t groups,
@@ -1580,7 +1575,7 @@ struct ReconstructBackward : torch::autograd::Node {
             const Tensor d_rows = grads[0].contiguous(), ids = index.unpack();
             // without a ReLU the operator does not read the rows it is given as output
             out.push_back(relu ? reconstruct_backward_with_signs("cluster_reconstruct backward", d_rows, ids, signs.unpack(), groups,
-                                                                 members, by_group, by_group)
+                                                                 members, by_group)
                                : cluster_reconstruct_backward(d_rows, ids, d_rows, groups, false, members));
             if (with_bias) out.push_back(task_should_compute_output(1) ? column_sums(out[0]) : Tensor());
         }
@@ -1595,35 +1590,36 @@ struct ReconstructBackward : torch::autograd::Node {
 };
 
 // Whether a layer keeps the bits of the representatives or those of the rows.  The former save a cache line a member where the
-// rows are summed; they cost the clearing of the tensor, one more launch, and where rows that follow each other belong to different
-// representatives their words are stored one by one, which costs most where a row ends inside a word.  So they are kept for many rows
-// a representative, of launches that take longer than the host does for them.  (us, a forward and its gradient, bits of the rows / of
-// the representatives: 2,449,029 rows of 41,000 representatives with 7 features 193 / 174, 64 395 / 356, 100 598 / 583, 256
-// 1,083 / 1,033; 1,000,003 of 31,000 with 33 130 / 121, 64 142 / 123, 128 303 / 295; 300,007 of 9,400 with 96 79 / 69, 192
-// 121 / 113, but 48 66 / 71.  A sixteenth as many representatives as rows, 2,449,029 rows with 33 376 / 375, 48 380 / 386, 64
-// 415 / 384; an eighth, 48 411 / 431, 100 729 / 749, 64 439 / 423, 128 810 / 774; a quarter, 300,007 rows with 192 141 / 147;
-// half, 1,000,003 with 33 194 / 204.)
+// rows are summed, and all but a row of words per representative of what is held until then (1.3 of 78 MB for 2,449,029 rows of 256
+// features); where rows that follow each other belong to different representatives their words are stored one by one, which costs most
+// where a row ends inside a word.  So they are kept for many rows a representative, or few where a row is one word or whole ones.  (us,
+// a forward and its gradient, bits of the rows / of the representatives: 2,449,029 rows of 41,000 representatives with 7 features
+// 193 / 171, 64 395 / 351, 100 598 / 576, 256 1,083 / 1,021; 300,007 of 9,400 with 96 79 / 66.  A sixteenth as many representatives
+// as rows, 2,449,029 with 33 376 / 369, 48 380 / 381; an eighth, with 48 411 / 426, 1,000,003 with 100 329 / 340, but 16 75 / 71;
+// a quarter, 1,000,003 with 64 178 / 168, 128 357 / 352, 256 665 / 658, but 33 159 / 161, 48 165 / 168; half, 64 224 / 219, 256
+// 760 / 762.)
 bool keeps_bits_of_groups(int64_t rows, int64_t groups, int64_t F) {
-    return rows >= (F % 32 == 0 ? 8 : 16) * groups && rows * F >= (1 << 24);
+    return rows >= (F <= 32 || F % 32 == 0 ? 4 : 16) * groups;
 }
 
 // rows[i] = act(reps[index[i]] + bias) with its gradients.  The ReLU mask of the gradient is kept as one bit
 // per element of a row or of a representative, written by the kernel that produces the rows (the reference keeps the rows themselves:
-// layer/CompressgnnReconstruct.py:16-22), in a tensor with a row of words per row of the output; without a ReLU nothing of the
-// [N, F] output is needed again, and without a gradient no bits are (16 features, 10^6 rows: 13.6 us with those of the rows,
-// 16.2 with those of the representatives, 12.5 without).
+// layer/CompressgnnReconstruct.py:16-22); without a ReLU nothing of the [N, F] output is needed again, and without a gradient
+// no bits are (16 features, 10^6 rows: 13.6 us with those of the rows, 16.2 with those of the representatives, 12.5 without).
+// Hooks on saved tensors are shown the bits of the rows: a row of words per row of the output, all of them written.
 c10::optional<Tensor> reconstruct(Tensor reps, Tensor index, c10::optional<Tensor> bias, bool relu, Members members) {
     if (needs_function(reps, bias)) return c10::nullopt;
     Tensor rows, signs, ids;
     const bool with_bias = bias.has_value() && bias->defined();
     const bool recorded = at::GradMode::is_enabled() && (reps.requires_grad() || (with_bias && bias->requires_grad()));
-    const bool by_group = reps.dim() == 2 && keeps_bits_of_groups(index.numel(), reps.size(0), reps.size(1));
+    const bool hooks = !at::SavedTensorDefaultHooks::get_tls_state().stack.empty();
+    const bool by_group = !hooks && reps.dim() == 2 && keeps_bits_of_groups(index.numel(), reps.size(0), reps.size(1));
     {
         at::AutoDispatchBelowADInplaceOrView plain;
         ids = index.contiguous();
         c10::optional<Tensor> b;
         if (with_bias) b = bias->contiguous();
-        if (relu && recorded) std::tie(rows, signs) = by_group ? cluster_reconstruct_masks(reps.contiguous(), ids, b, members, ids.numel())
+        if (relu && recorded) std::tie(rows, signs) = by_group ? cluster_reconstruct_masks(reps.contiguous(), ids, b, members)
                                                    : cluster_reconstruct_signs(reps.contiguous(), ids, b, members);
         else rows = cluster_reconstruct(reps.contiguous(), ids, b, relu, members);
     }
@@ -2103,8 +2099,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           "cluster_reconstruct_backward with ReLU, masked by the sign bits", py::arg("grad"), py::arg("index"),
           py::arg("signs"), py::arg("groups"), py::arg("members") = py::none());
     m.def("cluster_reconstruct_masks", &cluster_reconstruct_masks,
-          "cluster_reconstruct with ReLU -> (rows, one sign bit per element of a representative, zero for those without rows)", py::arg("reps"),
-          py::arg("index"), py::arg("bias"), py::arg("members") = py::none(), py::arg("room") = 0);
+          "cluster_reconstruct with ReLU -> (rows, one sign bit per element of a representative that has rows)", py::arg("reps"),
+          py::arg("index"), py::arg("bias"), py::arg("members") = py::none());
     m.def("cluster_reconstruct_backward_masks", &cluster_reconstruct_backward_masks,
           "cluster_reconstruct_backward with ReLU, masked by the representatives' sign bits", py::arg("grad"), py::arg("index"),
           py::arg("masks"), py::arg("groups"), py::arg("members") = py::none());
