@@ -681,6 +681,7 @@ __device__ __forceinline__ void once_stretch(const SpmmArgs<T> &a, const WideRow
             for (int u = 0; u < kAtOnce; ++u)
                 if (k + u * kBlock < count) row_of[k + u * kBlock] = lo[u];
         }
+        if (count <= 0 && threadIdx.x == 0) row_of[0] = r0;  // row pointers that descend: a row of Y all the same
         __syncthreads();
         return;
     }
