@@ -169,8 +169,8 @@ __global__ __launch_bounds__(kScanBlock) void merger_tile_sums_kernel(int32_t *_
 // store_now or added with an atomic -- and read with load_now: a release would write back the whole L2.  Arrivals at one counter come
 // one after the other, some 12 ns each (1,600: 32 us for a launch of 12), so more than kFew workgroups arrive at one of
 // kArrivalGroups counters first, and the last one there at the one for all.  Beyond kMany the launches behind stay.  (With the
-// launches / one counter up to kFew / so: 121,075 vertices of degree 10.2 at a frequency of 4 1,234 / 1,199 / 1,181 us a call,
-// 325,557 of 9.8 at 16 1,361 / 1,341 / 1,330.)
+// launches / one counter up to kFew / so: 121,075 vertices of degree 10.2 at a frequency of 4 1,234 / 1,199 / 1,181 us a call.
+// 325,557 of 9.8 at 16, three quarters of whose 1,350 us are the link and the counts, take the same within 3 %, as their runs differ.)
 constexpr unsigned kFew = 256, kArrivalGroups = 16, kMany = kFew * kArrivalGroups;
 constexpr int kLine = 32;  // integers of a cache line
 __device__ __forceinline__ void store_now(int32_t *p, int32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
