@@ -1472,21 +1472,20 @@ def test_which_bits_a_reconstruct_keeps(rows, clusters, width, of_groups):
     grad = torch.randn(rows, width, device=DEV, generator=gen)
     out, signs = rt.cluster_reconstruct_signs(reps.detach(), ids, None, None)
     want = rt.cluster_reconstruct_backward_signs(grad, ids, signs, clusters, None)
-    block = lambda n: -(-n * 4 // 512) * 512  # the allocator's
     words = signs.size(1)
 
     def held(mode):
         Compressgnn_Reconstruct()(reps, ids, activation="relu")  # what is made once per index is there
         torch.cuda.synchronize()
         gc.collect()
-        before = torch.cuda.memory_allocated()
+        before = _requested()  # what tensors ask for: what they are given depends on the blocks that earlier tests left
         with mode:
             layer = Compressgnn_Reconstruct()(reps, ids, activation="relu")
         assert torch.equal(layer, out)
-        return layer, torch.cuda.memory_allocated() - before - block(rows * width)
+        return layer, _requested() - before - 4 * rows * width
 
     layer, kept = held(torch.enable_grad())
-    assert kept == block((clusters if of_groups else rows) * words)
+    assert kept == 4 * (clusters if of_groups else rows) * words
     assert torch.equal(torch.autograd.grad(layer, reps, grad)[0].view(torch.int32), want.view(torch.int32))
     del layer
     assert held(torch.no_grad())[1] == 0
